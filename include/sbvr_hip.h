@@ -278,13 +278,11 @@ int sbvr_hip_mm_T(const uint32_t *l_bvr, const void *l_coeff_idx, int l_idx_byte
  * The same product with room for a split of K across workgroups: a workspace of
  * sbvr_hip_mm_T_workspace(M, N) bytes (M*N 64-bit accumulators, zero-filled once, 8-byte aligned,
  * left zero by every call; it may be the workspace of sbvr_hip_linear_f16, not used by two calls
- * at once).  One left row of up to 4 planes (the case the reference's kernels are written for,
- * sbvr_kernel.cu:464-562) at the decode kernel's shapes (N >= 16, K and G multiples of 128, G / 128
- * a power of two, 2, 3, 4, 6 or 8 right planes) runs on that kernel: the left operand's planes,
- * each times its coefficient, are its batch rows, the popcounts come out of the matrix cores and the
- * rows are added up in fp32 before the one rounding.  Where that launch splits K across workgroups
- * (N = 4096 at K = 14336 on an MI355X) it needs the workspace; without one, and for every other
- * shape, the popcount kernels of sbvr_hip_mm_T run.  The reference's operator has no such argument
+ * at once).  K and G multiples of 128, up to 16 left planes and 2, 3, 4, 6 or 8 right planes: the popcounts come out
+ * of the matrix cores, any number of left rows.  One left row of up to 4 planes against 8192 columns and more (G / 128
+ * a power of two) runs on the decode kernel, the left operand's planes, each times its coefficient, as its batch rows;
+ * where that launch splits K across workgroups it needs the workspace, without one it takes the former kernel.  Other
+ * shapes: popcounts on the vector ALU.  The reference's operator has no such argument
  * (sbvr_ops.cpp:35-76); its bindings here bring their own.
  */
 int sbvr_hip_mm_T_ws(const uint32_t *l_bvr, const void *l_coeff_idx, int l_idx_bytes,

@@ -1,0 +1,245 @@
+// Both operands SBVR-encoded, any number of left rows (libsbvr_hip.so, gfx950): the reference's product
+//   out[m, n] = sum_g sum_{l, r} popcount_g(L_l & R_r) a_l b_r      (sbvr_kernel.cu:462-562, sbvr_kernel.cpp:251-399)
+// with the popcounts coming out of the matrix cores.
+#include "sbvr_internal.h"
+#include "sbvr_device.h"
+
+namespace {
+
+constexpr int kMmSub = 128;          // elements of K per MFMA
+
+// A workgroup owns 16 columns and up to 16 * RT (left row, plane) pairs; its W waves take the sub-groups of 128
+// elements of K in turn and meet in LDS.  Per sub-group a lane holds one plane word of its column and plane r and one
+// word of each of its RT left rows, and v_mfma_f32_16x16x128_f8f6f4 with both operands fp4 multiplies the raw bits:
+// nibble q of dword t carries bit 4q + t, as 0.5, 1, 2, 2 on the right and as 2, 1, 0.5, 0.5 on the left, so a
+// product is 1 or 0 and the sums are the popcounts, exact integers in fp32.  A left row's planes are rows of their
+// own ((K / 32, M, Sl) is (K / 32, M * Sl) as it lies), so any number of planes on that side takes the same code.
+// Coefficients in fp32: those of the column per lane (its line, gathered one sub-group ahead), those of the left
+// rows from a small LDS table that the wave fills for itself.
+// Bound by the vector ALU: per 16 x 16 x 128 block and SR right planes 4 SR + 4 FMAs a lane, 7 operations to make the
+// left operand, against 16 clocks per MFMA; with few rows by the latency of the loads in front of it.  (Where the
+// one-thread-per-output kernel took 727 us, 16 rows of 8 planes x 4096 columns x 4096 with 4 right planes, it takes 9.7;
+// 4 rows of 4 planes 4.9 us where the popcount kernel took 9.0.)
+template <int SR, int RT, int W>
+__global__ void __launch_bounds__(64 * W)
+sbvr_mm_T_mfma_kernel(const MmArgs a)
+{
+    constexpr int R = 16 * RT;                       // (left row, plane) pairs of a workgroup
+    constexpr int CW = (SR + 1) / 2;
+    constexpr int PS = SR <= 4 ? SR : SR / 2, PH = SR / PS;     // planes of a step, steps per row tile
+    constexpr int NL = (R + 63) / 64;                // left coefficients a lane fetches per sub-group
+    __shared__ __align__(16) float red[W * R * 16];  // the partial results; before that the waves' coefficients
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, blk = lane >> 4;
+    const int M = a.M, N = a.N, Sl = a.Sl;
+    const int n = blockIdx.x * 16 + col, n_ld = min(n, N - 1);
+    const int m0 = blockIdx.y * a.m_per_wg, m_cnt = min(a.m_per_wg, M - m0);
+    const int rows = m_cnt * Sl, row0 = m0 * Sl, rows_all = M * Sl;
+    const int nsub = a.K / kMmSub;
+    float *const ca = red + wave * R;                // this wave's left coefficients
+
+    // the left coefficients this lane fetches: pair p = lane + 64 i is plane p % Sl of left row p / Sl
+    int lm[NL], lp[NL];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+        const int p = min(lane + 64 * i, rows - 1);
+        lm[i] = m0 + p / Sl;
+        lp[i] = p % Sl;
+    }
+
+    struct Stage {
+        Planes<SR> w;
+        uint32_t aw[RT];
+        int r_lo, r_hi, l_lo[NL], l_hi[NL];          // line indices, as loaded (one or two bytes)
+        uint32_t rc[CW];
+        uint16_t lc[NL];
+    };
+    auto load = [&](int sg, Stage &s) __attribute__((always_inline)) {
+        const size_t word = static_cast<size_t>(4 * sg + blk);
+        s.w = load_planes<SR>(a.r_bvr + (word * N + n_ld) * SR);
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+            s.aw[t] = a.l_bvr[word * rows_all + min(row0 + 16 * t + col, rows_all - 1)];
+        const int g = sg / a.spg;
+        const uint8_t *rb = static_cast<const uint8_t *>(a.r_idx), *lb = static_cast<const uint8_t *>(a.l_idx);
+        const size_t rat = (static_cast<size_t>(g) * N + n_ld) << a.r_idx16;
+        s.r_lo = rb[rat];
+        s.r_hi = rb[rat + a.r_idx16];
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const size_t lat = (static_cast<size_t>(g) * M + lm[i]) << a.l_idx16;
+            s.l_lo[i] = lb[lat];
+            s.l_hi[i] = lb[lat + a.l_idx16];
+        }
+    };
+    auto gather = [&](Stage &s) __attribute__((always_inline)) {
+        const int rline = min(a.r_idx16 ? s.r_lo | (s.r_hi << 8) : s.r_lo, a.Lr - 1);
+        load_line_words<SR>(a.r_cache + static_cast<size_t>(rline) * SR, s.rc);
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int lline = min(a.l_idx16 ? s.l_lo[i] | (s.l_hi[i] << 8) : s.l_lo[i], a.Ll - 1);
+            s.lc[i] = a.l_cache[static_cast<size_t>(lline) * Sl + lp[i]];
+        }
+    };
+
+    v4f y[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+        y[t] = v4f{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](const Stage &s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NL; ++i)
+            if (NL == 1 ? lane < R : true)
+                ca[lane + 64 * i] = h2f(s.lc[i]);
+        __builtin_amdgcn_wave_barrier();
+        v8i B[SR];
+        float c[SR];
+#pragma unroll
+        for (int j = 0; j < SR; ++j) {
+            const uint32_t w = s.w.w[j];
+            B[j] = v8i{static_cast<int>(w & 0x11111111u), static_cast<int>(w & 0x22222222u), static_cast<int>(w & 0x44444444u),
+                       static_cast<int>((w >> 1) & 0x44444444u), 0, 0, 0, 0};
+            c[j] = h2f(static_cast<uint16_t>(j & 1 ? s.rc[j / 2] >> 16 : s.rc[j / 2] & 0xffffu));
+        }
+        // A step is up to 4 planes of one row tile: its MFMAs are issued together, and the results of the step before
+        // are multiplied with their coefficients while they run (left to itself the compiler lets every MFMA's
+        // consumers wait for it before it issues the next one: 118 us against 110 for 64 rows of 8 planes x 14336 x 4096)
+        v4f D[2][PS];
+        v4f sum = v4f{0.f, 0.f, 0.f, 0.f};
+        auto consume = [&](int step) __attribute__((always_inline)) {
+            const int t = step / PH, ph = step % PH;
+#pragma unroll
+            for (int j = 0; j < PS; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    sum[i] = ph == 0 && j == 0 ? D[step & 1][j][i] * c[0] : fmaf(D[step & 1][j][i], c[ph * PS + j], sum[i]);
+            if (ph == PH - 1) {
+                const v4f la = *reinterpret_cast<const v4f *>(ca + 16 * t + 4 * blk);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    y[t][i] = fmaf(la[i], sum[i], y[t][i]);
+            }
+        };
+        v8i A;
+#pragma unroll
+        for (int step = 0; step < RT * PH; ++step) {
+            if (step % PH == 0) {
+                const uint32_t w = s.aw[step / PH];
+                A = v8i{static_cast<int>((w << 2) & 0x44444444u), static_cast<int>(w & 0x22222222u),
+                        static_cast<int>((w >> 2) & 0x11111111u), static_cast<int>((w >> 3) & 0x11111111u), 0, 0, 0, 0};
+            }
+#pragma unroll
+            for (int j = 0; j < PS; ++j)
+                D[step & 1][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B[(step % PH) * PS + j], v4f{0.f, 0.f, 0.f, 0.f},
+                                                                                  4, 4, 0, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (step > 0)
+                consume(step - 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        consume(RT * PH - 1);
+        __builtin_amdgcn_wave_barrier();
+    };
+
+    // (two register sets; a sub-group past the end repeats the last one and is not computed)
+    Stage s0, s1;
+    if (wave < nsub) {                               // wave-uniform
+        load(wave, s0);
+        gather(s0);
+        for (int sg = wave; sg < nsub; sg += 2 * W) {
+            load(min(sg + W, nsub - 1), s1);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(s0);
+            gather(s1);
+            if (sg + W >= nsub)
+                break;
+            load(min(sg + 2 * W, nsub - 1), s0);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(s1);
+            gather(s0);
+        }
+    }
+    __syncthreads();                                 // (the coefficients' place is free now)
+
+    // partial results: [wave][pair][column]
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            red[(wave * R + 16 * t + 4 * blk + i) * 16 + col] = y[t][i];
+    __syncthreads();
+    for (int o = threadIdx.x; o < rows * 16; o += 64 * W) {     // over the waves, per (pair, column)
+        float total = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w)
+            total += red[w * R * 16 + o];
+        red[o] = total;                              // (this thread's own slot of wave 0)
+    }
+    __syncthreads();
+    for (int o = threadIdx.x; o < m_cnt * 16; o += 64 * W) {    // over the planes of a left row
+        const int mm = o >> 4, cc = o & 15, nn = blockIdx.x * 16 + cc;
+        float total = 0.f;
+        for (int l = 0; l < Sl; ++l)
+            total += red[(mm * Sl + l) * 16 + cc];
+        if (nn < N) {
+            uint16_t v = f2h(total);
+            if (a.bias)
+                v = hadd(v, a.bias[nn]);
+            a.out[static_cast<size_t>(m0 + mm) * N + nn] = v;
+        }
+    }
+}
+
+template <int SR>
+hipError_t launch_rt(int RT, int W, const MmArgs &a, hipStream_t st)
+{
+    const dim3 grid(static_cast<unsigned>((a.N + 15) / 16), static_cast<unsigned>((a.M + a.m_per_wg - 1) / a.m_per_wg)), block(64 * W);
+    if (RT == 4)
+        hipLaunchKernelGGL((sbvr_mm_T_mfma_kernel<SR, 4, 8>), grid, block, 0, st, a);
+    else if (RT == 2 && W == 16)
+        hipLaunchKernelGGL((sbvr_mm_T_mfma_kernel<SR, 2, 16>), grid, block, 0, st, a);
+    else if (RT == 2)
+        hipLaunchKernelGGL((sbvr_mm_T_mfma_kernel<SR, 2, 8>), grid, block, 0, st, a);
+    else if (W == 16)
+        hipLaunchKernelGGL((sbvr_mm_T_mfma_kernel<SR, 1, 16>), grid, block, 0, st, a);
+    else
+        hipLaunchKernelGGL((sbvr_mm_T_mfma_kernel<SR, 1, 8>), grid, block, 0, st, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+bool mm_T_mfma_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r_bvr, const void *r_cache)
+{
+    return K % kMmSub == 0 && G % kMmSub == 0 && Sl <= 16 && (Sr == 2 || Sr == 3 || Sr == 4 || Sr == 6 || Sr == 8) &&
+           static_cast<double>(M) * Sl * (K / 32) < 2147483648.0 && static_cast<double>(N) * Sr * (K / 32) < 2147483648.0 &&
+           reinterpret_cast<uintptr_t>(r_bvr) % 16 == 0 && reinterpret_cast<uintptr_t>(r_cache) % 16 == 0;
+}
+
+hipError_t launch_mm_T_mfma(int Sr, int G, MmArgs a, int cus, hipStream_t st)
+{
+    a.spg = G / kMmSub;
+    // The fewest row tiles that hold all (left row, plane) pairs, up to 4; fewer again while the workgroups leave a
+    // quarter of the CUs without one (every workgroup of a column block reads its plane words again, out of the L2).
+    // Sixteen waves where that gives a CU about one workgroup, eight where there are two and more.  us by (row tiles,
+    // waves), 4 right planes: 16 rows of 8 planes, 4096 x 4096: (4, 8) 9.7, (8, 8) 9.8, (4, 16) 11.7, (2, 16) 15.4;
+    // 64 rows of 8 planes, 14336 x 4096: (4, 8) 89.5, (8, 8) 110, (4, 16) 133; 32 rows of 8, 512 x 14336: (2, 16) 10.0,
+    // (1, 16) 12.2, (4, 16) 13.5; 4 rows of 4, 4096 x 4096: (1, 16) 4.9, (1, 8) 5.3, (1, 4) 6.8.
+    const int rows = a.M * a.Sl, cols = (a.N + 15) / 16;
+    int RT = rows <= 16 ? 1 : (rows <= 32 ? 2 : 4);
+    auto m_per_wg = [&](int rt) { return 16 * rt / a.Sl; };
+    auto wgs = [&](int rt) { return static_cast<long>(cols) * ((a.M + m_per_wg(rt) - 1) / m_per_wg(rt)); };
+    while (RT > 1 && m_per_wg(RT / 2) >= 1 && wgs(RT) * 4 < 3L * cus)
+        RT /= 2;
+    a.m_per_wg = m_per_wg(RT);
+    const int W = RT == 4 || wgs(RT) >= 2L * cus ? 8 : 16;
+    if ((a.M + a.m_per_wg - 1) / a.m_per_wg > 65535)
+        return hipErrorInvalidConfiguration;
+    switch (Sr) {
+    case 2: return launch_rt<2>(RT, W, a, st);
+    case 3: return launch_rt<3>(RT, W, a, st);
+    case 4: return launch_rt<4>(RT, W, a, st);
+    case 6: return launch_rt<6>(RT, W, a, st);
+    default: return launch_rt<8>(RT, W, a, st);
+    }
+}

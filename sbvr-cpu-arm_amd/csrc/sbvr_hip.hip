@@ -57,12 +57,10 @@
 
 #include "../../include/sbvr_hip.h"
 #include "../../include/sbvr_hip_decoder.h"
+#include "sbvr_internal.h"
+#include "sbvr_device.h"
 
 namespace {
-
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
 thread_local char g_err[256] = "";
 thread_local int g_last_kernel = 0;       // SBVR_HIP_KERNEL_* of the last linear launched from this thread
@@ -86,28 +84,6 @@ DevInfo g_dev[16];
 std::mutex g_dev_lock;           // guards g_dev[] and the scratch addresses: first use may come from several threads
 
 // ------------------------------------------------------------------ helpers
-
-__device__ __forceinline__ float h2f(uint16_t h)
-{
-    return static_cast<float>(__builtin_bit_cast(_Float16, h));
-}
-
-__device__ __forceinline__ uint16_t f2h(float f)
-{
-    return __builtin_bit_cast(uint16_t, static_cast<_Float16>(f));
-}
-
-// fp16 add of two fp16 values: exact sum rounded once (what __hadd does).
-__device__ __forceinline__ uint16_t hadd(uint16_t a, uint16_t b)
-{
-    return f2h(h2f(a) + h2f(b));
-}
-
-template <typename IdxT>
-__device__ __forceinline__ int load_idx(const void *p, size_t i)
-{
-    return static_cast<int>(static_cast<const IdxT *>(p)[i]);
-}
 
 // ---------------------------------------------------- portable kernel (any shape)
 
@@ -221,77 +197,6 @@ __device__ __forceinline__ int a_image_byte_offset(int k, int row)
     return lane * 32 + p;
 }
 
-template <int S>
-struct Planes {
-    uint32_t w[S];
-};
-
-typedef uint32_t v2u __attribute__((ext_vector_type(2)));
-typedef uint32_t v3raw __attribute__((ext_vector_type(3)));
-typedef v3raw v3u __attribute__((aligned(4)));          // (as it lies in a row of 3 or 6 plane words)
-
-// The S plane words of one (word of K, column) pair.  kStream: non-temporal loads, for kernels that
-// read every plane word once per launch and are bound by that stream (measured on the decode kernel:
-// 8.3 us instead of 8.8 us at the 4096 -> 14336 shape, 13.5 instead of 14.5 us at 4096 -> 28672; the
-// 32-row, row-dequant and popcount kernels, bound by their arithmetic, gain nothing from it).
-template <int S, bool kStream = false>
-__device__ __forceinline__ Planes<S> load_planes(const uint32_t *p)
-{
-    auto ld4 = [](const uint32_t *q) __attribute__((always_inline)) -> v4u {
-        return kStream ? __builtin_nontemporal_load(reinterpret_cast<const v4u *>(q)) : *reinterpret_cast<const v4u *>(q);
-    };
-    auto ld2 = [](const uint32_t *q) __attribute__((always_inline)) -> v2u {
-        return kStream ? __builtin_nontemporal_load(reinterpret_cast<const v2u *>(q)) : *reinterpret_cast<const v2u *>(q);
-    };
-    Planes<S> r;
-    if constexpr (S == 4) {
-        const v4u v = ld4(p);
-        r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
-    } else if constexpr (S == 2) {
-        const v2u v = ld2(p);
-        r.w[0] = v.x; r.w[1] = v.y;
-    } else if constexpr (S == 8) {
-        const v4u v0 = ld4(p), v1 = ld4(p + 4);
-        r.w[0] = v0.x; r.w[1] = v0.y; r.w[2] = v0.z; r.w[3] = v0.w;
-        r.w[4] = v1.x; r.w[5] = v1.y; r.w[6] = v1.z; r.w[7] = v1.w;
-    } else if constexpr (S == 3) {
-        // (12 bytes in one request: a global load wants dword alignment only)
-        const v3raw v = kStream ? __builtin_nontemporal_load(reinterpret_cast<const v3u *>(p)) : *reinterpret_cast<const v3u *>(p);
-        r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z;
-    } else if constexpr (S == 6) {
-        const v3raw v0 = kStream ? __builtin_nontemporal_load(reinterpret_cast<const v3u *>(p)) : *reinterpret_cast<const v3u *>(p);
-        const v3raw v1 = kStream ? __builtin_nontemporal_load(reinterpret_cast<const v3u *>(p + 3)) : *reinterpret_cast<const v3u *>(p + 3);
-        r.w[0] = v0.x; r.w[1] = v0.y; r.w[2] = v0.z; r.w[3] = v1.x; r.w[4] = v1.y; r.w[5] = v1.z;
-    } else {
-#pragma unroll
-        for (int j = 0; j < S; ++j)
-            r.w[j] = kStream ? __builtin_nontemporal_load(p + j) : p[j];
-    }
-    return r;
-}
-
-// The S fp16 coefficients of table line p as (S + 1) / 2 dwords, in as few loads as the line's alignment allows.
-template <int S>
-__device__ __forceinline__ void load_line_words(const uint16_t *p, uint32_t (&c)[(S + 1) / 2])
-{
-    constexpr int CW = (S + 1) / 2;
-    if constexpr (S == 4) {
-        const uint2 t = *reinterpret_cast<const uint2 *>(p);
-        c[0] = t.x; c[1] = t.y;
-    } else if constexpr (S == 8) {
-        const uint4 t = *reinterpret_cast<const uint4 *>(p);
-        c[0] = t.x; c[1] = t.y; c[2] = t.z; c[3] = t.w;
-    } else if constexpr (S % 2 == 0) {
-#pragma unroll
-        for (int j = 0; j < CW; ++j)
-            c[j] = reinterpret_cast<const uint32_t *>(p)[j];
-    } else {
-#pragma unroll
-        for (int j = 0; j < CW; ++j)
-            c[j] = static_cast<uint32_t>(p[2 * j]) | (2 * j + 1 < S ? static_cast<uint32_t>(p[2 * j + 1]) << 16 : 0u);
-    }
-}
-
 // Waves per SIMD the register allocator is asked to leave room for: the A operands and the activations
 // they are made from, the results, the MFMA outputs and plane sums of a unit, the plane words in flight
 // and working registers.
@@ -310,9 +215,6 @@ constexpr int gemv_max_waves(int MT, int CT)
     return MT == 4 ? 8 : kMaxWaves;
 }
 
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef short v2s __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ v2h as_v2h(uint32_t u) { return __builtin_bit_cast(v2h, u); }
 __device__ __forceinline__ int as_int(v2s b) { return __builtin_bit_cast(int, b); }
 
 // max over the 64 lanes of a non-negative integer; the result is wave-uniform
@@ -1539,9 +1441,6 @@ constexpr int kGemmBM = 256, kGemmBN = 128, kGemmBK = 64, kGemmThreads = 768;   
 constexpr int kGemmABufs = 3;       // activation tiles in LDS: the one in use and the next two
 constexpr int kGemmATile = kGemmBM * kGemmBK * 2, kGemmBTile = kGemmBN * kGemmBK * 2;
 
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 struct GemmArgs {
     const uint16_t *x;
@@ -2124,102 +2023,6 @@ constexpr int kLutWaves = 8;
 // 5..8 rows and 17.9-20.9 us at 9..16 rows for the decode kernels (13.6-16.0 with 2 planes, 19.6-22.5 with 3).
 constexpr int kLutMinRows = 9;
 
-// ---- decode by table look-up, shared by sbvr_gemm_rows32_lut_kernel and sbvr_gemm_lut_kernel (2, 3 or 4 planes)
-template <int S>
-struct LutTables {
-    static constexpr int TW = S == 4 ? 4 : (S == 3 ? 2 : 1);       // dwords of a byte table
-    uint32_t lo[TW], hi[TW];       // low and high bytes of the subset sums 0..3, 4..7, ...
-};
-
-// The 2^S subset sums of a coefficient line, entries (2i, 2i + 1) as packed pairs, then as byte tables.  Entry i is
-// the sum of the coefficients whose bit is set in i, added up in fp32 and rounded to fp16 once: the reference's
-// decode() takes a weight from bin_combs @ coeff (sbvr/core.py:345-366, 927-949), the exact sum rounded once.  The
-// fp32 sums are exact, and the entries therefore decode()'s weights bit for bit, whenever the exponents of a line's
-// coefficients lie within 11 of each other (every partial sum is then a multiple of the smallest coefficient's
-// last place below 2^24 of them); a line that mixes coefficients 2^12 apart and more can differ from decode() in
-// the last place of an entry that lands on a rounding tie.
-template <int S>
-__device__ __forceinline__ void lut_build_tables(const uint32_t (&c)[(S + 1) / 2], LutTables<S> &t)
-{
-    float cf[S];
-#pragma unroll
-    for (int q = 0; q < S; ++q)
-        cf[q] = h2f(static_cast<uint16_t>(q & 1 ? c[q / 2] >> 16 : c[q / 2] & 0xffffu));
-    float s[1 << S];
-    s[0] = 0.f;
-#pragma unroll
-    for (int q = 0; q < S; ++q)
-#pragma unroll
-        for (int i = 0; i < (1 << q); ++i)
-            s[(1 << q) + i] = i == 0 ? cf[q] : s[i] + cf[q];
-    v2h e[1 << (S - 1)];
-#pragma unroll
-    for (int i = 0; i < (1 << (S - 1)); ++i) {
-        e[i][0] = static_cast<_Float16>(s[2 * i]);         // (one v_cvt_pk_f16_f32 per pair, round to nearest even)
-        e[i][1] = static_cast<_Float16>(s[2 * i + 1]);
-    }
-#pragma unroll
-    for (int i = 0; i < LutTables<S>::TW; ++i) {
-        const uint32_t e0 = __builtin_bit_cast(uint32_t, e[2 * i]), e1 = __builtin_bit_cast(uint32_t, e[2 * i + 1]);
-        t.lo[i] = __builtin_amdgcn_perm(e1, e0, 0x06040200u);
-        t.hi[i] = __builtin_amdgcn_perm(e1, e0, 0x07050301u);
-    }
-}
-
-// Nibble words of one word of K: nibble n of Q[p] = selector (one bit per plane) of element p + 4n.
-template <int S>
-__device__ __forceinline__ void lut_nibble_words(const uint32_t (&w)[S], uint32_t (&Q)[4])
-{
-    auto rotr = [](uint32_t v, int r) __attribute__((always_inline)) -> uint32_t {
-        return (r & 31) == 0 ? v : __builtin_amdgcn_alignbit(v, v, r & 31);
-    };
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        uint32_t v = rotr(w[0], p) & 0x11111111u;
-        v = (rotr(w[1], p - 1) & 0x22222222u) | v;
-        if constexpr (S >= 3)
-            v = (rotr(w[2], p - 2) & 0x44444444u) | v;
-        if constexpr (S == 4)
-            v = (rotr(w[3], p - 3) & 0x88888888u) | v;
-        Q[p] = v;
-    }
-}
-
-// The weights of elements p, p + 8 (w01) and p + 16, p + 24 (w23) of the word, p = 0..7, as packed fp16 pairs.
-template <int S>
-__device__ __forceinline__ void lut_look_up(const LutTables<S> &t, const uint32_t (&Q)[4], int p, uint32_t &w01, uint32_t &w23)
-{
-    const uint32_t qs = p < 4 ? Q[p & 3] : Q[p & 3] >> 4;
-    const uint32_t sel = qs & (S == 2 ? 0x03030303u : 0x07070707u);
-    uint32_t lo, hi;
-    if constexpr (S == 2) {
-        lo = __builtin_amdgcn_perm(t.lo[0], t.lo[0], sel);
-        hi = __builtin_amdgcn_perm(t.hi[0], t.hi[0], sel);
-    } else {
-        lo = __builtin_amdgcn_perm(t.lo[1], t.lo[0], sel);
-        hi = __builtin_amdgcn_perm(t.hi[1], t.hi[0], sel);
-    }
-    if constexpr (S == 4) {
-        // bytes of ones where selector bit 3 is set: a look-up in the two-entry table {0x00, 0xff}
-        const uint32_t upper = __builtin_amdgcn_perm(0x0000ff00u, 0x0000ff00u, (qs >> 3) & 0x01010101u);
-        const uint32_t lo_u = __builtin_amdgcn_perm(t.lo[3], t.lo[2], sel), hi_u = __builtin_amdgcn_perm(t.hi[3], t.hi[2], sel);
-        lo = (lo_u & upper) | (lo & ~upper);
-        hi = (hi_u & upper) | (hi & ~upper);
-    }
-    w01 = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
-    w23 = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
-}
-
-// The B operand of MFMA q = 0..3 of the word: elements 2q, 2q+8, 2q+16, 2q+24, 2q+1, 2q+9, 2q+17, 2q+25.
-template <int S>
-__device__ __forceinline__ v4u lut_operand(const LutTables<S> &t, const uint32_t (&Q)[4], int q)
-{
-    uint32_t b0, b1, b2, b3;
-    lut_look_up<S>(t, Q, 2 * q, b0, b1);
-    lut_look_up<S>(t, Q, 2 * q + 1, b2, b3);
-    return v4u{b0, b1, b2, b3};
-}
-
 // kHalfRows: up to 16 batch rows (the activation loads of rows 16..31 are left out); kShare: groups of a multiple
 // of 128 elements, so the two steps of a loop iteration (an even word pair and the next) share a coefficient line:
 // one index load, one gather and one table per two steps.
@@ -2776,6 +2579,8 @@ int current_cus()
 }
 
 // -------------------------------------------- trans=True and both-encoded forms
+
+constexpr int kMmDecodeMinN = 8192;      // columns from which one encoded left row takes the decode kernel (sbvr_hip_mm_T_ws)
 
 // One thread per output; the lanes of a wave share k and differ in n, so the
 // plane words and indices are wave-uniform broadcasts.
@@ -4390,10 +4195,10 @@ size_t sbvr_hip_row_deq_mm_T_workspace(int M, int N)
     return col_wgs * 2 < 3L * current_cus() / 4 ? static_cast<size_t>(M) * N * sizeof(unsigned long long) : 0;
 }
 
-// (only one left row runs on the decode kernel, the one form that may split K across workgroups)
+// (one left row against many columns runs on the decode kernel, the one form that may split K across workgroups)
 size_t sbvr_hip_mm_T_workspace(int M, int N)
 {
-    return M == 1 && N > 0 ? static_cast<size_t>(N) * sizeof(unsigned long long) : 0;
+    return M == 1 && N >= kMmDecodeMinN ? static_cast<size_t>(N) * sizeof(unsigned long long) : 0;
 }
 
 int sbvr_hip_mm_T(const uint32_t *l_bvr, const void *l_coeff_idx, int l_idx_bytes,
@@ -4426,10 +4231,10 @@ int sbvr_hip_mm_T_ws(const uint32_t *l_bvr, const void *l_coeff_idx, int l_idx_b
     const uint16_t *lc = static_cast<const uint16_t *>(l_coeff_cache), *rc = static_cast<const uint16_t *>(r_coeff_cache);
     const uint16_t *b = static_cast<const uint16_t *>(bias);
     uint16_t *o = static_cast<uint16_t *>(out);
-    // One left row of up to four planes (what the reference's kernels are written for), at the decode kernel's
-    // shapes: the decode kernel with the left operand's planes as its batch rows; the popcounts come out of the
-    // matrix cores.  4096 -> 14336, 4 x 4 planes: about 9 us against 11.5 us for the popcount kernel below.
-    if (M == 1 && Sl <= 4 && !env_switches().popc_q && mfma_path_ok(Sl, N, K, Sr, G) &&
+    // One left row of up to four planes against many columns, at the decode kernel's shapes: the decode kernel with
+    // the left operand's planes as its batch rows.  (us, 4 x 4 planes, this kernel against mm_ops.hip's, which takes
+    // the rest: 4096 -> 14336 8.9 and 9.6; 14336 -> 4096 9.7 and 9.1; 4096 -> 4096 7.0 and 5.0; 4096 -> 1024 4.5 and 4.4.)
+    if (M == 1 && N >= kMmDecodeMinN && Sl <= 4 && !env_switches().popc_q && mfma_path_ok(Sl, N, K, Sr, G) &&
         (l_idx_bytes == 2 || Ll <= 256) && (r_idx_bytes == 2 || Lr <= 256) &&
         reinterpret_cast<uintptr_t>(r_bvr) % 16 == 0 && reinterpret_cast<uintptr_t>(r_coeff_cache) % 16 == 0 &&
         reinterpret_cast<uintptr_t>(l_bvr) % 4 == 0 && reinterpret_cast<uintptr_t>(l_coeff_cache) % 2 == 0) {
@@ -4465,6 +4270,25 @@ int sbvr_hip_mm_T_ws(const uint32_t *l_bvr, const void *l_coeff_idx, int l_idx_b
             g_last_kernel = SBVR_HIP_KERNEL_DECODE;
             return SBVR_HIP_OK;
         }
+    }
+    // any number of left rows: popcounts on the matrix cores
+    if (mm_T_mfma_ok(M, N, K, Sl, Sr, G, r_bvr, r_coeff_cache)) {
+        MmArgs a{};
+        a.l_bvr = l_bvr;
+        a.l_idx = l_coeff_idx;
+        a.l_cache = lc;
+        a.r_bvr = r_bvr;
+        a.r_idx = r_coeff_idx;
+        a.r_cache = rc;
+        a.bias = b;
+        a.out = o;
+        a.M = M; a.N = N; a.K = K; a.Sl = Sl; a.Ll = Ll; a.Lr = Lr;
+        a.l_idx16 = l_idx_bytes == 2;
+        a.r_idx16 = r_idx_bytes == 2;
+        const hipError_t e = launch_mm_T_mfma(Sr, G, a, current_cus(), st);
+        if (e != hipSuccess)
+            return fail(SBVR_HIP_ELAUNCH, "mm_T launch: %s", hipGetErrorString(e));
+        return SBVR_HIP_OK;
     }
     // few left rows: lane-per-column popcount kernel
     const int wpg = G / 32;

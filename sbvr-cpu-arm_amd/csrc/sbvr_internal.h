@@ -1,0 +1,27 @@
+// What the translation units of libsbvr_hip.so call of each other (host side).
+#ifndef SBVR_INTERNAL_H
+#define SBVR_INTERNAL_H
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+// The product of two encoded operands on the matrix cores (mm_ops.hip).
+struct MmArgs {
+    const uint32_t *l_bvr;       // (K / 32, M, Sl)
+    const void *l_idx;           // (K / G, M)
+    const uint16_t *l_cache;     // (Ll, Sl)
+    const uint32_t *r_bvr;       // (K / 32, N, Sr)
+    const void *r_idx;
+    const uint16_t *r_cache;
+    const uint16_t *bias;
+    uint16_t *out;
+    int M, N, K, Sl, Ll, Lr;
+    int spg;                     // sub-groups of 128 elements per coefficient group
+    int l_idx16, r_idx16;
+    int m_per_wg;                // left rows of a workgroup
+};
+// Whether that kernel covers the shape (pointers: r_bvr and r_cache 16-byte aligned).
+bool mm_T_mfma_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r_bvr, const void *r_cache);
+hipError_t launch_mm_T_mfma(int Sr, int G, MmArgs a, int cus, hipStream_t st);
+
+#endif

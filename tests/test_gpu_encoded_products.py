@@ -1,0 +1,40 @@
+"""The matrix-core product of two encoded operands against the CPU oracle at the sizes where its tiling has edges."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _enc(rng, rows, K, S, G, L, oracle, scale=0.5):
+    sel = rng.integers(0, 1 << S, size=rows * K).astype(np.int32)
+    bvr = oracle.C.planes_to_default(oracle.C.sel_to_planes(sel, S, 32), rows, K)
+    idx = rng.integers(0, L, size=(K // G, rows)).astype(np.uint8 if L <= 256 else np.uint16)
+    return bvr, idx, (rng.standard_normal((L, S)) * scale).astype(np.float16)
+
+
+def _dev(*arrays):
+    return [torch.from_numpy(a).to("cuda:0") for a in arrays]
+
+
+# (left row, plane) pairs on both sides of the 16-pair tiles and of the 128-pair workgroups; ragged N; one sub-group
+# of K, fewer sub-groups than waves, several per wave; groups of one and of three sub-groups
+@pytest.mark.parametrize("M,N,K,Sl,Sr,G,Ll,Lr", [
+    (2, 1, 128, 8, 4, 128, 3, 9), (15, 17, 384, 1, 2, 384, 300, 7), (3, 100, 1024, 5, 3, 128, 9, 300),
+    (4, 4100, 4096, 4, 4, 256, 16, 256), (5, 33, 2304, 7, 6, 128, 5, 70), (11, 250, 512, 6, 8, 256, 4, 5),
+    (16, 520, 4352, 8, 4, 128, 40, 256), (17, 130, 2176, 8, 3, 128, 300, 16), (33, 64, 256, 4, 8, 128, 8, 8),
+    (64, 1030, 1280, 8, 2, 128, 16, 700), (1, 300, 7168, 8, 4, 256, 28, 256), (1, 40, 256, 16, 4, 128, 2, 3)])
+def test_mm_T_any_rows(oracle, M, N, K, Sl, Sr, G, Ll, Lr):
+    import sbvr
+    rng = np.random.default_rng(M * 1000 + N)
+    left, right = _enc(rng, M, K, Sl, G, Ll, oracle), _enc(rng, N, K, Sr, G, Lr, oracle)
+    bias = rng.standard_normal(N).astype(np.float16)
+    none = torch.zeros(0, dtype=torch.float16, device="cuda:0")
+    y = sbvr._sbvr_mm_T(*_dev(*left, *right), none, bvr_len=G).cpu().numpy()
+    _, yd = oracle.C.mm_T(*left, *right, G)
+    # exact popcounts and fp32 sums of K / 128 * Sl * Sr terms, then one rounding to fp16: within 2 fp16 ulps
+    rms = float(np.sqrt(np.mean(yd ** 2)))
+    assert (np.abs(y.astype(np.float64) - yd) / (np.maximum(np.abs(yd), rms) * 2.0 ** -10)).max() <= 2.0
+    # the bias is added to the rounded sum
+    yb = sbvr._sbvr_mm_T(*_dev(*left, *right, bias), bvr_len=G).cpu().numpy()
+    assert np.array_equal(yb, (y.astype(np.float32) + bias.astype(np.float32)).astype(np.float16))
