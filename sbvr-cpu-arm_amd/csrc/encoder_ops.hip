@@ -10,14 +10,10 @@
 // memory.  The arithmetic per element is the reference's: fp16 subtraction, fp16 square, minimum (packed,
 // two points per instruction), then an fp32 sum over the group in element order and one division.
 
-#include <hip/hip_runtime.h>
-#include <stdint.h>
-
 #include "../../include/sbvr_hip_encoder.h"
+#include "sbvr_device.h"
 
 namespace {
-
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 
 constexpr int kEncThreads = 256;
 constexpr int kEncMaxG = 4096;        // values of a group the LDS copy holds at a time (8 KiB)
@@ -103,6 +99,147 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
     }
 }
 
+// ------------------------------------------------------------------------------------ the dense weight again
+//
+// decode(): out[n, k] = the subset sum that the planes of (n, k) select from the line of n's group, the fp32 sum
+// rounded to fp16 once (reference sbvr/core.py:926-949), then converted to the tensor's own type (OUT: fp16, bf16
+// or fp32).  A wave takes 8 columns x 8 words of K: lane (n = lane % 8, word = lane / 8) loads its plane words (eight
+// neighbouring columns of a word are one or two cache lines) and decodes 32 weights in registers, by table look-up
+// for 2, 3 and 4 planes (S), otherwise plane by plane in fp32 (S = 0: any number of planes).  Eight words of a row are 512
+// bytes of output; the 64-byte pieces of the lanes go through 4 KiB of LDS to lanes that follow each other along a
+// row, so that a store instruction writes two runs of 512 bytes.  Bound by memory: 2 bytes out per weight against S / 8
+// in.  4096 -> 14336, 4 planes: 31 us = 4.7 TB/s, where a
+// large copy reaches 5.2 (the torch expression over unpacked 64-bit selectors took 4.4 ms); 6 planes 51 us, 8 planes 69 us.
+struct DecodeArgs {
+    const uint32_t *bvr;
+    const uint8_t *idx;
+    const uint16_t *cache;
+    void *out;
+    int N, words, S, wpg, L, idx16;
+    int k_out;                   // columns of the output: K without the padding
+    int wide;                    // rows of the output are 16-byte aligned
+};
+
+constexpr int kDecWaves = 4;
+enum { kOutF16 = 0, kOutBf16 = 1, kOutF32 = 2 };
+
+__device__ __forceinline__ uint32_t bf16_pair(uint32_t two)
+{
+    auto one = [](uint16_t h) __attribute__((always_inline)) -> uint32_t {
+        const uint32_t u = __float_as_uint(h2f(h));
+        return (u & 0x7fffffffu) > 0x7f800000u ? 0x7fc0u : (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+    };
+    return one(static_cast<uint16_t>(two & 0xffffu)) | (one(static_cast<uint16_t>(two >> 16)) << 16);
+}
+
+template <int S, int OUT>
+__global__ void __launch_bounds__(64 * kDecWaves)
+sbvr_decode_weight_kernel(const DecodeArgs a)
+{
+    __shared__ v4u tiles[kDecWaves][256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int w0 = (blockIdx.y * kDecWaves + wave) * 8, n0 = blockIdx.x * 8;
+    if (w0 >= a.words)                                        // wave-uniform; no barrier below
+        return;
+    v4u *const tile = tiles[wave];
+    const int ln = lane & 7, lw = lane >> 3;
+    const int n = min(n0 + ln, a.N - 1), word = min(w0 + lw, a.words - 1);
+    const size_t at = (static_cast<size_t>(word / a.wpg) * a.N + n) << a.idx16;
+    const int lo = a.idx[at], hi = a.idx[at + a.idx16];
+    const int line = min(a.idx16 ? lo | (hi << 8) : lo, a.L - 1);
+    uint32_t D[16];                                           // elements 2i, 2i + 1 of the word
+    if constexpr (S != 0) {
+        const Planes<S> pl = load_planes<S>(a.bvr + (static_cast<size_t>(word) * a.N + n) * S);
+        uint32_t c[(S + 1) / 2];
+        load_line_words<S>(a.cache + static_cast<size_t>(line) * S, c);
+        LutTables<S> t;
+        lut_build_tables<S>(c, t);
+        uint32_t Q[4];
+        lut_nibble_words<S>(pl.w, Q);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            uint32_t e01, e23, o01, o23;                      // elements p, p + 8 and p + 16, p + 24
+            lut_look_up<S>(t, Q, 2 * q, e01, e23);
+            lut_look_up<S>(t, Q, 2 * q + 1, o01, o23);
+            D[q] = __builtin_amdgcn_perm(o01, e01, 0x05040100u);
+            D[4 + q] = __builtin_amdgcn_perm(o01, e01, 0x07060302u);
+            D[8 + q] = __builtin_amdgcn_perm(o23, e23, 0x05040100u);
+            D[12 + q] = __builtin_amdgcn_perm(o23, e23, 0x07060302u);
+        }
+    } else {
+        float w[32];
+#pragma unroll
+        for (int i = 0; i < 32; ++i)
+            w[i] = 0.f;
+        const uint32_t *src = a.bvr + (static_cast<size_t>(word) * a.N + n) * a.S;
+        const uint16_t *cs = a.cache + static_cast<size_t>(line) * a.S;
+        for (int j = 0; j < a.S; ++j) {
+            const int bits = static_cast<int>(src[j]);
+            const uint32_t c = __float_as_uint(h2f(cs[j]));
+#pragma unroll
+            for (int i = 0; i < 32; ++i)
+                w[i] += __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_sbfe(bits, i, 1)) & c);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            D[i] = static_cast<uint32_t>(f2h(w[2 * i])) | (static_cast<uint32_t>(f2h(w[2 * i + 1])) << 16);
+    }
+    // 16-byte piece c of word w of row n lies at place (w ^ n) * 4 + c of the row's 32: eight lanes that store the same
+    // word of eight rows, and the lanes that read a row, meet different banks
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        tile[ln * 32 + ((lw ^ ln) << 2) + c] = v4u{D[4 * c], D[4 * c + 1], D[4 * c + 2], D[4 * c + 3]};
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const int row = 2 * s + (lane >> 5), q = lane & 31;
+        v4u v = tile[row * 32 + (((q >> 2) ^ row) << 2) + (q & 3)];
+        if constexpr (OUT == kOutBf16) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                v[i] = bf16_pair(v[i]);
+        }
+        const int k = w0 * 32 + 8 * q, nn = n0 + row;
+        if (nn >= a.N || k >= a.k_out)
+            continue;
+        const size_t o = static_cast<size_t>(nn) * a.k_out + k;
+        if (a.wide && k + 8 <= a.k_out) {
+            if constexpr (OUT == kOutF32) {
+                float *dst = static_cast<float *>(a.out) + o;
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    *reinterpret_cast<v4f *>(dst + 4 * i) =
+                        v4f{h2f(static_cast<uint16_t>(v[2 * i])), h2f(static_cast<uint16_t>(v[2 * i] >> 16)),
+                            h2f(static_cast<uint16_t>(v[2 * i + 1])), h2f(static_cast<uint16_t>(v[2 * i + 1] >> 16))};
+            } else {
+                *reinterpret_cast<v4u *>(static_cast<uint16_t *>(a.out) + o) = v;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (k + i < a.k_out) {
+                    const uint16_t h = static_cast<uint16_t>(v[i / 2] >> (16 * (i & 1)));
+                    if constexpr (OUT == kOutF32)
+                        static_cast<float *>(a.out)[o + i] = h2f(h);
+                    else
+                        static_cast<uint16_t *>(a.out)[o + i] = h;
+                }
+        }
+    }
+}
+
+template <int S>
+void launch_decode(int out_type, dim3 grid, hipStream_t st, const DecodeArgs &a)
+{
+    const dim3 block(64 * kDecWaves);
+    if (out_type == kOutF16)
+        hipLaunchKernelGGL((sbvr_decode_weight_kernel<S, kOutF16>), grid, block, 0, st, a);
+    else if (out_type == kOutBf16)
+        hipLaunchKernelGGL((sbvr_decode_weight_kernel<S, kOutBf16>), grid, block, 0, st, a);
+    else
+        hipLaunchKernelGGL((sbvr_decode_weight_kernel<S, kOutF32>), grid, block, 0, st, a);
+}
+
 }  // namespace
 
 extern "C" {
@@ -141,6 +278,33 @@ int sbvr_hip_online_encode_f16(const void *x, const void *points, uint32_t *bvr,
     const dim3 grid(static_cast<unsigned>((K + 63) / 64), static_cast<unsigned>(M)), block(64);
     hipLaunchKernelGGL(sbvr_online_encode_kernel, grid, block, 0, static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(x),
                        static_cast<const uint16_t *>(points), bvr, M, K, G, S);
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+int sbvr_hip_decode_weight(const uint32_t *bvr, const void *idx, int idx_bytes, const void *cache, void *out, int out_type, int N, int K,
+                           int k_out, int S, int G, int L, void *stream)
+{
+    if (!bvr || !idx || !cache || !out || N <= 0 || K <= 0 || S <= 0 || G <= 0 || L <= 0 || k_out <= 0 || k_out > K ||
+        (idx_bytes != 1 && idx_bytes != 2) || out_type < kOutF16 || out_type > kOutF32)
+        return -1;
+    const int words = K / 32;
+    const long gy = (static_cast<long>(words) + 8 * kDecWaves - 1) / (8 * kDecWaves);
+    if (G % 32 != 0 || K % G != 0 || gy > 65535)
+        return -2;
+    const size_t row_bytes = static_cast<size_t>(k_out) * (out_type == kOutF32 ? 4 : 2);
+    DecodeArgs a{bvr, static_cast<const uint8_t *>(idx), static_cast<const uint16_t *>(cache), out, N, words, S, G / 32, L,
+                 idx_bytes == 2 ? 1 : 0, k_out, row_bytes % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 ? 1 : 0};
+    const dim3 grid(static_cast<unsigned>((N + 7) / 8), static_cast<unsigned>(gy));
+    const bool aligned = reinterpret_cast<uintptr_t>(bvr) % 16 == 0 && reinterpret_cast<uintptr_t>(cache) % 16 == 0;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (aligned && S == 4)
+        launch_decode<4>(out_type, grid, st, a);
+    else if (aligned && S == 3)
+        launch_decode<3>(out_type, grid, st, a);
+    else if (aligned && S == 2)
+        launch_decode<2>(out_type, grid, st, a);
+    else
+        launch_decode<0>(out_type, grid, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

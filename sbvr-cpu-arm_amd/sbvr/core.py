@@ -280,6 +280,11 @@ class sbvr(torch.nn.Module):
         """The dense tensor this object stands for, in ``original_dtype``: every
         element is one of its group's 2^S points ``bin_combs @ line``
         (core.py:926-949)."""
+        if self.bvr.is_cuda and self.bvr.dtype == torch.uint32 and self.bvr.dim() == 3 and self.bvr.is_contiguous():
+            from . import hip
+            out = hip.decode_weight(self.bvr.data, self.coeff_idx.data, self.coeff_cache.data, self.bvr_len,
+                                    self.original_data_shape[-1], self.original_dtype)
+            return out.view(self.original_data_shape)
         sel = layout.default_to_sel(self.default_layout()).to(torch.int64)          # (rows, Kp)
         rows, kp = sel.shape
         points = (self._get_bin_combs().float() @ self.coeff_cache.data.float().T).T   # (lines, 2^S)

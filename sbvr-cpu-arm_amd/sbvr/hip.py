@@ -79,6 +79,7 @@ def _load():
                                                        vp, vp, vp, vp, vp]
     lib.sbvr_hip_encoder_group_mse_f16.argtypes = [vp, vp, vp, i, i, i, i, vp]
     lib.sbvr_hip_online_encode_f16.argtypes = [vp, vp, vp, i, i, i, i, vp]
+    lib.sbvr_hip_decode_weight.argtypes = [vp, vp, i, vp, vp, i, i, i, i, i, i, i, vp]
     _lib = lib
     return lib
 
@@ -576,3 +577,27 @@ def online_encode(x, points, bvr_len):
     if rc != 0:
         raise SbvrHipError(f"sbvr_hip_online_encode_f16: error {rc} (M={M} K={K} bvr_len={bvr_len} S={S})")
     return bvr
+
+
+_DECODE_TYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
+
+
+def decode_weight(bvr, coeff_idx, coeff_cache, bvr_len, cols, dtype):
+    """The dense (N, cols) weight of a default-layout encoding (cols: without the padding of K), every element its
+    coefficients' fp32 sum rounded to fp16 once, in ``dtype`` (sbvr/core.py:926-949)."""
+    dev = bvr.device
+    _want(bvr, "bvr", torch.uint32, 3)
+    _want(coeff_idx, "coeff_idx", (torch.uint8, torch.uint16), 2, dev)
+    _want(coeff_cache, "coeff_cache", torch.float16, 2, dev)
+    Kw, N, S = bvr.shape
+    L = coeff_cache.shape[0]
+    if coeff_idx.shape != (Kw * 32 // bvr_len, N) or coeff_cache.shape[1] != S:
+        raise ValueError("coeff_idx / coeff_cache shapes do not match bvr")
+    out = torch.empty((N, cols), dtype=dtype if dtype in _DECODE_TYPES else torch.float16, device=dev)
+    with torch.cuda.device(dev):
+        rc = _load().sbvr_hip_decode_weight(bvr.data_ptr(), coeff_idx.data_ptr(), coeff_idx.element_size(),
+                                            coeff_cache.data_ptr(), out.data_ptr(), _DECODE_TYPES[out.dtype], N, Kw * 32,
+                                            cols, S, bvr_len, L, _stream())
+    if rc != 0:
+        raise SbvrHipError(f"sbvr_hip_decode_weight: error {rc} (N={N} K={Kw * 32} cols={cols} S={S} bvr_len={bvr_len} L={L})")
+    return out.to(dtype)

@@ -1,4 +1,5 @@
-"""The matrix-core product of two encoded operands against the CPU oracle at the sizes where its tiling has edges."""
+"""The matrix-core product of two encoded operands, and the dense weight back from an encoding, against the CPU
+oracle at the sizes where their tilings have edges."""
 import numpy as np
 import pytest
 import torch
@@ -38,3 +39,20 @@ def test_mm_T_any_rows(oracle, M, N, K, Sl, Sr, G, Ll, Lr):
     # the bias is added to the rounded sum
     yb = sbvr._sbvr_mm_T(*_dev(*left, *right, bias), bvr_len=G).cpu().numpy()
     assert np.array_equal(yb, (y.astype(np.float32) + bias.astype(np.float32)).astype(np.float16))
+
+
+@pytest.mark.parametrize("N,K,S,G,L,cols,dtype", [
+    (1, 32, 4, 32, 1, 32, torch.float16), (9, 288, 4, 96, 300, 288, torch.bfloat16), (7, 256, 3, 64, 5, 250, torch.float16),
+    (65, 1280, 2, 256, 256, 1280, torch.float32), (130, 512, 3, 128, 700, 505, torch.float32), (40, 544, 6, 32, 17, 544, torch.float16),
+    (24, 256, 8, 128, 256, 248, torch.bfloat16), (8, 256, 1, 256, 4, 256, torch.float16), (16, 2048, 4, 128, 256, 2048, torch.float64),
+    (33, 64, 5, 64, 9, 64, torch.float16)])
+def test_decode_weight(oracle, N, K, S, G, L, cols, dtype):
+    import sbvr
+    rng = np.random.default_rng(N * 100 + K)
+    bvr, idx, cache = _enc(rng, N, K, S, G, L, oracle, 0.02)
+    # coefficients that are multiples of 2^-14 below 2^-3: every fp32 sum is exact, whatever its order
+    cache = (np.round(cache.astype(np.float64) * 2 ** 14) / 2 ** 14).astype(np.float16)
+    obj = sbvr.sbvr.from_parts(*_dev(bvr, idx, cache), G, original_shape=(N, cols), original_dtype=dtype)
+    got = obj.decode()
+    want = torch.from_numpy(oracle.C.decode(bvr, idx, cache, G)[:, :cols].astype(np.float16)).to(dtype)
+    assert got.shape == (N, cols) and got.dtype == dtype and torch.equal(got.cpu(), want)
