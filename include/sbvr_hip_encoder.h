@@ -31,6 +31,13 @@ int sbvr_hip_encoder_group_mse_f16(const void *data, const void *points, float *
  * None there) are placeholders for.  G a multiple of 32, K of G, S <= 8, M <= 65535. */
 int sbvr_hip_online_encode_f16(const void *x, const void *points, uint32_t *bvr, int M, int K, int G, int S, void *stream);
 
+/* The same encoding from the input coefficients themselves: lines (K/G, S) fp16, one line per group of K; the
+ * subset sums are worked out in the launch (fp32 sum in the order of the coefficients, rounded to fp16 once).  Also
+ * writes the line indices of the left operand, idx (K/G, M): idx[g, m] = g, uint8 (idx_bytes 1, K/G <= 256)
+ * or uint16 (idx_bytes 2). */
+int sbvr_hip_online_encode_lines_f16(const void *x, const void *lines, uint32_t *bvr, void *idx, int idx_bytes, int M, int K,
+                                     int G, int S, void *stream);
+
 /* The dense weight of an encoded one (sbvr/core.py:926-949, decode()): out (N, k_out), out[n, k] = the sum of the
  * coefficients cache[idx[k / G, n], j] whose plane j is set at (n, k), added up in fp32, rounded to fp16 once and
  * converted to out_type (0 fp16, 1 bf16, 2 fp32).  bvr (K/32, N, S) uint32, idx (K/G, N) uint8 or uint16 (idx_bytes),

@@ -67,35 +67,81 @@ sbvr_encoder_group_mse_kernel(const uint16_t *__restrict__ data, const uint16_t 
 // selectors: sbvr/core.py:492-494), and the 64 lanes' selector bits become two words per plane by ballot
 // (a selector counts the subset sums most significant coefficient first: plane j is its bit S - 1 - j,
 // core.py:345-351 and :842-876).
-// Grid: (ceil(K / 64), M), one wave per workgroup.
-__global__ void __launch_bounds__(64)
-sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ points, uint32_t *__restrict__ bvr,
-                          int M, int K, int G, int S)
+// A workgroup takes 64 elements of K (two words) of kOnlineRows rows, one row a wave at a time, and keeps the subset
+// sums of the (at most two) groups they lie in in LDS, where the waves read them four pairs at a time: built from
+// the group's coefficients (kLines: each the fp32 sum in the order of the planes, rounded to fp16 once), or copied
+// from a table of them.  The search is the vector ALU's: per two points a packed difference and square, then each
+// square's bits above its point's number as one key (squares are not negative: their bits order as they do) and a
+// three-way minimum, 2.5 operations a point.  (16 rows x 4096, 256 points: the lane that fetched every point from
+// memory for itself took 20.5 us.)
+constexpr int kOnlineWaves = 4, kOnlineRows = 4;
+
+template <bool kLines>
+__global__ void __launch_bounds__(64 * kOnlineWaves)
+sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ table, uint32_t *__restrict__ bvr,
+                          uint8_t *__restrict__ idx, int idx16, int M, int K, int G, int S)
 {
-    const int lane = threadIdx.x;
-    const int m = blockIdx.y;
-    const int k = blockIdx.x * 64 + lane;
-    const int P = 1 << S;
-    int sel = 0;
-    if (k < K) {
+    __shared__ __align__(16) uint16_t pts[2][256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int P = 1 << S, padded = max(P, 8);
+    const int k0 = blockIdx.x * 64;
+    const int words = K / 32;
+    const int groups = K / G, g0 = k0 / G, g1 = min((k0 + 32) / G, groups - 1);     // (G is a multiple of 32)
+    for (int i = threadIdx.x; i < 2 * padded; i += 64 * kOnlineWaves) {
+        const int which = i >= padded, p = min(which ? i - padded : i, P - 1);       // (the last point again behind the end)
+        const int g = which ? g1 : g0;
+        uint16_t v;
+        if constexpr (kLines) {
+            float sum = 0.f;
+            for (int j = 0; j < S; ++j) {
+                const float c = static_cast<float>(__builtin_bit_cast(_Float16, table[static_cast<size_t>(g) * S + j]));
+                sum += (p >> (S - 1 - j)) & 1 ? c : 0.f;
+            }
+            v = __builtin_bit_cast(uint16_t, static_cast<_Float16>(sum));
+        } else {
+            v = table[static_cast<size_t>(g) * P + p];
+        }
+        pts[which][which ? i - padded : i] = v;
+    }
+    __syncthreads();
+    const int k = min(k0 + lane, K - 1);
+    const uint4 *const mine = reinterpret_cast<const uint4 *>(pts[lane >> 5 & (g1 != g0)]);
+    for (int r = wave; r < kOnlineRows; r += kOnlineWaves) {
+        const int m = blockIdx.y * kOnlineRows + r;
+        if (m >= M)                                                                   // wave-uniform
+            break;
         const _Float16 d = __builtin_bit_cast(_Float16, x[static_cast<size_t>(m) * K + k]);
-        const uint16_t *pts = points + static_cast<size_t>(k / G) * P;
-        _Float16 best = static_cast<_Float16>(0.f);
-        for (int p = 0; p < P; ++p) {
-            const _Float16 diff = d - __builtin_bit_cast(_Float16, pts[p]);
-            const _Float16 sq = diff * diff;
-            if (p == 0 || sq < best) {
-                best = sq;
-                sel = p;
+        const v2h dd = {d, d};
+        uint32_t best = 0xffffffffu;
+#pragma unroll 4
+        for (int c = 0; c < padded / 8; ++c) {
+            const uint4 q = mine[c];
+            const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const v2h diff = dd - __builtin_bit_cast(v2h, w[i]);
+                const uint32_t sq = __builtin_bit_cast(uint32_t, diff * diff);
+                const uint32_t p = static_cast<uint32_t>(8 * c + 2 * i);
+                best = min(min(best, (sq << 16) | p), (sq & 0xffff0000u) | (p + 1));
             }
         }
-    }
-    const int words = K / 32;
-    for (int j = 0; j < S; ++j) {
-        const unsigned long long bits = __builtin_amdgcn_ballot_w64(((sel >> (S - 1 - j)) & 1) != 0);   // plane 0: the top bit
+        const uint32_t sel = best & 0xffffu;
+        uint32_t out = 0;
+        for (int j = 0; j < S; ++j) {                                                 // plane 0: the selector's top bit
+            const unsigned long long bits = __builtin_amdgcn_ballot_w64(((sel >> (S - 1 - j)) & 1) != 0);
+            out = (lane & 31) == j ? static_cast<uint32_t>(lane < 32 ? bits : bits >> 32) : out;
+        }
         const int kw = blockIdx.x * 2 + (lane >> 5);
-        if ((lane & 31) == 0 && kw < words)
-            bvr[(static_cast<size_t>(kw) * M + m) * S + j] = static_cast<uint32_t>(lane == 0 ? bits : bits >> 32);
+        if ((lane & 31) < S && kw < words)
+            bvr[(static_cast<size_t>(kw) * M + m) * S + (lane & 31)] = out;
+        // the left operand's line index of a group is the group's number
+        if (idx && (lane & 31) == 31 && kw < words && kw * 32 % G == 0) {
+            const int g = kw * 32 / G;
+            if (idx16)
+                reinterpret_cast<uint16_t *>(idx)[static_cast<size_t>(g) * M + m] = static_cast<uint16_t>(g);
+            else
+                idx[static_cast<size_t>(g) * M + m] = static_cast<uint8_t>(g);
+        }
     }
 }
 
@@ -275,9 +321,22 @@ int sbvr_hip_online_encode_f16(const void *x, const void *points, uint32_t *bvr,
         return -1;
     if (S > 8 || G % 32 != 0 || K % G != 0 || M > 65535)
         return -2;
-    const dim3 grid(static_cast<unsigned>((K + 63) / 64), static_cast<unsigned>(M)), block(64);
-    hipLaunchKernelGGL(sbvr_online_encode_kernel, grid, block, 0, static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(x),
-                       static_cast<const uint16_t *>(points), bvr, M, K, G, S);
+    const dim3 grid(static_cast<unsigned>((K + 63) / 64), static_cast<unsigned>((M + kOnlineRows - 1) / kOnlineRows)), block(64 * kOnlineWaves);
+    hipLaunchKernelGGL(sbvr_online_encode_kernel<false>, grid, block, 0, static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(x),
+                       static_cast<const uint16_t *>(points), bvr, nullptr, 0, M, K, G, S);
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+int sbvr_hip_online_encode_lines_f16(const void *x, const void *lines, uint32_t *bvr, void *idx, int idx_bytes, int M, int K, int G,
+                                     int S, void *stream)
+{
+    if (!x || !lines || !bvr || !idx || M <= 0 || K <= 0 || G <= 0 || S <= 0 || (idx_bytes != 1 && idx_bytes != 2))
+        return -1;
+    if (S > 8 || G % 32 != 0 || K % G != 0 || M > 65535 || (idx_bytes == 1 && K / G > 256) || K / G > 65536)
+        return -2;
+    const dim3 grid(static_cast<unsigned>((K + 63) / 64), static_cast<unsigned>((M + kOnlineRows - 1) / kOnlineRows)), block(64 * kOnlineWaves);
+    hipLaunchKernelGGL(sbvr_online_encode_kernel<true>, grid, block, 0, static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(x),
+                       static_cast<const uint16_t *>(lines), bvr, static_cast<uint8_t *>(idx), idx_bytes == 2 ? 1 : 0, M, K, G, S);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

@@ -370,11 +370,7 @@ class sbvr(torch.nn.Module):
         if x.shape[1] != k_pad:
             x = torch.nn.functional.pad(x, (0, k_pad - x.shape[1]))
         coeff = self.input_coeff.data
-        points = coeff @ layout.bin_combs(coeff.shape[1], self.compute_dtype, coeff.device).T
-        bvr = hip.online_encode(x.contiguous(), points.contiguous(), self.bvr_len)
-        groups = coeff.shape[0]
-        idx = torch.arange(groups, device=coeff.device).view(-1, 1).expand(groups, x.shape[0])
-        idx = idx.to(torch.uint8 if groups <= 256 else torch.uint16).contiguous()
+        bvr, idx = hip.online_encode_lines(x.contiguous(), coeff, self.bvr_len)
         return bvr, idx, coeff
 
     _online_transform = _online_tranfrom

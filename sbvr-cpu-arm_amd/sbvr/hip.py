@@ -79,6 +79,7 @@ def _load():
                                                        vp, vp, vp, vp, vp]
     lib.sbvr_hip_encoder_group_mse_f16.argtypes = [vp, vp, vp, i, i, i, i, vp]
     lib.sbvr_hip_online_encode_f16.argtypes = [vp, vp, vp, i, i, i, i, vp]
+    lib.sbvr_hip_online_encode_lines_f16.argtypes = [vp, vp, vp, vp, i, i, i, i, i, vp]
     lib.sbvr_hip_decode_weight.argtypes = [vp, vp, i, vp, vp, i, i, i, i, i, i, i, vp]
     _lib = lib
     return lib
@@ -577,6 +578,25 @@ def online_encode(x, points, bvr_len):
     if rc != 0:
         raise SbvrHipError(f"sbvr_hip_online_encode_f16: error {rc} (M={M} K={K} bvr_len={bvr_len} S={S})")
     return bvr
+
+
+def online_encode_lines(x, lines, bvr_len):
+    """``online_encode`` from one line of input coefficients per group of K, lines (K / bvr_len, S) fp16: returns
+    the left operand's (bvr, coeff_idx), coeff_idx (K / bvr_len, M) holding every group's own number."""
+    _want(x, "x", torch.float16, 2)
+    _want(lines, "lines", torch.float16, 2, x.device)
+    M, K = x.shape
+    groups, S = lines.shape
+    if K != groups * bvr_len:
+        raise ValueError(f"lines must be (K / bvr_len, S), got {tuple(lines.shape)} for K={K}, bvr_len={bvr_len}")
+    bvr = torch.empty((K // 32, M, S), dtype=torch.uint32, device=x.device)
+    idx = torch.empty((groups, M), dtype=torch.uint8 if groups <= 256 else torch.uint16, device=x.device)
+    with torch.cuda.device(x.device):
+        rc = _load().sbvr_hip_online_encode_lines_f16(x.data_ptr(), lines.data_ptr(), bvr.data_ptr(), idx.data_ptr(),
+                                                      idx.element_size(), M, K, bvr_len, S, _stream())
+    if rc != 0:
+        raise SbvrHipError(f"sbvr_hip_online_encode_lines_f16: error {rc} (M={M} K={K} bvr_len={bvr_len} S={S})")
+    return bvr, idx
 
 
 _DECODE_TYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}

@@ -1,5 +1,5 @@
-"""The matrix-core product of two encoded operands, and the dense weight back from an encoding, against the CPU
-oracle at the sizes where their tilings have edges."""
+"""The matrix-core product of two encoded operands, the dense weight back from an encoding, and activations encoded
+from their input coefficients, each against the CPU oracle at the sizes where its tiling has edges."""
 import numpy as np
 import pytest
 import torch
@@ -56,3 +56,17 @@ def test_decode_weight(oracle, N, K, S, G, L, cols, dtype):
     got = obj.decode()
     want = torch.from_numpy(oracle.C.decode(bvr, idx, cache, G)[:, :cols].astype(np.float16)).to(dtype)
     assert got.shape == (N, cols) and got.dtype == dtype and torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("S,G,M,K", [(2, 32, 1, 32), (4, 96, 5, 288), (8, 128, 3, 512), (8, 256, 4, 67072), (1, 64, 9, 64)])
+def test_online_encode_lines(S, G, M, K):
+    """The same planes as from the table of subset sums, and every group's own number as its line."""
+    from sbvr import hip, layout
+    gen = torch.Generator().manual_seed(K + S)
+    x = torch.randn((M, K), generator=gen).to(torch.float16).to("cuda:0")
+    lines = (torch.randint(-1000, 1000, (K // G, S), generator=gen) / 512).to(torch.float16).to("cuda:0")
+    points = (lines.float() @ layout.bin_combs(S, torch.float32, "cuda:0").T).to(torch.float16)   # (exact sums)
+    bvr, idx = hip.online_encode_lines(x, lines, G)
+    assert torch.equal(bvr.view(torch.int32), hip.online_encode(x, points, G).view(torch.int32))
+    assert idx.dtype == (torch.uint8 if K // G <= 256 else torch.uint16)
+    assert torch.equal(idx.to(torch.int64), torch.arange(K // G, device="cuda:0").view(-1, 1).expand(-1, M))
