@@ -5,6 +5,8 @@
 #ifndef SBVR_HIP_ENCODER_H
 #define SBVR_HIP_ENCODER_H
 
+#include <stdint.h>
+
 #ifdef __cplusplus
 extern "C" {
 #endif

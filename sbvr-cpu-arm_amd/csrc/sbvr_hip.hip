@@ -4195,10 +4195,10 @@ size_t sbvr_hip_row_deq_mm_T_workspace(int M, int N)
     return col_wgs * 2 < 3L * current_cus() / 4 ? static_cast<size_t>(M) * N * sizeof(unsigned long long) : 0;
 }
 
-// (one left row against many columns runs on the decode kernel, the one form that may split K across workgroups)
+// (only one left row may run on the decode kernel, the one form that may split K across workgroups)
 size_t sbvr_hip_mm_T_workspace(int M, int N)
 {
-    return M == 1 && N >= kMmDecodeMinN ? static_cast<size_t>(N) * sizeof(unsigned long long) : 0;
+    return M == 1 && N > 0 ? static_cast<size_t>(N) * sizeof(unsigned long long) : 0;
 }
 
 int sbvr_hip_mm_T(const uint32_t *l_bvr, const void *l_coeff_idx, int l_idx_bytes,

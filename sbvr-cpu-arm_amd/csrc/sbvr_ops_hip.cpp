@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/sbvr_hip.h"
+#include "../../include/sbvr_hip_encoder.h"
 
 namespace {
 
@@ -118,35 +119,70 @@ void sbvr_hip_init_current()
     check(sbvr_hip_init(static_cast<int>(at::hip::current_device())));
 }
 
+namespace {
+
+// The launch of a linear over operands that have been checked; out: M * N elements.
+void launch_linear(const torch::Tensor &x, const torch::Tensor &bvr, const torch::Tensor &coeff_idx, const torch::Tensor &coeff_cache,
+                   const Bias &bias, const torch::Tensor &out, const LinearShape &s, int flags)
+{
+    hipStream_t stream = current_stream();
+    const size_t need = sbvr_hip_linear_f16_workspace(s.M, s.N, s.K, s.S, s.G);
+    torch::Tensor ws = need ? workspace(need, x, stream) : torch::Tensor();
+    check(sbvr_hip_linear_f16(x.data_ptr(), static_cast<const uint32_t *>(bvr.data_ptr()), coeff_idx.data_ptr(), s.ib,
+                              coeff_cache.data_ptr(), bias_ptr(bias, s.N, x), out.data_ptr(), s.M, s.N, s.K, s.S, s.G,
+                              s.L, need ? ws.data_ptr() : nullptr, need ? ws.numel() : 0, flags, stream));
+}
+
+}  // namespace
+
 // y = x @ decode(W)^T (+ bias): x (M, K) fp16; W in the default layout, bvr (K/32, N, S) uint32,
 // coeff_idx (K/G, N), coeff_cache (L, S) fp16.  bvr_len <= 0: the group length follows from coeff_idx.
 // out: an (M, N) fp16 tensor to write into (a caller that records a HIP graph brings its own), or None.
-torch::Tensor sbvr_linear_f16(torch::Tensor x, torch::Tensor bvr, torch::Tensor coeff_idx, torch::Tensor coeff_cache,
-                              Bias bias, int64_t bvr_len, int64_t flags, c10::optional<torch::Tensor> out_opt)
+torch::Tensor sbvr_linear_f16(const torch::Tensor &x, const torch::Tensor &bvr, const torch::Tensor &coeff_idx,
+                              const torch::Tensor &coeff_cache, const Bias &bias, int64_t bvr_len, int64_t flags,
+                              const c10::optional<torch::Tensor> &out_opt)
 {
     want(x, "x", torch::kFloat16, 2, nullptr);
     const LinearShape s = linear_shape(x.size(0), x.size(1), bvr, coeff_idx, coeff_cache, bvr_len, x);
     const DeviceGuard guard(x.device());
-    hipStream_t stream = current_stream();
     torch::Tensor out;
     if (out_opt.has_value() && out_opt->defined()) {
         out = *out_opt;
         want(out, "out", torch::kFloat16, 2, &x);
         TORCH_CHECK(out.size(0) == s.M && out.size(1) == s.N, "out has the wrong shape");
     } else {
-        out = torch::empty({s.M, s.N}, torch::dtype(torch::kFloat16).device(x.device()));
+        out = at::empty({s.M, s.N}, x.options());
     }
-    const size_t need = sbvr_hip_linear_f16_workspace(s.M, s.N, s.K, s.S, s.G);
-    torch::Tensor ws = need ? workspace(need, x, stream) : torch::Tensor();
-    check(sbvr_hip_linear_f16(x.data_ptr(), static_cast<const uint32_t *>(bvr.data_ptr()), coeff_idx.data_ptr(), s.ib,
-                              coeff_cache.data_ptr(), bias_ptr(bias, s.N, x), out.data_ptr(), s.M, s.N, s.K, s.S, s.G,
-                              s.L, need ? ws.data_ptr() : nullptr, need ? ws.numel() : 0, static_cast<int>(flags), stream));
+    launch_linear(x, bvr, coeff_idx, coeff_cache, bias, out, s, static_cast<int>(flags));
     return out;
 }
 
+// SBVRLinear.forward in one call: x (..., in_features) of any floating type; K zero-padded to k_padded where the encoder
+// padded it, the output cut to out_features columns.  (Taking the steps of this one by one in Python cost as much
+// as the launch: 10.2 us a call at 4096 -> 1024, one row.)
+torch::Tensor sbvr_linear_forward(torch::Tensor x, const torch::Tensor &bvr, const torch::Tensor &coeff_idx,
+                                  const torch::Tensor &coeff_cache, const Bias &bias, int64_t bvr_len, int64_t k_padded,
+                                  int64_t out_features)
+{
+    TORCH_CHECK(x.is_cuda(), "x must be on a GPU (got ", x.device(), "); there is no CPU path");
+    TORCH_CHECK(x.dim() >= 1, "x must have at least one dimension");
+    if (x.scalar_type() != torch::kFloat16)
+        x = x.to(torch::kFloat16);
+    if (x.size(-1) != k_padded)
+        x = at::constant_pad_nd(x, {0, k_padded - x.size(-1)});
+    x = x.contiguous();
+    const LinearShape s = linear_shape(x.numel() / k_padded, k_padded, bvr, coeff_idx, coeff_cache, bvr_len, x);
+    const DeviceGuard guard(x.device());
+    c10::SmallVector<int64_t, 6> sizes(x.sizes().begin(), x.sizes().end());
+    sizes.back() = s.N;
+    torch::Tensor out = at::empty(sizes, x.options());
+    launch_linear(x, bvr, coeff_idx, coeff_cache, bias, out, s, 0);
+    return s.N == out_features ? out : out.narrow(-1, 0, out_features);
+}
+
 // The linear of fp16(fp16(silu(gate)) * up) for gate_up (1, 2K) = gate | up.
-torch::Tensor sbvr_linear_f16_swiglu(torch::Tensor gate_up, torch::Tensor bvr, torch::Tensor coeff_idx,
-                                     torch::Tensor coeff_cache, Bias bias, int64_t bvr_len)
+torch::Tensor sbvr_linear_f16_swiglu(const torch::Tensor &gate_up, const torch::Tensor &bvr, const torch::Tensor &coeff_idx,
+                                     const torch::Tensor &coeff_cache, const Bias &bias, int64_t bvr_len)
 {
     want(gate_up, "gate_up", torch::kFloat16, 2, nullptr);
     TORCH_CHECK(gate_up.size(1) % 2 == 0, "gate_up must have an even number of columns");
@@ -189,8 +225,10 @@ torch::Tensor sbvr_linear_f16_add_rmsnorm(torch::Tensor x, torch::Tensor delta, 
 }
 
 // Both operands encoded, default layout: l_bvr (K/32, M, Sl), r_bvr (K/32, N, Sr) (sbvr_ops.cpp:35-76).
-torch::Tensor sbvr_mm_T(torch::Tensor l_bvr, torch::Tensor l_coeff_idx, torch::Tensor l_coeff_cache, torch::Tensor r_bvr,
-                        torch::Tensor r_coeff_idx, torch::Tensor r_coeff_cache, Bias bias)
+// bvr_len <= 0: the group length follows from l_coeff_idx.
+torch::Tensor sbvr_mm_T(const torch::Tensor &l_bvr, const torch::Tensor &l_coeff_idx, const torch::Tensor &l_coeff_cache,
+                        const torch::Tensor &r_bvr, const torch::Tensor &r_coeff_idx, const torch::Tensor &r_coeff_cache,
+                        const Bias &bias, int64_t bvr_len)
 {
     want(l_bvr, "l_bvr", torch::kUInt32, 3, nullptr);
     want(r_bvr, "r_bvr", torch::kUInt32, 3, &l_bvr);
@@ -203,10 +241,10 @@ torch::Tensor sbvr_mm_T(torch::Tensor l_bvr, torch::Tensor l_coeff_idx, torch::T
     TORCH_CHECK(l_coeff_idx.size(1) == M && r_coeff_idx.size(1) == N && l_coeff_idx.size(0) == r_coeff_idx.size(0) &&
                     l_coeff_cache.size(1) == Sl && r_coeff_cache.size(1) == Sr,
                 "index / table shapes do not match the bit planes");
-    const int64_t G = K / l_coeff_idx.size(0);
+    const int64_t G = bvr_len > 0 ? bvr_len : K / l_coeff_idx.size(0);
     TORCH_CHECK(G * l_coeff_idx.size(0) == K, "coeff_idx has ", l_coeff_idx.size(0), " groups, K=", K);
     const DeviceGuard guard(l_bvr.device());
-    auto out = torch::empty({M, N}, torch::dtype(torch::kFloat16).device(l_bvr.device()));
+    auto out = at::empty({M, N}, l_coeff_cache.options());
     hipStream_t stream = current_stream();
     const size_t need = sbvr_hip_mm_T_workspace(static_cast<int>(M), static_cast<int>(N));
     torch::Tensor ws;                    // (no split of K for this call: no workspace, nothing allocated)
@@ -219,10 +257,49 @@ torch::Tensor sbvr_mm_T(torch::Tensor l_bvr, torch::Tensor l_coeff_idx, torch::T
     return out;
 }
 
+// Activations x (M, K) fp16 encoded against one line of input coefficients per group of K, lines (K/G, S) fp16: the
+// left operand's (bvr, coeff_idx) (what sbvr/core.py:1021-1022 of the reference is a placeholder for).
+std::tuple<torch::Tensor, torch::Tensor> sbvr_online_encode_lines(const torch::Tensor &x, const torch::Tensor &lines, int64_t bvr_len)
+{
+    want(x, "x", torch::kFloat16, 2, nullptr);
+    want(lines, "lines", torch::kFloat16, 2, &x);
+    const int64_t M = x.size(0), K = x.size(1), groups = lines.size(0), S = lines.size(1);
+    TORCH_CHECK(K == groups * bvr_len, "lines must be (K / bvr_len, S), got ", lines.sizes(), " for K=", K, ", bvr_len=", bvr_len);
+    const DeviceGuard guard(x.device());
+    auto bvr = at::empty({K / 32, M, S}, x.options().dtype(torch::kUInt32));
+    auto idx = at::empty({groups, M}, x.options().dtype(groups <= 256 ? torch::kUInt8 : torch::kUInt16));
+    const int rc = sbvr_hip_online_encode_lines_f16(x.data_ptr(), lines.data_ptr(), static_cast<uint32_t *>(bvr.data_ptr()), idx.data_ptr(),
+                                                    groups <= 256 ? 1 : 2, M, K, bvr_len, S, current_stream());
+    TORCH_CHECK(rc == 0, "sbvr_hip_online_encode_lines_f16: error ", rc, " (M=", M, " K=", K, " bvr_len=", bvr_len, " S=", S, ")");
+    return {bvr, idx};
+}
+
+// The dense (N, cols) weight of a default-layout encoding, fp16, bf16 or fp32 (sbvr/core.py:926-949).
+torch::Tensor sbvr_decode_weight(const torch::Tensor &bvr, const torch::Tensor &coeff_idx, const torch::Tensor &coeff_cache,
+                                 int64_t bvr_len, int64_t cols, c10::ScalarType dtype)
+{
+    want(bvr, "bvr", torch::kUInt32, 3, nullptr);
+    want(coeff_cache, "coeff_cache", torch::kFloat16, 2, &bvr);
+    TORCH_CHECK(coeff_idx.scalar_type() == torch::kUInt8 || coeff_idx.scalar_type() == torch::kUInt16, "coeff_idx must be uint8 or uint16");
+    want(coeff_idx, "coeff_idx", coeff_idx.scalar_type(), 2, &bvr);
+    const int64_t K = bvr.size(0) * 32, N = bvr.size(1), S = bvr.size(2), L = coeff_cache.size(0);
+    TORCH_CHECK(coeff_idx.size(0) * bvr_len == K && coeff_idx.size(1) == N && coeff_cache.size(1) == S,
+                "coeff_idx / coeff_cache shapes do not match bvr");
+    const int type = dtype == torch::kFloat32 ? 2 : (dtype == torch::kBFloat16 ? 1 : 0);
+    const DeviceGuard guard(bvr.device());
+    auto out = at::empty({N, cols}, coeff_cache.options().dtype(type == 2 ? torch::kFloat32 : (type == 1 ? torch::kBFloat16 : torch::kFloat16)));
+    const int rc = sbvr_hip_decode_weight(static_cast<const uint32_t *>(bvr.data_ptr()), coeff_idx.data_ptr(),
+                                          static_cast<int>(coeff_idx.element_size()), coeff_cache.data_ptr(), out.data_ptr(), type, N, K,
+                                          cols, S, bvr_len, L, current_stream());
+    TORCH_CHECK(rc == 0, "sbvr_hip_decode_weight: error ", rc, " (N=", N, " K=", K, " cols=", cols, " S=", S, " bvr_len=", bvr_len, ")");
+    return out.scalar_type() == dtype ? out : out.to(dtype);
+}
+
 // fp16 l_w (M, K) against a trans=True weight: r_bvr (N/32, K, S), r_coeff_idx (N/G, K) (sbvr_ops.cpp:79-120).
 // use_shfl chose between equivalent CUDA kernels in the reference and is ignored.
-torch::Tensor sbvr_row_deq_mm_T(torch::Tensor l_w, torch::Tensor r_bvr, torch::Tensor r_coeff_idx,
-                                torch::Tensor r_coeff_cache, Bias bias, int64_t use_shfl)
+// bvr_len <= 0: the group length follows from r_coeff_idx.
+torch::Tensor sbvr_row_deq_mm_T(const torch::Tensor &l_w, const torch::Tensor &r_bvr, const torch::Tensor &r_coeff_idx,
+                                const torch::Tensor &r_coeff_cache, const Bias &bias, int64_t use_shfl, int64_t bvr_len)
 {
     (void)use_shfl;
     want(l_w, "l_w", torch::kFloat16, 2, nullptr);
@@ -231,10 +308,10 @@ torch::Tensor sbvr_row_deq_mm_T(torch::Tensor l_w, torch::Tensor r_bvr, torch::T
     const int64_t M = l_w.size(0), K = l_w.size(1), N = r_bvr.size(0) * 32, S = r_bvr.size(2), L = r_coeff_cache.size(0);
     const int ib = idx_bytes(r_coeff_idx, L, "r_coeff_idx", l_w);
     TORCH_CHECK(r_bvr.size(1) == K && r_coeff_idx.size(1) == K && r_coeff_cache.size(1) == S, "operand shapes do not match");
-    const int64_t G = N / r_coeff_idx.size(0);
+    const int64_t G = bvr_len > 0 ? bvr_len : N / r_coeff_idx.size(0);
     TORCH_CHECK(G * r_coeff_idx.size(0) == N, "r_coeff_idx has ", r_coeff_idx.size(0), " groups, N=", N);
     const DeviceGuard guard(l_w.device());
-    auto out = torch::empty({M, N}, torch::dtype(torch::kFloat16).device(l_w.device()));
+    auto out = at::empty({M, N}, l_w.options());
     hipStream_t stream = current_stream();
     const size_t need = sbvr_hip_row_deq_mm_T_workspace(static_cast<int>(M), static_cast<int>(N));
     torch::Tensor ws;                    // (no split of K for this call: no workspace, nothing allocated)
@@ -252,12 +329,20 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("_sbvr_hip_init", &sbvr_hip_init_current, "Checks that the current device is a gfx950 part");
     m.def("_sbvr_cuda_init", &sbvr_hip_init_current, "Alias of _sbvr_hip_init under the reference's name");
     m.def("_sbvr_mm_T", &sbvr_mm_T, "SBVR x SBVR^T, both operands encoded", py::arg("l_bvr"), py::arg("l_coeff_idx"),
-          py::arg("l_coeff_cache"), py::arg("r_bvr"), py::arg("r_coeff_idx"), py::arg("r_coeff_cache"), py::arg("bias"));
+          py::arg("l_coeff_cache"), py::arg("r_bvr"), py::arg("r_coeff_idx"), py::arg("r_coeff_cache"), py::arg("bias"),
+          py::arg("bvr_len") = 0);
     m.def("_sbvr_row_deq_mm_T", &sbvr_row_deq_mm_T, "fp16 x SBVR^T over the trans=True layout", py::arg("l_w"),
-          py::arg("r_bvr"), py::arg("r_coeff_idx"), py::arg("r_coeff_cache"), py::arg("bias"), py::arg("use_shfl") = 0);
+          py::arg("r_bvr"), py::arg("r_coeff_idx"), py::arg("r_coeff_cache"), py::arg("bias"), py::arg("use_shfl") = 0,
+          py::arg("bvr_len") = 0);
     m.def("_sbvr_linear_f16", &sbvr_linear_f16, "fp16 x SBVR^T over the default layout", py::arg("x"), py::arg("bvr"),
           py::arg("coeff_idx"), py::arg("coeff_cache"), py::arg("bias") = py::none(), py::arg("bvr_len") = 0,
           py::arg("flags") = 0, py::arg("out") = py::none());
+    m.def("_linear_forward", &sbvr_linear_forward, "SBVRLinear.forward", py::arg("x"), py::arg("bvr"), py::arg("coeff_idx"),
+          py::arg("coeff_cache"), py::arg("bias"), py::arg("bvr_len"), py::arg("k_padded"), py::arg("out_features"));
+    m.def("_online_encode_lines", &sbvr_online_encode_lines, "activations to the arrays of an encoded left operand", py::arg("x"),
+          py::arg("lines"), py::arg("bvr_len"));
+    m.def("_decode_weight", &sbvr_decode_weight, "the dense weight of a default-layout encoding", py::arg("bvr"),
+          py::arg("coeff_idx"), py::arg("coeff_cache"), py::arg("bvr_len"), py::arg("cols"), py::arg("dtype"));
     m.def("last_kernel", &sbvr_hip_last_kernel, "which kernel the last linear call of this thread launched");
     m.def("_sbvr_linear_f16_swiglu", &sbvr_linear_f16_swiglu, "the linear of silu(gate) * up, one row", py::arg("gate_up"),
           py::arg("bvr"), py::arg("coeff_idx"), py::arg("coeff_cache"), py::arg("bias") = py::none(),

@@ -90,6 +90,26 @@ def _check(rc):
         raise SbvrHipError(f"libsbvr_hip: error {rc}: {_load().sbvr_hip_last_error().decode()}")
 
 
+_extension = None
+
+
+def _ext():
+    """The PyTorch extension over the same library (csrc/sbvr_ops_hip.cpp), or False where it is not built or another
+    copy of the library is asked for.  The operators below go through it: the same checks and the same launch, 4 to 6 us
+    a call where ctypes and the checks in Python take 16.  What it refuses goes through the checks below for their
+    error."""
+    global _extension
+    if _extension is None:
+        _extension = False
+        if not os.environ.get("SBVR_HIP_LIBRARY"):
+            try:
+                from . import _sbvr_hip_ops
+                _extension = _sbvr_hip_ops
+            except ImportError:
+                pass
+    return _extension
+
+
 KERNEL_PORTABLE, KERNEL_DECODE, KERNEL_ROWS32, KERNEL_PREFILL, KERNEL_PREFILL_SPLIT = 1, 2, 3, 4, 5
 
 
@@ -199,6 +219,12 @@ def _sbvr_linear_f16(x, bvr, coeff_idx, coeff_cache, bias=None, bvr_len=None, ou
     """y = x @ decode(W)^T (+ bias) for fp16 ``x`` (M, K) and a weight in the
     default uint32 layout: ``bvr`` (K/32, N, S), ``coeff_idx`` (K/G, N),
     ``coeff_cache`` (L, S).  Returns fp16 (M, N)."""
+    ext = _ext()
+    if ext:
+        try:
+            return ext._sbvr_linear_f16(x, bvr, coeff_idx, coeff_cache, bias, bvr_len or 0, flags, out)
+        except (RuntimeError, TypeError):
+            pass
     lib = _load()
     dev = x.device
     _want(x, "x", torch.float16, 2)
@@ -290,6 +316,12 @@ def _sbvr_row_deq_mm_T(l_w, r_bvr, r_coeff_idx, r_coeff_cache, bias, use_shfl=0,
     """fp16 ``l_w`` (M, K) against a ``trans=True`` weight: ``r_bvr`` (N/32, K, S),
     ``r_coeff_idx`` (N/G, K) (sbvr_ops.cpp:79-120).  ``use_shfl`` selected between
     equivalent CUDA kernels in the reference and is ignored."""
+    ext = _ext()
+    if ext:
+        try:
+            return ext._sbvr_row_deq_mm_T(l_w, r_bvr, r_coeff_idx, r_coeff_cache, bias, 0, bvr_len or 0)
+        except (RuntimeError, TypeError):
+            pass
     lib = _load()
     dev = l_w.device
     _want(l_w, "l_w", torch.float16, 2)
@@ -317,6 +349,12 @@ def _sbvr_row_deq_mm_T(l_w, r_bvr, r_coeff_idx, r_coeff_cache, bias, use_shfl=0,
 def _sbvr_mm_T(l_bvr, l_coeff_idx, l_coeff_cache, r_bvr, r_coeff_idx, r_coeff_cache, bias, bvr_len=None):
     """Both operands encoded, default uint32 layout: ``l_bvr`` (K/32, M, Sl),
     ``r_bvr`` (K/32, N, Sr) (sbvr_ops.cpp:35-76).  Returns fp16 (M, N)."""
+    ext = _ext()
+    if ext:
+        try:
+            return ext._sbvr_mm_T(l_bvr, l_coeff_idx, l_coeff_cache, r_bvr, r_coeff_idx, r_coeff_cache, bias, bvr_len or 0)
+        except (RuntimeError, TypeError):
+            pass
     lib = _load()
     dev = l_bvr.device
     _want(l_bvr, "l_bvr", torch.uint32, 3)
@@ -583,6 +621,12 @@ def online_encode(x, points, bvr_len):
 def online_encode_lines(x, lines, bvr_len):
     """``online_encode`` from one line of input coefficients per group of K, lines (K / bvr_len, S) fp16: returns
     the left operand's (bvr, coeff_idx), coeff_idx (K / bvr_len, M) holding every group's own number."""
+    ext = _ext()
+    if ext:
+        try:
+            return ext._online_encode_lines(x, lines, bvr_len)
+        except (RuntimeError, TypeError):
+            pass
     _want(x, "x", torch.float16, 2)
     _want(lines, "lines", torch.float16, 2, x.device)
     M, K = x.shape
@@ -605,6 +649,12 @@ _DECODE_TYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
 def decode_weight(bvr, coeff_idx, coeff_cache, bvr_len, cols, dtype):
     """The dense (N, cols) weight of a default-layout encoding (cols: without the padding of K), every element its
     coefficients' fp32 sum rounded to fp16 once, in ``dtype`` (sbvr/core.py:926-949)."""
+    ext = _ext()
+    if ext:
+        try:
+            return ext._decode_weight(bvr, coeff_idx, coeff_cache, bvr_len, cols, dtype)
+        except (RuntimeError, TypeError):
+            pass
     dev = bvr.device
     _want(bvr, "bvr", torch.uint32, 3)
     _want(coeff_idx, "coeff_idx", (torch.uint8, torch.uint16), 2, dev)

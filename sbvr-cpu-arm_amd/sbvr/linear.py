@@ -7,14 +7,19 @@ import torch
 from . import layout
 
 
-def _ops():
+_forward = None
+
+
+def _load_forward():
     """The PyTorch-ROCm extension over the library's C ABI (csrc/sbvr_ops_hip.cpp); there is no fallback."""
+    global _forward
     try:
         from . import _sbvr_hip_ops
     except ImportError as exc:
         raise RuntimeError("sbvr._sbvr_hip_ops is not built: run `make -C sbvr-cpu-arm_amd/csrc all` "
                            "(or __graft_entry__.build()); SBVRLinear has no other path") from exc
-    return _sbvr_hip_ops
+    _forward = _sbvr_hip_ops._linear_forward
+    return _forward
 
 
 class SBVRLinear(torch.nn.Module):
@@ -55,14 +60,8 @@ class SBVRLinear(torch.nn.Module):
                    encs[0].bvr_len, bias)
 
     def forward(self, x):
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1])
-        if x2.dtype != torch.float16:
-            x2 = x2.to(torch.float16)
-        if x2.shape[1] != self.k_padded:      # the encoder pads K to a multiple of bvr_len
-            x2 = torch.nn.functional.pad(x2, (0, self.k_padded - x2.shape[1]))
-        x2 = x2.contiguous()
-        # any number of rows: the operator picks the decode, 32-row or prefill kernel
-        y = _ops()._sbvr_linear_f16(x2, self.bvr, self.coeff_idx, self.coeff_cache, self.bias, self.bvr_len)
-        y = y[:, :self.out_features]
-        return y.reshape(*lead, self.out_features)
+        # any number of rows: the operator picks the decode, 32-row or prefill kernel.  Leading dimensions, other
+        # floating types, the encoder's padding of K to a multiple of bvr_len: all inside the one call
+        b = self._buffers
+        return (_forward or _load_forward())(x, b["bvr"], b["coeff_idx"], b["coeff_cache"], b["bias"], self.bvr_len,
+                                             self.k_padded, self.out_features)
