@@ -95,9 +95,10 @@ _extension = None
 
 def _ext():
     """The PyTorch extension over the same library (csrc/sbvr_ops_hip.cpp), or False where it is not built or another
-    copy of the library is asked for.  The operators below go through it: the same checks and the same launch, 4 to 6 us
-    a call where ctypes and the checks in Python take 16.  What it refuses goes through the checks below for their
-    error."""
+    copy of the library is asked for.  The products of encoded operands, the on-the-fly encoding and the dense decode
+    go through it: the same checks and the same launch, 4 to 6 us a call where ctypes and the checks in Python take 16.
+    What it refuses goes through the checks below for their error.  (The fp16 linears below stay on ctypes: they share
+    this module's workspace, and SBVRLinear.forward does not come this way.)"""
     global _extension
     if _extension is None:
         _extension = False
@@ -219,12 +220,6 @@ def _sbvr_linear_f16(x, bvr, coeff_idx, coeff_cache, bias=None, bvr_len=None, ou
     """y = x @ decode(W)^T (+ bias) for fp16 ``x`` (M, K) and a weight in the
     default uint32 layout: ``bvr`` (K/32, N, S), ``coeff_idx`` (K/G, N),
     ``coeff_cache`` (L, S).  Returns fp16 (M, N)."""
-    ext = _ext()
-    if ext:
-        try:
-            return ext._sbvr_linear_f16(x, bvr, coeff_idx, coeff_cache, bias, bvr_len or 0, flags, out)
-        except (RuntimeError, TypeError):
-            pass
     lib = _load()
     dev = x.device
     _want(x, "x", torch.float16, 2)
@@ -317,7 +312,7 @@ def _sbvr_row_deq_mm_T(l_w, r_bvr, r_coeff_idx, r_coeff_cache, bias, use_shfl=0,
     ``r_coeff_idx`` (N/G, K) (sbvr_ops.cpp:79-120).  ``use_shfl`` selected between
     equivalent CUDA kernels in the reference and is ignored."""
     ext = _ext()
-    if ext:
+    if ext and (bvr_len is None or bvr_len > 0):
         try:
             return ext._sbvr_row_deq_mm_T(l_w, r_bvr, r_coeff_idx, r_coeff_cache, bias, 0, bvr_len or 0)
         except (RuntimeError, TypeError):
@@ -350,7 +345,7 @@ def _sbvr_mm_T(l_bvr, l_coeff_idx, l_coeff_cache, r_bvr, r_coeff_idx, r_coeff_ca
     """Both operands encoded, default uint32 layout: ``l_bvr`` (K/32, M, Sl),
     ``r_bvr`` (K/32, N, Sr) (sbvr_ops.cpp:35-76).  Returns fp16 (M, N)."""
     ext = _ext()
-    if ext:
+    if ext and (bvr_len is None or bvr_len > 0):
         try:
             return ext._sbvr_mm_T(l_bvr, l_coeff_idx, l_coeff_cache, r_bvr, r_coeff_idx, r_coeff_cache, bias, bvr_len or 0)
         except (RuntimeError, TypeError):
