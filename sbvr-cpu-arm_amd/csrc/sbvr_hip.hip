@@ -2331,13 +2331,23 @@ hipError_t launch_gemm(int S, const GemmArgs &a, hipStream_t st)
 // 2, 3 or 4 planes, K and G multiples of 128 (the two steps of a loop iteration share a coefficient line).
 // K can be split across workgroups (blockIdx.z) as in sbvr_gemm_mfma_kernel: fp32 partial tiles, second pass.
 constexpr int kPfWaves = 8, kPfBM = 256, kPfBN = 256, kPfRow = 144;
-constexpr int kPfTile = kPfBM * kPfRow;
 
-template <int S>
+// RB: row blocks of 32 of a workgroup (2, 4, 6 or 8).  The matrix pipe and the decode take turns, so an MFMA of a row
+// block beyond M costs as much as one inside it: the rows are shared out evenly over the tiles (gemm_lut_row_blocks).
+// With 2, 4, 6 and 8 row blocks a step takes 0.94, 1.36, 1.84 and 2.08 us (8192 -> 28672, 4 planes); 64 / 128 / 192 /
+// 333 rows 60 / 87 / 118 / 198 us there, where 8 row blocks for any number of rows took 131 / 133 / 139 / 248.
+template <int S, int RB>
 __global__ void __launch_bounds__(64 * kPfWaves)
 sbvr_gemm_lut_kernel(const GemmArgs a)
 {
     static_assert(S >= 2 && S <= 4, "tables of 4, 8 or 16 entries");
+    static_assert(RB == 2 || RB == 4 || RB == 6 || RB == 8, "row blocks of a workgroup");
+    // of the four MFMA operands of a (row, word), a thread brings in NQ (1 or 2 where 512 threads then cover the rows)
+    constexpr int NQ = RB == 2 ? 1 : (RB == 4 ? 2 : 4);
+    constexpr int kTile = 32 * (RB == 6 ? 8 : RB) * kPfRow;         // (6 row blocks: the threads still cover 256 rows)
+    struct Part {
+        uint32_t w[4 * NQ];                                          // dword c * NQ + q: dword q0 + q of 16-byte chunk c
+    };
     extern __shared__ __align__(16) unsigned char psm[];
     constexpr int CW = (S + 1) / 2;
 
@@ -2345,15 +2355,16 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int N = a.N, K = a.K, M = a.M;
     const int j = lane & 31, h = lane >> 5;
-    const int n0 = blockIdx.x * kPfBN, m0 = blockIdx.y * kPfBM;
+    const int n0 = blockIdx.x * kPfBN, m0 = blockIdx.y * (32 * RB);
     const int n = n0 + 32 * wave + j, n_ld = min(n, N - 1);
     const int steps = K / 64 / a.ksplit;                 // of this workgroup, even
     const int p0 = blockIdx.z * steps, p_last = p0 + steps - 1;
     const int wpg = 2 * a.steps_per_group;               // words per group
 
-    // bringing activations in: thread t takes (row t / 2, word t % 2) of a step, 64 bytes
-    const uint16_t *xsrc = a.x + static_cast<size_t>(min(m0 + (tid >> 1), M - 1)) * K + 32 * (tid & 1);
-    unsigned char *const xdst = psm + (tid >> 1) * kPfRow + (tid & 1) * 64;
+    // bringing activations in: a thread takes operands q0 .. q0 + NQ - 1 of word xw of row xr of a step
+    const int xr = (tid * NQ) >> 3, xw = ((tid * NQ) >> 2) & 1, q0 = (tid * NQ) & 3;
+    const uint16_t *xsrc = a.x + static_cast<size_t>(min(m0 + xr, M - 1)) * K + 32 * xw + 2 * q0;
+    unsigned char *const xdst = psm + xr * kPfRow + xw * 64 + 16 * q0;
     const unsigned char *const xrd = psm + j * kPfRow + h * 64;      // + 32 rb rows, + 16 q
 
     struct Line {
@@ -2375,33 +2386,42 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
         for (int q = 0; q < S; ++q)
             w[q] = pl.w[q];
     };
-    auto load_x = [&](int ip, v4u (&x)[4]) __attribute__((always_inline)) {
-        const v4u *xp = reinterpret_cast<const v4u *>(xsrc + 64 * min(ip, p_last));
+    auto load_x = [&](int ip, Part &x) __attribute__((always_inline)) {
+        const uint16_t *xp = xsrc + 64 * min(ip, p_last);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            x[i] = xp[i];
+        for (int c = 0; c < 4; ++c) {
+            if constexpr (NQ == 4) {
+                const v4u v = *reinterpret_cast<const v4u *>(xp + 8 * c);
+                x.w[4 * c] = v.x; x.w[4 * c + 1] = v.y; x.w[4 * c + 2] = v.z; x.w[4 * c + 3] = v.w;
+            } else if constexpr (NQ == 2) {
+                const v2u v = *reinterpret_cast<const v2u *>(xp + 8 * c);
+                x.w[2 * c] = v.x; x.w[2 * c + 1] = v.y;
+            } else {
+                x.w[c] = *reinterpret_cast<const uint32_t *>(xp + 8 * c);
+            }
+        }
     };
     // the 32 elements of a (row, word), dword i = elements 2i, 2i + 1, into the order of the four MFMAs' A operands:
     // operand q = elements 2q, 2q+8, 2q+16, 2q+24, 2q+1, 2q+9, 2q+17, 2q+25
-    auto store_x = [&](const v4u (&x)[4], int buf) __attribute__((always_inline)) {
+    auto store_x = [&](const Part &x, int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t d0 = x[0][q], d1 = x[1][q], d2 = x[2][q], d3 = x[3][q];
+        for (int q = 0; q < NQ; ++q) {
+            const uint32_t d0 = x.w[q], d1 = x.w[NQ + q], d2 = x.w[2 * NQ + q], d3 = x.w[3 * NQ + q];
             v4u aw;
             aw.x = __builtin_amdgcn_perm(d1, d0, 0x05040100u);
             aw.y = __builtin_amdgcn_perm(d3, d2, 0x05040100u);
             aw.z = __builtin_amdgcn_perm(d1, d0, 0x07060302u);
             aw.w = __builtin_amdgcn_perm(d3, d2, 0x07060302u);
-            *reinterpret_cast<v4u *>(xdst + buf * kPfTile + 16 * q) = aw;
+            *reinterpret_cast<v4u *>(xdst + buf * kTile + 16 * q) = aw;
         }
     };
 
     LutTables<S> tables;
     auto build_table = [&](const uint32_t (&c)[CW]) __attribute__((always_inline)) { lut_build_tables<S>(c, tables); };
 
-    v16f acc[8];
+    v16f acc[RB];
 #pragma unroll
-    for (int rb = 0; rb < 8; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
             acc[rb][r] = 0.f;
@@ -2410,13 +2430,13 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
         uint32_t Q[4];
         lut_nibble_words<S>(w, Q);
         auto operand = [&](int q) __attribute__((always_inline)) -> v4u { return lut_operand<S>(tables, Q, q); };
-        // MFMA q of all 8 row blocks in a row (8 different accumulators), its 8 activation operands read while
+        // MFMA q of all row blocks in a row (RB different accumulators), its RB activation operands read while
         // MFMA q - 1 runs, and the look-ups of operand q + 1 in the shadow of the matrix pipe
-        const unsigned char *xt = xrd + buf * kPfTile;
-        v4u A[2][8];
-        auto read_a = [&](int q, v4u (&dst)[8]) __attribute__((always_inline)) {
+        const unsigned char *xt = xrd + buf * kTile;
+        v4u A[2][RB];
+        auto read_a = [&](int q, v4u (&dst)[RB]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int rb = 0; rb < 8; ++rb)
+            for (int rb = 0; rb < RB; ++rb)
                 dst[rb] = *reinterpret_cast<const v4u *>(xt + 32 * rb * kPfRow + 16 * q);
         };
         read_a(0, A[0]);
@@ -2430,7 +2450,7 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
                 Bn = operand(q + 1);
             }
 #pragma unroll
-            for (int rb = 0; rb < 8; ++rb)
+            for (int rb = 0; rb < RB; ++rb)
                 acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, A[q & 1][rb]), __builtin_bit_cast(v8h, Bq), acc[rb], 0, 0, 0);
             Bq = Bn;
         }
@@ -2439,7 +2459,7 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
     // -- prologue: the first step's activations into buffer 0, everything of the second in flight
     // (decoding a step's operands one step ahead, in the shadow of the step before's MFMAs, measured no faster)
     uint32_t wa[S], wb[S], c[CW], c_next[CW];
-    v4u xa[4];
+    Part xa;
     Line line = load_line(p0);
     load_words(p0, wa);
     load_x(p0, xa);
@@ -2479,7 +2499,7 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
     if (a.ksplit > 1) {
         float *mine = a.part + blockIdx.z * (static_cast<size_t>(M) * N);
 #pragma unroll
-        for (int rb = 0; rb < 8; ++rb)
+        for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m = m0 + 32 * rb + 8 * (r >> 2) + 4 * h + (r & 3);
@@ -2492,7 +2512,7 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
         return;
     const uint16_t bias = a.bias ? a.bias[n] : 0;
 #pragma unroll
-    for (int rb = 0; rb < 8; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int m = m0 + 32 * rb + 8 * (r >> 2) + 4 * h + (r & 3);
@@ -2526,13 +2546,22 @@ int gemm_lut_ksplit(int M, int N, int K)
     return ks;
 }
 
+// Row blocks of 32 a workgroup takes: the fewest (of 2, 4, 6 and 8) that cover the rows with as many tiles as 256 rows
+// each would.
+int gemm_lut_row_blocks(int M)
+{
+    const int tiles = (M + kPfBM - 1) / kPfBM;
+    return 2 * ((M + 64 * tiles - 1) / (64 * tiles));
+}
+
 hipError_t launch_gemm_lut(int S, const GemmArgs &a, hipStream_t st)
 {
-    const dim3 grid(static_cast<unsigned>((a.N + kPfBN - 1) / kPfBN), static_cast<unsigned>((a.M + kPfBM - 1) / kPfBM),
+    const int rb = gemm_lut_row_blocks(a.M);
+    const dim3 grid(static_cast<unsigned>((a.N + kPfBN - 1) / kPfBN), static_cast<unsigned>((a.M + 32 * rb - 1) / (32 * rb)),
                     static_cast<unsigned>(a.ksplit));
     const dim3 block(64 * kPfWaves);
-    const size_t lds = 2 * kPfTile;
-#define SBVR_PF_LAUNCH(SS)                                                                                     \
+    const size_t lds = 2 * 32 * (rb == 6 ? 8 : rb) * kPfRow;
+#define SBVR_PF_LAUNCH(SS, RR)                                                                                 \
     {                                                                                                          \
         static bool raised_on[16] = {};                                                                        \
         std::lock_guard<std::mutex> guard(g_dev_lock);                                                                        \
@@ -2541,23 +2570,32 @@ hipError_t launch_gemm_lut(int S, const GemmArgs &a, hipStream_t st)
             dev_now = 0;                                                                                       \
         bool &raised = raised_on[dev_now];                                                                     \
         if (!raised) {                                                                                         \
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(sbvr_gemm_lut_kernel<SS>), \
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(sbvr_gemm_lut_kernel<SS, RR>), \
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)); \
             if (e != hipSuccess)                                                                               \
                 return e;                                                                                      \
             raised = true;                                                                                     \
         }                                                                                                      \
-        hipLaunchKernelGGL(sbvr_gemm_lut_kernel<SS>, grid, block, lds, st, a);                                 \
+        hipLaunchKernelGGL((sbvr_gemm_lut_kernel<SS, RR>), grid, block, lds, st, a);                           \
+    }                                                                                                          \
+    break
+#define SBVR_PF_ROWS(SS)                                                                                       \
+    switch (rb) {                                                                                              \
+    case 2: SBVR_PF_LAUNCH(SS, 2);                                                                             \
+    case 4: SBVR_PF_LAUNCH(SS, 4);                                                                             \
+    case 6: SBVR_PF_LAUNCH(SS, 6);                                                                             \
+    default: SBVR_PF_LAUNCH(SS, 8);                                                                            \
     }                                                                                                          \
     break
     switch (S) {
-    case 4: SBVR_PF_LAUNCH(4);
+    case 4: SBVR_PF_ROWS(4);
 #ifndef SBVR_FAST_BUILD
-    case 2: SBVR_PF_LAUNCH(2);
-    case 3: SBVR_PF_LAUNCH(3);
+    case 2: SBVR_PF_ROWS(2);
+    case 3: SBVR_PF_ROWS(3);
 #endif
     default: return hipErrorInvalidConfiguration;
     }
+#undef SBVR_PF_ROWS
 #undef SBVR_PF_LAUNCH
     return hipGetLastError();
 }

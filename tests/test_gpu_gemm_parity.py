@@ -302,3 +302,11 @@ def test_k_split_without_workspace_is_not_split(oracle):
     _, yd = oracle.C.linear_f16(*ops)
     _, yd1 = oracle.C.linear_f16(*ops, mode=1)
     check(out, yd, yd1, parity.ROUNDING_DECODE, "unsplit launch without a workspace")
+
+
+@pytest.mark.parametrize("M", [64, 65, 128, 129, 192, 193, 256, 257, 384, 385, 513])
+@pytest.mark.parametrize("S", [2, 3, 4])
+def test_row_blocks_of_the_table_lookup_prefill(oracle, M, S):
+    """The row counts at which the prefill kernel's workgroups go from 2 to 4, 6 and 8 row blocks of 32, and from one
+    tile of rows to two and three; 16-bit indices and a bias at the odd ones."""
+    run_case(oracle, 260, 512, S, 128, M, 300 if M % 2 else 256, seed=1000 * S + M, bias=M % 2 == 1, expect=PREFILL)
