@@ -2330,10 +2330,12 @@ hipError_t launch_gemm(int S, const GemmArgs &a, hipStream_t st)
 // of the step after the next one's (activations, plane words) are in flight while a step is computed.
 // 2, 3 or 4 planes, K and G multiples of 128 (the two steps of a loop iteration share a coefficient line).
 // K can be split across workgroups (blockIdx.z) as in sbvr_gemm_mfma_kernel: fp32 partial tiles, second pass.
-constexpr int kPfWaves = 8, kPfBM = 256, kPfBN = 256, kPfRow = 144;
+constexpr int kPfWaves = 8, kPfBN = 256, kPfRow = 144;
 
-// RB: row blocks of 32 of a workgroup (2, 4, 6 or 8).  The matrix pipe and the decode take turns, so an MFMA of a row
-// block beyond M costs as much as one inside it: the rows are shared out evenly over the tiles (gemm_lut_row_blocks).
+constexpr int pf_loader_blocks(int rb) { return rb <= 2 ? 2 : (rb <= 4 ? 4 : 8); }
+
+// RB: row blocks of 32 of a workgroup (2 to 8).  The matrix pipe and the decode take turns, so an MFMA of a row
+// block beyond M costs as much as one inside it: the rows are shared out evenly over the tiles (gemm_lut_plan).
 // With 2, 4, 6 and 8 row blocks a step takes 0.94, 1.36, 1.84 and 2.08 us (8192 -> 28672, 4 planes); 64 / 128 / 192 /
 // 333 rows 60 / 87 / 118 / 198 us there, where 8 row blocks for any number of rows took 131 / 133 / 139 / 248.
 template <int S, int RB>
@@ -2341,10 +2343,10 @@ __global__ void __launch_bounds__(64 * kPfWaves)
 sbvr_gemm_lut_kernel(const GemmArgs a)
 {
     static_assert(S >= 2 && S <= 4, "tables of 4, 8 or 16 entries");
-    static_assert(RB == 2 || RB == 4 || RB == 6 || RB == 8, "row blocks of a workgroup");
+    static_assert(RB >= 2 && RB <= 8, "row blocks of a workgroup");
     // of the four MFMA operands of a (row, word), a thread brings in NQ (1 or 2 where 512 threads then cover the rows)
-    constexpr int NQ = RB == 2 ? 1 : (RB == 4 ? 2 : 4);
-    constexpr int kTile = 32 * (RB == 6 ? 8 : RB) * kPfRow;         // (6 row blocks: the threads still cover 256 rows)
+    constexpr int NQ = pf_loader_blocks(RB) / 2;
+    constexpr int kTile = 32 * pf_loader_blocks(RB) * kPfRow;       // (all rows the threads cover: 3 row blocks 128, 5 to 7 256)
     struct Part {
         uint32_t w[4 * NQ];                                          // dword c * NQ + q: dword q0 + q of 16-byte chunk c
     };
@@ -2531,36 +2533,49 @@ bool gemm_lut_path_ok(int M, int N, int K, int S, int G)
            static_cast<double>(K / 32) * N * S < 2147483648.0 && static_cast<double>(M) * K < 2147483648.0;
 }
 
-// Workgroups along K for the table look-up prefill kernel: until the 256 x 256 tiles times the parts give three
-// quarters of the chip's 256 CUs a workgroup, a part keeping 16 steps and more (an even number).  A function of the
-// shape only.  (8192 -> 28672: 112 tiles at 256 rows take 229-236 us unsplit and 187 us in two parts; 224 tiles at
-// 512 rows 293 us unsplit and 340 us in two parts.)
-int gemm_lut_ksplit(int M, int N, int K)
+// How the table look-up prefill kernel shares out a product: row blocks of 32 per workgroup, and parts of K (each an
+// even number of 16 steps and more).  A function of the shape only, so that the workspace can be sized without a device.
+// Few row blocks mean more workgroups and more decodes of the weights, more parts of K more workgroups and partial
+// results to write and add up: the plan is the one of least estimated time.  Estimate, from launches of 8192 -> 28672
+// with 2 to 8 row blocks (0.94, 1.36, 1.84, 2.08 us a step): a step takes 0.55 + 0.2 RB us, a workgroup 2 us beside its
+// steps, and a split 2 us and its partial results at 6 TB/s.  256 workgroups run at a time; beyond that the
+// last turn counts half (8192 -> 28672: 1.31 turns take the time of 1.70, 3.5 turns that of 3.68).
+// Against tiles of 256 rows throughout, 4 planes: 4096 -> 6144, 600 rows 86.5 -> 53.0 us (240 workgroups of 4 row blocks
+// for 144 of 7), 128 rows 30.6 -> 25.7; 4096 -> 4096, 192 rows 36.3 -> 26.0; 8192 -> 28672, 600 rows 472 -> 362.
+struct GemmLutPlan {
+    int rb, ksplit;
+};
+
+GemmLutPlan gemm_lut_plan(int M, int N, int K, bool may_split)
 {
-    const int tiles = ((N + kPfBN - 1) / kPfBN) * ((M + kPfBM - 1) / kPfBM), steps = K / 64;
-    int ks = 1;
-    if (N % 4)
-        return 1;
-    while (ks < 16 && tiles * ks * 4 < 3 * kGemmSplitCus && steps % (ks * 4) == 0 && steps / (ks * 2) >= 16)
-        ks *= 2;
-    return ks;
+    const int blocks = (M + 31) / 32, columns = (N + kPfBN - 1) / kPfBN, steps = K / 64;
+    GemmLutPlan best{8, 1};
+    double best_us = 0.;
+    for (int most = 8; most >= 2; --most) {
+        const int tiles = (blocks + most - 1) / most;
+        const int rb = max(2, (blocks + tiles - 1) / tiles);
+        for (int ks = 1; ks <= 16; ks *= 2) {
+            if (ks > 1 && (!may_split || N % 4 || steps % (ks * 2) || steps / ks < 16))
+                break;
+            const double turns = static_cast<double>(columns) * tiles * ks / kGemmSplitCus;
+            const double busy = turns <= 1. ? 1. : (ceil(turns) + turns) / 2.;
+            const double us = busy * (steps / ks * (0.55 + 0.2 * rb) + 2.) +
+                              (ks > 1 ? 2. + 4e-6 / 6. * ks * static_cast<double>(M) * N : 0.);
+            if (best_us == 0. || us < best_us) {
+                best = GemmLutPlan{rb, ks};
+                best_us = us;
+            }
+        }
+    }
+    return best;
 }
 
-// Row blocks of 32 a workgroup takes: the fewest (of 2, 4, 6 and 8) that cover the rows with as many tiles as 256 rows
-// each would.
-int gemm_lut_row_blocks(int M)
+hipError_t launch_gemm_lut(int S, int rb, const GemmArgs &a, hipStream_t st)
 {
-    const int tiles = (M + kPfBM - 1) / kPfBM;
-    return 2 * ((M + 64 * tiles - 1) / (64 * tiles));
-}
-
-hipError_t launch_gemm_lut(int S, const GemmArgs &a, hipStream_t st)
-{
-    const int rb = gemm_lut_row_blocks(a.M);
     const dim3 grid(static_cast<unsigned>((a.N + kPfBN - 1) / kPfBN), static_cast<unsigned>((a.M + 32 * rb - 1) / (32 * rb)),
                     static_cast<unsigned>(a.ksplit));
     const dim3 block(64 * kPfWaves);
-    const size_t lds = 2 * 32 * (rb == 6 ? 8 : rb) * kPfRow;
+    const size_t lds = 2 * 32 * pf_loader_blocks(rb) * kPfRow;
 #define SBVR_PF_LAUNCH(SS, RR)                                                                                 \
     {                                                                                                          \
         static bool raised_on[16] = {};                                                                        \
@@ -2582,8 +2597,11 @@ hipError_t launch_gemm_lut(int S, const GemmArgs &a, hipStream_t st)
 #define SBVR_PF_ROWS(SS)                                                                                       \
     switch (rb) {                                                                                              \
     case 2: SBVR_PF_LAUNCH(SS, 2);                                                                             \
+    case 3: SBVR_PF_LAUNCH(SS, 3);                                                                             \
     case 4: SBVR_PF_LAUNCH(SS, 4);                                                                             \
+    case 5: SBVR_PF_LAUNCH(SS, 5);                                                                             \
     case 6: SBVR_PF_LAUNCH(SS, 6);                                                                             \
+    case 7: SBVR_PF_LAUNCH(SS, 7);                                                                             \
     default: SBVR_PF_LAUNCH(SS, 8);                                                                            \
     }                                                                                                          \
     break
@@ -3771,7 +3789,7 @@ size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G)
     if (mfma_path_ok(M, N, K, S, G) || lut_path_ok(M, N, K, S, G))
         return static_cast<size_t>(M) * N * sizeof(unsigned long long);
     if (gemm_lut_path_ok(M, N, K, S, G)) {
-        const int ks = gemm_lut_ksplit(M, N, K);
+        const int ks = gemm_lut_plan(M, N, K, true).ksplit;
         return ks == 1 ? 0 : static_cast<size_t>(ks) * M * N * sizeof(float);
     }
     if (gemm_path_ok(M, N, K, S, G) && !rows32_path_ok(M, N, K, S, G))
@@ -3979,15 +3997,18 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         g.steps_per_group = G / kGemmBK;
         g.idx16 = idx_bytes == 2;
         g.ksplit = 1;
-        const int ks = gemm_lut_ksplit(M, N, K);
+        GemmLutPlan plan = gemm_lut_plan(M, N, K, true);
+        const int ks = plan.ksplit;
         const size_t need = ks > 1 ? static_cast<size_t>(ks) * M * N * sizeof(float) : 0;
         if (need && workspace && workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
             g.ksplit = ks;
             g.part = static_cast<float *>(workspace);
+        } else if (need) {
+            plan = gemm_lut_plan(M, N, K, false);      // no workspace for the parts: not split
         }
         if (env_switches().show_plan)
-            fprintf(stderr, "sbvr_hip table look-up prefill M=%d N=%d K=%d S=%d: ksplit=%d\n", M, N, K, S, g.ksplit);
-        hipError_t e = launch_gemm_lut(S, g, st);
+            fprintf(stderr, "sbvr_hip table look-up prefill M=%d N=%d K=%d S=%d: row blocks=%d ksplit=%d\n", M, N, K, S, plan.rb, g.ksplit);
+        hipError_t e = launch_gemm_lut(S, plan.rb, g, st);
         if (e == hipSuccess && g.ksplit > 1) {
             const size_t quads = (static_cast<size_t>(M) * N + 3) / 4;
             hipLaunchKernelGGL(sbvr_gemm_reduce_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, st,

@@ -304,9 +304,16 @@ def test_k_split_without_workspace_is_not_split(oracle):
     check(out, yd, yd1, parity.ROUNDING_DECODE, "unsplit launch without a workspace")
 
 
-@pytest.mark.parametrize("M", [64, 65, 128, 129, 192, 193, 256, 257, 384, 385, 513])
-@pytest.mark.parametrize("S", [2, 3, 4])
+@pytest.mark.parametrize("M,S", [(64, 4), (65, 2), (96, 3), (97, 4), (128, 2), (129, 4), (160, 3), (161, 4), (192, 2), (193, 4),
+                                 (224, 3), (225, 4), (256, 3), (257, 4), (513, 4)])
 def test_row_blocks_of_the_table_lookup_prefill(oracle, M, S):
-    """The row counts at which the prefill kernel's workgroups go from 2 to 4, 6 and 8 row blocks of 32, and from one
-    tile of rows to two and three; 16-bit indices and a bias at the odd ones."""
-    run_case(oracle, 260, 512, S, 128, M, 300 if M % 2 else 256, seed=1000 * S + M, bias=M % 2 == 1, expect=PREFILL)
+    """223 column tiles, so that the prefill kernel's workgroups take 2 to 8 row blocks of 32 as the rows grow, at the
+    edges of each, and several tiles of rows from 257; 16-bit indices and a bias at the odd ones."""
+    run_case(oracle, 57000, 256, S, 128, M, 300 if M % 2 else 256, seed=1000 * S + M, bias=M % 2 == 1, expect=PREFILL)
+
+
+@pytest.mark.parametrize("M", [64, 129, 300, 513])
+def test_two_row_blocks_where_tiles_are_few(oracle, M):
+    """One or two column tiles: two row blocks a workgroup whatever the number of rows, K split or not."""
+    run_case(oracle, 260, 512, 4, 128, M, 256, seed=M, expect=PREFILL)
+    run_case(oracle, 256, 4096, 3, 256, M, 256, seed=M + 1, expect=PREFILL_SPLIT)
