@@ -23,6 +23,15 @@ extern "C" {
 int sbvr_hip_encoder_group_mse_f16(const void *data, const void *points, float *mse, int groups, int G, int n, int P,
                                    void *stream);
 
+/* The candidate lines of one group's search (sbvr/core.py:368-403) and their errors in one launch.  data: the group,
+ * G fp16 values.  Lines 0 .. bs * ss * bases - 1: b[ib] + s[is] * base[ir, :] (fp16 product, fp16 sum), ir the fastest,
+ * ib the slowest; behind them steps^S lines whose coefficient q is axes[q, i_q], the last axis fastest.  base
+ * (bases, S), b (bs), s (ss), axes (S, steps): fp16.  lines (n, S) fp16 and mse (n) fp32 are written, mse as
+ * sbvr_hip_encoder_group_mse_f16 writes it for the line's subset sums (fp32 sums rounded to fp16 once).  2 <= S <= 6, G
+ * a multiple of 4 and at most 4096, at most 2^28 lines of either kind. */
+int sbvr_hip_encoder_candidates_f16(const void *data, int G, const void *base, int bases, const void *b, int bs, const void *s,
+                                    int ss, const void *axes, int steps, int S, void *lines, float *mse, void *stream);
+
 /* Activations to bit planes on the fly: x (M, K) fp16 -> bvr (K/32, M, S) uint32, bit k%32 of
  * bvr[k/32, m, j] = bit S-1-j of the selector of x[m, k] (point p of a line is the sum of the
  * coefficients j with bit S-1-j of p set, sbvr/core.py:345-351): the index of the first of the 2^S points of group

@@ -62,6 +62,91 @@ sbvr_encoder_group_mse_kernel(const uint16_t *__restrict__ data, const uint16_t 
         mse[static_cast<size_t>(b) * n + line] = sum / static_cast<float>(G);
 }
 
+// The candidate lines of one group's search, formed and measured in one launch: first the geometric families
+// b + s * base (reference sbvr/core.py:392-403; index (b, s, base), the last fastest; fp16 product, fp16 sum), then the
+// grid of S axes of `steps` values each (core.py:368-390; the last axis fastest).  A thread owns a candidate: its
+// coefficients go to `lines` as they are formed (the winner's are read back), its 2^S subset sums (fp32 sums rounded
+// to fp16 once) stay in registers, and its error follows as in the kernel above.  The order of a line's coefficients
+// does not change its points, so only the winner has to be sorted.  Bound by the vector ALU: three packed operations
+// per two points and value.  (Formed by torch, 2.6e5 to 4.6e5 lines of 4 coefficients were written, concatenated,
+// sorted, gathered and multiplied out to points before the kernel above read them: a 1024 x 4096 weight with groups of
+// 128 took 424-454 ms to encode, 294-307 ms with this launch.)
+struct CandidateArgs {
+    const uint16_t *data, *base, *b, *s, *axes;
+    uint16_t *lines;
+    float *mse;
+    int bases, ss, steps, family, n, G;
+};
+
+template <int S>
+__global__ void __launch_bounds__(kEncThreads)
+sbvr_encoder_candidates_kernel(const CandidateArgs a)
+{
+#pragma clang fp contract(off)
+    constexpr int P = 1 << S;
+    __shared__ __align__(16) uint16_t group[kEncMaxG];
+    for (int i = threadIdx.x; i < a.G; i += kEncThreads)
+        group[i] = a.data[i];
+    __syncthreads();
+    const int line = blockIdx.x * kEncThreads + threadIdx.x;
+    const int at = min(line, a.n - 1);
+    auto half_of = [](uint16_t v) __attribute__((always_inline)) -> _Float16 { return __builtin_bit_cast(_Float16, v); };
+    _Float16 c[S];
+    if (at < a.family) {
+        const int ir = at % a.bases, is = at / a.bases % a.ss, ib = at / a.bases / a.ss;
+        const _Float16 sv = half_of(a.s[is]), bv = half_of(a.b[ib]);
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            const _Float16 scaled = sv * half_of(a.base[ir * S + q]);
+            c[q] = bv + scaled;
+        }
+    } else {
+        int rest = at - a.family;
+#pragma unroll
+        for (int q = S - 1; q >= 0; --q) {
+            c[q] = half_of(a.axes[q * a.steps + rest % a.steps]);
+            rest /= a.steps;
+        }
+    }
+    float sums[P];
+    sums[0] = 0.f;
+#pragma unroll
+    for (int q = 0; q < S; ++q)
+#pragma unroll
+        for (int i = 0; i < (1 << q); ++i)
+            sums[(1 << q) + i] = sums[i] + static_cast<float>(c[q]);
+    v2h p[P / 2];
+#pragma unroll
+    for (int j = 0; j < P / 2; ++j)
+        p[j] = v2h{static_cast<_Float16>(sums[2 * j]), static_cast<_Float16>(sums[2 * j + 1])};
+
+    float sum = 0.f;
+    for (int g = 0; g < a.G; g += 4) {                        // (G is a multiple of 4)
+        const uint2 four = *reinterpret_cast<const uint2 *>(group + g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t pair = e < 2 ? four.x : four.y;
+            const _Float16 d = half_of(static_cast<uint16_t>(e & 1 ? pair >> 16 : pair));
+            const v2h dd = {d, d};
+            v2h best;
+#pragma unroll
+            for (int j = 0; j < P / 2; ++j) {
+                const v2h diff = dd - p[j];
+                const v2h sq = diff * diff;
+                best = j == 0 ? sq : __builtin_elementwise_min(best, sq);
+            }
+            const _Float16 m = best[0] < best[1] ? best[0] : best[1];
+            sum += static_cast<float>(m);
+        }
+    }
+    if (line < a.n) {
+#pragma unroll
+        for (int q = 0; q < S; ++q)
+            a.lines[static_cast<size_t>(line) * S + q] = __builtin_bit_cast(uint16_t, c[q]);
+        a.mse[line] = sum / static_cast<float>(a.G);
+    }
+}
+
 // Activations to bit planes on the fly: lane = one element x[m, k]; its selector is the first of the P
 // subset sums of its group's line that is nearest to it (fp16 difference and square, as the encoder chooses
 // selectors: sbvr/core.py:492-494), and the 64 lanes' selector bits become two words per plane by ballot
@@ -311,6 +396,34 @@ int sbvr_hip_encoder_group_mse_f16(const void *data, const void *points, float *
     case 64: hipLaunchKernelGGL(sbvr_encoder_group_mse_kernel<64>, grid, block, 0, st, d, p, mse, G, n); break;
     case 128: hipLaunchKernelGGL(sbvr_encoder_group_mse_kernel<128>, grid, block, 0, st, d, p, mse, G, n); break;
     default: hipLaunchKernelGGL(sbvr_encoder_group_mse_kernel<256>, grid, block, 0, st, d, p, mse, G, n); break;
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+int sbvr_hip_encoder_candidates_f16(const void *data, int G, const void *base, int bases, const void *b, int bs, const void *s, int ss,
+                                    const void *axes, int steps, int S, void *lines, float *mse, void *stream)
+{
+    if (!data || !base || !b || !s || !axes || !lines || !mse || G <= 0 || bases <= 0 || bs <= 0 || ss <= 0 || steps <= 0)
+        return -1;
+    if (S < 2 || S > 6 || G > kEncMaxG || G % 4 != 0)
+        return -2;
+    const long family = static_cast<long>(bases) * bs * ss;
+    long grid_lines = 1;
+    for (int q = 0; q < S && grid_lines <= (1L << 28); ++q)
+        grid_lines *= steps;
+    if (static_cast<double>(bases) * bs * ss > (1 << 28) || grid_lines > (1L << 28))
+        return -2;
+    const CandidateArgs a{static_cast<const uint16_t *>(data), static_cast<const uint16_t *>(base), static_cast<const uint16_t *>(b),
+                          static_cast<const uint16_t *>(s), static_cast<const uint16_t *>(axes), static_cast<uint16_t *>(lines), mse,
+                          bases, ss, steps, static_cast<int>(family), static_cast<int>(family + grid_lines), G};
+    const dim3 grid(static_cast<unsigned>((a.n + kEncThreads - 1) / kEncThreads)), block(kEncThreads);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    switch (S) {
+    case 2: hipLaunchKernelGGL(sbvr_encoder_candidates_kernel<2>, grid, block, 0, st, a); break;
+    case 3: hipLaunchKernelGGL(sbvr_encoder_candidates_kernel<3>, grid, block, 0, st, a); break;
+    case 4: hipLaunchKernelGGL(sbvr_encoder_candidates_kernel<4>, grid, block, 0, st, a); break;
+    case 5: hipLaunchKernelGGL(sbvr_encoder_candidates_kernel<5>, grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL(sbvr_encoder_candidates_kernel<6>, grid, block, 0, st, a); break;
     }
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }

@@ -72,6 +72,7 @@ class GroupEncoder:
         self.combs = layout.bin_combs(self.S, dtype, device)                 # (2^S, S)
         self.table = torch.zeros((max_lines, self.S), dtype=dtype, device=device)
         conf.coeff_cache = self.table
+        self._fixed = {}                          # _fixed_space, plain and extended
 
     # -- candidate lines ------------------------------------------------------
 
@@ -202,6 +203,68 @@ class GroupEncoder:
                     break
         return best, best_line, best_sel
 
+    def _search_new_fused(self, data, extended):
+        """``search(candidate_lines(data, extended), data, ...)`` for a group on a GPU with the candidates formed and
+        measured in one launch: (best error, line with its coefficients in order, points' selectors), or None where
+        the launch does not cover the case.  The bounds of the scales and axes come to the host in one copy, from the
+        expressions of ``candidate_lines`` (which waits for each of them by itself)."""
+        from . import hip
+        c, S = self.conf, self.S
+        if not (data.is_cuda and hip.encoder_candidates_supported(data.dtype, data.shape[0], S) and data.is_contiguous()):
+            return None
+        hi, lo, avg = torch.max(data), torch.min(data), torch.mean(data)
+        q95 = torch.quantile(data.to(torch.float), 0.95)
+        s_hi, s_lo = (hi - lo) * 1.1, 2 * q95
+        s_step = (s_hi - s_lo) / c.s_search_num
+        if extended:
+            s_step = s_step / c.extend_ratio
+        edges = torch.linspace(lo, hi, S + 1, device=data.device, dtype=data.dtype)
+        margin = edges[:S].abs() * 0.8
+        bounds = torch.cat((torch.stack((avg.float(), s_lo + s_step, s_hi + s_step, s_step)),
+                            (edges[:S] - margin).float(), (edges[1:] + margin).float())).tolist()
+        mean, s_from, s_to, s_step = bounds[:4]
+        # (beside a mean that moves the offsets, and values that are not finite: the general path)
+        if not all(map(math.isfinite, bounds)) or abs(mean) * 2.0 / S >= 0.29 or s_step == 0 or (s_to - s_from) / s_step <= 0:
+            return None
+        kw = dict(device=data.device, dtype=data.dtype)
+        s_list = torch.arange(s_from, s_to, s_step, **kw)
+        base, b_list, per_dim = self._fixed_space(extended, kw)
+        axes = torch.empty((S, per_dim + 1), **kw)
+        for i in range(S):
+            torch.linspace(bounds[4 + i], bounds[4 + S + i], per_dim + 1, out=axes[i])
+        n = base.shape[0] * b_list.shape[0] * s_list.shape[0] + (per_dim + 1) ** S
+        if s_list.shape[0] == 0 or n > c.search_batch_size or n >= 1 << 28:
+            return None
+        lines, mse = hip.encoder_candidates(data, base, b_list, s_list, axes)
+        at = mse.argmin()
+        line = lines[at].view(1, S)
+        line = torch.gather(line, dim=1, index=torch.sort(line.abs(), dim=1)[1])
+        sel = self._selectors(data.view(1, -1), line @ self.combs.T)[0]
+        return mse[at].item(), line[0], sel
+
+    def _fixed_space(self, extended, kw):
+        """What of the candidates is the same for every group: the scaled bases of the families, the offsets, and the
+        values per axis of the grid (see ``candidate_lines``)."""
+        if extended not in self._fixed:
+            c = self.conf
+            r0_lo, r0_hi = math.pi / 6, 0.94
+            r1_lo, r1_hi = 1.06, math.pi * 2 / 3
+            ratio = c.extend_ratio if extended else 1.0
+            r0_step = (r0_hi - r0_lo) / (c.r_search_num / 2) / ratio
+            r1_step = (r1_hi - r1_lo) / (c.r_search_num / 2) / ratio
+            b_step = (0.3 - -0.3) / c.b_search_num / ratio
+            r_list = torch.cat((-torch.arange(r0_lo + r0_step, r0_hi + r0_step, r0_step, **kw),
+                                -torch.arange(r1_lo + r1_step, r1_hi + r1_step, r1_step, **kw)))
+            base = r_list.unsqueeze(1) ** torch.arange(self.S, device=r_list.device).unsqueeze(0)
+            sums = base @ self.combs.T
+            spread = sums.max(dim=1)[0] - sums.min(dim=1)[0]
+            budget = c.r_search_num * c.b_search_num * c.s_search_num * 1.4
+            if extended:
+                budget *= c.search_extend_ratio ** 3
+            self._fixed[extended] = ((base / spread.unsqueeze(1)).contiguous(), torch.arange(-0.3, 0.3, b_step, **kw),
+                                     int(budget ** (1 / self.S)))
+        return self._fixed[extended]
+
     # -- per-group policy -----------------------------------------------------
 
     def encode_group(self, data):
@@ -220,10 +283,13 @@ class GroupEncoder:
                 return line_idx, sel
         if c.num_coeff_cache_lines < self.table.shape[0]:
             hit_rate = c.cache_hits / c.group_idx
-            lines, _, _, _, _ = self.candidate_lines(data, hit_rate > 0.6 or warming)
-            new_mse, new_at, new_sel = self.search(lines, data, c.acceptable_mse)
+            found = self._search_new_fused(data, hit_rate > 0.6 or warming)
+            if found is None:
+                lines, _, _, _, _ = self.candidate_lines(data, hit_rate > 0.6 or warming)
+                new_mse, new_at, new_sel = self.search(lines, data, c.acceptable_mse)
+                found = new_mse, lines[new_at] if new_mse < best else None, new_sel
+            new_mse, cand, new_sel = found
             if new_mse < best:
-                cand = lines[new_at]
                 same = (self.table - cand.unsqueeze(0)).abs().sum(-1) < cand.abs().sum(-1) * 0.0001
                 if same.any():
                     line_idx = same.nonzero(as_tuple=True)[0][0]

@@ -78,6 +78,7 @@ def _load():
     lib.sbvr_hip_dec_head_argmax_embed_f16.argtypes = [vp, vp, vp, ctypes.c_float, vp, i, i, vp, vp, vp, vp, i, vp, vp, i,
                                                        vp, vp, vp, vp, vp]
     lib.sbvr_hip_encoder_group_mse_f16.argtypes = [vp, vp, vp, i, i, i, i, vp]
+    lib.sbvr_hip_encoder_candidates_f16.argtypes = [vp, i, vp, i, vp, i, vp, i, vp, i, i, vp, vp, vp]
     lib.sbvr_hip_online_encode_f16.argtypes = [vp, vp, vp, i, i, i, i, vp]
     lib.sbvr_hip_online_encode_lines_f16.argtypes = [vp, vp, vp, vp, i, i, i, i, i, vp]
     lib.sbvr_hip_decode_weight.argtypes = [vp, vp, i, vp, vp, i, i, i, i, i, i, i, vp]
@@ -594,6 +595,31 @@ def encoder_group_mse(data, points):
 
 def encoder_group_mse_supported(dtype, G, P):
     return dtype == torch.float16 and P in (2, 4, 8, 16, 32, 64, 128, 256)
+
+
+def encoder_candidates(data, base, b, s, axes):
+    """The candidate lines of one group's search and their errors (``sbvr_hip_encoder_candidates_f16``): data (G),
+    base (bases, S), b, s, axes (S, steps), all fp16 -> lines (n, S) fp16, coefficients as formed, and mse (n) fp32."""
+    dev = data.device
+    for t, name, dim in ((data, "data", 1), (base, "base", 2), (b, "b", 1), (s, "s", 1), (axes, "axes", 2)):
+        _want(t, name, torch.float16, dim, dev)
+    S, steps = axes.shape
+    if base.shape[1] != S:
+        raise ValueError(f"base must be (bases, {S}), got {tuple(base.shape)}")
+    n = base.shape[0] * b.shape[0] * s.shape[0] + steps ** S
+    lines = torch.empty((n, S), dtype=torch.float16, device=dev)
+    mse = torch.empty(n, dtype=torch.float32, device=dev)
+    with torch.cuda.device(dev):
+        rc = _load().sbvr_hip_encoder_candidates_f16(data.data_ptr(), data.shape[0], base.data_ptr(), base.shape[0], b.data_ptr(),
+                                                     b.shape[0], s.data_ptr(), s.shape[0], axes.data_ptr(), steps, S,
+                                                     lines.data_ptr(), mse.data_ptr(), _stream())
+    if rc != 0:
+        raise SbvrHipError(f"sbvr_hip_encoder_candidates_f16: error {rc} (G={data.shape[0]} S={S} n={n})")
+    return lines, mse
+
+
+def encoder_candidates_supported(dtype, G, S):
+    return dtype == torch.float16 and 2 <= S <= 6 and G % 4 == 0 and G <= 4096
 
 
 def online_encode(x, points, bvr_len):

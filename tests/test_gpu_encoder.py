@@ -149,3 +149,29 @@ def test_real_4096_encoding_and_config1(oracle, golden):
     w = made.weight().numpy().astype(np.float64)
     dense = x.numpy().astype(np.float64) @ w.T
     assert np.mean((got - dense) ** 2) < 0.02 * np.mean(dense ** 2)
+
+
+@pytest.mark.parametrize("S,G,scale,shift", [(2, 128, 0.02, 0.0), (3, 256, 0.02, 0.001), (4, 128, 0.02, 0.0), (4, 256, 1.0, 0.1),
+                                             (5, 64, 0.3, 0.0), (6, 128, 0.02, 0.0), (4, 4, 0.02, 0.0), (4, 128, 1.0, 3.0)])
+@pytest.mark.parametrize("extended", [False, True])
+def test_fused_candidates_equal_the_general_search(S, G, scale, shift, extended):
+    """The search of new lines with the candidates formed in the launch against the one over candidate_lines(): the
+    same best error, line and selectors, bit for bit; the last case has a mean that the launch leaves to the other."""
+    from sbvr.encoder import EncoderConfig, GroupEncoder
+    dev = torch.device("cuda:0")
+    conf = EncoderConfig(num_sums=S, bvr_len=G, search_batch_size=1 << 24)
+    enc = GroupEncoder(conf, torch.float16, dev, max_lines=16)
+    gen = torch.Generator().manual_seed(S * 1000 + G)
+    taken = 0
+    for i in range(12):
+        data = (torch.randn(G, generator=gen) * scale * (1 + i % 3) + shift).to(torch.float16).to(dev)
+        found = enc._search_new_fused(data, extended)
+        if found is None:
+            continue
+        taken += 1
+        lines = enc.candidate_lines(data, extended)[0]
+        mse, at, sel = enc.search(lines, data, conf.acceptable_mse)
+        assert found[0] == mse, f"group {i}: error {found[0]} beside {mse}"
+        assert torch.equal(found[1], lines[at]), f"group {i}: line {found[1].tolist()} beside {lines[at].tolist()}"
+        assert torch.equal(found[2], sel), f"group {i}: selectors"
+    assert taken == (0 if shift >= 3 else 12)
