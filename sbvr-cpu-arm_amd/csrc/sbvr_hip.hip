@@ -2319,12 +2319,12 @@ hipError_t launch_gemm(int S, const GemmArgs &a, hipStream_t st)
 // ------------------------------------------- MFMA prefill with the weights decoded by table look-up
 //
 // The prefill contraction with the decode of sbvr_gemm_rows32_lut_kernel: no producer and consumer waves and no
-// weight tile in LDS.  A workgroup of 8 waves owns 256 rows x 256 columns of the output; wave w owns columns
-// 32w .. 32w+31 for all 256 rows (8 row blocks of 32: 128 accumulator registers a lane).  Per step of 64 elements
+// weight tile in LDS.  A workgroup of 8 waves owns RB row blocks of 32 x 256 columns of the output; wave w owns columns
+// 32w .. 32w+31 for all its rows (8 row blocks: 128 accumulator registers a lane).  Per step of 64 elements
 // of K a lane (column j, half h) decodes its word 2i + h of column j by table look-up straight into the B operands
-// of four MFMAs (16 registers), and the wave runs them against the 8 row blocks: 32 MFMAs per 32 weights decoded
-// per lane, so the decode (about 170 VALU instructions a step) hides behind the matrix pipe (32 x 32 clocks).
-// The activations of a step, 256 rows x 64 elements, are shared by the 8 waves through LDS, stored in the element
+// of four MFMAs (16 registers), and the wave runs them against the row blocks: 4 RB MFMAs of 32 clocks per 32
+// weights decoded per lane (about 170 VALU instructions a step).
+// The activations of a step, 32 RB rows x 64 elements, are shared by the 8 waves through LDS, stored in the element
 // order the MFMAs want (see sbvr_gemm_rows32_lut_kernel: that permutation is done once, by the thread that
 // brings a (row, word) in, not once per wave): rows 144 bytes apart, two buffers, one barrier per step.  The loads
 // of the step after the next one's (activations, plane words) are in flight while a step is computed.
