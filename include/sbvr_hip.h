@@ -109,7 +109,7 @@ size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G);
  *                   same S; with a workspace and few output tiles, K is split
  *                   across workgroups.  With 2, 3 or 4 planes and K and G multiples
  *                   of 128 it is the kernel that decodes by table look-up in
- *                   registers (256 x 256 output tiles, the weights never in LDS),
+ *                   registers (output tiles of 64 to 256 rows x 256, the weights never in LDS),
  *                   otherwise the one that decodes weight tiles into LDS; same
  *                   results up to the order of the fp32 additions;
  *   portable kernel everything else (one thread per output), and with flags bit 0.
