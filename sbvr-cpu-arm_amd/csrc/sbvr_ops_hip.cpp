@@ -87,6 +87,13 @@ torch::Tensor workspace(size_t nbytes, const torch::Tensor &like, hipStream_t st
     return it->second;
 }
 
+// Elements per coefficient group: bvr_len where it is given, otherwise what `groups` rows of indices leave to each.
+int64_t group_length(int64_t bvr_len, int64_t elements, int64_t groups, const char *name)
+{
+    TORCH_CHECK(groups > 0, name, " has no groups");            // (an integer division by 0 would end the process)
+    return bvr_len > 0 ? bvr_len : elements / groups;
+}
+
 struct LinearShape {
     int64_t M, N, K, S, G, L;
     int ib;
@@ -106,7 +113,7 @@ LinearShape linear_shape(int64_t M, int64_t K, const torch::Tensor &bvr, const t
     s.ib = idx_bytes(coeff_idx, s.L, "coeff_idx", like);
     TORCH_CHECK(bvr.size(0) * 32 == K, "x has K=", K, " but bvr holds ", bvr.size(0) * 32, " columns");
     TORCH_CHECK(coeff_idx.size(1) == s.N && coeff_cache.size(1) == s.S, "coeff_idx / coeff_cache shapes do not match bvr");
-    s.G = bvr_len > 0 ? bvr_len : K / coeff_idx.size(0);
+    s.G = group_length(bvr_len, K, coeff_idx.size(0), "coeff_idx");
     TORCH_CHECK(s.G * coeff_idx.size(0) == K, "coeff_idx has ", coeff_idx.size(0), " groups, K=", K, ", bvr_len=", s.G);
     return s;
 }
@@ -166,6 +173,7 @@ torch::Tensor sbvr_linear_forward(torch::Tensor x, const torch::Tensor &bvr, con
 {
     TORCH_CHECK(x.is_cuda(), "x must be on a GPU (got ", x.device(), "); there is no CPU path");
     TORCH_CHECK(x.dim() >= 1, "x must have at least one dimension");
+    TORCH_CHECK(k_padded > 0, "the weight has no columns");
     if (x.scalar_type() != torch::kFloat16)
         x = x.to(torch::kFloat16);
     if (x.size(-1) != k_padded)
@@ -241,7 +249,7 @@ torch::Tensor sbvr_mm_T(const torch::Tensor &l_bvr, const torch::Tensor &l_coeff
     TORCH_CHECK(l_coeff_idx.size(1) == M && r_coeff_idx.size(1) == N && l_coeff_idx.size(0) == r_coeff_idx.size(0) &&
                     l_coeff_cache.size(1) == Sl && r_coeff_cache.size(1) == Sr,
                 "index / table shapes do not match the bit planes");
-    const int64_t G = bvr_len > 0 ? bvr_len : K / l_coeff_idx.size(0);
+    const int64_t G = group_length(bvr_len, K, l_coeff_idx.size(0), "l_coeff_idx");
     TORCH_CHECK(G * l_coeff_idx.size(0) == K, "coeff_idx has ", l_coeff_idx.size(0), " groups, K=", K);
     const DeviceGuard guard(l_bvr.device());
     auto out = at::empty({M, N}, l_coeff_cache.options());
@@ -308,7 +316,7 @@ torch::Tensor sbvr_row_deq_mm_T(const torch::Tensor &l_w, const torch::Tensor &r
     const int64_t M = l_w.size(0), K = l_w.size(1), N = r_bvr.size(0) * 32, S = r_bvr.size(2), L = r_coeff_cache.size(0);
     const int ib = idx_bytes(r_coeff_idx, L, "r_coeff_idx", l_w);
     TORCH_CHECK(r_bvr.size(1) == K && r_coeff_idx.size(1) == K && r_coeff_cache.size(1) == S, "operand shapes do not match");
-    const int64_t G = bvr_len > 0 ? bvr_len : N / r_coeff_idx.size(0);
+    const int64_t G = group_length(bvr_len, N, r_coeff_idx.size(0), "r_coeff_idx");
     TORCH_CHECK(G * r_coeff_idx.size(0) == N, "r_coeff_idx has ", r_coeff_idx.size(0), " groups, N=", N);
     const DeviceGuard guard(l_w.device());
     auto out = at::empty({M, N}, l_w.options());
