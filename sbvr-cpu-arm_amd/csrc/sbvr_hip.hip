@@ -2636,7 +2636,19 @@ int current_cus()
 
 // -------------------------------------------- trans=True and both-encoded forms
 
-constexpr int kMmDecodeMinN = 8192;      // columns from which one encoded left row takes the decode kernel (sbvr_hip_mm_T_ws)
+// One encoded left row of up to four planes at the decode kernel's shapes: whether mm_ops.hip's kernel takes it.  That
+// one does not split K across workgroups, so it is the faster one only while its workgroups (16 columns each) find a
+// CU each, and then for short K, or for longer K where there are columns enough for most of the CUs; with one left
+// plane, and with three on the right, the decode kernel's launch has the least to do and keeps all but the shortest K.
+// us, decode kernel and mm_ops.hip's, by (left planes, right planes): 512 x 14336 (4, 4) 4.9 and 7.4, (2, 3) 4.3 and
+// 8.1; 600 x 28672 (4, 8) 8.2 and 16.3; 2048 x 14336 (2, 4) 6.7 and 7.6; 5120 x 14336 (4, 4) 12.6 and 12.8; against
+// 1024 x 1024 (4, 4) 4.0 and 3.2; 2048 x 2048 4.3 and 3.7; 4096 x 4096 6.5 and 4.5; 3072 x 10240 (4, 8) 13.2 and 8.5.
+// (Of 1920 shapes, 256 to 8176 columns, K 512 to 28672, 1 to 4 by 2 to 8 planes, the rule's choice is more than 4 %
+// slower than the decode kernel at one, by 5 %.)
+bool mm_one_row_matrix(int N, int K, int Sl, int Sr, int cus)
+{
+    return N <= 16 * cus && (K <= 1024 || (Sl >= 2 && Sr != 3 && (K <= 2048 || (N > 10 * cus && K <= 10240))));
+}
 
 // One thread per output; the lanes of a wave share k and differ in n, so the
 // plane words and indices are wave-uniform broadcasts.
@@ -4290,10 +4302,9 @@ int sbvr_hip_mm_T_ws(const uint32_t *l_bvr, const void *l_coeff_idx, int l_idx_b
     const uint16_t *lc = static_cast<const uint16_t *>(l_coeff_cache), *rc = static_cast<const uint16_t *>(r_coeff_cache);
     const uint16_t *b = static_cast<const uint16_t *>(bias);
     uint16_t *o = static_cast<uint16_t *>(out);
-    // One left row of up to four planes against many columns, at the decode kernel's shapes: the decode kernel with
-    // the left operand's planes as its batch rows.  (us, 4 x 4 planes, this kernel against mm_ops.hip's, which takes
-    // the rest: 4096 -> 14336 8.9 and 9.6; 14336 -> 4096 9.7 and 9.1; 4096 -> 4096 7.0 and 5.0; 4096 -> 1024 4.5 and 4.4.)
-    if (M == 1 && N >= kMmDecodeMinN && Sl <= 4 && !env_switches().popc_q && mfma_path_ok(Sl, N, K, Sr, G) &&
+    // One left row of up to four planes at the decode kernel's shapes: the decode kernel with the left operand's planes
+    // as its batch rows, unless the kernel below is the faster one.
+    if (M == 1 && Sl <= 4 && !mm_one_row_matrix(N, K, Sl, Sr, current_cus()) && !env_switches().popc_q && mfma_path_ok(Sl, N, K, Sr, G) &&
         (l_idx_bytes == 2 || Ll <= 256) && (r_idx_bytes == 2 || Lr <= 256) &&
         reinterpret_cast<uintptr_t>(r_bvr) % 16 == 0 && reinterpret_cast<uintptr_t>(r_coeff_cache) % 16 == 0 &&
         reinterpret_cast<uintptr_t>(l_bvr) % 4 == 0 && reinterpret_cast<uintptr_t>(l_coeff_cache) % 2 == 0) {

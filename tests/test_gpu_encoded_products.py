@@ -70,3 +70,32 @@ def test_online_encode_lines(S, G, M, K):
     assert torch.equal(bvr.view(torch.int32), hip.online_encode(x, points, G).view(torch.int32))
     assert idx.dtype == (torch.uint8 if K // G <= 256 else torch.uint16)
     assert torch.equal(idx.to(torch.int64), torch.arange(K // G, device="cuda:0").view(-1, 1).expand(-1, M))
+
+
+@pytest.mark.parametrize("N,K,Sl,Sr,decode_kernel", [
+    (512, 14336, 4, 4, True), (600, 4096, 2, 3, True), (1024, 14336, 1, 8, True), (2048, 2048, 3, 3, True),     # few columns, long K
+    (4112, 1024, 4, 4, True), (8192, 4096, 2, 2, True), (8200, 14336, 4, 6, True),                              # more columns than CUs x 16
+    (4096, 1024, 1, 3, False), (640, 2048, 4, 2, False), (4096, 4096, 2, 8, False), (3072, 10240, 4, 4, False)])
+def test_one_left_row_takes_the_kernel_that_is_faster_for_it(oracle, N, K, Sl, Sr, decode_kernel):
+    """One left row of up to four planes: where the columns leave the chip idle or outnumber its workgroups the decode
+    kernel (which splits K), otherwise the one that does not; the same bits on every call, the accumulators zero again."""
+    import sbvr
+    from sbvr import hip
+    dev = torch.device("cuda:0")
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the rule's columns are those of 256 CUs")
+    rng = np.random.default_rng(N + K)
+    left, right = _enc(rng, 1, K, Sl, 128, 16, oracle), _enc(rng, N, K, Sr, 128, 256, oracle)
+    none = torch.zeros(0, dtype=torch.float16, device=dev)
+    # (a launch of another kernel first: the report is of the last launch that makes one)
+    w, wi, wc = _dev(*_enc(rng, 64, 256, 4, 128, 16, oracle))
+    sbvr._sbvr_linear_f16(torch.zeros((40, 256), dtype=torch.float16, device=dev), w, wi, wc)
+    assert hip.last_kernel() != hip.KERNEL_DECODE
+    d = _dev(*left, *right)
+    y = sbvr._sbvr_mm_T(*d, none, bvr_len=128)
+    assert (hip.last_kernel() == hip.KERNEL_DECODE) == decode_kernel
+    _, yd = oracle.C.mm_T(*left, *right, 128)
+    rms = float(np.sqrt(np.mean(yd ** 2)))
+    assert (np.abs(y.cpu().numpy().astype(np.float64) - yd) / (np.maximum(np.abs(yd), rms) * 2.0 ** -10)).max() <= 2.0
+    for _ in range(3):                 # (words that a launch left behind would be in the next one's sums)
+        assert torch.equal(y, sbvr._sbvr_mm_T(*d, none, bvr_len=128))
