@@ -17,12 +17,30 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <stdexcept>
+#include <string>
 #include <vector>
 
 #include "../../include/sbvr_hip.h"
 #include "../../include/sbvr_hip_encoder.h"
 
 namespace {
+
+// Arguments that an operator does not take, as opposed to a device or an allocation that failed.
+struct Refused : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+
+// The library reported an error of the device.
+struct LaunchFailed : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+
+#define SBVR_WANT(cond, ...)                              \
+    do {                                                  \
+        if (!(cond))                                      \
+            throw Refused(c10::str(__VA_ARGS__));         \
+    } while (0)
 
 using DeviceGuard = c10::hip::HIPGuardMasqueradingAsCUDA;
 
@@ -33,12 +51,12 @@ hipStream_t current_stream()
 
 void want(const torch::Tensor &t, const char *name, c10::ScalarType dtype, int64_t dim, const torch::Tensor *like)
 {
-    TORCH_CHECK(t.is_cuda(), name, " must be on a GPU (got ", t.device(), "); there is no CPU path");
-    TORCH_CHECK(t.scalar_type() == dtype, name, " must have dtype ", dtype, ", got ", t.scalar_type());
-    TORCH_CHECK(t.dim() == dim, name, " must have ", dim, " dimensions, got ", t.dim());
-    TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
+    SBVR_WANT(t.is_cuda(), name, " must be on a GPU (got ", t.device(), "); there is no CPU path");
+    SBVR_WANT(t.scalar_type() == dtype, name, " must have dtype ", dtype, ", got ", t.scalar_type());
+    SBVR_WANT(t.dim() == dim, name, " must have ", dim, " dimensions, got ", t.dim());
+    SBVR_WANT(t.is_contiguous(), name, " must be contiguous");
     if (like)
-        TORCH_CHECK(t.device() == like->device(), name, " is on ", t.device(), ", expected ", like->device());
+        SBVR_WANT(t.device() == like->device(), name, " is on ", t.device(), ", expected ", like->device());
 }
 
 // uint8 indices for up to 256 lines, uint16 beyond (sbvr_kernel.cu:931-932)
@@ -63,7 +81,24 @@ const void *bias_ptr(const Bias &bias, int64_t n, const torch::Tensor &like)
 
 void check(int rc)
 {
-    TORCH_CHECK(rc == SBVR_HIP_OK, "libsbvr_hip: error ", rc, ": ", sbvr_hip_last_error());
+    if (rc == SBVR_HIP_OK)
+        return;
+    const std::string message = c10::str("libsbvr_hip: error ", rc, ": ", sbvr_hip_last_error());
+    if (rc == SBVR_HIP_ELAUNCH)
+        throw LaunchFailed(message);
+    throw Refused(message);
+}
+
+// (the entry points of sbvr_hip_encoder.h leave no message)
+template <typename... Args>
+void check_encoder(int rc, const char *what, const Args &...shape)
+{
+    if (rc == SBVR_HIP_OK)
+        return;
+    const std::string message = c10::str(what, ": error ", rc, shape...);
+    if (rc == SBVR_HIP_ELAUNCH)
+        throw LaunchFailed(message);
+    throw Refused(message);
 }
 
 // Zero-initialised split-K accumulators per (device, stream), grown on demand; the kernels
@@ -90,7 +125,7 @@ torch::Tensor workspace(size_t nbytes, const torch::Tensor &like, hipStream_t st
 // Elements per coefficient group: bvr_len where it is given, otherwise what `groups` rows of indices leave to each.
 int64_t group_length(int64_t bvr_len, int64_t elements, int64_t groups, const char *name)
 {
-    TORCH_CHECK(groups > 0, name, " has no groups");            // (an integer division by 0 would end the process)
+    SBVR_WANT(groups > 0, name, " has no groups");            // (an integer division by 0 would end the process)
     return bvr_len > 0 ? bvr_len : elements / groups;
 }
 
@@ -111,10 +146,10 @@ LinearShape linear_shape(int64_t M, int64_t K, const torch::Tensor &bvr, const t
     s.S = bvr.size(2);
     s.L = coeff_cache.size(0);
     s.ib = idx_bytes(coeff_idx, s.L, "coeff_idx", like);
-    TORCH_CHECK(bvr.size(0) * 32 == K, "x has K=", K, " but bvr holds ", bvr.size(0) * 32, " columns");
-    TORCH_CHECK(coeff_idx.size(1) == s.N && coeff_cache.size(1) == s.S, "coeff_idx / coeff_cache shapes do not match bvr");
+    SBVR_WANT(bvr.size(0) * 32 == K, "x has K=", K, " but bvr holds ", bvr.size(0) * 32, " columns");
+    SBVR_WANT(coeff_idx.size(1) == s.N && coeff_cache.size(1) == s.S, "coeff_idx / coeff_cache shapes do not match bvr");
     s.G = group_length(bvr_len, K, coeff_idx.size(0), "coeff_idx");
-    TORCH_CHECK(s.G * coeff_idx.size(0) == K, "coeff_idx has ", coeff_idx.size(0), " groups, K=", K, ", bvr_len=", s.G);
+    SBVR_WANT(s.G * coeff_idx.size(0) == K, "coeff_idx has ", coeff_idx.size(0), " groups, K=", K, ", bvr_len=", s.G);
     return s;
 }
 
@@ -156,7 +191,7 @@ torch::Tensor sbvr_linear_f16(const torch::Tensor &x, const torch::Tensor &bvr, 
     if (out_opt.has_value() && out_opt->defined()) {
         out = *out_opt;
         want(out, "out", torch::kFloat16, 2, &x);
-        TORCH_CHECK(out.size(0) == s.M && out.size(1) == s.N, "out has the wrong shape");
+        SBVR_WANT(out.size(0) == s.M && out.size(1) == s.N, "out has the wrong shape");
     } else {
         out = at::empty({s.M, s.N}, x.options());
     }
@@ -171,9 +206,9 @@ torch::Tensor sbvr_linear_forward(torch::Tensor x, const torch::Tensor &bvr, con
                                   const torch::Tensor &coeff_cache, const Bias &bias, int64_t bvr_len, int64_t k_padded,
                                   int64_t out_features)
 {
-    TORCH_CHECK(x.is_cuda(), "x must be on a GPU (got ", x.device(), "); there is no CPU path");
-    TORCH_CHECK(x.dim() >= 1, "x must have at least one dimension");
-    TORCH_CHECK(k_padded > 0, "the weight has no columns");
+    SBVR_WANT(x.is_cuda(), "x must be on a GPU (got ", x.device(), "); there is no CPU path");
+    SBVR_WANT(x.dim() >= 1, "x must have at least one dimension");
+    SBVR_WANT(k_padded > 0, "the weight has no columns");
     if (x.scalar_type() != torch::kFloat16)
         x = x.to(torch::kFloat16);
     if (x.size(-1) != k_padded)
@@ -193,7 +228,7 @@ torch::Tensor sbvr_linear_f16_swiglu(const torch::Tensor &gate_up, const torch::
                                      const torch::Tensor &coeff_cache, const Bias &bias, int64_t bvr_len)
 {
     want(gate_up, "gate_up", torch::kFloat16, 2, nullptr);
-    TORCH_CHECK(gate_up.size(1) % 2 == 0, "gate_up must have an even number of columns");
+    SBVR_WANT(gate_up.size(1) % 2 == 0, "gate_up must have an even number of columns");
     const LinearShape s = linear_shape(gate_up.size(0), gate_up.size(1) / 2, bvr, coeff_idx, coeff_cache, bvr_len, gate_up);
     const DeviceGuard guard(gate_up.device());
     hipStream_t stream = current_stream();
@@ -215,7 +250,7 @@ torch::Tensor sbvr_linear_f16_add_rmsnorm(torch::Tensor x, torch::Tensor delta, 
     want(delta, "delta", torch::kFloat16, 2, &x);
     want(x_out, "x_out", torch::kFloat16, 2, &x);
     want(norm_weight, "norm_weight", torch::kFloat16, 1, &x);
-    TORCH_CHECK(x.size(0) == 1 && delta.sizes() == x.sizes() && x_out.sizes() == x.sizes() &&
+    SBVR_WANT(x.size(0) == 1 && delta.sizes() == x.sizes() && x_out.sizes() == x.sizes() &&
                     norm_weight.size(0) == x.size(1),
                 "x, delta and x_out must be (1, K) and norm_weight (K)");
     const LinearShape s = linear_shape(1, x.size(1), bvr, coeff_idx, coeff_cache, bvr_len, x);
@@ -244,13 +279,13 @@ torch::Tensor sbvr_mm_T(const torch::Tensor &l_bvr, const torch::Tensor &l_coeff
     want(r_coeff_cache, "r_coeff_cache", torch::kFloat16, 2, &l_bvr);
     const int64_t M = l_bvr.size(1), N = r_bvr.size(1), K = l_bvr.size(0) * 32;
     const int64_t Sl = l_bvr.size(2), Sr = r_bvr.size(2), Ll = l_coeff_cache.size(0), Lr = r_coeff_cache.size(0);
-    TORCH_CHECK(l_bvr.size(0) == r_bvr.size(0), "operands disagree on K: ", K, " vs ", r_bvr.size(0) * 32);
+    SBVR_WANT(l_bvr.size(0) == r_bvr.size(0), "operands disagree on K: ", K, " vs ", r_bvr.size(0) * 32);
     const int lib = idx_bytes(l_coeff_idx, Ll, "l_coeff_idx", l_bvr), rib = idx_bytes(r_coeff_idx, Lr, "r_coeff_idx", l_bvr);
-    TORCH_CHECK(l_coeff_idx.size(1) == M && r_coeff_idx.size(1) == N && l_coeff_idx.size(0) == r_coeff_idx.size(0) &&
+    SBVR_WANT(l_coeff_idx.size(1) == M && r_coeff_idx.size(1) == N && l_coeff_idx.size(0) == r_coeff_idx.size(0) &&
                     l_coeff_cache.size(1) == Sl && r_coeff_cache.size(1) == Sr,
                 "index / table shapes do not match the bit planes");
     const int64_t G = group_length(bvr_len, K, l_coeff_idx.size(0), "l_coeff_idx");
-    TORCH_CHECK(G * l_coeff_idx.size(0) == K, "coeff_idx has ", l_coeff_idx.size(0), " groups, K=", K);
+    SBVR_WANT(G * l_coeff_idx.size(0) == K, "coeff_idx has ", l_coeff_idx.size(0), " groups, K=", K);
     const DeviceGuard guard(l_bvr.device());
     auto out = at::empty({M, N}, l_coeff_cache.options());
     hipStream_t stream = current_stream();
@@ -272,13 +307,13 @@ std::tuple<torch::Tensor, torch::Tensor> sbvr_online_encode_lines(const torch::T
     want(x, "x", torch::kFloat16, 2, nullptr);
     want(lines, "lines", torch::kFloat16, 2, &x);
     const int64_t M = x.size(0), K = x.size(1), groups = lines.size(0), S = lines.size(1);
-    TORCH_CHECK(K == groups * bvr_len, "lines must be (K / bvr_len, S), got ", lines.sizes(), " for K=", K, ", bvr_len=", bvr_len);
+    SBVR_WANT(K == groups * bvr_len, "lines must be (K / bvr_len, S), got ", lines.sizes(), " for K=", K, ", bvr_len=", bvr_len);
     const DeviceGuard guard(x.device());
     auto bvr = at::empty({K / 32, M, S}, x.options().dtype(torch::kUInt32));
     auto idx = at::empty({groups, M}, x.options().dtype(groups <= 256 ? torch::kUInt8 : torch::kUInt16));
     const int rc = sbvr_hip_online_encode_lines_f16(x.data_ptr(), lines.data_ptr(), static_cast<uint32_t *>(bvr.data_ptr()), idx.data_ptr(),
                                                     groups <= 256 ? 1 : 2, M, K, bvr_len, S, current_stream());
-    TORCH_CHECK(rc == 0, "sbvr_hip_online_encode_lines_f16: error ", rc, " (M=", M, " K=", K, " bvr_len=", bvr_len, " S=", S, ")");
+    check_encoder(rc, "sbvr_hip_online_encode_lines_f16", " (M=", M, " K=", K, " bvr_len=", bvr_len, " S=", S, ")");
     return {bvr, idx};
 }
 
@@ -288,10 +323,10 @@ torch::Tensor sbvr_decode_weight(const torch::Tensor &bvr, const torch::Tensor &
 {
     want(bvr, "bvr", torch::kUInt32, 3, nullptr);
     want(coeff_cache, "coeff_cache", torch::kFloat16, 2, &bvr);
-    TORCH_CHECK(coeff_idx.scalar_type() == torch::kUInt8 || coeff_idx.scalar_type() == torch::kUInt16, "coeff_idx must be uint8 or uint16");
+    SBVR_WANT(coeff_idx.scalar_type() == torch::kUInt8 || coeff_idx.scalar_type() == torch::kUInt16, "coeff_idx must be uint8 or uint16");
     want(coeff_idx, "coeff_idx", coeff_idx.scalar_type(), 2, &bvr);
     const int64_t K = bvr.size(0) * 32, N = bvr.size(1), S = bvr.size(2), L = coeff_cache.size(0);
-    TORCH_CHECK(coeff_idx.size(0) * bvr_len == K && coeff_idx.size(1) == N && coeff_cache.size(1) == S,
+    SBVR_WANT(coeff_idx.size(0) * bvr_len == K && coeff_idx.size(1) == N && coeff_cache.size(1) == S,
                 "coeff_idx / coeff_cache shapes do not match bvr");
     const int type = dtype == torch::kFloat32 ? 2 : (dtype == torch::kBFloat16 ? 1 : 0);
     const DeviceGuard guard(bvr.device());
@@ -299,7 +334,7 @@ torch::Tensor sbvr_decode_weight(const torch::Tensor &bvr, const torch::Tensor &
     const int rc = sbvr_hip_decode_weight(static_cast<const uint32_t *>(bvr.data_ptr()), coeff_idx.data_ptr(),
                                           static_cast<int>(coeff_idx.element_size()), coeff_cache.data_ptr(), out.data_ptr(), type, N, K,
                                           cols, S, bvr_len, L, current_stream());
-    TORCH_CHECK(rc == 0, "sbvr_hip_decode_weight: error ", rc, " (N=", N, " K=", K, " cols=", cols, " S=", S, " bvr_len=", bvr_len, ")");
+    check_encoder(rc, "sbvr_hip_decode_weight", " (N=", N, " K=", K, " cols=", cols, " S=", S, " bvr_len=", bvr_len, ")");
     return out.scalar_type() == dtype ? out : out.to(dtype);
 }
 
@@ -315,9 +350,9 @@ torch::Tensor sbvr_row_deq_mm_T(const torch::Tensor &l_w, const torch::Tensor &r
     want(r_coeff_cache, "r_coeff_cache", torch::kFloat16, 2, &l_w);
     const int64_t M = l_w.size(0), K = l_w.size(1), N = r_bvr.size(0) * 32, S = r_bvr.size(2), L = r_coeff_cache.size(0);
     const int ib = idx_bytes(r_coeff_idx, L, "r_coeff_idx", l_w);
-    TORCH_CHECK(r_bvr.size(1) == K && r_coeff_idx.size(1) == K && r_coeff_cache.size(1) == S, "operand shapes do not match");
+    SBVR_WANT(r_bvr.size(1) == K && r_coeff_idx.size(1) == K && r_coeff_cache.size(1) == S, "operand shapes do not match");
     const int64_t G = group_length(bvr_len, N, r_coeff_idx.size(0), "r_coeff_idx");
-    TORCH_CHECK(G * r_coeff_idx.size(0) == N, "r_coeff_idx has ", r_coeff_idx.size(0), " groups, N=", N);
+    SBVR_WANT(G * r_coeff_idx.size(0) == N, "r_coeff_idx has ", r_coeff_idx.size(0), " groups, N=", N);
     const DeviceGuard guard(l_w.device());
     auto out = at::empty({M, N}, l_w.options());
     hipStream_t stream = current_stream();
@@ -334,6 +369,8 @@ torch::Tensor sbvr_row_deq_mm_T(const torch::Tensor &l_w, const torch::Tensor &r
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     namespace py = pybind11;
+    py::register_exception<Refused>(m, "Refused", PyExc_RuntimeError);
+    py::register_exception<LaunchFailed>(m, "LaunchFailed", PyExc_RuntimeError);
     m.def("_sbvr_hip_init", &sbvr_hip_init_current, "Checks that the current device is a gfx950 part");
     m.def("_sbvr_cuda_init", &sbvr_hip_init_current, "Alias of _sbvr_hip_init under the reference's name");
     m.def("_sbvr_mm_T", &sbvr_mm_T, "SBVR x SBVR^T, both operands encoded", py::arg("l_bvr"), py::arg("l_coeff_idx"),

@@ -98,7 +98,7 @@ def _ext():
     """The PyTorch extension over the same library (csrc/sbvr_ops_hip.cpp), or False where it is not built or another
     copy of the library is asked for.  The products of encoded operands, the on-the-fly encoding and the dense decode
     go through it: the same checks and the same launch, 4 to 6 us a call where ctypes and the checks in Python take 16.
-    What it refuses goes through the checks below for their error.  (The fp16 linears below stay on ctypes: they share
+    (The fp16 linears below stay on ctypes: they share
     this module's workspace, and SBVRLinear.forward does not come this way.)"""
     global _extension
     if _extension is None:
@@ -110,6 +110,21 @@ def _ext():
             except ImportError:
                 pass
     return _extension
+
+
+def _native(name, *args):
+    """The operator ``name`` of the extension over ``args``; None where it is not there or does not take them: the
+    checks behind the call then say why, or take them after all.  A launch that failed is an error here and now, and
+    what torch raises (out of memory) is passed on: neither is tried a second time."""
+    ext = _ext()
+    if not ext:
+        return None
+    try:
+        return getattr(ext, name)(*args)
+    except (ext.Refused, TypeError):
+        return None
+    except ext.LaunchFailed as exc:
+        raise SbvrHipError(str(exc)) from None
 
 
 KERNEL_PORTABLE, KERNEL_DECODE, KERNEL_ROWS32, KERNEL_PREFILL, KERNEL_PREFILL_SPLIT = 1, 2, 3, 4, 5
@@ -312,12 +327,10 @@ def _sbvr_row_deq_mm_T(l_w, r_bvr, r_coeff_idx, r_coeff_cache, bias, use_shfl=0,
     """fp16 ``l_w`` (M, K) against a ``trans=True`` weight: ``r_bvr`` (N/32, K, S),
     ``r_coeff_idx`` (N/G, K) (sbvr_ops.cpp:79-120).  ``use_shfl`` selected between
     equivalent CUDA kernels in the reference and is ignored."""
-    ext = _ext()
-    if ext and (bvr_len is None or bvr_len > 0):
-        try:
-            return ext._sbvr_row_deq_mm_T(l_w, r_bvr, r_coeff_idx, r_coeff_cache, bias, 0, bvr_len or 0)
-        except (RuntimeError, TypeError):
-            pass
+    if bvr_len is None or bvr_len > 0:
+        out = _native("_sbvr_row_deq_mm_T", l_w, r_bvr, r_coeff_idx, r_coeff_cache, bias, 0, bvr_len or 0)
+        if out is not None:
+            return out
     lib = _load()
     dev = l_w.device
     _want(l_w, "l_w", torch.float16, 2)
@@ -345,12 +358,10 @@ def _sbvr_row_deq_mm_T(l_w, r_bvr, r_coeff_idx, r_coeff_cache, bias, use_shfl=0,
 def _sbvr_mm_T(l_bvr, l_coeff_idx, l_coeff_cache, r_bvr, r_coeff_idx, r_coeff_cache, bias, bvr_len=None):
     """Both operands encoded, default uint32 layout: ``l_bvr`` (K/32, M, Sl),
     ``r_bvr`` (K/32, N, Sr) (sbvr_ops.cpp:35-76).  Returns fp16 (M, N)."""
-    ext = _ext()
-    if ext and (bvr_len is None or bvr_len > 0):
-        try:
-            return ext._sbvr_mm_T(l_bvr, l_coeff_idx, l_coeff_cache, r_bvr, r_coeff_idx, r_coeff_cache, bias, bvr_len or 0)
-        except (RuntimeError, TypeError):
-            pass
+    if bvr_len is None or bvr_len > 0:
+        out = _native("_sbvr_mm_T", l_bvr, l_coeff_idx, l_coeff_cache, r_bvr, r_coeff_idx, r_coeff_cache, bias, bvr_len or 0)
+        if out is not None:
+            return out
     lib = _load()
     dev = l_bvr.device
     _want(l_bvr, "l_bvr", torch.uint32, 3)
@@ -642,12 +653,9 @@ def online_encode(x, points, bvr_len):
 def online_encode_lines(x, lines, bvr_len):
     """``online_encode`` from one line of input coefficients per group of K, lines (K / bvr_len, S) fp16: returns
     the left operand's (bvr, coeff_idx), coeff_idx (K / bvr_len, M) holding every group's own number."""
-    ext = _ext()
-    if ext:
-        try:
-            return ext._online_encode_lines(x, lines, bvr_len)
-        except (RuntimeError, TypeError):
-            pass
+    made = _native("_online_encode_lines", x, lines, bvr_len)
+    if made is not None:
+        return made
     _want(x, "x", torch.float16, 2)
     _want(lines, "lines", torch.float16, 2, x.device)
     M, K = x.shape
@@ -670,12 +678,9 @@ _DECODE_TYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
 def decode_weight(bvr, coeff_idx, coeff_cache, bvr_len, cols, dtype):
     """The dense (N, cols) weight of a default-layout encoding (cols: without the padding of K), every element its
     coefficients' fp32 sum rounded to fp16 once, in ``dtype`` (sbvr/core.py:926-949)."""
-    ext = _ext()
-    if ext:
-        try:
-            return ext._decode_weight(bvr, coeff_idx, coeff_cache, bvr_len, cols, dtype)
-        except (RuntimeError, TypeError):
-            pass
+    out = _native("_decode_weight", bvr, coeff_idx, coeff_cache, bvr_len, cols, dtype)
+    if out is not None:
+        return out
     dev = bvr.device
     _want(bvr, "bvr", torch.uint32, 3)
     _want(coeff_idx, "coeff_idx", (torch.uint8, torch.uint16), 2, dev)
