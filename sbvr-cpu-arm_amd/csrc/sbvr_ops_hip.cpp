@@ -103,23 +103,35 @@ void check_encoder(int rc, const char *what, const Args &...shape)
 
 // Zero-initialised split-K accumulators per (device, stream), grown on demand; the kernels
 // leave the part that must be zero zeroed.  A buffer that is outgrown is kept until the process
-// ends: a HIP graph captured earlier on that stream still holds its address.
-torch::Tensor workspace(size_t nbytes, const torch::Tensor &like, hipStream_t stream)
+// ends: a HIP graph captured earlier on that stream still holds its address.  The only pool of the process: the
+// functions of sbvr/hip.py ask for theirs here, so that a stream that one operator has warmed is warm for all.
+torch::Tensor workspace(size_t nbytes, c10::Device device, hipStream_t stream)
 {
     static std::mutex mu;
     static std::map<std::tuple<int, hipStream_t>, torch::Tensor> held;
     static std::vector<torch::Tensor> outgrown;
-    std::lock_guard<std::mutex> lock(mu);
-    auto key = std::make_tuple(static_cast<int>(like.get_device()), stream);
-    auto it = held.find(key);
-    if (it == held.end() || static_cast<size_t>(it->second.numel()) < nbytes) {
-        if (it != held.end())
-            outgrown.push_back(it->second);
-        const int64_t size = static_cast<int64_t>(nbytes > (1u << 20) ? nbytes : (1u << 20));
-        held[key] = torch::zeros({size}, torch::dtype(torch::kUInt8).device(like.device()));
-        it = held.find(key);
+    const auto key = std::make_tuple(static_cast<int>(device.index()), stream);
+    auto enough = [&]() -> torch::Tensor {
+        const auto it = held.find(key);
+        return it != held.end() && static_cast<size_t>(it->second.numel()) >= nbytes ? it->second : torch::Tensor();
+    };
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        torch::Tensor have = enough();
+        if (have.defined())
+            return have;
     }
-    return it->second;
+    // (allocated without the lock: torch may run Python on the way)
+    const int64_t size = static_cast<int64_t>(nbytes > (1u << 20) ? nbytes : (1u << 20));
+    torch::Tensor made = torch::zeros({size}, torch::dtype(torch::kUInt8).device(device));
+    std::lock_guard<std::mutex> lock(mu);
+    torch::Tensor have = enough();           // (another thread on this stream was faster)
+    if (have.defined())
+        return have;
+    if (held.count(key))
+        outgrown.push_back(held[key]);
+    held[key] = made;
+    return made;
 }
 
 // Elements per coefficient group: bvr_len where it is given, otherwise what `groups` rows of indices leave to each.
@@ -169,7 +181,7 @@ void launch_linear(const torch::Tensor &x, const torch::Tensor &bvr, const torch
 {
     hipStream_t stream = current_stream();
     const size_t need = sbvr_hip_linear_f16_workspace(s.M, s.N, s.K, s.S, s.G);
-    torch::Tensor ws = need ? workspace(need, x, stream) : torch::Tensor();
+    torch::Tensor ws = need ? workspace(need, x.device(), stream) : torch::Tensor();
     check(sbvr_hip_linear_f16(x.data_ptr(), static_cast<const uint32_t *>(bvr.data_ptr()), coeff_idx.data_ptr(), s.ib,
                               coeff_cache.data_ptr(), bias_ptr(bias, s.N, x), out.data_ptr(), s.M, s.N, s.K, s.S, s.G,
                               s.L, need ? ws.data_ptr() : nullptr, need ? ws.numel() : 0, flags, stream));
@@ -234,7 +246,7 @@ torch::Tensor sbvr_linear_f16_swiglu(const torch::Tensor &gate_up, const torch::
     hipStream_t stream = current_stream();
     auto out = torch::empty({s.M, s.N}, torch::dtype(torch::kFloat16).device(gate_up.device()));
     const size_t need = sbvr_hip_linear_f16_workspace(s.M, s.N, s.K, s.S, s.G);
-    torch::Tensor ws = need ? workspace(need, gate_up, stream) : torch::Tensor();
+    torch::Tensor ws = need ? workspace(need, gate_up.device(), stream) : torch::Tensor();
     check(sbvr_hip_linear_f16_swiglu(gate_up.data_ptr(), static_cast<const uint32_t *>(bvr.data_ptr()), coeff_idx.data_ptr(),
                                      s.ib, coeff_cache.data_ptr(), bias_ptr(bias, s.N, gate_up), out.data_ptr(), s.M, s.N,
                                      s.K, s.S, s.G, s.L, need ? ws.data_ptr() : nullptr, need ? ws.numel() : 0, stream));
@@ -258,7 +270,7 @@ torch::Tensor sbvr_linear_f16_add_rmsnorm(torch::Tensor x, torch::Tensor delta, 
     hipStream_t stream = current_stream();
     auto out = torch::empty({1, s.N}, torch::dtype(torch::kFloat16).device(x.device()));
     const size_t need = sbvr_hip_linear_f16_workspace(1, s.N, s.K, s.S, s.G);
-    torch::Tensor ws = need ? workspace(need, x, stream) : torch::Tensor();
+    torch::Tensor ws = need ? workspace(need, x.device(), stream) : torch::Tensor();
     check(sbvr_hip_linear_f16_add_rmsnorm(x.data_ptr(), delta.data_ptr(), norm_weight.data_ptr(), static_cast<float>(eps),
                                           x_out.data_ptr(), static_cast<const uint32_t *>(bvr.data_ptr()),
                                           coeff_idx.data_ptr(), s.ib, coeff_cache.data_ptr(), bias_ptr(bias, s.N, x),
@@ -292,7 +304,7 @@ torch::Tensor sbvr_mm_T(const torch::Tensor &l_bvr, const torch::Tensor &l_coeff
     const size_t need = sbvr_hip_mm_T_workspace(static_cast<int>(M), static_cast<int>(N));
     torch::Tensor ws;                    // (no split of K for this call: no workspace, nothing allocated)
     if (need)
-        ws = workspace(need, l_bvr, stream);
+        ws = workspace(need, l_bvr.device(), stream);
     check(sbvr_hip_mm_T_ws(static_cast<const uint32_t *>(l_bvr.data_ptr()), l_coeff_idx.data_ptr(), lib,
                            l_coeff_cache.data_ptr(), static_cast<const uint32_t *>(r_bvr.data_ptr()), r_coeff_idx.data_ptr(),
                            rib, r_coeff_cache.data_ptr(), bias_ptr(bias, N, l_bvr), out.data_ptr(), M, N, K, Sl, Sr, G, Ll,
@@ -359,11 +371,19 @@ torch::Tensor sbvr_row_deq_mm_T(const torch::Tensor &l_w, const torch::Tensor &r
     const size_t need = sbvr_hip_row_deq_mm_T_workspace(static_cast<int>(M), static_cast<int>(N));
     torch::Tensor ws;                    // (no split of K for this call: no workspace, nothing allocated)
     if (need)
-        ws = workspace(need, l_w, stream);
+        ws = workspace(need, l_w.device(), stream);
     check(sbvr_hip_row_deq_mm_T_ws(l_w.data_ptr(), static_cast<const uint32_t *>(r_bvr.data_ptr()), r_coeff_idx.data_ptr(), ib,
                                    r_coeff_cache.data_ptr(), bias_ptr(bias, N, l_w), out.data_ptr(), M, N, K, S, G, L,
                                    need ? ws.data_ptr() : nullptr, need, stream));
     return out;
+}
+
+// The workspace of the current stream of a device, for launches that are made through the C ABI.
+torch::Tensor workspace_of_current_stream(int64_t nbytes, int64_t device)
+{
+    const c10::Device dev(c10::DeviceType::CUDA, static_cast<c10::DeviceIndex>(device));
+    const DeviceGuard guard(dev);
+    return workspace(static_cast<size_t>(nbytes), dev, current_stream());
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
@@ -388,6 +408,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
           py::arg("lines"), py::arg("bvr_len"));
     m.def("_decode_weight", &sbvr_decode_weight, "the dense weight of a default-layout encoding", py::arg("bvr"),
           py::arg("coeff_idx"), py::arg("coeff_cache"), py::arg("bvr_len"), py::arg("cols"), py::arg("dtype"));
+    m.def("_workspace", &workspace_of_current_stream, "the split-K workspace of the device's current stream", py::arg("nbytes"),
+          py::arg("device"));
     m.def("last_kernel", &sbvr_hip_last_kernel, "which kernel the last linear call of this thread launched");
     m.def("_sbvr_linear_f16_swiglu", &sbvr_linear_f16_swiglu, "the linear of silu(gate) * up, one row", py::arg("gate_up"),
           py::arg("bvr"), py::arg("coeff_idx"), py::arg("coeff_cache"), py::arg("bias") = py::none(),

@@ -14,7 +14,7 @@ import torch
 
 _LIB_NAME = "libsbvr_hip.so"
 _lib = None
-_workspaces = {}
+_workspaces = {}      # the latest workspace per (device index, stream)
 _outgrown = []        # workspaces that were replaced by larger ones (HIP graphs captured earlier still point at them)
 
 
@@ -98,8 +98,7 @@ def _ext():
     """The PyTorch extension over the same library (csrc/sbvr_ops_hip.cpp), or False where it is not built or another
     copy of the library is asked for.  The products of encoded operands, the on-the-fly encoding and the dense decode
     go through it: the same checks and the same launch, 4 to 6 us a call where ctypes and the checks in Python take 16.
-    (The fp16 linears below stay on ctypes: they share
-    this module's workspace, and SBVRLinear.forward does not come this way.)"""
+    (The fp16 linears below stay on ctypes; SBVRLinear.forward does not come this way.)"""
     global _extension
     if _extension is None:
         _extension = False
@@ -193,8 +192,13 @@ def _stream():
 def _workspace(nbytes, device):
     """Zero-initialised scratch per (device, stream); grown on demand.  The
     kernels leave the part that must be zero zeroed.  A buffer that is outgrown
-    stays allocated: a HIP graph recorded earlier on the stream keeps its address."""
+    stays allocated: a HIP graph recorded earlier on the stream keeps its address.
+    The pool is the extension's, one for every operator of the process."""
     key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    ext = _ext()
+    if ext:
+        ws = _workspaces[key] = ext._workspace(nbytes, device.index)
+        return ws
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         if ws is not None:

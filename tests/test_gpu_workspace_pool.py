@@ -1,0 +1,54 @@
+"""The split-K workspace: one pool for the operators of the extension and for those that go through ctypes."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda:0")
+
+
+def _encoded(rows, K, S=4, G=128, L=16, seed=0):
+    from sbvr import synth
+    return [t.to(DEV) for t in synth.random_encoding(rows, K, S, G, L, seed=seed)]
+
+
+def test_a_stream_warmed_by_one_operator_is_warm_for_all():
+    """After the functional linear (ctypes) the products of encoded operands (extension) and SBVRLinear find their
+    accumulators on that stream: no allocation but their outputs', inside a capture as well, and right replays."""
+    import sbvr
+    from sbvr import _sbvr_hip_ops as ops, hip
+    N, K = 1024, 2048
+    w = _encoded(N, K, seed=1)
+    l = _encoded(1, K, seed=2)
+    t = _encoded(K, N, seed=3)                                 # (the transposed weight)
+    x = torch.randn((2, K), generator=torch.Generator().manual_seed(4)).to(torch.float16).to(DEV)
+    none = torch.zeros(0, dtype=torch.float16, device=DEV)
+    lib = hip._load()
+    assert lib.sbvr_hip_row_deq_mm_T_workspace(2, N) > 0 and lib.sbvr_hip_mm_T_workspace(1, N) > 0
+    linear = sbvr.SBVRLinear(K, N, *w, 128)
+    want = [sbvr._sbvr_row_deq_mm_T(x, *t, none, bvr_len=128), sbvr._sbvr_mm_T(*l, *w, none, bvr_len=128), linear(x)]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        assert lib.sbvr_hip_linear_f16_workspace(2, N, K, 4, 128) > 0
+        sbvr._sbvr_linear_f16(x, *w, bvr_len=128)              # warms the stream
+        ws = hip._workspaces[(DEV.index, side.cuda_stream)]
+        assert ops._workspace(1, DEV.index).data_ptr() == ws.data_ptr()
+        side.synchronize()
+        before = torch.cuda.memory_allocated()
+        got = [sbvr._sbvr_row_deq_mm_T(x, *t, none, bvr_len=128), sbvr._sbvr_mm_T(*l, *w, none, bvr_len=128), linear(x)]
+        assert torch.cuda.memory_allocated() - before <= sum((2 * y.numel() + 511) // 512 * 512 for y in got)
+        side.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        got = [sbvr._sbvr_row_deq_mm_T(x, *t, none, bvr_len=128), sbvr._sbvr_mm_T(*l, *w, none, bvr_len=128), linear(x)]
+        assert ops._workspace(1, DEV.index).data_ptr() == ws.data_ptr()
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        with torch.cuda.stream(side):                          # eager work on the same workspace in between
+            assert torch.equal(sbvr._sbvr_row_deq_mm_T(x, *t, none, bvr_len=128), want[0])
+        side.synchronize()
+    assert int(ws.count_nonzero()) == 0
