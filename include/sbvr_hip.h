@@ -66,10 +66,10 @@ int sbvr_hip_init(int device);
  * none).  The workspace must be zero-filled once after allocation; every call
  * leaves it zero-filled.  Calls that share a workspace must not overlap in
  * time.  Where the decode kernel splits K across workgroups the workspace is
- * required; for the 32-row kernel with few columns and the prefill kernel with
- * few output tiles it is optional: without it that launch is not split along K,
- * which is slower but gives the same result up to the order of the fp32
- * additions. */
+ * required; for the 32-row kernel with few columns and the prefill kernel where
+ * it is faster with K in parts (at most 96 MiB of partial results with 2, 3 or 4
+ * planes) it is optional: without it that launch is not split along K, which is
+ * slower but gives the same result up to the order of the fp32 additions. */
 size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G);
 
 /*
@@ -106,8 +106,8 @@ size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G);
  *                   5..16 rows of shapes the decode kernel does not cover (N < 16,
  *                   K or G not a multiple of 128);
  *   prefill kernel  M > 32 (or 17..32 with flags bit 1), K and G multiples of 64,
- *                   same S; with a workspace and few output tiles, K is split
- *                   across workgroups.  With 2, 3 or 4 planes and K and G multiples
+ *                   same S; with a workspace, and where that is the faster, K is
+ *                   split across workgroups.  With 2, 3 or 4 planes and K and G multiples
  *                   of 128 it is the kernel that decodes by table look-up in
  *                   registers (output tiles of 64 to 256 rows x 256, the weights never in LDS),
  *                   otherwise the one that decodes weight tiles into LDS; same

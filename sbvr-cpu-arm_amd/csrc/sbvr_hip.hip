@@ -2542,6 +2542,11 @@ bool gemm_lut_path_ok(int M, int N, int K, int S, int G)
 // last turn counts half (8192 -> 28672: 1.31 turns take the time of 1.70, 3.5 turns that of 3.68).
 // Against tiles of 256 rows throughout, 4 planes: 4096 -> 6144, 600 rows 86.5 -> 53.0 us (240 workgroups of 4 row blocks
 // for 144 of 7), 128 rows 30.6 -> 25.7; 4096 -> 4096, 192 rows 36.3 -> 26.0; 8192 -> 28672, 600 rows 472 -> 362.
+// The partial results take at most kGemmLutMaxParts bytes (384 tiles of 256 x 256): the bindings keep a workspace of the
+// largest size asked for, and beyond that a split gains nothing (8192 columns, K 28672, 768 rows: 429 us in 8 parts,
+// 201 MB, and 432 in 2).
+constexpr double kGemmLutMaxParts = 96. * 1024 * 1024;
+
 struct GemmLutPlan {
     int rb, ksplit;
 };
@@ -2555,7 +2560,8 @@ GemmLutPlan gemm_lut_plan(int M, int N, int K, bool may_split)
         const int tiles = (blocks + most - 1) / most;
         const int rb = max(2, (blocks + tiles - 1) / tiles);
         for (int ks = 1; ks <= 16; ks *= 2) {
-            if (ks > 1 && (!may_split || N % 4 || steps % (ks * 2) || steps / ks < 16))
+            if (ks > 1 && (!may_split || N % 4 || steps % (ks * 2) || steps / ks < 16 ||
+                           4. * ks * static_cast<double>(M) * N > kGemmLutMaxParts))
                 break;
             const double turns = static_cast<double>(columns) * tiles * ks / kGemmSplitCus;
             const double busy = turns <= 1. ? 1. : (ceil(turns) + turns) / 2.;

@@ -17,6 +17,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <algorithm>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -101,9 +102,10 @@ void check_encoder(int rc, const char *what, const Args &...shape)
     throw Refused(message);
 }
 
-// Zero-initialised split-K accumulators per (device, stream), grown on demand; the kernels
-// leave the part that must be zero zeroed.  A buffer that is outgrown is kept until the process
-// ends: a HIP graph captured earlier on that stream still holds its address.  The only pool of the process: the
+// Zero-initialised split-K accumulators per (device, stream), grown on demand to twice their size at least; the
+// kernels leave the part that must be zero zeroed.  A buffer that is outgrown is kept until the process
+// ends: a HIP graph captured earlier on that stream still holds its address (all of them together are smaller than
+// the one in use).  The only pool of the process: the
 // functions of sbvr/hip.py ask for theirs here, so that a stream that one operator has warmed is warm for all.
 torch::Tensor workspace(size_t nbytes, c10::Device device, hipStream_t stream)
 {
@@ -115,15 +117,17 @@ torch::Tensor workspace(size_t nbytes, c10::Device device, hipStream_t stream)
         const auto it = held.find(key);
         return it != held.end() && static_cast<size_t>(it->second.numel()) >= nbytes ? it->second : torch::Tensor();
     };
+    size_t size = std::max(nbytes, static_cast<size_t>(1) << 20);
     {
         std::lock_guard<std::mutex> lock(mu);
         torch::Tensor have = enough();
         if (have.defined())
             return have;
+        if (held.count(key))
+            size = std::max(size, 2 * static_cast<size_t>(held[key].numel()));
     }
     // (allocated without the lock: torch may run Python on the way)
-    const int64_t size = static_cast<int64_t>(nbytes > (1u << 20) ? nbytes : (1u << 20));
-    torch::Tensor made = torch::zeros({size}, torch::dtype(torch::kUInt8).device(device));
+    torch::Tensor made = torch::zeros({static_cast<int64_t>(size)}, torch::dtype(torch::kUInt8).device(device));
     std::lock_guard<std::mutex> lock(mu);
     torch::Tensor have = enough();           // (another thread on this stream was faster)
     if (have.defined())

@@ -190,7 +190,7 @@ def _stream():
 
 
 def _workspace(nbytes, device):
-    """Zero-initialised scratch per (device, stream); grown on demand.  The
+    """Zero-initialised scratch per (device, stream); grown on demand to twice its size at least.  The
     kernels leave the part that must be zero zeroed.  A buffer that is outgrown
     stays allocated: a HIP graph recorded earlier on the stream keeps its address.
     The pool is the extension's, one for every operator of the process."""
@@ -201,9 +201,11 @@ def _workspace(nbytes, device):
         return ws
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
+        size = max(nbytes, 1 << 20)
         if ws is not None:
             _outgrown.append(ws)
-        ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+            size = max(size, 2 * ws.numel())
+        ws = torch.zeros(size, dtype=torch.uint8, device=device)
         _workspaces[key] = ws
     return ws
 

@@ -183,6 +183,21 @@ def test_workspace_sizes_follow_the_split_predicates():
     assert lib.sbvr_hip_row_deq_mm_T_workspace(2048, 14336) == 0      # prefill-sized: the columns fill the device
 
 
+def test_the_parts_of_a_prefill_stay_within_their_bound():
+    """K is split into parts of at most 96 MiB together, whatever the row count (the bindings keep the largest workspace
+    that was asked for)."""
+    from sbvr import hip
+    lib = hip._load()
+    split = 0
+    for N, K in ((512, 28672), (1024, 4096), (4096, 14336), (6144, 4096), (8192, 28672), (28672, 8192), (28672, 28672)):
+        for S in (2, 3, 4):
+            for M in list(range(33, 4200, 61)) + [768, 1024, 1500, 2048, 10000, 65536]:
+                need = lib.sbvr_hip_linear_f16_workspace(M, N, K, S, 128)
+                assert need <= 96 << 20, (M, N, K, S, need)
+                split += need > 0
+    assert split > 100
+
+
 def test_decode_plans_respect_the_launch_bounds():
     """Every launch shape the planners pick for up to 16 rows stays within the waves its kernel
     instance is compiled for (a launch beyond them fails), over a grid of shapes and device sizes."""

@@ -52,3 +52,17 @@ def test_a_stream_warmed_by_one_operator_is_warm_for_all():
             assert torch.equal(sbvr._sbvr_row_deq_mm_T(x, *t, none, bvr_len=128), want[0])
         side.synchronize()
     assert int(ws.count_nonzero()) == 0
+
+
+def test_growing_requests_hold_little_more_than_the_largest():
+    """Rising requests on one stream: the buffers that were outgrown (kept for graphs that point at them) and the one
+    in use together stay below four times the largest request."""
+    from sbvr import _sbvr_hip_ops as ops, hip
+    with torch.cuda.stream(torch.cuda.Stream()):
+        sizes = {}
+        for mib in range(2, 26):
+            for ws in (ops._workspace(mib << 20, DEV.index), hip._workspace(mib << 20, DEV)):
+                assert ws.numel() >= mib << 20 and ws.data_ptr() % 16 == 0
+                sizes[ws.data_ptr()] = ws.numel()
+        assert int(ws.count_nonzero()) == 0
+        assert sum(sizes.values()) <= 4 * (25 << 20)
