@@ -209,9 +209,12 @@ hipError_t launch_rt(int RT, int W, const MmArgs &a, hipStream_t st)
 
 }  // namespace
 
+// (at most 65535 blocks of left rows, of 64 (row, plane) pairs each where there are that many: the grid's y)
 bool mm_T_mfma_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r_bvr, const void *r_cache)
 {
-    return K % kMmSub == 0 && G % kMmSub == 0 && Sl <= 16 && (Sr == 2 || Sr == 3 || Sr == 4 || Sr == 6 || Sr == 8) &&
+    if (Sl > 16 || (static_cast<long>(M) + 64 / Sl - 1) / (64 / Sl) > 65535)
+        return false;
+    return K % kMmSub == 0 && G % kMmSub == 0 && (Sr == 2 || Sr == 3 || Sr == 4 || Sr == 6 || Sr == 8) &&
            static_cast<double>(M) * Sl * (K / 32) < 2147483648.0 && static_cast<double>(N) * Sr * (K / 32) < 2147483648.0 &&
            reinterpret_cast<uintptr_t>(r_bvr) % 16 == 0 && reinterpret_cast<uintptr_t>(r_cache) % 16 == 0;
 }
@@ -233,8 +236,6 @@ hipError_t launch_mm_T_mfma(int Sr, int G, MmArgs a, int cus, hipStream_t st)
         RT /= 2;
     a.m_per_wg = m_per_wg(RT);
     const int W = RT == 4 || wgs(RT) >= 2L * cus ? 8 : 16;
-    if ((a.M + a.m_per_wg - 1) / a.m_per_wg > 65535)
-        return hipErrorInvalidConfiguration;
     switch (Sr) {
     case 2: return launch_rt<2>(RT, W, a, st);
     case 3: return launch_rt<3>(RT, W, a, st);

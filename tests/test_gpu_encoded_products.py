@@ -99,3 +99,21 @@ def test_one_left_row_takes_the_kernel_that_is_faster_for_it(oracle, N, K, Sl, S
     assert (np.abs(y.cpu().numpy().astype(np.float64) - yd) / (np.maximum(np.abs(yd), rms) * 2.0 ** -10)).max() <= 2.0
     for _ in range(3):                 # (words that a launch left behind would be in the next one's sums)
         assert torch.equal(y, sbvr._sbvr_mm_T(*d, none, bvr_len=128))
+
+
+@pytest.mark.parametrize("M", [262140, 262141])
+def test_left_rows_beyond_the_grid_go_on_to_the_portable_kernel(oracle, M):
+    """16 left planes: 65535 blocks of four rows still fit the grid of the matrix-core kernel, one row more does not."""
+    import sbvr
+    K, N, Sl, Sr = 128, 16, 16, 2
+    rng = np.random.default_rng(M)
+    lb = rng.integers(0, 1 << 32, size=(K // 32, M, Sl), dtype=np.uint32)
+    li = rng.integers(0, 5, size=(1, M)).astype(np.uint8)
+    lc = (rng.standard_normal((5, Sl)) * 0.05).astype(np.float16)
+    right = _enc(rng, N, K, Sr, 128, 7, oracle)
+    none = torch.zeros(0, dtype=torch.float16, device="cuda:0")
+    y = sbvr._sbvr_mm_T(*_dev(lb, li, lc, *right), none, bvr_len=128).cpu().numpy()
+    some = np.r_[0:40, M // 2:M // 2 + 40, M - 40:M]
+    _, yd = oracle.C.mm_T(np.ascontiguousarray(lb[:, some]), np.ascontiguousarray(li[:, some]), lc, *right, 128)
+    rms = float(np.sqrt(np.mean(yd ** 2)))
+    assert (np.abs(y[some].astype(np.float64) - yd) / (np.maximum(np.abs(yd), rms) * 2.0 ** -10)).max() <= 2.0
