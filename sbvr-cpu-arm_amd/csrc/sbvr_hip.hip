@@ -4348,7 +4348,7 @@ int sbvr_hip_mm_T_ws(const uint32_t *l_bvr, const void *l_coeff_idx, int l_idx_b
         }
     }
     // any number of left rows: popcounts on the matrix cores
-    if (mm_T_mfma_ok(M, N, K, Sl, Sr, G, r_bvr, r_coeff_cache)) {
+    if (!env_switches().popc_q && mm_T_mfma_ok(M, N, K, Sl, Sr, G, r_bvr, r_coeff_cache)) {
         MmArgs a{};
         a.l_bvr = l_bvr;
         a.l_idx = l_coeff_idx;
