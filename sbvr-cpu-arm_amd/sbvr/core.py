@@ -14,6 +14,8 @@ Differences from the reference, all additive: ``encoder_config`` accepts
 from existing arrays; ``decode`` is vectorised and understands all three
 layouts; nothing is printed unless ``verbose_level`` > 0.
 """
+import math
+
 import numpy as np
 import torch
 
@@ -275,15 +277,37 @@ class sbvr(torch.nn.Module):
         """Flat selectors of the padded tensor (core.py:879-901)."""
         return layout.default_to_sel(self.default_layout()).reshape(-1)
 
+    def _decode_kernel_covers(self, bvr, idx, cache):
+        """Whether ``decode`` is one launch over these arrays: on one GPU, uint32 words in the default layout, the
+        types and the layout that the kernel reads, as many rows and columns as the tensor's own shape padded.
+        Anything else (strided or wider indices, a table of another type, no rows) takes the torch expressions, and
+        what these refuse stays refused."""
+        if not (bvr.is_cuda and idx.device == bvr.device and cache.device == bvr.device):
+            return False
+        if (bvr.dtype != torch.uint32 or idx.dtype not in (torch.uint8, torch.uint16) or cache.dtype != torch.float16 or
+                self.compute_dtype != torch.float16):
+            return False
+        if bvr.dim() != 3 or idx.dim() != 2 or cache.dim() != 2 or not (bvr.is_contiguous() and idx.is_contiguous() and
+                                                                        cache.is_contiguous()):
+            return False
+        words, rows, S = bvr.shape
+        shape = self.original_data_shape
+        if len(shape) == 0 or shape[-1] == 0 or rows == 0 or S == 0 or S != self.num_sums or cache.shape[0] == 0:
+            return False
+        if words > 32 * 65535:                  # (the launch's grid: 32 words a workgroup along K)
+            return False
+        return (_padded(shape[-1], self.bvr_len) == words * 32 and math.prod(shape[:-1]) == rows and
+                idx.shape == (words * 32 // self.bvr_len, rows) and cache.shape[1] == S)
+
     @torch.inference_mode()
     def decode(self):
         """The dense tensor this object stands for, in ``original_dtype``: every
         element is one of its group's 2^S points ``bin_combs @ line``
         (core.py:926-949)."""
-        if self.bvr.is_cuda and self.bvr.dtype == torch.uint32 and self.bvr.dim() == 3 and self.bvr.is_contiguous():
+        bvr, idx, cache = self.bvr.data, self.coeff_idx.data, self.coeff_cache.data
+        if self._decode_kernel_covers(bvr, idx, cache):
             from . import hip
-            out = hip.decode_weight(self.bvr.data, self.coeff_idx.data, self.coeff_cache.data, self.bvr_len,
-                                    self.original_data_shape[-1], self.original_dtype)
+            out = hip.decode_weight(bvr, idx, cache, self.bvr_len, self.original_data_shape[-1], self.original_dtype)
             return out.view(self.original_data_shape)
         sel = layout.default_to_sel(self.default_layout()).to(torch.int64)          # (rows, Kp)
         rows, kp = sel.shape

@@ -58,6 +58,44 @@ def test_decode_weight(oracle, N, K, S, G, L, cols, dtype):
     assert got.shape == (N, cols) and got.dtype == dtype and torch.equal(got.cpu(), want)
 
 
+def _dense(bvr, idx, cache, G, oracle):
+    return torch.from_numpy(oracle.C.decode(bvr, idx, cache, G).astype(np.float16))
+
+
+def test_decode_takes_every_form_it_took_on_the_cpu(oracle):
+    """Strides, types and shapes beside those that the one launch reads: the same values as on the CPU, on the GPU."""
+    import sbvr
+    rng = np.random.default_rng(8)
+    N, K, S, G, L = 6, 256, 4, 64, 9
+    bvr, idx, cache = _enc(rng, N, K, S, G, L, oracle, 0.02)
+    cache = (np.round(cache.astype(np.float64) * 2 ** 14) / 2 ** 14).astype(np.float16)
+    want = _dense(bvr, idx, cache, G, oracle)
+    db, di, dc = _dev(bvr, idx, cache)
+    strided_idx = di.t().contiguous().t()
+    strided_cache = torch.cat((dc, dc), dim=1)[:, :S]
+    strided_bvr = torch.cat((db.view(torch.int32), db.view(torch.int32)), dim=2)[:, :, :S].view(torch.uint32)
+    assert not (strided_idx.is_contiguous() or strided_cache.is_contiguous() or strided_bvr.is_contiguous())
+    for b, i, c in ((db, di, dc), (db, strided_idx, dc), (db, di, strided_cache), (strided_bvr, di, dc), (db, di.to(torch.int64), dc),
+                    (db, di.to(torch.int32), dc), (db, di, dc.float()), (db, di, dc.double())):
+        got = sbvr.sbvr.from_parts(b, i, c, G).decode()
+        assert got.dtype == torch.float16 and torch.equal(got.cpu(), want), (i.dtype, i.stride(), c.dtype, c.stride(), b.stride())
+    # leading dimensions; no rows
+    assert torch.equal(sbvr.sbvr.from_parts(db, di, dc, G, original_shape=(2, 3, K)).decode().cpu(), want.view(2, 3, K))
+    assert torch.equal(sbvr.sbvr.from_parts(db[:, :1].contiguous(), di[:, :1].contiguous(), dc, G, original_shape=(K - 5,)).decode().cpu(),
+                       want[0, :K - 5])
+    empty = sbvr.sbvr.from_parts(db[:, :0].contiguous(), di[:, :0].contiguous(), dc, G).decode()
+    assert empty.shape == (0, K) and empty.dtype == torch.float16
+
+
+@pytest.mark.parametrize("shape", [(6, 100), (5, 256), (7, 256), (6, 512)])
+def test_decode_refuses_a_shape_that_is_not_the_arrays(oracle, shape):
+    """A shape that does not pad to the rows and columns of the arrays is an error, not a part of them."""
+    import sbvr
+    arrays = _dev(*_enc(np.random.default_rng(9), 6, 256, 4, 64, 9, oracle))
+    with pytest.raises(RuntimeError):
+        sbvr.sbvr.from_parts(*arrays, 64, original_shape=shape).decode()
+
+
 @pytest.mark.parametrize("S,G,M,K", [(2, 32, 1, 32), (4, 96, 5, 288), (8, 128, 3, 512), (8, 256, 4, 67072), (1, 64, 9, 64)])
 def test_online_encode_lines(S, G, M, K):
     """The same planes as from the table of subset sums, and every group's own number as its line."""
