@@ -239,7 +239,7 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
 // for 2, 3 and 4 planes (S), otherwise plane by plane in fp32 (S = 0: any number of planes).  Eight words of a row are 512
 // bytes of output; the 64-byte pieces of the lanes go through 4 KiB of LDS to lanes that follow each other along a
 // row, so that a store instruction writes two runs of 512 bytes.  Bound by memory: 2 bytes out per weight against S / 8
-// in.  4096 -> 14336, 4 planes: 31 us = 4.7 TB/s, where a
+// in.  An index beyond the table gives NaN (torch's indexing ends the process there).  4096 -> 14336, 4 planes: 31 us = 4.7 TB/s, where a
 // large copy reaches 5.2 (the torch expression over unpacked 64-bit selectors took 4.4 ms); 6 planes 51 us, 8 planes 69 us.
 struct DecodeArgs {
     const uint32_t *bvr;
@@ -277,7 +277,7 @@ sbvr_decode_weight_kernel(const DecodeArgs a)
     const int n = min(n0 + ln, a.N - 1), word = min(w0 + lw, a.words - 1);
     const size_t at = (static_cast<size_t>(word / a.wpg) * a.N + n) << a.idx16;
     const int lo = a.idx[at], hi = a.idx[at + a.idx16];
-    const int line = min(a.idx16 ? lo | (hi << 8) : lo, a.L - 1);
+    const int line_read = a.idx16 ? lo | (hi << 8) : lo, line = min(line_read, a.L - 1);
     uint32_t D[16];                                           // elements 2i, 2i + 1 of the word
     if constexpr (S != 0) {
         const Planes<S> pl = load_planes<S>(a.bvr + (static_cast<size_t>(word) * a.N + n) * S);
@@ -315,6 +315,10 @@ sbvr_decode_weight_kernel(const DecodeArgs a)
         for (int i = 0; i < 16; ++i)
             D[i] = static_cast<uint32_t>(f2h(w[2 * i])) | (static_cast<uint32_t>(f2h(w[2 * i + 1])) << 16);
     }
+    if (line_read >= a.L)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            D[i] = 0x7e007e00u;
     // 16-byte piece c of word w of row n lies at place (w ^ n) * 4 + c of the row's 32: eight lanes that store the same
     // word of eight rows, and the lanes that read a row, meet different banks
 #pragma unroll

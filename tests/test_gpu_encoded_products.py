@@ -87,6 +87,23 @@ def test_decode_takes_every_form_it_took_on_the_cpu(oracle):
     assert empty.shape == (0, K) and empty.dtype == torch.float16
 
 
+@pytest.mark.parametrize("S,L,dtype", [(2, 5, torch.float16), (3, 300, torch.bfloat16), (4, 16, torch.float32), (6, 17, torch.float16)])
+def test_decode_shows_an_index_beyond_the_table(oracle, S, L, dtype):
+    """A group whose index is not below the number of lines decodes to NaN, and nothing else does."""
+    import sbvr
+    rng = np.random.default_rng(S)
+    N, K, G = 11, 512, 64
+    bvr, idx, cache = _enc(rng, N, K, S, G, L, oracle, 0.02)
+    cache = (np.round(cache.astype(np.float64) * 2 ** 14) / 2 ** 14).astype(np.float16)
+    bad = rng.random(idx.shape) < 0.3
+    bad[0, 0] = True
+    marked = np.where(bad, L + rng.integers(0, 200, size=idx.shape), idx).astype(idx.dtype)
+    got = sbvr.sbvr.from_parts(*_dev(bvr, marked, cache), G, original_dtype=dtype).decode().cpu()
+    want = _dense(bvr, idx, cache, G, oracle).to(dtype)
+    want[torch.from_numpy(np.repeat(bad.T, G, axis=1))] = float("nan")
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
 @pytest.mark.parametrize("shape", [(6, 100), (5, 256), (7, 256), (6, 512)])
 def test_decode_refuses_a_shape_that_is_not_the_arrays(oracle, shape):
     """A shape that does not pad to the rows and columns of the arrays is an error, not a part of them."""
