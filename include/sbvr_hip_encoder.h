@@ -53,7 +53,8 @@ int sbvr_hip_online_encode_lines_f16(const void *x, const void *lines, uint32_t 
  * coefficients cache[idx[k / G, n], j] whose plane j is set at (n, k), added up in fp32, rounded to fp16 once and
  * converted to out_type (0 fp16, 1 bf16, 2 fp32).  bvr (K/32, N, S) uint32, idx (K/G, N) uint8 or uint16 (idx_bytes),
  * cache (L, S) fp16; k_out <= K leaves the padding of the last dimension out;
- * the elements of a group whose index is not below L are NaN.  Any S; G a multiple of 32, K of G. */
+ * the elements of a group whose index is not below L are NaN.  A coefficient that is not finite counts as 0 * c = NaN
+ * where its plane is not set, as in the product of the selector bits with the line.  Any S; G a multiple of 32, K of G. */
 int sbvr_hip_decode_weight(const uint32_t *bvr, const void *idx, int idx_bytes, const void *cache, void *out, int out_type,
                            int N, int K, int k_out, int S, int G, int L, void *stream);
 

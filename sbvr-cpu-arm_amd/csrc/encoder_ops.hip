@@ -263,6 +263,8 @@ __device__ __forceinline__ uint32_t bf16_pair(uint32_t two)
     return one(static_cast<uint16_t>(two & 0xffffu)) | (one(static_cast<uint16_t>(two >> 16)) << 16);
 }
 
+__device__ __forceinline__ bool not_finite(uint16_t h) { return (h & 0x7c00u) == 0x7c00u; }
+
 template <int S, int OUT>
 __global__ void __launch_bounds__(64 * kDecWaves)
 sbvr_decode_weight_kernel(const DecodeArgs a)
@@ -297,6 +299,19 @@ sbvr_decode_weight_kernel(const DecodeArgs a)
             D[8 + q] = __builtin_amdgcn_perm(o23, e23, 0x05040100u);
             D[12 + q] = __builtin_amdgcn_perm(o23, e23, 0x07060302u);
         }
+        // an infinite or NaN coefficient counts in the elements that do not select it too, as 0 * inf = NaN
+        uint32_t poison = 0;
+#pragma unroll
+        for (int j = 0; j < S; ++j)
+            if (not_finite(static_cast<uint16_t>(j & 1 ? c[j / 2] >> 16 : c[j / 2])))
+                poison |= ~pl.w[j];
+        if (poison) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                D[i] = (poison >> (2 * i)) & 1u ? (D[i] & 0xffff0000u) | 0x7e00u : D[i];
+                D[i] = (poison >> (2 * i + 1)) & 1u ? (D[i] & 0xffffu) | 0x7e000000u : D[i];
+            }
+        }
     } else {
         float w[32];
 #pragma unroll
@@ -306,10 +321,12 @@ sbvr_decode_weight_kernel(const DecodeArgs a)
         const uint16_t *cs = a.cache + static_cast<size_t>(line) * a.S;
         for (int j = 0; j < a.S; ++j) {
             const int bits = static_cast<int>(src[j]);
-            const uint32_t c = __float_as_uint(h2f(cs[j]));
+            const uint32_t c = __float_as_uint(h2f(cs[j])), without = not_finite(cs[j]) ? 0x7fc00000u : 0u;   // (0 * c)
 #pragma unroll
-            for (int i = 0; i < 32; ++i)
-                w[i] += __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_sbfe(bits, i, 1)) & c);
+            for (int i = 0; i < 32; ++i) {
+                const uint32_t set = static_cast<uint32_t>(__builtin_amdgcn_sbfe(bits, i, 1));
+                w[i] += __uint_as_float((set & c) | (~set & without));
+            }
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i)

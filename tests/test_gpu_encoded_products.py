@@ -104,6 +104,29 @@ def test_decode_shows_an_index_beyond_the_table(oracle, S, L, dtype):
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
 
 
+@pytest.mark.parametrize("S,dtype", [(2, torch.float16), (3, torch.float32), (4, torch.bfloat16), (4, torch.float16), (1, torch.float16),
+                                     (6, torch.float16)])
+def test_decode_of_coefficients_that_are_not_finite(oracle, S, dtype):
+    """Infinite and NaN coefficients, one and several of a line, and sums beyond fp16: as the torch expressions give
+    them on the CPU (a coefficient counts as 0 * c where its bit is not set)."""
+    import sbvr
+    rng = np.random.default_rng(20 + S)
+    N, K, G, L = 19, 512, 32, 12
+    bvr, idx, cache = _enc(rng, N, K, S, G, L, oracle, 1.0)
+    cache = (np.round(cache.astype(np.float64) * 2 ** 8) / 2 ** 8).astype(np.float16)
+    cache[0, 0] = cache[1, S - 1] = np.inf
+    cache[2, 0] = -np.inf
+    cache[3, S // 2] = np.nan
+    cache[4, 0], cache[4, S - 1] = np.inf, -np.inf
+    cache[5] = np.inf
+    cache[6] = 60000.0
+    parts = [torch.from_numpy(a) for a in (bvr, idx, cache)]
+    want = sbvr.sbvr.from_parts(*parts, G, original_dtype=dtype).decode()
+    got = sbvr.sbvr.from_parts(*(p.to("cuda:0") for p in parts), G, original_dtype=dtype).decode().cpu()
+    assert want.isnan().any() and want.isinf().any() and want.isfinite().any()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[~want.isnan()], want[~want.isnan()])
+
+
 @pytest.mark.parametrize("shape", [(6, 100), (5, 256), (7, 256), (6, 512)])
 def test_decode_refuses_a_shape_that_is_not_the_arrays(oracle, shape):
     """A shape that does not pad to the rows and columns of the arrays is an error, not a part of them."""
