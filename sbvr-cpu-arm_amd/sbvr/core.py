@@ -394,7 +394,7 @@ class sbvr(torch.nn.Module):
         if x.shape[1] != k_pad:
             x = torch.nn.functional.pad(x, (0, k_pad - x.shape[1]))
         coeff = self.input_coeff.data
-        bvr, idx = hip.online_encode_lines(x.contiguous(), coeff, self.bvr_len)
+        bvr, idx = hip.online_encode_lines(x.contiguous(), coeff.contiguous(), self.bvr_len)
         return bvr, idx, coeff
 
     _online_transform = _online_tranfrom

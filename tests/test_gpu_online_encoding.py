@@ -100,3 +100,22 @@ def test_input_coefficients_survive_save_and_load(tmp_path):
     assert back.input_num_sums == 3 and torch.equal(back.input_coeff.data, obj.input_coeff.data)
     x = torch.randn((1, 256), generator=gen).to(torch.float16).to(dev)
     assert torch.equal(back.online_mm_T(x), obj.online_mm_T(x))
+
+
+def test_input_coefficients_of_any_strides():
+    """The on-the-fly encoding reads input coefficients that are a view of something else."""
+    import sbvr
+    from sbvr import synth
+    dev = torch.device("cuda:0")
+    K, G, S = 512, 128, 4
+    enc = sbvr.sbvr.from_parts(*(t.to(dev) for t in synth.random_encoding(32, K, 4, G, 16, seed=1)), G)
+    lines = synth.make_lines(K // G, S, 1.0, 7).to(dev)
+    x = torch.randn((3, K), generator=torch.Generator().manual_seed(2)).to(torch.float16).to(dev)
+    enc.input_num_sums = S
+    enc.input_coeff = torch.nn.Parameter(lines, requires_grad=False)
+    bvr, idx, _ = enc._online_tranfrom(x)
+    strided = torch.nn.Parameter(lines.t().contiguous().t(), requires_grad=False)
+    assert not strided.is_contiguous()
+    enc.input_coeff = strided
+    bvr2, idx2, coeff = enc._online_tranfrom(x)
+    assert torch.equal(bvr.view(torch.int32), bvr2.view(torch.int32)) and torch.equal(idx, idx2) and torch.equal(coeff, lines)
