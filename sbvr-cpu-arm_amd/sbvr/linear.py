@@ -62,6 +62,14 @@ class SBVRLinear(torch.nn.Module):
     def forward(self, x):
         # any number of rows: the operator picks the decode, 32-row or prefill kernel.  Leading dimensions, other
         # floating types, the encoder's padding of K to a multiple of bvr_len: all inside the one call
-        b = self._buffers
-        return (_forward or _load_forward())(x, b["bvr"], b["coeff_idx"], b["coeff_cache"], b["bias"], self.bvr_len,
-                                             self.k_padded, self.out_features)
+        call = _forward or _load_forward()
+        if type(self) is SBVRLinear:
+            # (straight from the buffers: four look-ups through Module.__getattr__ are 1 us of a call's 5)
+            b = self._buffers
+            try:
+                arrays = b["bvr"], b["coeff_idx"], b["coeff_cache"], b["bias"]
+            except KeyError:                      # one was replaced by a parameter or a plain attribute
+                arrays = self.bvr, self.coeff_idx, self.coeff_cache, self.bias
+        else:                                     # a subclass, or parametrized: the name may be anything's
+            arrays = self.bvr, self.coeff_idx, self.coeff_cache, self.bias
+        return call(x, *arrays, self.bvr_len, self.k_padded, self.out_features)
