@@ -395,23 +395,25 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     namespace py = pybind11;
     py::register_exception<Refused>(m, "Refused", PyExc_RuntimeError);
     py::register_exception<LaunchFailed>(m, "LaunchFailed", PyExc_RuntimeError);
+    // (the operators that sbvr/hip.py calls: other Python threads run on while a launch waits for room in its queue)
+    const py::call_guard<py::gil_scoped_release> no_gil;
     m.def("_sbvr_hip_init", &sbvr_hip_init_current, "Checks that the current device is a gfx950 part");
     m.def("_sbvr_cuda_init", &sbvr_hip_init_current, "Alias of _sbvr_hip_init under the reference's name");
     m.def("_sbvr_mm_T", &sbvr_mm_T, "SBVR x SBVR^T, both operands encoded", py::arg("l_bvr"), py::arg("l_coeff_idx"),
           py::arg("l_coeff_cache"), py::arg("r_bvr"), py::arg("r_coeff_idx"), py::arg("r_coeff_cache"), py::arg("bias"),
-          py::arg("bvr_len") = 0);
+          py::arg("bvr_len") = 0, no_gil);
     m.def("_sbvr_row_deq_mm_T", &sbvr_row_deq_mm_T, "fp16 x SBVR^T over the trans=True layout", py::arg("l_w"),
           py::arg("r_bvr"), py::arg("r_coeff_idx"), py::arg("r_coeff_cache"), py::arg("bias"), py::arg("use_shfl") = 0,
-          py::arg("bvr_len") = 0);
+          py::arg("bvr_len") = 0, no_gil);
     m.def("_sbvr_linear_f16", &sbvr_linear_f16, "fp16 x SBVR^T over the default layout", py::arg("x"), py::arg("bvr"),
           py::arg("coeff_idx"), py::arg("coeff_cache"), py::arg("bias") = py::none(), py::arg("bvr_len") = 0,
           py::arg("flags") = 0, py::arg("out") = py::none());
     m.def("_linear_forward", &sbvr_linear_forward, "SBVRLinear.forward", py::arg("x"), py::arg("bvr"), py::arg("coeff_idx"),
           py::arg("coeff_cache"), py::arg("bias"), py::arg("bvr_len"), py::arg("k_padded"), py::arg("out_features"));
     m.def("_online_encode_lines", &sbvr_online_encode_lines, "activations to the arrays of an encoded left operand", py::arg("x"),
-          py::arg("lines"), py::arg("bvr_len"));
+          py::arg("lines"), py::arg("bvr_len"), no_gil);
     m.def("_decode_weight", &sbvr_decode_weight, "the dense weight of a default-layout encoding", py::arg("bvr"),
-          py::arg("coeff_idx"), py::arg("coeff_cache"), py::arg("bvr_len"), py::arg("cols"), py::arg("dtype"));
+          py::arg("coeff_idx"), py::arg("coeff_cache"), py::arg("bvr_len"), py::arg("cols"), py::arg("dtype"), no_gil);
     m.def("_workspace", &workspace_of_current_stream, "the split-K workspace of the device's current stream", py::arg("nbytes"),
           py::arg("device"));
     m.def("last_kernel", &sbvr_hip_last_kernel, "which kernel the last linear call of this thread launched");
