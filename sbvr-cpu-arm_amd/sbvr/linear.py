@@ -67,9 +67,10 @@ class SBVRLinear(torch.nn.Module):
             # (straight from the buffers: four look-ups through Module.__getattr__ are 1 us of a call's 5)
             b = self._buffers
             try:
-                arrays = b["bvr"], b["coeff_idx"], b["coeff_cache"], b["bias"]
-            except KeyError:                      # one was replaced by a parameter or a plain attribute
-                arrays = self.bvr, self.coeff_idx, self.coeff_cache, self.bias
-        else:                                     # a subclass, or parametrized: the name may be anything's
-            arrays = self.bvr, self.coeff_idx, self.coeff_cache, self.bias
-        return call(x, *arrays, self.bvr_len, self.k_padded, self.out_features)
+                return call(x, b["bvr"], b["coeff_idx"], b["coeff_cache"], b["bias"], self.bvr_len, self.k_padded,
+                            self.out_features)
+            except KeyError:
+                if "bvr" in b and "coeff_idx" in b and "coeff_cache" in b and "bias" in b:
+                    raise
+        # one was replaced by a parameter or a plain attribute, or is a subclass's or a parametrization's
+        return call(x, self.bvr, self.coeff_idx, self.coeff_cache, self.bias, self.bvr_len, self.k_padded, self.out_features)
