@@ -18,13 +18,23 @@ def _dev(*arrays):
     return [torch.from_numpy(a).to("cuda:0") for a in arrays]
 
 
-# (left row, plane) pairs on both sides of the 16-pair tiles and of the 128-pair workgroups; ragged N; one sub-group
-# of K, fewer sub-groups than waves, several per wave; groups of one and of three sub-groups
+# (left row, plane) pairs on both sides of the 16-pair tiles and of the 64-pair workgroups; ragged N; one sub-group
+# of K, fewer sub-groups than waves, several per wave; groups of one and of three sub-groups; and, on 256 CUs, every
+# pair of row tiles and waves that the launch picks
 @pytest.mark.parametrize("M,N,K,Sl,Sr,G,Ll,Lr", [
     (2, 1, 128, 8, 4, 128, 3, 9), (15, 17, 384, 1, 2, 384, 300, 7), (3, 100, 1024, 5, 3, 128, 9, 300),
     (4, 4100, 4096, 4, 4, 256, 16, 256), (5, 33, 2304, 7, 6, 128, 5, 70), (11, 250, 512, 6, 8, 256, 4, 5),
     (16, 520, 4352, 8, 4, 128, 40, 256), (17, 130, 2176, 8, 3, 128, 300, 16), (33, 64, 256, 4, 8, 128, 8, 8),
-    (64, 1030, 1280, 8, 2, 128, 16, 700), (1, 300, 7168, 8, 4, 256, 28, 256), (1, 40, 256, 16, 4, 128, 2, 3)])
+    (64, 1030, 1280, 8, 2, 128, 16, 700), (1, 300, 7168, 8, 4, 256, 28, 256), (1, 40, 256, 16, 4, 128, 2, 3),
+    # four row tiles, eight waves, the last block of rows ragged
+    (19, 4099, 256, 8, 3, 128, 5, 9), (19, 4099, 256, 8, 4, 128, 5, 9), (19, 4099, 384, 8, 6, 128, 5, 9), (19, 4099, 256, 8, 8, 256, 5, 9),
+    (70, 4099, 256, 3, 4, 128, 5, 300),
+    # two row tiles, sixteen waves: up to 32 pairs, and more of them where the columns are few
+    (4, 4099, 256, 8, 3, 128, 5, 9), (5, 4099, 2304, 6, 8, 128, 5, 9), (17, 1000, 384, 8, 4, 128, 5, 9), (17, 1000, 256, 8, 6, 128, 5, 9),
+    # two row tiles, eight waves
+    (3, 8200, 256, 8, 4, 128, 5, 9), (3, 8200, 256, 8, 8, 128, 5, 9), (7, 8200, 384, 4, 6, 128, 5, 9), (7, 8200, 256, 4, 3, 128, 5, 300),
+    # one row tile, eight waves
+    (2, 8200, 256, 8, 4, 128, 5, 9), (2, 8200, 1408, 5, 6, 128, 5, 9)])
 def test_mm_T_any_rows(oracle, M, N, K, Sl, Sr, G, Ll, Lr):
     import sbvr
     rng = np.random.default_rng(M * 1000 + N)

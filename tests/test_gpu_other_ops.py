@@ -34,7 +34,13 @@ def _close(y, yd, ulps=2.0):
                                                  (1, 48, 512, 2, 3, 256, 7, 9), (1, 4096, 4096, 4, 4, 128, 16, 256),
                                                  (1, 14336, 4096, 4, 4, 128, 16, 256), (1, 1000, 1024, 1, 8, 128, 5, 40),
                                                  (1, 4096, 14336, 4, 4, 128, 16, 256),  # K split across workgroups
-                                                 (1, 2048, 7168, 4, 2, 256, 16, 300), (1, 512, 4096, 4, 6, 128, 9, 256)])
+                                                 (1, 2048, 7168, 4, 2, 256, 16, 300), (1, 512, 4096, 4, 6, 128, 9, 256),
+                                                 (1, 8192, 1024, 4, 2, 128, 16, 256), (1, 8200, 1024, 3, 3, 128, 16, 300),
+                                                 (1, 8192, 2048, 2, 6, 256, 16, 256), (1, 9000, 1024, 4, 8, 128, 16, 256),
+                                                 # groups of 32 and 64: the popcount kernel, by planes
+                                                 (2, 100, 256, 2, 3, 32, 16, 256), (5, 130, 320, 3, 2, 64, 300, 9),
+                                                 (1, 70, 512, 2, 4, 32, 9, 300), (3, 200, 192, 3, 3, 32, 9, 9),
+                                                 (64, 33, 128, 2, 2, 64, 9, 9), (65, 33, 128, 3, 4, 64, 9, 9)])
 def test_mm_T(oracle, M, N, K, Sl, Sr, G, Ll, Lr):
     import sbvr
     dev = torch.device("cuda:0")
@@ -54,8 +60,9 @@ def test_mm_T(oracle, M, N, K, Sl, Sr, G, Ll, Lr):
 
 
 def test_mm_T_without_workspace_and_repeatable(oracle):
-    """The reference-shaped entry point (no workspace) at a shape whose decode launch would split K across
-    workgroups: it must still answer (through the popcount kernel); and the split form twice, bit for bit."""
+    """The reference-shaped entry point (no workspace) at a shape whose decode launch splits K across workgroups: it
+    must still answer (through the matrix-core kernel, which does not split); and the split form, bit for bit on every
+    call, its accumulators zero again."""
     import ctypes
     import sbvr
     from sbvr import hip
@@ -77,11 +84,32 @@ def test_mm_T_without_workspace_and_repeatable(oracle):
     _, yd = oracle.C.mm_T(lb, li, lc, rb, ri, rc_, G)
     _close(out, yd)
     none = torch.zeros(0, dtype=torch.float16, device=dev)
+    plan = (ctypes.c_int * 8)()
+    assert lib.sbvr_hip_decode_plan(S, N, K, S, G, torch.cuda.get_device_properties(dev).multi_processor_count, plan) == 0
+    assert plan[0] == 1 and plan[6] > 1                      # the left planes as four rows, K in parts
     first = sbvr._sbvr_mm_T(*d, none, bvr_len=G)
+    assert hip.last_kernel() == hip.KERNEL_DECODE
     _close(first, yd)
     for _ in range(4):
         again = sbvr._sbvr_mm_T(*d, none, bvr_len=G)
         assert torch.equal(first, again)
+    assert int(hip._workspace(8 * N, dev).count_nonzero()) == 0
+
+
+def test_mm_T_with_a_table_of_less_alignment(oracle):
+    """A right table that is not 16-byte aligned (a slice of a longer one): the popcount kernel at groups of 128 and
+    256, and the portable one beyond its planes."""
+    import sbvr
+    dev = torch.device("cuda:0")
+    for M, N, K, Sl, Sr, G in ((2, 130, 1024, 4, 4, 128), (1, 70, 512, 3, 2, 256), (3, 65, 256, 2, 3, 128), (2, 40, 256, 8, 4, 128)):
+        rng = np.random.default_rng(N)
+        left, right = _rand_enc(rng, M, K, Sl, G, 9, oracle), _rand_enc(rng, N, K, Sr, G, 30, oracle)
+        d = [torch.from_numpy(a).to(dev) for a in (*left, *right)]
+        d[5] = torch.cat((d[5][:1], d[5]))[1:]
+        assert d[5].is_contiguous() and d[5].data_ptr() % 16 != 0
+        y = sbvr._sbvr_mm_T(*d, torch.zeros(0, dtype=torch.float16, device=dev), bvr_len=G)
+        _, yd = oracle.C.mm_T(*left, *right, G)
+        _close(y, yd)
 
 
 def test_mm_T_object_api(oracle, golden):

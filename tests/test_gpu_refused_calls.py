@@ -38,6 +38,49 @@ def test_an_index_without_groups_is_an_error():
         sbvr.SBVRLinear(256, 64, rb[:0], ri[:0], rc, 128)(x)
 
 
+def test_errors_of_the_operators_keep_their_kinds():
+    """What the extension refuses is refused by the checks in Python, each with its own kind of error."""
+    import sbvr
+    from sbvr import hip, synth
+    none = torch.zeros(0, dtype=torch.float16, device=DEV)
+    l, r, t = _encoded(2, seed=1), _encoded(64, seed=2), _encoded(256, 256, seed=3)
+    x = torch.zeros((2, 256), dtype=torch.float16, device=DEV)
+    lines = synth.make_lines(2, 4, 1.0, 7).to(DEV)
+    longer = _encoded(64, 512, seed=4)
+    strided = torch.zeros((2, 512), dtype=torch.float16, device=DEV)[:, ::2]
+
+    def swapped(arrays, at, value):
+        return [value if i == at else a for i, a in enumerate(arrays)]
+
+    both = [*l, *r]
+    for error, args in ((TypeError, swapped(both, 2, l[2].float())), (TypeError, swapped(both, 4, r[1].to(torch.int32).to(torch.uint16))),
+                        (TypeError, swapped(both, 1, None)), (ValueError, [*l, *longer]), (ValueError, swapped(both, 5, r[2][0])),
+                        (ValueError, swapped(both, 1, l[1].t())), (sbvr.hip.SbvrHipError, swapped(both, 3, r[0].cpu()))):
+        with pytest.raises(error):
+            sbvr._sbvr_mm_T(*args, none, bvr_len=128)
+    with pytest.raises(ValueError):
+        sbvr._sbvr_mm_T(*both, none, bvr_len=64)
+    with pytest.raises(TypeError):
+        sbvr._sbvr_mm_T(*both, torch.zeros(64, device=DEV), bvr_len=128)      # a bias of another type
+    for error, args in ((TypeError, [x.float(), *t]), (ValueError, [strided, *t]), (ValueError, [x[:, :128].contiguous(), *t]),
+                        (ValueError, [x[0], *t]), (sbvr.hip.SbvrHipError, [x.cpu(), *t])):
+        with pytest.raises(error):
+            sbvr._sbvr_row_deq_mm_T(*args, none, bvr_len=128)
+    for error, args in ((TypeError, (x.float(), lines, 128)), (ValueError, (x, lines[:1], 128)), (ValueError, (strided, lines, 128)),
+                        (hip.SbvrHipError, (x[:0], lines, 128)), (hip.SbvrHipError, (x.cpu(), lines, 128))):
+        with pytest.raises(error):
+            hip.online_encode_lines(*args)
+    for error, args in ((TypeError, swapped(r, 2, r[2].float())), (ValueError, swapped(r, 1, r[1][:1])), (ValueError, swapped(r, 1, r[1].t())),
+                        (hip.SbvrHipError, swapped(r, 0, r[0].cpu()))):
+        with pytest.raises(error):
+            hip.decode_weight(*args, 128, 256, torch.float16)
+    with pytest.raises(hip.SbvrHipError):
+        hip.decode_weight(*r, 128, 257, torch.float16)                        # more columns than there are
+    # and everything still answers
+    assert sbvr._sbvr_mm_T(*both, none, bvr_len=128).shape == (2, 64)
+    assert hip.decode_weight(*r, 128, 256, torch.float16).shape == (64, 256)
+
+
 def test_the_operators_let_other_threads_run():
     """The products of encoded operands, the encoding on the fly and the decode release the interpreter's lock: with
     a switch interval that never ends, a second thread runs during these calls alone."""
