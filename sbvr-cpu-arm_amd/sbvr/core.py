@@ -14,8 +14,6 @@ Differences from the reference, all additive: ``encoder_config`` accepts
 from existing arrays; ``decode`` is vectorised and understands all three
 layouts; nothing is printed unless ``verbose_level`` > 0.
 """
-import math
-
 import numpy as np
 import torch
 
@@ -277,38 +275,28 @@ class sbvr(torch.nn.Module):
         """Flat selectors of the padded tensor (core.py:879-901)."""
         return layout.default_to_sel(self.default_layout()).reshape(-1)
 
-    def _decode_kernel_covers(self, bvr, idx, cache):
-        """Whether ``decode`` is one launch over these arrays: on one GPU, uint32 words in the default layout, the
-        types and the layout that the kernel reads, as many rows and columns as the tensor's own shape padded.
-        Anything else (strided or wider indices, a table of another type, no rows) takes the torch expressions, and
-        what these refuse stays refused."""
-        if not (bvr.is_cuda and idx.device == bvr.device and cache.device == bvr.device):
-            return False
-        if (bvr.dtype != torch.uint32 or idx.dtype not in (torch.uint8, torch.uint16) or cache.dtype != torch.float16 or
-                self.compute_dtype != torch.float16):
-            return False
-        if bvr.dim() != 3 or idx.dim() != 2 or cache.dim() != 2 or not (bvr.is_contiguous() and idx.is_contiguous() and
-                                                                        cache.is_contiguous()):
+    def _shape_is_the_arrays(self, bvr):
+        """Whether the tensor's own shape, padded, is rows and columns of ``bvr`` in the default uint32 layout."""
+        shape = self.original_data_shape
+        if bvr.dtype != torch.uint32 or bvr.dim() != 3 or len(shape) == 0 or self.compute_dtype != torch.float16:
             return False
         words, rows, S = bvr.shape
-        shape = self.original_data_shape
-        if len(shape) == 0 or shape[-1] == 0 or rows == 0 or S == 0 or S != self.num_sums or cache.shape[0] == 0:
-            return False
-        if words > 32 * 65535:                  # (the launch's grid: 32 words a workgroup along K)
-            return False
-        return (_padded(shape[-1], self.bvr_len) == words * 32 and math.prod(shape[:-1]) == rows and
-                idx.shape == (words * 32 // self.bvr_len, rows) and cache.shape[1] == S)
+        return (S == self.num_sums and shape.numel() == rows * shape[-1] and
+                _padded(shape[-1], self.bvr_len) == words * 32)
 
     @torch.inference_mode()
     def decode(self):
         """The dense tensor this object stands for, in ``original_dtype``: every
         element is one of its group's 2^S points ``bin_combs @ line``
         (core.py:926-949)."""
-        bvr, idx, cache = self.bvr.data, self.coeff_idx.data, self.coeff_cache.data
-        if self._decode_kernel_covers(bvr, idx, cache):
+        bvr = self.bvr
+        if bvr.is_cuda and self._shape_is_the_arrays(bvr):
             from . import hip
-            out = hip.decode_weight(bvr, idx, cache, self.bvr_len, self.original_data_shape[-1], self.original_dtype)
-            return out.view(self.original_data_shape)
+            out = hip.decode_weight_if_covered(bvr, self.coeff_idx, self.coeff_cache, self.bvr_len,
+                                               self.original_data_shape[-1], self.original_dtype)
+            if out is not None:
+                return out.view(self.original_data_shape)
+        # strided or wider indices, a table of another type, no rows, another layout, the CPU
         sel = layout.default_to_sel(self.default_layout()).to(torch.int64)          # (rows, Kp)
         rows, kp = sel.shape
         points = (self._get_bin_combs().float() @ self.coeff_cache.data.float().T).T   # (lines, 2^S)

@@ -681,6 +681,18 @@ def online_encode_lines(x, lines, bvr_len):
 _DECODE_TYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
 
 
+def decode_weight_if_covered(bvr, coeff_idx, coeff_cache, bvr_len, cols, dtype):
+    """``decode_weight``, or None where the arrays are not what the launch reads (types, strides, no rows): for a
+    caller that has another way."""
+    if _ext():
+        return _native("_decode_weight", bvr, coeff_idx, coeff_cache, bvr_len, cols, dtype)
+    if (bvr.dim() != 3 or coeff_idx.dtype not in (torch.uint8, torch.uint16) or coeff_cache.dtype != torch.float16 or
+            not (bvr.is_contiguous() and coeff_idx.is_contiguous() and coeff_cache.is_contiguous()) or
+            0 in bvr.shape or coeff_cache.shape[0] == 0 or cols == 0 or bvr.shape[0] > 32 * 65535):
+        return None
+    return decode_weight(bvr, coeff_idx, coeff_cache, bvr_len, cols, dtype)
+
+
 def decode_weight(bvr, coeff_idx, coeff_cache, bvr_len, cols, dtype):
     """The dense (N, cols) weight of a default-layout encoding (cols: without the padding of K), every element its
     coefficients' fp32 sum rounded to fp16 once, in ``dtype`` (sbvr/core.py:926-949)."""
