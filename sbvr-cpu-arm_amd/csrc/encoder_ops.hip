@@ -239,8 +239,10 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
 // for 2, 3 and 4 planes (S), otherwise plane by plane in fp32 (S = 0: any number of planes).  Eight words of a row are 512
 // bytes of output; the 64-byte pieces of the lanes go through 4 KiB of LDS to lanes that follow each other along a
 // row, so that a store instruction writes two runs of 512 bytes.  Bound by memory: 2 bytes out per weight against S / 8
-// in.  An index beyond the table gives NaN (torch's indexing ends the process there).  4096 -> 14336, 4 planes: 31 us = 4.7 TB/s, where a
-// large copy reaches 5.2 (the torch expression over unpacked 64-bit selectors took 4.4 ms); 6 planes 51 us, 8 planes 69 us.
+// in.  An index beyond the table gives NaN (torch's indexing ends the process there).  4096 -> 14336, 4 planes: 27.8 us the
+// launch, 34.8 a call among others on weights that take turns = 4.2 TB/s, where a large copy reaches 5.2 (the torch
+// expression over unpacked 64-bit selectors took 4.4 ms); 2, 3, 6 and 8 planes 30.5, 32, 62 and 80 us the launch, the
+// last two bound by the vector ALU.
 struct DecodeArgs {
     const uint32_t *bvr;
     const uint8_t *idx;
@@ -336,8 +338,9 @@ sbvr_decode_weight_kernel(const DecodeArgs a)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
             D[i] = 0x7e007e00u;
-    // 16-byte piece c of word w of row n lies at place (w ^ n) * 4 + c of the row's 32: eight lanes that store the same
-    // word of eight rows, and the lanes that read a row, meet different banks
+    // 16-byte piece c of word w of row n lies at place (w ^ n) * 4 + c of the row's 32: the lanes that read a row meet
+    // different banks; eight lanes that store piece c of one word of eight rows still share a quarter of them (24 clocks
+    // more a store by SQ_LDS_BANK_CONFLICT, in the shadow of memory)
 #pragma unroll
     for (int c = 0; c < 4; ++c)
         tile[ln * 32 + ((lw ^ ln) << 2) + c] = v4u{D[4 * c], D[4 * c + 1], D[4 * c + 2], D[4 * c + 3]};

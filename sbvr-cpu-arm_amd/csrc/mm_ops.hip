@@ -18,8 +18,8 @@ constexpr int kMmSub = 128;          // elements of K per MFMA
 // rows from a small LDS table that the wave fills for itself.
 // Bound by the vector ALU: per 16 x 16 x 128 block and SR right planes 4 SR + 4 FMAs a lane, 7 operations to make the
 // left operand, against 16 clocks per MFMA; with few rows by the latency of the loads in front of it.  (Where the
-// one-thread-per-output kernel took 727 us, 16 rows of 8 planes x 4096 columns x 4096 with 4 right planes, it takes 9.7;
-// 4 rows of 4 planes 4.9 us where the popcount kernel took 9.0.)
+// one-thread-per-output kernel took 727 us, 16 rows of 8 planes x 4096 columns x 4096 with 4 right planes, it takes 9.8;
+// 4 rows of 4 planes 4.7 us where the popcount kernel took 9.3.)
 template <int SR, int RT, int W>
 __global__ void __launch_bounds__(64 * W)
 sbvr_mm_T_mfma_kernel(const MmArgs a)
@@ -103,7 +103,7 @@ sbvr_mm_T_mfma_kernel(const MmArgs a)
         }
         // A step is up to 4 planes of one row tile: its MFMAs are issued together, and the results of the step before
         // are multiplied with their coefficients while they run (left to itself the compiler lets every MFMA's
-        // consumers wait for it before it issues the next one: 118 us against 110 for 64 rows of 8 planes x 14336 x 4096)
+        // consumers wait for it before it issues the next one: 118 us against 110 for 64 rows of 8 planes x 14336 x 4096 with 8 row tiles)
         v4f D[2][PS];
         v4f sum = v4f{0.f, 0.f, 0.f, 0.f};
         auto consume = [&](int step) __attribute__((always_inline)) {
@@ -226,7 +226,7 @@ hipError_t launch_mm_T_mfma(int Sr, int G, MmArgs a, int cus, hipStream_t st)
     // quarter of the CUs without one (every workgroup of a column block reads its plane words again, out of the L2).
     // Sixteen waves where that gives a CU about one workgroup, eight where there are two and more.  us by (row tiles,
     // waves), 4 right planes: 16 rows of 8 planes, 4096 x 4096: (4, 8) 9.7, (8, 8) 9.8, (4, 16) 11.7, (2, 16) 15.4;
-    // 64 rows of 8 planes, 14336 x 4096: (4, 8) 89.5, (8, 8) 110, (4, 16) 133; 32 rows of 8, 512 x 14336: (2, 16) 10.0,
+    // 64 rows of 8 planes, 14336 x 4096: (4, 8) 89.5 to 99, (8, 8) 110, (4, 16) 133; 32 rows of 8, 512 x 14336: (2, 16) 10.0,
     // (1, 16) 12.2, (4, 16) 13.5; 4 rows of 4, 4096 x 4096: (1, 16) 4.9, (1, 8) 5.3, (1, 4) 6.8.
     const int rows = a.M * a.Sl, cols = (a.N + 15) / 16;
     int RT = rows <= 16 ? 1 : (rows <= 32 ? 2 : 4);

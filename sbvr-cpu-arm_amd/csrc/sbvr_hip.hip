@@ -38,9 +38,10 @@
 // registers -- by table look-up for 2..4 planes (sbvr_gemm_rows32_lut_kernel),
 // arithmetically otherwise (sbvr_gemm_rows32_kernel).
 //
-// The reference's own operator forms: both operands encoded: the decode kernel
-// with the left operand's planes as batch rows (one left row of up to 4 planes),
-// else sbvr_mm_T_popc_kernel (popcounts per group, lane per column);
+// The reference's own operator forms: both operands encoded: the matrix-core
+// kernel of mm_ops.hip (K and G multiples of 128), one left row of up to 4 planes
+// mostly on the decode kernel with the left planes as batch rows, groups of 32 and
+// 64 on sbvr_mm_T_popc_kernel (popcounts per group, lane per column);
 // sbvr_row_deq_mfma_kernel (trans=True
 // weight: bits transposed across lanes, then the decode path's plane sums) and
 // sbvr_row_deq_lanes_kernel (the same for other plane counts, lanes along K).
@@ -2538,7 +2539,8 @@ bool gemm_lut_path_ok(int M, int N, int K, int S, int G)
 // Few row blocks mean more workgroups and more decodes of the weights, more parts of K more workgroups and partial
 // results to write and add up: the plan is the one of least estimated time.  Estimate, from launches of 8192 -> 28672
 // with 2 to 8 row blocks (0.94, 1.36, 1.84, 2.08 us a step): a step takes 0.55 + 0.2 RB us, a workgroup 2 us beside its
-// steps, and a split 2 us and its partial results at 6 TB/s.  256 workgroups run at a time; beyond that the
+// steps, and a split 2 us and its partial results once at 6 TB/s (the second pass reads and clears them: 9.9 us
+// at 333 rows x 6144 columns in 4 parts, where this says 7.5).  256 workgroups run at a time; beyond that the
 // last turn counts half (8192 -> 28672: 1.31 turns take the time of 1.70, 3.5 turns that of 3.68).
 // Against tiles of 256 rows throughout, 4 planes: 4096 -> 6144, 600 rows 86.5 -> 53.0 us (240 workgroups of 4 row blocks
 // for 144 of 7), 128 rows 30.6 -> 25.7; 4096 -> 4096, 192 rows 36.3 -> 26.0; 8192 -> 28672, 600 rows 472 -> 362.
