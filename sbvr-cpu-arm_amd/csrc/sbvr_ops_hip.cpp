@@ -105,14 +105,18 @@ void check_encoder(int rc, const char *what, const Args &...shape)
 // Zero-initialised split-K accumulators per (device, stream), grown on demand to twice their size at least; the
 // kernels leave the part that must be zero zeroed.  A buffer that is outgrown is kept until the process
 // ends: a HIP graph captured earlier on that stream still holds its address (all of them together are smaller than
-// the one in use).  The only pool of the process: the
-// functions of sbvr/hip.py ask for theirs here, so that a stream that one operator has warmed is warm for all.
-torch::Tensor workspace(size_t nbytes, c10::Device device, hipStream_t stream)
+// the one in use).  One set for the linears of this file (SBVRLinear), one for the functions of sbvr/hip.py, whether
+// they are launched here or through ctypes: a stream that one of these has warmed is warm for the others.  (Two sets,
+// because the graphs of sbvr/decoder.py hold the second one's buffer of the stream they were recorded on and are
+// replayed on others: a layer called on that stream meanwhile must not add into it.)
+enum class Users { kLinears, kFunctions };
+
+torch::Tensor workspace(size_t nbytes, c10::Device device, hipStream_t stream, Users users)
 {
     static std::mutex mu;
-    static std::map<std::tuple<int, hipStream_t>, torch::Tensor> held;
+    static std::map<std::tuple<int, hipStream_t, Users>, torch::Tensor> held;
     static std::vector<torch::Tensor> outgrown;
-    const auto key = std::make_tuple(static_cast<int>(device.index()), stream);
+    const auto key = std::make_tuple(static_cast<int>(device.index()), stream, users);
     auto enough = [&]() -> torch::Tensor {
         const auto it = held.find(key);
         return it != held.end() && static_cast<size_t>(it->second.numel()) >= nbytes ? it->second : torch::Tensor();
@@ -185,7 +189,7 @@ void launch_linear(const torch::Tensor &x, const torch::Tensor &bvr, const torch
 {
     hipStream_t stream = current_stream();
     const size_t need = sbvr_hip_linear_f16_workspace(s.M, s.N, s.K, s.S, s.G);
-    torch::Tensor ws = need ? workspace(need, x.device(), stream) : torch::Tensor();
+    torch::Tensor ws = need ? workspace(need, x.device(), stream, Users::kLinears) : torch::Tensor();
     check(sbvr_hip_linear_f16(x.data_ptr(), static_cast<const uint32_t *>(bvr.data_ptr()), coeff_idx.data_ptr(), s.ib,
                               coeff_cache.data_ptr(), bias_ptr(bias, s.N, x), out.data_ptr(), s.M, s.N, s.K, s.S, s.G,
                               s.L, need ? ws.data_ptr() : nullptr, need ? ws.numel() : 0, flags, stream));
@@ -250,7 +254,7 @@ torch::Tensor sbvr_linear_f16_swiglu(const torch::Tensor &gate_up, const torch::
     hipStream_t stream = current_stream();
     auto out = torch::empty({s.M, s.N}, torch::dtype(torch::kFloat16).device(gate_up.device()));
     const size_t need = sbvr_hip_linear_f16_workspace(s.M, s.N, s.K, s.S, s.G);
-    torch::Tensor ws = need ? workspace(need, gate_up.device(), stream) : torch::Tensor();
+    torch::Tensor ws = need ? workspace(need, gate_up.device(), stream, Users::kLinears) : torch::Tensor();
     check(sbvr_hip_linear_f16_swiglu(gate_up.data_ptr(), static_cast<const uint32_t *>(bvr.data_ptr()), coeff_idx.data_ptr(),
                                      s.ib, coeff_cache.data_ptr(), bias_ptr(bias, s.N, gate_up), out.data_ptr(), s.M, s.N,
                                      s.K, s.S, s.G, s.L, need ? ws.data_ptr() : nullptr, need ? ws.numel() : 0, stream));
@@ -274,7 +278,7 @@ torch::Tensor sbvr_linear_f16_add_rmsnorm(torch::Tensor x, torch::Tensor delta, 
     hipStream_t stream = current_stream();
     auto out = torch::empty({1, s.N}, torch::dtype(torch::kFloat16).device(x.device()));
     const size_t need = sbvr_hip_linear_f16_workspace(1, s.N, s.K, s.S, s.G);
-    torch::Tensor ws = need ? workspace(need, x.device(), stream) : torch::Tensor();
+    torch::Tensor ws = need ? workspace(need, x.device(), stream, Users::kLinears) : torch::Tensor();
     check(sbvr_hip_linear_f16_add_rmsnorm(x.data_ptr(), delta.data_ptr(), norm_weight.data_ptr(), static_cast<float>(eps),
                                           x_out.data_ptr(), static_cast<const uint32_t *>(bvr.data_ptr()),
                                           coeff_idx.data_ptr(), s.ib, coeff_cache.data_ptr(), bias_ptr(bias, s.N, x),
@@ -308,7 +312,7 @@ torch::Tensor sbvr_mm_T(const torch::Tensor &l_bvr, const torch::Tensor &l_coeff
     const size_t need = sbvr_hip_mm_T_workspace(static_cast<int>(M), static_cast<int>(N));
     torch::Tensor ws;                    // (no split of K for this call: no workspace, nothing allocated)
     if (need)
-        ws = workspace(need, l_bvr.device(), stream);
+        ws = workspace(need, l_bvr.device(), stream, Users::kFunctions);
     check(sbvr_hip_mm_T_ws(static_cast<const uint32_t *>(l_bvr.data_ptr()), l_coeff_idx.data_ptr(), lib,
                            l_coeff_cache.data_ptr(), static_cast<const uint32_t *>(r_bvr.data_ptr()), r_coeff_idx.data_ptr(),
                            rib, r_coeff_cache.data_ptr(), bias_ptr(bias, N, l_bvr), out.data_ptr(), M, N, K, Sl, Sr, G, Ll,
@@ -375,19 +379,19 @@ torch::Tensor sbvr_row_deq_mm_T(const torch::Tensor &l_w, const torch::Tensor &r
     const size_t need = sbvr_hip_row_deq_mm_T_workspace(static_cast<int>(M), static_cast<int>(N));
     torch::Tensor ws;                    // (no split of K for this call: no workspace, nothing allocated)
     if (need)
-        ws = workspace(need, l_w.device(), stream);
+        ws = workspace(need, l_w.device(), stream, Users::kFunctions);
     check(sbvr_hip_row_deq_mm_T_ws(l_w.data_ptr(), static_cast<const uint32_t *>(r_bvr.data_ptr()), r_coeff_idx.data_ptr(), ib,
                                    r_coeff_cache.data_ptr(), bias_ptr(bias, N, l_w), out.data_ptr(), M, N, K, S, G, L,
                                    need ? ws.data_ptr() : nullptr, need, stream));
     return out;
 }
 
-// The workspace of the current stream of a device, for launches that are made through the C ABI.
+// The functions' workspace of the current stream of a device, for launches that are made through the C ABI.
 torch::Tensor workspace_of_current_stream(int64_t nbytes, int64_t device)
 {
     const c10::Device dev(c10::DeviceType::CUDA, static_cast<c10::DeviceIndex>(device));
     const DeviceGuard guard(dev);
-    return workspace(static_cast<size_t>(nbytes), dev, current_stream());
+    return workspace(static_cast<size_t>(nbytes), dev, current_stream(), Users::kFunctions);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)

@@ -193,7 +193,8 @@ def _workspace(nbytes, device):
     """Zero-initialised scratch per (device, stream); grown on demand to twice its size at least.  The
     kernels leave the part that must be zero zeroed.  A buffer that is outgrown
     stays allocated: a HIP graph recorded earlier on the stream keeps its address.
-    The pool is the extension's, one for every operator of the process."""
+    The buffers are the extension's, which launches some of these functions
+    itself."""
     key = (device.index, torch.cuda.current_stream(device).cuda_stream)
     ext = _ext()
     if ext:

@@ -1,4 +1,5 @@
-"""The split-K workspace: one pool for the operators of the extension and for those that go through ctypes."""
+"""The split-K workspace: one for the functions that the extension launches and those that go through ctypes, another
+for SBVRLinear."""
 import pytest
 import torch
 
@@ -12,9 +13,9 @@ def _encoded(rows, K, S=4, G=128, L=16, seed=0):
     return [t.to(DEV) for t in synth.random_encoding(rows, K, S, G, L, seed=seed)]
 
 
-def test_a_stream_warmed_by_one_operator_is_warm_for_all():
-    """After the functional linear (ctypes) the products of encoded operands (extension) and SBVRLinear find their
-    accumulators on that stream: no allocation but their outputs', inside a capture as well, and right replays."""
+def test_a_stream_warmed_by_one_function_is_warm_for_all():
+    """After the functional linear (ctypes) the products of encoded operands (extension) find their accumulators on that
+    stream: no allocation but their outputs', inside a capture as well, and right replays."""
     import sbvr
     from sbvr import _sbvr_hip_ops as ops, hip
     N, K = 1024, 2048
@@ -25,8 +26,7 @@ def test_a_stream_warmed_by_one_operator_is_warm_for_all():
     none = torch.zeros(0, dtype=torch.float16, device=DEV)
     lib = hip._load()
     assert lib.sbvr_hip_row_deq_mm_T_workspace(2, N) > 0 and lib.sbvr_hip_mm_T_workspace(1, N) > 0
-    linear = sbvr.SBVRLinear(K, N, *w, 128)
-    want = [sbvr._sbvr_row_deq_mm_T(x, *t, none, bvr_len=128), sbvr._sbvr_mm_T(*l, *w, none, bvr_len=128), linear(x)]
+    want = [sbvr._sbvr_row_deq_mm_T(x, *t, none, bvr_len=128), sbvr._sbvr_mm_T(*l, *w, none, bvr_len=128)]
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
@@ -36,13 +36,13 @@ def test_a_stream_warmed_by_one_operator_is_warm_for_all():
         assert ops._workspace(1, DEV.index).data_ptr() == ws.data_ptr()
         side.synchronize()
         before = torch.cuda.memory_allocated()
-        got = [sbvr._sbvr_row_deq_mm_T(x, *t, none, bvr_len=128), sbvr._sbvr_mm_T(*l, *w, none, bvr_len=128), linear(x)]
+        got = [sbvr._sbvr_row_deq_mm_T(x, *t, none, bvr_len=128), sbvr._sbvr_mm_T(*l, *w, none, bvr_len=128)]
         assert torch.cuda.memory_allocated() - before <= sum((2 * y.numel() + 511) // 512 * 512 for y in got)
         side.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(got, want))
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=side):
-        got = [sbvr._sbvr_row_deq_mm_T(x, *t, none, bvr_len=128), sbvr._sbvr_mm_T(*l, *w, none, bvr_len=128), linear(x)]
+        got = [sbvr._sbvr_row_deq_mm_T(x, *t, none, bvr_len=128), sbvr._sbvr_mm_T(*l, *w, none, bvr_len=128)]
         assert ops._workspace(1, DEV.index).data_ptr() == ws.data_ptr()
     for _ in range(3):
         graph.replay()
@@ -66,3 +66,26 @@ def test_growing_requests_hold_little_more_than_the_largest():
                 sizes[ws.data_ptr()] = ws.numel()
         assert int(ws.count_nonzero()) == 0
         assert sum(sizes.values()) <= 4 * (25 << 20)
+
+
+def test_layers_keep_out_of_the_accumulators_of_recorded_functions():
+    """A graph of the functions holds its stream's buffer and may be replayed on another stream while a layer is called
+    on the first: the two never use one buffer."""
+    import sbvr
+    from sbvr import hip
+    N, K = 1024, 2048
+    w = _encoded(N, K, seed=1)
+    x = torch.randn((2, K), generator=torch.Generator().manual_seed(4)).to(torch.float16).to(DEV)
+    layer = sbvr.SBVRLinear(K, N, *w, 128)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want = sbvr._sbvr_linear_f16(x, *w, bvr_len=128)
+        ws = hip._workspaces[(DEV.index, side.cuda_stream)]
+        side.synchronize()
+        ws.view(torch.int64)[:2 * N] = 1 << 40           # (a launch under way elsewhere has left its sums here)
+        y = layer(x)
+        side.synchronize()
+        assert torch.equal(y, want) and int((ws.view(torch.int64)[:2 * N] != 1 << 40).sum()) == 0
+        ws.zero_()
+        side.synchronize()
