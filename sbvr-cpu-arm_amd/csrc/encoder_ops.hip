@@ -180,7 +180,7 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
             float sum = 0.f;
             for (int j = 0; j < S; ++j) {
                 const float c = static_cast<float>(__builtin_bit_cast(_Float16, table[static_cast<size_t>(g) * S + j]));
-                sum += (p >> (S - 1 - j)) & 1 ? c : 0.f;
+                sum += (p >> (S - 1 - j)) & 1 ? c : 0.f * c;       // (NaN where c is not finite, as a product would have it)
             }
             v = __builtin_bit_cast(uint16_t, static_cast<_Float16>(sum));
         } else {
@@ -210,7 +210,9 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
                 best = min(min(best, (sq << 16) | p), (sq & 0xffff0000u) | (p + 1));
             }
         }
-        const uint32_t sel = best & 0xffffu;
+        // (a distance that is no number is never the nearest, but the first of them stays: the search starts with it)
+        const _Float16 d0 = d - __builtin_bit_cast(v2h, mine[0].x)[0], first = d0 * d0;
+        const uint32_t sel = first != first ? 0u : best & 0xffffu;
         uint32_t out = 0;
         for (int j = 0; j < S; ++j) {                                                 // plane 0: the selector's top bit
             const unsigned long long bits = __builtin_amdgcn_ballot_w64(((sel >> (S - 1 - j)) & 1) != 0);

@@ -102,6 +102,50 @@ def test_input_coefficients_survive_save_and_load(tmp_path):
     assert torch.equal(back.online_mm_T(x), obj.online_mm_T(x))
 
 
+def _first_nearest(x, points, G):
+    """Selectors (M, K): the search goes on to a later point only where its squared distance, in fp16, is smaller."""
+    with np.errstate(all="ignore"):
+        d = x[:, :, None] - np.repeat(points, G, axis=0)[None]
+        sq = (d * d).astype(np.float16)
+        best, sel = sq[..., 0].copy(), np.zeros(x.shape, dtype=np.int64)
+        for p in range(1, points.shape[1]):
+            less = sq[..., p] < best
+            best, sel = np.where(less, sq[..., p], best), np.where(less, p, sel)
+    return sel
+
+
+@pytest.mark.parametrize("S", [1, 2, 4, 8])
+def test_values_and_points_that_are_not_finite(S):
+    """Infinite and NaN activations, tables and lines with such entries, distances beyond fp16, ties: the rule of the
+    search over finite numbers, and the first point where it has no number to start with."""
+    from sbvr import hip, layout
+    dev = torch.device("cuda:0")
+    G, K, M = 32, 32 * 8, 5
+    rng = np.random.default_rng(S)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    x[0, ::5], x[1, ::7], x[2, ::3], x[3, ::4] = np.inf, -np.inf, np.nan, 60000.0
+    lines = (rng.integers(-8, 8, size=(K // G, S)) / 8).astype(np.float16)
+    lines[1, 0], lines[2, S - 1], lines[3, S // 2], lines[4] = np.inf, -np.inf, np.nan, 50000.0
+    combs = layout.bin_combs(S, torch.float32, "cpu").numpy()
+    with np.errstate(all="ignore"):
+        # (0 * inf is NaN in the product of the selector bits with the line; the finite sums are exact)
+        points = (combs[None] * lines.astype(np.float32)[:, None]).sum(-1).astype(np.float16)
+
+    def planes(sel):
+        # bit k % 32 of word k / 32 of plane j = bit S - 1 - j of the selector
+        bits = (sel[:, :, None] >> (S - 1 - np.arange(S))) & 1
+        words = (bits.reshape(M, K // 32, 32, S).astype(np.uint64) << np.arange(32, dtype=np.uint64)[None, None, :, None]).sum(2)
+        return torch.from_numpy(words.transpose(1, 0, 2).astype(np.uint32).astype(np.int64))
+
+    t = lambda a: torch.from_numpy(a).to(dev)
+    got, _ = hip.online_encode_lines(t(x), t(lines), G)
+    assert torch.equal(got.cpu().view(torch.int32).to(torch.int64) & 0xffffffff, planes(_first_nearest(x, points, G)))
+    points[5, 0] = np.nan
+    points[6, -1], points[7, -1] = np.nan, np.inf
+    got = hip.online_encode(t(x), t(points), G)
+    assert torch.equal(got.cpu().view(torch.int32).to(torch.int64) & 0xffffffff, planes(_first_nearest(x, points, G)))
+
+
 def test_input_coefficients_of_any_strides():
     """The on-the-fly encoding reads input coefficients that are a view of something else."""
     import sbvr
