@@ -279,12 +279,12 @@ int sbvr_hip_mm_T(const uint32_t *l_bvr, const void *l_coeff_idx, int l_idx_byte
  * sbvr_hip_mm_T_workspace(M, N) bytes (M*N 64-bit accumulators, zero-filled once, 8-byte aligned,
  * left zero by every call; it may be the workspace of sbvr_hip_linear_f16, not used by two calls
  * at once).  K and G multiples of 128, up to 16 left planes and 2, 3, 4, 6 or 8 right planes: the popcounts come out
- * of the matrix cores, any number of left rows.  One left row of up to 4 planes (G / 128 a power of two), except for
- * short K and few columns, runs on the decode kernel, the left operand's planes, each times its coefficient, as its
- * batch rows; where that launch splits K across workgroups it needs the workspace, without one it takes the former
- * kernel.  Other
- * shapes: popcounts on the vector ALU.  The reference's operator has no such argument
- * (sbvr_ops.cpp:35-76); its bindings here bring their own.
+ * of the matrix cores, any number of left rows (up to 65535 blocks of 64 rows times planes).  One left row of up to 4
+ * planes (N >= 16, G / 128 a power of two) runs on the decode kernel, the left operand's planes, each times its
+ * coefficient, as its batch rows, unless K is short or the columns fill most CUs of the former kernel; where the
+ * decode launch splits K across workgroups it needs the workspace, without one the call takes the former kernel.
+ * Other shapes: popcounts on the vector ALU.  The reference's operator has no such argument (sbvr_ops.cpp:35-76); its
+ * bindings here bring their own.
  */
 int sbvr_hip_mm_T_ws(const uint32_t *l_bvr, const void *l_coeff_idx, int l_idx_bytes,
                      const void *l_coeff_cache, const uint32_t *r_bvr,

@@ -111,8 +111,10 @@ def test_the_operators_let_other_threads_run():
         thread.start()
         for call in calls:
             before = ran[0]
-            for _ in range(500):
+            for _ in range(20000):           # (the waiting thread has to wake up while the lock is free)
                 call()
+                if ran[0] > before:
+                    break
             assert ran[0] > before
     finally:
         sys.setswitchinterval(interval)
