@@ -1024,12 +1024,12 @@ struct GemvPlan {
     int wstride;
 };
 
-// Development switches.  A library built with -DSBVR_DEV_SWITCHES reads them from the environment once per
-// process (SBVR_HIP_CT, _SP, _WAVES, _WSTRIDE, _SHOW_PLAN, _POPC_Q, _ROWDEQ_LANES, _LUT_ROWS, _PF_LUT); the
+// Development switches.  A library built with -DSBVR_DEV_SWITCHES reads them from the environment at every
+// call (SBVR_HIP_CT, _SP, _WAVES, _WSTRIDE, _SHOW_PLAN, _POPC_Q, _ROWDEQ_LANES, _LUT_ROWS, _PF_LUT, _PF_RB, _PF_KS); the
 // library as shipped does not look at the environment: launch shapes and the choice of kernel (and with it the
 // rounding) depend on the arguments of a call alone.
 struct EnvSwitches {
-    int ct, sp, waves, wstride, show_plan, popc_q, rowdeq_lanes, lut_rows, pf_lut;
+    int ct, sp, waves, wstride, show_plan, popc_q, rowdeq_lanes, lut_rows, pf_lut, pf_rb, pf_ks;
 };
 
 #ifndef SBVR_DEV_SWITCHES
@@ -1041,13 +1041,15 @@ const EnvSwitches &env_switches()
 #else
 const EnvSwitches &env_switches()
 {
-    static const EnvSwitches e = [] {
+    static thread_local EnvSwitches e;
+    e = [] {
         auto get = [](const char *name) {
             const char *v = getenv(name);
             return v && *v ? atoi(v) : 0;
         };
         return EnvSwitches{get("SBVR_HIP_CT"), get("SBVR_HIP_SP"), get("SBVR_HIP_WAVES"), get("SBVR_HIP_WSTRIDE"),
-                           get("SBVR_HIP_SHOW_PLAN"), get("SBVR_HIP_POPC_Q"), get("SBVR_HIP_ROWDEQ_LANES"), get("SBVR_HIP_LUT_ROWS"), get("SBVR_HIP_PF_LUT")};
+                           get("SBVR_HIP_SHOW_PLAN"), get("SBVR_HIP_POPC_Q"), get("SBVR_HIP_ROWDEQ_LANES"), get("SBVR_HIP_LUT_ROWS"), get("SBVR_HIP_PF_LUT"),
+                           get("SBVR_HIP_PF_RB"), get("SBVR_HIP_PF_KS")};
     }();
     return e;
 }
@@ -1454,11 +1456,16 @@ struct GemmArgs {
     int steps_per_group;   // G / 64
     int idx16;
     int ksplit;            // workgroups along K (blockIdx.z); 1: results go straight to out
+    int part_steps;        // steps of 64 along K of a part (the last one's may be fewer); table look-up kernel only
     float *part;           // ksplit > 1: (ksplit, M, N) fp32 partial results, all zero between launches
 #ifdef SBVR_TRACE
     unsigned long long *trace;
 #endif
 };
+
+// Floats from one part's partial results to the next's: M * N, and up to a multiple of 4, so that every part starts on
+// 16 bytes and the second pass takes four outputs at a time whatever N is.
+__host__ __device__ inline size_t part_floats(int M, int N) { return (static_cast<size_t>(M) * N + 3) & ~static_cast<size_t>(3); }
 
 // The S fp16 coefficients of one table line as packed pairs, in as few load instructions as the
 // line's alignment allows (a line starts at a multiple of 2*S bytes; the table is 16-byte aligned).
@@ -1731,7 +1738,7 @@ sbvr_gemm_mfma_kernel(const GemmArgs a)
     if (a.ksplit > 1) {
         // K split across workgroups: every workgroup leaves its fp32 tile in `part`; sbvr_gemm_reduce_kernel,
         // launched behind this kernel, adds the tiles up in the order of blockIdx.z and rounds once.
-        float *mine = a.part + blockIdx.z * (static_cast<size_t>(M) * N);
+        float *mine = a.part + blockIdx.z * part_floats(M, N);
 #pragma unroll
         for (int bj = 0; bj < 2; ++bj) {
             const int n = n0 + wn * 64 + bj * 32 + (lane & 31);
@@ -1769,32 +1776,37 @@ sbvr_gemm_mfma_kernel(const GemmArgs a)
 
 // Second pass of a split prefill launch: out[m, n] = fp16(sum over z, in order, of part[z][m][n]) (+ bias),
 // and the partial results are set back to zero (the workspace is shared with the decode kernel's
-// accumulators, which must find zeros).  Four outputs per thread.
+// accumulators, which must find zeros).  Four outputs per thread, of two rows where N is no multiple of 4.
 __global__ void __launch_bounds__(256)
 sbvr_gemm_reduce_kernel(float *__restrict__ part, const uint16_t *__restrict__ bias, uint16_t *__restrict__ out,
                         int M, int N, int ksplit)
 {
-    const size_t total = static_cast<size_t>(M) * N;
+    const size_t total = static_cast<size_t>(M) * N, stride = part_floats(M, N);
     const size_t at = (static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
     if (at >= total)
         return;
-    // (N is a multiple of 4 here, so the four outputs share a row and the 16-byte accesses are aligned)
     v4f sum = {0.f, 0.f, 0.f, 0.f};
     for (int z = 0; z < ksplit; ++z) {
-        v4f *cell = reinterpret_cast<v4f *>(part + z * total + at);
+        v4f *cell = reinterpret_cast<v4f *>(part + z * stride + at);
         sum += *cell;
         *cell = v4f{0.f, 0.f, 0.f, 0.f};
     }
-    const int n = static_cast<int>(at % N);
     uint16_t r[4];
+    int n = bias ? static_cast<int>(at % N) : 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         r[i] = f2h(sum[i]);
-        if (bias)
-            r[i] = hadd(r[i], bias[n + i]);
+        if (bias) {
+            r[i] = hadd(r[i], bias[n]);
+            n = n + 1 == N ? 0 : n + 1;
+        }
     }
-    *reinterpret_cast<uint2 *>(out + at) = uint2{static_cast<uint32_t>(r[0]) | (static_cast<uint32_t>(r[1]) << 16),
-                                                 static_cast<uint32_t>(r[2]) | (static_cast<uint32_t>(r[3]) << 16)};
+    if (at + 4 <= total)
+        *reinterpret_cast<uint2 *>(out + at) = uint2{static_cast<uint32_t>(r[0]) | (static_cast<uint32_t>(r[1]) << 16),
+                                                     static_cast<uint32_t>(r[2]) | (static_cast<uint32_t>(r[3]) << 16)};
+    else
+        for (int i = 0; i < static_cast<int>(total - at); ++i)
+            out[at + i] = r[i];
 }
 
 // ------------------------------------------------- MFMA, 5 to 32 batch rows
@@ -2265,8 +2277,6 @@ int gemm_ksplit(int M, int N, int K)
 {
     const int tiles = gemm_tiles(M, N), steps = K / kGemmBK;
     int ks = 1;
-    if (N % 4)                  // the second pass works on four outputs of a row at a time
-        return 1;
     while (ks < kGemmMaxKsplit && tiles * ks * 2 <= kGemmSplitCus && steps % (ks * 2) == 0 && steps / (ks * 2) >= 16)
         ks *= 2;
     return ks;
@@ -2276,7 +2286,7 @@ int gemm_ksplit(int M, int N, int K)
 size_t gemm_workspace_bytes(int M, int N, int K)
 {
     const int ks = gemm_ksplit(M, N, K);
-    return ks == 1 ? 0 : static_cast<size_t>(ks) * M * N * sizeof(float);
+    return ks == 1 ? 0 : ks * part_floats(M, N) * sizeof(float);
 }
 
 hipError_t launch_gemm(int S, const GemmArgs &a, hipStream_t st)
@@ -2360,8 +2370,7 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
     const int j = lane & 31, h = lane >> 5;
     const int n0 = blockIdx.x * kPfBN, m0 = blockIdx.y * (32 * RB);
     const int n = n0 + 32 * wave + j, n_ld = min(n, N - 1);
-    const int steps = K / 64 / a.ksplit;                 // of this workgroup, even
-    const int p0 = blockIdx.z * steps, p_last = p0 + steps - 1;
+    const int p0 = blockIdx.z * a.part_steps, p_last = min(p0 + a.part_steps, K / 64) - 1;      // this workgroup's steps: an even number
     const int wpg = 2 * a.steps_per_group;               // words per group
 
     // bringing activations in: a thread takes operands q0 .. q0 + NQ - 1 of word xw of row xr of a step
@@ -2500,7 +2509,7 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
 
     // ---- D[i][jj] of a row block sits in lane jj + 32*((i/4)%2), register (i%4) + 4*(i/8)
     if (a.ksplit > 1) {
-        float *mine = a.part + blockIdx.z * (static_cast<size_t>(M) * N);
+        float *mine = a.part + blockIdx.z * part_floats(M, N);
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -2535,42 +2544,54 @@ bool gemm_lut_path_ok(int M, int N, int K, int S, int G)
 }
 
 // How the table look-up prefill kernel shares out a product: row blocks of 32 per workgroup, and parts of K (each an
-// even number of 16 steps and more).  A function of the shape only, so that the workspace can be sized without a device.
+// even number of steps, the last one perhaps fewer than the others).  A function of the shape only, so that the workspace
+// can be sized without a device.
 // Few row blocks mean more workgroups and more decodes of the weights, more parts of K more workgroups and partial
-// results to write and add up: the plan is the one of least estimated time.  Estimate, from launches of 8192 -> 28672
-// with 2 to 8 row blocks (0.94, 1.36, 1.84, 2.08 us a step): a step takes 0.55 + 0.2 RB us, a workgroup 2 us beside its
-// steps, and a split 2 us and its partial results once at 6 TB/s (the second pass reads and clears them: 9.9 us
-// at 333 rows x 6144 columns in 4 parts, where this says 7.5).  256 workgroups run at a time; beyond that the
-// last turn counts half (8192 -> 28672: 1.31 turns take the time of 1.70, 3.5 turns that of 3.68).
-// Against tiles of 256 rows throughout, 4 planes: 4096 -> 6144, 600 rows 86.5 -> 53.0 us (240 workgroups of 4 row blocks
-// for 144 of 7), 128 rows 30.6 -> 25.7; 4096 -> 4096, 192 rows 36.3 -> 26.0; 8192 -> 28672, 600 rows 472 -> 362.
+// results to write and add up: the plan is the one of least estimated time.  Estimate, fitted to 3600 launches (110 shapes,
+// 33 to 2048 rows, 512 to 28672 columns, K 512 to 28672, every number of row blocks, 1 to 16 parts; 8 % off on average, the
+// plan it picks 1.1 % behind the fastest): a step takes 0.38, 0.21 or 0.18 us (4, 3, 2 planes) and 0.2 us a row block, a
+// workgroup 3.6 us beside its steps, a split 3.3 us and 0.33 us per MB of partial results (written, read and cleared).
+// 256 workgroups run at a time, up to 13 % faster where fewer do; beyond that a last turn that is not full counts 0.63.
+// Against one tile height and parts by powers of two: 87 rows x 5378 columns, K 19456, 3 planes, 181 us unsplit (N no
+// multiple of 4 was never split) -> 37.5; 371 x 890, K 6144, 74.9 -> 23.2; 128 x 6144, K 4096, 30.6 -> 25.7.
 // The partial results take at most kGemmLutMaxParts bytes (384 tiles of 256 x 256): the bindings keep a workspace of the
 // largest size asked for, and beyond that a split gains nothing (8192 columns, K 28672, 768 rows: 429 us in 8 parts,
 // 201 MB, and 432 in 2).
 constexpr double kGemmLutMaxParts = 96. * 1024 * 1024;
+// Up to 16 steps (K = 1024) stay whole; longer ones are cut into parts of 4 steps and more.  (63 rows x 830 columns, K 1280:
+// 18.5 us whole, 13.3 in 2 parts of 10 steps, 10.1 in 5 of 4.)
+constexpr int kGemmLutWhole = 16, kGemmLutMinPart = 4;
 
 struct GemmLutPlan {
-    int rb, ksplit;
+    int rb, ksplit, part_steps;
 };
 
-GemmLutPlan gemm_lut_plan(int M, int N, int K, bool may_split)
+GemmLutPlan gemm_lut_plan(int M, int N, int K, int S, bool may_split)
 {
+    const double decode_us = S == 4 ? 0.38 : (S == 3 ? 0.21 : 0.18);
     const int blocks = (M + 31) / 32, columns = (N + kPfBN - 1) / kPfBN, steps = K / 64;
-    GemmLutPlan best{8, 1};
+    GemmLutPlan best{8, 1, steps};
     double best_us = 0.;
+    const int only_rb = env_switches().pf_rb, only_ks = env_switches().pf_ks;
+    int before = 0;
     for (int most = 8; most >= 2; --most) {
         const int tiles = (blocks + most - 1) / most;
-        const int rb = max(2, (blocks + tiles - 1) / tiles);
-        for (int ks = 1; ks <= 16; ks *= 2) {
-            if (ks > 1 && (!may_split || N % 4 || steps % (ks * 2) || steps / ks < 16 ||
-                           4. * ks * static_cast<double>(M) * N > kGemmLutMaxParts))
+        const int rb = only_rb ? only_rb : max(2, (blocks + tiles - 1) / tiles);
+        if (rb == before)                   // the same tiles again
+            continue;
+        before = rb;
+        for (int parts = 1; parts <= 16; ++parts) {
+            const int part_steps = (steps + 2 * parts - 1) / (2 * parts) * 2, ks = (steps + part_steps - 1) / part_steps;
+            if (ks != parts || (only_ks && ks != only_ks))
+                continue;
+            if (ks > 1 && (!may_split || steps <= kGemmLutWhole || part_steps < kGemmLutMinPart || 4. * ks * part_floats(M, N) > kGemmLutMaxParts))
                 break;
             const double turns = static_cast<double>(columns) * tiles * ks / kGemmSplitCus;
-            const double busy = turns <= 1. ? 1. : (ceil(turns) + turns) / 2.;
-            const double us = busy * (steps / ks * (0.55 + 0.2 * rb) + 2.) +
-                              (ks > 1 ? 2. + 4e-6 / 6. * ks * static_cast<double>(M) * N : 0.);
+            const double busy = turns <= 1. ? 0.87 + 0.13 * turns : 0.63 * ceil(turns) + 0.37 * turns;
+            const double us = busy * (part_steps * (decode_us + 0.2 * rb) + 3.6) +
+                              (ks > 1 ? 3.3 + 0.33e-6 * 4. * ks * part_floats(M, N) : 0.);
             if (best_us == 0. || us < best_us) {
-                best = GemmLutPlan{rb, ks};
+                best = GemmLutPlan{rb, ks, part_steps};
                 best_us = us;
             }
         }
@@ -3809,8 +3830,8 @@ size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G)
     if (mfma_path_ok(M, N, K, S, G) || lut_path_ok(M, N, K, S, G))
         return static_cast<size_t>(M) * N * sizeof(unsigned long long);
     if (gemm_lut_path_ok(M, N, K, S, G)) {
-        const int ks = gemm_lut_plan(M, N, K, true).ksplit;
-        return ks == 1 ? 0 : static_cast<size_t>(ks) * M * N * sizeof(float);
+        const int ks = gemm_lut_plan(M, N, K, S, true).ksplit;
+        return ks == 1 ? 0 : ks * part_floats(M, N) * sizeof(float);
     }
     if (gemm_path_ok(M, N, K, S, G) && !rows32_path_ok(M, N, K, S, G))
         return gemm_workspace_bytes(M, N, K);
@@ -4017,14 +4038,16 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         g.steps_per_group = G / kGemmBK;
         g.idx16 = idx_bytes == 2;
         g.ksplit = 1;
-        GemmLutPlan plan = gemm_lut_plan(M, N, K, true);
+        g.part_steps = K / kGemmBK;
+        GemmLutPlan plan = gemm_lut_plan(M, N, K, S, true);
         const int ks = plan.ksplit;
-        const size_t need = ks > 1 ? static_cast<size_t>(ks) * M * N * sizeof(float) : 0;
+        const size_t need = ks > 1 ? ks * part_floats(M, N) * sizeof(float) : 0;
         if (need && workspace && workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
             g.ksplit = ks;
+            g.part_steps = plan.part_steps;
             g.part = static_cast<float *>(workspace);
         } else if (need) {
-            plan = gemm_lut_plan(M, N, K, false);      // no workspace for the parts: not split
+            plan = gemm_lut_plan(M, N, K, S, false);      // no workspace for the parts: not split
         }
         if (env_switches().show_plan)
             fprintf(stderr, "sbvr_hip table look-up prefill M=%d N=%d K=%d S=%d: row blocks=%d ksplit=%d\n", M, N, K, S, plan.rb, g.ksplit);

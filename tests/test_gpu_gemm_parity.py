@@ -317,3 +317,22 @@ def test_two_row_blocks_where_tiles_are_few(oracle, M):
     """One or two column tiles: two row blocks a workgroup whatever the number of rows, K split or not."""
     run_case(oracle, 260, 512, 4, 128, M, 256, seed=M, expect=PREFILL)
     run_case(oracle, 256, 4096, 3, 256, M, 256, seed=M + 1, expect=PREFILL_SPLIT)
+
+
+@pytest.mark.parametrize("M,N,K,S,L,bias", [
+    (33, 1, 1152, 4, 256, True),           # 18 steps: parts of 4 and one of 2; a single column
+    (45, 333, 1280, 2, 300, False),        # an odd number of outputs: the last thread of the second pass has one
+    (70, 514, 1920, 3, 256, True),         # N even, no multiple of 4
+    (257, 1023, 2176, 4, 256, True),       # two column tiles, rows past a tile
+])
+def test_k_split_at_any_width_and_in_uneven_parts(oracle, M, N, K, S, L, bias):
+    """N no multiple of 4 and parts of K of different lengths: against the oracle, repeatable, the workspace left clean."""
+    import sbvr
+    from sbvr import hip, synth
+    dev = torch.device("cuda:0")
+    run_case(oracle, N, K, S, 128, M, L, seed=N + M, bias=bias, expect=PREFILL_SPLIT)
+    bvr, idx, cache = (t.to(dev) for t in synth.random_encoding(N, K, S, 128, L, seed=1))
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(2)).to(torch.float16).to(dev)
+    a = sbvr._sbvr_linear_f16(x, bvr, idx, cache, bvr_len=128)
+    assert torch.equal(a, sbvr._sbvr_linear_f16(x, bvr, idx, cache, bvr_len=128))
+    assert int(hip._workspaces[(dev.index, torch.cuda.current_stream(dev).cuda_stream)].count_nonzero()) == 0
