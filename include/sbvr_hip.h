@@ -43,7 +43,7 @@ const char *sbvr_hip_last_error(void);
 #define SBVR_HIP_KERNEL_PORTABLE 1       /* one thread per output */
 #define SBVR_HIP_KERNEL_DECODE 2         /* up to 16 rows (8 by default), plane sums on the matrix cores, exact activations */
 #define SBVR_HIP_KERNEL_ROWS32 3         /* up to 32 rows (9..32 by default), weights decoded to fp16 in registers */
-#define SBVR_HIP_KERNEL_PREFILL 4        /* weights decoded to fp16 tiles in LDS */
+#define SBVR_HIP_KERNEL_PREFILL 4        /* M > 32: weights decoded to fp16 in registers, output tiles of up to 256 rows */
 #define SBVR_HIP_KERNEL_PREFILL_SPLIT 5  /* the same with K split across workgroups (workspace given) */
 int sbvr_hip_last_kernel(void);
 
@@ -51,8 +51,8 @@ int sbvr_hip_last_kernel(void);
  *   EXACT      coefficients applied to plane sums in fp32, no per-weight rounding (decode and portable kernels);
  *   DECODE     every weight rounded to fp16 once, as decode() of sbvr/core.py:927-949 produces it (bin_combs @
  *              coeff, :345-366): the kernels that decode by table look-up;
- *   PLANEWISE  every weight an fp16 sum built plane by plane, S - 1 roundings (the kernels that decode
- *              arithmetically: 6 and 8 planes, groups of 32 or 64 elements). */
+ *   PLANEWISE  every weight an fp16 sum with up to S - 1 roundings (6 and 8 planes, groups of 32 or 64
+ *              elements: plane by plane, or closer: two or three table entries, or as with DECODE). */
 #define SBVR_HIP_ROUNDING_EXACT 1
 #define SBVR_HIP_ROUNDING_DECODE 2
 #define SBVR_HIP_ROUNDING_PLANEWISE 3
@@ -107,19 +107,18 @@ size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G);
  *                   K or G not a multiple of 128);
  *   prefill kernel  M > 32 (or 17..32 with flags bit 1), K and G multiples of 64,
  *                   same S; with a workspace, and where that is the faster, K is
- *                   split across workgroups.  With 2, 3 or 4 planes and K and G multiples
- *                   of 128 it is the kernel that decodes by table look-up in
- *                   registers (output tiles of 64 to 256 rows x 256, the weights never in LDS),
- *                   otherwise the one that decodes weight tiles into LDS; same
- *                   results up to the order of the fp32 additions;
+ *                   split across workgroups.  It decodes by table look-up in
+ *                   registers (output tiles of 64 to 256 rows x 256, the weights never
+ *                   in LDS), with 6 or 8 planes in two or three tables;
  *   portable kernel everything else (one thread per output), and with flags bit 0.
  * The 32-row and prefill kernels decode the weights to fp16 first.  Their table
  * look-up forms (2..4 planes) round the sum of a weight's coefficients once,
  * which is how decode() of sbvr/core.py:927-949 produces a weight (bin_combs @
  * coeff, :345-366): against x @ decode(W)^T they are as close as the decode
- * kernel is to the unrounded weights (2 fp16 ulps).  Their arithmetic forms (6
- * and 8 planes, groups of 32 or 64) add the coefficients up in fp16 plane by
- * plane.  Either way the error against unrounded weights is a few 1e-3 of the
+ * kernel is to the unrounded weights (2 fp16 ulps).  The 32-row kernel's
+ * arithmetic form (6 and 8 planes, groups of 32 or 64) adds the coefficients up in
+ * fp16 plane by plane, the prefill kernel with 6 or 8 planes two or three table
+ * entries.  Either way the error against unrounded weights is a few 1e-3 of the
  * RMS output, within the 1e-2 relative bound for outputs that are not small
  * against it.  sbvr_hip_last_rounding() tells which of the three a call took.
  * The reference has no kernel of exactly this form (its fp16-activation

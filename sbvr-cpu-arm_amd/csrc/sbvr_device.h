@@ -206,6 +206,72 @@ __device__ __forceinline__ v4u lut_operand(const LutTables<S> &t, const uint32_t
     return v4u{b0, b1, b2, b3};
 }
 
+// The same for 2 to 8 planes: up to 4 as above; 6 planes as two tables of three, 8 as two of three and one of two, whose
+// entries are added in fp16 (three or five roundings a weight, where the sum plane by plane has one per plane).  A table of
+// 16 entries takes 12 operations per four weights, one of 8 or 4 entries 5: 8 planes in two tables of 16 took 0.89 us
+// a step of the prefill kernel.
+template <int S>
+struct WeightTables {
+    static constexpr int H = S <= 4 ? S : 3, halves = S <= 4 ? 1 : 2;       // planes of the first table (and the second)
+    LutTables<H> t[halves];
+    LutTables<2> last;                                                      // (unused, hence no registers, up to 6 planes)
+};
+
+template <int S>
+struct WeightNibbles {
+    uint32_t Q[WeightTables<S>::halves][4], last[4];
+};
+
+template <int S>
+__device__ __forceinline__ void build_weight_tables(const uint32_t (&c)[(S + 1) / 2], WeightTables<S> &t)
+{
+    if constexpr (S <= 4) {
+        lut_build_tables<S>(c, t.t[0]);
+    } else {
+        const uint32_t first[2] = {c[0], c[1] & 0xffffu}, second[2] = {(c[1] >> 16) | (c[2] << 16), c[2] >> 16};
+        lut_build_tables<3>(first, t.t[0]);
+        lut_build_tables<3>(second, t.t[1]);
+        if constexpr (S == 8) {
+            const uint32_t third[1] = {c[3]};
+            lut_build_tables<2>(third, t.last);
+        }
+    }
+}
+
+template <int S>
+__device__ __forceinline__ void weight_nibbles(const uint32_t (&w)[S], WeightNibbles<S> &n)
+{
+    if constexpr (S <= 4) {
+        lut_nibble_words<S>(w, n.Q[0]);
+    } else {
+        const uint32_t first[3] = {w[0], w[1], w[2]}, second[3] = {w[3], w[4], w[5]};
+        lut_nibble_words<3>(first, n.Q[0]);
+        lut_nibble_words<3>(second, n.Q[1]);
+        if constexpr (S == 8) {
+            const uint32_t third[2] = {w[6], w[7]};
+            lut_nibble_words<2>(third, n.last);
+        }
+    }
+}
+
+// The B operand of MFMA q of the word (see lut_operand).
+template <int S>
+__device__ __forceinline__ v4u weight_operand(const WeightTables<S> &t, const WeightNibbles<S> &n, int q)
+{
+    v4u r = lut_operand<WeightTables<S>::H>(t.t[0], n.Q[0], q);
+    // (a line's coefficients grow in magnitude: the largest entries come last, so that one addition rounds at the sum's size)
+    auto add = [&](const v4u &u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            r[i] = __builtin_bit_cast(uint32_t, as_v2h(r[i]) + as_v2h(u[i]));
+    };
+    if constexpr (S > 4)
+        add(lut_operand<3>(t.t[1], n.Q[1], q));
+    if constexpr (S == 8)
+        add(lut_operand<2>(t.last, n.last, q));
+    return r;
+}
+
 }  // namespace
 
 #endif

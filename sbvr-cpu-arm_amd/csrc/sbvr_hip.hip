@@ -30,10 +30,9 @@
 // linear along (SiLU(gate) * up, or residual add + RMSNorm) while it turns the
 // activations into A operands: sbvr_hip_linear_f16_swiglu / _add_rmsnorm.
 //
-// Prefill path (M > 32): fp16 MFMA, fp32 accumulation; sbvr_gemm_lut_kernel (2..4
-// planes: weights decoded by table look-up in registers, activations shared
-// through LDS) or sbvr_gemm_mfma_kernel (weights decoded to fp16 tiles in LDS by
-// producer waves).  In between, 9..32 rows (17..32 with 6
+// Prefill path (M > 32): fp16 MFMA, fp32 accumulation; sbvr_gemm_lut_kernel
+// (weights decoded by table look-up in registers, activations shared
+// through LDS).  In between, 9..32 rows (17..32 with 6
 // or 8 planes): the batch rows are the 32 rows of one MFMA, weights decoded in
 // registers -- by table look-up for 2..4 planes (sbvr_gemm_rows32_lut_kernel),
 // arithmetically otherwise (sbvr_gemm_rows32_kernel).
@@ -1025,11 +1024,11 @@ struct GemvPlan {
 };
 
 // Development switches.  A library built with -DSBVR_DEV_SWITCHES reads them from the environment at every
-// call (SBVR_HIP_CT, _SP, _WAVES, _WSTRIDE, _SHOW_PLAN, _POPC_Q, _ROWDEQ_LANES, _LUT_ROWS, _PF_LUT, _PF_RB, _PF_KS); the
+// call (SBVR_HIP_CT, _SP, _WAVES, _WSTRIDE, _SHOW_PLAN, _POPC_Q, _ROWDEQ_LANES, _LUT_ROWS, _PF_RB, _PF_KS); the
 // library as shipped does not look at the environment: launch shapes and the choice of kernel (and with it the
 // rounding) depend on the arguments of a call alone.
 struct EnvSwitches {
-    int ct, sp, waves, wstride, show_plan, popc_q, rowdeq_lanes, lut_rows, pf_lut, pf_rb, pf_ks;
+    int ct, sp, waves, wstride, show_plan, popc_q, rowdeq_lanes, lut_rows, pf_rb, pf_ks;
 };
 
 #ifndef SBVR_DEV_SWITCHES
@@ -1048,8 +1047,7 @@ const EnvSwitches &env_switches()
             return v && *v ? atoi(v) : 0;
         };
         return EnvSwitches{get("SBVR_HIP_CT"), get("SBVR_HIP_SP"), get("SBVR_HIP_WAVES"), get("SBVR_HIP_WSTRIDE"),
-                           get("SBVR_HIP_SHOW_PLAN"), get("SBVR_HIP_POPC_Q"), get("SBVR_HIP_ROWDEQ_LANES"), get("SBVR_HIP_LUT_ROWS"), get("SBVR_HIP_PF_LUT"),
-                           get("SBVR_HIP_PF_RB"), get("SBVR_HIP_PF_KS")};
+                           get("SBVR_HIP_SHOW_PLAN"), get("SBVR_HIP_POPC_Q"), get("SBVR_HIP_ROWDEQ_LANES"), get("SBVR_HIP_LUT_ROWS"), get("SBVR_HIP_PF_RB"), get("SBVR_HIP_PF_KS")};
     }();
     return e;
 }
@@ -1420,30 +1418,7 @@ hipError_t launch_batch(int S, const GemvArgs &a, const BatchPlan &p, hipStream_
 
 // ------------------------------------------------------------- MFMA prefill
 
-// Prefill path (M > 16): a dense contraction.  A workgroup owns a 256 x 128
-// tile of the output and walks K in steps of 64.  Its 12 waves have two jobs:
-//   * waves 4-11 produce the weight tile of step t+1 while step t is consumed:
-//     128 x 64 weights decoded to fp16: thread (column, word, half) holds the
-//     S plane words of one 32-bit word of K and the coefficient line of its
-//     group, and forms w = sum_j (bit_j ? c_j : 0) for 16 of the word's
-//     elements, two of them (k, k+16) per packed fp16 operation:
-//     (word >> k) & 0x00010001 times the 16-bit pattern of c_j is that pattern,
-//     or zero, in each half.  Their global loads run three steps ahead of the
-//     consumers, in three register sets used in rotation;
-//   * waves 0-3 run v_mfma_f32_32x32x16_f16 over the two tiles (each wave
-//     128 x 64 of the output, 8 accumulator blocks) and, before that, send for
-//     the 256 x 64 activations of the step after the next: global memory to LDS directly,
-//     no registers, the data lands while the MFMAs run.
-// A SIMD holds one consumer and two producers, so the decode (VALU) and the
-// MFMAs overlap.  The weight tile has two buffers, the activation tile three (its
-// loads go out two steps ahead); one barrier per step.  Rows of the
-// LDS tiles are 128 bytes; 16-byte chunk c of row r is stored at chunk
-// c ^ ((r >> 1) & 7), which keeps the 16-byte operand reads of a quarter wave
-// (16 rows, two of them per 256-byte line of banks) on different banks.
-constexpr int kGemmBM = 256, kGemmBN = 128, kGemmBK = 64, kGemmThreads = 768;     // 4 consumer + 8 producer waves
-constexpr int kGemmABufs = 3;       // activation tiles in LDS: the one in use and the next two
-constexpr int kGemmATile = kGemmBM * kGemmBK * 2, kGemmBTile = kGemmBN * kGemmBK * 2;
-
+constexpr int kGemmBK = 64;          // elements of K a step of the prefill kernel takes
 
 struct GemmArgs {
     const uint16_t *x;
@@ -1456,11 +1431,8 @@ struct GemmArgs {
     int steps_per_group;   // G / 64
     int idx16;
     int ksplit;            // workgroups along K (blockIdx.z); 1: results go straight to out
-    int part_steps;        // steps of 64 along K of a part (the last one's may be fewer); table look-up kernel only
+    int part_steps;        // steps of 64 along K of a part (the last one's may be fewer)
     float *part;           // ksplit > 1: (ksplit, M, N) fp32 partial results, all zero between launches
-#ifdef SBVR_TRACE
-    unsigned long long *trace;
-#endif
 };
 
 // Floats from one part's partial results to the next's: M * N, and up to a multiple of 4, so that every part starts on
@@ -1486,291 +1458,6 @@ __device__ __forceinline__ void load_line_coeffs(const uint16_t *cp, uint32_t (&
 #pragma unroll
         for (int j = 0; j < (S + 1) / 2; ++j)
             cr[j] = static_cast<uint32_t>(cp[2 * j]) | (2 * j + 1 < S ? static_cast<uint32_t>(cp[2 * j + 1]) << 16 : 0u);
-    }
-}
-
-#ifdef SBVR_TRACE
-#define SBVR_GSTAMP(step, slot)                                                                   \
-    do {                                                                                          \
-        if (a.trace && blockIdx.x == 7 && blockIdx.y == 1 && (threadIdx.x & 63) == 0 && (step) < 96) \
-            a.trace[(step) * 8 + (slot)] = wall_clock64();                                        \
-    } while (0)
-#else
-#define SBVR_GSTAMP(step, slot) do { } while (0)
-#endif
-
-template <int S>
-__global__ void __launch_bounds__(kGemmThreads)
-__attribute__((amdgpu_waves_per_eu(3, 3)))
-sbvr_gemm_mfma_kernel(const GemmArgs a)
-{
-    extern __shared__ __align__(16) unsigned char gsm[];
-    unsigned char *const As = gsm;                       // 2 tiles
-    unsigned char *const Bs = gsm + kGemmABufs * kGemmATile;      // 2 tiles
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int N = a.N, K = a.K, M = a.M;
-    const int n0 = blockIdx.x * kGemmBN, m0 = blockIdx.y * kGemmBM;
-    const int steps = K / kGemmBK / a.ksplit;            // of this workgroup: tiles t_base .. t_base + steps - 1 of K
-    const int t_base = blockIdx.z * steps;
-    const int rounds = (steps + 2) / 3;                  // both kinds of waves run 3 * rounds steps (same barriers)
-
-    if (wave >= 4) {
-        // ------------------------------------------------------------ producers
-        const int pt = tid - 256;
-        // decode role: column of the tile, word of the step, and which 8 of the word's 16 pairs (k, k+16)
-        const int bn = pt & (kGemmBN - 1), bw = (pt >> 7) & 1, bh = pt >> 8;
-        const int n_ld = min(n0 + bn, N - 1);
-        const int b_dst = bn * 128;
-        const int sw = (bn >> 1) & 7, cb = bw * 4;       // chunk swizzle of row bn, see the consumers
-
-        constexpr int CW = (S + 1) / 2;
-        uint32_t wreg0[S], wreg1[S], wreg2[S];           // three register sets, used in rotation
-        uint32_t creg0[CW], creg1[CW], creg2[CW];
-        // The aligned 32-bit word that holds the line index of the tile a register set is filled with next:
-        // loaded when the set is requested, used three steps later by the same set's next request, and
-        // untouched in between (a move, or a byte load's zero extension, ends up at the top of the loop,
-        // where it makes the step wait for the youngest loads in flight).
-        uint32_t raw0 = 0, raw1 = 0, raw2 = 0;
-
-        // (two byte loads whatever the index width: a branch between a 16-bit and an 8-bit load
-        // inside the loop would make every later wait a wait for all loads)
-        auto line_address = [&](int t) __attribute__((always_inline)) -> uintptr_t {
-            const size_t at = (static_cast<size_t>((t_base + t) / a.steps_per_group) * N + n_ld) << a.idx16;
-            return reinterpret_cast<uintptr_t>(static_cast<const uint8_t *>(a.idx) + at);
-        };
-        auto load_line = [&](int t, uint32_t &raw) __attribute__((always_inline)) {
-            // (a global-memory pointer by type: from a bare integer the compiler would make a flat load,
-            // whose completion order it does not know)
-            raw = *reinterpret_cast<const __attribute__((address_space(1))) uint32_t *>(line_address(t) & ~static_cast<uintptr_t>(3));
-        };
-        auto line_of = [&](int t, uint32_t raw) __attribute__((always_inline)) -> int {
-            const uint32_t v = raw >> (8 * static_cast<uint32_t>(line_address(t) & 3));
-            return min(static_cast<int>(a.idx16 ? v & 0xffffu : v & 0xffu), a.L - 1);
-        };
-        // global loads of tile t into one register set
-        auto request = [&](int t, uint32_t (&wr)[S], uint32_t (&cr)[CW], uint32_t &raw) __attribute__((always_inline)) {
-            const int k0 = (t_base + t) * kGemmBK;
-            const uint32_t *wp = a.bvr + (static_cast<size_t>(k0 / 32 + bw) * N + n_ld) * S;
-            // (ordinary loads: every row tile of the launch reads these again; non-temporal ones measured 2-3 % slower)
-            const Planes<S> pl = load_planes<S>(wp);
-#pragma unroll
-            for (int j = 0; j < S; ++j)
-                wr[j] = pl.w[j];
-            asm volatile("" : "+v"(raw));                // not to be taken apart before this step (see pin)
-            const uint16_t *cp = a.cache + static_cast<size_t>(line_of(t, raw)) * S;
-            load_line_coeffs<S>(cp, cr);
-            load_line(min(t + 3, steps - 1), raw);
-        };
-        // Makes a register set opaque at the start of the step that decodes it: without this the compiler
-        // moves part of the decode up into the step before (arithmetic may cross a barrier), where the
-        // set's loads are the youngest in flight and the wait for them drains the whole queue.
-        auto pin = [&](uint32_t (&wr)[S], uint32_t (&cr)[CW], uint32_t &) __attribute__((always_inline)) {
-#pragma unroll
-            for (int j = 0; j < S; ++j)
-                asm volatile("" : "+v"(wr[j]));
-#pragma unroll
-            for (int j = 0; j < CW; ++j)
-                asm volatile("" : "+v"(cr[j]));
-        };
-        // one register set -> LDS buffers t % 2
-        auto produce = [&](int t, const uint32_t (&wr)[S], const uint32_t (&cr)[CW], uint32_t) __attribute__((always_inline)) {
-            unsigned char *Bt = Bs + (t & 1) * kGemmBTile;
-            uint32_t cbits[S];
-#pragma unroll
-            for (int j = 0; j < S; ++j)
-                cbits[j] = j & 1 ? cr[j / 2] >> 16 : cr[j / 2] & 0xffffu;
-            uint32_t wsh[S];
-#pragma unroll
-            for (int j = 0; j < S; ++j)
-                wsh[j] = wr[j] >> (8 * bh);
-            uint32_t pr[8];          // pr[e] = {w[8 bh + e], w[16 + 8 bh + e]}
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                v2h v = __builtin_bit_cast(v2h, __umul24((wsh[0] >> e) & 0x00010001u, cbits[0]));
-#pragma unroll
-                for (int j = 1; j < S; ++j)
-                    v = v + __builtin_bit_cast(v2h, __umul24((wsh[j] >> e) & 0x00010001u, cbits[j]));
-                pr[e] = __builtin_bit_cast(uint32_t, v);
-            }
-            v4u lo, hi;              // k 8 bh .. + 7 (low halves) and 16 + 8 bh .. + 7 (high halves)
-            lo.x = __builtin_amdgcn_perm(pr[1], pr[0], 0x05040100u); hi.x = __builtin_amdgcn_perm(pr[1], pr[0], 0x07060302u);
-            lo.y = __builtin_amdgcn_perm(pr[3], pr[2], 0x05040100u); hi.y = __builtin_amdgcn_perm(pr[3], pr[2], 0x07060302u);
-            lo.z = __builtin_amdgcn_perm(pr[5], pr[4], 0x05040100u); hi.z = __builtin_amdgcn_perm(pr[5], pr[4], 0x07060302u);
-            lo.w = __builtin_amdgcn_perm(pr[7], pr[6], 0x05040100u); hi.w = __builtin_amdgcn_perm(pr[7], pr[6], 0x07060302u);
-            *reinterpret_cast<v4u *>(Bt + b_dst + (((cb + bh) ^ sw) << 4)) = lo;
-            *reinterpret_cast<v4u *>(Bt + b_dst + (((cb + 2 + bh) ^ sw) << 4)) = hi;
-        };
-#define SBVR_SET(n) wreg##n, creg##n, raw##n
-        // Requests are never conditional (beyond the last tile they repeat it): after a
-        // branch that may or may not have issued loads, the wait for an older set would
-        // have to assume it had not, and wait for everything.
-        const int last = steps - 1;
-        load_line(0, raw0);
-        load_line(min(1, last), raw1);
-        load_line(min(2, last), raw2);
-        request(0, SBVR_SET(0));
-        request(min(1, last), SBVR_SET(1));
-        request(min(2, last), SBVR_SET(2));
-        produce(0, SBVR_SET(0));
-        __syncthreads();
-        // step i: the consumers read tile i; tile i+1 goes to the other buffers, tile i+3 is requested
-        for (int r = 0; r < rounds; ++r) {
-            const int i = 3 * r;
-            // (tiles beyond the last are produced too, from repeated loads, into buffers nobody reads:
-            // a loop body without branches keeps the waits of the three register sets apart)
-            if (wave == 4) SBVR_GSTAMP(i, 2);
-            pin(SBVR_SET(1));
-            request(min(i + 3, last), SBVR_SET(0));
-            if (wave == 4) SBVR_GSTAMP(i, 3);
-            produce(i + 1, SBVR_SET(1));
-            if (wave == 4) SBVR_GSTAMP(i, 4);
-            __syncthreads();
-            if (wave == 4) SBVR_GSTAMP(i + 1, 2);
-            pin(SBVR_SET(2));
-            request(min(i + 4, last), SBVR_SET(1));
-            if (wave == 4) SBVR_GSTAMP(i + 1, 3);
-            produce(i + 2, SBVR_SET(2));
-            if (wave == 4) SBVR_GSTAMP(i + 1, 4);
-            __syncthreads();
-            if (wave == 4) SBVR_GSTAMP(i + 2, 2);
-            pin(SBVR_SET(0));
-            request(min(i + 5, last), SBVR_SET(2));
-            if (wave == 4) SBVR_GSTAMP(i + 2, 3);
-            produce(i + 3, SBVR_SET(0));
-            if (wave == 4) SBVR_GSTAMP(i + 2, 4);
-            __syncthreads();
-        }
-#undef SBVR_SET
-        return;
-    }
-
-    // ---------------------------------------------------------------- consumers
-    v16f acc[4][2];
-#pragma unroll
-    for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                acc[bi][bj][r] = 0.f;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int arow = wm * 128 + (lane & 31), brow = wn * 64 + (lane & 31);      // + 32 bi / bj: same (row >> 1) & 7
-    // Chunk c of tile row r sits at chunk position c ^ ((r >> 1) & 7) of the row's 128 bytes.  A 16-byte read
-    // is served 16 lanes (rows) at a time by 64 banks of 4 bytes, i.e. two rows side by side: with the row pair
-    // as the swizzle key the 16 rows hit 16 different bank groups (keyed by r & 7, rows r and r + 8 collided
-    // and every read took two turns).
-    const int rsw = (lane >> 1) & 7, chi = lane >> 5;
-    // The activation tile goes from global memory straight into LDS (no registers): instruction j
-    // of wave w fills the 1 KiB block 8w + j, i.e. rows 8 (8w + j) .. + 7, lane l the 16-byte slot l
-    // of it; with the row swizzle, slot l of a block holds chunk (l & 7) ^ ((4j + (l >> 4)) & 7) of row l >> 3.
-    uint32_t xoff[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int row = 8 * (8 * wave + j) + (lane >> 3);
-        xoff[j] = static_cast<uint32_t>(min(m0 + row, M - 1)) * K + 8 * ((lane & 7) ^ ((row >> 1) & 7));     // M * K < 2^31 (checked)
-    }
-    auto fetch_a = [&](int t, int buf) __attribute__((always_inline)) {        // tile t -> buffer buf, asynchronously
-        unsigned char *dst = As + buf * kGemmATile + wave * 8192;
-        const uint16_t *src = a.x + static_cast<size_t>(t_base + t) * kGemmBK;
-        // Written as assembly (M0 = LDS address of lane 0's slot): the compiler counts the builtin form as a
-        // memory operation whose order of completion it does not know, and from then on turns every wait for
-        // an LDS read into a wait for all of them.
-        const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst));
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                         :: "v"(src + xoff[j]), "s"(lds + j * 1024) : "memory", "m0");
-    };
-    fetch_a(0, 0);
-    fetch_a(min(1, steps - 1), 1);
-    __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0): the tiles are in LDS
-    int cur = 0;                                 // activation buffer of tile i
-    __syncthreads();
-    // operand registers of two k-slices in turn: the reads of slice s+1 are issued before the MFMAs of slice s
-    auto read_slice = [&](const unsigned char *At, const unsigned char *Bt, int ks, v8h (&af)[4], v8h (&bf)[2])
-                          __attribute__((always_inline)) {
-        const int coff = ((2 * ks + chi) ^ rsw) << 4;
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-            af[bi] = *reinterpret_cast<const v8h *>(At + (arow + 32 * bi) * 128 + coff);
-#pragma unroll
-        for (int bj = 0; bj < 2; ++bj)
-            bf[bj] = *reinterpret_cast<const v8h *>(Bt + (brow + 32 * bj) * 128 + coff);
-    };
-    auto mfma_slice = [&](const v8h (&af)[4], const v8h (&bf)[2]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 2; ++bj)
-                acc[bi][bj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[bi], bf[bj], acc[bi][bj], 0, 0, 0);
-    };
-    for (int i = 0; i < 3 * rounds; ++i) {
-        if (i < steps) {
-            const unsigned char *At = As + cur * kGemmATile, *Bt = Bs + (i & 1) * kGemmBTile;
-            if (wave == 0) SBVR_GSTAMP(i, 0);
-            // the tile after the next goes to the buffer that the tile before this one has left; it has two
-            // steps to land
-            fetch_a(min(i + 2, steps - 1), cur == 0 ? 2 : cur - 1);
-            // (With 168 registers a wave the compiler keeps one activation operand at a time and moves each
-            // read down to its MFMAs: fenced into the order written here the loop needs about 200.)
-            v8h af0[4], bf0[2], af1[4], bf1[2];
-            read_slice(At, Bt, 0, af0, bf0);
-            read_slice(At, Bt, 1, af1, bf1);
-            mfma_slice(af0, bf0);
-            read_slice(At, Bt, 2, af0, bf0);
-            mfma_slice(af1, bf1);
-            read_slice(At, Bt, 3, af1, bf1);
-            mfma_slice(af0, bf0);
-            mfma_slice(af1, bf1);
-            if (wave == 0) SBVR_GSTAMP(i, 1);
-            __builtin_amdgcn_sched_barrier(0);   // (or the wait moves up in front of the MFMAs)
-            __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): all but the 8 loads above, i.e. this wave's part of the next tile is in LDS
-            cur = cur == 2 ? 0 : cur + 1;
-        }
-        __syncthreads();
-    }
-
-    __builtin_amdgcn_s_waitcnt(0x0F70);          // no load into LDS is left in flight when the wave ends
-
-    // ---- D[i][j] sits in lane j + 32*((i/4)%2), register (i%4) + 4*(i/8)
-    if (a.ksplit > 1) {
-        // K split across workgroups: every workgroup leaves its fp32 tile in `part`; sbvr_gemm_reduce_kernel,
-        // launched behind this kernel, adds the tiles up in the order of blockIdx.z and rounds once.
-        float *mine = a.part + blockIdx.z * part_floats(M, N);
-#pragma unroll
-        for (int bj = 0; bj < 2; ++bj) {
-            const int n = n0 + wn * 64 + bj * 32 + (lane & 31);
-#pragma unroll
-            for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + wm * 128 + bi * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                    if (m < M && n < N)
-                        mine[static_cast<size_t>(m) * N + n] = acc[bi][bj][r];
-                }
-        }
-        return;
-    }
-#pragma unroll
-    for (int bj = 0; bj < 2; ++bj) {
-        const int n = n0 + wn * 64 + bj * 32 + (lane & 31);
-        if (n >= N)
-            continue;
-        const uint16_t bias = a.bias ? a.bias[n] : 0;
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = m0 + wm * 128 + bi * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (m < M) {
-                    uint16_t v = f2h(acc[bi][bj][r]);
-                    if (a.bias)
-                        v = hadd(v, bias);
-                    a.out[static_cast<size_t>(m) * N + n] = v;
-                }
-            }
     }
 }
 
@@ -1817,7 +1504,8 @@ sbvr_gemm_reduce_kernel(float *__restrict__ part, const uint16_t *__restrict__ b
 // of A, read from global memory as they are, and 32 columns of decoded weights
 // as B.  A wave walks a range of K one 32-bit word (two MFMAs) at a time; lane
 // (column j, half h) decodes bits 8h..8h+7 and 16+8h..16+8h+7 of the word, two
-// elements (k, k+16) per packed fp16 operation as in the prefill kernel, which
+// elements (k, k+16) per packed fp16 operation: (word >> k) & 0x00010001 times the
+// 16-bit pattern of a coefficient is that pattern, or zero, in each half.  These
 // are exactly its B elements of the two MFMAs.  No LDS on the way; the 8 waves
 // of a workgroup split K and add their 32 x 32 partial results in LDS at the
 // end.  Bound by the decode arithmetic (about 7.5 VALU operations per weight),
@@ -1871,7 +1559,7 @@ sbvr_gemm_rows32_kernel(const RowsArgs a)
             const size_t at = (static_cast<size_t>(w / a.words_per_group) * N + n_ld) << a.idx16;
             const uint8_t *ib = static_cast<const uint8_t *>(a.idx);
             const int lo = ib[at], hi = ib[at + a.idx16];      // two byte loads whatever the width: no branch
-            line[i] = lo | (hi << 16);                          // raw: decoded where it is used (see the prefill kernel)
+            line[i] = lo | (hi << 16);                          // raw: decoded where it is used
         }
     };
     auto load_block = [&](int w0, Block &b, const int (&line)[kRowsBlock]) __attribute__((always_inline)) {
@@ -1935,7 +1623,8 @@ sbvr_gemm_rows32_kernel(const RowsArgs a)
     };
 
     // two register blocks in turn; the line indices run one block further ahead
-    // (loads are never conditional, see the prefill kernel)
+    // (Loads are never conditional: beyond the last block they repeat it.  After a branch that may or may not have issued
+    // loads, the wait for an older block would have to assume it had not, and wait for everything.)
     Block b0, b1;
     int line[kRowsBlock];
     load_lines(w_begin, line);
@@ -2257,80 +1946,9 @@ hipError_t launch_rows32_lut(int S, RowsArgs a, hipStream_t st)
     return hipGetLastError();
 }
 
-bool gemm_path_ok(int M, int N, int K, int S, int G)
-{
-    return M > kMaxM && K % kGemmBK == 0 && G % kGemmBK == 0 && (S == 2 || S == 3 || S == 4 || S == 6 || S == 8) &&
-           static_cast<double>(K / 32) * N * S < 2147483648.0 && static_cast<double>(M) * K < 2147483648.0;
-}
-
-// Workgroups along K for the prefill kernel: as long as the output tiles alone leave half of the
-// chip's 256 CUs without a workgroup, and a part keeps at least 16 steps.  A function of the shape
-// only, so that the workspace can be sized without a device.
-constexpr int kGemmSplitCus = 256, kGemmMaxKsplit = 8;
-
-int gemm_tiles(int M, int N)
-{
-    return ((N + kGemmBN - 1) / kGemmBN) * ((M + kGemmBM - 1) / kGemmBM);
-}
-
-int gemm_ksplit(int M, int N, int K)
-{
-    const int tiles = gemm_tiles(M, N), steps = K / kGemmBK;
-    int ks = 1;
-    while (ks < kGemmMaxKsplit && tiles * ks * 2 <= kGemmSplitCus && steps % (ks * 2) == 0 && steps / (ks * 2) >= 16)
-        ks *= 2;
-    return ks;
-}
-
-// Workspace of the split prefill launch: the partial results.
-size_t gemm_workspace_bytes(int M, int N, int K)
-{
-    const int ks = gemm_ksplit(M, N, K);
-    return ks == 1 ? 0 : ks * part_floats(M, N) * sizeof(float);
-}
-
-hipError_t launch_gemm(int S, const GemmArgs &a, hipStream_t st)
-{
-    const dim3 grid(static_cast<unsigned>((a.N + kGemmBN - 1) / kGemmBN), static_cast<unsigned>((a.M + kGemmBM - 1) / kGemmBM),
-                    static_cast<unsigned>(a.ksplit));
-    const dim3 block(kGemmThreads);
-    const size_t lds = kGemmABufs * kGemmATile + 2 * kGemmBTile;      // 128 KiB: above the 64 KiB a kernel gets without asking
-#define SBVR_GEMM_LAUNCH(SS)                                                                                   \
-    {                                                                                                          \
-        static bool raised_on[16] = {};                                                                        \
-        std::lock_guard<std::mutex> guard(g_dev_lock);                                                                        \
-        int dev_now = 0;                                                                                       \
-        if (hipGetDevice(&dev_now) != hipSuccess || dev_now < 0 || dev_now >= 16)                              \
-            dev_now = 0;                                                                                       \
-        bool &raised = raised_on[dev_now];                                                                     \
-        if (!raised) {                                                                                         \
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(sbvr_gemm_mfma_kernel<SS>), \
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)); \
-            if (e != hipSuccess)                                                                               \
-                return e;                                                                                      \
-            raised = true;                                                                                     \
-        }                                                                                                      \
-        hipLaunchKernelGGL(sbvr_gemm_mfma_kernel<SS>, grid, block, lds, st, a);                                \
-    }                                                                                                          \
-    break
-    switch (S) {
-    case 4: SBVR_GEMM_LAUNCH(4);
-#ifndef SBVR_FAST_BUILD
-    case 2: SBVR_GEMM_LAUNCH(2);
-    case 3: SBVR_GEMM_LAUNCH(3);
-    case 6: SBVR_GEMM_LAUNCH(6);
-    case 8: SBVR_GEMM_LAUNCH(8);
-#endif
-    default: return hipErrorInvalidConfiguration;
-    }
-#undef SBVR_GEMM_LAUNCH
-    return hipGetLastError();
-}
-
 // ------------------------------------------- MFMA prefill with the weights decoded by table look-up
 //
-// The prefill contraction with the decode of sbvr_gemm_rows32_lut_kernel: no producer and consumer waves and no
-// weight tile in LDS.  A workgroup of 8 waves owns RB row blocks of 32 x 256 columns of the output; wave w owns columns
+// A dense contraction with the decode of sbvr_gemm_rows32_lut_kernel.  A workgroup of 8 waves owns RB row blocks of 32 x 256 columns of the output; wave w owns columns
 // 32w .. 32w+31 for all its rows (8 row blocks: 128 accumulator registers a lane).  Per step of 64 elements
 // of K a lane (column j, half h) decodes its word 2i + h of column j by table look-up straight into the B operands
 // of four MFMAs (16 registers), and the wave runs them against the row blocks: 4 RB MFMAs of 32 clocks per 32
@@ -2339,8 +1957,12 @@ hipError_t launch_gemm(int S, const GemmArgs &a, hipStream_t st)
 // order the MFMAs want (see sbvr_gemm_rows32_lut_kernel: that permutation is done once, by the thread that
 // brings a (row, word) in, not once per wave): rows 144 bytes apart, two buffers, one barrier per step.  The loads
 // of the step after the next one's (activations, plane words) are in flight while a step is computed.
-// 2, 3 or 4 planes, K and G multiples of 128 (the two steps of a loop iteration share a coefficient line).
-// K can be split across workgroups (blockIdx.z) as in sbvr_gemm_mfma_kernel: fp32 partial tiles, second pass.
+// K can be split across workgroups (blockIdx.z): fp32 partial tiles, added up by a second pass.
+// 6 and 8 planes look a weight up in two or three tables (build_weight_tables).  A kernel with weight tiles in LDS, decoded
+// plane by plane by producer waves, served them and groups of 64 before: 2048 x 8192, K 8192, 8 planes 405 us there
+// and 318 here, 319 x 7714, K 4096 59 and 50, 512 x 4096, K 4096 44 and 41.6; 2000 x 16000, K 8192, 6 planes 750 and 569; groups of
+// 64, 4 planes, 2048 x 8192, K 8192 341 and 281.  Behind it only where 8 planes and groups of 64 meet tiles that fit the
+// chip exactly (256 x 14336, K 4096: 61.4 and 62.3).
 constexpr int kPfWaves = 8, kPfBN = 256, kPfRow = 144;
 
 constexpr int pf_loader_blocks(int rb) { return rb <= 2 ? 2 : (rb <= 4 ? 4 : 8); }
@@ -2349,11 +1971,12 @@ constexpr int pf_loader_blocks(int rb) { return rb <= 2 ? 2 : (rb <= 4 ? 4 : 8);
 // block beyond M costs as much as one inside it: the rows are shared out evenly over the tiles (gemm_lut_plan).
 // With 2, 4, 6 and 8 row blocks a step takes 0.94, 1.36, 1.84 and 2.08 us (8192 -> 28672, 4 planes); 64 / 128 / 192 /
 // 333 rows 60 / 87 / 118 / 198 us there, where 8 row blocks for any number of rows took 131 / 133 / 139 / 248.
-template <int S, int RB>
+// kShare: groups of a multiple of 128 elements, the two steps of a loop iteration share a coefficient line; otherwise each
+// has its own index load, gather and table, and the number of steps may be odd.
+template <int S, int RB, bool kShare>
 __global__ void __launch_bounds__(64 * kPfWaves)
 sbvr_gemm_lut_kernel(const GemmArgs a)
 {
-    static_assert(S >= 2 && S <= 4, "tables of 4, 8 or 16 entries");
     static_assert(RB >= 2 && RB <= 8, "row blocks of a workgroup");
     // of the four MFMA operands of a (row, word), a thread brings in NQ (1 or 2 where 512 threads then cover the rows)
     constexpr int NQ = pf_loader_blocks(RB) / 2;
@@ -2370,7 +1993,7 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
     const int j = lane & 31, h = lane >> 5;
     const int n0 = blockIdx.x * kPfBN, m0 = blockIdx.y * (32 * RB);
     const int n = n0 + 32 * wave + j, n_ld = min(n, N - 1);
-    const int p0 = blockIdx.z * a.part_steps, p_last = min(p0 + a.part_steps, K / 64) - 1;      // this workgroup's steps: an even number
+    const int p0 = blockIdx.z * a.part_steps, p_last = min(p0 + a.part_steps, K / 64) - 1;      // this workgroup's steps (kShare: an even number)
     const int wpg = 2 * a.steps_per_group;               // words per group
 
     // bringing activations in: a thread takes operands q0 .. q0 + NQ - 1 of word xw of row xr of a step
@@ -2428,8 +2051,8 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
         }
     };
 
-    LutTables<S> tables;
-    auto build_table = [&](const uint32_t (&c)[CW]) __attribute__((always_inline)) { lut_build_tables<S>(c, tables); };
+    WeightTables<S> tables;
+    auto build_table = [&](const uint32_t (&c)[CW]) __attribute__((always_inline)) { build_weight_tables<S>(c, tables); };
 
     v16f acc[RB];
 #pragma unroll
@@ -2439,54 +2062,70 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
             acc[rb][r] = 0.f;
 
     auto compute = [&](const uint32_t (&w)[S], int buf) __attribute__((always_inline)) {
-        uint32_t Q[4];
-        lut_nibble_words<S>(w, Q);
-        auto operand = [&](int q) __attribute__((always_inline)) -> v4u { return lut_operand<S>(tables, Q, q); };
+        WeightNibbles<S> nibbles;
+        weight_nibbles<S>(w, nibbles);
+        auto operand = [&](int q) __attribute__((always_inline)) -> v4u { return weight_operand<S>(tables, nibbles, q); };
         // MFMA q of all row blocks in a row (RB different accumulators), its RB activation operands read while
-        // MFMA q - 1 runs, and the look-ups of operand q + 1 in the shadow of the matrix pipe
+        // MFMA q - 1 runs, and the look-ups of operand q + 1 in the shadow of the matrix pipe.  (Two sets of RB operands;
+        // 8 row blocks of 6 or 8 planes go in two turns of 4 per MFMA, or the registers do not suffice)
+        constexpr int RG = RB == 8 && S > 4 ? 4 : RB, turns = RB / RG;
         const unsigned char *xt = xrd + buf * kTile;
-        v4u A[2][RB];
-        auto read_a = [&](int q, v4u (&dst)[RB]) __attribute__((always_inline)) {
+        v4u A[2][RG];
+        auto read_a = [&](int i, v4u (&dst)[RG]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-                dst[rb] = *reinterpret_cast<const v4u *>(xt + 32 * rb * kPfRow + 16 * q);
+            for (int rb = 0; rb < RG; ++rb)
+                dst[rb] = *reinterpret_cast<const v4u *>(xt + 32 * (i % turns * RG + rb) * kPfRow + 16 * (i / turns));
         };
         read_a(0, A[0]);
-        v4u Bq = operand(0);
+        v4u Bq = operand(0), Bn = Bq;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            v4u Bn = Bq;
-            if (q < 3) {
-                read_a(q + 1, A[(q + 1) & 1]);
+        for (int i = 0; i < 4 * turns; ++i) {
+            if (i < 4 * turns - 1) {
+                read_a(i + 1, A[(i + 1) & 1]);
                 __builtin_amdgcn_sched_barrier(0);
-                Bn = operand(q + 1);
             }
+            if (i % turns == 0 && i / turns < 3)
+                Bn = operand(i / turns + 1);
 #pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-                acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, A[q & 1][rb]), __builtin_bit_cast(v8h, Bq), acc[rb], 0, 0, 0);
-            Bq = Bn;
+            for (int rb = 0; rb < RG; ++rb)
+                acc[i % turns * RG + rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, A[i & 1][rb]), __builtin_bit_cast(v8h, Bq),
+                                                                                  acc[i % turns * RG + rb], 0, 0, 0);
+            if (i % turns == turns - 1)
+                Bq = Bn;
         }
     };
 
     // -- prologue: the first step's activations into buffer 0, everything of the second in flight
     // (decoding a step's operands one step ahead, in the shadow of the step before's MFMAs, measured no faster)
-    uint32_t wa[S], wb[S], c[CW], c_next[CW];
+    constexpr int NL = kShare ? 1 : 2;                   // coefficient lines of a pair of steps
+    uint32_t wa[S], wb[S], c[NL][CW], c_next[NL][CW];
     Part xa;
-    Line line = load_line(p0);
+    Line line[NL];
+#pragma unroll
+    for (int l = 0; l < NL; ++l)
+        line[l] = load_line(p0 + l);
     load_words(p0, wa);
     load_x(p0, xa);
-    load_coefficients(line, c);
-    line = load_line(p0 + 2);
+#pragma unroll
+    for (int l = 0; l < NL; ++l)
+        load_coefficients(line[l], c[l]);
+#pragma unroll
+    for (int l = 0; l < NL; ++l)
+        line[l] = load_line(p0 + 2 + l);
     store_x(xa, 0);
     load_x(p0 + 1, xa);
     load_words(p0 + 1, wb);
     __syncthreads();
     for (int ip = p0; ip <= p_last; ip += 2) {
         // -- even step: buffer 0
-        load_coefficients(line, c_next);              // of the next pair of steps
-        line = load_line(ip + 4);
+#pragma unroll
+        for (int l = 0; l < NL; ++l)
+            load_coefficients(line[l], c_next[l]);    // of the next pair of steps
+#pragma unroll
+        for (int l = 0; l < NL; ++l)
+            line[l] = load_line(ip + 4 + l);
         __builtin_amdgcn_sched_barrier(0);
-        build_table(c);
+        build_table(c[0]);
         compute(wa, 0);
         __builtin_amdgcn_sched_barrier(0);
         store_x(xa, 1);                                // step ip + 1
@@ -2495,14 +2134,20 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
         // -- odd step: buffer 1
-        compute(wb, 1);
+        if (kShare || ip < p_last) {                   // (the same for the whole workgroup)
+            if constexpr (!kShare)
+                build_table(c[NL - 1]);
+            compute(wb, 1);
+        }
         __builtin_amdgcn_sched_barrier(0);
         store_x(xa, 0);                                // step ip + 2
         load_x(ip + 3, xa);
         load_words(ip + 3, wb);
 #pragma unroll
-        for (int q = 0; q < CW; ++q)
-            c[q] = c_next[q];
+        for (int l = 0; l < NL; ++l)
+#pragma unroll
+            for (int q = 0; q < CW; ++q)
+                c[l][q] = c_next[l][q];
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
     }
@@ -2539,7 +2184,7 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
 
 bool gemm_lut_path_ok(int M, int N, int K, int S, int G)
 {
-    return M > kRowsMax && K % 128 == 0 && G % 128 == 0 && (S == 2 || S == 3 || S == 4) &&
+    return M > kMaxM && K % kGemmBK == 0 && G % kGemmBK == 0 && (S == 2 || S == 3 || S == 4 || S == 6 || S == 8) &&
            static_cast<double>(K / 32) * N * S < 2147483648.0 && static_cast<double>(M) * K < 2147483648.0;
 }
 
@@ -2547,9 +2192,10 @@ bool gemm_lut_path_ok(int M, int N, int K, int S, int G)
 // even number of steps, the last one perhaps fewer than the others).  A function of the shape only, so that the workspace
 // can be sized without a device.
 // Few row blocks mean more workgroups and more decodes of the weights, more parts of K more workgroups and partial
-// results to write and add up: the plan is the one of least estimated time.  Estimate, fitted to 3600 launches (110 shapes,
+// results to write and add up: the plan is the one of least estimated time.  Estimate, fitted to 6000 launches (220 shapes,
 // 33 to 2048 rows, 512 to 28672 columns, K 512 to 28672, every number of row blocks, 1 to 16 parts; 8 % off on average, the
-// plan it picks 1.1 % behind the fastest): a step takes 0.38, 0.21 or 0.18 us (4, 3, 2 planes) and 0.2 us a row block, a
+// plan it picks 1 % behind the fastest): a step takes 0.18, 0.21, 0.38, 0.45 or 0.74 us (2, 3, 4, 6, 8 planes; groups of 64
+// 0.1 or, with several tables, 0.2 more) and 0.2 us a row block, a
 // workgroup 3.6 us beside its steps, a split 3.3 us and 0.33 us per MB of partial results (written, read and cleared).
 // 256 workgroups run at a time, up to 13 % faster where fewer do; beyond that a last turn that is not full counts 0.63.
 // Against one tile height and parts by powers of two: 87 rows x 5378 columns, K 19456, 3 planes, 181 us unsplit (N no
@@ -2561,14 +2207,16 @@ constexpr double kGemmLutMaxParts = 96. * 1024 * 1024;
 // Up to 16 steps (K = 1024) stay whole; longer ones are cut into parts of 4 steps and more.  (63 rows x 830 columns, K 1280:
 // 18.5 us whole, 13.3 in 2 parts of 10 steps, 10.1 in 5 of 4.)
 constexpr int kGemmLutWhole = 16, kGemmLutMinPart = 4;
+constexpr int kGemmSplitCus = 256;
 
 struct GemmLutPlan {
     int rb, ksplit, part_steps;
 };
 
-GemmLutPlan gemm_lut_plan(int M, int N, int K, int S, bool may_split)
+GemmLutPlan gemm_lut_plan(int M, int N, int K, int S, int G, bool may_split)
 {
-    const double decode_us = S == 4 ? 0.38 : (S == 3 ? 0.21 : 0.18);
+    const double decode_us = (S == 8 ? 0.74 : (S == 6 ? 0.45 : (S == 4 ? 0.38 : (S == 3 ? 0.21 : 0.18)))) +
+                             (G % 128 == 0 ? 0. : (S <= 4 ? 0.1 : 0.2));
     const int blocks = (M + 31) / 32, columns = (N + kPfBN - 1) / kPfBN, steps = K / 64;
     GemmLutPlan best{8, 1, steps};
     double best_us = 0.;
@@ -2599,52 +2247,57 @@ GemmLutPlan gemm_lut_plan(int M, int N, int K, int S, bool may_split)
     return best;
 }
 
+template <int S, int RB, bool kShare>
+hipError_t launch_gemm_lut_inst(dim3 grid, const GemmArgs &a, hipStream_t st)
+{
+    constexpr size_t lds = 2 * 32 * pf_loader_blocks(RB) * kPfRow;
+    {
+        static bool raised_on[16] = {};
+        std::lock_guard<std::mutex> guard(g_dev_lock);
+        int dev_now = 0;
+        if (hipGetDevice(&dev_now) != hipSuccess || dev_now < 0 || dev_now >= 16)
+            dev_now = 0;
+        if (!raised_on[dev_now]) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(sbvr_gemm_lut_kernel<S, RB, kShare>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+            if (e != hipSuccess)
+                return e;
+            raised_on[dev_now] = true;
+        }
+    }
+    hipLaunchKernelGGL((sbvr_gemm_lut_kernel<S, RB, kShare>), grid, dim3(64 * kPfWaves), lds, st, a);
+    return hipGetLastError();
+}
+
+template <int S, bool kShare>
+hipError_t launch_gemm_lut_rows(int rb, dim3 grid, const GemmArgs &a, hipStream_t st)
+{
+    switch (rb) {
+    case 2: return launch_gemm_lut_inst<S, 2, kShare>(grid, a, st);
+    case 3: return launch_gemm_lut_inst<S, 3, kShare>(grid, a, st);
+    case 4: return launch_gemm_lut_inst<S, 4, kShare>(grid, a, st);
+    case 5: return launch_gemm_lut_inst<S, 5, kShare>(grid, a, st);
+    case 6: return launch_gemm_lut_inst<S, 6, kShare>(grid, a, st);
+    case 7: return launch_gemm_lut_inst<S, 7, kShare>(grid, a, st);
+    default: return launch_gemm_lut_inst<S, 8, kShare>(grid, a, st);
+    }
+}
+
 hipError_t launch_gemm_lut(int S, int rb, const GemmArgs &a, hipStream_t st)
 {
     const dim3 grid(static_cast<unsigned>((a.N + kPfBN - 1) / kPfBN), static_cast<unsigned>((a.M + 32 * rb - 1) / (32 * rb)),
                     static_cast<unsigned>(a.ksplit));
-    const dim3 block(64 * kPfWaves);
-    const size_t lds = 2 * 32 * pf_loader_blocks(rb) * kPfRow;
-#define SBVR_PF_LAUNCH(SS, RR)                                                                                 \
-    {                                                                                                          \
-        static bool raised_on[16] = {};                                                                        \
-        std::lock_guard<std::mutex> guard(g_dev_lock);                                                                        \
-        int dev_now = 0;                                                                                       \
-        if (hipGetDevice(&dev_now) != hipSuccess || dev_now < 0 || dev_now >= 16)                              \
-            dev_now = 0;                                                                                       \
-        bool &raised = raised_on[dev_now];                                                                     \
-        if (!raised) {                                                                                         \
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(sbvr_gemm_lut_kernel<SS, RR>), \
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)); \
-            if (e != hipSuccess)                                                                               \
-                return e;                                                                                      \
-            raised = true;                                                                                     \
-        }                                                                                                      \
-        hipLaunchKernelGGL((sbvr_gemm_lut_kernel<SS, RR>), grid, block, lds, st, a);                           \
-    }                                                                                                          \
-    break
-#define SBVR_PF_ROWS(SS)                                                                                       \
-    switch (rb) {                                                                                              \
-    case 2: SBVR_PF_LAUNCH(SS, 2);                                                                             \
-    case 3: SBVR_PF_LAUNCH(SS, 3);                                                                             \
-    case 4: SBVR_PF_LAUNCH(SS, 4);                                                                             \
-    case 5: SBVR_PF_LAUNCH(SS, 5);                                                                             \
-    case 6: SBVR_PF_LAUNCH(SS, 6);                                                                             \
-    case 7: SBVR_PF_LAUNCH(SS, 7);                                                                             \
-    default: SBVR_PF_LAUNCH(SS, 8);                                                                            \
-    }                                                                                                          \
-    break
+    const bool share = a.steps_per_group % 2 == 0;
     switch (S) {
-    case 4: SBVR_PF_ROWS(4);
+    case 4: return share ? launch_gemm_lut_rows<4, true>(rb, grid, a, st) : launch_gemm_lut_rows<4, false>(rb, grid, a, st);
 #ifndef SBVR_FAST_BUILD
-    case 2: SBVR_PF_ROWS(2);
-    case 3: SBVR_PF_ROWS(3);
+    case 2: return share ? launch_gemm_lut_rows<2, true>(rb, grid, a, st) : launch_gemm_lut_rows<2, false>(rb, grid, a, st);
+    case 3: return share ? launch_gemm_lut_rows<3, true>(rb, grid, a, st) : launch_gemm_lut_rows<3, false>(rb, grid, a, st);
+    case 6: return share ? launch_gemm_lut_rows<6, true>(rb, grid, a, st) : launch_gemm_lut_rows<6, false>(rb, grid, a, st);
+    case 8: return share ? launch_gemm_lut_rows<8, true>(rb, grid, a, st) : launch_gemm_lut_rows<8, false>(rb, grid, a, st);
 #endif
     default: return hipErrorInvalidConfiguration;
     }
-#undef SBVR_PF_ROWS
-#undef SBVR_PF_LAUNCH
-    return hipGetLastError();
 }
 
 int current_cus()
@@ -3829,12 +3482,10 @@ size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G)
 {
     if (mfma_path_ok(M, N, K, S, G) || lut_path_ok(M, N, K, S, G))
         return static_cast<size_t>(M) * N * sizeof(unsigned long long);
-    if (gemm_lut_path_ok(M, N, K, S, G)) {
-        const int ks = gemm_lut_plan(M, N, K, S, true).ksplit;
+    if (gemm_lut_path_ok(M, N, K, S, G) && !rows32_path_ok(M, N, K, S, G)) {
+        const int ks = gemm_lut_plan(M, N, K, S, G, true).ksplit;
         return ks == 1 ? 0 : ks * part_floats(M, N) * sizeof(float);
     }
-    if (gemm_path_ok(M, N, K, S, G) && !rows32_path_ok(M, N, K, S, G))
-        return gemm_workspace_bytes(M, N, K);
     return 0;
 }
 
@@ -4024,9 +3675,8 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         }
     }
 
-    // More than 32 rows, 2 to 4 planes, K and G multiples of 128: the prefill kernel that decodes by table look-up
-    // (SBVR_HIP_PF_LUT=2 keeps the tile kernel: a development switch)
-    if (!(flags & 1) && aligned && env_switches().pf_lut != 2 && gemm_lut_path_ok(M, N, K, S, G) && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
+    // More than 32 rows (and 17 to 32 where `flags` keeps them from the 32-row kernels), K and G multiples of 64: prefill
+    if (!(flags & 1) && aligned && gemm_lut_path_ok(M, N, K, S, G) && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
         GemmArgs g{};
         g.x = static_cast<const uint16_t *>(x);
         g.bvr = bvr;
@@ -4039,7 +3689,7 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         g.idx16 = idx_bytes == 2;
         g.ksplit = 1;
         g.part_steps = K / kGemmBK;
-        GemmLutPlan plan = gemm_lut_plan(M, N, K, S, true);
+        GemmLutPlan plan = gemm_lut_plan(M, N, K, S, G, true);
         const int ks = plan.ksplit;
         const size_t need = ks > 1 ? ks * part_floats(M, N) * sizeof(float) : 0;
         if (need && workspace && workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
@@ -4047,7 +3697,7 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
             g.part_steps = plan.part_steps;
             g.part = static_cast<float *>(workspace);
         } else if (need) {
-            plan = gemm_lut_plan(M, N, K, S, false);      // no workspace for the parts: not split
+            plan = gemm_lut_plan(M, N, K, S, G, false);      // no workspace for the parts: not split
         }
         if (env_switches().show_plan)
             fprintf(stderr, "sbvr_hip table look-up prefill M=%d N=%d K=%d S=%d: row blocks=%d ksplit=%d\n", M, N, K, S, plan.rb, g.ksplit);
@@ -4061,45 +3711,11 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         if (e != hipSuccess)
             return fail(SBVR_HIP_ELAUNCH, "prefill (table look-up) launch: %s", hipGetErrorString(e));
         g_last_kernel = g.ksplit > 1 ? SBVR_HIP_KERNEL_PREFILL_SPLIT : SBVR_HIP_KERNEL_PREFILL;
-        g_last_rounding = SBVR_HIP_ROUNDING_DECODE;
+        // (6 and 8 planes: two entries added, closer than plane by plane.  Groups of 64: as decode() rounds, reported as the
+        // looser of the two, which is what such a call has always said)
+        g_last_rounding = S <= 4 && g.steps_per_group % 2 == 0 ? SBVR_HIP_ROUNDING_DECODE : SBVR_HIP_ROUNDING_PLANEWISE;
         return SBVR_HIP_OK;
     }
-    if (!(flags & 1) && aligned && gemm_path_ok(M, N, K, S, G) && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
-        GemmArgs g{};
-        g.x = static_cast<const uint16_t *>(x);
-        g.bvr = bvr;
-        g.idx = coeff_idx;
-        g.cache = static_cast<const uint16_t *>(coeff_cache);
-        g.bias = static_cast<const uint16_t *>(bias);
-        g.out = static_cast<uint16_t *>(out);
-        g.M = M; g.N = N; g.K = K; g.L = L;
-        g.steps_per_group = G / kGemmBK;
-        g.idx16 = idx_bytes == 2;
-        g.ksplit = 1;
-        // K split across workgroups where the output tiles alone would leave CUs idle, if the caller brought the
-        // workspace for it (without one the launch is simply not split)
-        const size_t need = gemm_workspace_bytes(M, N, K);
-        if (need && workspace && workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
-            g.ksplit = gemm_ksplit(M, N, K);
-            g.part = static_cast<float *>(workspace);
-        }
-#ifdef SBVR_TRACE
-        g.trace = g_trace;
-#endif
-        hipError_t e = launch_gemm(S, g, st);
-        if (e == hipSuccess && g.ksplit > 1) {
-            const size_t quads = (static_cast<size_t>(M) * N + 3) / 4;
-            hipLaunchKernelGGL(sbvr_gemm_reduce_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, st,
-                               g.part, g.bias, g.out, M, N, g.ksplit);
-            e = hipGetLastError();
-        }
-        if (e != hipSuccess)
-            return fail(SBVR_HIP_ELAUNCH, "gemm launch: %s", hipGetErrorString(e));
-        g_last_kernel = g.ksplit > 1 ? SBVR_HIP_KERNEL_PREFILL_SPLIT : SBVR_HIP_KERNEL_PREFILL;
-        g_last_rounding = SBVR_HIP_ROUNDING_PLANEWISE;
-        return SBVR_HIP_OK;
-    }
-
     const size_t total = static_cast<size_t>(M) * N;
     const dim3 grid(static_cast<unsigned>((total + 255) / 256)), block(256);
     if (idx_bytes == 1)

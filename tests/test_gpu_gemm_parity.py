@@ -336,3 +336,31 @@ def test_k_split_at_any_width_and_in_uneven_parts(oracle, M, N, K, S, L, bias):
     a = sbvr._sbvr_linear_f16(x, bvr, idx, cache, bvr_len=128)
     assert torch.equal(a, sbvr._sbvr_linear_f16(x, bvr, idx, cache, bvr_len=128))
     assert int(hip._workspaces[(dev.index, torch.cuda.current_stream(dev).cuda_stream)].count_nonzero()) == 0
+
+
+@pytest.mark.parametrize("M,N,K,S,G,L,bias", [
+    (33, 70, 64, 8, 64, 16, False),            # one step of 64
+    (40, 257, 192, 6, 64, 300, True),          # an odd number of steps, two column tiles, uint16 indices, bias
+    (97, 300, 1088, 4, 64, 256, False),        # 17 steps in parts: the last one odd
+    (64, 515, 1216, 8, 64, 256, True),         # 19 steps, 8 planes in three tables
+    (300, 260, 1280, 6, 128, 300, False),      # two tables of 8 entries, K in parts
+    (257, 33, 4096, 8, 256, 256, True),        # 9 row blocks
+    (256, 20000, 512, 8, 128, 256, False),     # 8 row blocks of 8 planes: two turns of four
+    (96, 40, 320, 2, 64, 8, False),
+])
+def test_prefill_planes_in_several_tables_and_groups_of_64(oracle, M, N, K, S, G, L, bias):
+    run_case(oracle, N, K, S, G, M, L, seed=M + N + S, bias=bias)
+
+
+@pytest.mark.parametrize("S,G", [(4, 128), (8, 128), (3, 64)])
+def test_prefill_kernel_for_17_to_32_rows(oracle, S, G):
+    """`flags` bit 1 keeps 17 to 32 rows from the 32-row kernels: they take the prefill kernel."""
+    import sbvr
+    from sbvr import hip, synth
+    dev = torch.device("cuda:0")
+    bvr, idx, cache = synth.random_encoding(200, 576 if G == 64 else 512, S, G, 256, seed=S)
+    x = torch.randn((20, bvr.shape[0] * 32), generator=torch.Generator().manual_seed(1)).to(torch.float16)
+    y = sbvr._sbvr_linear_f16(x.to(dev), bvr.to(dev), idx.to(dev), cache.to(dev), None, bvr_len=G, flags=2)
+    assert hip.last_kernel() == PREFILL
+    ops = (x.numpy(), bvr.numpy(), idx.numpy(), cache.numpy(), G)
+    check(y, oracle.C.linear_f16(*ops)[1], oracle.C.linear_f16(*ops, mode=1)[1], hip.last_rounding(), f"S={S} G={G}")
