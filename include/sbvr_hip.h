@@ -90,7 +90,8 @@ size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G);
  *   decode kernel   M <= 16, N >= 16, K and G multiples of 128 with G/128 a power
  *                   of two, S in {2,3,4,6,8}: plane sums on the matrix cores over
  *                   the raw bit planes, the fp16 activations represented exactly;
- *                   within 2 fp16 ulps of the exact sum.  Taken for up to 8 rows
+ *                   within 2 fp16 ulps of the exact sum.  Also groups of 64 for up
+ *                   to 4 rows (K a multiple of 128).  Taken for up to 8 rows
  *                   of such a shape, and for 9..16 rows where the 32-row kernel's
  *                   table look-up form has no instance (6 or 8 planes) or flags
  *                   bit 1 is set (5..16 rows in a variant whose waves share the

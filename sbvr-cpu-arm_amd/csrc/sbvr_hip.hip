@@ -263,6 +263,12 @@ constexpr int kXFloor = 4;      // measurement aid: the launch's plane-word and 
 //           or 0 per element (exact in fp16, hence in the three fp8 terms), so the MFMAs give
 //           sum_k a_r L_r[k] R_j[k] = a_r * popcount(L_r & R_j) per sub-group, and the rows are added up at the end.
 constexpr int kXPlanes = 5;
+// kXHalves: groups of 64.  A batch row takes two rows of the A operands, one for each half of the sub-group with zeros in the
+//           other, so every operand row meets one coefficient line; the two are added up at the end.  Up to 4 batch rows
+//           (5 rows on: the 32-row kernels).  One thread per output, which took them before, 4096 -> 14336, 4 planes,
+//           one row: 1067 us; here 7.3.  (12800 -> 731, 6 planes, one row 4911 and 5.4; 8192 -> 28672, 2 rows 2219 and 30.)
+constexpr int kXHalves = 6;
+constexpr int kHalvesMaxRows = 4;
 constexpr int kNormChunksMax = 2;             // 16-byte chunks of x a thread sums for the norm, at most
 
 __device__ __forceinline__ uint32_t swiglu_pair(uint32_t g, uint32_t u)
@@ -353,6 +359,7 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
     // -- 1. requests.  Unit u = (sub-group u / CT, column tile u % CT).
     constexpr int U = SP * CT;
     constexpr bool kNorm = XM == kXAddNorm || XM == kXAddNorm2;
+    constexpr int H = XM == kXHalves ? 2 : 1;                           // coefficient groups of a sub-group
     constexpr int NV = XM == kXAddNorm2 ? 2 : 1;                        // chunks of x and of delta per thread
     uint32_t xx[SP][MT][4];
     uint32_t x2[XM == kXSwiGLU ? SP : 1][XM == kXSwiGLU ? MT : 1][4];   // up (SwiGLU)
@@ -381,6 +388,21 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
                     }
                 }
         }
+    } else if constexpr (XM == kXHalves) {
+        // operand rows 2m and 2m + 1: batch row m with the second half of the sub-group, or the first, left out
+#pragma unroll
+        for (int sgi = 0; sgi < SP; ++sgi)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int r = 0; r < 4; r += 2) {
+                    uint32_t v = 0u;
+                    if (mt * 2 + r / 2 < a.M)                       // wave-uniform
+                        v = reinterpret_cast<const uint32_t *>(a.x + static_cast<size_t>(mt * 2 + r / 2) * a.xstride +
+                                                               static_cast<size_t>(sg0 + sgi) * kSub)[lane];
+                    xx[sgi][mt][r] = lane < 32 ? v : 0u;
+                    xx[sgi][mt][r + 1] = lane < 32 ? 0u : v;
+                }
     } else if constexpr (!kNorm) {
 #pragma unroll
         for (int sgi = 0; sgi < SP; ++sgi)
@@ -419,18 +441,25 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
     // n_base + 64*iw + l; they are handed to the (tile, column) lanes later, in LDS permutes: every
     // vector-memory instruction saved is tens of nanoseconds of issue time
     constexpr int IW = (16 * CT + 63) / 64;
-    int lraw[SP][IW];
+    int lraw[SP][H][IW];
 #pragma unroll
     for (int iw = 0; iw < IW; ++iw) {
         const uint32_t lane_i = static_cast<uint32_t>(n_base + min(64 * iw + lane, 16 * CT - 1));
+        auto group_of = [&](int sgi, int h) __attribute__((always_inline)) -> size_t {
+            return static_cast<size_t>(XM == kXHalves ? 2 * (sg0 + sgi) + h : (sg0 + sgi) >> a.gshift);
+        };
         if (a.idx16) {
 #pragma unroll
             for (int sgi = 0; sgi < SP; ++sgi)
-                lraw[sgi][iw] = static_cast<const uint16_t *>(a.idx)[static_cast<size_t>((sg0 + sgi) >> a.gshift) * N + lane_i];
+#pragma unroll
+                for (int h = 0; h < H; ++h)
+                    lraw[sgi][h][iw] = static_cast<const uint16_t *>(a.idx)[group_of(sgi, h) * N + lane_i];
         } else {
 #pragma unroll
             for (int sgi = 0; sgi < SP; ++sgi)
-                lraw[sgi][iw] = static_cast<const uint8_t *>(a.idx)[static_cast<size_t>((sg0 + sgi) >> a.gshift) * N + lane_i];
+#pragma unroll
+                for (int h = 0; h < H; ++h)
+                    lraw[sgi][h][iw] = static_cast<const uint8_t *>(a.idx)[group_of(sgi, h) * N + lane_i];
         }
     }
     Planes<S> q[U];
@@ -452,7 +481,7 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
         for (int sgi = 0; sgi < SP; ++sgi)
 #pragma unroll
             for (int iw = 0; iw < IW; ++iw)
-                seen ^= static_cast<uint32_t>(lraw[sgi][iw]);
+                seen ^= static_cast<uint32_t>(lraw[sgi][0][iw]);
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -533,7 +562,7 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
     __builtin_amdgcn_s_setprio(3);
     v8i A[SP][MT];
     float scale[SP][MT];         // of this lane's batch row (blk)
-    const int m_rows = XM == kXPlain || XM == kXPlanes ? a.M : 1;
+    const int m_rows = XM == kXPlain || XM == kXPlanes || XM == kXHalves ? H * a.M : 1;
     // Lane l = 4g + t of a row's 64 takes elements 8g + t and 8g + t + 4 of the sub-group: the same bit t of two
     // neighbouring nibbles of a plane word, which are neighbouring bytes of the A image (one 16-bit store per
     // term) and share the weight of their B digits (0.5, 1, 2, 2 for t = 0..3, made up for here: 4, 2, 1, 1).
@@ -599,14 +628,16 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
     // -- 3. coefficient lines (S fp16 each): lane l gathers the line of column n_base + l for each
     //       sub-group, then the (tile, column) lanes pick theirs up with LDS permutes
     constexpr int CW = (S + 1) / 2;          // dwords per line
-    uint32_t cl[SP][IW][CW];
+    uint32_t cl[SP][H][IW][CW];
 #pragma unroll
     for (int sgi = 0; sgi < SP; ++sgi)
 #pragma unroll
-        for (int iw = 0; iw < IW; ++iw) {
-            const uint32_t line = static_cast<uint32_t>(min(lraw[sgi][iw], a.L - 1));
-            load_line_words<S>(a.cache + line * S, cl[sgi][iw]);
-        }
+        for (int h = 0; h < H; ++h)
+#pragma unroll
+            for (int iw = 0; iw < IW; ++iw) {
+                const uint32_t line = static_cast<uint32_t>(min(lraw[sgi][h][iw], a.L - 1));
+                load_line_words<S>(a.cache + line * S, cl[sgi][h][iw]);
+            }
     SBVR_STAMP(3);
 
     // -- 4. the units: plane sums of every (unit, row tile, plane), and one unit behind them
@@ -625,9 +656,14 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
     auto fetch_coefficients = [&](int u) __attribute__((always_inline)) {
         const int sgi = u / CT, ct = u % CT;
 #pragma unroll
-        for (int j = 0; j < CW; ++j)
-            cqu[j] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(((ct * 16 + col) & 63) * 4,
-                                                                          static_cast<int>(cl[sgi][(ct * 16) / 64][j])));
+        for (int j = 0; j < CW; ++j) {
+            const int from = ((ct * 16 + col) & 63) * 4;
+            cqu[j] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from, static_cast<int>(cl[sgi][0][(ct * 16) / 64][j])));
+            if constexpr (H == 2) {              // (odd operand rows: the second half's line)
+                const uint32_t second = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from, static_cast<int>(cl[sgi][1][(ct * 16) / 64][j])));
+                cqu[j] = blk & 1 ? second : cqu[j];
+            }
+        }
     };
     auto apply_coefficients = [&](int u) __attribute__((always_inline)) {
         const int sgi = u / CT, ct = u % CT;
@@ -718,8 +754,10 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
             total += __shfl_xor(total, 16, 64);
             total += __shfl_xor(total, 32, 64);
         }
-        const int n = n_base + ct * 16 + col, m = mt * 4 + blk;
-        const bool valid = (XM == kXPlanes ? m == 0 : m < a.M) && (!shifted || n >= n_own) && n < n_own + a.wstride;
+        if constexpr (XM == kXHalves)        // (rows 2m and 2m + 1: the two halves of row m)
+            total += __shfl_xor(total, 16, 64);
+        const int n = n_base + ct * 16 + col, m = XM == kXHalves ? mt * 2 + (blk >> 1) : mt * 4 + blk;
+        const bool valid = (XM == kXPlanes ? m == 0 : m < a.M && (XM != kXHalves || (blk & 1) == 0)) && (!shifted || n >= n_own) && n < n_own + a.wstride;
         const size_t at = static_cast<size_t>(m) * N + n;
         if (a.ksplit > 1) {
             // through the accumulators: the adder that completes the count converts
@@ -1195,6 +1233,11 @@ bool mfma_path_ok(int M, int N, int K, int S, int G)
            static_cast<double>(K / 32) * N * S < 2147483648.0;
 }
 
+bool halves_path_ok(int M, int N, int K, int S, int G)
+{
+    return G == kSub / 2 && M <= kHalvesMaxRows && mfma_path_ok(M, N, K, S, kSub);
+}
+
 template <int S, int MT, int CT, int SP, int XM>
 hipError_t launch_gemv_inst(const GemvArgs &a, const GemvPlan &p, hipStream_t st)
 {
@@ -1245,6 +1288,9 @@ hipError_t launch_gemv_mt(const GemvArgs &a, const GemvPlan &p, int xm, hipStrea
         return p.MT == 1 ? launch_gemv_shape<S, 1, kXFloor>(a, p, st) : hipErrorInvalidConfiguration;
     if (xm == kXPlanes)
         return p.MT == 1 ? launch_gemv_shape<S, 1, kXPlanes>(a, p, st) : hipErrorInvalidConfiguration;
+    if (xm == kXHalves)
+        return p.MT == 1 ? launch_gemv_shape<S, 1, kXHalves>(a, p, st)
+                         : (p.MT == 2 ? launch_gemv_shape<S, 2, kXHalves>(a, p, st) : hipErrorInvalidConfiguration);
     switch (p.MT) {
     case 1: return launch_gemv_shape<S, 1, kXPlain>(a, p, st);
     case 2: return launch_gemv_shape<S, 2, kXPlain>(a, p, st);
@@ -3480,7 +3526,7 @@ int sbvr_hip_init(int device)
 
 size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G)
 {
-    if (mfma_path_ok(M, N, K, S, G) || lut_path_ok(M, N, K, S, G))
+    if (mfma_path_ok(M, N, K, S, G) || lut_path_ok(M, N, K, S, G) || halves_path_ok(M, N, K, S, G))
         return static_cast<size_t>(M) * N * sizeof(unsigned long long);
     if (gemm_lut_path_ok(M, N, K, S, G) && !rows32_path_ok(M, N, K, S, G)) {
         const int ks = gemm_lut_plan(M, N, K, S, G, true).ksplit;
@@ -3675,6 +3721,34 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         }
     }
 
+    // Groups of 64, up to 4 rows.  (Where that launch splits K and there is no workspace for it: the portable kernel)
+    if (pro.mode == kXPlain && !(flags & 1) && aligned && halves_path_ok(M, N, K, S, G)) {
+        const GemvPlan p = plan_gemv(2 * M, N, K, S, current_cus());
+        const bool room = workspace && workspace_bytes >= static_cast<size_t>(M) * N * sizeof(unsigned long long) &&
+                          reinterpret_cast<uintptr_t>(workspace) % 8 == 0;
+        if (p.CT > 0 && (p.ksplit == 1 || room)) {
+            GemvArgs a{};
+            a.x = static_cast<const uint16_t *>(x);
+            a.bvr = bvr;
+            a.idx = coeff_idx;
+            a.cache = static_cast<const uint16_t *>(coeff_cache);
+            a.bias = static_cast<const uint16_t *>(bias);
+            a.out = static_cast<uint16_t *>(out);
+            a.M = M; a.N = N; a.K = K; a.L = L;
+            a.idx16 = idx_bytes == 2;
+            a.ksplit = p.ksplit;
+            a.xstride = K;
+            a.wstride = p.wstride;
+            a.acc = static_cast<unsigned long long *>(workspace);
+            const hipError_t e = launch_gemv(S, a, p, kXHalves, st);
+            if (e != hipSuccess)
+                return fail(SBVR_HIP_ELAUNCH, "gemv launch, groups of 64 (CT=%d SP=%d MT=%d waves=%d ksplit=%d): %s", p.CT, p.SP, p.MT, p.waves, p.ksplit, hipGetErrorString(e));
+            g_last_kernel = SBVR_HIP_KERNEL_DECODE;
+            g_last_rounding = SBVR_HIP_ROUNDING_EXACT;
+            return SBVR_HIP_OK;
+        }
+    }
+
     // More than 32 rows (and 17 to 32 where `flags` keeps them from the 32-row kernels), K and G multiples of 64: prefill
     if (!(flags & 1) && aligned && gemm_lut_path_ok(M, N, K, S, G) && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
         GemmArgs g{};
@@ -3761,7 +3835,7 @@ int sbvr_hip_linear_f16_noalloc(const void *x, const uint32_t *bvr, const void *
     // is refused.
     void *ws = nullptr;
     size_t ws_bytes = 0;
-    if (M >= 1 && N >= 1 && (mfma_path_ok(M, N, K, S, G) || lut_path_ok(M, N, K, S, G)) && !(flags & 1) &&
+    if (M >= 1 && N >= 1 && (mfma_path_ok(M, N, K, S, G) || lut_path_ok(M, N, K, S, G) || halves_path_ok(M, N, K, S, G)) && !(flags & 1) &&
         static_cast<size_t>(M) * N * sizeof(unsigned long long) <= kScratchBytes) {
         const int rc = scratch_on_current_device(&ws);
         if (rc != SBVR_HIP_OK)

@@ -331,3 +331,30 @@ def test_linearity_full_size(oracle):
     y1, y2, y12 = f(x1), f(x2), f(x1 + x2)
     rms = y12.pow(2).mean().sqrt()
     assert ((y1 + y2 - y12).abs().max() <= 3 * 2.0 ** -10 * torch.maximum(y12.abs().max(), rms)).item()
+
+
+@pytest.mark.parametrize("N,K,S,M,L,bias", [
+    (16, 128, 4, 1, 16, False),          # one sub-group, one column tile
+    (17, 128, 8, 4, 300, True),          # a window moved left, two row tiles, uint16 indices
+    (1000, 1280, 6, 3, 256, True),       # ten sub-groups, K in parts
+    (731, 12800, 6, 1, 16, False),
+    (4099, 4096, 3, 2, 256, False),      # one row tile, full
+    (14336, 4096, 4, 1, 256, False),
+    (28672, 2048, 2, 4, 300, False),
+])
+def test_groups_of_64_up_to_4_rows(oracle, N, K, S, M, L, bias):
+    """Groups of 64 on the decode kernel: two operand rows a batch row, one per half of a sub-group; rows of different
+    magnitude in the two halves.  Against the oracle, and against one thread per output (flags bit 0)."""
+    import sbvr
+    from sbvr import hip, synth
+    run_case(oracle, N, K, S, 64, M, L, seed=N + M, bias=bias)
+    assert hip.last_kernel() == DECODE
+    dev = _dev()
+    ops = [t.to(dev) for t in synth.random_encoding(N, K, S, 64, L, seed=2)]
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(3))
+    x = (x * torch.where(torch.arange(K) // 64 % 2 == 0, 30.0, 0.01)).to(torch.float16).to(dev)
+    y = sbvr._sbvr_linear_f16(x, *ops, None, bvr_len=64)
+    assert torch.equal(y, sbvr._sbvr_linear_f16(x, *ops, None, bvr_len=64))
+    want = sbvr._sbvr_linear_f16(x, *ops, None, bvr_len=64, flags=1)
+    # (both exact in weights and activations: the order of the fp32 sums and one rounding)
+    check(y, want.float().cpu().numpy().astype(np.float64), "against the portable kernel")
