@@ -5,6 +5,7 @@
 #ifndef SBVR_HIP_ENCODER_H
 #define SBVR_HIP_ENCODER_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #ifdef __cplusplus
@@ -31,6 +32,44 @@ int sbvr_hip_encoder_group_mse_f16(const void *data, const void *points, float *
  * a multiple of 4 and at most 4096, at most 2^28 lines of either kind. */
 int sbvr_hip_encoder_candidates_f16(const void *data, int G, const void *base, int bases, const void *b, int bs, const void *s,
                                     int ss, const void *axes, int steps, int S, void *lines, float *mse, void *stream);
+
+/* The encoder's policy over `groups` groups in order (sbvr/core.py:555-653), on the device: rounds of two launches, each of
+ * which takes the next group that the table does not serve through its search and settles what the groups behind it
+ * see.  The caller brings, all on the device: data (groups, G) fp16; q95 and mean (groups) fp32, every group's 0.95
+ * quantile and mean; table (table_lines, S) fp16; best (groups) fp32 and line (groups), the least error over the
+ * table's lines and the first line that has it (infinity and -1 without lines); line_of (groups) and sel (groups, G), what
+ * comes out; settled (groups), zeros; history, the errors of the searches so far, with room for one more per group; and
+ * state, sbvr_hip_encoder_state_bytes() bytes: two slots of {int lines, misses, history, status, miss, unused; uint64
+ * found}.  Slot 0 starts as {lines in the table, groups so far that were no table hits, errors in `history`, 0, the first
+ * group that misses, 0, all ones}.  A round reads slot and writes the other.  Afterwards the slot that the last round wrote
+ * holds the same; miss >= groups: nothing misses any more; status 1: group `miss` is left to the caller.
+ * [0] and [1]: the plainer and the wider search: base (bases, S) and offsets fp16 as for
+ * sbvr_hip_encoder_candidates_f16, axis_values values per axis of the grid.  scale_step, scale_narrow: 1 / number of scales,
+ * 1 / what the wider search narrows their step by.  warmup, window, acceptable: lines before the table is used, errors in
+ * the cut-off's mean, the least cut-off.  before: groups encoded before data's first.
+ * lines: candidates of a search, for the launch's size (a search of more goes over its threads again).
+ * 2 <= S <= 6, G a multiple of 4 and at most 4096, S * axis_values <= 4096. */
+typedef struct {
+    const void *data;
+    const float *q95, *mean;
+    void *table;
+    float *best;
+    int *line, *line_of, *sel;
+    unsigned char *settled;
+    void *state;
+    double *history;
+    const void *base[2], *offsets[2];
+    int bases[2], n_offsets[2], axis_values[2];
+    float scale_step, scale_narrow;
+    int groups, G, warmup, window, table_lines;
+    long long before;
+    double acceptable;
+} sbvr_hip_encoder_run;
+size_t sbvr_hip_encoder_state_bytes(void);
+int sbvr_hip_encoder_rounds_f16(const sbvr_hip_encoder_run *run, int S, int lines, int slot, int rounds, void *stream);
+
+/* sel and line_of of groups first .. first + groups - 1 that are not settled, against the table line `line` names. */
+int sbvr_hip_encoder_selectors_f16(const sbvr_hip_encoder_run *run, int S, int first, int groups, void *stream);
 
 /* Activations to bit planes on the fly: x (M, K) fp16 -> bvr (K/32, M, S) uint32, bit k%32 of
  * bvr[k/32, m, j] = bit S-1-j of the selector of x[m, k] (point p of a line is the sum of the

@@ -147,6 +147,491 @@ sbvr_encoder_candidates_kernel(const CandidateArgs a)
     }
 }
 
+// ------------------------------------------------------------------- the search of new lines, group after group
+//
+// The encoder's policy is a chain: a group that the table does not serve (its best error is not below the cut-off)
+// searches the candidate lines, the line it finds may join the table and moves the cut-off, and both decide what the
+// groups behind it find (sbvr/core.py:555-653).  Here the chain runs on the device: every group carries its best error
+// over the table (best, line), and a round of two launches takes the next group that misses through its search,
+//   search:  the bounds and axes of its candidates, worked out by every workgroup for itself, then a candidate a thread;
+//   settle:  the winner joins the table or not, the cut-off moves, every group behind it meets the new line, and the
+//            first of those that now misses is the next round's (an atomic minimum).
+// The host queues rounds ahead and looks at the state now and then; rounds behind the last miss do nothing, and so do
+// those behind a group whose candidates these kernels do not form (status 1: the host takes that group through
+// the general path).  State: two slots, read one and written the other by turns, so that workgroups of a launch never
+// read what it changes.
+// A workgroup's search is bound by the vector ALU (3 packed operations per two points and value); a wave stops when
+// all of its 64 lines are above the best error known.  1024 x 4096, groups of 128, 4 planes (241 misses): 269 to 327 ms
+// with about 50 launches and two waits a miss, 14.6 to 17.2 here: 23 us a search (2.6e5 to 4.6e5 lines; 38 to 59 without
+// the bound), 17 us to settle it over up to 32768 groups.  512 x 2048, 3 planes 117 -> 5.2 ms; 64 x 512, 2 planes 36.6 -> 2.4.
+struct EncoderState {
+    int lines, misses, history, status, miss, pad;
+    unsigned long long found;            // error's bits << 32 | candidate: the least so far (all ones: none)
+};
+
+constexpr int kEncMaxScales = 160, kEncMaxAxes = 4096;    // scales of a search, values of all its axes, at most
+constexpr int kEncSettleValues = 4096;                    // squared distances of a workgroup's groups in LDS
+constexpr int kEncNone = 0x7fffffff;
+
+// What torch's kernels do where a result in fp16 is a product and a sum: one rounding (v_fma_mix).
+__device__ __forceinline__ _Float16 fma_half(float a, float b, float c)
+{
+    uint32_t r = 0;
+    asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "+v"(r) : "v"(a), "v"(b), "v"(c));
+    return __builtin_bit_cast(_Float16, static_cast<uint16_t>(r));
+}
+
+// torch.linspace in fp16: the step rounded, values from either end.
+__device__ __forceinline__ _Float16 line_space(_Float16 lo, _Float16 hi, int n, int i)
+{
+#pragma clang fp contract(off)
+    const _Float16 span = hi - lo;
+    const _Float16 step = static_cast<_Float16>(static_cast<float>(span) / static_cast<float>(static_cast<_Float16>(static_cast<float>(n - 1))));
+    const float s = static_cast<float>(step);
+    return i < n / 2 ? fma_half(s, static_cast<float>(i), static_cast<float>(lo))
+                     : fma_half(-s, static_cast<float>(n - 1 - i), static_cast<float>(hi));
+}
+
+struct SearchSpace {
+    _Float16 scales[kEncMaxScales], axes[kEncMaxAxes];
+    uint16_t group[kEncMaxG];
+    float red[2][kEncThreads / 64];
+    int scales_n, extended, covered;
+};
+
+// The bounds of the candidates of group m (GroupEncoder.candidate_lines): its scales and axes into LDS, by the whole workgroup.
+template <int S>
+__device__ __forceinline__ void make_search_space(const sbvr_hip_encoder_run &a, const EncoderState &st, SearchSpace &sp)
+{
+#pragma clang fp contract(off)
+    const int tid = threadIdx.x, m = st.miss;
+    const _Float16 *mine = static_cast<const _Float16 *>(a.data) + static_cast<size_t>(m) * a.G;
+    float lo = INFINITY, hi = -INFINITY;
+    for (int i = tid; i < a.G; i += kEncThreads) {
+        const _Float16 v = mine[i];
+        sp.group[i] = __builtin_bit_cast(uint16_t, v);
+        lo = fminf(lo, static_cast<float>(v));
+        hi = fmaxf(hi, static_cast<float>(v));
+    }
+    for (int d = 32; d >= 1; d >>= 1) {
+        lo = fminf(lo, __shfl_xor(lo, d, 64));
+        hi = fmaxf(hi, __shfl_xor(hi, d, 64));
+    }
+    if ((tid & 63) == 0) {
+        sp.red[0][tid >> 6] = lo;
+        sp.red[1][tid >> 6] = hi;
+    }
+    __syncthreads();
+    for (int w = 0; w < kEncThreads / 64; ++w) {
+        lo = fminf(lo, sp.red[0][w]);
+        hi = fmaxf(hi, sp.red[1][w]);
+    }
+    // hits so far over groups so far, this one counted: above 0.6 (and while the table fills) the wider search
+    const double seen = static_cast<double>(a.before) + m;
+    const bool wide = st.lines < a.warmup || (seen - st.misses) / (seen + 1.) > 0.6;
+    const _Float16 hl = static_cast<_Float16>(lo), hh = static_cast<_Float16>(hi);
+    const _Float16 s_hi = fma_half(static_cast<float>(static_cast<_Float16>(hh - hl)), 1.1f, 0.f);
+    const float s_lo = 2.f * a.q95[m];
+    float step = (static_cast<float>(s_hi) - s_lo) * a.scale_step;
+    if (wide)
+        step = step * a.scale_narrow;
+    const float from = s_lo + step, to = static_cast<float>(s_hi) + step;
+    const double count = ceil((static_cast<double>(to) - static_cast<double>(from)) / static_cast<double>(step));
+    const int steps = a.axis_values[wide];
+    bool covered = fabsf(a.mean[m]) * 2.f / S < 0.28f && step != 0.f && count > 0. && count <= kEncMaxScales && st.lines < a.table_lines &&
+                   fabsf(from) < INFINITY && fabsf(to) < INFINITY && fabsf(lo) < INFINITY && fabsf(hi) < INFINITY;
+    const int n = covered ? static_cast<int>(count) : 0;
+    for (int i = tid; i < n; i += kEncThreads)
+        sp.scales[i] = fma_half(step, static_cast<float>(i), from);
+    // axis q: from a margin below the data's edge q to one above edge q + 1
+    bool finite = true;
+    for (int i = tid; i < S * steps; i += kEncThreads) {
+        const int q = i / steps;
+        const _Float16 e0 = line_space(hl, hh, S + 1, q), e1 = line_space(hl, hh, S + 1, q + 1);
+        const _Float16 margin = fma_half(fabsf(static_cast<float>(e0)), 0.8f, 0.f);
+        const _Float16 a0 = e0 - margin, a1 = e1 + margin;
+        finite = finite && fabsf(static_cast<float>(a0)) < INFINITY && fabsf(static_cast<float>(a1)) < INFINITY;
+        sp.axes[i] = line_space(a0, a1, steps, i % steps);
+    }
+    covered = __syncthreads_and(covered && finite);
+    if (tid == 0) {
+        sp.scales_n = n;
+        sp.extended = wide;
+        sp.covered = covered;
+    }
+    __syncthreads();
+}
+
+// Candidate `at` (see sbvr_encoder_candidates_kernel for the order).
+template <int S>
+__device__ __forceinline__ void form_candidate(const sbvr_hip_encoder_run &a, const SearchSpace &sp, int at, _Float16 (&c)[S])
+{
+#pragma clang fp contract(off)
+    const int wide = sp.extended, bases = a.bases[wide], family = bases * a.n_offsets[wide] * sp.scales_n, steps = a.axis_values[wide];
+    const _Float16 *base = static_cast<const _Float16 *>(a.base[wide]), *offsets = static_cast<const _Float16 *>(a.offsets[wide]);
+    if (at < family) {
+        const int ir = at % bases, is = at / bases % sp.scales_n, ib = at / bases / sp.scales_n;
+        const _Float16 sv = sp.scales[is], bv = offsets[ib];
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            const _Float16 scaled = sv * base[ir * S + q];
+            c[q] = bv + scaled;
+        }
+    } else {
+        int rest = at - family;
+#pragma unroll
+        for (int q = S - 1; q >= 0; --q) {
+            c[q] = sp.axes[q * steps + rest % steps];
+            rest /= steps;
+        }
+    }
+}
+
+// The 2^S subset sums of a line as packed pairs, entry i the sum of the coefficients of i's bits (fp32, rounded once).
+template <int S>
+__device__ __forceinline__ void subset_sums(const _Float16 (&c)[S], v2h (&p)[1 << (S - 1)])
+{
+#pragma clang fp contract(off)
+    float sums[1 << S];
+    sums[0] = 0.f;
+#pragma unroll
+    for (int q = 0; q < S; ++q)
+#pragma unroll
+        for (int i = 0; i < (1 << q); ++i)
+            sums[(1 << q) + i] = sums[i] + static_cast<float>(c[q]);
+#pragma unroll
+    for (int j = 0; j < (1 << (S - 1)); ++j)
+        p[j] = v2h{static_cast<_Float16>(sums[2 * j]), static_cast<_Float16>(sums[2 * j + 1])};
+}
+
+// The least squared distance of a value to the points: fp16 difference, fp16 square.
+template <int S>
+__device__ __forceinline__ float least_square(uint16_t raw, const v2h (&p)[1 << (S - 1)])
+{
+#pragma clang fp contract(off)
+    const _Float16 d = __builtin_bit_cast(_Float16, raw);
+    const v2h dd = {d, d};
+    v2h best;
+#pragma unroll
+    for (int j = 0; j < (1 << (S - 1)); ++j) {
+        const v2h diff = dd - p[j];
+        const v2h sq = diff * diff;
+        best = j == 0 ? sq : __builtin_elementwise_min(best, sq);
+    }
+    return static_cast<float>(best[0] < best[1] ? best[0] : best[1]);
+}
+
+// Selectors of a group's values against a line: the first nearest of its points, most significant plane first.
+template <int S>
+__device__ __forceinline__ void write_selectors(const uint16_t *group, int G, const _Float16 (&c)[S], int *out)
+{
+#pragma clang fp contract(off)
+    _Float16 p[1 << S];
+#pragma unroll
+    for (int i = 0; i < (1 << S); ++i) {
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < S; ++j)
+            sum += (i >> (S - 1 - j)) & 1 ? static_cast<float>(c[j]) : 0.f;
+        p[i] = static_cast<_Float16>(sum);
+    }
+    for (int g = threadIdx.x; g < G; g += kEncThreads) {
+        const _Float16 d = __builtin_bit_cast(_Float16, group[g]);
+        int sel = 0;
+        _Float16 least{};
+#pragma unroll
+        for (int i = 0; i < (1 << S); ++i) {
+            const _Float16 diff = d - p[i], sq = diff * diff;
+            if (i == 0 || sq < least) {
+                least = sq;
+                sel = i;
+            }
+        }
+        out[g] = sel;
+    }
+}
+
+template <int S>
+__global__ void __launch_bounds__(kEncThreads)
+sbvr_encoder_search_kernel(const sbvr_hip_encoder_run a, int slot)
+{
+    __shared__ __align__(16) SearchSpace sp;
+    __shared__ unsigned long long least[kEncThreads / 64];
+    EncoderState *const states = static_cast<EncoderState *>(a.state);
+    const EncoderState st = states[slot];
+    const bool idle = st.status != 0 || st.miss >= a.groups;
+    const int tid = threadIdx.x;
+    if (!idle)
+        make_search_space<S>(a, st, sp);
+    if (blockIdx.x == 0 && tid == 0) {
+        // the other slot: what the settling launch finds there before it takes minima
+        const bool stays = idle || !sp.covered;
+        states[slot ^ 1].miss = stays ? st.miss : kEncNone;
+        states[slot ^ 1].found = ~0ull;
+        if (!idle && !sp.covered)
+            states[slot].status = 1;
+    }
+    if (idle || !sp.covered)
+        return;
+    const int wide = sp.extended, steps = a.axis_values[wide];
+    int n = a.bases[wide] * a.n_offsets[wide] * sp.scales_n, grid = 1;
+#pragma unroll
+    for (int q = 0; q < S; ++q)
+        grid *= steps;
+    n += grid;
+    const float known = st.lines < a.warmup ? INFINITY : a.best[st.miss];
+    // (more lines than the launch has threads, which the host's bound on the scales rules out, would go round again)
+    for (int first = blockIdx.x * kEncThreads; first < n; first += gridDim.x * kEncThreads) {
+        const int line = first + tid, at = min(line, n - 1);
+        _Float16 c[S];
+        form_candidate<S>(a, sp, at, c);
+        v2h p[1 << (S - 1)];
+        subset_sums<S>(c, p);
+        // no candidate above the best error known counts; the margin covers the division by G
+        const unsigned long long now = __hip_atomic_load(&states[slot].found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const float bound = now == ~0ull ? known : fminf(known, __uint_as_float(static_cast<uint32_t>(now >> 32)));
+        const float limit = bound * static_cast<float>(a.G) * 1.000001f;
+        float sum = 0.f;
+        int g = 0;
+        for (; g < a.G; g += 4) {                                  // (G is a multiple of 4)
+            const uint2 four = *reinterpret_cast<const uint2 *>(sp.group + g);
+            sum += least_square<S>(static_cast<uint16_t>(four.x), p);
+            sum += least_square<S>(static_cast<uint16_t>(four.x >> 16), p);
+            sum += least_square<S>(static_cast<uint16_t>(four.y), p);
+            sum += least_square<S>(static_cast<uint16_t>(four.y >> 16), p);
+            if ((g & 12) == 12 && __all(sum > limit))
+                break;
+        }
+        const float mse = sum / static_cast<float>(a.G);
+        unsigned long long key = g >= a.G && line < n && mse < known ? (static_cast<unsigned long long>(__float_as_uint(mse)) << 32) | static_cast<uint32_t>(line)
+                                                                      : ~0ull;
+        for (int d = 32; d >= 1; d >>= 1) {
+            const unsigned long long other = __shfl_xor(key, d, 64);
+            key = other < key ? other : key;
+        }
+        __syncthreads();
+        if ((tid & 63) == 0)
+            least[tid >> 6] = key;
+        __syncthreads();
+        if (tid == 0) {
+            for (int w = 1; w < kEncThreads / 64; ++w)
+                key = least[w] < key ? least[w] : key;
+            if (key != ~0ull)
+                atomicMin(&states[slot].found, key);
+        }
+    }
+}
+
+template <int S>
+__global__ void __launch_bounds__(kEncThreads)
+sbvr_encoder_settle_kernel(const sbvr_hip_encoder_run a, int slot)
+{
+#pragma clang fp contract(off)
+    __shared__ __align__(16) union {
+        SearchSpace sp;
+        float squares[kEncSettleValues + 64];
+    } sh;
+    __shared__ int twin, first_miss;
+    EncoderState *const states = static_cast<EncoderState *>(a.state);
+    const EncoderState st = states[slot];
+    const int tid = threadIdx.x, m = st.miss;
+    _Float16 *const table = static_cast<_Float16 *>(a.table);
+    EncoderState next = st;                                            // (miss and found: written by the search and by minima)
+    const bool found = st.found != ~0ull;
+    // (nothing left, a group for the host, or one that neither the table nor any candidate has an error for: the state stays)
+    const bool stays = st.status != 0 || m >= a.groups, unserved = !stays && !found && a.line[m] < 0;
+    if (stays || unserved) {
+        if (blockIdx.x == 0 && tid == 0) {
+            states[slot ^ 1].lines = st.lines;
+            states[slot ^ 1].misses = st.misses;
+            states[slot ^ 1].history = st.history;
+            states[slot ^ 1].status = unserved ? 1 : st.status;
+            if (unserved)
+                atomicMin(&states[slot ^ 1].miss, m);
+        }
+        return;
+    }
+    make_search_space<S>(a, st, sh.sp);
+    _Float16 c[S];
+    if (found) {
+        _Float16 raw[S];
+        form_candidate<S>(a, sh.sp, static_cast<int>(st.found & 0xffffffffu), raw);
+        // coefficients by magnitude, equal ones in their order
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            int rank = 0;
+#pragma unroll
+            for (int o = 0; o < S; ++o) {
+                const float vo = fabsf(static_cast<float>(raw[o])), vq = fabsf(static_cast<float>(raw[q]));
+                rank += vo < vq || (vo == vq && o < q);
+            }
+#pragma unroll
+            for (int o = 0; o < S; ++o)
+                c[o] = rank == o ? raw[q] : c[o];
+        }
+    } else {
+        const _Float16 *have = table + static_cast<size_t>(a.line[m]) * S;
+#pragma unroll
+        for (int q = 0; q < S; ++q)
+            c[q] = have[q];
+    }
+    if (tid == 0)
+        twin = kEncNone;
+    __syncthreads();
+    // a line of the table that is the same but for 1e-4 takes its place
+    if (found) {
+        float size = 0.f;
+#pragma unroll
+        for (int q = 0; q < S; ++q)
+            size += fabsf(static_cast<float>(c[q]));
+        const _Float16 bound = fma_half(static_cast<float>(static_cast<_Float16>(size)), 0.0001f, 0.f);
+        for (int l = tid; l < st.lines; l += kEncThreads) {
+            float off = 0.f;
+#pragma unroll
+            for (int q = 0; q < S; ++q)
+                off += fabsf(static_cast<float>(static_cast<_Float16>(table[static_cast<size_t>(l) * S + q] - c[q])));
+            if (static_cast<_Float16>(off) < bound) {
+                atomicMin(&twin, l);
+                break;
+            }
+        }
+    }
+    __syncthreads();
+    const bool joins = found && twin == kEncNone;
+    const int chosen = !found ? a.line[m] : (joins ? st.lines : twin);
+    const double error = static_cast<double>(__uint_as_float(static_cast<uint32_t>(st.found >> 32)));
+    next.lines = st.lines + joins;
+    next.misses = st.misses + 1;
+    next.history = st.history + found;
+    // the cut-off over the last errors, in the order the host adds them up
+    double cutoff = 0.;
+    {
+        const int len = min(next.history, a.window);
+        double sum = 0.;
+        for (int i = next.history - len; i < next.history; ++i)
+            sum += found && i == st.history ? error : a.history[i];
+        cutoff = sum / len * 0.99;
+        cutoff = cutoff < a.acceptable ? a.acceptable : cutoff;
+    }
+    if (blockIdx.x == 0) {
+        write_selectors<S>(sh.sp.group, a.G, c, a.sel + static_cast<size_t>(m) * a.G);
+        if (tid == 0) {
+            a.line_of[m] = chosen;
+            a.settled[m] = 1;
+            if (joins)
+#pragma unroll
+                for (int q = 0; q < S; ++q)
+                    table[static_cast<size_t>(st.lines) * S + q] = c[q];
+            if (found)
+                a.history[st.history] = error;
+            states[slot ^ 1].lines = next.lines;
+            states[slot ^ 1].misses = next.misses;
+            states[slot ^ 1].history = next.history;
+            states[slot ^ 1].status = 0;
+            // (groups are searched one after the other until the table has its first lines)
+            if (next.lines < a.warmup || m + 1 >= a.groups)
+                atomicMin(&states[slot ^ 1].miss, m + 1);
+        }
+    }
+    const bool looks = next.lines >= a.warmup;
+    if (!joins && !looks)
+        return;
+    v2h p[1 << (S - 1)];
+    subset_sums<S>(c, p);
+    const int per = max(1, min(16, kEncSettleValues / a.G)), stride = a.G + 1;
+    for (int g0 = m + 1 + static_cast<int>(blockIdx.x) * per; g0 < a.groups; g0 += static_cast<int>(gridDim.x) * per) {
+        const int many = min(per, a.groups - g0);
+        __syncthreads();
+        if (tid == 0)
+            first_miss = kEncNone;
+        if (joins)
+            for (int i = tid; i < many * a.G; i += kEncThreads)
+                sh.squares[i / a.G * stride + i % a.G] = least_square<S>(static_cast<const uint16_t *>(a.data)[static_cast<size_t>(g0) * a.G + i], p);
+        __syncthreads();
+        if (tid < many) {
+            const int g = g0 + tid;
+            float best = a.best[g];
+            if (joins) {
+                float sum = 0.f;
+#pragma unroll 8
+                for (int i = 0; i < a.G; ++i)
+                    sum += sh.squares[tid * stride + i];
+                const float mse = sum / static_cast<float>(a.G);
+                if (mse < best) {
+                    best = mse;
+                    a.best[g] = mse;
+                    a.line[g] = chosen;
+                }
+            }
+            if (looks && !(static_cast<double>(best) < cutoff))
+                atomicMin(&first_miss, g);
+        }
+        __syncthreads();
+        if (tid == 0 && first_miss != kEncNone)
+            atomicMin(&states[slot ^ 1].miss, first_miss);
+    }
+}
+
+// Selectors of the groups that a table line serves: a workgroup a group.
+template <int S>
+__global__ void __launch_bounds__(kEncThreads)
+sbvr_encoder_selectors_kernel(const sbvr_hip_encoder_run a, int first, int groups)
+{
+    __shared__ __align__(16) uint16_t group[kEncMaxG];
+    for (int g = first + static_cast<int>(blockIdx.x); g < first + groups; g += static_cast<int>(gridDim.x)) {
+        if (a.settled[g])                                          // (the same for the whole workgroup)
+            continue;
+        __syncthreads();
+        for (int i = threadIdx.x; i < a.G; i += kEncThreads)
+            group[i] = static_cast<const uint16_t *>(a.data)[static_cast<size_t>(g) * a.G + i];
+        __syncthreads();
+        _Float16 c[S];
+#pragma unroll
+        for (int q = 0; q < S; ++q)
+            c[q] = static_cast<const _Float16 *>(a.table)[static_cast<size_t>(max(a.line[g], 0)) * S + q];
+        write_selectors<S>(group, a.G, c, a.sel + static_cast<size_t>(g) * a.G);
+        if (threadIdx.x == 0)
+            a.line_of[g] = a.line[g];
+    }
+}
+
+template <int S>
+void launch_rounds(const sbvr_hip_encoder_run &a, unsigned search_grid, int slot, int rounds, hipStream_t st)
+{
+    const int per = max(1, min(16, kEncSettleValues / a.G));
+    const unsigned settle_grid = static_cast<unsigned>(max(1, min((a.groups + per - 1) / per, 2048)));
+    for (int r = 0; r < rounds; ++r) {
+        hipLaunchKernelGGL(sbvr_encoder_search_kernel<S>, dim3(search_grid), dim3(kEncThreads), 0, st, a, (slot + r) & 1);
+        hipLaunchKernelGGL(sbvr_encoder_settle_kernel<S>, dim3(settle_grid), dim3(kEncThreads), 0, st, a, (slot + r) & 1);
+    }
+}
+
+template <int S>
+void launch_selectors(const sbvr_hip_encoder_run &a, int first, int groups, hipStream_t st)
+{
+    hipLaunchKernelGGL(sbvr_encoder_selectors_kernel<S>, dim3(static_cast<unsigned>(min(groups, 8192))), dim3(kEncThreads), 0, st, a, first, groups);
+}
+
+bool run_ok(const sbvr_hip_encoder_run *a)
+{
+    return a && a->data && a->q95 && a->mean && a->table && a->best && a->line && a->line_of && a->sel && a->settled && a->state && a->history &&
+           a->base[0] && a->base[1] && a->offsets[0] && a->offsets[1] && a->groups > 0 && a->G > 0 && a->bases[0] > 0 && a->bases[1] > 0 &&
+           a->n_offsets[0] > 0 && a->n_offsets[1] > 0 && a->axis_values[0] > 1 && a->axis_values[1] > 1 && a->window > 0 && a->warmup > 0 &&
+           a->table_lines > 0;
+}
+
+// The lines of a search of the wider or the plainer kind, at most; 0 where the kernels have no room for it.
+long run_lines(const sbvr_hip_encoder_run &a, int wide, int S)
+{
+    if (static_cast<long>(S) * a.axis_values[wide] > kEncMaxAxes)
+        return 0;
+    double grid = 1.;
+    for (int q = 0; q < S; ++q)
+        grid *= a.axis_values[wide];
+    const double n = static_cast<double>(a.bases[wide]) * a.n_offsets[wide] * kEncMaxScales + grid;
+    return n < (1 << 28) ? static_cast<long>(n) : 0;
+}
+
 // Activations to bit planes on the fly: lane = one element x[m, k]; its selector is the first of the P
 // subset sums of its group's line that is nearest to it (fp16 difference and square, as the encoder chooses
 // selectors: sbvr/core.py:492-494), and the 64 lanes' selector bits become two words per plane by ballot
@@ -450,6 +935,43 @@ int sbvr_hip_encoder_candidates_f16(const void *data, int G, const void *base, i
     case 4: hipLaunchKernelGGL(sbvr_encoder_candidates_kernel<4>, grid, block, 0, st, a); break;
     case 5: hipLaunchKernelGGL(sbvr_encoder_candidates_kernel<5>, grid, block, 0, st, a); break;
     default: hipLaunchKernelGGL(sbvr_encoder_candidates_kernel<6>, grid, block, 0, st, a); break;
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+size_t sbvr_hip_encoder_state_bytes(void) { return 2 * sizeof(EncoderState); }
+
+int sbvr_hip_encoder_rounds_f16(const sbvr_hip_encoder_run *run, int S, int lines, int slot, int rounds, void *stream)
+{
+    if (!run_ok(run) || lines <= 0 || slot < 0 || slot > 1 || rounds <= 0)
+        return -1;
+    if (S < 2 || S > 6 || run->G > kEncMaxG || run->G % 4 != 0 || !run_lines(*run, 0, S) || !run_lines(*run, 1, S))
+        return -2;
+    const unsigned grid = static_cast<unsigned>((lines + kEncThreads - 1) / kEncThreads);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    switch (S) {
+    case 2: launch_rounds<2>(*run, grid, slot, rounds, st); break;
+    case 3: launch_rounds<3>(*run, grid, slot, rounds, st); break;
+    case 4: launch_rounds<4>(*run, grid, slot, rounds, st); break;
+    case 5: launch_rounds<5>(*run, grid, slot, rounds, st); break;
+    default: launch_rounds<6>(*run, grid, slot, rounds, st); break;
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+int sbvr_hip_encoder_selectors_f16(const sbvr_hip_encoder_run *run, int S, int first, int groups, void *stream)
+{
+    if (!run_ok(run) || first < 0 || groups <= 0 || first + groups > run->groups)
+        return -1;
+    if (S < 2 || S > 6 || run->G > kEncMaxG)
+        return -2;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    switch (S) {
+    case 2: launch_selectors<2>(*run, first, groups, st); break;
+    case 3: launch_selectors<3>(*run, first, groups, st); break;
+    case 4: launch_selectors<4>(*run, first, groups, st); break;
+    case 5: launch_selectors<5>(*run, first, groups, st); break;
+    default: launch_selectors<6>(*run, first, groups, st); break;
     }
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }

@@ -231,10 +231,11 @@ class sbvr(torch.nn.Module):
         if self.verbose_level > 0:
             from tqdm import tqdm
             bar = tqdm(total=n_groups, ncols=80, desc="Encoding SBVR groups", unit="g")
-        # table look-ups for a block of groups at a time on a GPU; the reference's one-group loop on the CPU
+        # the policy on the device, or table look-ups for a block of groups at a time, on a GPU; the reference's
+        # one-group loop on the CPU
         block = getattr(conf, "group_block", None)
-        if block is None:
-            block = 512 if data.is_cuda else 1
+        if block is None and not data.is_cuda:
+            block = 1
         line_tmp = torch.empty(n_groups, dtype=torch.int32, device=data.device)
         enc.encode_all(flat, line_tmp, sel, block=block, progress=bar.update if bar is not None else None)
         line_of.copy_(line_tmp.to(torch.uint16) if line_of.dtype == torch.uint16 else line_tmp)

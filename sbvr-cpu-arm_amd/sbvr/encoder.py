@@ -14,7 +14,9 @@ same lines and selectors.  On a GPU two things differ from the reference's loop
     another order, so on near-ties a GPU run can pick another line than a CPU run
     (parity of GPU encodings with the reference's own GPU runs is unpinned; they are
     compared by their error);
-  * table look-ups run for a block of groups at once (``encode_all``): the
+  * the per-group policy runs on the device where its kernels serve the encoding
+    (``_encode_chunk_on_device``); otherwise, and with ``group_block`` given,
+    table look-ups run for a block of groups at once (``encode_all``): the
     groups of a block are looked up against the table as it stands, the leading
     hits are taken, the first miss goes through the one-group path (which may add
     a line and move the cut-off), and the look-up restarts behind it.  The policy
@@ -49,7 +51,8 @@ class EncoderConfig:
             self.mse_history = []
         # extension: the reference fixes the group length at 256 (core.py:222)
         self.bvr_len = kwargs.get("bvr_len", 256)
-        # extension: groups looked up in the table at a time (None: 512 on a GPU, 1 on the CPU; see encode_all)
+        # extension: groups looked up in the table at a time (None: the policy on the device on a GPU, 1 on the CPU; see
+        # encode_all)
         self.group_block = kwargs.get("group_block", None)
 
     def describe(self):
@@ -343,11 +346,129 @@ class GroupEncoder:
             live = still
         return best, line, torch.cat(all_points, dim=0)
 
-    def encode_all(self, flat, line_of, sel, block=512, progress=None):
+    # -- all groups on the device ------------------------------------------------
+
+    def _covered_on_device(self, flat):
+        """Whether the policy's kernels serve this encoding; what of the search space they need, per kind of search."""
+        from . import hip
+        c, S, G = self.conf, self.S, self.conf.bvr_len
+        if not (flat.is_cuda and flat.is_contiguous() and hip.encoder_candidates_supported(flat.dtype, G, S) and
+                c.cache_warmup_num >= 1 and c.mse_window_size >= 1 and c.s_search_num > 0 and c.extend_ratio > 0 and
+                (c.num_coeff_cache_lines == 0 or c.mse_history)):
+            return None
+        kw = dict(device=flat.device, dtype=flat.dtype)
+        spaces = [self._fixed_space(extended, kw) for extended in (False, True)]
+        # (a search must be one batch of the policy's scan; the number of scales is the step's count, or one or two more)
+        lines = [base.shape[0] * b.shape[0] * (math.ceil(c.s_search_num * ratio) + 2) + (per_dim + 1) ** S
+                 for (base, b, per_dim), ratio in zip(spaces, (1.0, max(1.0, c.extend_ratio)))]
+        if max(lines) > min(c.search_batch_size, 1 << 27) or any(S * (p + 1) > 4096 or p < 1 or 0 in base.shape or b.numel() == 0
+                                                                for base, b, p in spaces):
+            return None
+        return spaces, lines
+
+    def _encode_chunk_on_device(self, datas, line_of, sel, spaces, lines, progress):
+        """The groups of ``datas`` (groups, G) in order, the table and the counts as they stand: rounds of launches are queued
+        ahead (``hip.encoder_rounds``), the state is looked at once per batch of them.  A group whose candidates the
+        kernels do not form goes through ``encode_group``."""
+        from . import hip
+        c, S, dev = self.conf, self.S, datas.device
+        n, G = datas.shape
+        start, known = c.group_idx, c.num_coeff_cache_lines
+        flat32 = datas.float()
+        stats = torch.stack((torch.quantile(flat32, 0.95, dim=1) if n * G < 1 << 24 else
+                             torch.cat([torch.quantile(p, 0.95, dim=1) for p in flat32.split(max(1, (1 << 23) // G))]),
+                             flat32.mean(dim=1)))
+        best = torch.full((n,), float("inf"), dtype=torch.float32, device=dev)
+        line = torch.full((n,), -1, dtype=torch.int32, device=dev)
+        settled = torch.zeros(n, dtype=torch.uint8, device=dev)
+        history = torch.zeros(len(c.mse_history) + n, dtype=torch.float64, device=dev)
+        if c.mse_history:
+            history[:len(c.mse_history)] = torch.tensor(c.mse_history, dtype=torch.float64)
+        if known:
+            self._look_up(datas, 0, 0, best, line)
+        state = torch.zeros(hip.encoder_state_words(), dtype=torch.int32, device=dev)
+        run = hip.EncoderRun()
+        run.data, run.q95, run.mean, run.table = datas.data_ptr(), stats[0].data_ptr(), stats[1].data_ptr(), self.table.data_ptr()
+        run.best, run.line, run.line_of, run.sel = best.data_ptr(), line.data_ptr(), line_of.data_ptr(), sel.data_ptr()
+        run.settled, run.state, run.history = settled.data_ptr(), state.data_ptr(), history.data_ptr()
+        for wide, (base, b, per_dim) in enumerate(spaces):
+            run.base[wide], run.offsets[wide] = base.data_ptr(), b.data_ptr()
+            run.bases[wide], run.n_offsets[wide], run.axis_values[wide] = base.shape[0], b.shape[0], per_dim + 1
+        run.scale_step, run.scale_narrow = 1.0 / c.s_search_num, float(torch.tensor(1.0) / torch.tensor(c.extend_ratio, dtype=torch.float32))
+        run.groups, run.G, run.warmup, run.window = n, G, c.cache_warmup_num, c.mse_window_size
+        run.table_lines, run.before, run.acceptable = self.table.shape[0], start, c.acceptable_mse
+
+        def put(miss):
+            missed = c.group_idx - c.cache_hits
+            state.copy_(torch.tensor([c.num_coeff_cache_lines, missed, len(c.mse_history), 0, miss, 0, -1, -1] * 2, dtype=torch.int32))
+
+        def next_miss(first):
+            if c.num_coeff_cache_lines < c.cache_warmup_num:
+                return first
+            missing = (~(best[first:].double() < self._cutoff())).nonzero()
+            return first + int(missing[0]) if missing.numel() else n
+
+        miss = next_miss(0)
+        c.group_idx, c.cache_hits = start + miss, c.cache_hits + miss
+        put(miss)
+        shown, rounds = 0, 16
+        while miss < n:
+            hip.encoder_rounds(run, S, max(lines), 0, rounds, dev)          # (an even number: the result is in slot 0 again)
+            had = len(c.mse_history)
+            now = state[:5].tolist()
+            c.num_coeff_cache_lines, missed, errors, status, miss = now
+            miss = min(miss, n)                                             # (above n: none misses any more)
+            c.mse_history.extend(history[had:errors].tolist())
+            c.group_idx, c.cache_hits = start + miss, start + miss - missed
+            if progress is not None:
+                progress(miss - shown)
+                shown = miss
+            if status:
+                known = c.num_coeff_cache_lines
+                found, s = self.encode_group(datas[miss])
+                line_of[miss], sel[miss * G:(miss + 1) * G], settled[miss] = found, s, 1
+                history[errors:len(c.mse_history)] = torch.tensor(c.mse_history[errors:], dtype=torch.float64)
+                if miss + 1 < n and c.num_coeff_cache_lines > known:
+                    self._look_up(datas, miss + 1, known, best, line)
+                miss = next_miss(miss + 1)
+                c.group_idx, c.cache_hits = start + miss, c.cache_hits + miss - (c.group_idx - start)
+                put(miss)
+            rounds = min(64, 2 * rounds)
+        hip.encoder_selectors(run, S, 0, n, dev)
+        if progress is not None:
+            progress(n - shown)
+
+    def _look_up(self, datas, first, from_line, best, line):
+        """Least error, and the first line that has it, of the groups from ``first`` on: over the table lines from
+        ``from_line`` on and what ``best`` and ``line`` hold of those before."""
+        points = self.table[from_line:self.conf.num_coeff_cache_lines] @ self.combs.T
+        step = max(1, (1 << 25) // points.shape[0])
+        for lo in range(first, datas.shape[0], step):
+            mse = self._mse_matrix(datas[lo:lo + step], points)
+            at = mse.argmin(dim=1)
+            val = mse.gather(1, at.view(-1, 1)).view(-1)
+            part = slice(lo, lo + val.shape[0])
+            less = val < best[part]
+            line[part] = torch.where(less, (at + from_line).to(torch.int32), line[part])
+            best[part] = torch.where(less, val, best[part])
+
+    def encode_all(self, flat, line_of, sel, block=None, progress=None):
         """Encodes the groups of ``flat`` (a multiple of bvr_len values) in order into ``line_of`` (one
         line index per group) and ``sel`` (one selector per value).  ``block`` groups are looked up in the
-        table at a time; 1 is the reference's loop (core.py:711-722)."""
+        table at a time; 1 is the reference's loop (core.py:711-722); None: the policy runs on the device where its
+        kernels serve the encoding (2 to 6 planes, fp16), in blocks of 512 otherwise."""
         c = self.conf
+        if block is None:
+            covered = self._covered_on_device(flat)
+            if covered is not None:
+                # (65536 groups at a time: every new line meets all of those behind it in one launch)
+                datas, span = flat.view(-1, c.bvr_len), 1 << 16
+                for lo in range(0, datas.shape[0], span):
+                    part = datas[lo:lo + span]
+                    self._encode_chunk_on_device(part, line_of[lo:lo + span], sel[lo * c.bvr_len:(lo + span) * c.bvr_len], *covered,
+                                                 progress)
+                return
+            block = 512
         G = c.bvr_len
         n_groups = flat.numel() // G
         i = 0

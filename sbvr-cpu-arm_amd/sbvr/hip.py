@@ -31,6 +31,18 @@ def library_path():
     return os.path.join(os.path.dirname(here), "csrc", _LIB_NAME)
 
 
+class EncoderRun(ctypes.Structure):
+    """``sbvr_hip_encoder_run`` of include/sbvr_hip_encoder.h."""
+    _fields_ = [("data", ctypes.c_void_p), ("q95", ctypes.c_void_p), ("mean", ctypes.c_void_p), ("table", ctypes.c_void_p),
+                ("best", ctypes.c_void_p), ("line", ctypes.c_void_p), ("line_of", ctypes.c_void_p), ("sel", ctypes.c_void_p),
+                ("settled", ctypes.c_void_p), ("state", ctypes.c_void_p), ("history", ctypes.c_void_p),
+                ("base", ctypes.c_void_p * 2), ("offsets", ctypes.c_void_p * 2),
+                ("bases", ctypes.c_int * 2), ("n_offsets", ctypes.c_int * 2), ("axis_values", ctypes.c_int * 2),
+                ("scale_step", ctypes.c_float), ("scale_narrow", ctypes.c_float),
+                ("groups", ctypes.c_int), ("G", ctypes.c_int), ("warmup", ctypes.c_int), ("window", ctypes.c_int),
+                ("table_lines", ctypes.c_int), ("before", ctypes.c_longlong), ("acceptable", ctypes.c_double)]
+
+
 def _load():
     global _lib
     if _lib is not None:
@@ -78,6 +90,9 @@ def _load():
     lib.sbvr_hip_dec_head_argmax_embed_f16.argtypes = [vp, vp, vp, ctypes.c_float, vp, i, i, vp, vp, vp, vp, i, vp, vp, i,
                                                        vp, vp, vp, vp, vp]
     lib.sbvr_hip_encoder_group_mse_f16.argtypes = [vp, vp, vp, i, i, i, i, vp]
+    lib.sbvr_hip_encoder_state_bytes.restype = sz
+    lib.sbvr_hip_encoder_rounds_f16.argtypes = [ctypes.POINTER(EncoderRun), i, i, i, i, vp]
+    lib.sbvr_hip_encoder_selectors_f16.argtypes = [ctypes.POINTER(EncoderRun), i, i, i, vp]
     lib.sbvr_hip_encoder_candidates_f16.argtypes = [vp, i, vp, i, vp, i, vp, i, vp, i, i, vp, vp, vp]
     lib.sbvr_hip_online_encode_f16.argtypes = [vp, vp, vp, i, i, i, i, vp]
     lib.sbvr_hip_online_encode_lines_f16.argtypes = [vp, vp, vp, vp, i, i, i, i, i, vp]
@@ -634,6 +649,27 @@ def encoder_candidates(data, base, b, s, axes):
     if rc != 0:
         raise SbvrHipError(f"sbvr_hip_encoder_candidates_f16: error {rc} (G={data.shape[0]} S={S} n={n})")
     return lines, mse
+
+
+def encoder_rounds(run, S, lines, slot, rounds, device):
+    """Queues ``rounds`` rounds of the encoder's policy (``sbvr_hip_encoder_rounds_f16``); ``run``: an EncoderRun."""
+    with torch.cuda.device(device):
+        rc = _load().sbvr_hip_encoder_rounds_f16(ctypes.byref(run), S, lines, slot, rounds, _stream())
+    if rc != 0:
+        raise SbvrHipError(f"sbvr_hip_encoder_rounds_f16: error {rc} (G={run.G} S={S} groups={run.groups})")
+
+
+def encoder_selectors(run, S, first, groups, device):
+    """Line indices and selectors of the groups of ``run`` that a table line serves."""
+    with torch.cuda.device(device):
+        rc = _load().sbvr_hip_encoder_selectors_f16(ctypes.byref(run), S, first, groups, _stream())
+    if rc != 0:
+        raise SbvrHipError(f"sbvr_hip_encoder_selectors_f16: error {rc} (G={run.G} S={S} first={first} groups={groups})")
+
+
+def encoder_state_words():
+    """Size of an EncoderRun's state in 32-bit words (two slots)."""
+    return _load().sbvr_hip_encoder_state_bytes() // 4
 
 
 def encoder_candidates_supported(dtype, G, S):

@@ -175,3 +175,78 @@ def test_fused_candidates_equal_the_general_search(S, G, scale, shift, extended)
         assert torch.equal(found[1], lines[at]), f"group {i}: line {found[1].tolist()} beside {lines[at].tolist()}"
         assert torch.equal(found[2], sel), f"group {i}: selectors"
     assert taken == (0 if shift >= 3 else 12)
+
+
+def _encode_both_ways(w, conf):
+    import sbvr
+    made = [sbvr.sbvr(w, encoder_config=dict(conf, **more), device=w.device, verbose_level=0) for more in ({}, {"group_block": 512})]
+    for part in ("bvr", "coeff_idx", "coeff_cache"):
+        assert torch.equal(getattr(made[0], part).data, getattr(made[1], part).data), part
+    assert made[0].encoder_stats == made[1].encoder_stats
+    return made[0].encoder_stats
+
+
+@pytest.mark.parametrize("shape,S,G,scale,more", [
+    ((64, 512), 2, 256, 0.02, {}),
+    ((100, 768), 3, 128, 0.02, {}),
+    ((192, 1024), 4, 128, 0.02, {}),
+    ((33, 512), 4, 64, 1.0, {}),                                     # distances out of fp16's subnormals
+    ((16, 256), 5, 32, 0.3, {}),
+    ((12, 256), 6, 64, 0.02, {}),
+    ((5, 20), 4, 32, 0.02, {}),                                      # padded groups
+    ((40, 512), 4, 128, 0.02, {"cache_warmup_num": 3, "mse_window_size": 2, "s_search_num": 17, "extend_ratio": 1.3}),
+    ((64, 512), 4, 128, 1e-4, {}),                                   # values whose squares vanish: ties everywhere
+])
+def test_the_policy_on_the_device_equals_the_block_loop(shape, S, G, scale, more):
+    """The rounds of search and settle launches leave the arrays and the counts of the loop over blocks, bit for bit."""
+    dev = torch.device("cuda:0")
+    w = (torch.randn(shape, generator=torch.Generator().manual_seed(S + G)) * scale).to(torch.float16).to(dev)
+    stats = _encode_both_ways(w, dict(num_sums=S, bvr_len=G, **more))
+    assert stats["groups"] == w.shape[0] * -(-w.shape[1] // G)
+
+
+@pytest.mark.parametrize("kind", ["mean", "zeros", "outliers", "repeats", "constant"])
+def test_groups_that_the_device_leaves_to_the_host(kind):
+    """Groups beside a mean that moves the offsets, of zeros or of one value between ordinary ones, and groups that
+    repeat, whose lines the table has already."""
+    dev = torch.device("cuda:0")
+    w = torch.randn((48, 512), generator=torch.Generator().manual_seed(5)) * 0.02
+    if kind == "mean":
+        w[::3] += 2.0
+    elif kind == "zeros":
+        w[::5] = 0
+    elif kind == "outliers":
+        w[::4, 7] = 3.0
+    elif kind == "constant":
+        w[::4] = 0.25
+    else:
+        w[24:] = w[:24]
+    _encode_both_ways(w.to(torch.float16).to(dev), dict(num_sums=4, bvr_len=128))
+
+
+@pytest.mark.parametrize("block", [None, 512])
+def test_values_that_are_not_numbers_are_refused_as_before(block):
+    import sbvr
+    w = torch.randn((8, 256), generator=torch.Generator().manual_seed(8)).to(torch.float16)
+    w[5, 3] = float("nan")
+    with pytest.raises(RuntimeError, match="step must be nonzero"):
+        sbvr.sbvr(w.cuda(), encoder_config=dict(num_sums=4, bvr_len=128, group_block=block), device="cuda:0", verbose_level=0)
+
+
+def test_the_device_policy_over_several_chunks():
+    """Chunks of groups that begin with a table of lines and a history of errors."""
+    from sbvr import encoder
+    dev = torch.device("cuda:0")
+    w = (torch.randn((96, 512), generator=torch.Generator().manual_seed(6)) * 0.02).to(torch.float16).to(dev)
+    flat, out = w.reshape(-1), []
+    for parts in ([384], [5, 30, 349], [100, 284]):
+        conf = encoder.EncoderConfig(num_sums=3, bvr_len=128, search_batch_size=1 << 24)
+        enc = encoder.GroupEncoder(conf, torch.float16, dev)
+        line_of, sel = torch.zeros(384, dtype=torch.int32, device=dev), torch.zeros(flat.numel(), dtype=torch.int32, device=dev)
+        at = 0
+        for n in parts:
+            enc.encode_all(flat[at * 128:(at + n) * 128], line_of[at:at + n], sel[at * 128:(at + n) * 128])
+            at += n
+        out.append((line_of, sel, enc.table[:conf.num_coeff_cache_lines].clone(), conf.mse_history, conf.cache_hits, conf.group_idx))
+    for other in out[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(out[0][:3], other[:3])) and out[0][3:] == other[3:]
