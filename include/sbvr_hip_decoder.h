@@ -122,6 +122,35 @@ int sbvr_hip_dec_head_argmax_embed_f16(const void *x, const void *delta, const v
                                        const float *sin_table, int head_dim, float *rot_now, void *workspace,
                                        const void *embed, void *x_next, void *stream);
 
+/* A prompt's tokens, up to 4 at a time, through a layer, every row bit for bit what the one-row launches of a decode step
+ * give it (the same parts of K in the same order, the same roundings), so that a prompt leaves the same caches whichever
+ * way it came in.  out (rows, N) = the linear (default layout, as sbvr_hip_linear_f16) of
+ *   ADD_RMSNORM  x_out = fp16(x + delta), RMSNorm of it: x, delta, x_out and h (rows, K), h left with the normed rows; the
+ *                rows of sbvr_hip_linear_f16_add_rmsnorm;
+ *   SWIGLU       fp16(silu(gate)) * up, x (rows, 2K) = gate | up: the rows of sbvr_hip_linear_f16_swiglu;
+ *   HEADS        x (rows, K) as it is, K summed up in fours of 128 as by sbvr_hip_dec_attention_o_f16.
+ * Shapes of the decode kernel (K and G multiples of 128, G / 128 a power of two, S in {2,3,4,6,8}, N >= 16; HEADS: N >= 32,
+ * K a multiple of 512), -2 otherwise.  16-byte alignment but for bias, indices and out; workspace: 8 * rows * N bytes,
+ * zero-filled once and left so, not shared by launches that overlap. */
+#define SBVR_HIP_DEC_ROWS_ADD_RMSNORM 1
+#define SBVR_HIP_DEC_ROWS_SWIGLU 2
+#define SBVR_HIP_DEC_ROWS_HEADS 3
+int sbvr_hip_dec_rows_linear_f16(int prologue, const void *x, const void *delta, const void *norm_weight, float eps, void *x_out,
+                                 void *h, const uint32_t *bvr, const void *coeff_idx, int idx_bytes, const void *coeff_cache,
+                                 const void *bias, void *out, int rows, int N, int K, int S, int G, int L, void *workspace,
+                                 size_t workspace_bytes, void *stream);
+
+/* The attention of those tokens: qkv (rows, (heads + 2 kv_heads) * 128), token i at position *pos + i; their keys and values
+ * are appended to the caches (blocked, shapes as for sbvr_hip_dec_attention_o_f16), ctx (rows, heads * 128) are the
+ * context rows that launch would report.  *pos + rows must not exceed max_seq. */
+int sbvr_hip_dec_rows_attention_f16(const void *qkv, const float *cos_table, const float *sin_table, const long long *pos,
+                                    void *kcache, void *vcache, void *ctx, int rows, int heads, int kv_heads, int head_dim,
+                                    int max_seq, void *stream);
+
+/* *pos <- *pos + rows, rot_now as sbvr_hip_dec_argmax_advance_f16 leaves it. */
+int sbvr_hip_dec_rows_advance(long long *pos, int rows, int max_seq, const float *cos_table, const float *sin_table, int head_dim,
+                              float *rot_now, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

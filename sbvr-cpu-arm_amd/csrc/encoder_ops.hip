@@ -173,14 +173,6 @@ constexpr int kEncMaxScales = 160, kEncMaxAxes = 4096;    // scales of a search,
 constexpr int kEncSettleValues = 4096;                    // squared distances of a workgroup's groups in LDS
 constexpr int kEncNone = 0x7fffffff;
 
-// What torch's kernels do where a result in fp16 is a product and a sum: one rounding (v_fma_mix).
-__device__ __forceinline__ _Float16 fma_half(float a, float b, float c)
-{
-    uint32_t r = 0;
-    asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "+v"(r) : "v"(a), "v"(b), "v"(c));
-    return __builtin_bit_cast(_Float16, static_cast<uint16_t>(r));
-}
-
 // torch.linspace in fp16: the step rounded, values from either end.
 __device__ __forceinline__ _Float16 line_space(_Float16 lo, _Float16 hi, int n, int i)
 {

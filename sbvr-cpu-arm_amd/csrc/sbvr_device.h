@@ -34,6 +34,15 @@ __device__ __forceinline__ uint16_t hadd(uint16_t a, uint16_t b)
     return f2h(h2f(a) + h2f(b));
 }
 
+// fp16 of a * b + c rounded once (v_fma_mix), which is what a product and a sum converted to fp16 compile to in most
+// places, but not in all: for results that have to be another kernel's bit for bit.
+__device__ __forceinline__ _Float16 fma_half(float a, float b, float c)
+{
+    uint32_t r = 0;
+    asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "+v"(r) : "v"(a), "v"(b), "v"(c));
+    return __builtin_bit_cast(_Float16, static_cast<uint16_t>(r));
+}
+
 template <typename IdxT>
 __device__ __forceinline__ int load_idx(const void *p, size_t i)
 {

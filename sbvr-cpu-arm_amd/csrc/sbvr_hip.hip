@@ -268,8 +268,15 @@ constexpr int kXPlanes = 5;
 //           (5 rows on: the 32-row kernels).  One thread per output, which took them before, 4096 -> 14336, 4 planes,
 //           one row: 1067 us; here 7.3.  (12800 -> 731, 6 planes, one row 4911 and 5.4; 8192 -> 28672, 2 rows 2219 and 30.)
 constexpr int kXHalves = 6;
+// A prompt's tokens, up to 4 rows, with the sums of the one-row launches they stand for, bit for bit:
+//   kXSwiGLURows  kXSwiGLU for every row;
+//   kXPairs       x itself, the four waves' results added pairwise as the one-launch attention + projection adds its heads'.
+// Four rows cost little more than one (the weight stream is read once): a layer of an 8B
+// shape takes four tokens in 47 us where four steps take 157.
+constexpr int kXSwiGLURows = 7, kXPairs = 8;
 constexpr int kHalvesMaxRows = 4;
 constexpr int kNormChunksMax = 2;             // 16-byte chunks of x a thread sums for the norm, at most
+constexpr int kAoGroup = 4;                   // query heads per key/value head of the one-launch attention + projection
 
 __device__ __forceinline__ uint32_t swiglu_pair(uint32_t g, uint32_t u)
 {
@@ -359,10 +366,11 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
     // -- 1. requests.  Unit u = (sub-group u / CT, column tile u % CT).
     constexpr int U = SP * CT;
     constexpr bool kNorm = XM == kXAddNorm || XM == kXAddNorm2;
+    constexpr bool kSwiGLU = XM == kXSwiGLU || XM == kXSwiGLURows;
     constexpr int H = XM == kXHalves ? 2 : 1;                           // coefficient groups of a sub-group
     constexpr int NV = XM == kXAddNorm2 ? 2 : 1;                        // chunks of x and of delta per thread
     uint32_t xx[SP][MT][4];
-    uint32_t x2[XM == kXSwiGLU ? SP : 1][XM == kXSwiGLU ? MT : 1][4];   // up (SwiGLU)
+    uint32_t x2[kSwiGLU ? SP : 1][kSwiGLU ? MT : 1][4];                 // up (SwiGLU)
     uint32_t xw[kNorm ? SP : 1];                                        // norm weights
     v4u sx[NV], sd[NV];                                                 // this thread's share of all of x and delta
     if constexpr (XM == kXFloor) {
@@ -411,12 +419,12 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     xx[sgi][mt][r] = 0u;
-                    if constexpr (XM == kXSwiGLU)
+                    if constexpr (kSwiGLU)
                         x2[sgi][mt][r] = 0u;
-                    if (XM != kXPlain ? mt * 4 + r < 1 : mt * 4 + r < a.M) {    // wave-uniform; one row with a prologue
+                    if (XM == kXSwiGLU ? mt * 4 + r < 1 : mt * 4 + r < a.M) {    // wave-uniform
                         const size_t at = static_cast<size_t>(mt * 4 + r) * a.xstride + static_cast<size_t>(sg0 + sgi) * kSub;
                         xx[sgi][mt][r] = reinterpret_cast<const uint32_t *>(a.x + at)[lane];
-                        if constexpr (XM == kXSwiGLU)
+                        if constexpr (kSwiGLU)
                             x2[sgi][mt][r] = reinterpret_cast<const uint32_t *>(a.x + at + K)[lane];
                     }
                 }
@@ -562,7 +570,7 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
     __builtin_amdgcn_s_setprio(3);
     v8i A[SP][MT];
     float scale[SP][MT];         // of this lane's batch row (blk)
-    const int m_rows = XM == kXPlain || XM == kXPlanes || XM == kXHalves ? H * a.M : 1;
+    const int m_rows = XM == kXSwiGLU || kNorm ? 1 : H * a.M;
     // Lane l = 4g + t of a row's 64 takes elements 8g + t and 8g + t + 4 of the sub-group: the same bit t of two
     // neighbouring nibbles of a plane word, which are neighbouring bytes of the A image (one 16-bit store per
     // term) and share the weight of their B digits (0.5, 1, 2, 2 for t = 0..3, made up for here: 4, 2, 1, 1).
@@ -584,7 +592,7 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
                 for (int r = 0; r < 4; ++r) {
                     if (mt * 4 + r < m_rows) {      // wave-uniform
                         uint32_t v = xx[sgi][mt][r];
-                        if constexpr (XM == kXSwiGLU)
+                        if constexpr (kSwiGLU)
                             v = swiglu_pair(v, x2[sgi][mt][r]);
                         if constexpr (kNorm)
                             v = norm_pair(v, xw[sgi], inv);
@@ -748,8 +756,12 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
     for (int o = wave; o < CT * MT; o += waves) {    // wave-uniform
         const int ct = o / MT, mt = o % MT;
         float total = 0.f;
-        for (int w = 0; w < waves; ++w)
-            total += red[w * kRedStride + o * 64 + lane];
+        if constexpr (XM == kXPairs)             // (a workgroup of four waves)
+            total = (red[o * 64 + lane] + red[kRedStride + o * 64 + lane]) +
+                    (red[2 * kRedStride + o * 64 + lane] + red[3 * kRedStride + o * 64 + lane]);
+        else
+            for (int w = 0; w < waves; ++w)
+                total += red[w * kRedStride + o * 64 + lane];
         if constexpr (XM == kXPlanes) {      // the rows are the left operand's planes: the output is their sum
             total += __shfl_xor(total, 16, 64);
             total += __shfl_xor(total, 32, 64);
@@ -1288,6 +1300,10 @@ hipError_t launch_gemv_mt(const GemvArgs &a, const GemvPlan &p, int xm, hipStrea
         return p.MT == 1 ? launch_gemv_shape<S, 1, kXFloor>(a, p, st) : hipErrorInvalidConfiguration;
     if (xm == kXPlanes)
         return p.MT == 1 ? launch_gemv_shape<S, 1, kXPlanes>(a, p, st) : hipErrorInvalidConfiguration;
+    if (xm == kXSwiGLURows)
+        return p.MT == 1 ? launch_gemv_shape<S, 1, kXSwiGLURows>(a, p, st) : hipErrorInvalidConfiguration;
+    if (xm == kXPairs)
+        return p.MT == 1 && p.CT == 2 && p.SP == 1 && p.waves == kAoGroup ? launch_gemv_inst<S, 1, 2, 1, kXPairs>(a, p, st) : hipErrorInvalidConfiguration;
     if (xm == kXHalves)
         return p.MT == 1 ? launch_gemv_shape<S, 1, kXHalves>(a, p, st)
                          : (p.MT == 2 ? launch_gemv_shape<S, 2, kXHalves>(a, p, st) : hipErrorInvalidConfiguration);
@@ -2991,6 +3007,80 @@ sbvr_read_floor_kernel(const v4u *__restrict__ base, uint32_t units, int pattern
 
 namespace {
 
+// norm_pair as the decode kernel's instances compile it: r * inv rounded once.
+__device__ __forceinline__ uint32_t norm_pair_once(uint32_t r, uint32_t w, float inv)
+{
+    auto one = [&](uint16_t rh, uint16_t wh) __attribute__((always_inline)) -> uint32_t {
+        return f2h(h2f(wh) * static_cast<float>(fma_half(h2f(rh), inv, 0.f)));
+    };
+    return one(static_cast<uint16_t>(r & 0xffffu), static_cast<uint16_t>(w & 0xffffu)) |
+           (one(static_cast<uint16_t>(r >> 16), static_cast<uint16_t>(w >> 16)) << 16);
+}
+
+// The residual add and RMSNorm of a prompt's tokens, a workgroup a row: the sums of kXAddNorm's workgroups in their order
+// (the same threads take the same chunks), so that a row comes out bit for bit as there.
+template <int NV>
+__global__ void __launch_bounds__(64 * kMaxWaves)
+sbvr_rows_add_norm_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ delta, const uint16_t *__restrict__ norm_w,
+                          uint16_t *__restrict__ x_out, uint16_t *__restrict__ h, int K, float eps)
+{
+    __shared__ float sums[kMaxWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = static_cast<int>(blockDim.x >> 6);
+    const size_t row = static_cast<size_t>(blockIdx.x) * K;
+    v4u sx[NV];
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = tid + j * static_cast<int>(blockDim.x);
+        const bool counts = c < (K >> 3);
+        const int cc = min(c, (K >> 3) - 1);
+        sx[j] = reinterpret_cast<const v4u *>(x + row)[cc];
+        const v4u sd = reinterpret_cast<const v4u *>(delta + row)[cc];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t r = add_pair(sx[j][e], sd[e]);
+            sx[j][e] = r;
+            const float lo = h2f(static_cast<uint16_t>(r & 0xffffu)), hi = h2f(static_cast<uint16_t>(r >> 16));
+            ss += counts ? fmaf(lo, lo, hi * hi) : 0.f;
+        }
+    }
+    ss = wave_fsum(ss);
+    if (lane == 0)
+        sums[wave] = ss;
+    __syncthreads();
+    float total = 0.f;
+    for (int w = 0; w < waves; ++w)
+        total += sums[w];
+    const float inv = rsqrtf(total / static_cast<float>(K) + eps);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = tid + j * static_cast<int>(blockDim.x);
+        if (c >= (K >> 3))
+            continue;
+        reinterpret_cast<v4u *>(x_out + row)[c] = sx[j];
+        const v4u w = reinterpret_cast<const v4u *>(norm_w)[c];
+        v4u n;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            n[e] = norm_pair_once(sx[j][e], w[e], inv);
+        reinterpret_cast<v4u *>(h + row)[c] = n;
+    }
+}
+
+// *pos moves on by `rows`, and rot_now becomes the rotary tables' row of the new position.
+__global__ void sbvr_rows_advance_kernel(long long *pos, int rows, int max_seq, const float *cos_t, const float *sin_t, int half, float *rot_now)
+{
+    const long long now = *pos + rows;
+    __syncthreads();
+    const int at = now < 0 ? 0 : (now >= max_seq ? max_seq - 1 : static_cast<int>(now));
+    for (int i = threadIdx.x; i < half; i += blockDim.x) {
+        rot_now[i] = cos_t[static_cast<size_t>(at) * half + i];
+        rot_now[half + i] = sin_t[static_cast<size_t>(at) * half + i];
+    }
+    if (threadIdx.x == 0)
+        *pos = now;
+}
+
 // ------------------------------------ attention and output projection of one decoded token, one launch
 //
 // The decoder layer's attention (rotary embedding, cache append, softmax(q k^T / sqrt(d)) v over the cached
@@ -3026,7 +3116,6 @@ namespace {
 // projection is exact in its activations (three fp8 terms) with one rounding at the end.
 constexpr int kAoWaves = 16, kAoThreads = 64 * kAoWaves;
 constexpr int kAoHead = 128;         // head size
-constexpr int kAoGroup = 4;          // query heads per key/value head
 constexpr int kAoCols = 128;         // output columns of a workgroup: per head 4 waves x 2 column tiles
 constexpr int kAoMaxSeq = 4096;      // 24 bytes of LDS per cache position
 constexpr int kAoLdsFixed = 8192 + kAoWaves * 2048;
@@ -3048,6 +3137,7 @@ struct AttnOArgs {
     uint16_t *out;                // (N)
     unsigned long long *acc;      // (N) split-K accumulators, all zero between calls (kv_heads > 1)
     int N, L, gshift, idx16;
+    int qkv_stride;               // kRows: elements between the tokens' rows of qkv; ctx (tokens, heads * 128)
 };
 
 typedef v4u __attribute__((may_alias)) v4u_alias;      // 16-byte reads of memory written as fp16 elements
@@ -3063,15 +3153,18 @@ __device__ unsigned long long g_ao_trace[2 * 16 * 12];      // development build
 #define SBVR_AOSTAMP(i) do { } while (0)
 #endif
 
-template <int S>
+// kRows: the attention alone of up to 4 tokens of a prompt, workgroup (g, e) for token e, which stands at position *pos_p + e.
+// Its keys and values of the tokens before it in the same launch come from their rows of qkv (their cache rows are being
+// written meanwhile); the rest, and every sum, is as above.
+template <int S, bool kRows = false>
 __global__ void __launch_bounds__(kAoThreads)
 sbvr_attn_o_kernel(const AttnOArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const int max_seq = a.max_seq;
     uint16_t *const qn = reinterpret_cast<uint16_t *>(smem);               // rotated queries of the group: 4 x 128
-    uint16_t *const kn = qn + kAoGroup * kAoHead;                          // rotated new key
-    uint16_t *const vn = kn + kAoHead;                                     // new value
+    uint16_t *const kn = kRows ? reinterpret_cast<uint16_t *>(smem + 6144) : qn + kAoGroup * kAoHead;      // rotated new key (kRows: keys)
+    uint16_t *const vn = kRows ? kn + 4 * kAoHead : kn + kAoHead;                                            // new value (kRows: values)
     float *const red_max = reinterpret_cast<float *>(smem + 1536);         // [wave][head]
     float *const red_sum = red_max + kAoWaves * kAoGroup;                  // [wave]
     float *const a_scale = red_sum + kAoWaves;                             // [head]: 2^-(e+1) of its A operand
@@ -3092,13 +3185,21 @@ sbvr_attn_o_kernel(const AttnOArgs a)
     uint16_t *const vc = a.vcache + static_cast<size_t>(g) * max_seq * kAoHead;
 
     // -- 1. requests that need no position, in the order they are wanted
-    const long long p64 = *a.pos_p;
+    const long long p64 = *a.pos_p + (kRows ? e : 0);
     SBVR_AOSTAMP(0);
     // the new token: waves 0..3 take query head `wave` of the group, wave 4 the key, wave 5 the value; lane d
     // holds elements d and d + 64 (a rotation pair)
     uint16_t na = 0, nb = 0;
     float c_now = 0.f, s_now = 0.f;
-    if (wave < 6) {                          // wave-uniform
+    const int fresh = wave & 3;              // (kRows: waves 4 to 7 the tokens' keys, 8 to 11 their values, up to token e)
+    if constexpr (kRows) {
+        if (wave < 4 || (wave < 12 && fresh <= e)) {
+            const int row = wave < 4 ? kAoGroup * g + wave : (wave < 8 ? a.heads + g : a.heads + a.kv_heads + g);
+            const uint16_t *src = a.qkv + static_cast<size_t>(wave < 4 ? e : fresh) * a.qkv_stride + static_cast<size_t>(row) * kAoHead;
+            na = src[lane];
+            nb = src[lane + kAoHead / 2];
+        }
+    } else if (wave < 6) {                   // wave-uniform
         const int row = wave < 4 ? kAoGroup * g + wave : (wave == 4 ? a.heads + g : a.heads + a.kv_heads + g);
         const uint16_t *src = a.qkv + static_cast<size_t>(row) * kAoHead;
         na = src[lane];
@@ -3113,9 +3214,12 @@ sbvr_attn_o_kernel(const AttnOArgs a)
     const int hq = wave >> 2;
     const int sgk = kAoGroup * g + hq;
     const int n0 = e * kAoCols + 32 * (wave & 3);
-    const size_t irow = static_cast<size_t>(sgk >> a.gshift) * N + n0 + (lane & 31);
-    const int lraw = a.idx16 ? static_cast<int>(static_cast<const uint16_t *>(a.idx)[irow])
-                             : static_cast<int>(static_cast<const uint8_t *>(a.idx)[irow]);
+    int lraw = 0;
+    if constexpr (!kRows) {
+        const size_t irow = static_cast<size_t>(sgk >> a.gshift) * N + n0 + (lane & 31);
+        lraw = a.idx16 ? static_cast<int>(static_cast<const uint16_t *>(a.idx)[irow])
+                       : static_cast<int>(static_cast<const uint8_t *>(a.idx)[irow]);
+    }
     // keys: wave w takes the 16-position blocks w, w + 16, ...: 2048 elements each, four requests of 1 KiB
     v4u kpre[4];
     {
@@ -3133,7 +3237,34 @@ sbvr_attn_o_kernel(const AttnOArgs a)
     // -- 2. the position is here: rotate, leave q, k, v of the new token in LDS, append (e == 0)
     const int p = p64 < 0 ? 0 : (p64 >= max_seq ? max_seq - 1 : static_cast<int>(p64));
     SBVR_AOSTAMP(2);
-    if (wave < 5) {
+    if constexpr (kRows) {
+        if (wave < 8 && (wave < 4 || fresh <= e)) {
+            const int at_row = wave < 4 ? p : max(p - e + fresh, 0);
+            c_now = a.cos_t[static_cast<size_t>(at_row) * (kAoHead / 2) + lane];
+            s_now = a.sin_t[static_cast<size_t>(at_row) * (kAoHead / 2) + lane];
+            // (the products and roundings that the one-token form compiles to)
+            const float xa = h2f(na), xb = h2f(nb), sb = __fmul_rn(s_now, xb), cb = __fmul_rn(c_now, xb);
+            const uint16_t r0 = __builtin_bit_cast(uint16_t, fma_half(c_now, xa, -sb)), r1 = __builtin_bit_cast(uint16_t, fma_half(s_now, xa, cb));
+            uint16_t *const dst = wave < 4 ? qn + wave * kAoHead : kn + fresh * kAoHead;
+            dst[lane] = r0;
+            dst[lane + kAoHead / 2] = r1;
+            if (wave >= 4 && fresh == e) {
+                uint16_t *const at = kc + static_cast<size_t>(p >> 4) * 2048 + (lane >> 5) * 512 + ((lane & 31) >> 3) * 128 +
+                                     (p & 15) * 8 + (lane & 7);
+                at[0] = r0;
+                at[1024] = r1;
+            }
+        } else if (wave >= 8 && wave < 12 && fresh <= e) {
+            vn[fresh * kAoHead + lane] = na;
+            vn[fresh * kAoHead + lane + kAoHead / 2] = nb;
+            if (fresh == e) {
+                uint16_t *const at = vc + static_cast<size_t>(p >> 5) * 4096 + (lane >> 4) * 512 + ((p & 31) >> 3) * 128 +
+                                     (lane & 15) * 8 + (p & 7);
+                at[0] = na;
+                at[2048] = nb;
+            }
+        }
+    } else if (wave < 5) {
         if (!a.rot_now) {
             c_now = a.cos_t[static_cast<size_t>(p) * (kAoHead / 2) + lane];
             s_now = a.sin_t[static_cast<size_t>(p) * (kAoHead / 2) + lane];
@@ -3174,7 +3305,10 @@ sbvr_attn_o_kernel(const AttnOArgs a)
     // (the line indices came with the position: lane l gathers the coefficient line of column n0 + l % 32)
     constexpr int CW = (S + 1) / 2;
     uint32_t cl[CW];
-    load_line_words<S>(a.cache + static_cast<size_t>(min(lraw, a.L - 1)) * S, cl);
+    if constexpr (!kRows)
+        load_line_words<S>(a.cache + static_cast<size_t>(min(lraw, a.L - 1)) * S, cl);
+    // the first position whose key and value are not taken from the cache
+    const int p_new = kRows ? max(p - e, 0) : p;
     __builtin_amdgcn_sched_barrier(0);
 
     // -- 3. scores of the group's four heads: columns 0..3 of the product.  (The other twelve columns of B repeat
@@ -3186,11 +3320,13 @@ sbvr_attn_o_kernel(const AttnOArgs a)
         qb[j] = __builtin_bit_cast(v8h, v4u(*reinterpret_cast<const v4u_alias *>(qn + (col & (kAoGroup - 1)) * kAoHead + 32 * j + 8 * blk)));
     float mx = -INFINITY;                     // of head `col` over the positions this lane sees
     auto score_block = [&](int tb, v4u (&kw)[4]) __attribute__((always_inline)) {
-        if ((p >> 4) == tb) {                 // wave-uniform: the block of the new key, which is not taken from the cache
-            if (col == (p & 15)) {
+        if (kRows ? 16 * tb + 15 >= p_new : (p >> 4) == tb) {      // wave-uniform: a block of new keys, which are not taken from the cache
+            const int t = 16 * tb + col;
+            if (kRows ? t >= p_new && t <= p : col == (p & 15)) {
+                const uint16_t *const key = kRows ? kn + (t - p_new) * kAoHead : kn;
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    kw[j] = *reinterpret_cast<const v4u_alias *>(kn + 32 * j + 8 * blk);
+                    kw[j] = *reinterpret_cast<const v4u_alias *>(key + 32 * j + 8 * blk);
             }
         }
         v4f d = {0.f, 0.f, 0.f, 0.f};
@@ -3229,7 +3365,7 @@ sbvr_attn_o_kernel(const AttnOArgs a)
     SBVR_AOSTAMP(4);
     // the plane words of the wave's two units of the projection
     Planes<S> q[2];
-    {
+    if constexpr (!kRows) {
         const uint32_t *wrow = a.bvr + (static_cast<size_t>(4 * sgk + blk) * N + n0 + col) * S;
 #pragma unroll
         for (int u = 0; u < 2; ++u)
@@ -3265,7 +3401,17 @@ sbvr_attn_o_kernel(const AttnOArgs a)
     v4f o = {0.f, 0.f, 0.f, 0.f};
     const uint16_t *const wrow_l = wts + (col & (kAoGroup - 1)) * max_seq + 8 * blk;
     auto context_block = [&](int pb, v4u vw) __attribute__((always_inline)) {
-        if (32 * pb + 31 >= p) {              // wave-uniform: the block of p (later blocks are not visited)
+        if constexpr (kRows) {
+            if (32 * pb + 31 >= p_new) {
+                const int ts = 32 * pb + 8 * blk;
+                auto value = [&](int t, uint32_t cached) __attribute__((always_inline)) -> uint32_t {
+                    return t < p_new ? cached : (t <= p ? static_cast<uint32_t>(vn[(t - p_new) * kAoHead + 16 * db + col]) : 0u);
+                };
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    vw[c] = value(ts + 2 * c, vw[c] & 0xffffu) | (value(ts + 2 * c + 1, vw[c] >> 16) << 16);
+            }
+        } else if (32 * pb + 31 >= p) {       // wave-uniform: the block of p (later blocks are not visited)
             // positions before p come from the cache, p itself from the new token, later ones may hold anything
             const int ts = 32 * pb + 8 * blk;     // the lane's positions ts .. ts + 7 of dimension 16 db + col
             const uint32_t vfresh = vn[16 * db + col];
@@ -3299,6 +3445,10 @@ sbvr_attn_o_kernel(const AttnOArgs a)
         const float2 c0 = reinterpret_cast<const float2 *>(part + hq * kAoHead)[lane];
         const float2 c1 = reinterpret_cast<const float2 *>(part + (kAoGroup + hq) * kAoHead)[lane];
         const uint32_t v = static_cast<uint32_t>(f2h(c0.x + c1.x)) | (static_cast<uint32_t>(f2h(c0.y + c1.y)) << 16);
+        if constexpr (kRows) {
+            reinterpret_cast<uint32_t *>(a.ctx + (static_cast<size_t>(e) * a.heads + sgk) * kAoHead)[lane] = v;
+            return;
+        }
         if (a.ctx && e == 0)
             reinterpret_cast<uint32_t *>(a.ctx + static_cast<size_t>(sgk) * kAoHead)[lane] = v;
         unsigned char *const mine = abuf + hq * 2048;
@@ -3327,6 +3477,8 @@ sbvr_attn_o_kernel(const AttnOArgs a)
         *reinterpret_cast<short *>(mine + off + 1 * 32) = b[1];
         *reinterpret_cast<short *>(mine + off + 2 * 32) = b3[0];
     }
+    if constexpr (kRows)
+        return;
     __syncthreads();
     const v8i A = *reinterpret_cast<const v8i *>(abuf + hq * 2048 + lane * 32);
     const float scale = a_scale[hq];
@@ -3390,10 +3542,11 @@ sbvr_attn_o_kernel(const AttnOArgs a)
     SBVR_AOSTAMP(9);
 }
 
-template <int S>
-hipError_t launch_attn_o_inst(const AttnOArgs &a, hipStream_t st)
+// tokens > 0: the attention of that many tokens (kRows)
+template <int S, bool kRows = false>
+hipError_t launch_attn_o_inst(const AttnOArgs &a, hipStream_t st, int tokens = 0)
 {
-    const dim3 grid(static_cast<unsigned>(a.kv_heads), static_cast<unsigned>(a.N / kAoCols)), block(kAoThreads);
+    const dim3 grid(static_cast<unsigned>(a.kv_heads), static_cast<unsigned>(kRows ? tokens : a.N / kAoCols)), block(kAoThreads);
     const size_t lds = kAoLdsFixed + 24 * static_cast<size_t>(a.max_seq);
     if (lds > 65536) {          // above what a kernel gets without asking
         static bool raised_on[16] = {};
@@ -3402,14 +3555,14 @@ hipError_t launch_attn_o_inst(const AttnOArgs &a, hipStream_t st)
         if (hipGetDevice(&dev_now) != hipSuccess || dev_now < 0 || dev_now >= 16)
             dev_now = 0;
         if (!raised_on[dev_now]) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(sbvr_attn_o_kernel<S>),
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(sbvr_attn_o_kernel<S, kRows>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
             if (e != hipSuccess)
                 return e;
             raised_on[dev_now] = true;
         }
     }
-    hipLaunchKernelGGL((sbvr_attn_o_kernel<S>), grid, block, lds, st, a);
+    hipLaunchKernelGGL((sbvr_attn_o_kernel<S, kRows>), grid, block, lds, st, a);
     return hipGetLastError();
 }
 
@@ -4191,6 +4344,115 @@ int sbvr_hip_dec_attention_o_f16(const void *qkv, const float *cos_table, const 
     g_last_kernel = SBVR_HIP_KERNEL_DECODE;
     g_last_rounding = SBVR_HIP_ROUNDING_EXACT;
     return SBVR_HIP_OK;
+}
+
+int sbvr_hip_dec_rows_linear_f16(int prologue, const void *x, const void *delta, const void *norm_weight, float eps, void *x_out, void *h,
+                                 const uint32_t *bvr, const void *coeff_idx, int idx_bytes, const void *coeff_cache, const void *bias,
+                                 void *out, int rows, int N, int K, int S, int G, int L, void *workspace, size_t workspace_bytes,
+                                 void *stream)
+{
+    if (!x || !bvr || !coeff_idx || !coeff_cache || !out || (prologue == SBVR_HIP_DEC_ROWS_ADD_RMSNORM && (!delta || !norm_weight || !x_out || !h)))
+        return fail(SBVR_HIP_EINVAL, "null pointer argument");
+    if (rows <= 0 || N <= 0 || K <= 0 || S <= 0 || G <= 0 || L <= 0 || (idx_bytes != 1 && idx_bytes != 2) || (idx_bytes == 1 && L > 256) ||
+        G % 32 != 0 || K % G != 0)
+        return fail(SBVR_HIP_EINVAL, "rows=%d N=%d K=%d S=%d G=%d L=%d idx_bytes=%d", rows, N, K, S, G, L, idx_bytes);
+    const uintptr_t wide = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(delta) | reinterpret_cast<uintptr_t>(norm_weight) |
+                           reinterpret_cast<uintptr_t>(x_out) | reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(bvr) |
+                           reinterpret_cast<uintptr_t>(coeff_cache);
+    if (wide % 16 != 0)
+        return fail(SBVR_HIP_EINVAL, "x, delta, norm_weight, x_out, h, bvr and coeff_cache must be 16-byte aligned");
+    if (rows > 4 || !mfma_path_ok(rows, N, K, S, G) || prologue < SBVR_HIP_DEC_ROWS_ADD_RMSNORM || prologue > SBVR_HIP_DEC_ROWS_HEADS)
+        return fail(SBVR_HIP_EUNSUPPORTED, "rows of a prompt: prologue=%d rows=%d N=%d K=%d S=%d G=%d", prologue, rows, N, K, S, G);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    // the launch shapes of the one-row calls these rows stand for: the same parts of K in the same order
+    GemvPlan p;
+    int xm = kXPlain;
+    if (prologue == SBVR_HIP_DEC_ROWS_ADD_RMSNORM) {
+        p = plan_gemv(1, N, K, S, current_cus(), (K / 8 + 64 * kNormChunksMax - 1) / (64 * kNormChunksMax));
+    } else if (prologue == SBVR_HIP_DEC_ROWS_SWIGLU) {
+        p = plan_gemv(1, N, K, S, current_cus(), 1);
+        xm = kXSwiGLURows;
+    } else {
+        // one workgroup per four sub-groups (the heads of a key/value head) and 32 columns
+        if (K % (kAoGroup * kSub) != 0 || N < 32 || K / (kAoGroup * kSub) > kMaxKsplit)
+            return fail(SBVR_HIP_EUNSUPPORTED, "rows of a prompt after attention: N=%d K=%d", N, K);
+        p = GemvPlan{2, 1, 1, kAoGroup, (N + 31) / 32, K / (kAoGroup * kSub), 0, 32};
+        p.lds = static_cast<size_t>(p.waves) * 2048;
+        xm = kXPairs;
+    }
+    if (p.CT == 0)
+        return fail(SBVR_HIP_EUNSUPPORTED, "no launch shape for N=%d K=%d S=%d", N, K, S);
+    if (p.ksplit > 1 && (!workspace || workspace_bytes < static_cast<size_t>(rows) * N * sizeof(unsigned long long) || reinterpret_cast<uintptr_t>(workspace) % 8 != 0))
+        return fail(SBVR_HIP_EWORKSPACE, "workspace of %zu bytes needed, %zu given", static_cast<size_t>(rows) * N * sizeof(unsigned long long), workspace_bytes);
+    GemvArgs a{};
+    a.x = static_cast<const uint16_t *>(prologue == SBVR_HIP_DEC_ROWS_ADD_RMSNORM ? h : x);
+    a.bvr = bvr;
+    a.idx = coeff_idx;
+    a.cache = static_cast<const uint16_t *>(coeff_cache);
+    a.bias = static_cast<const uint16_t *>(bias);
+    a.out = static_cast<uint16_t *>(out);
+    a.acc = static_cast<unsigned long long *>(workspace);
+    a.M = rows; a.N = N; a.K = K; a.L = L;
+    a.gshift = __builtin_ctz(static_cast<unsigned>(G / kSub));
+    a.idx16 = idx_bytes == 2;
+    a.ksplit = p.ksplit;
+    a.xstride = prologue == SBVR_HIP_DEC_ROWS_SWIGLU ? 2 * K : K;
+    a.wstride = p.wstride;
+    if (prologue == SBVR_HIP_DEC_ROWS_ADD_RMSNORM) {
+        const dim3 grid(static_cast<unsigned>(rows)), block(64 * p.waves);
+        const uint16_t *xs = static_cast<const uint16_t *>(x), *ds = static_cast<const uint16_t *>(delta), *ws = static_cast<const uint16_t *>(norm_weight);
+        uint16_t *xo = static_cast<uint16_t *>(x_out), *hs = static_cast<uint16_t *>(h);
+        if (K / 8 > 64 * p.waves)
+            hipLaunchKernelGGL(sbvr_rows_add_norm_kernel<2>, grid, block, 0, st, xs, ds, ws, xo, hs, K, eps);
+        else
+            hipLaunchKernelGGL(sbvr_rows_add_norm_kernel<1>, grid, block, 0, st, xs, ds, ws, xo, hs, K, eps);
+    }
+    hipError_t e = launch_gemv(S, a, p, xm, st);
+    if (e == hipSuccess)
+        e = hipGetLastError();
+    if (e != hipSuccess)
+        return fail(SBVR_HIP_ELAUNCH, "rows of a prompt (prologue %d): %s", prologue, hipGetErrorString(e));
+    g_last_kernel = SBVR_HIP_KERNEL_DECODE;
+    g_last_rounding = SBVR_HIP_ROUNDING_EXACT;
+    return SBVR_HIP_OK;
+}
+
+int sbvr_hip_dec_rows_attention_f16(const void *qkv, const float *cos_table, const float *sin_table, const long long *pos, void *kcache,
+                                    void *vcache, void *ctx, int rows, int heads, int kv_heads, int head_dim, int max_seq, void *stream)
+{
+    if (!qkv || !cos_table || !sin_table || !pos || !kcache || !vcache || !ctx)
+        return fail(SBVR_HIP_EINVAL, "null pointer argument");
+    if (rows <= 0 || rows > 4 || !sbvr_hip_dec_attention_o_supported(heads, kv_heads, head_dim, max_seq, kAoCols, 4, kSub))
+        return fail(SBVR_HIP_EUNSUPPORTED, "attention of a prompt's tokens: rows=%d heads=%d kv_heads=%d head_dim=%d max_seq=%d", rows, heads, kv_heads,
+                    head_dim, max_seq);
+    if ((reinterpret_cast<uintptr_t>(kcache) | reinterpret_cast<uintptr_t>(vcache)) % 16 || reinterpret_cast<uintptr_t>(qkv) % 2 ||
+        reinterpret_cast<uintptr_t>(ctx) % 4)
+        return fail(SBVR_HIP_EINVAL, "caches must be 16-byte aligned, ctx 4-byte, qkv 2-byte");
+    AttnOArgs a{};
+    a.qkv = static_cast<const uint16_t *>(qkv);
+    a.cos_t = cos_table;
+    a.sin_t = sin_table;
+    a.pos_p = pos;
+    a.kcache = static_cast<uint16_t *>(kcache);
+    a.vcache = static_cast<uint16_t *>(vcache);
+    a.ctx = static_cast<uint16_t *>(ctx);
+    a.heads = heads; a.kv_heads = kv_heads; a.max_seq = max_seq;
+    a.qkv_stride = (heads + 2 * kv_heads) * head_dim;
+    const hipError_t e = launch_attn_o_inst<4, true>(a, static_cast<hipStream_t>(stream), rows);       // (the planes of the projection do not matter)
+    if (e != hipSuccess)
+        return fail(SBVR_HIP_ELAUNCH, "attention of a prompt's tokens: %s", hipGetErrorString(e));
+    return SBVR_HIP_OK;
+}
+
+int sbvr_hip_dec_rows_advance(long long *pos, int rows, int max_seq, const float *cos_table, const float *sin_table, int head_dim,
+                              float *rot_now, void *stream)
+{
+    if (!pos || !cos_table || !sin_table || !rot_now || rows <= 0 || max_seq <= 0 || head_dim <= 0 || head_dim % 2 != 0)
+        return fail(SBVR_HIP_EINVAL, "null pointer argument or size");
+    hipLaunchKernelGGL(sbvr_rows_advance_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), pos, rows, max_seq, cos_table, sin_table,
+                       head_dim / 2, rot_now);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? SBVR_HIP_OK : fail(SBVR_HIP_ELAUNCH, "advance: %s", hipGetErrorString(e));
 }
 
 int sbvr_hip_read_floor(const void *buf, size_t buf_bytes, size_t bytes, int workgroups, int waves, int ahead, int pattern,

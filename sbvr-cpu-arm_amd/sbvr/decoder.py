@@ -123,7 +123,15 @@ class SbvrLlamaDecoder:
         self.generated = torch.zeros(max_seq, dtype=torch.int64, device=dev)
         self.logits = torch.empty((1, s.vocab), dtype=torch.float16, device=dev)
         self.head_ws = torch.zeros(2, dtype=torch.int64, device=dev)              # cross-workgroup argmax of the head kernel
-        self.graph = None
+        # a prompt's tokens go through the layers a few at a time where attention + projection have their one launch
+        self.prompt_rows = hip.DEC_ROWS if self.attention_o else 0
+        if self.prompt_rows:
+            rows = self.prompt_rows
+            self.rows_tok = torch.zeros(rows, dtype=torch.int64, device=dev)
+            self.rows = {name: torch.zeros((rows, n), dtype=torch.float16, device=dev)
+                         for name, n in (("x", s.hidden), ("x_alt", s.hidden), ("zero", s.hidden), ("h", s.hidden), ("ctx", q_out),
+                                         ("qkv", q_out + 2 * kv_out), ("o", s.hidden), ("gate_up", 2 * s.ffn), ("down", s.hidden))}
+        self.graph = self.graph_rows = None
         self.graph_many, self.steps_per_replay = None, 1
         self.stream = torch.cuda.Stream(device=dev)
         # probe(layer, residual): called by an eager fused step with the residual stream as it enters each layer
@@ -206,6 +214,24 @@ class SbvrLlamaDecoder:
         hip.dec_argmax_advance(logits, self.tok, self.generated, self.pos, self.cos, self.sin, self.rot_now)
         return logits
 
+    def _rows_step(self):
+        """``prompt_rows`` tokens of a prompt (``rows_tok``) through all layers: the caches and the position as that many
+        steps leave them, bit for bit; no head (a prompt's last token goes through a step of its own).  7 launches a
+        layer for 4 tokens where steps take 16: every launch of a step, and every byte of weight it reads, serves one token."""
+        s, r = self.shape, self.rows
+        a, b, delta = r["x"], r["x_alt"], r["zero"]
+        torch.index_select(self.embed, 0, self.rows_tok, out=a)
+        for layer in self.layers:
+            qkv, o, gate_up, down = (layer[k] for k in ("qkv", "o", "gate_up", "down"))
+            hip.dec_rows_add_rmsnorm(a, delta, layer["norm1"], s.rms_eps, b, r["h"], qkv.bvr, qkv.idx, qkv.cache, qkv.bvr_len, r["qkv"])
+            hip.dec_rows_attention(r["qkv"], self.cos, self.sin, self.pos, layer["k"], layer["v"], r["ctx"], s.heads, s.kv_heads,
+                                   s.head_dim)
+            hip.dec_rows_heads(r["ctx"], o.bvr, o.idx, o.cache, o.bvr_len, r["o"])
+            hip.dec_rows_add_rmsnorm(b, r["o"], layer["norm2"], s.rms_eps, a, r["h"], gate_up.bvr, gate_up.idx, gate_up.cache,
+                                     gate_up.bvr_len, r["gate_up"])
+            delta = hip.dec_rows_swiglu(r["gate_up"], down.bvr, down.idx, down.cache, down.bvr_len, r["down"])
+        hip.dec_rows_advance(self.pos, self.prompt_rows, self.cos, self.sin, self.rot_now)
+
     # -- driving ---------------------------------------------------------------
     def capture(self, steps_per_replay=16):
         """Records one step into a HIP graph (after one eager step on the same
@@ -220,6 +246,14 @@ class SbvrLlamaDecoder:
             with torch.cuda.graph(self.graph, stream=self.stream):
                 self.step()
             torch.cuda.synchronize()
+            self.graph_rows = None
+            if self.prompt_rows and self.probe is None:
+                self._rows_step()
+                torch.cuda.synchronize()
+                self.graph_rows = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(self.graph_rows, stream=self.stream):
+                    self._rows_step()
+                torch.cuda.synchronize()
             self.graph_many, self.steps_per_replay = None, int(steps_per_replay)
             if self.steps_per_replay > 1:
                 self.graph_many = torch.cuda.CUDAGraph()
@@ -246,14 +280,23 @@ class SbvrLlamaDecoder:
             self.step()
 
     def generate(self, prompt, new_tokens):
-        """Feeds `prompt` (1-D int64 tensor) token by token, then decodes
-        `new_tokens` greedily.  Returns (tokens, seconds spent on the new tokens)."""
+        """Feeds `prompt` (1-D int64 tensor) `prompt_rows` tokens at a time, the rest and
+        the last one by themselves, then decodes `new_tokens` greedily.  Returns (tokens, seconds spent on the new tokens)."""
         if len(prompt) + new_tokens > self.max_seq:
             raise ValueError("prompt + new tokens exceed the cache length")
         self.reset()
         prompt = prompt.to(self.device)
         with torch.cuda.stream(self.stream):
-            for t in range(len(prompt)):
+            fed = 0
+            # (a probe looks at one step's residual stream at a time)
+            while self.prompt_rows and self.probe is None and len(prompt) - fed > self.prompt_rows:
+                self.rows_tok.copy_(prompt[fed:fed + self.prompt_rows])
+                if self.graph is not None and self.graph_rows is not None:
+                    self.graph_rows.replay()
+                else:
+                    self._rows_step()
+                fed += self.prompt_rows
+            for t in range(fed, len(prompt)):
                 self.tok.copy_(prompt[t:t + 1])
                 self._advance()
             torch.cuda.synchronize()

@@ -89,6 +89,10 @@ def _load():
                                                  vp, vp, vp]
     lib.sbvr_hip_dec_head_argmax_embed_f16.argtypes = [vp, vp, vp, ctypes.c_float, vp, i, i, vp, vp, vp, vp, i, vp, vp, i,
                                                        vp, vp, vp, vp, vp]
+    lib.sbvr_hip_dec_rows_linear_f16.argtypes = [i, vp, vp, vp, ctypes.c_float, vp, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i,
+                                                 vp, sz, vp]
+    lib.sbvr_hip_dec_rows_attention_f16.argtypes = [vp, vp, vp, vp, vp, vp, vp, i, i, i, i, i, vp]
+    lib.sbvr_hip_dec_rows_advance.argtypes = [vp, i, i, vp, vp, i, vp, vp]
     lib.sbvr_hip_encoder_group_mse_f16.argtypes = [vp, vp, vp, i, i, i, i, vp]
     lib.sbvr_hip_encoder_state_bytes.restype = sz
     lib.sbvr_hip_encoder_rounds_f16.argtypes = [ctypes.POINTER(EncoderRun), i, i, i, i, vp]
@@ -527,6 +531,72 @@ def dec_attention_o(qkv, cos, sin, pos, kcache, vcache, heads, kv_heads, head_di
             _bias_ptr(bias, N, dev), out.data_ptr(), N, S, G, L,
             ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _stream()))
     return out
+
+
+DEC_ROWS = 4                                  # tokens of a prompt that a launch takes at most
+_ROWS_ADD_RMSNORM, _ROWS_SWIGLU, _ROWS_HEADS = 1, 2, 3
+
+
+def _dec_rows_linear(prologue, x, K, bvr, coeff_idx, coeff_cache, bvr_len, out, extra=(None, None, None, None), eps=0.0):
+    lib, dev = _load(), x.device
+    for t, name in ((x, "x"), (out, "out")) + tuple((t, "rows") for t in extra if t is not None):
+        _want(t, name, torch.float16, None, dev)
+    _want(bvr, "bvr", torch.uint32, 3, dev)
+    _want(coeff_idx, "coeff_idx", (torch.uint8, torch.uint16), 2, dev)
+    _want(coeff_cache, "coeff_cache", torch.float16, 2, dev)
+    Kw, N, S = bvr.shape
+    L, rows = coeff_cache.shape[0], x.shape[0]
+    if Kw * 32 != K or coeff_idx.shape != (K // bvr_len, N) or coeff_cache.shape[1] != S or tuple(out.shape) != (rows, N) or \
+            any(t is not None and t.numel() != n for t, n in zip(extra, (rows * K, K, rows * K, rows * K))):
+        raise ValueError("operand shapes do not match")
+    delta, weight, x_out, h = (t.data_ptr() if t is not None else None for t in extra)
+    with torch.cuda.device(dev):
+        ws = _workspace(8 * rows * N, dev)
+        _check(lib.sbvr_hip_dec_rows_linear_f16(prologue, x.data_ptr(), delta, weight, eps, x_out, h, bvr.data_ptr(), coeff_idx.data_ptr(),
+                                                _idx_bytes(coeff_idx, L, "coeff_idx"), coeff_cache.data_ptr(), None, out.data_ptr(),
+                                                rows, N, K, S, bvr_len, L, ws.data_ptr(), ws.numel(), _stream()))
+    return out
+
+
+def dec_rows_add_rmsnorm(x, delta, weight, eps, x_out, h, bvr, coeff_idx, coeff_cache, bvr_len, out):
+    """Up to DEC_ROWS tokens of a prompt: x_out <- x + delta, out <- the linear of its RMSNorm (left in ``h``), every row bit
+    for bit as ``_sbvr_linear_f16_add_rmsnorm`` gives it."""
+    return _dec_rows_linear(_ROWS_ADD_RMSNORM, x, x.shape[1], bvr, coeff_idx, coeff_cache, bvr_len, out, (delta, weight, x_out, h), eps)
+
+
+def dec_rows_swiglu(gate_up, bvr, coeff_idx, coeff_cache, bvr_len, out):
+    """The rows of ``_sbvr_linear_f16_swiglu``, up to DEC_ROWS."""
+    return _dec_rows_linear(_ROWS_SWIGLU, gate_up, gate_up.shape[1] // 2, bvr, coeff_idx, coeff_cache, bvr_len, out)
+
+
+def dec_rows_heads(ctx, bvr, coeff_idx, coeff_cache, bvr_len, out):
+    """The projection of up to DEC_ROWS context rows with ``dec_attention_o``'s sums."""
+    return _dec_rows_linear(_ROWS_HEADS, ctx, ctx.shape[1], bvr, coeff_idx, coeff_cache, bvr_len, out)
+
+
+def dec_rows_attention(qkv, cos, sin, pos, kcache, vcache, ctx, heads, kv_heads, head_dim):
+    """The attention of up to DEC_ROWS tokens at positions pos, pos + 1, ..., their keys and values appended to the blocked
+    caches; ``ctx`` (rows, heads * head_dim) receives the context rows."""
+    rows, max_seq, dev = qkv.shape[0], kcache.shape[1], qkv.device
+    for t, name in ((qkv, "qkv"), (kcache, "kcache"), (vcache, "vcache"), (ctx, "ctx")):
+        _want(t, name, torch.float16, None, dev)
+    for t, name in ((cos, "cos"), (sin, "sin")):
+        _want(t, name, torch.float32, None, dev)
+    _want(pos, "pos", torch.int64, None, dev)
+    if kcache.shape != (kv_heads, max_seq, head_dim) or vcache.shape != kcache.shape or cos.shape != (max_seq, head_dim // 2) or \
+            sin.shape != cos.shape or qkv.numel() != rows * (heads + 2 * kv_heads) * head_dim or ctx.numel() != rows * heads * head_dim:
+        raise SbvrHipError("dec_rows_attention: tensor shapes do not match rows/heads/kv_heads/head_dim/max_seq")
+    with torch.cuda.device(dev):
+        _check(_load().sbvr_hip_dec_rows_attention_f16(qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), kcache.data_ptr(),
+                                                       vcache.data_ptr(), ctx.data_ptr(), rows, heads, kv_heads, head_dim, max_seq,
+                                                       _stream()))
+    return ctx
+
+
+def dec_rows_advance(pos, rows, cos, sin, rot_now):
+    """pos <- pos + rows; rot_now <- cos | sin of the new position."""
+    _check(_load().sbvr_hip_dec_rows_advance(pos.data_ptr(), rows, cos.shape[0], cos.data_ptr(), sin.data_ptr(), rot_now.numel(),
+                                             rot_now.data_ptr(), _stream()))
 
 
 def dec_silu_mul(gate_up, out):

@@ -370,3 +370,32 @@ def test_decoder_with_fused_head(oracle):
             dec.graph.replay()
         torch.cuda.synchronize()
     assert torch.equal(dec.generated[:len(tokens)], eager)
+
+
+@pytest.mark.parametrize("shape,S,G,prompt,capture", [
+    (dict(hidden=512, layers=2, heads=4, kv_heads=1, ffn=768, vocab=1000), 4, 128, 5, False),
+    (dict(hidden=1024, layers=3, heads=8, kv_heads=2, ffn=1536, vocab=1000), 3, 128, 70, True),    # across blocks of 16 and 32
+    (dict(hidden=4096, layers=2, heads=32, kv_heads=8, ffn=14336, vocab=4000), 4, 128, 39, True),
+    (dict(hidden=2048, layers=2, heads=16, kv_heads=4, ffn=5632, vocab=1000), 8, 256, 12, False),
+])
+def test_prompt_rows_leave_what_single_steps_leave(shape, S, G, prompt, capture):
+    """A prompt four tokens at a time: the caches (bit for bit), the tokens and the logits of the prompt fed token by token,
+    twice on the same decoder."""
+    import torch
+    from sbvr.decoder import LlamaShape, SbvrLlamaDecoder
+    made = []
+    tokens = torch.randint(0, shape["vocab"], (prompt,), generator=torch.Generator().manual_seed(prompt))
+    for rows in (True, False):
+        dec = SbvrLlamaDecoder(LlamaShape(**shape), "cuda:0", num_sums=S, bvr_len=G, max_seq=128, seed=3)
+        assert dec.attention_o and dec.prompt_rows == 4
+        if not rows:
+            dec.prompt_rows = 0
+        if capture:
+            dec.capture()
+        for _ in range(2):
+            out, _ = dec.generate(tokens, 6)
+            caches = [t.clone() for layer in dec.layers for t in (layer["k"], layer["v"])]
+            made.append((out, dec.logits.clone(), caches))
+    for other in made[1:]:
+        assert all(torch.equal(x, y) for x, y in zip(made[0][2], other[2])), "caches differ"
+        assert torch.equal(made[0][1], other[1]) and torch.equal(made[0][0], other[0])
