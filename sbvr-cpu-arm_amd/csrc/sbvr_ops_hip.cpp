@@ -337,6 +337,27 @@ std::tuple<torch::Tensor, torch::Tensor> sbvr_online_encode_lines(const torch::T
     return {bvr, idx};
 }
 
+// sbvr.online_mm_T in one call: x (..., K) activations of any floating type, K zero-padded to the groups of `lines`, encoded
+// against them and multiplied with the encoded weight.  (Step by step from Python a call took 20 us, 12 of them the host's.)
+torch::Tensor sbvr_online_mm_T(torch::Tensor x, const torch::Tensor &lines, const torch::Tensor &r_bvr, const torch::Tensor &r_coeff_idx,
+                               const torch::Tensor &r_coeff_cache, const Bias &bias, int64_t bvr_len)
+{
+    const c10::InferenceMode inference;             // (what the method it serves runs under)
+    SBVR_WANT(x.is_cuda() && x.device() == r_bvr.device(), "x must be on the weight's GPU");
+    SBVR_WANT(lines.dim() == 2 && bvr_len > 0, "lines must be (K / bvr_len, S)");
+    const int64_t K = lines.size(0) * bvr_len;
+    SBVR_WANT(x.dim() >= 1 && x.size(-1) > 0 && x.size(-1) <= K && K - x.size(-1) < bvr_len, "x does not fit the input coefficients");
+    if (x.dim() != 2)
+        x = x.reshape({-1, x.size(-1)});
+    if (x.scalar_type() != torch::kFloat16)
+        x = x.to(torch::kFloat16);
+    if (x.size(1) != K)
+        x = at::constant_pad_nd(x, {0, K - x.size(1)});
+    const torch::Tensor table = lines.contiguous();
+    const auto [bvr, idx] = sbvr_online_encode_lines(x.contiguous(), table, bvr_len);
+    return sbvr_mm_T(bvr, idx, table, r_bvr, r_coeff_idx, r_coeff_cache, bias, 0);
+}
+
 // The dense (N, cols) weight of a default-layout encoding, fp16, bf16 or fp32 (sbvr/core.py:926-949).
 torch::Tensor sbvr_decode_weight(const torch::Tensor &bvr, const torch::Tensor &coeff_idx, const torch::Tensor &coeff_cache,
                                  int64_t bvr_len, int64_t cols, c10::ScalarType dtype)
@@ -356,6 +377,14 @@ torch::Tensor sbvr_decode_weight(const torch::Tensor &bvr, const torch::Tensor &
                                           cols, S, bvr_len, L, current_stream());
     check_encoder(rc, "sbvr_hip_decode_weight", " (N=", N, " K=", K, " cols=", cols, " S=", S, " bvr_len=", bvr_len, ")");
     return out.scalar_type() == dtype ? out : out.to(dtype);
+}
+
+// The same under the inference mode of sbvr.decode.
+torch::Tensor sbvr_decode(const torch::Tensor &bvr, const torch::Tensor &coeff_idx, const torch::Tensor &coeff_cache, int64_t bvr_len,
+                          int64_t cols, c10::ScalarType dtype)
+{
+    const c10::InferenceMode inference;
+    return sbvr_decode_weight(bvr, coeff_idx, coeff_cache, bvr_len, cols, dtype);
 }
 
 // fp16 l_w (M, K) against a trans=True weight: r_bvr (N/32, K, S), r_coeff_idx (N/G, K) (sbvr_ops.cpp:79-120).
@@ -416,8 +445,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
           py::arg("coeff_cache"), py::arg("bias"), py::arg("bvr_len"), py::arg("k_padded"), py::arg("out_features"));
     m.def("_online_encode_lines", &sbvr_online_encode_lines, "activations to the arrays of an encoded left operand", py::arg("x"),
           py::arg("lines"), py::arg("bvr_len"), no_gil);
+    m.def("_online_mm_T", &sbvr_online_mm_T, "sbvr.online_mm_T", py::arg("x"), py::arg("lines"), py::arg("r_bvr"), py::arg("r_coeff_idx"),
+          py::arg("r_coeff_cache"), py::arg("bias"), py::arg("bvr_len"), no_gil);
     m.def("_decode_weight", &sbvr_decode_weight, "the dense weight of a default-layout encoding", py::arg("bvr"),
           py::arg("coeff_idx"), py::arg("coeff_cache"), py::arg("bvr_len"), py::arg("cols"), py::arg("dtype"), no_gil);
+    m.def("_decode", &sbvr_decode, "sbvr.decode", py::arg("bvr"), py::arg("coeff_idx"), py::arg("coeff_cache"), py::arg("bvr_len"),
+          py::arg("cols"), py::arg("dtype"), no_gil);
     m.def("_workspace", &workspace_of_current_stream, "the split-K workspace of the device's current stream", py::arg("nbytes"),
           py::arg("device"));
     m.def("last_kernel", &sbvr_hip_last_kernel, "which kernel the last linear call of this thread launched");

@@ -103,6 +103,22 @@ class _sbvr_serialized():
                 self.input_num_sums, input_coeff)
 
 
+@torch.inference_mode()
+def _view(t, shape):
+    return t.view(shape)
+
+
+_hip_module = None
+
+
+def _hip():
+    global _hip_module
+    if _hip_module is None:
+        from . import hip
+        _hip_module = hip
+    return _hip_module
+
+
 class sbvr(torch.nn.Module):
     """An SBVR-encoded tensor.  Constructor arguments as core.py:205-215:
     ``data`` to encode or ``sbvr_serialized`` to restore; ``trans`` encodes the
@@ -285,12 +301,22 @@ class sbvr(torch.nn.Module):
         return (S == self.num_sums and shape.numel() == rows * shape[-1] and
                 _padded(shape[-1], self.bvr_len) == words * 32)
 
-    @torch.inference_mode()
     def decode(self):
         """The dense tensor this object stands for, in ``original_dtype``: every
         element is one of its group's 2^S points ``bin_combs @ line``
         (core.py:926-949)."""
         bvr = self.bvr
+        shape = self.original_data_shape
+        if bvr.is_cuda and self._shape_is_the_arrays(bvr):
+            hip = _hip()
+            if hip._ext():
+                out = hip._native("_decode", bvr, self.coeff_idx, self.coeff_cache, self.bvr_len, shape[-1], self.original_dtype)
+                if out is not None:
+                    return out if len(shape) == 2 else _view(out, shape)
+        return self._decode_general(bvr)
+
+    @torch.inference_mode()
+    def _decode_general(self, bvr):
         if bvr.is_cuda and self._shape_is_the_arrays(bvr):
             from . import hip
             out = hip.decode_weight_if_covered(bvr, self.coeff_idx, self.coeff_cache, self.bvr_len,
@@ -388,10 +414,19 @@ class sbvr(torch.nn.Module):
 
     _online_transform = _online_tranfrom
 
-    @torch.inference_mode()
     def online_mm_T(self, rhs, bias=None):
         """``rhs`` (M, K) activations, encoded on the fly against the profiled input coefficients, times this
         encoded weight transposed: (M, N) fp16 through the both-encoded operator."""
+        p = self._parameters
+        if "input_coeff" in p and type(self) is sbvr and isinstance(rhs, torch.Tensor):
+            # (straight from the parameters: look-ups through Module.__getattr__ cost as much as the checks in the call)
+            out = _hip()._native("_online_mm_T", rhs, p["input_coeff"], p.get("bvr"), p.get("coeff_idx"), p.get("coeff_cache"), bias, self.bvr_len)
+            if out is not None:
+                return out
+        return self._online_mm_T_general(rhs, bias)
+
+    @torch.inference_mode()
+    def _online_mm_T_general(self, rhs, bias):
         from . import hip
         if bias is None:
             bias = self._get_dummy_bias()
@@ -403,7 +438,14 @@ class sbvr(torch.nn.Module):
 def mm_T(lhs, rhs, bias):
     """lhs @ rhs^T for two encoded operands in the default uint32 layout
     (core.py:1029-1039)."""
-    from . import hip
+    hip = _hip()
+    if type(lhs) is sbvr and type(rhs) is sbvr:
+        # (straight from the parameters, and no tensor made for "no bias": half of what a call cost the host)
+        l, r = lhs._parameters, rhs._parameters
+        out = hip._native("_sbvr_mm_T", l.get("bvr"), l.get("coeff_idx"), l.get("coeff_cache"), r.get("bvr"), r.get("coeff_idx"),
+                          r.get("coeff_cache"), bias)
+        if out is not None:
+            return out
     if bias is None:
         bias = lhs._get_dummy_bias()
     return hip._sbvr_mm_T(lhs.bvr, lhs.coeff_idx, lhs.coeff_cache,

@@ -163,3 +163,24 @@ def test_input_coefficients_of_any_strides():
     enc.input_coeff = strided
     bvr2, idx2, coeff = enc._online_tranfrom(x)
     assert torch.equal(bvr.view(torch.int32), bvr2.view(torch.int32)) and torch.equal(idx, idx2) and torch.equal(coeff, lines)
+
+
+@pytest.mark.parametrize("K,shape,dtype,bias", [(256, (3, 256), torch.float16, False), (250, (5, 250), torch.float32, True),
+                                                (250, (2, 4, 250), torch.bfloat16, False), (256, (1, 256), torch.float16, True)])
+def test_online_mm_T_in_one_call_equals_its_steps(K, shape, dtype, bias):
+    """Activations of other types and shapes, K padded, a bias: the one native call against the transform and the
+    product by themselves; both leave inference tensors."""
+    import sbvr
+    from sbvr import hip, synth
+    dev = torch.device("cuda:0")
+    bvr, idx, cache = (t.to(dev) for t in synth.random_encoding(70, 256, 4, 128, 64, seed=1))
+    enc = sbvr.sbvr.from_parts(bvr, idx, cache, 128, original_shape=(70, K))
+    enc.input_num_sums = 8
+    enc.input_coeff = torch.nn.Parameter(synth.make_lines(2, 8, 1.0, 3).to(dev), requires_grad=False)
+    x = torch.randn(shape, generator=torch.Generator().manual_seed(2)).to(dtype).to(dev)
+    b = torch.randn(70, generator=torch.Generator().manual_seed(3)).to(torch.float16).to(dev) if bias else None
+    y, want = enc.online_mm_T(x, b), enc._online_mm_T_general(x, b)
+    assert torch.equal(y, want) and y.is_inference() == want.is_inference()
+    d, general = enc.decode(), enc._decode_general(enc.bvr)
+    assert torch.equal(d, general) and d.shape == (70, K) and d.is_inference() == general.is_inference()
+    assert torch.equal(sbvr.mm_T(enc, enc, None), hip._sbvr_mm_T(bvr, idx, cache, bvr, idx, cache, enc._get_dummy_bias()))
