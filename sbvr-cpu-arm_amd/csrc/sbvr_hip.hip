@@ -2748,6 +2748,251 @@ sbvr_row_deq_mfma_kernel(const uint16_t *__restrict__ x, const uint32_t *__restr
     }
 }
 
+// The trans=True product for several batch rows (2 to 4 planes): every weight decoded once for up to 32 rows.
+// A lane owns two neighbouring rows k of the weight and decodes their 32 columns by table look-up (sbvr_gemm_rows32_lut_kernel):
+// the row's 2^S subset sums as fp16 and, scaled by 2^11, what that rounding left over, so that a weight is the sum of two
+// fp16 values to 22 bits: as exact as the fp32 sums of the kernels above, whose error against 64 bits it does not exceed.  The pairs (k, k + 1) go to a
+// tile of 32 columns x 128 k in LDS (a lane's dwords of a column lie side by side; columns 272 bytes apart, so that 16 lanes
+// reading 16 columns meet different banks) and come back as the B operands of eight v_mfma_f32_32x32x16_f16 each, with the
+// batch rows, read from memory as they are, as A.  A workgroup owns 32 columns and 32 batch rows; its waves
+// take the tiles of K in turn and meet in LDS, and K is split across workgroups through the 64-bit accumulators.
+// Bound by the vector ALU: 684 operations a tile and wave with 4 planes (308 of them permutes), whatever the
+// number of rows, where the kernels above take 384 per 64 k and row or an A image per row.  Four waves a workgroup and one
+// tile each, so that three workgroups share a CU (two tiles a wave and eight waves: 8 rows x 12032, K 4853 45 us, 34 so).
+constexpr int kDeqRowsWaves = 4, kDeqTile = 32 * 272;         // bytes of a tile
+
+struct RowDeqArgs {
+    const uint16_t *x;
+    const uint32_t *bvr;
+    const void *idx;
+    const uint16_t *cache;
+    const uint16_t *bias;
+    uint16_t *out;
+    unsigned long long *acc;
+    int M, N, K, L, G, idx16, ksplit, per_part;               // per_part: tiles of 128 along K of a part
+};
+
+// The subset sums of a line in two fp16 parts, as byte tables: the sum rounded, and 2^11 times what is left.
+template <int S>
+__device__ __forceinline__ void build_split_tables(const uint32_t (&c)[(S + 1) / 2], LutTables<S> &head, LutTables<S> &rest)
+{
+    float s[1 << S];
+    s[0] = 0.f;
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+        const float cf = h2f(static_cast<uint16_t>(q & 1 ? c[q / 2] >> 16 : c[q / 2] & 0xffffu));
+#pragma unroll
+        for (int i = 0; i < (1 << q); ++i)
+            s[(1 << q) + i] = i == 0 ? cf : s[i] + cf;
+    }
+    uint32_t eh[1 << (S - 1)], er[1 << (S - 1)];
+#pragma unroll
+    for (int i = 0; i < (1 << (S - 1)); ++i) {
+        v2h h, r;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            h[e] = static_cast<_Float16>(s[2 * i + e]);
+            r[e] = static_cast<_Float16>((s[2 * i + e] - static_cast<float>(h[e])) * 2048.f);
+        }
+        eh[i] = __builtin_bit_cast(uint32_t, h);
+        er[i] = __builtin_bit_cast(uint32_t, r);
+    }
+#pragma unroll
+    for (int i = 0; i < LutTables<S>::TW; ++i) {
+        head.lo[i] = __builtin_amdgcn_perm(eh[2 * i + 1], eh[2 * i], 0x06040200u);
+        head.hi[i] = __builtin_amdgcn_perm(eh[2 * i + 1], eh[2 * i], 0x07050301u);
+        rest.lo[i] = __builtin_amdgcn_perm(er[2 * i + 1], er[2 * i], 0x06040200u);
+        rest.hi[i] = __builtin_amdgcn_perm(er[2 * i + 1], er[2 * i], 0x07050301u);
+    }
+}
+
+typedef v4u __attribute__((aligned(2))) v4u_half_aligned;
+
+template <int S>
+__global__ void __launch_bounds__(64 * kDeqRowsWaves)
+__attribute__((amdgpu_waves_per_eu(3, 8)))
+sbvr_row_deq_rows_kernel(const RowDeqArgs a)
+{
+    extern __shared__ __align__(16) unsigned char dsm[];
+    constexpr int CW = (S + 1) / 2;
+    const int lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = static_cast<int>(blockDim.x >> 6);
+    const int M = a.M, N = a.N, K = a.K;
+    const int nw = blockIdx.x, m0 = blockIdx.y * 32;
+    const int tiles = (K + 127) / 128;
+    const int t_begin = blockIdx.z * a.per_part, t_end = min(tiles, t_begin + a.per_part);
+    const uint32_t *const words = a.bvr + static_cast<size_t>(nw) * K * S;
+    const size_t ibase = static_cast<size_t>((nw * 32) / a.G) * K;
+    const uint16_t *const xrow = a.x + static_cast<size_t>(min(m0 + j, M - 1)) * K;     // (rows past M repeat the last one; dropped at the end)
+    unsigned char *const tile = dsm + wave * kDeqTile;
+
+    struct Stage {
+        Planes<S> w[2];
+        int lo[2], hi[2];                   // the two bytes of a line index, as loaded
+    };
+    auto load = [&](int t, Stage &s) __attribute__((always_inline)) {
+        const uint8_t *ib = static_cast<const uint8_t *>(a.idx);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int k = min(128 * t + 2 * lane + e, K - 1);
+            s.w[e] = load_planes<S>(words + static_cast<size_t>(k) * S);
+            const size_t at = (ibase + static_cast<size_t>(k)) << a.idx16;
+            s.lo[e] = ib[at];
+            s.hi[e] = ib[at + a.idx16];
+        }
+    };
+    auto gather = [&](const Stage &s, uint32_t (&c)[2][CW]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int line = min(a.idx16 ? s.lo[e] | (s.hi[e] << 8) : s.lo[e], a.L - 1);
+            load_line_words<S>(a.cache + static_cast<size_t>(line) * S, c[e]);
+        }
+    };
+
+    v16f acc_head, acc_rest;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        acc_head[r] = acc_rest[r] = 0.f;
+
+    Stage now;
+    uint32_t c[2][CW];
+    if (t_begin + wave < t_end) {           // wave-uniform
+        load(t_begin + wave, now);
+        gather(now, c);
+    }
+    for (int t = t_begin + wave; t < t_end; t += waves) {
+        Stage next;
+        load(min(t + waves, tiles - 1), next);
+        // -- the batch rows of the tile: elements 16 s + 8 h .. + 7 of row j for slice s
+        v4u x[8];
+        if (128 * t + 128 <= K) {           // wave-uniform
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+                x[s] = *reinterpret_cast<const v4u_half_aligned *>(xrow + 128 * t + 16 * s + 8 * h);
+        } else {                            // the last tile: whole slices, the one with the end of K element by element, zeros
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const int k0 = 128 * t + 16 * s, k = k0 + 8 * h;
+                x[s] = v4u{0u, 0u, 0u, 0u};
+                if (k0 + 16 <= K) {
+                    x[s] = *reinterpret_cast<const v4u_half_aligned *>(xrow + k);
+                } else if (k0 < K) {
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const uint32_t e0 = xrow[min(k + 2 * d, K - 1)], e1 = xrow[min(k + 2 * d + 1, K - 1)];
+                        x[s][d] = (k + 2 * d < K ? e0 : 0u) | (k + 2 * d + 1 < K ? e1 << 16 : 0u);
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // -- decode: rows 128 t + 2 lane and + 1, 32 columns each
+        LutTables<S> head[2], rest[2];
+        uint32_t Q[2][4];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            build_split_tables<S>(c[e], head[e], rest[e]);
+            uint32_t w[S];
+            const bool in = 128 * t + 2 * lane + e < K;      // (a row past the end selects the empty sum)
+#pragma unroll
+            for (int q = 0; q < S; ++q)
+                w[q] = in ? now.w[e].w[q] : 0u;
+            lut_nibble_words<S>(w, Q[e]);
+        }
+        // the first fp16 values through the wave's tile and the MFMAs, then what they left over (the LDS serves a wave's
+        // accesses in order)
+        auto multiply = [&](const LutTables<S> (&tab)[2], v16f &acc) __attribute__((always_inline)) {
+#pragma unroll
+            for (int p = 0; p < 8; ++p) {
+                uint32_t a01, a23, b01, b23;
+                lut_look_up<S>(tab[0], Q[0], p, a01, a23);
+                lut_look_up<S>(tab[1], Q[1], p, b01, b23);
+                uint32_t *const at = reinterpret_cast<uint32_t *>(tile + p * 272) + lane;
+                at[0 * 68] = __builtin_amdgcn_perm(b01, a01, 0x05040100u);
+                at[8 * 68] = __builtin_amdgcn_perm(b01, a01, 0x07060302u);
+                at[16 * 68] = __builtin_amdgcn_perm(b23, a23, 0x05040100u);
+                at[24 * 68] = __builtin_amdgcn_perm(b23, a23, 0x07060302u);
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const v4u b = *reinterpret_cast<const v4u *>(tile + j * 272 + 32 * s + 16 * h);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, x[s]), __builtin_bit_cast(v8h, b), acc, 0, 0, 0);
+            }
+            __builtin_amdgcn_wave_barrier();
+        };
+        multiply(head, acc_head);
+        gather(next, c);
+        multiply(rest, acc_rest);
+        now = next;
+    }
+    // ---- partial results meet in LDS; D[i][jj] sits in lane jj + 32*((i/4)%2), register (i%4) + 4*(i/8)
+    __syncthreads();                        // (over the tiles)
+    float *const red = reinterpret_cast<float *>(dsm);
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        red[(wave * 16 + r) * 64 + lane] = fmaf(acc_rest[r], 1.f / 2048.f, acc_head[r]);
+    __syncthreads();
+    const int n = nw * 32 + j;
+    for (int r = wave; r < 16; r += waves) {                  // wave-uniform
+        float total = 0.f;
+        for (int w = 0; w < waves; ++w)
+            total += red[(w * 16 + r) * 64 + lane];
+        const int m = m0 + 8 * (r >> 2) + 4 * h + (r & 3);
+        if (m >= M)                                           // (N is a multiple of 32)
+            continue;
+        const size_t at = static_cast<size_t>(m) * N + n;
+        if (a.ksplit > 1) {
+            unsigned long long tot = (1ull << 56) + static_cast<unsigned long long>(to_fixed(total) + kAccBias);
+            tot += __hip_atomic_fetch_add(a.acc + at, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (static_cast<int>(tot >> 56) != a.ksplit)
+                continue;
+            const long long sum = static_cast<long long>(tot & ((1ull << 56) - 1)) - (static_cast<long long>(a.ksplit) << 47);
+            const float hi = static_cast<float>(static_cast<int>(sum >> 24));
+            const float lo = static_cast<float>(static_cast<int>(sum & 0xffffff));
+            total = fmaf(hi, 1.f / (1 << (kAccFracBits - 24)), lo * (1.f / (1 << kAccFracBits)));
+            __hip_atomic_store(a.acc + at, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        a.out[at] = f2h(a.bias ? total + h2f(a.bias[n]) : total);
+    }
+}
+
+// Whether several rows go that way.  Not while a CU has no more than one workgroup of the one-row kernels and each of its
+// waves at most one step (K up to 704: 2 rows x 1024, K 513 8.4 us against 6.8; from K 768 on it is even or ahead), and not
+// two rows of the matrix-core kernel's shapes with columns enough for all CUs (14336 columns, K 4096: 28 us against 25).
+// us, these kernels and the one above: 3 rows x 4096, K 4096, 4 planes 12.7 and 10.1; 4096 columns, K 4100 2 / 8 / 32 rows
+// 14.9 / 52 / 200 and 13.2 / 13.6 / 16.5; 2048 columns, K 2050, 2 planes, 2 / 8 / 32 rows 8.3 / 15.7 / 54 and 7.4 / 7.7 / 9.9;
+// 14336 columns, K 10858, 3 planes, 32 rows 1397 and 65.
+bool row_deq_rows(int M, int N, int K, int S, int G, int cus)
+{
+    if (M < 2 || S < 2 || S > 4 || (K <= 704 && static_cast<long>(N / 32) * M <= cus))
+        return false;
+    return !(M == 2 && S == 4 && K % kSub == 0 && G % 64 == 0 && (N / 32 + 1) / 2 * 2 >= cus);
+}
+
+template <int S>
+hipError_t launch_row_deq_rows(const RowDeqArgs &a, int waves, hipStream_t st)
+{
+    const dim3 grid(static_cast<unsigned>(a.N / 32), static_cast<unsigned>((a.M + 31) / 32), static_cast<unsigned>(a.ksplit));
+    const size_t lds = static_cast<size_t>(waves) * kDeqTile;
+    {
+        static bool raised_on[16] = {};
+        std::lock_guard<std::mutex> guard(g_dev_lock);
+        int dev_now = 0;
+        if (hipGetDevice(&dev_now) != hipSuccess || dev_now < 0 || dev_now >= 16)
+            dev_now = 0;
+        if (!raised_on[dev_now]) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(sbvr_row_deq_rows_kernel<S>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kDeqRowsWaves * kDeqTile);
+            if (e != hipSuccess)
+                return e;
+            raised_on[dev_now] = true;
+        }
+    }
+    hipLaunchKernelGGL(sbvr_row_deq_rows_kernel<S>, grid, dim3(64 * waves), lds, st, a);
+    return hipGetLastError();
+}
+
 template <typename LIdxT, typename RIdxT>
 __global__ void __launch_bounds__(256)
 sbvr_mm_T_kernel(const uint32_t *__restrict__ l_bvr, const void *__restrict__ l_idx,
@@ -4049,6 +4294,26 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
     if (idx_bytes == 1 && L > 256)
         return fail(SBVR_HIP_EINVAL, "uint8 indices cannot address L=%d lines", L);
     const bool tables_aligned = reinterpret_cast<uintptr_t>(r_bvr) % 16 == 0 && reinterpret_cast<uintptr_t>(r_coeff_cache) % 16 == 0;
+    if (row_deq_rows(M, N, K, S, G, current_cus()) && tables_aligned && (static_cast<long>(M) + 31) / 32 <= 65535 && !env_switches().rowdeq_lanes) {
+        // every weight decoded once for all rows; K in as many parts as give the CUs a workgroup each
+        const int tiles = (K + 127) / 128;
+        const long wgs = static_cast<long>(N / 32) * ((M + 31) / 32);
+        int ksplit = 1;
+        if (workspace && reinterpret_cast<uintptr_t>(workspace) % 8 == 0 &&
+            workspace_bytes >= static_cast<size_t>(M) * N * sizeof(unsigned long long))
+            while (ksplit < 32 && wgs * ksplit < 2L * current_cus() && tiles >= 8 * ksplit)
+                ksplit *= 2;
+        RowDeqArgs a{static_cast<const uint16_t *>(x), r_bvr, r_coeff_idx, static_cast<const uint16_t *>(r_coeff_cache),
+                     static_cast<const uint16_t *>(bias), static_cast<uint16_t *>(out), static_cast<unsigned long long *>(workspace),
+                     M, N, K, L, G, idx_bytes == 2 ? 1 : 0, 1, 1};
+        a.per_part = (tiles + ksplit - 1) / ksplit;
+        a.ksplit = (tiles + a.per_part - 1) / a.per_part;       // (no empty parts)
+        const int waves = a.per_part < kDeqRowsWaves ? a.per_part : kDeqRowsWaves;
+        const hipError_t e = S == 4 ? launch_row_deq_rows<4>(a, waves, st) : (S == 3 ? launch_row_deq_rows<3>(a, waves, st) : launch_row_deq_rows<2>(a, waves, st));
+        if (e != hipSuccess)
+            return fail(SBVR_HIP_ELAUNCH, "row_deq launch: %s", hipGetErrorString(e));
+        return SBVR_HIP_OK;
+    }
     if (M <= 65535 && S == 4 && K % kSub == 0 && G % 64 == 0 && tables_aligned && reinterpret_cast<uintptr_t>(x) % 4 == 0 &&
         reinterpret_cast<uintptr_t>(r_coeff_idx) % 4 == 0 && !env_switches().rowdeq_lanes) {
         // plane sums on the matrix cores over bits transposed across lanes
@@ -4136,6 +4401,8 @@ size_t sbvr_hip_row_deq_mm_T_workspace(int M, int N)
 {
     if (M <= 0 || N <= 0)
         return 0;
+    if (M >= 2)
+        return static_cast<long>(N / 32) * ((M + 31) / 32) < 2L * current_cus() ? static_cast<size_t>(M) * N * sizeof(unsigned long long) : 0;
     const long col_wgs = static_cast<long>((N / 32 + 1) / 2) * M;
     return col_wgs * 2 < 3L * current_cus() / 4 ? static_cast<size_t>(M) * N * sizeof(unsigned long long) : 0;
 }

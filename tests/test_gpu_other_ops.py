@@ -148,6 +148,38 @@ def test_row_deq_mm_T(oracle, M, N, K, S, G, L):
     assert d.max() <= 2.0 ** -9 * max(np.abs(want).max(), 1.0)
 
 
+@pytest.mark.parametrize("M,N,K,S,G,L,bias", [
+    (2, 8192, 705, 4, 64, 300, True),           # the smallest K of its rule; the last tile has one row, K odd
+    (33, 512, 1, 3, 32, 9, False),              # one row of the weight, two blocks of batch rows
+    (32, 544, 127, 2, 32, 256, False),          # one tile, one row short
+    (17, 1024, 129, 4, 256, 40, True),          # a second tile with one row
+    (3, 4096, 4096, 4, 256, 256, False),        # K in parts
+    (8, 512, 4143, 2, 256, 768, True),          # K in parts of different lengths, uint16 indices
+    (65, 256, 1001, 4, 128, 256, False),        # three blocks of batch rows
+])
+def test_row_deq_mm_T_of_several_rows(oracle, M, N, K, S, G, L, bias):
+    """Every weight decoded once for all rows, as two fp16 values: within 2 fp16 ulps of the sums in 64 bits (the fp32 additions
+    and one rounding), the same bits on a second call, the accumulators left zero."""
+    import sbvr
+    from sbvr import hip
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(N + K)
+    bvr, idx, cache = _rand_enc(rng, K, N, S, G, L, oracle)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    b = rng.standard_normal(N).astype(np.float16) if bias else np.zeros(0, np.float16)
+    args = [torch.from_numpy(a).to(dev) for a in (x, bvr, idx, cache, b)]
+    y = sbvr._sbvr_row_deq_mm_T(*args, 0, bvr_len=G)
+    assert torch.equal(y, sbvr._sbvr_row_deq_mm_T(*args, 0, bvr_len=G))
+    bits = (bvr[:, :, None, :] >> np.arange(32, dtype=np.uint32)[None, None, :, None]) & 1          # (N/32, K, 32, S)
+    line = cache.astype(np.float64)[idx.astype(np.int64)]                                          # (N/G, K, S)
+    w = np.einsum("nkbs,nks->nkb", bits.astype(np.float64), np.repeat(line, G // 32, axis=0))
+    want = x.astype(np.float64) @ w.transpose(1, 0, 2).reshape(K, N) + (b.astype(np.float64) if bias else 0.0)
+    rms = np.sqrt(np.mean(want ** 2))
+    err = np.abs(y.float().cpu().numpy() - want) / (np.maximum(np.abs(want), rms) * 2.0 ** -10)
+    assert err.max() <= 2.0, err.max()
+    assert int(hip._workspace(8 * M * N, dev).count_nonzero()) == 0
+
+
 def test_row_deq_mm_T_without_workspace_and_repeatable(oracle):
     """The reference-shaped entry point (no workspace: K is never split across workgroups) against the oracle at a
     shape the binding would split, and the split form twice: the fixed-point accumulators make it repeatable."""
