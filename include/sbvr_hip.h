@@ -96,16 +96,17 @@ size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G);
  *                   table look-up form has no instance (6 or 8 planes) or flags
  *                   bit 1 is set (5..16 rows in a variant whose waves share the
  *                   activation operands, where N >= 32 for up to 8 rows, 64 beyond);
- *   32-row kernel   up to 32 rows.  Its table look-up form (2, 3 or 4 planes, K and
+ *   32-row kernel   up to 32 rows.  Its table look-up form (K and
  *                   G multiples of 64: a weight is looked up among the subset sums
- *                   of its group's coefficient line; with a workspace and few
+ *                   of its group's coefficient line, with 6 or 8 planes in two or
+ *                   three tables; with a workspace and few
  *                   columns K is split across workgroups through the decode
- *                   kernel's accumulators) is taken for 9..32 rows: from 9 rows on
- *                   it is the faster one (4096 -> 14336, 4 planes, 16 rows: 15.4 us
- *                   against 20 us).  Its arithmetic form (K and G multiples of 32,
- *                   S in {2,3,4,6,8}; same results) takes 17..32 rows otherwise, and
- *                   5..16 rows of shapes the decode kernel does not cover (N < 16,
- *                   K or G not a multiple of 128);
+ *                   kernel's accumulators) is taken for 9..32 rows with 2 to 4
+ *                   planes: from 9 rows on it is the faster one (4096 -> 14336, 4
+ *                   planes, 16 rows: 15.4 us against 20 us); for 17..32 rows with 6
+ *                   or 8; and for 5..16 rows of shapes the decode kernel does not
+ *                   cover (N < 16, groups of 64).  Its arithmetic form (K and G
+ *                   multiples of 32, S in {2,3,4,6,8}) takes 5..32 rows otherwise;
  *   prefill kernel  M > 32 (or 17..32 with flags bit 1), K and G multiples of 64,
  *                   same S; with a workspace, and where that is the faster, K is
  *                   split across workgroups.  It decodes by table look-up in
@@ -117,9 +118,8 @@ size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G);
  * which is how decode() of sbvr/core.py:927-949 produces a weight (bin_combs @
  * coeff, :345-366): against x @ decode(W)^T they are as close as the decode
  * kernel is to the unrounded weights (2 fp16 ulps).  The 32-row kernel's
- * arithmetic form (6 and 8 planes, groups of 32 or 64) adds the coefficients up in
- * fp16 plane by plane, the prefill kernel with 6 or 8 planes two or three table
- * entries.  Either way the error against unrounded weights is a few 1e-3 of the
+ * arithmetic form adds the coefficients up in fp16 plane by plane, the look-up
+ * forms with 6 or 8 planes two or three table entries.  Either way the error against unrounded weights is a few 1e-3 of the
  * RMS output, within the 1e-2 relative bound for outputs that are not small
  * against it.  sbvr_hip_last_rounding() tells which of the three a call took.
  * The reference has no kernel of exactly this form (its fp16-activation

@@ -34,8 +34,8 @@
 // (weights decoded by table look-up in registers, activations shared
 // through LDS).  In between, 9..32 rows (17..32 with 6
 // or 8 planes): the batch rows are the 32 rows of one MFMA, weights decoded in
-// registers -- by table look-up for 2..4 planes (sbvr_gemm_rows32_lut_kernel),
-// arithmetically otherwise (sbvr_gemm_rows32_kernel).
+// registers -- by table look-up (sbvr_gemm_rows32_lut_kernel; K and G multiples
+// of 64), arithmetically otherwise (sbvr_gemm_rows32_kernel).
 //
 // The reference's own operator forms: both operands encoded: the matrix-core
 // kernel of mm_ops.hip (K and G multiples of 128), one left row of up to 4 planes
@@ -1732,8 +1732,8 @@ bool rows32_path_ok(int M, int N, int K, int S, int G)
            static_cast<double>(K / 32) * N * S < 2147483648.0;
 }
 
-// The arithmetic form of the 32-row kernel: for 17..32 rows where the table look-up form has no instance (6 or 8
-// planes, K or G not a multiple of 64), and for 5..16 rows of shapes the decode kernels do not cover.
+// The 32-row kernels for 17..32 rows, and for 5..16 rows of shapes the decode kernels do not cover; the arithmetic form where
+// the table look-up form has no instance (K or G not a multiple of 64).
 bool rows32_preferred(int M, int N, int K, int S, int G, int cus)
 {
     (void)cus;
@@ -1781,6 +1781,9 @@ hipError_t launch_rows32(int S, RowsArgs a, hipStream_t st)
 // the lane's word for MFMA q = 0..3 of a step; the activations (the lane's batch row, the same 32 elements:
 // 64 bytes, four loads) are put into that order with four permutes per MFMA.
 // K can be split across workgroups (blockIdx.y) through the decode kernel's 64-bit accumulators.
+// 6 and 8 planes look a weight up in two or three tables (build_weight_tables); the arithmetic form, which does not split K,
+// took 84 us where this takes 19 (24 rows x 1304, K 19200, 8 planes), 37 and 25 (32 x 14336, K 4096, 8 planes), 72 and 52
+// (26 x 9346, K 10496, 6 planes in groups of 64); 5 to 8 rows in groups of 64: 12.4 and 7.6 (6 x 4096, K 4096, 4 planes).
 constexpr int kLutWaves = 8;
 // Batch rows from which the linear takes this kernel.  Measured at 4096 -> 14336 / 14336 -> 4096, 4 planes: 15.3-16.1 us
 // for any row count up to 16 (17.3-17.5 at 32; 11.4-12.5 with 2 planes, 12.6-13.7 with 3), against 11.7-12.5 us at
@@ -1794,7 +1797,6 @@ template <int S, bool kHalfRows, bool kShare>
 __global__ void __launch_bounds__(64 * kLutWaves)
 sbvr_gemm_rows32_lut_kernel(const RowsArgs a)
 {
-    static_assert(S >= 2 && S <= 4, "tables of 4, 8 or 16 entries");
     __shared__ float red[kLutWaves][16][64];
     // a wave's activations of one step: 32 rows of 128 bytes (the word pair), rows 144 bytes apart so that 16 lanes
     // reading the same 16-byte chunk of 16 rows hit 16 different bank groups
@@ -1859,8 +1861,8 @@ sbvr_gemm_rows32_lut_kernel(const RowsArgs a)
     for (int r = 0; r < 16; ++r)
         acc[r] = 0.f;
 
-    LutTables<S> tables;
-    auto build_table = [&](const uint32_t (&c)[CW]) __attribute__((always_inline)) { lut_build_tables<S>(c, tables); };
+    WeightTables<S> tables;
+    auto build_table = [&](const uint32_t (&c)[CW]) __attribute__((always_inline)) { build_weight_tables<S>(c, tables); };
     auto compute = [&](const Step &st) __attribute__((always_inline)) {
         // ---- activations: rows as loaded -> LDS -> a row per lane (the LDS serves a wave's accesses in order)
 #pragma unroll
@@ -1872,11 +1874,11 @@ sbvr_gemm_rows32_lut_kernel(const RowsArgs a)
         for (int i = 0; i < 4; ++i)
             xl[i] = *reinterpret_cast<const v4u *>(xr + 16 * i);
         __builtin_amdgcn_wave_barrier();
-        uint32_t Q[4];
-        lut_nibble_words<S>(st.w, Q);
+        WeightNibbles<S> nibbles;
+        weight_nibbles<S>(st.w, nibbles);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const v4u bw = lut_operand<S>(tables, Q, q);
+            const v4u bw = weight_operand<S>(tables, nibbles, q);
             v4u aw;
             // dword i of the lane's 64 bytes of activations holds elements 2i, 2i + 1
             const uint32_t d0 = xl[0][q], d1 = xl[1][q], d2 = xl[2][q], d3 = xl[3][q];
@@ -1964,7 +1966,7 @@ sbvr_gemm_rows32_lut_kernel(const RowsArgs a)
 
 bool lut_path_ok(int M, int N, int K, int S, int G)
 {
-    return M >= 1 && M <= kRowsMax && K % 64 == 0 && G % 64 == 0 && (S == 2 || S == 3 || S == 4) &&
+    return M >= 1 && M <= kRowsMax && K % 64 == 0 && G % 64 == 0 && (S == 2 || S == 3 || S == 4 || S == 6 || S == 8) &&
            static_cast<double>(K / 32) * N * S < 2147483648.0;
 }
 
@@ -2001,6 +2003,8 @@ hipError_t launch_rows32_lut(int S, RowsArgs a, hipStream_t st)
 #ifndef SBVR_FAST_BUILD
     case 2: SBVR_LUT(2);
     case 3: SBVR_LUT(3);
+    case 6: SBVR_LUT(6);
+    case 8: SBVR_LUT(8);
 #endif
     default: return hipErrorInvalidConfiguration;
     }
@@ -3981,10 +3985,11 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
                 return fail(SBVR_HIP_EINVAL, "x_out must not alias x or delta (other workgroups still read them)");
         }
     }
-    // from kLutMinRows batch rows on, with 2 to 4 planes: the 32-row kernel that decodes by table look-up
-    // (SBVR_HIP_LUT_ROWS moves the threshold: a development switch)
+    // from kLutMinRows batch rows on with 2 to 4 planes, and wherever the decode kernels have no shape: the 32-row kernel that
+    // decodes by table look-up (SBVR_HIP_LUT_ROWS moves the threshold: a development switch)
     const int lut_rows = env_switches().lut_rows > 0 ? env_switches().lut_rows : kLutMinRows;
-    if (pro.mode == kXPlain && !(flags & 3) && aligned && M >= lut_rows && lut_path_ok(M, N, K, S, G) &&
+    if (pro.mode == kXPlain && !(flags & 3) && aligned && lut_path_ok(M, N, K, S, G) &&
+        ((S <= 4 && M >= lut_rows) || rows32_preferred(M, N, K, S, G, current_cus())) &&
         reinterpret_cast<uintptr_t>(x) % 16 == 0) {
         RowsArgs r{};
         r.x = static_cast<const uint16_t *>(x);
@@ -4008,7 +4013,9 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         if (e != hipSuccess)
             return fail(SBVR_HIP_ELAUNCH, "rows32 (table look-up) launch: %s", hipGetErrorString(e));
         g_last_kernel = SBVR_HIP_KERNEL_ROWS32;
-        g_last_rounding = SBVR_HIP_ROUNDING_DECODE;
+        // (6 and 8 planes: table entries added, closer than plane by plane.  5 to 8 rows: as decode() rounds, reported as the
+        // looser of the two, which is what such a call has always said)
+        g_last_rounding = S <= 4 && M >= kLutMinRows ? SBVR_HIP_ROUNDING_DECODE : SBVR_HIP_ROUNDING_PLANEWISE;
         return SBVR_HIP_OK;
     }
     if (pro.mode == kXPlain && !(flags & 3) && aligned && rows32_preferred(M, N, K, S, G, current_cus()) && reinterpret_cast<uintptr_t>(x) % 16 == 0) {

@@ -364,3 +364,16 @@ def test_prefill_kernel_for_17_to_32_rows(oracle, S, G):
     assert hip.last_kernel() == PREFILL
     ops = (x.numpy(), bvr.numpy(), idx.numpy(), cache.numpy(), G)
     check(y, oracle.C.linear_f16(*ops)[1], oracle.C.linear_f16(*ops, mode=1)[1], hip.last_rounding(), f"S={S} G={G}")
+
+
+@pytest.mark.parametrize("M,N,K,S,G,L,bias", [
+    (17, 96, 768, 8, 128, 200, False),
+    (32, 70, 4160, 6, 64, 300, True),          # 65 word pairs: parts and waves of different lengths; uint16 indices, bias
+    (24, 1304, 19200, 8, 256, 256, False),     # K in 8 parts
+    (5, 100, 64, 8, 64, 16, False),            # fewer rows than 9, one word pair
+    (16, 33, 192, 6, 64, 256, True),           # half the rows, three word pairs
+    (7, 200, 8192, 4, 64, 256, False),         # 4 planes below 9 rows, K in parts
+    (31, 2000, 1024, 8, 512, 256, False),
+])
+def test_rows32_table_look_up_of_more_planes_and_fewer_rows(oracle, M, N, K, S, G, L, bias):
+    run_case(oracle, N, K, S, G, M, L, seed=M + N + S, bias=bias, expect=ROWS32)
