@@ -140,6 +140,15 @@ int sbvr_hip_linear_f16(const void *x, const uint32_t *bvr, const void *coeff_id
                         void *workspace, size_t workspace_bytes, int flags,
                         void *stream);
 
+/* sbvr_hip_linear_f16 with scratch memory for a prefill's partial results: sbvr_hip_linear_f16_parts bytes (0 where a call
+ * makes none), 16-byte aligned, in any state and left in any.  Such a call needs no workspace; one whose `parts` is missing
+ * or too small keeps its partial results in the workspace, as sbvr_hip_linear_f16 does. */
+size_t sbvr_hip_linear_f16_parts(int M, int N, int K, int S, int G);
+int sbvr_hip_linear_f16_scratch(const void *x, const uint32_t *bvr, const void *coeff_idx, int idx_bytes,
+                                const void *coeff_cache, const void *bias, void *out, int M, int N, int K, int S, int G,
+                                int L, void *workspace, size_t workspace_bytes, void *parts, size_t parts_bytes, int flags,
+                                void *stream);
+
 /*
  * sbvr_hip_linear_f16 for callers that cannot allocate device memory or bring
  * a workspace (code under HIP graph capture, tight serving loops, harnesses

@@ -188,11 +188,15 @@ void launch_linear(const torch::Tensor &x, const torch::Tensor &bvr, const torch
                    const Bias &bias, const torch::Tensor &out, const LinearShape &s, int flags)
 {
     hipStream_t stream = current_stream();
-    const size_t need = sbvr_hip_linear_f16_workspace(s.M, s.N, s.K, s.S, s.G);
+    // a prefill's partial results go to memory of the call's own (torch keeps it for the stream), which need not be cleared
+    const size_t parts = sbvr_hip_linear_f16_parts(s.M, s.N, s.K, s.S, s.G);
+    const size_t need = parts ? 0 : sbvr_hip_linear_f16_workspace(s.M, s.N, s.K, s.S, s.G);
     torch::Tensor ws = need ? workspace(need, x.device(), stream, Users::kLinears) : torch::Tensor();
-    check(sbvr_hip_linear_f16(x.data_ptr(), static_cast<const uint32_t *>(bvr.data_ptr()), coeff_idx.data_ptr(), s.ib,
-                              coeff_cache.data_ptr(), bias_ptr(bias, s.N, x), out.data_ptr(), s.M, s.N, s.K, s.S, s.G,
-                              s.L, need ? ws.data_ptr() : nullptr, need ? ws.numel() : 0, flags, stream));
+    torch::Tensor scratch = parts ? at::empty({static_cast<int64_t>(parts)}, x.options().dtype(torch::kUInt8)) : torch::Tensor();
+    check(sbvr_hip_linear_f16_scratch(x.data_ptr(), static_cast<const uint32_t *>(bvr.data_ptr()), coeff_idx.data_ptr(), s.ib,
+                                      coeff_cache.data_ptr(), bias_ptr(bias, s.N, x), out.data_ptr(), s.M, s.N, s.K, s.S, s.G, s.L,
+                                      need ? ws.data_ptr() : nullptr, need ? ws.numel() : 0, parts ? scratch.data_ptr() : nullptr, parts,
+                                      flags, stream));
 }
 
 }  // namespace

@@ -60,6 +60,8 @@ def _load():
     lib.sbvr_hip_init.argtypes = [i]
     lib.sbvr_hip_linear_f16_workspace.restype = sz
     lib.sbvr_hip_linear_f16_workspace.argtypes = [i, i, i, i, i]
+    lib.sbvr_hip_linear_f16_parts.restype = sz
+    lib.sbvr_hip_linear_f16_parts.argtypes = [i, i, i, i, i]
     lib.sbvr_hip_linear_f16.argtypes = [vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, vp, sz, i, vp]
     lib.sbvr_hip_linear_f16_swiglu.argtypes = [vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, vp, sz, vp]
     lib.sbvr_hip_linear_f16_add_rmsnorm.argtypes = [vp, vp, vp, ctypes.c_float, vp, vp, vp, i, vp, vp, vp,

@@ -103,3 +103,22 @@ def test_inputs_that_are_refused(oracle):
     lin.coeff_idx = lin.coeff_idx.to(torch.int32).to(torch.uint16)
     with pytest.raises(RuntimeError):
         lin(torch.zeros((1, K), dtype=torch.float16, device=DEV))  # 16 lines want uint8 indices
+
+
+@pytest.mark.parametrize("M,N,K,S,G,bias", [(371, 890, 6144, 4, 256, True), (33, 1, 1152, 3, 128, False), (64, 515, 1216, 8, 64, True)])
+def test_prefill_parts_in_memory_of_their_own(M, N, K, S, G, bias):
+    """SBVRLinear keeps a prefill's partial results outside the shared workspace: the same bits as the function whose
+    partial results lie in it, twice, with other work on the stream in between."""
+    import sbvr
+    from sbvr import hip, synth
+    dev = torch.device("cuda:0")
+    bvr, idx, cache = (t.to(dev) for t in synth.random_encoding(N, K, S, G, 256, seed=4))
+    b = torch.randn(N, generator=torch.Generator().manual_seed(5)).to(torch.float16).to(dev) if bias else None
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(6)).to(torch.float16).to(dev)
+    assert hip._load().sbvr_hip_linear_f16_parts(M, N, K, S, G) > 0 and hip._load().sbvr_hip_linear_f16_parts(4, N, K, S, G) == 0
+    layer = sbvr.SBVRLinear(K, N, bvr, idx, cache, G, b)
+    want = sbvr._sbvr_linear_f16(x, bvr, idx, cache, b, bvr_len=G)
+    assert hip.last_kernel() == 5                      # K split
+    first = layer(x)
+    torch.full((1 << 20,), float("nan"), device=dev)
+    assert torch.equal(first, want) and torch.equal(layer(x), want)
