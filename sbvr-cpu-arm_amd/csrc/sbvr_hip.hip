@@ -2933,6 +2933,35 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
         multiply(rest, acc_rest);
         now = next;
     }
+    // A sum that is not finite: activations or coefficients that are not, or a weight beyond fp16.  The products of such an
+    // activation with the zeros of either fp16 value would make NaN of outputs that do not select it, so the wave adds its
+    // share up again as the one-row kernel does: the selected coefficients alone, products in fp32.
+    bool odd = false;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        odd = odd || !(fabsf(acc_head[r]) < INFINITY) || !(fabsf(acc_rest[r]) < INFINITY);
+    if (__any(odd)) {                       // wave-uniform
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            acc_head[r] = acc_rest[r] = 0.f;
+        for (int t = t_begin + wave; t < t_end; t += waves)
+            for (int k = 128 * t; k < min(K, 128 * t + 128); ++k) {
+                const size_t at = (ibase + static_cast<size_t>(k)) << a.idx16;
+                const uint8_t *ib = static_cast<const uint8_t *>(a.idx);
+                const int line = min(a.idx16 ? ib[at] | (ib[at + 1] << 8) : ib[at], a.L - 1);
+#pragma unroll
+                for (int q = 0; q < S; ++q) {
+                    const bool set = (words[static_cast<size_t>(k) * S + q] >> j) & 1u;
+                    const float cq = h2f(a.cache[static_cast<size_t>(line) * S + q]);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int m = min(m0 + 8 * (r >> 2) + 4 * h + (r & 3), M - 1);
+                        const float z = h2f(a.x[static_cast<size_t>(m) * K + k]) * cq;
+                        acc_head[r] += set ? z : 0.f;
+                    }
+                }
+            }
+    }
     // ---- partial results meet in LDS; D[i][jj] sits in lane jj + 32*((i/4)%2), register (i%4) + 4*(i/8)
     __syncthreads();                        // (over the tiles)
     float *const red = reinterpret_cast<float *>(dsm);
@@ -2965,14 +2994,15 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
 }
 
 // Whether several rows go that way.  Not while a CU has no more than one workgroup of the one-row kernels and each of its
-// waves at most one step (K up to 704: 2 rows x 1024, K 513 8.4 us against 6.8; from K 768 on it is even or ahead), and not
+// waves one step or two (K up to 1408: 2 rows x 1024, K 513 9.0 us against 6.8, 4 x 1024, K 800 8.2 against 8.0; from K 2000 on
+// it is ahead), and not
 // two rows of the matrix-core kernel's shapes with columns enough for all CUs (14336 columns, K 4096: 28 us against 25).
-// us, these kernels and the one above: 3 rows x 4096, K 4096, 4 planes 12.7 and 10.1; 4096 columns, K 4100 2 / 8 / 32 rows
+// us, these kernels and the one above: 3 rows x 4096, K 4096, 4 planes 12.7 and 11.2; 4096 columns, K 4100 2 / 8 / 32 rows
 // 14.9 / 52 / 200 and 13.2 / 13.6 / 16.5; 2048 columns, K 2050, 2 planes, 2 / 8 / 32 rows 8.3 / 15.7 / 54 and 7.4 / 7.7 / 9.9;
 // 14336 columns, K 10858, 3 planes, 32 rows 1397 and 65.
 bool row_deq_rows(int M, int N, int K, int S, int G, int cus)
 {
-    if (M < 2 || S < 2 || S > 4 || (K <= 704 && static_cast<long>(N / 32) * M <= cus))
+    if (M < 2 || S < 2 || S > 4 || (K <= 1408 && static_cast<long>(N / 32) * M <= cus))
         return false;
     return !(M == 2 && S == 4 && K % kSub == 0 && G % 64 == 0 && (N / 32 + 1) / 2 * 2 >= cus);
 }

@@ -180,6 +180,33 @@ def test_row_deq_mm_T_of_several_rows(oracle, M, N, K, S, G, L, bias):
     assert int(hip._workspace(8 * M * N, dev).count_nonzero()) == 0
 
 
+def test_row_deq_mm_T_of_several_rows_with_values_that_are_not_finite(oracle):
+    """Infinite and NaN activations, an infinite coefficient and a weight beyond fp16 in the launch of several rows: every
+    output is finite, infinite or NaN as in the launch of that row by itself, and the finite ones agree."""
+    import sbvr
+    dev = torch.device("cuda:0")
+    M, N, K, S, G, L = 5, 8192, 790, 3, 128, 40
+    rng = np.random.default_rng(12)
+    bvr, idx, cache = _rand_enc(rng, K, N, S, G, L, oracle)
+    cache[7, 1] = np.inf
+    cache[9] = [60000, 40000, 50000]
+    x = (rng.standard_normal((M, K)) * 0.01).astype(np.float16)
+    x[0, 3], x[1, 789], x[2, 300], x[2, 301] = np.inf, -np.inf, np.nan, np.inf
+    idx[:, 3] = idx[:, 300:302] = 0
+    idx[:, 5:] = np.where(np.isin(idx[:, 5:], (7, 9)) & (rng.random(idx[:, 5:].shape) < 0.98), 1, idx[:, 5:])
+    args = [torch.from_numpy(a).to(dev) for a in (bvr, idx, cache)]
+    none = torch.zeros(0, dtype=torch.float16, device=dev)
+    y = sbvr._sbvr_row_deq_mm_T(torch.from_numpy(x).to(dev), *args, none, 0, bvr_len=G).float().cpu().numpy()
+    one = np.concatenate([sbvr._sbvr_row_deq_mm_T(torch.from_numpy(x[m:m + 1]).to(dev), *args, none, 0, bvr_len=G).float().cpu().numpy()
+                          for m in range(M)])
+    assert np.array_equal(np.isnan(y), np.isnan(one)) and np.array_equal(np.isposinf(y), np.isposinf(one))
+    assert np.array_equal(np.isneginf(y), np.isneginf(one))
+    finite = np.isfinite(one)
+    assert 0 < finite.sum() < finite.size
+    scale = np.sqrt(np.mean(one[finite].astype(np.float64) ** 2))
+    assert (np.abs(y[finite] - one[finite]) <= 2.0 ** -9 * np.maximum(np.abs(one[finite]), scale)).all()
+
+
 def test_row_deq_mm_T_without_workspace_and_repeatable(oracle):
     """The reference-shaped entry point (no workspace: K is never split across workgroups) against the oracle at a
     shape the binding would split, and the split form twice: the fixed-point accumulators make it repeatable."""
