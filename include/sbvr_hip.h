@@ -262,7 +262,10 @@ int sbvr_hip_row_deq_mm_T(const void *x, const uint32_t *r_bvr, const void *r_co
  * never split, e.g. any prefill-sized M).  With 4 planes, K a multiple of 128 and groups of 64 columns and more the
  * plane sums run on the matrix cores, and where the columns alone would leave CUs idle (N = 4096
  * on an MI355X) the parts of K are summed through the accumulators, in fixed point, so the result
- * does not depend on their order.  workspace NULL: as sbvr_hip_row_deq_mm_T.  The reference's
+ * does not depend on their order.  Several rows with 2 to 4 planes (every weight decoded once, as two fp16 values) are
+ * split the same way; there a partial sum that fixed point cannot hold (not finite, or beyond +-130000) has its
+ * output added up again in 64 bits, the selected coefficients alone.  One row keeps the range of the decode kernel's split
+ * (see sbvr_hip_linear_f16).  workspace NULL: as sbvr_hip_row_deq_mm_T.  The reference's
  * operator has no such argument (sbvr_ops.cpp:79-120); its bindings here bring their own.
  */
 int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r_coeff_idx,
@@ -270,6 +273,14 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
                              void *out, int M, int N, int K, int S, int G, int L,
                              void *workspace, size_t workspace_bytes, void *stream);
 size_t sbvr_hip_row_deq_mm_T_workspace(int M, int N);
+
+/* Which kernel the last of these calls on this thread launched (0 before the first), and its parts of K across workgroups. */
+#define SBVR_HIP_ROW_DEQ_PORTABLE 1      /* one thread per output */
+#define SBVR_HIP_ROW_DEQ_LANES 2         /* lanes along K */
+#define SBVR_HIP_ROW_DEQ_MFMA 3          /* row by row, plane sums on the matrix cores */
+#define SBVR_HIP_ROW_DEQ_ROWS 4          /* several rows, every weight decoded once */
+int sbvr_hip_row_deq_last_kernel(void);
+int sbvr_hip_row_deq_last_parts(void);
 
 /*
  * Both operands SBVR-encoded (default uint32 layout on both sides):

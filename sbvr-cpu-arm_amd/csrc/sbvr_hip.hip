@@ -65,6 +65,8 @@ namespace {
 thread_local char g_err[256] = "";
 thread_local int g_last_kernel = 0;       // SBVR_HIP_KERNEL_* of the last linear launched from this thread
 thread_local int g_last_rounding = 0;     // SBVR_HIP_ROUNDING_* of that launch
+thread_local int g_row_deq_kernel = 0;    // SBVR_HIP_ROW_DEQ_* of this thread's last transposed product
+thread_local int g_row_deq_parts = 0;     // and its parts of K across workgroups
 
 int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 int fail(int code, const char *fmt, ...)
@@ -140,7 +142,7 @@ constexpr float kLastTermScale = 256.f;  // third fp8 term of an activation hold
 // workgroup comes first.  The adder that finds count == ksplit-1 owns the total.
 constexpr int kAccFracBits = 30;
 constexpr long long kAccBias = 1ll << 47;
-constexpr float kAccClamp = 130000.f;    // |partial| beyond this becomes +-inf in fp16 anyway
+constexpr float kAccClamp = 130000.f;    // (a partial beyond this is twice the fp16 range off; add_part() marks it)
 constexpr int kMaxKsplit = 255;
 
 struct GemvArgs {
@@ -311,6 +313,31 @@ __device__ __forceinline__ long long to_fixed(float y)
     const float hi = __builtin_rintf(y * static_cast<float>(1 << (kAccFracBits - 24)));
     const float lo = fmaf(hi, -16777216.f, y * static_cast<float>(1 << kAccFracBits));
     return (static_cast<long long>(static_cast<int>(hi)) << 24) + static_cast<long long>(static_cast<int>(lo));
+}
+
+// The same for launches that also take partial sums the fixed point cannot hold (not finite, or beyond kAccClamp, where
+// parts may still cancel): such an adder marks the word before it counts itself, which the count in 7 bits (at most
+// kMaxMarkedKsplit parts) leaves room for, and the one that completes the count adds the output up again from its
+// operands.  Returns whether the calling lane completed it: `total` then is the sum, or `marked` is set.  (An atomic more for
+// the marked alone: 3 rows x 4096, K 4096 and 24 x 1304, K 19200, 8 planes as fast as without.)
+constexpr unsigned long long kAccMark = 1ull << 63;
+constexpr int kMaxMarkedKsplit = 127;
+
+__device__ __forceinline__ bool add_part(unsigned long long *word, int ksplit, float &total, bool &marked)
+{
+    if (!(fabsf(total) <= kAccClamp))       // (NaN as well)
+        __hip_atomic_fetch_or(word, kAccMark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned long long tot = (1ull << 56) + static_cast<unsigned long long>(to_fixed(total) + kAccBias);
+    tot += __hip_atomic_fetch_add(word, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((static_cast<int>(tot >> 56) & 0x7f) != ksplit)
+        return false;
+    marked = (tot & kAccMark) != 0;
+    const long long sum = static_cast<long long>(tot & ((1ull << 56) - 1)) - (static_cast<long long>(ksplit) << 47);
+    const float hi = static_cast<float>(static_cast<int>(sum >> 24));
+    const float lo = static_cast<float>(static_cast<int>(sum & 0xffffff));
+    total = fmaf(hi, 1.f / (1 << (kAccFracBits - 24)), lo * (1.f / (1 << kAccFracBits)));
+    __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
 }
 
 // S planes, MT row tiles (4 batch rows each), CT column tiles of 16 columns,
@@ -2815,6 +2842,24 @@ __device__ __forceinline__ void build_split_tables(const uint32_t (&c)[(S + 1) /
 
 typedef v4u __attribute__((aligned(2))) v4u_half_aligned;
 
+// sum + the share of row k of the weight in output (m, column j of word nw), as in the one-row kernels: the selected
+// coefficients alone, products in fp32 (exact there).
+template <int S, typename Sum>
+__device__ __forceinline__ Sum row_deq_add(const RowDeqArgs &a, int nw, int j, int k, int m, Sum sum)
+{
+    const size_t at = (static_cast<size_t>((nw * 32) / a.G) * a.K + static_cast<size_t>(k)) << a.idx16;
+    const uint8_t *ib = static_cast<const uint8_t *>(a.idx);
+    const int line = min(a.idx16 ? ib[at] | (ib[at + 1] << 8) : ib[at], a.L - 1);
+    const uint32_t *w = a.bvr + (static_cast<size_t>(nw) * a.K + static_cast<size_t>(k)) * S;
+    const float x = h2f(a.x[static_cast<size_t>(m) * a.K + k]);
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+        const float z = x * h2f(a.cache[static_cast<size_t>(line) * S + q]);
+        sum += static_cast<Sum>((w[q] >> j) & 1u ? z : 0.f);
+    }
+    return sum;
+}
+
 template <int S>
 __global__ void __launch_bounds__(64 * kDeqRowsWaves)
 __attribute__((amdgpu_waves_per_eu(3, 8)))
@@ -2945,22 +2990,10 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
         for (int r = 0; r < 16; ++r)
             acc_head[r] = acc_rest[r] = 0.f;
         for (int t = t_begin + wave; t < t_end; t += waves)
-            for (int k = 128 * t; k < min(K, 128 * t + 128); ++k) {
-                const size_t at = (ibase + static_cast<size_t>(k)) << a.idx16;
-                const uint8_t *ib = static_cast<const uint8_t *>(a.idx);
-                const int line = min(a.idx16 ? ib[at] | (ib[at + 1] << 8) : ib[at], a.L - 1);
+            for (int k = 128 * t; k < min(K, 128 * t + 128); ++k)
 #pragma unroll
-                for (int q = 0; q < S; ++q) {
-                    const bool set = (words[static_cast<size_t>(k) * S + q] >> j) & 1u;
-                    const float cq = h2f(a.cache[static_cast<size_t>(line) * S + q]);
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int m = min(m0 + 8 * (r >> 2) + 4 * h + (r & 3), M - 1);
-                        const float z = h2f(a.x[static_cast<size_t>(m) * K + k]) * cq;
-                        acc_head[r] += set ? z : 0.f;
-                    }
-                }
-            }
+                for (int r = 0; r < 16; ++r)
+                    acc_head[r] = row_deq_add<S>(a, nw, j, k, min(m0 + 8 * (r >> 2) + 4 * h + (r & 3), M - 1), acc_head[r]);
     }
     // ---- partial results meet in LDS; D[i][jj] sits in lane jj + 32*((i/4)%2), register (i%4) + 4*(i/8)
     __syncthreads();                        // (over the tiles)
@@ -2979,15 +3012,15 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
             continue;
         const size_t at = static_cast<size_t>(m) * N + n;
         if (a.ksplit > 1) {
-            unsigned long long tot = (1ull << 56) + static_cast<unsigned long long>(to_fixed(total) + kAccBias);
-            tot += __hip_atomic_fetch_add(a.acc + at, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (static_cast<int>(tot >> 56) != a.ksplit)
+            bool marked = false;
+            if (!add_part(a.acc + at, a.ksplit, total, marked))
                 continue;
-            const long long sum = static_cast<long long>(tot & ((1ull << 56) - 1)) - (static_cast<long long>(a.ksplit) << 47);
-            const float hi = static_cast<float>(static_cast<int>(sum >> 24));
-            const float lo = static_cast<float>(static_cast<int>(sum & 0xffffff));
-            total = fmaf(hi, 1.f / (1 << (kAccFracBits - 24)), lo * (1.f / (1 << kAccFracBits)));
-            __hip_atomic_store(a.acc + at, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (marked) {
+                double sum = 0.;                              // (one lane adds up all of K: in 64 bits, or rounding would show)
+                for (int k = 0; k < K; ++k)
+                    sum = row_deq_add<S>(a, nw, j, k, m, sum);
+                total = static_cast<float>(sum);
+            }
         }
         a.out[at] = f2h(a.bias ? total + h2f(a.bias[n]) : total);
     }
@@ -4373,6 +4406,8 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
         const hipError_t e = S == 4 ? launch_row_deq_rows<4>(a, waves, st) : (S == 3 ? launch_row_deq_rows<3>(a, waves, st) : launch_row_deq_rows<2>(a, waves, st));
         if (e != hipSuccess)
             return fail(SBVR_HIP_ELAUNCH, "row_deq launch: %s", hipGetErrorString(e));
+        g_row_deq_kernel = SBVR_HIP_ROW_DEQ_ROWS;
+        g_row_deq_parts = a.ksplit;
         return SBVR_HIP_OK;
     }
     if (M <= 65535 && S == 4 && K % kSub == 0 && G % 64 == 0 && tables_aligned && reinterpret_cast<uintptr_t>(x) % 4 == 0 &&
@@ -4409,6 +4444,8 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess)
             return fail(SBVR_HIP_ELAUNCH, "row_deq launch: %s", hipGetErrorString(e));
+        g_row_deq_kernel = SBVR_HIP_ROW_DEQ_MFMA;
+        g_row_deq_parts = ksplit;
         return SBVR_HIP_OK;
     }
     if (M <= 65535 && (S == 2 || S == 3 || S == 4 || S == 6 || S == 8) && tables_aligned) {
@@ -4430,6 +4467,8 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess)
             return fail(SBVR_HIP_ELAUNCH, "row_deq launch: %s", hipGetErrorString(e));
+        g_row_deq_kernel = SBVR_HIP_ROW_DEQ_LANES;
+        g_row_deq_parts = 1;
         return SBVR_HIP_OK;
     }
     const size_t total = static_cast<size_t>(M) * N;
@@ -4445,6 +4484,8 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return fail(SBVR_HIP_ELAUNCH, "row_deq launch: %s", hipGetErrorString(e));
+    g_row_deq_kernel = SBVR_HIP_ROW_DEQ_PORTABLE;
+    g_row_deq_parts = 1;
     return SBVR_HIP_OK;
 }
 
@@ -4455,6 +4496,10 @@ int sbvr_hip_row_deq_mm_T(const void *x, const uint32_t *r_bvr, const void *r_co
 {
     return sbvr_hip_row_deq_mm_T_ws(x, r_bvr, r_coeff_idx, idx_bytes, r_coeff_cache, bias, out, M, N, K, S, G, L, nullptr, 0, stream);
 }
+
+int sbvr_hip_row_deq_last_kernel(void) { return g_row_deq_kernel; }
+
+int sbvr_hip_row_deq_last_parts(void) { return g_row_deq_parts; }
 
 // (the launch splits K only while its column workgroups cover less than three quarters of the CUs: the predicate
 // of sbvr_hip_row_deq_mm_T_ws; a prefill-sized call needs nothing)

@@ -57,6 +57,8 @@ def _load():
     lib.sbvr_hip_last_error.restype = ctypes.c_char_p
     lib.sbvr_hip_last_kernel.restype = i
     lib.sbvr_hip_last_rounding.restype = i
+    lib.sbvr_hip_row_deq_last_kernel.restype = i
+    lib.sbvr_hip_row_deq_last_parts.restype = i
     lib.sbvr_hip_init.argtypes = [i]
     lib.sbvr_hip_linear_f16_workspace.restype = sz
     lib.sbvr_hip_linear_f16_workspace.argtypes = [i, i, i, i, i]
@@ -163,6 +165,15 @@ def last_rounding():
     ROUNDING_DECODE (each weight rounded to fp16 once, as the reference's decode() does) or ROUNDING_PLANEWISE
     (an fp16 sum built plane by plane)."""
     return _load().sbvr_hip_last_rounding()
+
+
+ROW_DEQ_PORTABLE, ROW_DEQ_LANES, ROW_DEQ_MFMA, ROW_DEQ_ROWS = 1, 2, 3, 4
+
+
+def row_deq_last():
+    """Which kernel the last transposed product of this thread launched (one of the ROW_DEQ_* codes), and in how many
+    parts of K across workgroups."""
+    return _load().sbvr_hip_row_deq_last_kernel(), _load().sbvr_hip_row_deq_last_parts()
 
 
 def _sbvr_hip_init(device=None):

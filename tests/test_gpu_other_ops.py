@@ -207,6 +207,70 @@ def test_row_deq_mm_T_of_several_rows_with_values_that_are_not_finite(oracle):
     assert (np.abs(y[finite] - one[finite]) <= 2.0 ** -9 * np.maximum(np.abs(one[finite]), scale)).all()
 
 
+def _transposed_sums(x, bvr, idx, cache, G):
+    """Per output the sum in 64 bits of the selected coefficients alone, and the largest magnitude its fp32 partial sums can
+    reach (of the finite terms)."""
+    bits = ((bvr[:, :, None, :] >> np.arange(32, dtype=np.uint32)[None, None, :, None]) & 1).astype(bool)   # (N/32, K, 32, S)
+    line = np.repeat(cache.astype(np.float64)[idx.astype(np.int64)], G // 32, axis=0)                      # (N/32, K, S)
+    out = np.zeros((x.shape[0], bvr.shape[0] * 32))
+    peak = np.zeros_like(out)
+    with np.errstate(invalid="ignore"):
+        for m in range(x.shape[0]):
+            z = np.where(bits, (x[m].astype(np.float64)[None, :, None] * line)[:, :, None, :], 0.0)
+            out[m] = z.sum(axis=(1, 3)).ravel()
+            peak[m] = np.where(np.isfinite(z), np.abs(z), 0.0).sum(axis=(1, 3)).ravel()
+    return out, peak
+
+
+def _same_class_and_close(y, want, peak):
+    """NaN, +inf and -inf where the sums in 64 bits have them (beyond fp16: infinite), finite values within 2 fp16 ulps
+    and the fp32 rounding inside parts that the accumulators hold (two of up to 130000; eight MFMAs a tile, four tiles and four waves
+    a part at most, 36 roundings and the last one's; an output with larger parts is summed in 64 bits)."""
+    want = np.where(np.abs(want) >= 65520.0, np.sign(want) * np.inf, want)
+    assert np.array_equal(np.isnan(y), np.isnan(want))
+    assert np.array_equal(np.isposinf(y), np.isposinf(want)) and np.array_equal(np.isneginf(y), np.isneginf(want))
+    finite = np.isfinite(want)
+    rms = np.sqrt(np.mean(want[finite] ** 2))
+    bound = 2.0 ** -9 * np.maximum(np.abs(want), min(rms, 10.0)) + 40 * 2.0 ** -24 * np.minimum(peak, 260000.0)
+    assert (np.abs(y[finite] - want[finite]) <= bound[finite]).all()
+    return finite
+
+
+@pytest.mark.parametrize("M,N,K,S,G,L", [(8, 2048, 4096, 4, 256, 256), (8, 512, 4143, 2, 256, 768), (7, 1024, 2100, 3, 32, 40)])
+def test_row_deq_mm_T_with_values_that_the_accumulators_cannot_hold(oracle, M, N, K, S, G, L):
+    """K in parts: NaN, infinities of one and of both signs in different parts, partial sums beyond the fixed point's range
+    that cancel and that do not, an infinite coefficient."""
+    import sbvr
+    from sbvr import hip
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(N + K)
+    bvr, idx, cache = _rand_enc(rng, K, N, S, G, L, oracle)
+    cache[7 % L] = [8] * S
+    cache[9 % L, S - 1] = np.inf
+    far = K - 30
+    idx[:] = np.where(np.isin(idx, (7 % L, 9 % L)), 1, idx)
+    idx[:, [5, far]] = 7 % L
+    bvr[:, far] = bvr[:, 5]
+    idx[:1, 77] = 9 % L                                        # (the first columns only)
+    x = (rng.standard_normal((M, K)) * 0.1).astype(np.float16)
+    x[:, [5, far]] = 0
+    x[1, 300] = np.nan
+    x[2, 400] = np.inf
+    x[3, 400], x[3, far - 1] = np.inf, -np.inf
+    x[4, 5], x[4, far] = 30000, -29000                         # up to 960000 in one part, 928000 back in the last
+    x[5, 5] = -60000
+    args = [torch.from_numpy(a).to(dev) for a in (bvr, idx, cache)]
+    none = torch.zeros(0, dtype=torch.float16, device=dev)
+    y = sbvr._sbvr_row_deq_mm_T(torch.from_numpy(x).to(dev), *args, none, 0, bvr_len=G)
+    kernel, parts = hip.row_deq_last()
+    assert kernel == hip.ROW_DEQ_ROWS and parts > 1
+    want, peak = _transposed_sums(x, bvr, idx, cache, G)
+    finite = _same_class_and_close(y.float().cpu().numpy().astype(np.float64), want, peak)
+    assert finite[0, -32:].all() and finite[4, -32:].all() and not finite[1:4].all(axis=1).any()
+    assert np.abs(np.where(finite[4], peak[4], 0)).max() > 4 * 130000
+    assert int(hip._workspace(8 * M * N, dev).count_nonzero()) == 0
+
+
 def test_row_deq_mm_T_without_workspace_and_repeatable(oracle):
     """The reference-shaped entry point (no workspace: K is never split across workgroups) against the oracle at a
     shape the binding would split, and the split form twice: the fixed-point accumulators make it repeatable."""
