@@ -46,6 +46,7 @@ const char *sbvr_hip_last_error(void);
 #define SBVR_HIP_KERNEL_PREFILL 4        /* M > 32: weights decoded to fp16 in registers, output tiles of up to 256 rows */
 #define SBVR_HIP_KERNEL_PREFILL_SPLIT 5  /* the same with K split across workgroups (workspace given) */
 int sbvr_hip_last_kernel(void);
+int sbvr_hip_last_parts(void);           /* parts of K across workgroups of that launch (1: not split) */
 
 /* How that launch treated the weights (0 before the first):
  *   EXACT      coefficients applied to plane sums in fp32, no per-weight rounding (decode and portable kernels);
@@ -129,10 +130,11 @@ size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G);
  * flags: bit 0 forces the portable kernel; bit 1 keeps the 32-row kernel out
  * (5..16 rows then take the decode kernel, exact in weights and activations,
  * 17..32 the prefill kernel).
- * Range: where the decode kernel splits K across workgroups, a workgroup's
- * partial sum is clamped to +-130000 before it is added up in fixed point;
- * partial sums beyond twice the fp16 range that would cancel to a finite total
- * come out as a wrong finite value instead.
+ * Range: where the decode kernel splits K across workgroups (groups of 128 and
+ * more), a workgroup's partial sum is clamped to +-130000, NaN to -130000, before
+ * it is added up in fixed point; partial sums beyond twice the fp16 range that
+ * would cancel to a finite total come out as a wrong finite value instead.  Groups of 64 have such outputs added up again
+ * as the portable kernel does, from the selected activations alone.
  */
 int sbvr_hip_linear_f16(const void *x, const uint32_t *bvr, const void *coeff_idx,
                         int idx_bytes, const void *coeff_cache, const void *bias,

@@ -64,6 +64,7 @@ namespace {
 
 thread_local char g_err[256] = "";
 thread_local int g_last_kernel = 0;       // SBVR_HIP_KERNEL_* of the last linear launched from this thread
+thread_local int g_last_parts = 0;        // and its parts of K across workgroups
 thread_local int g_last_rounding = 0;     // SBVR_HIP_ROUNDING_* of that launch
 thread_local int g_row_deq_kernel = 0;    // SBVR_HIP_ROW_DEQ_* of this thread's last transposed product
 thread_local int g_row_deq_parts = 0;     // and its parts of K across workgroups
@@ -89,23 +90,16 @@ std::mutex g_dev_lock;           // guards g_dev[] and the scratch addresses: fi
 
 // ---------------------------------------------------- portable kernel (any shape)
 
-// One thread per output element.  Slow; used for shapes the MFMA kernel does
-// not take and as a second implementation to test against.
+// The sum of one output in fp32: selected activations added up plane by plane, then the coefficients applied.  A line index
+// beyond `last_line` counts as that one.
 template <typename IdxT>
-__global__ void __launch_bounds__(256)
-sbvr_linear_portable_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ bvr,
-                            const void *__restrict__ idx, const uint16_t *__restrict__ cache,
-                            const uint16_t *__restrict__ bias, uint16_t *__restrict__ out,
-                            int M, int N, int K, int S, int G)
+__device__ __forceinline__ float linear_output(const uint16_t *__restrict__ x, const uint32_t *__restrict__ bvr, const void *__restrict__ idx,
+                                               const uint16_t *__restrict__ cache, int m, int n, int N, int K, int S, int G, int last_line)
 {
-    const size_t o = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (o >= static_cast<size_t>(M) * N)
-        return;
-    const int m = static_cast<int>(o / N), n = static_cast<int>(o % N);
     const int wpg = G / 32;
     float acc = 0.f;
     for (int g = 0; g < K / G; ++g) {
-        const int line = load_idx<IdxT>(idx, static_cast<size_t>(g) * N + n);
+        const int line = min(load_idx<IdxT>(idx, static_cast<size_t>(g) * N + n), last_line);
         for (int j = 0; j < S; ++j) {
             float ps = 0.f;
             for (int w = 0; w < wpg; ++w) {
@@ -121,7 +115,23 @@ sbvr_linear_portable_kernel(const uint16_t *__restrict__ x, const uint32_t *__re
             acc = fmaf(h2f(cache[static_cast<size_t>(line) * S + j]), ps, acc);
         }
     }
-    uint16_t r = f2h(acc);
+    return acc;
+}
+
+// One thread per output element.  Slow; used for shapes the MFMA kernel does
+// not take and as a second implementation to test against.
+template <typename IdxT>
+__global__ void __launch_bounds__(256)
+sbvr_linear_portable_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ bvr,
+                            const void *__restrict__ idx, const uint16_t *__restrict__ cache,
+                            const uint16_t *__restrict__ bias, uint16_t *__restrict__ out,
+                            int M, int N, int K, int S, int G)
+{
+    const size_t o = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (o >= static_cast<size_t>(M) * N)
+        return;
+    const int m = static_cast<int>(o / N), n = static_cast<int>(o % N);
+    uint16_t r = f2h(linear_output<IdxT>(x, bvr, idx, cache, m, n, N, K, S, G, 0x7fffffff));
     if (bias)
         r = hadd(r, bias[n]);
     out[o] = r;
@@ -266,7 +276,8 @@ constexpr int kXFloor = 4;      // measurement aid: the launch's plane-word and 
 //           sum_k a_r L_r[k] R_j[k] = a_r * popcount(L_r & R_j) per sub-group, and the rows are added up at the end.
 constexpr int kXPlanes = 5;
 // kXHalves: groups of 64.  A batch row takes two rows of the A operands, one for each half of the sub-group with zeros in the
-//           other, so every operand row meets one coefficient line; the two are added up at the end.  Up to 4 batch rows
+//           other, so every operand row meets one coefficient line; the two are added up at the end.  Outputs that are not
+//           finite that way are summed again as the portable kernel does, from the selected activations alone.  Up to 4 batch rows
 //           (5 rows on: the 32-row kernels).  One thread per output, which took them before, 4096 -> 14336, 4 planes,
 //           one row: 1067 us; here 7.3.  (12800 -> 731, 6 planes, one row 4911 and 5.4; 8192 -> 28672, 2 rows 2219 and 30.)
 constexpr int kXHalves = 6;
@@ -630,6 +641,8 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
                         const int e = 20 - eh;
                         if (blk == r)            // products come out as 2 * x * 2^e
                             scale[sgi][mt] = __uint_as_float(static_cast<uint32_t>(126 - e) << 23);
+                        if (XM == kXHalves && blk == r && amax >= 0x7c00u)     // not finite, which fp8 terms cannot tell: NaN, see the end
+                            scale[sgi][mt] = NAN;
                         // the lane's two elements, from the dwords (2l, 2l + 1) the lanes of its quad loaded
                         const int va = __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x50, 0xF, 0xF, true);   // quad_perm 0,0,1,1
                         const int vb = __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xFA, 0xF, 0xF, true);   // quad_perm 2,2,3,3
@@ -798,7 +811,15 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
         const int n = n_base + ct * 16 + col, m = XM == kXHalves ? mt * 2 + (blk >> 1) : mt * 4 + blk;
         const bool valid = (XM == kXPlanes ? m == 0 : m < a.M && (XM != kXHalves || (blk & 1) == 0)) && (!shifted || n >= n_own) && n < n_own + a.wstride;
         const size_t at = static_cast<size_t>(m) * N + n;
-        if (a.ksplit > 1) {
+        if constexpr (XM == kXHalves) {
+            // activations or coefficients that are not finite, or parts the accumulators cannot hold: as the portable kernel sums
+            bool again = !(fabsf(total) < INFINITY);
+            if (!valid || (a.ksplit > 1 && !add_part(a.acc + at, a.ksplit, total, again)))
+                continue;
+            if (again)
+                total = a.idx16 ? linear_output<uint16_t>(a.x, a.bvr, a.idx, a.cache, m, n, N, K, S, kSub / 2, a.L - 1)
+                                : linear_output<uint8_t>(a.x, a.bvr, a.idx, a.cache, m, n, N, K, S, kSub / 2, a.L - 1);
+        } else if (a.ksplit > 1) {
             // through the accumulators: the adder that completes the count converts
             unsigned long long tot = (1ull << 56) + static_cast<unsigned long long>(to_fixed(total) + kAccBias);
             unsigned long long old = 0ull;
@@ -3957,6 +3978,8 @@ const char *sbvr_hip_last_error(void) { return g_err; }
 
 int sbvr_hip_last_kernel(void) { return g_last_kernel; }
 
+int sbvr_hip_last_parts(void) { return g_last_parts; }
+
 int sbvr_hip_last_rounding(void) { return g_last_rounding; }
 
 int sbvr_hip_init(int device)
@@ -4079,6 +4102,7 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         if (e != hipSuccess)
             return fail(SBVR_HIP_ELAUNCH, "rows32 (table look-up) launch: %s", hipGetErrorString(e));
         g_last_kernel = SBVR_HIP_KERNEL_ROWS32;
+        g_last_parts = r.ksplit;
         // (6 and 8 planes: table entries added, closer than plane by plane.  5 to 8 rows: as decode() rounds, reported as the
         // looser of the two, which is what such a call has always said)
         g_last_rounding = S <= 4 && M >= kLutMinRows ? SBVR_HIP_ROUNDING_DECODE : SBVR_HIP_ROUNDING_PLANEWISE;
@@ -4099,6 +4123,7 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         if (e != hipSuccess)
             return fail(SBVR_HIP_ELAUNCH, "rows32 launch: %s", hipGetErrorString(e));
         g_last_kernel = SBVR_HIP_KERNEL_ROWS32;
+        g_last_parts = 1;
         g_last_rounding = SBVR_HIP_ROUNDING_PLANEWISE;
         return SBVR_HIP_OK;
     }
@@ -4136,6 +4161,7 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
             if (e != hipSuccess)
                 return fail(SBVR_HIP_ELAUNCH, "batch launch (MT=%d CTW=%d SP=%d waves=%d ksplit=%d): %s", p.MT, p.CTW, p.SP, p.waves, p.ksplit, hipGetErrorString(e));
             g_last_kernel = SBVR_HIP_KERNEL_DECODE;
+            g_last_parts = p.ksplit;
             g_last_rounding = SBVR_HIP_ROUNDING_EXACT;
             return SBVR_HIP_OK;
         }
@@ -4187,17 +4213,19 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         if (e != hipSuccess)
             return fail(SBVR_HIP_ELAUNCH, "gemv launch (CT=%d SP=%d MT=%d waves=%d ksplit=%d): %s", p.CT, p.SP, p.MT, p.waves, p.ksplit, hipGetErrorString(e));
         g_last_kernel = SBVR_HIP_KERNEL_DECODE;
+        g_last_parts = p.ksplit;
         g_last_rounding = SBVR_HIP_ROUNDING_EXACT;
         return SBVR_HIP_OK;
         }
     }
 
-    // Groups of 64, up to 4 rows.  (Where that launch splits K and there is no workspace for it: the portable kernel)
+    // Groups of 64, up to 4 rows.  (Where that launch splits K and there is no workspace for it, or in more parts than the
+    // accumulators can mark: the portable kernel)
     if (pro.mode == kXPlain && !(flags & 1) && aligned && halves_path_ok(M, N, K, S, G)) {
         const GemvPlan p = plan_gemv(2 * M, N, K, S, current_cus());
         const bool room = workspace && workspace_bytes >= static_cast<size_t>(M) * N * sizeof(unsigned long long) &&
                           reinterpret_cast<uintptr_t>(workspace) % 8 == 0;
-        if (p.CT > 0 && (p.ksplit == 1 || room)) {
+        if (p.CT > 0 && (p.ksplit == 1 || (room && p.ksplit <= kMaxMarkedKsplit))) {
             GemvArgs a{};
             a.x = static_cast<const uint16_t *>(x);
             a.bvr = bvr;
@@ -4215,6 +4243,7 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
             if (e != hipSuccess)
                 return fail(SBVR_HIP_ELAUNCH, "gemv launch, groups of 64 (CT=%d SP=%d MT=%d waves=%d ksplit=%d): %s", p.CT, p.SP, p.MT, p.waves, p.ksplit, hipGetErrorString(e));
             g_last_kernel = SBVR_HIP_KERNEL_DECODE;
+            g_last_parts = p.ksplit;
             g_last_rounding = SBVR_HIP_ROUNDING_EXACT;
             return SBVR_HIP_OK;
         }
@@ -4260,6 +4289,7 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         if (e != hipSuccess)
             return fail(SBVR_HIP_ELAUNCH, "prefill (table look-up) launch: %s", hipGetErrorString(e));
         g_last_kernel = g.ksplit > 1 ? SBVR_HIP_KERNEL_PREFILL_SPLIT : SBVR_HIP_KERNEL_PREFILL;
+        g_last_parts = g.ksplit;
         // (6 and 8 planes: two entries added, closer than plane by plane.  Groups of 64: as decode() rounds, reported as the
         // looser of the two, which is what such a call has always said)
         g_last_rounding = S <= 4 && g.steps_per_group % 2 == 0 ? SBVR_HIP_ROUNDING_DECODE : SBVR_HIP_ROUNDING_PLANEWISE;
@@ -4279,6 +4309,7 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
     if (e != hipSuccess)
         return fail(SBVR_HIP_ELAUNCH, "portable launch: %s", hipGetErrorString(e));
     g_last_kernel = SBVR_HIP_KERNEL_PORTABLE;
+    g_last_parts = 1;
     g_last_rounding = SBVR_HIP_ROUNDING_EXACT;
     return SBVR_HIP_OK;
 }
@@ -4585,6 +4616,7 @@ int sbvr_hip_mm_T_ws(const uint32_t *l_bvr, const void *l_coeff_idx, int l_idx_b
                 return fail(SBVR_HIP_ELAUNCH, "mm_T launch through the decode kernel (CT=%d SP=%d waves=%d ksplit=%d): %s", p.CT, p.SP, p.waves,
                             p.ksplit, hipGetErrorString(e));
             g_last_kernel = SBVR_HIP_KERNEL_DECODE;
+            g_last_parts = p.ksplit;
             return SBVR_HIP_OK;
         }
     }
@@ -4715,6 +4747,7 @@ int sbvr_hip_dec_attention_o_f16(const void *qkv, const float *cos_table, const 
     if (e != hipSuccess)
         return fail(SBVR_HIP_ELAUNCH, "attention + projection launch: %s", hipGetErrorString(e));
     g_last_kernel = SBVR_HIP_KERNEL_DECODE;
+    g_last_parts = kv_heads;
     g_last_rounding = SBVR_HIP_ROUNDING_EXACT;
     return SBVR_HIP_OK;
 }
@@ -4786,6 +4819,7 @@ int sbvr_hip_dec_rows_linear_f16(int prologue, const void *x, const void *delta,
     if (e != hipSuccess)
         return fail(SBVR_HIP_ELAUNCH, "rows of a prompt (prologue %d): %s", prologue, hipGetErrorString(e));
     g_last_kernel = SBVR_HIP_KERNEL_DECODE;
+    g_last_parts = p.ksplit;
     g_last_rounding = SBVR_HIP_ROUNDING_EXACT;
     return SBVR_HIP_OK;
 }

@@ -56,6 +56,7 @@ def _load():
     lib.sbvr_hip_version.restype = i
     lib.sbvr_hip_last_error.restype = ctypes.c_char_p
     lib.sbvr_hip_last_kernel.restype = i
+    lib.sbvr_hip_last_parts.restype = i
     lib.sbvr_hip_last_rounding.restype = i
     lib.sbvr_hip_row_deq_last_kernel.restype = i
     lib.sbvr_hip_row_deq_last_parts.restype = i
@@ -155,6 +156,11 @@ KERNEL_PORTABLE, KERNEL_DECODE, KERNEL_ROWS32, KERNEL_PREFILL, KERNEL_PREFILL_SP
 def last_kernel():
     """Which kernel the last linear call of this thread launched (one of the KERNEL_* codes)."""
     return _load().sbvr_hip_last_kernel()
+
+
+def last_parts():
+    """In how many parts of K across workgroups that call ran."""
+    return _load().sbvr_hip_last_parts()
 
 
 ROUNDING_EXACT, ROUNDING_DECODE, ROUNDING_PLANEWISE = 1, 2, 3

@@ -358,3 +358,43 @@ def test_groups_of_64_up_to_4_rows(oracle, N, K, S, M, L, bias):
     want = sbvr._sbvr_linear_f16(x, *ops, None, bvr_len=64, flags=1)
     # (both exact in weights and activations: the order of the fp32 sums and one rounding)
     check(y, want.float().cpu().numpy().astype(np.float64), "against the portable kernel")
+
+
+@pytest.mark.parametrize("N,K,S,M,parts", [(731, 12800, 4, 4, True), (1000, 1280, 6, 3, True), (4099, 4096, 3, 2, False), (4096, 4096, 8, 4, False)])
+def test_groups_of_64_with_values_that_sums_cannot_hold(N, K, S, M, parts):
+    """Groups of 64 on the decode kernel, K in parts and not: NaN, infinite activations (which the fp8 terms cannot tell), an
+    infinite coefficient, and parts beyond the accumulators' range that cancel: NaN, infinite or finite as with one thread per
+    output, the finite ones as close as fp32 sums of terms that large are."""
+    import sbvr
+    from sbvr import hip, synth
+    dev = _dev()
+    bvr, idx, cache = synth.random_encoding(N, K, S, 64, 256, seed=N)
+    far = K - 64 + 5
+    cache[7], cache[9] = torch.tensor(8.0), torch.tensor(float("inf"))
+    idx[(idx == 7) | (idx == 9)] = 1
+    idx[0] = idx[-1] = 7
+    idx[2, :40] = 9
+    bvr.view(torch.int32)[far // 32] = bvr.view(torch.int32)[0]            # (element 5 of its word as element 5 of the first)
+    for special in range(4):
+        x = (torch.randn((M, K), generator=torch.Generator().manual_seed(special)) * 0.1).to(torch.float16)
+        x[:, :64] = x[:, -64:] = 0
+        if special == 0:
+            x[0, 300], x[M - 1, 100] = float("nan"), float("inf")
+        elif special == 1:
+            x[0, 70], x[0, K - 70], x[M - 1, 500] = float("inf"), float("-inf"), float("-inf")
+        elif special == 2:
+            x[0, 5], x[0, far], x[M - 1, 5] = 30000, -29000, -60000
+        ops = [t.to(dev) for t in (x, bvr, idx, cache)]
+        y = sbvr._sbvr_linear_f16(*ops, None, bvr_len=64)
+        assert hip.last_kernel() == DECODE and (hip.last_parts() > 1) == parts
+        ws = hip._workspaces[(dev.index or 0, torch.cuda.current_stream().cuda_stream)]
+        y, want = (t.float().cpu().numpy().astype(np.float64) for t in (y, sbvr._sbvr_linear_f16(*ops, None, bvr_len=64, flags=1)))
+        for same in (np.isnan, np.isposinf, np.isneginf):
+            assert np.array_equal(same(y), same(want)), special
+        finite = np.isfinite(want)
+        assert finite[:, 40:].any() and not (special < 2 and finite[0].all())
+        # (a partial sum rounds at most once per coefficient and group, at the size the two large terms have there)
+        large = 2.0 ** -24 * (K // 64 * S) * 2 * 8 * S * 30000 * (np.arange(M) == 0) * (special == 2)
+        rms = np.sqrt(np.mean(want[finite & (np.abs(want) < 100)] ** 2))
+        assert (np.abs(y[finite] - want[finite]) <= (2.0 ** -9 * np.maximum(np.abs(want), rms) + large[:, None])[finite]).all(), special
+        assert int(ws.count_nonzero()) == 0
