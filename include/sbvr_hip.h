@@ -134,7 +134,7 @@ size_t sbvr_hip_linear_f16_workspace(int M, int N, int K, int S, int G);
  * more), a workgroup's partial sum is clamped to +-130000, NaN to -130000, before
  * it is added up in fixed point; partial sums beyond twice the fp16 range that
  * would cancel to a finite total come out as a wrong finite value instead.  Groups of 64 have such outputs added up again
- * as the portable kernel does, from the selected activations alone.
+ * as the portable kernel does, from the selected activations alone, and the 32-row kernel over its fp16 weights in 64 bits.
  */
 int sbvr_hip_linear_f16(const void *x, const uint32_t *bvr, const void *coeff_idx,
                         int idx_bytes, const void *coeff_cache, const void *bias,

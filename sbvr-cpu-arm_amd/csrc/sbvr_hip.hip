@@ -1841,6 +1841,35 @@ constexpr int kLutWaves = 8;
 // 5..8 rows and 17.9-20.9 us at 9..16 rows for the decode kernels (13.6-16.0 with 2 planes, 19.6-22.5 with 3).
 constexpr int kLutMinRows = 9;
 
+// Output (m, n) over all of K by one lane, the weights as build_weight_tables leaves them; in 64 bits, where so long a sum
+// keeps what the parts' own sums would.
+template <int S>
+__device__ __forceinline__ float lut_output(const RowsArgs &a, int m, int n)
+{
+    constexpr int H = WeightTables<S>::H;
+    const uint16_t *const x = a.x + static_cast<size_t>(m) * a.K;
+    double sum = 0.;
+    for (int word = 0; word < a.K / 32; ++word) {
+        const size_t at = (static_cast<size_t>(word / a.words_per_group) * a.N + n) << a.idx16;
+        const uint8_t *ib = static_cast<const uint8_t *>(a.idx);
+        const int line = min(a.idx16 ? ib[at] | (ib[at + 1] << 8) : ib[at], a.L - 1);
+        const uint32_t *w = a.bvr + (static_cast<size_t>(word) * a.N + n) * S;
+        for (int b = 0; b < 32; ++b) {
+            _Float16 weight{};
+#pragma unroll
+            for (int first = 0; first < S; first += H) {
+                float entry = 0.f;
+#pragma unroll
+                for (int q = first; q < first + H && q < S; ++q)
+                    entry += (w[q] >> b) & 1u ? h2f(a.cache[static_cast<size_t>(line) * S + q]) : 0.f;
+                weight = first == 0 ? static_cast<_Float16>(entry) : weight + static_cast<_Float16>(entry);
+            }
+            sum += static_cast<double>(h2f(x[32 * word + b])) * static_cast<double>(weight);
+        }
+    }
+    return static_cast<float>(sum);
+}
+
 // kHalfRows: up to 16 batch rows (the activation loads of rows 16..31 are left out); kShare: groups of a multiple
 // of 128 elements, so the two steps of a loop iteration (an even word pair and the next) share a coefficient line:
 // one index load, one gather and one table per two steps.
@@ -1993,18 +2022,11 @@ sbvr_gemm_rows32_lut_kernel(const RowsArgs a)
         const bool valid = m < M && n < N;
         const size_t at = static_cast<size_t>(m) * N + n;
         if (a.ksplit > 1) {
-            unsigned long long tot = (1ull << 56) + static_cast<unsigned long long>(to_fixed(total) + kAccBias);
-            unsigned long long old = 0ull;
-            if (valid)
-                old = __hip_atomic_fetch_add(a.acc + at, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            tot += old;
-            if (!valid || static_cast<int>(tot >> 56) != a.ksplit)
+            bool marked = false;
+            if (!valid || !add_part(a.acc + at, a.ksplit, total, marked))
                 continue;
-            const long long sum = static_cast<long long>(tot & ((1ull << 56) - 1)) - (static_cast<long long>(a.ksplit) << 47);
-            const float hi = static_cast<float>(static_cast<int>(sum >> 24));
-            const float lo = static_cast<float>(static_cast<int>(sum & 0xffffff));
-            total = fmaf(hi, 1.f / (1 << (kAccFracBits - 24)), lo * (1.f / (1 << kAccFracBits)));
-            __hip_atomic_store(a.acc + at, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (marked)
+                total = lut_output<S>(a, m, n);
         } else if (!valid) {
             continue;
         }

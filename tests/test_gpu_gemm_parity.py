@@ -377,3 +377,51 @@ def test_prefill_kernel_for_17_to_32_rows(oracle, S, G):
 ])
 def test_rows32_table_look_up_of_more_planes_and_fewer_rows(oracle, M, N, K, S, G, L, bias):
     run_case(oracle, N, K, S, G, M, L, seed=M + N + S, bias=bias, expect=ROWS32)
+
+
+@pytest.mark.parametrize("M,N,K,S,G,L,parts", [(24, 1304, 19200, 8, 128, 256, True), (12, 512, 8192, 4, 64, 300, True),
+                                               (7, 200, 8192, 6, 64, 256, True), (32, 1000, 8192, 3, 256, 256, True),
+                                               (20, 9000, 1024, 8, 128, 256, False)])
+def test_rows32_with_values_that_sums_cannot_hold(M, N, K, S, G, L, parts):
+    """The table look-up form, K in parts and not: NaN, infinities of one and of both signs, an infinite coefficient, parts
+    beyond the accumulators' range that cancel.  Infinite, NaN and finite as in sums in 64 bits of x times the weights."""
+    import sbvr
+    from sbvr import hip, synth
+    dev = torch.device("cuda:0")
+    bvr, idx, cache = synth.random_encoding(N, K, S, G, L, seed=N)
+    far = K - G + 5
+    cache[7], cache[9] = torch.tensor(8.0), torch.tensor(float("inf"))
+    idx_int = idx.to(torch.int64)
+    idx_int[(idx_int == 7) | (idx_int == 9)] = 1
+    idx_int[0] = idx_int[-1] = 7
+    idx_int[1, :40] = 9
+    idx = idx_int.to(idx.dtype)
+    bvr.view(torch.int32)[far // 32] = bvr.view(torch.int32)[0]            # (element 5 of its word as element 5 of the first)
+    x = (torch.randn((M, K), generator=torch.Generator().manual_seed(M)) * 0.1).to(torch.float16)
+    x[:, :G] = x[:, -G:] = 0
+    x[0, 2 * G + 30], x[1, 2 * G + 100 % G], x[2, 3 * G], x[2, K - 2 * G] = float("nan"), float("inf"), float("inf"), float("-inf")
+    x[3, 5], x[3, far] = 30000, -29000                                     # up to 240000 * S in one part, nearly as much back in the last
+    x[4, 5] = -60000
+    y = sbvr._sbvr_linear_f16(*(t.to(dev) for t in (x, bvr, idx, cache)), None, bvr_len=G)
+    assert hip.last_kernel() == ROWS32 and (hip.last_parts() > 1) == parts
+    bits = (bvr.numpy()[:, None] >> np.arange(32, dtype=np.uint32)[None, :, None, None]) & 1        # (K/32, 32, N, S)
+    line = np.repeat(cache.numpy().astype(np.float64)[idx_int.numpy()], G, axis=0).reshape(K // 32, 32, N, S)
+    # (the kernel's fp16 weights: one that the rounding makes zero gives NaN beside an infinite activation)
+    entries = [np.where(bits != 0, line, 0.0)[..., q:q + (S if S <= 4 else 3)].sum(axis=3).astype(np.float16) for q in range(0, S, S if S <= 4 else 3)]
+    w = sum(entries[1:], entries[0]).astype(np.float64).reshape(K, N)
+    xd = x.numpy().astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = np.stack([(row[:, None] * w).sum(axis=0) for row in xd])
+        peak = np.abs(xd[:, 5:6] * w[5][None, :]) + np.abs(xd[:, far:far + 1] * w[far][None, :])
+    want = np.where(np.abs(want) >= 65520.0, np.sign(want) * np.inf, want)
+    y = y.float().cpu().numpy().astype(np.float64)
+    for same in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(same(y), same(want))
+    finite = np.isfinite(want)
+    assert finite[3:, 40:].any() and not finite[:3].any() and not finite[:, :40].all(axis=1).any()
+    # (weights rounded to fp16; the rounding of fp32 sums while a large term is in them: at most K / 16 MFMAs, eight waves' sums, one
+    # more for the total, unless the parts do not fit and the output is summed in 64 bits)
+    rms = np.sqrt(np.mean(want[4:, 40:][finite[4:, 40:]] ** 2))
+    bound = 3e-3 * rms + 2.0 ** -9 * np.abs(want) + (K // 16 + 9) * 2.0 ** -24 * (np.minimum(peak, 260000.0) if parts else peak)
+    assert (np.abs(y[finite] - want[finite]) <= bound[finite]).all()
+    assert int(hip._workspaces[(0, torch.cuda.current_stream().cuda_stream)].count_nonzero()) == 0
