@@ -275,6 +275,8 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
                              void *out, int M, int N, int K, int S, int G, int L,
                              void *workspace, size_t workspace_bytes, void *stream);
 size_t sbvr_hip_row_deq_mm_T_workspace(int M, int N);
+/* The same for one call's K, planes and groups: 0 where it is not split.  (N a multiple of 32, as the call wants it.) */
+size_t sbvr_hip_row_deq_mm_T_workspace_for(int M, int N, int K, int S, int G);
 
 /* Which kernel the last of these calls on this thread launched (0 before the first), and its parts of K across workgroups. */
 #define SBVR_HIP_ROW_DEQ_PORTABLE 1      /* one thread per output */

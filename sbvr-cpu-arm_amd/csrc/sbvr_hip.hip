@@ -3083,6 +3083,40 @@ bool row_deq_rows(int M, int N, int K, int S, int G, int cus)
     return !(M == 2 && S == 4 && K % kSub == 0 && G % 64 == 0 && (N / 32 + 1) / 2 * 2 >= cus);
 }
 
+// Parts of K where the caller brings the accumulators.  Several rows: as many as give the CUs two workgroups each, of 4 tiles and
+// more.
+int row_deq_rows_parts(int M, int N, int K, int cus)
+{
+    const int tiles = (K + 127) / 128;
+    const long wgs = static_cast<long>(N / 32) * ((M + 31) / 32);
+    int ksplit = 1;
+    while (ksplit < 32 && wgs * ksplit < 2L * cus && tiles >= 8 * ksplit)
+        ksplit *= 2;
+    const int per_part = (tiles + ksplit - 1) / ksplit;
+    return (tiles + per_part - 1) / per_part;                // (no empty parts)
+}
+
+bool row_deq_mfma_ok(int M, int K, int S, int G)
+{
+    return M <= 65535 && S == 4 && K % kSub == 0 && G % 64 == 0;
+}
+
+// The matrix-core launch row by row: while its column workgroups, two column words each, leave more than five eighths of the CUs
+// idle (measured at 4096 -> 4096 / 14336 -> 4096, 64 column workgroups: 13.2 / 39.0 us unsplit, 7.1 / 14.1 in 4
+// parts, 7.2 / 18.5 in 8; at 4096 -> 14336, 224 of them: 15.3 unsplit, 18.4 in 2).
+int row_deq_mfma_parts(int M, int N, int K, int cus)
+{
+    const int nsub = K / kSub;
+    const long col_wgs = static_cast<long>((N / 32 + 1) / 2) * M;
+    if (col_wgs * 2 >= 3L * cus / 4)
+        return 1;
+    int ksplit = 1;
+    while (ksplit < 32 && col_wgs * ksplit < 3L * cus / 4 && nsub / (ksplit * 2) >= 4)
+        ksplit *= 2;
+    const int per_part = (nsub + ksplit - 1) / ksplit;
+    return (nsub + per_part - 1) / per_part;
+}
+
 template <int S>
 hipError_t launch_row_deq_rows(const RowDeqArgs &a, int waves, hipStream_t st)
 {
@@ -4441,20 +4475,16 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
     if (idx_bytes == 1 && L > 256)
         return fail(SBVR_HIP_EINVAL, "uint8 indices cannot address L=%d lines", L);
     const bool tables_aligned = reinterpret_cast<uintptr_t>(r_bvr) % 16 == 0 && reinterpret_cast<uintptr_t>(r_coeff_cache) % 16 == 0;
+    const bool room = workspace && reinterpret_cast<uintptr_t>(workspace) % 8 == 0 &&
+                      workspace_bytes >= static_cast<size_t>(M) * N * sizeof(unsigned long long);
     if (row_deq_rows(M, N, K, S, G, current_cus()) && tables_aligned && (static_cast<long>(M) + 31) / 32 <= 65535 && !env_switches().rowdeq_lanes) {
-        // every weight decoded once for all rows; K in as many parts as give the CUs a workgroup each
+        // every weight decoded once for all rows
         const int tiles = (K + 127) / 128;
-        const long wgs = static_cast<long>(N / 32) * ((M + 31) / 32);
-        int ksplit = 1;
-        if (workspace && reinterpret_cast<uintptr_t>(workspace) % 8 == 0 &&
-            workspace_bytes >= static_cast<size_t>(M) * N * sizeof(unsigned long long))
-            while (ksplit < 32 && wgs * ksplit < 2L * current_cus() && tiles >= 8 * ksplit)
-                ksplit *= 2;
         RowDeqArgs a{static_cast<const uint16_t *>(x), r_bvr, r_coeff_idx, static_cast<const uint16_t *>(r_coeff_cache),
                      static_cast<const uint16_t *>(bias), static_cast<uint16_t *>(out), static_cast<unsigned long long *>(workspace),
                      M, N, K, L, G, idx_bytes == 2 ? 1 : 0, 1, 1};
-        a.per_part = (tiles + ksplit - 1) / ksplit;
-        a.ksplit = (tiles + a.per_part - 1) / a.per_part;       // (no empty parts)
+        a.ksplit = room ? row_deq_rows_parts(M, N, K, current_cus()) : 1;
+        a.per_part = (tiles + a.ksplit - 1) / a.ksplit;
         const int waves = a.per_part < kDeqRowsWaves ? a.per_part : kDeqRowsWaves;
         const hipError_t e = S == 4 ? launch_row_deq_rows<4>(a, waves, st) : (S == 3 ? launch_row_deq_rows<3>(a, waves, st) : launch_row_deq_rows<2>(a, waves, st));
         if (e != hipSuccess)
@@ -4463,25 +4493,15 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
         g_row_deq_parts = a.ksplit;
         return SBVR_HIP_OK;
     }
-    if (M <= 65535 && S == 4 && K % kSub == 0 && G % 64 == 0 && tables_aligned && reinterpret_cast<uintptr_t>(x) % 4 == 0 &&
+    if (row_deq_mfma_ok(M, K, S, G) && tables_aligned && reinterpret_cast<uintptr_t>(x) % 4 == 0 &&
         reinterpret_cast<uintptr_t>(r_coeff_idx) % 4 == 0 && !env_switches().rowdeq_lanes) {
         // plane sums on the matrix cores over bits transposed across lanes
         const int nsub = K / kSub;
         // (128 columns per workgroup, one A image for twice the columns, measured slower: 17.3 against 15.6 us at
         // 4096 -> 14336: it wants more than 128 registers)
         const int nww = 2;
-        const long col_wgs = static_cast<long>((N / 32 + nww - 1) / nww) * M;
-        // K in as many parts as give the CUs a workgroup each, if the caller brought the accumulators
-        int ksplit = 1;
-        if (workspace && reinterpret_cast<uintptr_t>(workspace) % 8 == 0 &&
-            workspace_bytes >= static_cast<size_t>(M) * N * sizeof(unsigned long long)) {
-            // (measured at 4096 -> 4096 / 14336 -> 4096, 64 column workgroups: 13.2 / 39.0 us unsplit, 7.1 / 14.1 in 4
-            // parts, 7.2 / 18.5 in 8; at 4096 -> 14336, 224 of them: 15.3 unsplit, 18.4 in 2)
-            while (ksplit < 32 && col_wgs * ksplit < 3L * current_cus() / 4 && nsub / (ksplit * 2) >= 4)
-                ksplit *= 2;
-        }
+        const int ksplit = room ? row_deq_mfma_parts(M, N, K, current_cus()) : 1;
         const int per_part = (nsub + ksplit - 1) / ksplit;
-        ksplit = (nsub + per_part - 1) / per_part;              // (no empty parts)
         const int waves = per_part < kRowDeqWaves ? per_part : kRowDeqWaves;
         const dim3 grid(static_cast<unsigned>((N / 32 + nww - 1) / nww), static_cast<unsigned>(M), static_cast<unsigned>(ksplit)), block(64 * waves);
         if (nww == 4)
@@ -4554,16 +4574,25 @@ int sbvr_hip_row_deq_last_kernel(void) { return g_row_deq_kernel; }
 
 int sbvr_hip_row_deq_last_parts(void) { return g_row_deq_parts; }
 
-// (the launch splits K only while its column workgroups cover less than three quarters of the CUs: the predicate
-// of sbvr_hip_row_deq_mm_T_ws; a prefill-sized call needs nothing)
+size_t sbvr_hip_row_deq_mm_T_workspace_for(int M, int N, int K, int S, int G)
+{
+    if (M <= 0 || N <= 0 || K <= 0)
+        return 0;
+    const int cus = current_cus();
+    const int parts = row_deq_rows(M, N, K, S, G, cus) ? row_deq_rows_parts(M, N, K, cus)
+                                                       : (row_deq_mfma_ok(M, K, S, G) ? row_deq_mfma_parts(M, N, K, cus) : 1);
+    return parts > 1 ? static_cast<size_t>(M) * N * sizeof(unsigned long long) : 0;
+}
+
+// (of any K, planes and groups: several rows are split while their column workgroups are fewer than two a CU, which covers the
+// launch row by row; a prefill-sized call needs nothing)
 size_t sbvr_hip_row_deq_mm_T_workspace(int M, int N)
 {
     if (M <= 0 || N <= 0)
         return 0;
-    if (M >= 2)
-        return static_cast<long>(N / 32) * ((M + 31) / 32) < 2L * current_cus() ? static_cast<size_t>(M) * N * sizeof(unsigned long long) : 0;
-    const long col_wgs = static_cast<long>((N / 32 + 1) / 2) * M;
-    return col_wgs * 2 < 3L * current_cus() / 4 ? static_cast<size_t>(M) * N * sizeof(unsigned long long) : 0;
+    const int cus = current_cus();
+    const bool splits = M >= 2 ? static_cast<long>(N / 32) * ((M + 31) / 32) < 2L * cus : static_cast<long>((N / 32 + 1) / 2) * 2 < 3L * cus / 4;
+    return splits ? static_cast<size_t>(M) * N * sizeof(unsigned long long) : 0;
 }
 
 // (only one left row may run on the decode kernel, the one form that may split K across workgroups)

@@ -409,7 +409,8 @@ torch::Tensor sbvr_row_deq_mm_T(const torch::Tensor &l_w, const torch::Tensor &r
     const DeviceGuard guard(l_w.device());
     auto out = at::empty({M, N}, l_w.options());
     hipStream_t stream = current_stream();
-    const size_t need = sbvr_hip_row_deq_mm_T_workspace(static_cast<int>(M), static_cast<int>(N));
+    const size_t need = sbvr_hip_row_deq_mm_T_workspace_for(static_cast<int>(M), static_cast<int>(N), static_cast<int>(K),
+                                                            static_cast<int>(S), static_cast<int>(G));
     torch::Tensor ws;                    // (no split of K for this call: no workspace, nothing allocated)
     if (need)
         ws = workspace(need, l_w.device(), stream, Users::kFunctions);

@@ -76,6 +76,8 @@ def _load():
     lib.sbvr_hip_read_floor.argtypes = [vp, sz, sz, i, i, i, i, i, i, vp, vp]
     lib.sbvr_hip_row_deq_mm_T_workspace.restype = sz
     lib.sbvr_hip_row_deq_mm_T_workspace.argtypes = [i, i]
+    lib.sbvr_hip_row_deq_mm_T_workspace_for.restype = sz
+    lib.sbvr_hip_row_deq_mm_T_workspace_for.argtypes = [i, i, i, i, i]
     lib.sbvr_hip_mm_T.argtypes = [vp, vp, i, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, i, i, vp]
     lib.sbvr_hip_mm_T_ws.argtypes = [vp, vp, i, vp, vp, vp, i, vp, vp, vp, i, i, i, i, i, i, i, i, vp, sz, vp]
     lib.sbvr_hip_mm_T_workspace.restype = sz
@@ -392,7 +394,7 @@ def _sbvr_row_deq_mm_T(l_w, r_bvr, r_coeff_idx, r_coeff_cache, bias, use_shfl=0,
     ib = _idx_bytes(r_coeff_idx, L, "r_coeff_idx")
     out = torch.empty((M, N), dtype=torch.float16, device=dev)
     with torch.cuda.device(dev):
-        need = lib.sbvr_hip_row_deq_mm_T_workspace(M, N)
+        need = lib.sbvr_hip_row_deq_mm_T_workspace_for(M, N, K, S, G)
         ws = _workspace(need, dev) if need else None          # (0: the call does not split K)
         _check(lib.sbvr_hip_row_deq_mm_T_ws(l_w.data_ptr(), r_bvr.data_ptr(), r_coeff_idx.data_ptr(), ib,
                                             r_coeff_cache.data_ptr(), _bias_ptr(bias, N, dev), out.data_ptr(),

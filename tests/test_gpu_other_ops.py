@@ -271,6 +271,36 @@ def test_row_deq_mm_T_with_values_that_the_accumulators_cannot_hold(oracle, M, N
     assert int(hip._workspace(8 * M * N, dev).count_nonzero()) == 0
 
 
+@pytest.mark.parametrize("M,N,K,S,G,kernel,parts", [(3, 2048, 1024, 4, 128, 3, 1), (2, 4096, 1024, 4, 128, 3, 1),      # many column workgroups
+                                                    (1, 2048, 1024, 4, 128, 3, 2), (2, 1024, 1024, 4, 128, 3, 2),
+                                                    (3, 4096, 4096, 6, 128, 2, 1),                                    # no launch that splits
+                                                    (4, 14336, 2048, 3, 128, 4, 2), (3, 4096, 4096, 4, 256, 4, 4)])
+def test_row_deq_mm_T_splits_where_it_asks_for_the_accumulators(M, N, K, S, G, kernel, parts):
+    """K in parts only where the call's own rule says so, not wherever a caller brings accumulators: those of a call that is not
+    split stay as they are (here: not zero), and it asks for none."""
+    import ctypes
+    import sbvr
+    from sbvr import hip, synth
+    dev = torch.device("cuda:0")
+    lib, vp = hip._load(), ctypes.c_void_p
+    db, di, dc = (t.to(dev) for t in synth.random_encoding(K, N, S, G, 256, seed=N + M))
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(M)).to(torch.float16).to(dev)
+    ws = torch.full((M * N,), 0 if parts > 1 else 1 << 40, dtype=torch.int64, device=dev)
+    outs = []
+    for w in (ws, None):
+        out = torch.empty((M, N), dtype=torch.float16, device=dev)
+        rc = lib.sbvr_hip_row_deq_mm_T_ws(vp(x.data_ptr()), vp(db.data_ptr()), vp(di.data_ptr()), 1, vp(dc.data_ptr()), None, vp(out.data_ptr()),
+                                          M, N, K, S, G, 256, vp(w.data_ptr()) if w is not None else None, 8 * M * N if w is not None else 0,
+                                          vp(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0 and hip.row_deq_last() == (kernel, parts if w is not None else 1)
+        outs.append(out)
+    need = lib.sbvr_hip_row_deq_mm_T_workspace_for(M, N, K, S, G)
+    assert (need > 0) == (parts > 1) and need in (0, 8 * M * N) and lib.sbvr_hip_row_deq_mm_T_workspace(M, N) >= need
+    assert bool((ws == (0 if parts > 1 else 1 << 40)).all())
+    if parts == 1:
+        assert torch.equal(*outs)
+
+
 def test_row_deq_mm_T_without_workspace_and_repeatable(oracle):
     """The reference-shaped entry point (no workspace: K is never split across workgroups) against the oracle at a
     shape the binding would split, and the split form twice: the fixed-point accumulators make it repeatable."""
