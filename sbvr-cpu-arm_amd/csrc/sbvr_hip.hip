@@ -1849,11 +1849,13 @@ __device__ __forceinline__ float lut_output(const RowsArgs &a, int m, int n)
     constexpr int H = WeightTables<S>::H;
     const uint16_t *const x = a.x + static_cast<size_t>(m) * a.K;
     double sum = 0.;
+#pragma unroll 1
     for (int word = 0; word < a.K / 32; ++word) {
         const size_t at = (static_cast<size_t>(word / a.words_per_group) * a.N + n) << a.idx16;
         const uint8_t *ib = static_cast<const uint8_t *>(a.idx);
         const int line = min(a.idx16 ? ib[at] | (ib[at + 1] << 8) : ib[at], a.L - 1);
         const uint32_t *w = a.bvr + (static_cast<size_t>(word) * a.N + n) * S;
+#pragma unroll 1                          // (unrolled, with 8 planes it takes the kernel's registers)
         for (int b = 0; b < 32; ++b) {
             _Float16 weight{};
 #pragma unroll
