@@ -229,13 +229,19 @@ constexpr int gemv_max_waves(int MT, int CT)
 
 __device__ __forceinline__ int as_int(v2s b) { return __builtin_bit_cast(int, b); }
 
-// max over the 64 lanes of a non-negative integer; the result is wave-uniform
-__device__ __forceinline__ uint32_t wave_umax(uint32_t v)
+// max over each row of 16 lanes of a non-negative integer, in all of its lanes
+__device__ __forceinline__ uint32_t row_umax(uint32_t v)
 {
     v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xB1, 0xF, 0xF, true)));   // quad_perm 1,0,3,2
     v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, true)));   // quad_perm 2,3,0,1
     v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xF, 0xF, true)));  // row_half_mirror
-    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xF, 0xF, true)));  // row_mirror
+    return max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xF, 0xF, true)));  // row_mirror
+}
+
+// max over the 64 lanes of a non-negative integer; the result is wave-uniform
+__device__ __forceinline__ uint32_t wave_umax(uint32_t v)
+{
+    v = row_umax(v);
     const uint32_t r0 = __builtin_amdgcn_readlane(v, 0), r1 = __builtin_amdgcn_readlane(v, 16);
     const uint32_t r2 = __builtin_amdgcn_readlane(v, 32), r3 = __builtin_amdgcn_readlane(v, 48);
     return max(max(r0, r1), max(r2, r3));
@@ -279,7 +285,7 @@ constexpr int kXPlanes = 5;
 //           other, so every operand row meets one coefficient line; the two are added up at the end.  Outputs that are not
 //           finite that way are summed again as the portable kernel does, from the selected activations alone.  Up to 4 batch rows
 //           (5 rows on: the 32-row kernels).  One thread per output, which took them before, 4096 -> 14336, 4 planes,
-//           one row: 1067 us; here 7.3.  (12800 -> 731, 6 planes, one row 4911 and 5.4; 8192 -> 28672, 2 rows 2219 and 30.)
+//           one row: 1067 us; here 6.7.  (12800 -> 731, 6 planes, one row 4911 and 5.0; 8192 -> 28672, 2 rows 2219 and 25.7.)
 constexpr int kXHalves = 6;
 // A prompt's tokens, up to 4 rows, with the sums of the one-row launches they stand for, bit for bit:
 //   kXSwiGLURows  kXSwiGLU for every row;
@@ -435,19 +441,17 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
                 }
         }
     } else if constexpr (XM == kXHalves) {
-        // operand rows 2m and 2m + 1: batch row m with the second half of the sub-group, or the first, left out
+        // operand rows 2m and 2m + 1: the first half of the sub-group of batch row m (lanes 0 to 31), and the second
 #pragma unroll
         for (int sgi = 0; sgi < SP; ++sgi)
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
                 for (int r = 0; r < 4; r += 2) {
-                    uint32_t v = 0u;
+                    xx[sgi][mt][r] = xx[sgi][mt][r + 1] = 0u;
                     if (mt * 2 + r / 2 < a.M)                       // wave-uniform
-                        v = reinterpret_cast<const uint32_t *>(a.x + static_cast<size_t>(mt * 2 + r / 2) * a.xstride +
-                                                               static_cast<size_t>(sg0 + sgi) * kSub)[lane];
-                    xx[sgi][mt][r] = lane < 32 ? v : 0u;
-                    xx[sgi][mt][r + 1] = lane < 32 ? 0u : v;
+                        xx[sgi][mt][r] = reinterpret_cast<const uint32_t *>(a.x + static_cast<size_t>(mt * 2 + r / 2) * a.xstride +
+                                                                           static_cast<size_t>(sg0 + sgi) * kSub)[lane];
                 }
     } else if constexpr (!kNorm) {
 #pragma unroll
@@ -627,8 +631,46 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
             for (int mt = MT - 1; mt >= 0; --mt) {
                 scale[sgi][mt] = 0.f;
 #pragma unroll
+                for (int r = 0; r < 4; r += 2) {
+                    if (XM == kXHalves && mt * 4 + r < m_rows) {      // wave-uniform
+                        // rows r and r + 1 at once: a lane's two elements belong to one of them, the other's bytes stay zero
+                        const uint32_t v = xx[sgi][mt][r];
+                        const uint32_t rows = row_umax(max(v & 0x7fffu, (v >> 16) & 0x7fffu));
+                        int eh_mine = 0;
+#pragma unroll
+                        for (int half = 0; half < 2; ++half) {
+                            const uint32_t amax = max(__builtin_amdgcn_readlane(rows, 32 * half), __builtin_amdgcn_readlane(rows, 32 * half + 16));
+                            const int eh = min(max(static_cast<int>(amax >> 10), 1), 30);
+                            if (blk == r + half)     // (a largest one that is not finite, which fp8 terms cannot tell: NaN, see the end)
+                                scale[sgi][mt] = amax < 0x7c00u ? __uint_as_float(static_cast<uint32_t>(106 + eh) << 23) : NAN;
+                            eh_mine = lane >> 5 == half ? eh : eh_mine;
+                        }
+                        const int va = __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x50, 0xF, 0xF, true);   // quad_perm 0,0,1,1
+                        const int vb = __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xFA, 0xF, 0xF, true);   // quad_perm 2,2,3,3
+                        const uint32_t zb = __builtin_amdgcn_perm(static_cast<uint32_t>(vb), static_cast<uint32_t>(va), half_sel);
+                        const float sc = __uint_as_float(static_cast<uint32_t>(107 + eh_mine - fac_log2) << 23);
+                        const float sc_last = __uint_as_float(static_cast<uint32_t>(99 + eh_mine - fac_log2) << 23);
+                        // (a sum of products keeps 2^-12 of its largest one's binade: of an element 2^9 below the largest and
+                        // further the first term would lose bits, and the other two hold what counts of it.  Without this the
+                        // sums were 2.5e-6 to 6.4e-6 of their own size off, with it 1e-7, one thread per output 3e-7)
+                        const uint32_t least = static_cast<uint32_t>(max(eh_mine - 9, 0)) << 10;
+                        const v2h first = as_v2h(((zb & 0x7fffu) < least ? 0u : zb & 0xffffu) | ((zb >> 16 & 0x7fffu) < least ? 0u : zb & 0xffff0000u));
+                        v2h z = as_v2h(zb);
+                        v2s b = {0, 0};
+                        b = __builtin_amdgcn_cvt_scalef32_pk_fp8_f16(b, first, sc, false);
+                        z -= __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(as_int(b), sc, false);
+                        b = __builtin_amdgcn_cvt_scalef32_pk_fp8_f16(b, z, sc, true);
+                        z -= __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(as_int(b), sc, true);
+                        const v2s b3 = __builtin_amdgcn_cvt_scalef32_pk_fp8_f16(v2s{0, 0}, z, sc_last, false);
+                        unsigned char *const at = mine + off + (r + (lane >> 5)) * 128;
+                        *reinterpret_cast<short *>(at) = b[0];
+                        *reinterpret_cast<short *>(at + 32) = b[1];
+                        *reinterpret_cast<short *>(at + 64) = b3[0];
+                    }
+                }
+#pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    if (mt * 4 + r < m_rows) {      // wave-uniform
+                    if (XM != kXHalves && mt * 4 + r < m_rows) {      // wave-uniform
                         uint32_t v = xx[sgi][mt][r];
                         if constexpr (kSwiGLU)
                             v = swiglu_pair(v, x2[sgi][mt][r]);
@@ -641,8 +683,6 @@ sbvr_gemv_mfma_kernel(const GemvArgs a)
                         const int e = 20 - eh;
                         if (blk == r)            // products come out as 2 * x * 2^e
                             scale[sgi][mt] = __uint_as_float(static_cast<uint32_t>(126 - e) << 23);
-                        if (XM == kXHalves && blk == r && amax >= 0x7c00u)     // not finite, which fp8 terms cannot tell: NaN, see the end
-                            scale[sgi][mt] = NAN;
                         // the lane's two elements, from the dwords (2l, 2l + 1) the lanes of its quad loaded
                         const int va = __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x50, 0xF, 0xF, true);   // quad_perm 0,0,1,1
                         const int vb = __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xFA, 0xF, 0xF, true);   // quad_perm 2,2,3,3

@@ -398,3 +398,27 @@ def test_groups_of_64_with_values_that_sums_cannot_hold(N, K, S, M, parts):
         rms = np.sqrt(np.mean(want[finite & (np.abs(want) < 100)] ** 2))
         assert (np.abs(y[finite] - want[finite]) <= (2.0 ** -9 * np.maximum(np.abs(want), rms) + large[:, None])[finite]).all(), special
         assert int(ws.count_nonzero()) == 0
+
+
+@pytest.mark.parametrize("N,K,S,M", [(4096, 4096, 4, 1), (512, 8192, 4, 2), (1000, 4096, 2, 4)])
+def test_groups_of_64_are_as_exact_as_fp32_sums(N, K, S, M):
+    """The second half of K is the first with its groups and their elements in another order and the activations negated, so that
+    every sum is zero and what the kernel leaves is its own error: at most one rounding (2^-24) per group of 64 of the sum of
+    a half, whatever small activations stand beside large ones."""
+    import sbvr
+    from sbvr import hip, synth
+    rng = np.random.default_rng(K + M)
+    H = K // 2
+    bits, idx = rng.integers(0, 2, (H, N, S), dtype=np.uint32), rng.integers(0, 256, (H // 64, N))
+    groups, elements = rng.permutation(H // 64), rng.permutation(64)
+    order = (groups[:, None] * 64 + elements[None, :]).ravel()
+    x = rng.standard_normal((M, H)).astype(np.float16)
+    bits, idx = np.concatenate((bits, bits[order])), np.concatenate((idx, idx[groups])).astype(np.uint8)
+    bvr = (bits.reshape(K // 32, 32, N, S) << np.arange(32, dtype=np.uint32)[None, :, None, None]).sum(axis=1, dtype=np.uint32)
+    cache = synth.make_lines(256, S, 0.02, K)
+    y = sbvr._sbvr_linear_f16(*(torch.from_numpy(a).to(_dev()) for a in (np.concatenate((x, -x[:, order]), axis=1), bvr, idx)), cache.to(_dev()),
+                              None, bvr_len=64)
+    assert hip.last_kernel() == DECODE
+    w = (bits[:H] * np.repeat(cache.numpy().astype(np.float64)[idx[:H // 64]], 64, axis=0)).sum(axis=2)
+    half = np.sqrt(np.mean((x.astype(np.float64) @ w) ** 2))
+    assert float(y.float().abs().max()) <= (K // 64) * 2.0 ** -24 * half
