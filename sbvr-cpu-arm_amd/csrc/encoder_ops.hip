@@ -159,13 +159,15 @@ sbvr_encoder_candidates_kernel(const CandidateArgs a)
 // The host queues rounds ahead and looks at the state now and then; rounds behind the last miss do nothing, and so do
 // those behind a group whose candidates these kernels do not form (status 1: the host takes that group through
 // the general path).  State: two slots, read one and written the other by turns, so that workgroups of a launch never
-// read what it changes.
+// read what it changes, but for `found` of the slot read, which the search takes minima into (and reads as a bound).  That a group
+// is left to the host the search says in the other slot, for the settling launch alone.
 // A workgroup's search is bound by the vector ALU (3 packed operations per two points and value); a wave stops when
 // all of its 64 lines are above the best error known.  1024 x 4096, groups of 128, 4 planes (241 misses): 269 to 327 ms
 // with about 50 launches and two waits a miss, 14.6 to 17.2 here: 23 us a search (2.6e5 to 4.6e5 lines; 38 to 59 without
 // the bound), 17 us to settle it over up to 32768 groups.  512 x 2048, 3 planes 117 -> 5.2 ms; 64 x 512, 2 planes 36.6 -> 2.4.
 struct EncoderState {
-    int lines, misses, history, status, miss, pad;
+    int lines, misses, history, status, miss;
+    int uncovered;                       // written by the search for the settling launch behind it: the group is the host's
     unsigned long long found;            // error's bits << 32 | candidate: the least so far (all ones: none)
 };
 
@@ -360,8 +362,7 @@ sbvr_encoder_search_kernel(const sbvr_hip_encoder_run a, int slot)
         const bool stays = idle || !sp.covered;
         states[slot ^ 1].miss = stays ? st.miss : kEncNone;
         states[slot ^ 1].found = ~0ull;
-        if (!idle && !sp.covered)
-            states[slot].status = 1;
+        states[slot ^ 1].uncovered = !idle && !sp.covered;
     }
     if (idle || !sp.covered)
         return;
@@ -431,13 +432,14 @@ sbvr_encoder_settle_kernel(const sbvr_hip_encoder_run a, int slot)
     EncoderState next = st;                                            // (miss and found: written by the search and by minima)
     const bool found = st.found != ~0ull;
     // (nothing left, a group for the host, or one that neither the table nor any candidate has an error for: the state stays)
-    const bool stays = st.status != 0 || m >= a.groups, unserved = !stays && !found && a.line[m] < 0;
+    const bool uncovered = states[slot ^ 1].uncovered != 0;            // (no workgroup of this launch writes it)
+    const bool stays = st.status != 0 || m >= a.groups || uncovered, unserved = !stays && !found && a.line[m] < 0;
     if (stays || unserved) {
         if (blockIdx.x == 0 && tid == 0) {
             states[slot ^ 1].lines = st.lines;
             states[slot ^ 1].misses = st.misses;
             states[slot ^ 1].history = st.history;
-            states[slot ^ 1].status = unserved ? 1 : st.status;
+            states[slot ^ 1].status = unserved || uncovered ? 1 : st.status;
             if (unserved)
                 atomicMin(&states[slot ^ 1].miss, m);
         }

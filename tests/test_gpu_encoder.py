@@ -250,3 +250,28 @@ def test_the_device_policy_over_several_chunks():
         out.append((line_of, sel, enc.table[:conf.num_coeff_cache_lines].clone(), conf.mse_history, conf.cache_hits, conf.group_idx))
     for other in out[1:]:
         assert all(torch.equal(a, b) for a, b in zip(out[0][:3], other[:3])) and out[0][3:] == other[3:]
+
+
+def test_a_round_leaves_the_slot_it_reads(monkeypatch):
+    """A group whose candidates the search does not form: the round says so in the slot it writes, and leaves the one that
+    all of its workgroups read as it is."""
+    import sys
+    import sbvr
+    from sbvr import hip
+    real, seen = hip.encoder_rounds, []
+
+    def rounds(run, S, lines, slot, many, device):
+        if not seen:
+            state = sys._getframe(1).f_locals["state"]
+            before = state.clone()
+            real(run, S, lines, 0, 1, device)
+            seen.append((before.tolist(), state.tolist()))
+            state.copy_(before)
+        real(run, S, lines, slot, many, device)
+
+    monkeypatch.setattr(hip, "encoder_rounds", rounds)
+    w = torch.randn((8, 512), generator=torch.Generator().manual_seed(5)) * 0.02
+    w[0, :128] += 2.0                                            # (a mean that moves the offsets)
+    _encode_both_ways(w.to(torch.float16).to("cuda:0"), dict(num_sums=4, bvr_len=128))
+    (before, after), = seen
+    assert after[:8] == before[:8] and after[8:13] == before[:3] + [1, before[4]]
