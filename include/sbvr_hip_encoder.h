@@ -67,6 +67,9 @@ typedef struct {
     double acceptable;
 } sbvr_hip_encoder_run;
 size_t sbvr_hip_encoder_state_bytes(void);
+/* The most scales a search of this space may have for the rounds to take it (a group with more is left to the caller), 0 where
+ * they take no such search. */
+int sbvr_hip_encoder_scales(int S, int G, int bases, int n_offsets, int axis_values);
 int sbvr_hip_encoder_rounds_f16(const sbvr_hip_encoder_run *run, int S, int lines, int slot, int rounds, void *stream);
 
 /* sel and line_of of groups first .. first + groups - 1 that are not settled, against the table line `line` names. */

@@ -935,6 +935,15 @@ int sbvr_hip_encoder_candidates_f16(const void *data, int G, const void *base, i
 
 size_t sbvr_hip_encoder_state_bytes(void) { return 2 * sizeof(EncoderState); }
 
+int sbvr_hip_encoder_scales(int S, int G, int bases, int n_offsets, int axis_values)
+{
+    sbvr_hip_encoder_run space{};
+    space.bases[0] = bases;
+    space.n_offsets[0] = n_offsets;
+    space.axis_values[0] = axis_values;
+    return S >= 2 && S <= 6 && G > 0 && G <= kEncMaxG && G % 4 == 0 && bases > 0 && n_offsets > 0 && axis_values > 1 && run_lines(space, 0, S) ? kEncMaxScales : 0;
+}
+
 int sbvr_hip_encoder_rounds_f16(const sbvr_hip_encoder_run *run, int S, int lines, int slot, int rounds, void *stream)
 {
     if (!run_ok(run) || lines <= 0 || slot < 0 || slot > 1 || rounds <= 0)

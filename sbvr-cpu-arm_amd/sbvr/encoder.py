@@ -358,11 +358,14 @@ class GroupEncoder:
             return None
         kw = dict(device=flat.device, dtype=flat.dtype)
         spaces = [self._fixed_space(extended, kw) for extended in (False, True)]
-        # (a search must be one batch of the policy's scan; the number of scales is the step's count, or one or two more)
-        lines = [base.shape[0] * b.shape[0] * (math.ceil(c.s_search_num * ratio) + 2) + (per_dim + 1) ** S
-                 for (base, b, per_dim), ratio in zip(spaces, (1.0, max(1.0, c.extend_ratio)))]
-        if max(lines) > min(c.search_batch_size, 1 << 27) or any(S * (p + 1) > 4096 or p < 1 or 0 in base.shape or b.numel() == 0
-                                                                for base, b, p in spaces):
+        # (a search, and a look-up in the table, must be one batch of the policy's scan; the number of scales is the step's count,
+        # or one or two more)
+        scales = [math.ceil(c.s_search_num * ratio) + 2 for ratio in (1.0, max(1.0, c.extend_ratio))]
+        lines = [base.shape[0] * b.shape[0] * n + (per_dim + 1) ** S for (base, b, per_dim), n in zip(spaces, scales)]
+        most_lines = min(self.table.shape[0], c.num_coeff_cache_lines + flat.numel() // G)
+        if max(lines) > 1 << 27 or max(lines + [most_lines]) > c.search_batch_size:
+            return None
+        if any(n > hip.encoder_scales(S, G, base.shape[0], b.numel(), per_dim + 1) for (base, b, per_dim), n in zip(spaces, scales)):
             return None
         return spaces, lines
 

@@ -102,6 +102,7 @@ def _load():
     lib.sbvr_hip_dec_rows_advance.argtypes = [vp, i, i, vp, vp, i, vp, vp]
     lib.sbvr_hip_encoder_group_mse_f16.argtypes = [vp, vp, vp, i, i, i, i, vp]
     lib.sbvr_hip_encoder_state_bytes.restype = sz
+    lib.sbvr_hip_encoder_scales.argtypes = [i, i, i, i, i]
     lib.sbvr_hip_encoder_rounds_f16.argtypes = [ctypes.POINTER(EncoderRun), i, i, i, i, vp]
     lib.sbvr_hip_encoder_selectors_f16.argtypes = [ctypes.POINTER(EncoderRun), i, i, i, vp]
     lib.sbvr_hip_encoder_candidates_f16.argtypes = [vp, i, vp, i, vp, i, vp, i, vp, i, i, vp, vp, vp]
@@ -756,6 +757,11 @@ def encoder_selectors(run, S, first, groups, device):
         rc = _load().sbvr_hip_encoder_selectors_f16(ctypes.byref(run), S, first, groups, _stream())
     if rc != 0:
         raise SbvrHipError(f"sbvr_hip_encoder_selectors_f16: error {rc} (G={run.G} S={S} first={first} groups={groups})")
+
+
+def encoder_scales(S, G, bases, offsets, axis_values):
+    """The most scales a search of this space may have for ``encoder_rounds`` to take its groups; 0: none."""
+    return _load().sbvr_hip_encoder_scales(S, G, bases, offsets, axis_values)
 
 
 def encoder_state_words():

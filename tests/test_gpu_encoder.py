@@ -275,3 +275,23 @@ def test_a_round_leaves_the_slot_it_reads(monkeypatch):
     _encode_both_ways(w.to(torch.float16).to("cuda:0"), dict(num_sums=4, bvr_len=128))
     (before, after), = seen
     assert after[:8] == before[:8] and after[8:13] == before[:3] + [1, before[4]]
+
+
+@pytest.mark.parametrize("S,covered,more", [
+    (3, True, {"s_search_num": 131}), (3, False, {"s_search_num": 134}), (3, False, {"s_search_num": 200}),      # 160 scales at most, 1.2 times as many when wide
+    (2, False, {"r_search_num": 1200, "b_search_num": 1200, "s_search_num": 1}),      # too many families for a launch's candidate numbers
+    (3, False, {"search_batch_size": 9000, "r_search_num": 16, "b_search_num": 8, "s_search_num": 8}),
+])
+def test_the_rounds_take_what_their_launches_take(S, covered, more):
+    """What the rounds' launches refuse, or could leave to the host group after group, goes through the block loop; the last
+    case by a table that may grow beyond a batch of the look-up's scan."""
+    from sbvr.encoder import EncoderConfig, GroupEncoder
+    dev = torch.device("cuda:0")
+    conf = dict(num_sums=S, bvr_len=64, **dict({"search_batch_size": 1 << 24}, **more))
+    enc = GroupEncoder(EncoderConfig(**conf), torch.float16, dev)
+    flat = torch.zeros(64 * (10000 if "search_batch_size" in more else 40), dtype=torch.float16, device=dev)
+    assert (enc._covered_on_device(flat) is not None) == covered
+    if "search_batch_size" in more:
+        assert enc._covered_on_device(flat[:64 * 9000]) is not None
+    w = (torch.randn((5, 512), generator=torch.Generator().manual_seed(S)) * 0.02).to(torch.float16).to(dev)
+    _encode_both_ways(w, conf)
