@@ -436,7 +436,9 @@ class GroupEncoder:
                 miss = next_miss(miss + 1)
                 c.group_idx, c.cache_hits = start + miss, c.cache_hits + miss - (c.group_idx - start)
                 put(miss)
-            rounds = min(64, 2 * rounds)
+                rounds = 2                          # (groups like this one, or a table that is full, may follow each other)
+            else:
+                rounds = min(64, 2 * rounds)
         hip.encoder_selectors(run, S, 0, n, dev)
         if progress is not None:
             progress(n - shown)

@@ -295,3 +295,20 @@ def test_the_rounds_take_what_their_launches_take(S, covered, more):
         assert enc._covered_on_device(flat[:64 * 9000]) is not None
     w = (torch.randn((5, 512), generator=torch.Generator().manual_seed(S)) * 0.02).to(torch.float16).to(dev)
     _encode_both_ways(w, conf)
+
+
+def test_few_rounds_are_queued_behind_a_group_for_the_host(monkeypatch):
+    """Groups left to the host one after the other: two launches at a time are queued behind such a group, not dozens."""
+    from sbvr import hip
+    real, queued = hip.encoder_rounds, []
+
+    def rounds(run, S, lines, slot, many, device):
+        queued.append(many)
+        real(run, S, lines, slot, many, device)
+
+    monkeypatch.setattr(hip, "encoder_rounds", rounds)
+    w = torch.randn((48, 512), generator=torch.Generator().manual_seed(5)) * 0.02
+    w[::2] += 2.0
+    stats = _encode_both_ways(w.to(torch.float16).to("cuda:0"), dict(num_sums=4, bvr_len=128))
+    misses = stats["groups"] - stats["cache_hits"]
+    assert sum(queued) <= 16 + 4 * misses
