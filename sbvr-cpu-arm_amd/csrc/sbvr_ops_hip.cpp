@@ -13,6 +13,7 @@
 #include <ATen/hip/HIPContext.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <hip/hip_runtime_api.h>
 
 #include <map>
 #include <mutex>
@@ -111,16 +112,22 @@ void check_encoder(int rc, const char *what, const Args &...shape)
 // replayed on others: a layer called on that stream meanwhile must not add into it.)
 enum class Users { kLinears, kFunctions };
 
+// While a graph is recorded on a stream whose buffer is missing or too small, the call gets one of the recording: its memory is
+// the graph's, and the zeros are a node of the graph that has not run, so it is not kept for calls outside.  One per stream and
+// set, dropped by the next such recording or the next buffer of its own.
 torch::Tensor workspace(size_t nbytes, c10::Device device, hipStream_t stream, Users users)
 {
+    using Key = std::tuple<int, hipStream_t, Users>;
     static std::mutex mu;
-    static std::map<std::tuple<int, hipStream_t, Users>, torch::Tensor> held;
+    static std::map<Key, torch::Tensor> held;
+    static std::map<Key, std::pair<unsigned long long, torch::Tensor>> recorded;       // (the recording's number, its buffer)
     static std::vector<torch::Tensor> outgrown;
-    const auto key = std::make_tuple(static_cast<int>(device.index()), stream, users);
+    const Key key(static_cast<int>(device.index()), stream, users);
     auto enough = [&]() -> torch::Tensor {
         const auto it = held.find(key);
         return it != held.end() && static_cast<size_t>(it->second.numel()) >= nbytes ? it->second : torch::Tensor();
     };
+    auto zeros = [&](size_t size) { return torch::zeros({static_cast<int64_t>(size)}, torch::dtype(torch::kUInt8).device(device)); };
     size_t size = std::max(nbytes, static_cast<size_t>(1) << 20);
     {
         std::lock_guard<std::mutex> lock(mu);
@@ -130,14 +137,41 @@ torch::Tensor workspace(size_t nbytes, c10::Device device, hipStream_t stream, U
         if (held.count(key))
             size = std::max(size, 2 * static_cast<size_t>(held[key].numel()));
     }
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long recording = 0;
+    if (hipStreamGetCaptureInfo(stream, &status, &recording) != hipSuccess) {
+        status = hipStreamCaptureStatusNone;
+        (void)hipGetLastError();             // (not the next launch's)
+    }
+    torch::Tensor made, dropped;             // (dropped: let go without the lock, as Python may hold the other end)
+    if (status != hipStreamCaptureStatusNone) {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            const auto it = recorded.find(key);
+            if (it != recorded.end() && it->second.first == recording && static_cast<size_t>(it->second.second.numel()) >= nbytes)
+                return it->second.second;
+        }
+        // (a smaller one of this recording: nodes recorded before keep its address, whose memory may serve nodes behind them)
+        made = zeros(nbytes);
+        std::lock_guard<std::mutex> lock(mu);
+        auto &slot = recorded[key];
+        dropped = std::move(slot.second);
+        slot = {recording, made};
+        return made;
+    }
     // (allocated without the lock: torch may run Python on the way)
-    torch::Tensor made = torch::zeros({static_cast<int64_t>(size)}, torch::dtype(torch::kUInt8).device(device));
+    made = zeros(size);
     std::lock_guard<std::mutex> lock(mu);
     torch::Tensor have = enough();           // (another thread on this stream was faster)
     if (have.defined())
         return have;
     if (held.count(key))
         outgrown.push_back(held[key]);
+    const auto it = recorded.find(key);
+    if (it != recorded.end()) {
+        dropped = std::move(it->second.second);
+        recorded.erase(it);
+    }
     held[key] = made;
     return made;
 }

@@ -234,15 +234,20 @@ def _workspace(nbytes, device):
     """Zero-initialised scratch per (device, stream); grown on demand to twice its size at least.  The
     kernels leave the part that must be zero zeroed.  A buffer that is outgrown
     stays allocated: a HIP graph recorded earlier on the stream keeps its address.
+    While a graph is recorded on a stream without such a buffer, one that belongs to the recording and is not kept.
     The buffers are the extension's, which launches some of these functions
     itself."""
     key = (device.index, torch.cuda.current_stream(device).cuda_stream)
     ext = _ext()
     if ext:
-        ws = _workspaces[key] = ext._workspace(nbytes, device.index)
+        ws = ext._workspace(nbytes, device.index)
+        if _workspaces.get(key) is not ws and not torch.cuda.is_current_stream_capturing():
+            _workspaces[key] = ws
         return ws
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
+        if torch.cuda.is_current_stream_capturing():       # (the recording's own, see csrc/sbvr_ops_hip.cpp)
+            return torch.zeros(nbytes, dtype=torch.uint8, device=device)
         size = max(nbytes, 1 << 20)
         if ws is not None:
             _outgrown.append(ws)

@@ -89,3 +89,66 @@ def test_layers_keep_out_of_the_accumulators_of_recorded_functions():
         assert torch.equal(y, want) and int((ws.view(torch.int64)[:2 * N] != 1 << 40).sum()) == 0
         ws.zero_()
         side.synchronize()
+
+
+def _pool_of(t):
+    return [seg["segment_pool_id"] for seg in torch.cuda.memory_snapshot()
+            if seg["address"] <= t.data_ptr() < seg["address"] + seg["total_size"]]
+
+
+@pytest.mark.parametrize("grow", [False, True])
+def test_a_graph_recorded_on_a_stream_that_no_call_has_warmed(grow):
+    """The accumulators of such a recording are the graph's own: calls on the stream before the first replay, between replays
+    and after the graph's end have theirs, and every replay is right.  grow: the stream's buffer is there but too small."""
+    import sbvr
+    from sbvr import hip
+    N, K = 4096, 4096
+    x = torch.randn((24, K), generator=torch.Generator().manual_seed(4)).to(torch.float16).to(DEV)
+    none = torch.zeros(0, dtype=torch.float16, device=DEV)
+    t, small = _encoded(K, N, seed=3, L=256), _encoded(1024, K, seed=4)
+    halves = sbvr.SBVRLinear(12800, 731, *_encoded(731, 12800, G=64, seed=5), 64)
+    wide = sbvr.SBVRLinear(8192, 1304, *_encoded(1304, 8192, S=8, seed=6), 128)
+    xh, xw = x.reshape(-1)[:12800].view(1, -1), x.reshape(-1)[:24 * 4096 // 8192 * 8192].view(-1, 8192).repeat(2, 1)
+    calls = [lambda: sbvr._sbvr_linear_f16(x[:1], *small, bvr_len=128), lambda: sbvr._sbvr_row_deq_mm_T(x[:3], *t, none, bvr_len=128),
+             lambda: sbvr._sbvr_row_deq_mm_T(x[:8], *t, none, bvr_len=128), lambda: halves(xh), lambda: wide(xw)]
+    want, parts = [], []
+    for call in calls:
+        want.append(call())
+        parts.append(max(hip.last_parts(), hip.row_deq_last()[1]))
+    assert xw.shape[0] == 24 and min(parts) > 1
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    if grow:
+        many = x.repeat(2, 1)                                  # 48 rows x 4096: more than the least buffer of 1 MiB holds
+        calls.append(lambda: sbvr._sbvr_row_deq_mm_T(many, *t, none, bvr_len=128))
+        want.append(calls[-1]())
+        assert hip.row_deq_last()[1] > 1 and 8 * many.shape[0] * N > 1 << 20
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            assert all(torch.equal(call(), y) for call, y in zip(calls[:1], want))
+            assert hip._workspace(1, DEV).numel() == 1 << 20
+        side.synchronize()
+    never_run, graph = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(never_run, stream=side):
+        got = [call() for call in calls]
+        of_the_first = hip._workspace(8 * 48 * N, DEV)
+    with torch.cuda.graph(graph, stream=side):
+        got = [call() for call in calls]
+        assert hip._workspace(8 * 48 * N, DEV).data_ptr() != of_the_first.data_ptr()
+    del never_run, of_the_first
+    with torch.cuda.stream(side):
+        for call, y in zip(calls, want):
+            assert torch.equal(call(), y)
+        ws = hip._workspace(8 * 8 * N, DEV)
+        assert _pool_of(ws) == [(0, 0)] and int(ws.count_nonzero()) == 0
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        with torch.cuda.stream(side):
+            assert all(torch.equal(call(), y) for call, y in zip(calls, want))
+        torch.cuda.synchronize()
+    del graph, got
+    with torch.cuda.stream(side):
+        assert all(torch.equal(call(), y) for call, y in zip(calls, want))
+    torch.cuda.synchronize()
