@@ -3111,20 +3111,6 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
     }
 }
 
-// Whether several rows go that way.  Not while a CU has no more than one workgroup of the one-row kernels and each of its
-// waves one step or two (K up to 1408: 2 rows x 1024, K 513 9.0 us against 6.8, 4 x 1024, K 800 8.2 against 8.0; from K 2000 on
-// it is ahead), and not
-// two rows of the matrix-core kernel's shapes with columns enough for all CUs (14336 columns, K 4096: 28 us against 25).
-// us, these kernels and the one above: 3 rows x 4096, K 4096, 4 planes 12.7 and 11.2; 4096 columns, K 4100 2 / 8 / 32 rows
-// 14.9 / 52 / 200 and 13.2 / 13.6 / 16.5; 2048 columns, K 2050, 2 planes, 2 / 8 / 32 rows 8.3 / 15.7 / 54 and 7.4 / 7.7 / 9.9;
-// 14336 columns, K 10858, 3 planes, 32 rows 1397 and 65.
-bool row_deq_rows(int M, int N, int K, int S, int G, int cus)
-{
-    if (M < 2 || S < 2 || S > 4 || (K <= 1408 && static_cast<long>(N / 32) * M <= cus))
-        return false;
-    return !(M == 2 && S == 4 && K % kSub == 0 && G % 64 == 0 && (N / 32 + 1) / 2 * 2 >= cus);
-}
-
 // Parts of K where the caller brings the accumulators.  Several rows: as many as give the CUs two workgroups each, of 4 tiles and
 // more.
 int row_deq_rows_parts(int M, int N, int K, int cus)
@@ -3157,6 +3143,32 @@ int row_deq_mfma_parts(int M, int N, int K, int cus)
         ksplit *= 2;
     const int per_part = (nsub + ksplit - 1) / ksplit;
     return (nsub + per_part - 1) / per_part;
+}
+
+// Whether several rows go that way; parts: of K in either launch, 1 without the accumulators.
+// Against the lanes launch: from K 1409 on, 705 with 2 and 3 planes, or once a CU has more than one of its workgroups and ten of its
+// waves.  (us, lanes and here: up to 4 rows x 2048, 4 planes, K 400 / 600 / 800 / 1000 / 1300 5.5 / 6.5 / 8.0 / 7.8 / 8.5 and 6.2 / 8.3
+// / 8.3 / 6.8 / 8.8; 3 planes 5.3 / 6.5 / 7.9 / 7.7 / 8.4 and 5.6 / 7.1 / 7.0 / 6.2 / 7.5; 4 planes, K 100, 8 rows x 4096 / 16 x 4096 5.6 /
+// 8.2 and 6.9 / 7.1; K 250, 8 rows x 2048 / 4096 5.7 / 8.0 and 6.5; 14336 columns, K 10858, 3 planes, 32 rows 1397 and 57.)
+// Against the matrix-core launch, which takes rows one by one: by estimates fitted to 240 shapes (2 to 32 rows, 512 to 8192
+// columns, K 1024 to 8192; us, that launch and here: 2 rows x 1024, K 2048 5.0 and 6.4; 3 x 2048, K 1280 / 2048 6.5 / 7.7 and
+// 8.4 / 6.6; 3 x 4096, K 3072 / 4096 10.0 / 12.9 and 10.8 / 11.0; 8 x 512, K 4096 / 8192 6.0 / 8.3 and 6.7 / 7.0).  There: 0.3 us a
+// sub-group of a part, times its workgroups over the CUs rounded up.  Here: 2.05 us for each tile of a wave, 1.25 us more per
+// workgroup of a CU beyond the first.
+bool row_deq_rows(int M, int N, int K, int S, int G, int cus, bool room)
+{
+    if (M < 2 || S < 2 || S > 4)
+        return false;
+    if (!row_deq_mfma_ok(M, K, S, G))
+        return K > (S == 4 ? 1408 : 704) ||
+               (static_cast<long>(N / 32) * M > cus && static_cast<long>(N / 32) * M * std::min((K + 63) / 64, kRowDeqWaves) > 10L * cus);
+    const int theirs = room ? row_deq_mfma_parts(M, N, K, cus) : 1, ours = room ? row_deq_rows_parts(M, N, K, cus) : 1;
+    const int per_part = (K / kSub + theirs - 1) / theirs, tiles = ((K + 127) / 128 + ours - 1) / ours;
+    const double turns = ceil(static_cast<double>((N / 32 + 1) / 2) * M * theirs / cus);
+    const double load = std::max(0., static_cast<double>(N / 32) * ((M + 31) / 32) * ours / cus - 1.);
+    const double their_us = 2.9 + (theirs > 1 ? 0.7 : 0.) + 0.3 * per_part * turns;
+    const double our_us = 4.3 + 0.4 * load + (tiles + kDeqRowsWaves - 1) / kDeqRowsWaves * (2.05 + 1.25 * load) + (M > 16 ? 2.1 : (M > 8 ? 0.6 : 0.));
+    return our_us < their_us;
 }
 
 template <int S>
@@ -4519,7 +4531,7 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
     const bool tables_aligned = reinterpret_cast<uintptr_t>(r_bvr) % 16 == 0 && reinterpret_cast<uintptr_t>(r_coeff_cache) % 16 == 0;
     const bool room = workspace && reinterpret_cast<uintptr_t>(workspace) % 8 == 0 &&
                       workspace_bytes >= static_cast<size_t>(M) * N * sizeof(unsigned long long);
-    if (row_deq_rows(M, N, K, S, G, current_cus()) && tables_aligned && (static_cast<long>(M) + 31) / 32 <= 65535 && !env_switches().rowdeq_lanes) {
+    if (row_deq_rows(M, N, K, S, G, current_cus(), room) && tables_aligned && (static_cast<long>(M) + 31) / 32 <= 65535 && !env_switches().rowdeq_lanes) {
         // every weight decoded once for all rows
         const int tiles = (K + 127) / 128;
         RowDeqArgs a{static_cast<const uint16_t *>(x), r_bvr, r_coeff_idx, static_cast<const uint16_t *>(r_coeff_cache),
@@ -4621,7 +4633,7 @@ size_t sbvr_hip_row_deq_mm_T_workspace_for(int M, int N, int K, int S, int G)
     if (M <= 0 || N <= 0 || K <= 0)
         return 0;
     const int cus = current_cus();
-    const int parts = row_deq_rows(M, N, K, S, G, cus) ? row_deq_rows_parts(M, N, K, cus)
+    const int parts = row_deq_rows(M, N, K, S, G, cus, true) ? row_deq_rows_parts(M, N, K, cus)
                                                        : (row_deq_mfma_ok(M, K, S, G) ? row_deq_mfma_parts(M, N, K, cus) : 1);
     return parts > 1 ? static_cast<size_t>(M) * N * sizeof(unsigned long long) : 0;
 }
