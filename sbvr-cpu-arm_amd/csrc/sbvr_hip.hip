@@ -2870,12 +2870,15 @@ sbvr_row_deq_mfma_kernel(const uint16_t *__restrict__ x, const uint32_t *__restr
 // The trans=True product for several batch rows (2 to 4 planes): every weight decoded once for up to 32 rows.
 // A lane owns two neighbouring rows k of the weight and decodes their 32 columns by table look-up (sbvr_gemm_rows32_lut_kernel):
 // the row's 2^S subset sums as fp16 and, scaled by 2^11, what that rounding left over, so that a weight is the sum of two
-// fp16 values to 22 bits: as exact as the fp32 sums of the kernels above, whose error against 64 bits it does not exceed.  The pairs (k, k + 1) go to a
+// fp16 values to 22 bits.  The MFMAs of half a tile (and of all it left over, a 2^-11th) add up from zero before they join the sum,
+// or their roundings at the size of the whole sum, several an MFMA, would show: sums then are 0.73 to 1.03e-7 of the RMS output
+// off 64 bits (K 800 to 12032), where fp32 sums of exact products (the lanes kernel above) are 0.76 to 1.07e-7 and one chain of MFMAs
+// 0.95 to 1.75e-7; no slower so (3 rows x 4096, K 4096 11.3 us, 14336 columns, K 10858, 3 planes, 32 rows 63).  The pairs (k, k + 1) go to a
 // tile of 32 columns x 128 k in LDS (a lane's dwords of a column lie side by side; columns 272 bytes apart, so that 16 lanes
 // reading 16 columns meet different banks) and come back as the B operands of eight v_mfma_f32_32x32x16_f16 each, with the
 // batch rows, read from memory as they are, as A.  A workgroup owns 32 columns and 32 batch rows; its waves
 // take the tiles of K in turn and meet in LDS, and K is split across workgroups through the 64-bit accumulators.
-// Bound by the vector ALU: 684 operations a tile and wave with 4 planes (308 of them permutes), whatever the
+// Bound by the vector ALU: 731 operations a tile and wave with 4 planes (308 of them permutes), whatever the
 // number of rows, where the kernels above take 384 per 64 k and row or an A image per row.  Four waves a workgroup and one
 // tile each, so that three workgroups share a CU (two tiles a wave and eight waves: 8 rows x 12032, K 4853 45 us, 34 so).
 constexpr int kDeqRowsWaves = 4, kDeqTile = 32 * 272;         // bytes of a tile
@@ -2986,10 +2989,10 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
         }
     };
 
-    v16f acc_head, acc_rest;
+    v16f sum;
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-        acc_head[r] = acc_rest[r] = 0.f;
+        sum[r] = 0.f;
 
     Stage now;
     uint32_t c[2][CW];
@@ -3036,9 +3039,20 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
                 w[q] = in ? now.w[e].w[q] : 0u;
             lut_nibble_words<S>(w, Q[e]);
         }
-        // the first fp16 values through the wave's tile and the MFMAs, then what they left over (the LDS serves a wave's
-        // accesses in order)
-        auto multiply = [&](const LutTables<S> (&tab)[2], v16f &acc) __attribute__((always_inline)) {
+        // what the first fp16 values left over through the wave's tile and the MFMAs, then these themselves (the LDS serves a
+        // wave's accesses in order), in sums of half a tile
+        v16f acc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            acc[r] = 0.f;
+        auto settle = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                sum[r] += acc[r];
+                acc[r] = 0.f;
+            }
+        };
+        auto multiply = [&](const LutTables<S> (&tab)[2], bool in_halves) __attribute__((always_inline)) {
 #pragma unroll
             for (int p = 0; p < 8; ++p) {
                 uint32_t a01, a23, b01, b23;
@@ -3055,12 +3069,18 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
             for (int s = 0; s < 8; ++s) {
                 const v4u b = *reinterpret_cast<const v4u *>(tile + j * 272 + 32 * s + 16 * h);
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, x[s]), __builtin_bit_cast(v8h, b), acc, 0, 0, 0);
+                if (in_halves && s == 3)
+                    settle();
             }
             __builtin_amdgcn_wave_barrier();
         };
-        multiply(head, acc_head);
+        multiply(rest, false);
         gather(next, c);
-        multiply(rest, acc_rest);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            acc[r] *= 1.f / 2048.f;
+        multiply(head, true);
+        settle();
         now = next;
     }
     // A sum that is not finite: activations or coefficients that are not, or a weight beyond fp16.  The products of such an
@@ -3069,23 +3089,23 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
     bool odd = false;
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-        odd = odd || !(fabsf(acc_head[r]) < INFINITY) || !(fabsf(acc_rest[r]) < INFINITY);
+        odd = odd || !(fabsf(sum[r]) < INFINITY);
     if (__any(odd)) {                       // wave-uniform
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-            acc_head[r] = acc_rest[r] = 0.f;
+            sum[r] = 0.f;
         for (int t = t_begin + wave; t < t_end; t += waves)
             for (int k = 128 * t; k < min(K, 128 * t + 128); ++k)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
-                    acc_head[r] = row_deq_add<S>(a, nw, j, k, min(m0 + 8 * (r >> 2) + 4 * h + (r & 3), M - 1), acc_head[r]);
+                    sum[r] = row_deq_add<S>(a, nw, j, k, min(m0 + 8 * (r >> 2) + 4 * h + (r & 3), M - 1), sum[r]);
     }
     // ---- partial results meet in LDS; D[i][jj] sits in lane jj + 32*((i/4)%2), register (i%4) + 4*(i/8)
     __syncthreads();                        // (over the tiles)
     float *const red = reinterpret_cast<float *>(dsm);
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-        red[(wave * 16 + r) * 64 + lane] = fmaf(acc_rest[r], 1.f / 2048.f, acc_head[r]);
+        red[(wave * 16 + r) * 64 + lane] = sum[r];
     __syncthreads();
     const int n = nw * 32 + j;
     for (int r = wave; r < 16; r += waves) {                  // wave-uniform
@@ -3101,10 +3121,10 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
             if (!add_part(a.acc + at, a.ksplit, total, marked))
                 continue;
             if (marked) {
-                double sum = 0.;                              // (one lane adds up all of K: in 64 bits, or rounding would show)
+                double again = 0.;                            // (one lane adds up all of K: in 64 bits, or rounding would show)
                 for (int k = 0; k < K; ++k)
-                    sum = row_deq_add<S>(a, nw, j, k, m, sum);
-                total = static_cast<float>(sum);
+                    again = row_deq_add<S>(a, nw, j, k, m, again);
+                total = static_cast<float>(again);
             }
         }
         a.out[at] = f2h(a.bias ? total + h2f(a.bias[n]) : total);

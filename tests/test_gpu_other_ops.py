@@ -184,6 +184,30 @@ def test_row_deq_mm_T_of_several_rows(oracle, M, N, K, S, G, L, bias):
     assert int(hip._workspace(8 * M * N, dev).count_nonzero()) == 0
 
 
+@pytest.mark.parametrize("N,K,S,G", [(2048, 800, 2, 128), (4096, 4100, 4, 128), (2048, 12032, 3, 256)])
+def test_row_deq_mm_T_of_several_rows_is_as_exact_as_fp32_sums(N, K, S, G):
+    """The sums before their rounding to fp16: a bias takes all but a rounding's remainder away, and of the columns those count
+    whose remainder is so small (2^-14 of the RMS output) that its own rounding, 2^-25, does not show.  Several rows, K in parts
+    or not, against the row by itself on the lanes launch: exact products, added up in fp32."""
+    import sbvr
+    from sbvr import hip, synth
+    dev = torch.device("cuda:0")
+    bvr, idx, cache = synth.random_encoding(K, N, S, G, 256, seed=N + K)
+    x = torch.randn((1, K), generator=torch.Generator().manual_seed(K)).to(torch.float16)
+    want = _transposed_sums(x.numpy(), bvr.numpy(), idx.numpy(), cache.numpy(), G)[0][0]
+    bias = (-want).astype(np.float16)
+    rest, rms = want + bias.astype(np.float64), np.sqrt(np.mean(want ** 2))
+    near = np.abs(rest) < 2.0 ** -14 * rms
+    assert near.sum() > 200
+    args = [t.to(dev) for t in (bvr, idx, cache, torch.from_numpy(bias))]
+    error = {}
+    for M in (1, 5):
+        y = sbvr._sbvr_row_deq_mm_T(x.to(dev).repeat(M, 1), *args, 0, bvr_len=G).float().cpu().numpy().astype(np.float64)
+        assert hip.row_deq_last()[0] == (hip.ROW_DEQ_LANES if M == 1 else hip.ROW_DEQ_ROWS)
+        error[M] = np.sqrt(np.mean((y - rest)[:, near] ** 2))
+    assert error[5] <= error[1], (error[5] / rms, error[1] / rms)
+
+
 def test_row_deq_mm_T_of_several_rows_with_values_that_are_not_finite(oracle):
     """Infinite and NaN activations, an infinite coefficient and a weight beyond fp16 in the launch of several rows: every
     output is finite, infinite or NaN as in the launch of that row by itself, and the finite ones agree."""
