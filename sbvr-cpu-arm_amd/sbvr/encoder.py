@@ -24,6 +24,7 @@ same lines and selectors.  On a GPU two things differ from the reference's loop
     give the same table, indices and selectors.
 """
 import math
+from numbers import Integral
 
 import torch
 
@@ -353,7 +354,7 @@ class GroupEncoder:
         from . import hip
         c, S, G = self.conf, self.S, self.conf.bvr_len
         if not (flat.is_cuda and flat.is_contiguous() and hip.encoder_candidates_supported(flat.dtype, G, S) and
-                c.cache_warmup_num >= 1 and c.mse_window_size >= 1 and c.s_search_num > 0 and c.extend_ratio > 0 and
+                c.cache_warmup_num >= 1 and c.mse_window_size >= 1 and isinstance(c.mse_window_size, Integral) and c.s_search_num > 0 and c.extend_ratio > 0 and
                 (c.num_coeff_cache_lines == 0 or c.mse_history)):
             return None
         kw = dict(device=flat.device, dtype=flat.dtype)
@@ -398,8 +399,9 @@ class GroupEncoder:
             run.base[wide], run.offsets[wide] = base.data_ptr(), b.data_ptr()
             run.bases[wide], run.n_offsets[wide], run.axis_values[wide] = base.shape[0], b.shape[0], per_dim + 1
         run.scale_step, run.scale_narrow = 1.0 / c.s_search_num, float(torch.tensor(1.0) / torch.tensor(c.extend_ratio, dtype=torch.float32))
-        run.groups, run.G, run.warmup, run.window = n, G, c.cache_warmup_num, c.mse_window_size
-        run.table_lines, run.before, run.acceptable = self.table.shape[0], start, c.acceptable_mse
+        # (a table has fewer lines, and a chunk fewer errors, than the bound; lines < 3.5 is lines < 4)
+        run.warmup, run.window = (math.ceil(min(v, 1 << 30)) for v in (c.cache_warmup_num, c.mse_window_size))
+        run.groups, run.G, run.table_lines, run.before, run.acceptable = n, G, self.table.shape[0], start, c.acceptable_mse
 
         def put(miss):
             missed = c.group_idx - c.cache_hits

@@ -312,3 +312,18 @@ def test_few_rounds_are_queued_behind_a_group_for_the_host(monkeypatch):
     stats = _encode_both_ways(w.to(torch.float16).to("cuda:0"), dict(num_sums=4, bvr_len=128))
     misses = stats["groups"] - stats["cache_hits"]
     assert sum(queued) <= 16 + 4 * misses
+
+
+@pytest.mark.parametrize("more", [
+    {"cache_warmup_num": 3.0}, {"cache_warmup_num": 2.5}, {"cache_warmup_num": np.int64(3)}, {"cache_warmup_num": 10 ** 10}, {"cache_warmup_num": float("inf")},
+    {"mse_window_size": np.int64(2)}, {"mse_window_size": 10 ** 10}, {"acceptable_mse": 0},
+])
+def test_search_options_of_any_kind_of_number(more):
+    """Options that are no plain ints, or larger than 32 bits, on the device as in the block loop."""
+    from sbvr.encoder import EncoderConfig, GroupEncoder
+    dev = torch.device("cuda:0")
+    conf = dict(num_sums=3, bvr_len=64, **more)
+    w = (torch.randn((6, 512), generator=torch.Generator().manual_seed(9)) * 0.02).to(torch.float16).to(dev)
+    enc = GroupEncoder(EncoderConfig(search_batch_size=1 << 24, **conf), torch.float16, dev)
+    assert enc._covered_on_device(w.reshape(-1)) is not None
+    _encode_both_ways(w, conf)
