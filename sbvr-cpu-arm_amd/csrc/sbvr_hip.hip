@@ -2379,6 +2379,9 @@ bool gemm_lut_path_ok(int M, int N, int K, int S, int G)
 // 0.1 or, with several tables, 0.2 more) and 0.2 us a row block, a
 // workgroup 3.6 us beside its steps, a split 3.3 us and 0.33 us per MB of partial results (written, read and cleared).
 // 256 workgroups run at a time, up to 13 % faster where fewer do; beyond that a last turn that is not full counts 0.63.
+// (Fitted to launches whose parts lie in the workspace.  Parts in memory of the call's own need no clearing, which saves 4 to 5 us of
+// 39 to 42, see sbvr_gemm_reduce_kernel; the estimate does not tell the two apart, so that both run the same parts and give the
+// same bits, and the 1 % is the former's.)
 // Against one tile height and parts by powers of two: 87 rows x 5378 columns, K 19456, 3 planes, 181 us unsplit (N no
 // multiple of 4 was never split) -> 37.5; 371 x 890, K 6144, 74.9 -> 23.2; 128 x 6144, K 4096, 30.6 -> 25.7.
 // The partial results take at most kGemmLutMaxParts bytes (384 tiles of 256 x 256): the bindings keep a workspace of the

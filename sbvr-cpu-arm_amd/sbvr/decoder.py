@@ -281,7 +281,9 @@ class SbvrLlamaDecoder:
 
     def generate(self, prompt, new_tokens):
         """Feeds `prompt` (1-D int64 tensor) `prompt_rows` tokens at a time, the rest and
-        the last one by themselves, then decodes `new_tokens` greedily.  Returns (tokens, seconds spent on the new tokens)."""
+        the last one by themselves, then decodes `new_tokens` greedily.  Returns (tokens, seconds spent on the new tokens).
+        `generated` holds what followed each position that a step took; those of the prompt that went through the layers
+        with others, without the head, stay 0."""
         if len(prompt) + new_tokens > self.max_seq:
             raise ValueError("prompt + new tokens exceed the cache length")
         self.reset()

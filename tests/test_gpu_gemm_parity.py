@@ -1,4 +1,4 @@
-"""Prefill path (M > 32: weights decoded to fp16 tiles in LDS, fp16 MFMA) and the 32-row kernel
+"""Prefill path (M > 32: weights decoded to fp16 in registers, fp16 MFMA) and the 32-row kernel
 (weights decoded to fp16 in registers) against the oracle.  Both round each decoded weight to fp16
 (as the reference's decode() does, sbvr/core.py:927-949) and accumulate in fp32; the bar is the
 stated 1e-2 relative on fp16 outputs, and every test names the kernel it expects to have run."""
@@ -17,7 +17,7 @@ def check(y_gpu, yd, yd1, rounding, what):
     """The kernels here round every decoded weight to fp16.  The table look-up forms round it once, as the
     reference's decode() does: against the oracle's sums over such weights (mode 1) they are held to the decode
     kernel's bound (1e-2 relative with a 1 %-of-RMS floor, 2 fp16 ulps of max(|ref|, RMS)).  The arithmetic
-    forms (6 and 8 planes, groups of 32 or 64) build the fp16 sum plane by plane: at most 3e-3 of the RMS
+    forms (groups of 32) build the fp16 sum plane by plane, 6 and 8 planes of two or three entries: at most 3e-3 of the RMS
     output off (2.2e-3 is the largest seen), 1e-2 relative for outputs above 0.3 RMS.  tests/parity.py."""
     return parity.judge(y_gpu.float().cpu().numpy(), yd, yd1, rounding, what)
 
@@ -58,6 +58,9 @@ def run_case(oracle, N, K, S, G, M, L, seed=0, bias=False, expect=None):
         # (the bias is added after the rounding to fp16: judged with the loose bound only)
         yd = yd + b.numpy().astype(np.float64)
         return parity.loose(y.float().cpu().numpy(), yd, f"N={N} K={K} S={S} G={G} M={M} L={L} with bias")
+    # (2 to 4 planes in groups of 64 look their weights up as well, rounded once, though they report the looser of the two)
+    if rounding == parity.ROUNDING_PLANEWISE and S <= 4 and G % 64 == 0:
+        rounding = parity.ROUNDING_DECODE
     check(y, yd, yd1, rounding, f"N={N} K={K} S={S} G={G} M={M} L={L}")
 
 
