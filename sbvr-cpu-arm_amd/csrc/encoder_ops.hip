@@ -770,7 +770,7 @@ sbvr_decode_weight_kernel(const DecodeArgs a)
         load_line_words<S>(a.cache + static_cast<size_t>(line) * S, c);
         LutTables<S> t;
         lut_build_tables<S>(c, t);
-        uint32_t Q[4];
+        Nibbles<S> Q;
         lut_nibble_words<S>(pl.w, Q);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {

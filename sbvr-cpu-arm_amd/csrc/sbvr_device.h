@@ -161,30 +161,68 @@ __device__ __forceinline__ void lut_build_tables(const uint32_t (&c)[(S + 1) / 2
     }
 }
 
-// Nibble words of one word of K: nibble n of Q[p] = selector (one bit per plane) of element p + 4n.
-template <int S>
-__device__ __forceinline__ void lut_nibble_words(const uint32_t (&w)[S], uint32_t (&Q)[4])
+// bits of a where mask is set, of b elsewhere (written out: with a constant mask the compiler takes the expression apart
+// into two ands and an or)
+__device__ __forceinline__ uint32_t bit_select(uint32_t mask, uint32_t a, uint32_t b)
 {
-    auto rotr = [](uint32_t v, int r) __attribute__((always_inline)) -> uint32_t {
-        return (r & 31) == 0 ? v : __builtin_amdgcn_alignbit(v, v, r & 31);
-    };
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        uint32_t v = rotr(w[0], p) & 0x11111111u;
-        v = (rotr(w[1], p - 1) & 0x22222222u) | v;
-        if constexpr (S >= 3)
-            v = (rotr(w[2], p - 2) & 0x44444444u) | v;
-        if constexpr (S == 4)
-            v = (rotr(w[3], p - 3) & 0x88888888u) | v;
-        Q[p] = v;
+    uint32_t r;
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "s"(mask), "v"(a), "v"(b));
+    return r;
+}
+
+// Selector words of one word of K: nibble n of Q[p] holds, in its low min(S, 3) bits, the first planes' bits of element
+// p + 4n (the other bits are anything), and top the fourth plane's word.  Two planes at a time: their bits of the even and of the
+// odd elements side by side, then these pairs next to the third plane's, 13 operations with 3 and 4 planes, 6 with 2.
+template <int S>
+struct Nibbles {
+    uint32_t Q[4], top;
+};
+
+template <int S>
+__device__ __forceinline__ void lut_nibble_pairs(const uint32_t (&w)[S], uint32_t (&pair)[2])
+{
+    pair[0] = bit_select(0x55555555u, w[0], w[1] << 1);
+    pair[1] = bit_select(0x55555555u, w[0] >> 1, w[1]);
+}
+
+template <int S>
+__device__ __forceinline__ void lut_nibble_word(const uint32_t (&w)[S], const uint32_t (&pair)[2], Nibbles<S> &n, int p)
+{
+    const uint32_t two = p < 2 ? pair[p & 1] : pair[p & 1] >> 2;
+    if constexpr (S == 2) {
+        n.Q[p] = two;
+    } else {
+        const uint32_t third = p == 0 ? w[2] << 2 : (p == 1 ? w[2] << 1 : (p == 2 ? w[2] : w[2] >> 1));
+        n.Q[p] = bit_select(0x33333333u, two, third);
     }
+    if constexpr (S == 4)
+        n.top = w[3];
+}
+
+template <int S>
+__device__ __forceinline__ void lut_nibble_words(const uint32_t (&w)[S], Nibbles<S> &n)
+{
+    uint32_t pair[2];
+    lut_nibble_pairs<S>(w, pair);
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+        lut_nibble_word<S>(w, pair, n, p);
+}
+
+// The selector of v_perm_b32 that takes byte b of its first operand where the fourth plane has element p + 8b, of its
+// second elsewhere.
+__device__ __forceinline__ uint32_t lut_halves(const Nibbles<4> &n, int p)
+{
+    uint32_t low = 0x03020100u;
+    asm("" : "+v"(low));                 // (in a register: with both constants literal, and and or are two operations)
+    return ((p < 2 ? n.top << (2 - p) : n.top >> (p - 2)) & 0x04040404u) | low;
 }
 
 // The weights of elements p, p + 8 (w01) and p + 16, p + 24 (w23) of the word, p = 0..7, as packed fp16 pairs.
 template <int S>
-__device__ __forceinline__ void lut_look_up(const LutTables<S> &t, const uint32_t (&Q)[4], int p, uint32_t &w01, uint32_t &w23)
+__device__ __forceinline__ void lut_look_up(const LutTables<S> &t, const Nibbles<S> &n, int p, uint32_t &w01, uint32_t &w23)
 {
-    const uint32_t qs = p < 4 ? Q[p & 3] : Q[p & 3] >> 4;
+    const uint32_t qs = p < 4 ? n.Q[p & 3] : n.Q[p & 3] >> 4;
     const uint32_t sel = qs & (S == 2 ? 0x03030303u : 0x07070707u);
     uint32_t lo, hi;
     if constexpr (S == 2) {
@@ -195,11 +233,10 @@ __device__ __forceinline__ void lut_look_up(const LutTables<S> &t, const uint32_
         hi = __builtin_amdgcn_perm(t.hi[1], t.hi[0], sel);
     }
     if constexpr (S == 4) {
-        // bytes of ones where selector bit 3 is set: a look-up in the two-entry table {0x00, 0xff}
-        const uint32_t upper = __builtin_amdgcn_perm(0x0000ff00u, 0x0000ff00u, (qs >> 3) & 0x01010101u);
-        const uint32_t lo_u = __builtin_amdgcn_perm(t.lo[3], t.lo[2], sel), hi_u = __builtin_amdgcn_perm(t.hi[3], t.hi[2], sel);
-        lo = (lo_u & upper) | (lo & ~upper);
-        hi = (hi_u & upper) | (hi & ~upper);
+        // byte b of the upper half's look-up where the fourth plane has element p + 8b, of the lower half's elsewhere
+        const uint32_t half = lut_halves(n, p);
+        lo = __builtin_amdgcn_perm(__builtin_amdgcn_perm(t.lo[3], t.lo[2], sel), lo, half);
+        hi = __builtin_amdgcn_perm(__builtin_amdgcn_perm(t.hi[3], t.hi[2], sel), hi, half);
     }
     w01 = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
     w23 = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
@@ -207,11 +244,11 @@ __device__ __forceinline__ void lut_look_up(const LutTables<S> &t, const uint32_
 
 // The B operand of MFMA q = 0..3 of the word: elements 2q, 2q+8, 2q+16, 2q+24, 2q+1, 2q+9, 2q+17, 2q+25.
 template <int S>
-__device__ __forceinline__ v4u lut_operand(const LutTables<S> &t, const uint32_t (&Q)[4], int q)
+__device__ __forceinline__ v4u lut_operand(const LutTables<S> &t, const Nibbles<S> &n, int q)
 {
     uint32_t b0, b1, b2, b3;
-    lut_look_up<S>(t, Q, 2 * q, b0, b1);
-    lut_look_up<S>(t, Q, 2 * q + 1, b2, b3);
+    lut_look_up<S>(t, n, 2 * q, b0, b1);
+    lut_look_up<S>(t, n, 2 * q + 1, b2, b3);
     return v4u{b0, b1, b2, b3};
 }
 
@@ -228,7 +265,8 @@ struct WeightTables {
 
 template <int S>
 struct WeightNibbles {
-    uint32_t Q[WeightTables<S>::halves][4], last[4];
+    Nibbles<WeightTables<S>::H> t[WeightTables<S>::halves];
+    Nibbles<2> last;
 };
 
 template <int S>
@@ -251,11 +289,11 @@ template <int S>
 __device__ __forceinline__ void weight_nibbles(const uint32_t (&w)[S], WeightNibbles<S> &n)
 {
     if constexpr (S <= 4) {
-        lut_nibble_words<S>(w, n.Q[0]);
+        lut_nibble_words<S>(w, n.t[0]);
     } else {
         const uint32_t first[3] = {w[0], w[1], w[2]}, second[3] = {w[3], w[4], w[5]};
-        lut_nibble_words<3>(first, n.Q[0]);
-        lut_nibble_words<3>(second, n.Q[1]);
+        lut_nibble_words<3>(first, n.t[0]);
+        lut_nibble_words<3>(second, n.t[1]);
         if constexpr (S == 8) {
             const uint32_t third[2] = {w[6], w[7]};
             lut_nibble_words<2>(third, n.last);
@@ -267,7 +305,7 @@ __device__ __forceinline__ void weight_nibbles(const uint32_t (&w)[S], WeightNib
 template <int S>
 __device__ __forceinline__ v4u weight_operand(const WeightTables<S> &t, const WeightNibbles<S> &n, int q)
 {
-    v4u r = lut_operand<WeightTables<S>::H>(t.t[0], n.Q[0], q);
+    v4u r = lut_operand<WeightTables<S>::H>(t.t[0], n.t[0], q);
     // (a line's coefficients grow in magnitude: the largest entries come last, so that one addition rounds at the sum's size)
     auto add = [&](const v4u &u) __attribute__((always_inline)) {
 #pragma unroll
@@ -275,7 +313,7 @@ __device__ __forceinline__ v4u weight_operand(const WeightTables<S> &t, const We
             r[i] = __builtin_bit_cast(uint32_t, as_v2h(r[i]) + as_v2h(u[i]));
     };
     if constexpr (S > 4)
-        add(lut_operand<3>(t.t[1], n.Q[1], q));
+        add(lut_operand<3>(t.t[1], n.t[1], q));
     if constexpr (S == 8)
         add(lut_operand<2>(t.last, n.last, q));
     return r;

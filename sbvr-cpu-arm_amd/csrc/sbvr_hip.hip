@@ -1862,12 +1862,12 @@ hipError_t launch_rows32(int S, RowsArgs a, hipStream_t st)
 // (each the fp32 sum rounded to fp16 once, as the reference's decode() rounds a weight) and keeps
 // them as byte tables: the low bytes of entries 0..3, 4..7, ... and the high bytes likewise.  A lane owns a
 // whole word of K per step (half h of the wave takes word 2i + h of the word pair i).  Its plane words are
-// merged into four "nibble words" Q_p, p = 0..3: nibble n of Q_p is the S-bit selector of element p + 4n, at
-// the cost of a rotate and an and-or per plane and p.  Then (Q_p >> 0 or 4) & 0x07070707 is four selectors in
-// four bytes, for elements p (+ 4), + 8, + 16, + 24, i.e. a ready v_perm_b32 selector into the byte tables:
-// two permutes fetch the low and the high bytes of four weights (four permutes and two bit-field inserts
-// with 16 entries, where selector bit 3 chooses between the table halves), two more interleave them into
-// packed fp16 pairs.  About 4 VALU operations per weight against 7.5 for the arithmetic decode.
+// merged into four "nibble words" Q_p, p = 0..3: nibble n of Q_p is the selector of element p + 4n in the first
+// three planes (lut_nibble_words: two planes' bits side by side, the third next to them).  Then (Q_p >> 0 or 4) & 0x07070707 is
+// four selectors in four bytes, for elements p (+ 4), + 8, + 16, + 24, i.e. a ready v_perm_b32 selector into the byte
+// tables: two permutes fetch the low and the high bytes of four weights (six with 16 entries, where the fourth plane's bits
+// choose between the table halves), two more interleave them into packed fp16 pairs.  About 3.3 VALU operations per weight
+// against 7.5 for the arithmetic decode.
 // The k order inside an MFMA follows from that: elements 2q, 2q+8, 2q+16, 2q+24, 2q+1, 2q+9, 2q+17, 2q+25 of
 // the lane's word for MFMA q = 0..3 of a step; the activations (the lane's batch row, the same 32 elements:
 // 64 bytes, four loads) are put into that order with four permutes per MFMA.
@@ -2133,7 +2133,7 @@ hipError_t launch_rows32_lut(int S, RowsArgs a, hipStream_t st)
 // 32w .. 32w+31 for all its rows (8 row blocks: 128 accumulator registers a lane).  Per step of 64 elements
 // of K a lane (column j, half h) decodes its word 2i + h of column j by table look-up straight into the B operands
 // of four MFMAs (16 registers), and the wave runs them against the row blocks: 4 RB MFMAs of 32 clocks per 32
-// weights decoded per lane (about 170 VALU instructions a step).
+// weights decoded per lane (about 150 VALU instructions a step).
 // The activations of a step, 32 RB rows x 64 elements, are shared by the 8 waves through LDS, stored in the element
 // order the MFMAs want (see sbvr_gemm_rows32_lut_kernel: that permutation is done once, by the thread that
 // brings a (row, word) in, not once per wave): rows 144 bytes apart, two buffers, one barrier per step.  The loads
@@ -3031,7 +3031,7 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
         __builtin_amdgcn_sched_barrier(0);
         // -- decode: rows 128 t + 2 lane and + 1, 32 columns each
         LutTables<S> head[2], rest[2];
-        uint32_t Q[2][4];
+        Nibbles<S> Q[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             build_split_tables<S>(c[e], head[e], rest[e]);
