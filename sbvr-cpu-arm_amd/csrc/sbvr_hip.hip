@@ -1570,25 +1570,6 @@ hipError_t launch_batch(int S, const GemvArgs &a, const BatchPlan &p, hipStream_
 
 constexpr int kGemmBK = 64;          // elements of K a step of the prefill kernel takes
 
-struct GemmArgs {
-    const uint16_t *x;
-    const uint32_t *bvr;
-    const void *idx;
-    const uint16_t *cache;
-    const uint16_t *bias;
-    uint16_t *out;
-    int M, N, K, L;
-    int steps_per_group;   // G / 64
-    int idx16;
-    int ksplit;            // workgroups along K (blockIdx.z); 1: results go straight to out
-    int part_steps;        // steps of 64 along K of a part (the last one's may be fewer)
-    float *part;           // ksplit > 1: (ksplit, M, N) fp32 partial results, all zero between launches
-};
-
-// Floats from one part's partial results to the next's: M * N, and up to a multiple of 4, so that every part starts on
-// 16 bytes and the second pass takes four outputs at a time whatever N is.
-__host__ __device__ inline size_t part_floats(int M, int N) { return (static_cast<size_t>(M) * N + 3) & ~static_cast<size_t>(3); }
-
 // The S fp16 coefficients of one table line as packed pairs, in as few load instructions as the
 // line's alignment allows (a line starts at a multiple of 2*S bytes; the table is 16-byte aligned).
 template <int S>
@@ -2129,8 +2110,8 @@ hipError_t launch_rows32_lut(int S, RowsArgs a, hipStream_t st)
 
 // ------------------------------------------- MFMA prefill with the weights decoded by table look-up
 //
-// A dense contraction with the decode of sbvr_gemm_rows32_lut_kernel.  A workgroup of 8 waves owns RB row blocks of 32 x 256 columns of the output; wave w owns columns
-// 32w .. 32w+31 for all its rows (8 row blocks: 128 accumulator registers a lane).  Per step of 64 elements
+// A dense contraction with the decode of sbvr_gemm_rows32_lut_kernel.  A workgroup of 8 waves owns RB row blocks of 32 x 256
+// columns of the output; wave w owns columns 32w .. 32w+31 for all its rows.  Per step of 64 elements
 // of K a lane (column j, half h) decodes its word 2i + h of column j by table look-up straight into the B operands
 // of four MFMAs (16 registers), and the wave runs them against the row blocks: 4 RB MFMAs of 32 clocks per 32
 // weights decoded per lane (about 150 VALU instructions a step).
@@ -2146,22 +2127,22 @@ hipError_t launch_rows32_lut(int S, RowsArgs a, hipStream_t st)
 // chip exactly (256 x 14336, K 4096: 61.4 and 62.3).
 constexpr int kPfWaves = 8, kPfBN = 256, kPfRow = 144;
 
-constexpr int pf_loader_blocks(int rb) { return rb <= 2 ? 2 : (rb <= 4 ? 4 : 8); }
+constexpr int pf_loader_blocks(int rb) { return rb <= 2 ? 2 : 4; }
 
-// RB: row blocks of 32 of a workgroup (2 to 8).  The matrix pipe and the decode take turns, so an MFMA of a row
-// block beyond M costs as much as one inside it: the rows are shared out evenly over the tiles (gemm_lut_plan).
-// With 2, 4, 6 and 8 row blocks a step takes 0.94, 1.36, 1.84 and 2.08 us (8192 -> 28672, 4 planes); 64 / 128 / 192 /
-// 333 rows 60 / 87 / 118 / 198 us there, where 8 row blocks for any number of rows took 131 / 133 / 139 / 248.
+// RB: row blocks of 32 of a workgroup, 2 to 4 here; prefill_ops.hip's kernel takes 5 to 8.  An MFMA of a row block beyond M
+// costs as much as one inside it: the rows are shared out evenly over the tiles (gemm_lut_plan).  With 2 and 4 row blocks the
+// vector ALU has more to do than the matrix pipe and bounds the step (0.94 and 1.36 us, 8192 -> 28672, 4 planes), and a
+// step laid out by hand as there is no faster: 512 rows x 4096, K 8192, 4 row blocks, 8 planes 67 us here and 71 so, 4 planes 54.5 and 56.6.
 // kShare: groups of a multiple of 128 elements, the two steps of a loop iteration share a coefficient line; otherwise each
 // has its own index load, gather and table, and the number of steps may be odd.
 template <int S, int RB, bool kShare>
 __global__ void __launch_bounds__(64 * kPfWaves)
 sbvr_gemm_lut_kernel(const GemmArgs a)
 {
-    static_assert(RB >= 2 && RB <= 8, "row blocks of a workgroup");
-    // of the four MFMA operands of a (row, word), a thread brings in NQ (1 or 2 where 512 threads then cover the rows)
+    static_assert(RB >= 2 && RB <= 4, "row blocks of a workgroup");
+    // of the four MFMA operands of a (row, word), a thread brings in NQ (1 or 2: 512 threads cover the rows)
     constexpr int NQ = pf_loader_blocks(RB) / 2;
-    constexpr int kTile = 32 * pf_loader_blocks(RB) * kPfRow;       // (all rows the threads cover: 3 row blocks 128, 5 to 7 256)
+    constexpr int kTile = 32 * pf_loader_blocks(RB) * kPfRow;       // (all rows the threads cover: 3 row blocks 128)
     struct Part {
         uint32_t w[4 * NQ];                                          // dword c * NQ + q: dword q0 + q of 16-byte chunk c
     };
@@ -2206,10 +2187,7 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
         const uint16_t *xp = xsrc + 64 * min(ip, p_last);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            if constexpr (NQ == 4) {
-                const v4u v = *reinterpret_cast<const v4u *>(xp + 8 * c);
-                x.w[4 * c] = v.x; x.w[4 * c + 1] = v.y; x.w[4 * c + 2] = v.z; x.w[4 * c + 3] = v.w;
-            } else if constexpr (NQ == 2) {
+            if constexpr (NQ == 2) {
                 const v2u v = *reinterpret_cast<const v2u *>(xp + 8 * c);
                 x.w[2 * c] = v.x; x.w[2 * c + 1] = v.y;
             } else {
@@ -2247,32 +2225,27 @@ sbvr_gemm_lut_kernel(const GemmArgs a)
         weight_nibbles<S>(w, nibbles);
         auto operand = [&](int q) __attribute__((always_inline)) -> v4u { return weight_operand<S>(tables, nibbles, q); };
         // MFMA q of all row blocks in a row (RB different accumulators), its RB activation operands read while
-        // MFMA q - 1 runs, and the look-ups of operand q + 1 in the shadow of the matrix pipe.  (Two sets of RB operands;
-        // 8 row blocks of 6 or 8 planes go in two turns of 4 per MFMA, or the registers do not suffice)
-        constexpr int RG = RB == 8 && S > 4 ? 4 : RB, turns = RB / RG;
+        // MFMA q - 1 runs, and the look-ups of operand q + 1 in the shadow of the matrix pipe
         const unsigned char *xt = xrd + buf * kTile;
-        v4u A[2][RG];
-        auto read_a = [&](int i, v4u (&dst)[RG]) __attribute__((always_inline)) {
+        v4u A[2][RB];
+        auto read_a = [&](int q, v4u (&dst)[RB]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int rb = 0; rb < RG; ++rb)
-                dst[rb] = *reinterpret_cast<const v4u *>(xt + 32 * (i % turns * RG + rb) * kPfRow + 16 * (i / turns));
+            for (int rb = 0; rb < RB; ++rb)
+                dst[rb] = *reinterpret_cast<const v4u *>(xt + 32 * rb * kPfRow + 16 * q);
         };
         read_a(0, A[0]);
         v4u Bq = operand(0), Bn = Bq;
 #pragma unroll
-        for (int i = 0; i < 4 * turns; ++i) {
-            if (i < 4 * turns - 1) {
-                read_a(i + 1, A[(i + 1) & 1]);
+        for (int q = 0; q < 4; ++q) {
+            if (q < 3) {
+                read_a(q + 1, A[(q + 1) & 1]);
                 __builtin_amdgcn_sched_barrier(0);
+                Bn = operand(q + 1);
             }
-            if (i % turns == 0 && i / turns < 3)
-                Bn = operand(i / turns + 1);
 #pragma unroll
-            for (int rb = 0; rb < RG; ++rb)
-                acc[i % turns * RG + rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, A[i & 1][rb]), __builtin_bit_cast(v8h, Bq),
-                                                                                  acc[i % turns * RG + rb], 0, 0, 0);
-            if (i % turns == turns - 1)
-                Bq = Bn;
+            for (int rb = 0; rb < RB; ++rb)
+                acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, A[q & 1][rb]), __builtin_bit_cast(v8h, Bq), acc[rb], 0, 0, 0);
+            Bq = Bn;
         }
     };
 
@@ -2459,11 +2432,7 @@ hipError_t launch_gemm_lut_rows(int rb, dim3 grid, const GemmArgs &a, hipStream_
     switch (rb) {
     case 2: return launch_gemm_lut_inst<S, 2, kShare>(grid, a, st);
     case 3: return launch_gemm_lut_inst<S, 3, kShare>(grid, a, st);
-    case 4: return launch_gemm_lut_inst<S, 4, kShare>(grid, a, st);
-    case 5: return launch_gemm_lut_inst<S, 5, kShare>(grid, a, st);
-    case 6: return launch_gemm_lut_inst<S, 6, kShare>(grid, a, st);
-    case 7: return launch_gemm_lut_inst<S, 7, kShare>(grid, a, st);
-    default: return launch_gemm_lut_inst<S, 8, kShare>(grid, a, st);
+    default: return launch_gemm_lut_inst<S, 4, kShare>(grid, a, st);
     }
 }
 
@@ -2472,6 +2441,8 @@ hipError_t launch_gemm_lut(int S, int rb, const GemmArgs &a, hipStream_t st)
     const dim3 grid(static_cast<unsigned>((a.N + kPfBN - 1) / kPfBN), static_cast<unsigned>((a.M + 32 * rb - 1) / (32 * rb)),
                     static_cast<unsigned>(a.ksplit));
     const bool share = a.steps_per_group % 2 == 0;
+    if (rb > 4)
+        return launch_gemm_lut_pipelined(S, rb, a, st);
     switch (S) {
     case 4: return share ? launch_gemm_lut_rows<4, true>(rb, grid, a, st) : launch_gemm_lut_rows<4, false>(rb, grid, a, st);
 #ifndef SBVR_FAST_BUILD

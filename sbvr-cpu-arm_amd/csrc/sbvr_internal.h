@@ -24,4 +24,27 @@ struct MmArgs {
 bool mm_T_mfma_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r_bvr, const void *r_cache);
 hipError_t launch_mm_T_mfma(int Sr, int G, MmArgs a, int cus, hipStream_t st);
 
+// The prefill kernels (sbvr_hip.hip, prefill_ops.hip).
+struct GemmArgs {
+    const uint16_t *x;
+    const uint32_t *bvr;
+    const void *idx;
+    const uint16_t *cache;
+    const uint16_t *bias;
+    uint16_t *out;
+    int M, N, K, L;
+    int steps_per_group;   // G / 64
+    int idx16;
+    int ksplit;            // workgroups along K (blockIdx.z); 1: results go straight to out
+    int part_steps;        // steps of 64 along K of a part (the last one's may be fewer)
+    float *part;           // ksplit > 1: (ksplit, M, N) fp32 partial results, all zero between launches
+};
+
+// Floats from one part's partial results to the next's: M * N, and up to a multiple of 4, so that every part starts on
+// 16 bytes and the second pass takes four outputs at a time whatever N is.
+__host__ __device__ inline size_t part_floats(int M, int N) { return (static_cast<size_t>(M) * N + 3) & ~static_cast<size_t>(3); }
+
+// Five to eight row blocks of 32 a workgroup (prefill_ops.hip).
+hipError_t launch_gemm_lut_pipelined(int S, int rb, const GemmArgs &a, hipStream_t st);
+
 #endif
