@@ -170,9 +170,14 @@ struct EncoderState {
     int uncovered;                       // written by the search for the settling launch behind it: the group is the host's
     unsigned long long found;            // error's bits << 32 | candidate: the least so far (all ones: none)
 };
+struct EncoderStates {
+    EncoderState slot[2];
+    int covered[2];                      // of either slot: groups below it have met every line of the table
+};
 
 constexpr int kEncMaxScales = 160, kEncMaxAxes = 4096;    // scales of a search, values of all its axes, at most
-constexpr int kEncSettleValues = 4096;                    // squared distances of a workgroup's groups in LDS
+constexpr int kEncSettleValues = 1024;                    // squared distances of a workgroup's groups in LDS (of one, where it is longer)
+constexpr int kEncWindow = 2048;                          // groups that meet the table in one go
 constexpr int kEncNone = 0x7fffffff;
 
 // torch.linspace in fp16: the step rounded, values from either end.
@@ -186,6 +191,45 @@ __device__ __forceinline__ _Float16 line_space(_Float16 lo, _Float16 hi, int n, 
                      : fma_half(-s, static_cast<float>(n - 1 - i), static_cast<float>(hi));
 }
 
+// The scales of a group's search (GroupEncoder.candidate_lines): from, from + step, ...
+struct Scales {
+    float from, step;
+    double count;
+    int wide;
+};
+
+__device__ __forceinline__ Scales search_scales(const sbvr_hip_encoder_run &a, const EncoderState &st, float q95, _Float16 hl, _Float16 hh)
+{
+#pragma clang fp contract(off)
+    Scales r;
+    // hits so far over groups so far, this one counted: above 0.6 (and while the table fills) the wider search
+    const double seen = static_cast<double>(a.before) + st.miss;
+    r.wide = st.lines < a.warmup || (seen - st.misses) / (seen + 1.) > 0.6;
+    const _Float16 s_hi = fma_half(static_cast<float>(static_cast<_Float16>(hh - hl)), 1.1f, 0.f);
+    const float s_lo = 2.f * q95;
+    r.step = (static_cast<float>(s_hi) - s_lo) * a.scale_step;
+    if (r.wide)
+        r.step = r.step * a.scale_narrow;
+    r.from = s_lo + r.step;
+    const float to = static_cast<float>(s_hi) + r.step;
+    r.count = ceil((static_cast<double>(to) - static_cast<double>(r.from)) / static_cast<double>(r.step));
+    if (!(fabsf(to) < INFINITY))
+        r.count = 0.;
+    return r;
+}
+
+// Value i of axis q: from a margin below the data's edge q to one above edge q + 1.
+template <int S>
+__device__ __forceinline__ _Float16 axis_value(_Float16 hl, _Float16 hh, int steps, int q, int i, bool &finite)
+{
+#pragma clang fp contract(off)
+    const _Float16 e0 = line_space(hl, hh, S + 1, q), e1 = line_space(hl, hh, S + 1, q + 1);
+    const _Float16 margin = fma_half(fabsf(static_cast<float>(e0)), 0.8f, 0.f);
+    const _Float16 a0 = e0 - margin, a1 = e1 + margin;
+    finite = finite && fabsf(static_cast<float>(a0)) < INFINITY && fabsf(static_cast<float>(a1)) < INFINITY;
+    return line_space(a0, a1, steps, i);
+}
+
 struct SearchSpace {
     _Float16 scales[kEncMaxScales], axes[kEncMaxAxes];
     uint16_t group[kEncMaxG];
@@ -193,19 +237,20 @@ struct SearchSpace {
     int scales_n, extended, covered;
 };
 
-// The bounds of the candidates of group m (GroupEncoder.candidate_lines): its scales and axes into LDS, by the whole workgroup.
+// The bounds of the candidates of group m: its scales and axes into LDS, by the whole workgroup.
 template <int S>
 __device__ __forceinline__ void make_search_space(const sbvr_hip_encoder_run &a, const EncoderState &st, SearchSpace &sp)
 {
 #pragma clang fp contract(off)
     const int tid = threadIdx.x, m = st.miss;
-    const _Float16 *mine = static_cast<const _Float16 *>(a.data) + static_cast<size_t>(m) * a.G;
+    const uint16_t *mine = static_cast<const uint16_t *>(a.data) + static_cast<size_t>(m) * a.G;
+    const float q95 = a.q95[m], mean = a.mean[m];                      // (asked for with the values, not behind the barrier)
     float lo = INFINITY, hi = -INFINITY;
     for (int i = tid; i < a.G; i += kEncThreads) {
-        const _Float16 v = mine[i];
-        sp.group[i] = __builtin_bit_cast(uint16_t, v);
-        lo = fminf(lo, static_cast<float>(v));
-        hi = fmaxf(hi, static_cast<float>(v));
+        const uint16_t v = mine[i];
+        sp.group[i] = v;
+        lo = fminf(lo, h2f(v));
+        hi = fmaxf(hi, h2f(v));
     }
     for (int d = 32; d >= 1; d >>= 1) {
         lo = fminf(lo, __shfl_xor(lo, d, 64));
@@ -220,51 +265,62 @@ __device__ __forceinline__ void make_search_space(const sbvr_hip_encoder_run &a,
         lo = fminf(lo, sp.red[0][w]);
         hi = fmaxf(hi, sp.red[1][w]);
     }
-    // hits so far over groups so far, this one counted: above 0.6 (and while the table fills) the wider search
-    const double seen = static_cast<double>(a.before) + m;
-    const bool wide = st.lines < a.warmup || (seen - st.misses) / (seen + 1.) > 0.6;
     const _Float16 hl = static_cast<_Float16>(lo), hh = static_cast<_Float16>(hi);
-    const _Float16 s_hi = fma_half(static_cast<float>(static_cast<_Float16>(hh - hl)), 1.1f, 0.f);
-    const float s_lo = 2.f * a.q95[m];
-    float step = (static_cast<float>(s_hi) - s_lo) * a.scale_step;
-    if (wide)
-        step = step * a.scale_narrow;
-    const float from = s_lo + step, to = static_cast<float>(s_hi) + step;
-    const double count = ceil((static_cast<double>(to) - static_cast<double>(from)) / static_cast<double>(step));
-    const int steps = a.axis_values[wide];
-    bool covered = fabsf(a.mean[m]) * 2.f / S < 0.28f && step != 0.f && count > 0. && count <= kEncMaxScales && st.lines < a.table_lines &&
-                   fabsf(from) < INFINITY && fabsf(to) < INFINITY && fabsf(lo) < INFINITY && fabsf(hi) < INFINITY;
-    const int n = covered ? static_cast<int>(count) : 0;
+    const Scales scales = search_scales(a, st, q95, hl, hh);
+    const int steps = a.axis_values[scales.wide];
+    bool covered = fabsf(mean) * 2.f / S < 0.28f && scales.step != 0.f && scales.count > 0. && scales.count <= kEncMaxScales &&
+                   st.lines < a.table_lines && fabsf(scales.from) < INFINITY && fabsf(lo) < INFINITY && fabsf(hi) < INFINITY;
+    const int n = covered ? static_cast<int>(scales.count) : 0;
     for (int i = tid; i < n; i += kEncThreads)
-        sp.scales[i] = fma_half(step, static_cast<float>(i), from);
-    // axis q: from a margin below the data's edge q to one above edge q + 1
+        sp.scales[i] = fma_half(scales.step, static_cast<float>(i), scales.from);
     bool finite = true;
-    for (int i = tid; i < S * steps; i += kEncThreads) {
-        const int q = i / steps;
-        const _Float16 e0 = line_space(hl, hh, S + 1, q), e1 = line_space(hl, hh, S + 1, q + 1);
-        const _Float16 margin = fma_half(fabsf(static_cast<float>(e0)), 0.8f, 0.f);
-        const _Float16 a0 = e0 - margin, a1 = e1 + margin;
-        finite = finite && fabsf(static_cast<float>(a0)) < INFINITY && fabsf(static_cast<float>(a1)) < INFINITY;
-        sp.axes[i] = line_space(a0, a1, steps, i % steps);
-    }
+    for (int i = tid; i < S * steps; i += kEncThreads)
+        sp.axes[i] = axis_value<S>(hl, hh, steps, i / steps, i % steps, finite);
     covered = __syncthreads_and(covered && finite);
     if (tid == 0) {
         sp.scales_n = n;
-        sp.extended = wide;
+        sp.extended = scales.wide;
         sp.covered = covered;
     }
     __syncthreads();
 }
 
-// Candidate `at` (see sbvr_encoder_candidates_kernel for the order).
-template <int S>
-__device__ __forceinline__ void form_candidate(const sbvr_hip_encoder_run &a, const SearchSpace &sp, int at, _Float16 (&c)[S])
+// Quotient and remainder of numbers below 2^24 by a divisor that many share: a product, corrected.
+struct Divider {
+    uint32_t by;
+    float reciprocal;
+    __device__ __forceinline__ explicit Divider(int d) : by(static_cast<uint32_t>(d)), reciprocal(1.f / static_cast<float>(d)) {}
+    __device__ __forceinline__ int operator()(int &x) const        // returns the quotient, leaves the remainder
+    {
+        int q = static_cast<int>(static_cast<float>(x) * reciprocal), rest = x - static_cast<int>(__umul24(static_cast<uint32_t>(q), by));
+        q += rest < 0 ? -1 : (rest >= static_cast<int>(by) ? 1 : 0);
+        rest += rest < 0 ? static_cast<int>(by) : (rest >= static_cast<int>(by) ? -static_cast<int>(by) : 0);
+        x = rest;
+        return q;
+    }
+};
+
+struct Dividers {
+    Divider bases, scales, steps;
+};
+
+// Candidate `at` (see sbvr_encoder_candidates_kernel for the order).  kSmall: there are fewer than 2^24.
+template <int S, bool kSmall>
+__device__ __forceinline__ void form_candidate(const sbvr_hip_encoder_run &a, const SearchSpace &sp, const Dividers &by, int family, int at,
+                                               _Float16 (&c)[S])
 {
 #pragma clang fp contract(off)
-    const int wide = sp.extended, bases = a.bases[wide], family = bases * a.n_offsets[wide] * sp.scales_n, steps = a.axis_values[wide];
-    const _Float16 *base = static_cast<const _Float16 *>(a.base[wide]), *offsets = static_cast<const _Float16 *>(a.offsets[wide]);
+    auto divide = [](int &x, const Divider &d) __attribute__((always_inline)) -> int {
+        if constexpr (kSmall)
+            return d(x);
+        const int q = x / static_cast<int>(d.by);
+        x -= q * static_cast<int>(d.by);
+        return q;
+    };
+    const int wide = sp.extended, steps = static_cast<int>(by.steps.by);
     if (at < family) {
-        const int ir = at % bases, is = at / bases % sp.scales_n, ib = at / bases / sp.scales_n;
+        const _Float16 *base = static_cast<const _Float16 *>(a.base[wide]), *offsets = static_cast<const _Float16 *>(a.offsets[wide]);
+        int ir = at, is = divide(ir, by.bases), ib = divide(is, by.scales);
         const _Float16 sv = sp.scales[is], bv = offsets[ib];
 #pragma unroll
         for (int q = 0; q < S; ++q) {
@@ -275,8 +331,9 @@ __device__ __forceinline__ void form_candidate(const sbvr_hip_encoder_run &a, co
         int rest = at - family;
 #pragma unroll
         for (int q = S - 1; q >= 0; --q) {
-            c[q] = sp.axes[q * steps + rest % steps];
-            rest /= steps;
+            int i = rest;
+            rest = divide(i, by.steps);
+            c[q] = sp.axes[q * steps + i];
         }
     }
 }
@@ -298,19 +355,23 @@ __device__ __forceinline__ void subset_sums(const _Float16 (&c)[S], v2h (&p)[1 <
         p[j] = v2h{static_cast<_Float16>(sums[2 * j]), static_cast<_Float16>(sums[2 * j + 1])};
 }
 
-// The least squared distance of a value to the points: fp16 difference, fp16 square.
+// The least squared distance of a value to the points: fp16 difference, fp16 square, and a packed minimum of three (which
+// gives NaN for NaN: the values are finite here, and the points' sums at most infinite).  With v_pk_min_f16 four operations more of 25.
 template <int S>
 __device__ __forceinline__ float least_square(uint16_t raw, const v2h (&p)[1 << (S - 1)])
 {
 #pragma clang fp contract(off)
     const _Float16 d = __builtin_bit_cast(_Float16, raw);
     const v2h dd = {d, d};
-    v2h best;
-#pragma unroll
-    for (int j = 0; j < (1 << (S - 1)); ++j) {
+    auto square = [&](int j) __attribute__((always_inline)) -> v2h {
         const v2h diff = dd - p[j];
-        const v2h sq = diff * diff;
-        best = j == 0 ? sq : __builtin_elementwise_min(best, sq);
+        return diff * diff;
+    };
+    v2h best = __builtin_elementwise_min(square(0), square(1));
+#pragma unroll
+    for (int j = 2; j < (1 << (S - 1)); j += 2) {
+        const v2h one = square(j), two = square(j + 1);
+        asm("v_pk_minimum3_f16 %0, %0, %1, %2" : "+v"(best) : "v"(one), "v"(two));
     }
     return static_cast<float>(best[0] < best[1] ? best[0] : best[1]);
 }
@@ -345,43 +406,27 @@ __device__ __forceinline__ void write_selectors(const uint16_t *group, int G, co
     }
 }
 
-template <int S>
-__global__ void __launch_bounds__(kEncThreads)
-sbvr_encoder_search_kernel(const sbvr_hip_encoder_run a, int slot)
+template <int S, bool kSmall>
+__device__ __forceinline__ void search_candidates(const sbvr_hip_encoder_run &a, const SearchSpace &sp, float known,
+                                                  unsigned long long *found, unsigned long long *least)
 {
-    __shared__ __align__(16) SearchSpace sp;
-    __shared__ unsigned long long least[kEncThreads / 64];
-    EncoderState *const states = static_cast<EncoderState *>(a.state);
-    const EncoderState st = states[slot];
-    const bool idle = st.status != 0 || st.miss >= a.groups;
-    const int tid = threadIdx.x;
-    if (!idle)
-        make_search_space<S>(a, st, sp);
-    if (blockIdx.x == 0 && tid == 0) {
-        // the other slot: what the settling launch finds there before it takes minima
-        const bool stays = idle || !sp.covered;
-        states[slot ^ 1].miss = stays ? st.miss : kEncNone;
-        states[slot ^ 1].found = ~0ull;
-        states[slot ^ 1].uncovered = !idle && !sp.covered;
-    }
-    if (idle || !sp.covered)
-        return;
-    const int wide = sp.extended, steps = a.axis_values[wide];
-    int n = a.bases[wide] * a.n_offsets[wide] * sp.scales_n, grid = 1;
+    const int tid = threadIdx.x, wide = sp.extended;
+    const int family = a.bases[wide] * a.n_offsets[wide] * sp.scales_n;
+    const Dividers by{Divider(a.bases[wide]), Divider(sp.scales_n), Divider(a.axis_values[wide])};
+    int n = family, grid = 1;
 #pragma unroll
     for (int q = 0; q < S; ++q)
-        grid *= steps;
+        grid *= a.axis_values[wide];
     n += grid;
-    const float known = st.lines < a.warmup ? INFINITY : a.best[st.miss];
     // (more lines than the launch has threads, which the host's bound on the scales rules out, would go round again)
     for (int first = blockIdx.x * kEncThreads; first < n; first += gridDim.x * kEncThreads) {
         const int line = first + tid, at = min(line, n - 1);
         _Float16 c[S];
-        form_candidate<S>(a, sp, at, c);
+        form_candidate<S, kSmall>(a, sp, by, family, at, c);
         v2h p[1 << (S - 1)];
         subset_sums<S>(c, p);
         // no candidate above the best error known counts; the margin covers the division by G
-        const unsigned long long now = __hip_atomic_load(&states[slot].found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long now = __hip_atomic_load(found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const float bound = now == ~0ull ? known : fminf(known, __uint_as_float(static_cast<uint32_t>(now >> 32)));
         const float limit = bound * static_cast<float>(a.G) * 1.000001f;
         float sum = 0.f;
@@ -392,7 +437,7 @@ sbvr_encoder_search_kernel(const sbvr_hip_encoder_run a, int slot)
             sum += least_square<S>(static_cast<uint16_t>(four.x >> 16), p);
             sum += least_square<S>(static_cast<uint16_t>(four.y), p);
             sum += least_square<S>(static_cast<uint16_t>(four.y >> 16), p);
-            if ((g & 12) == 12 && __all(sum > limit))
+            if (((g & 4) || g < 16) && __all(sum > limit))
                 break;
         }
         const float mse = sum / static_cast<float>(a.G);
@@ -410,7 +455,175 @@ sbvr_encoder_search_kernel(const sbvr_hip_encoder_run a, int slot)
             for (int w = 1; w < kEncThreads / 64; ++w)
                 key = least[w] < key ? least[w] : key;
             if (key != ~0ull)
-                atomicMin(&states[slot].found, key);
+                atomicMin(found, key);
+        }
+    }
+}
+
+template <int S>
+__global__ void __launch_bounds__(kEncThreads)
+sbvr_encoder_search_kernel(const sbvr_hip_encoder_run a, int slot)
+{
+    __shared__ __align__(16) SearchSpace sp;
+    __shared__ unsigned long long least[kEncThreads / 64];
+    EncoderState *const states = static_cast<EncoderStates *>(a.state)->slot;
+    const EncoderState st = states[slot];
+    const int have_met = static_cast<EncoderStates *>(a.state)->covered[slot];
+    const bool idle = st.status != 0 || st.miss >= have_met, extends = st.status == 0 && idle && have_met < a.groups;
+    const int tid = threadIdx.x;
+    const float known = idle || st.lines < a.warmup ? INFINITY : a.best[st.miss];
+    if (!idle)
+        make_search_space<S>(a, st, sp);
+    if (blockIdx.x == 0 && tid == 0) {
+        // the other slot: what the settling launch finds there before it takes minima
+        const bool stays = idle ? !extends : !sp.covered;
+        states[slot ^ 1].miss = stays ? st.miss : kEncNone;
+        states[slot ^ 1].found = ~0ull;
+        states[slot ^ 1].uncovered = !idle && !sp.covered;
+    }
+    if (idle || !sp.covered)
+        return;
+    const int wide = sp.extended;
+    long lines = static_cast<long>(a.bases[wide]) * a.n_offsets[wide] * sp.scales_n, grid = 1;
+#pragma unroll
+    for (int q = 0; q < S; ++q)
+        grid *= a.axis_values[wide];
+    if (lines + grid < (1 << 24))
+        search_candidates<S, true>(a, sp, known, &states[slot].found, least);
+    else
+        search_candidates<S, false>(a, sp, known, &states[slot].found, least);
+}
+
+// The cut-off over the last errors, added up in the host's order; `last`: one that is not in the history yet.
+__device__ __forceinline__ double cut_off(const sbvr_hip_encoder_run &a, int history, bool with_last, double last, double *part)
+{
+#pragma clang fp contract(off)
+    const int len = min(history, a.window), from = history - len;
+    double sum = 0.;
+    for (int i0 = 0; i0 < len; i0 += kEncThreads) {
+        __syncthreads();
+        const int i = i0 + static_cast<int>(threadIdx.x);
+        if (i < len)
+            part[threadIdx.x] = with_last && from + i == history - 1 ? last : a.history[from + i];
+        __syncthreads();
+        for (int k = 0; k < min(kEncThreads, len - i0); ++k)
+            sum += part[k];
+    }
+    const double cutoff = sum / len * 0.99;
+    return cutoff < a.acceptable ? a.acceptable : cutoff;
+}
+
+// The winner of the search of group m = st.miss, its coefficients by magnitude, equal ones in their order.  Every wave works
+// it out for itself.
+template <int S>
+__device__ __forceinline__ void winner(const sbvr_hip_encoder_run &a, const EncoderState &st, _Float16 (&c)[S])
+{
+#pragma clang fp contract(off)
+    const uint16_t *mine = static_cast<const uint16_t *>(a.data) + static_cast<size_t>(st.miss) * a.G;
+    const float q95 = a.q95[st.miss];
+    float lo = INFINITY, hi = -INFINITY;
+    for (int i = threadIdx.x & 63; i < a.G; i += 64) {
+        lo = fminf(lo, h2f(mine[i]));
+        hi = fmaxf(hi, h2f(mine[i]));
+    }
+    for (int d = 32; d >= 1; d >>= 1) {
+        lo = fminf(lo, __shfl_xor(lo, d, 64));
+        hi = fmaxf(hi, __shfl_xor(hi, d, 64));
+    }
+    const _Float16 hl = static_cast<_Float16>(lo), hh = static_cast<_Float16>(hi);
+    const Scales scales = search_scales(a, st, q95, hl, hh);
+    const int wide = scales.wide, bases = a.bases[wide], steps = a.axis_values[wide], n = static_cast<int>(scales.count);
+    const int family = bases * a.n_offsets[wide] * n, at = static_cast<int>(st.found & 0xffffffffu);
+    _Float16 raw[S];
+    if (at < family) {
+        const _Float16 *base = static_cast<const _Float16 *>(a.base[wide]) + static_cast<size_t>(at % bases) * S;
+        const _Float16 sv = fma_half(scales.step, static_cast<float>(at / bases % n), scales.from);
+        const _Float16 bv = static_cast<const _Float16 *>(a.offsets[wide])[at / bases / n];
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            const _Float16 scaled = sv * base[q];
+            raw[q] = bv + scaled;
+        }
+    } else {
+        int rest = at - family;
+        bool finite = true;
+#pragma unroll
+        for (int q = S - 1; q >= 0; --q) {
+            raw[q] = axis_value<S>(hl, hh, steps, q, rest % steps, finite);
+            rest /= steps;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+        int rank = 0;
+#pragma unroll
+        for (int o = 0; o < S; ++o) {
+            const float vo = fabsf(static_cast<float>(raw[o])), vq = fabsf(static_cast<float>(raw[q]));
+            rank += vo < vq || (vo == vq && o < q);
+        }
+#pragma unroll
+        for (int o = 0; o < S; ++o)
+            c[o] = rank == o ? raw[q] : c[o];
+    }
+}
+
+// The next groups meet the whole table: a workgroup a group, a thread every 256th line; the least error and the first line
+// that has it.
+template <int S>
+__device__ __forceinline__ void meet_table(const sbvr_hip_encoder_run &a, const EncoderState &st, int have_met, EncoderState *other,
+                                           int *other_met, uint16_t *group, unsigned long long *least, double *part)
+{
+    const int tid = threadIdx.x, end = min(a.groups, have_met + kEncWindow);
+    const bool looks = st.lines >= a.warmup;
+    const double cutoff = looks ? cut_off(a, st.history, false, 0., part) : 0.;
+    if (blockIdx.x == 0 && tid == 0) {
+        other->lines = st.lines;
+        other->misses = st.misses;
+        other->history = st.history;
+        other->status = 0;
+        *other_met = end;
+        atomicMin(&other->miss, looks ? end : have_met);
+    }
+    for (int g = have_met + static_cast<int>(blockIdx.x); g < end; g += static_cast<int>(gridDim.x)) {
+        __syncthreads();
+        for (int i = tid; i < a.G; i += kEncThreads)
+            group[i] = static_cast<const uint16_t *>(a.data)[static_cast<size_t>(g) * a.G + i];
+        __syncthreads();
+        unsigned long long key = (static_cast<unsigned long long>(__float_as_uint(INFINITY)) << 32) | 0xffffffffu;
+        for (int l = tid; l < st.lines; l += kEncThreads) {
+            _Float16 c[S];
+#pragma unroll
+            for (int q = 0; q < S; ++q)
+                c[q] = static_cast<const _Float16 *>(a.table)[static_cast<size_t>(l) * S + q];
+            v2h p[1 << (S - 1)];
+            subset_sums<S>(c, p);
+            float sum = 0.f;
+            for (int i = 0; i < a.G; i += 4) {
+                const uint2 four = *reinterpret_cast<const uint2 *>(group + i);
+                sum += least_square<S>(static_cast<uint16_t>(four.x), p);
+                sum += least_square<S>(static_cast<uint16_t>(four.x >> 16), p);
+                sum += least_square<S>(static_cast<uint16_t>(four.y), p);
+                sum += least_square<S>(static_cast<uint16_t>(four.y >> 16), p);
+            }
+            const float mse = sum / static_cast<float>(a.G);
+            if (mse < __uint_as_float(static_cast<uint32_t>(key >> 32)))
+                key = (static_cast<unsigned long long>(__float_as_uint(mse)) << 32) | static_cast<uint32_t>(l);
+        }
+        for (int d = 32; d >= 1; d >>= 1) {
+            const unsigned long long o = __shfl_xor(key, d, 64);
+            key = o < key ? o : key;
+        }
+        if ((tid & 63) == 0)
+            least[tid >> 6] = key;
+        __syncthreads();
+        if (tid == 0) {
+            for (int w = 1; w < kEncThreads / 64; ++w)
+                key = least[w] < key ? least[w] : key;
+            const float best = __uint_as_float(static_cast<uint32_t>(key >> 32));
+            a.best[g] = best;
+            a.line[g] = static_cast<int>(static_cast<uint32_t>(key));      // (-1 without a line)
+            if (looks && !(static_cast<double>(best) < cutoff))
+                atomicMin(&other->miss, g);
         }
     }
 }
@@ -421,48 +634,45 @@ sbvr_encoder_settle_kernel(const sbvr_hip_encoder_run a, int slot)
 {
 #pragma clang fp contract(off)
     __shared__ __align__(16) union {
-        SearchSpace sp;
-        float squares[kEncSettleValues + 64];
+        uint16_t group[kEncMaxG];
+        float squares[kEncMaxG + 64];
     } sh;
+    __shared__ double part[kEncThreads];
+    __shared__ unsigned long long least[kEncThreads / 64];
     __shared__ int twin, first_miss;
-    EncoderState *const states = static_cast<EncoderState *>(a.state);
-    const EncoderState st = states[slot];
+    EncoderStates *const both = static_cast<EncoderStates *>(a.state);
+    EncoderState *const other = &both->slot[slot ^ 1];
+    const EncoderState st = both->slot[slot];
+    const int have_met = both->covered[slot];
     const int tid = threadIdx.x, m = st.miss;
     _Float16 *const table = static_cast<_Float16 *>(a.table);
+    if (st.status == 0 && m >= have_met && have_met < a.groups) {
+        meet_table<S>(a, st, have_met, other, &both->covered[slot ^ 1], sh.group, least, part);
+        return;
+    }
     EncoderState next = st;                                            // (miss and found: written by the search and by minima)
     const bool found = st.found != ~0ull;
     // (nothing left, a group for the host, or one that neither the table nor any candidate has an error for: the state stays)
-    const bool uncovered = states[slot ^ 1].uncovered != 0;            // (no workgroup of this launch writes it)
+    const bool uncovered = other->uncovered != 0;                      // (no workgroup of this launch writes it)
     const bool stays = st.status != 0 || m >= a.groups || uncovered, unserved = !stays && !found && a.line[m] < 0;
     if (stays || unserved) {
         if (blockIdx.x == 0 && tid == 0) {
-            states[slot ^ 1].lines = st.lines;
-            states[slot ^ 1].misses = st.misses;
-            states[slot ^ 1].history = st.history;
-            states[slot ^ 1].status = unserved || uncovered ? 1 : st.status;
+            other->lines = st.lines;
+            other->misses = st.misses;
+            other->history = st.history;
+            both->covered[slot ^ 1] = have_met;
+            other->status = unserved || uncovered ? 1 : st.status;
             if (unserved)
-                atomicMin(&states[slot ^ 1].miss, m);
+                atomicMin(&other->miss, m);
         }
         return;
     }
-    make_search_space<S>(a, st, sh.sp);
+    const int per = max(1, kEncSettleValues / a.G), stride = a.G + 4;
+    if (blockIdx.x > 0 && m + 1 + static_cast<int>(blockIdx.x) * per >= have_met)      // (nothing to show the line to; warming up or not)
+        return;
     _Float16 c[S];
     if (found) {
-        _Float16 raw[S];
-        form_candidate<S>(a, sh.sp, static_cast<int>(st.found & 0xffffffffu), raw);
-        // coefficients by magnitude, equal ones in their order
-#pragma unroll
-        for (int q = 0; q < S; ++q) {
-            int rank = 0;
-#pragma unroll
-            for (int o = 0; o < S; ++o) {
-                const float vo = fabsf(static_cast<float>(raw[o])), vq = fabsf(static_cast<float>(raw[q]));
-                rank += vo < vq || (vo == vq && o < q);
-            }
-#pragma unroll
-            for (int o = 0; o < S; ++o)
-                c[o] = rank == o ? raw[q] : c[o];
-        }
+        winner<S>(a, st, c);
     } else {
         const _Float16 *have = table + static_cast<size_t>(a.line[m]) * S;
 #pragma unroll
@@ -497,18 +707,9 @@ sbvr_encoder_settle_kernel(const sbvr_hip_encoder_run a, int slot)
     next.lines = st.lines + joins;
     next.misses = st.misses + 1;
     next.history = st.history + found;
-    // the cut-off over the last errors, in the order the host adds them up
-    double cutoff = 0.;
-    {
-        const int len = min(next.history, a.window);
-        double sum = 0.;
-        for (int i = next.history - len; i < next.history; ++i)
-            sum += found && i == st.history ? error : a.history[i];
-        cutoff = sum / len * 0.99;
-        cutoff = cutoff < a.acceptable ? a.acceptable : cutoff;
-    }
+    const double cutoff = cut_off(a, next.history, found, error, part);
     if (blockIdx.x == 0) {
-        write_selectors<S>(sh.sp.group, a.G, c, a.sel + static_cast<size_t>(m) * a.G);
+        write_selectors<S>(static_cast<const uint16_t *>(a.data) + static_cast<size_t>(m) * a.G, a.G, c, a.sel + static_cast<size_t>(m) * a.G);
         if (tid == 0) {
             a.line_of[m] = chosen;
             a.settled[m] = 1;
@@ -518,13 +719,13 @@ sbvr_encoder_settle_kernel(const sbvr_hip_encoder_run a, int slot)
                     table[static_cast<size_t>(st.lines) * S + q] = c[q];
             if (found)
                 a.history[st.history] = error;
-            states[slot ^ 1].lines = next.lines;
-            states[slot ^ 1].misses = next.misses;
-            states[slot ^ 1].history = next.history;
-            states[slot ^ 1].status = 0;
+            other->lines = next.lines;
+            other->misses = next.misses;
+            other->history = next.history;
+            both->covered[slot ^ 1] = have_met;
+            other->status = 0;
             // (groups are searched one after the other until the table has its first lines)
-            if (next.lines < a.warmup || m + 1 >= a.groups)
-                atomicMin(&states[slot ^ 1].miss, m + 1);
+            atomicMin(&other->miss, next.lines < a.warmup ? m + 1 : have_met);
         }
     }
     const bool looks = next.lines >= a.warmup;
@@ -532,9 +733,8 @@ sbvr_encoder_settle_kernel(const sbvr_hip_encoder_run a, int slot)
         return;
     v2h p[1 << (S - 1)];
     subset_sums<S>(c, p);
-    const int per = max(1, min(16, kEncSettleValues / a.G)), stride = a.G + 1;
-    for (int g0 = m + 1 + static_cast<int>(blockIdx.x) * per; g0 < a.groups; g0 += static_cast<int>(gridDim.x) * per) {
-        const int many = min(per, a.groups - g0);
+    for (int g0 = m + 1 + static_cast<int>(blockIdx.x) * per; g0 < have_met; g0 += static_cast<int>(gridDim.x) * per) {
+        const int many = min(per, have_met - g0);
         __syncthreads();
         if (tid == 0)
             first_miss = kEncNone;
@@ -548,8 +748,13 @@ sbvr_encoder_settle_kernel(const sbvr_hip_encoder_run a, int slot)
             if (joins) {
                 float sum = 0.f;
 #pragma unroll 8
-                for (int i = 0; i < a.G; ++i)
-                    sum += sh.squares[tid * stride + i];
+                for (int i = 0; i < a.G; i += 4) {                     // (element order)
+                    const v4f four = *reinterpret_cast<const v4f *>(sh.squares + tid * stride + i);
+                    sum += four.x;
+                    sum += four.y;
+                    sum += four.z;
+                    sum += four.w;
+                }
                 const float mse = sum / static_cast<float>(a.G);
                 if (mse < best) {
                     best = mse;
@@ -562,7 +767,7 @@ sbvr_encoder_settle_kernel(const sbvr_hip_encoder_run a, int slot)
         }
         __syncthreads();
         if (tid == 0 && first_miss != kEncNone)
-            atomicMin(&states[slot ^ 1].miss, first_miss);
+            atomicMin(&other->miss, first_miss);
     }
 }
 
@@ -592,8 +797,9 @@ sbvr_encoder_selectors_kernel(const sbvr_hip_encoder_run a, int first, int group
 template <int S>
 void launch_rounds(const sbvr_hip_encoder_run &a, unsigned search_grid, int slot, int rounds, hipStream_t st)
 {
-    const int per = max(1, min(16, kEncSettleValues / a.G));
-    const unsigned settle_grid = static_cast<unsigned>(max(1, min((a.groups + per - 1) / per, 2048)));
+    // (a workgroup for two groups that meet the table; showing them one line takes a quarter of these: with 1024 at work on that
+    // it took 13 to 16 us, 8 so)
+    const unsigned settle_grid = static_cast<unsigned>(max(1, (min(a.groups, kEncWindow) + 1) / 2));
     for (int r = 0; r < rounds; ++r) {
         hipLaunchKernelGGL(sbvr_encoder_search_kernel<S>, dim3(search_grid), dim3(kEncThreads), 0, st, a, (slot + r) & 1);
         hipLaunchKernelGGL(sbvr_encoder_settle_kernel<S>, dim3(settle_grid), dim3(kEncThreads), 0, st, a, (slot + r) & 1);
@@ -933,7 +1139,7 @@ int sbvr_hip_encoder_candidates_f16(const void *data, int G, const void *base, i
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-size_t sbvr_hip_encoder_state_bytes(void) { return 2 * sizeof(EncoderState); }
+size_t sbvr_hip_encoder_state_bytes(void) { return sizeof(EncoderStates); }
 
 int sbvr_hip_encoder_scales(int S, int G, int bases, int n_offsets, int axis_values)
 {

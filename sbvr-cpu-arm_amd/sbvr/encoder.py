@@ -377,7 +377,7 @@ class GroupEncoder:
         from . import hip
         c, S, dev = self.conf, self.S, datas.device
         n, G = datas.shape
-        start, known = c.group_idx, c.num_coeff_cache_lines
+        start = c.group_idx
         flat32 = datas.float()
         stats = torch.stack((torch.quantile(flat32, 0.95, dim=1) if n * G < 1 << 24 else
                              torch.cat([torch.quantile(p, 0.95, dim=1) for p in flat32.split(max(1, (1 << 23) // G))]),
@@ -388,8 +388,6 @@ class GroupEncoder:
         history = torch.zeros(len(c.mse_history) + n, dtype=torch.float64, device=dev)
         if c.mse_history:
             history[:len(c.mse_history)] = torch.tensor(c.mse_history, dtype=torch.float64)
-        if known:
-            self._look_up(datas, 0, 0, best, line)
         state = torch.zeros(hip.encoder_state_words(), dtype=torch.int32, device=dev)
         run = hip.EncoderRun()
         run.data, run.q95, run.mean, run.table = datas.data_ptr(), stats[0].data_ptr(), stats[1].data_ptr(), self.table.data_ptr()
@@ -403,26 +401,27 @@ class GroupEncoder:
         run.warmup, run.window = (math.ceil(min(v, 1 << 30)) for v in (c.cache_warmup_num, c.mse_window_size))
         run.groups, run.G, run.table_lines, run.before, run.acceptable = n, G, self.table.shape[0], start, c.acceptable_mse
 
-        def put(miss):
+        # (groups below `covered` have met the whole table, and one that misses is looked for among them; the kernels take it on)
+        def put(miss, covered):
             missed = c.group_idx - c.cache_hits
-            state.copy_(torch.tensor([c.num_coeff_cache_lines, missed, len(c.mse_history), 0, miss, 0, -1, -1] * 2, dtype=torch.int32))
+            state.copy_(torch.tensor([c.num_coeff_cache_lines, missed, len(c.mse_history), 0, miss, 0, -1, -1] * 2 + [covered] * 2,
+                                     dtype=torch.int32))
 
-        def next_miss(first):
+        def next_miss(first, covered):
             if c.num_coeff_cache_lines < c.cache_warmup_num:
                 return first
-            missing = (~(best[first:].double() < self._cutoff())).nonzero()
-            return first + int(missing[0]) if missing.numel() else n
+            missing = (~(best[first:covered].double() < self._cutoff())).nonzero()
+            return first + int(missing[0]) if missing.numel() else covered
 
-        miss = next_miss(0)
-        c.group_idx, c.cache_hits = start + miss, c.cache_hits + miss
-        put(miss)
+        miss = 0
+        put(0, 0 if c.num_coeff_cache_lines else 1)                         # (an empty table has nothing to meet)
         shown, rounds = 0, 16
         while miss < n:
             hip.encoder_rounds(run, S, max(lines), 0, rounds, dev)          # (an even number: the result is in slot 0 again)
             had = len(c.mse_history)
-            now = state[:5].tolist()
-            c.num_coeff_cache_lines, missed, errors, status, miss = now
-            miss = min(miss, n)                                             # (above n: none misses any more)
+            now = state.tolist()
+            c.num_coeff_cache_lines, missed, errors, status, miss = now[:5]
+            covered = now[-2]
             c.mse_history.extend(history[had:errors].tolist())
             c.group_idx, c.cache_hits = start + miss, start + miss - missed
             if progress is not None:
@@ -433,11 +432,11 @@ class GroupEncoder:
                 found, s = self.encode_group(datas[miss])
                 line_of[miss], sel[miss * G:(miss + 1) * G], settled[miss] = found, s, 1
                 history[errors:len(c.mse_history)] = torch.tensor(c.mse_history[errors:], dtype=torch.float64)
-                if miss + 1 < n and c.num_coeff_cache_lines > known:
-                    self._look_up(datas, miss + 1, known, best, line)
-                miss = next_miss(miss + 1)
+                if miss + 1 < covered and c.num_coeff_cache_lines > known:
+                    self._look_up(datas[:covered], miss + 1, known, best, line)
+                miss = next_miss(miss + 1, covered)
                 c.group_idx, c.cache_hits = start + miss, c.cache_hits + miss - (c.group_idx - start)
-                put(miss)
+                put(miss, covered)
                 rounds = 2                          # (groups like this one, or a table that is full, may follow each other)
             else:
                 rounds = min(64, 2 * rounds)
@@ -468,7 +467,7 @@ class GroupEncoder:
         if block is None:
             covered = self._covered_on_device(flat)
             if covered is not None:
-                # (65536 groups at a time: every new line meets all of those behind it in one launch)
+                # (65536 groups at a time)
                 datas, span = flat.view(-1, c.bvr_len), 1 << 16
                 for lo in range(0, datas.shape[0], span):
                     part = datas[lo:lo + span]
