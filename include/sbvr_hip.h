@@ -282,7 +282,7 @@ size_t sbvr_hip_row_deq_mm_T_workspace_for(int M, int N, int K, int S, int G);
 #define SBVR_HIP_ROW_DEQ_PORTABLE 1      /* one thread per output */
 #define SBVR_HIP_ROW_DEQ_LANES 2         /* lanes along K */
 #define SBVR_HIP_ROW_DEQ_MFMA 3          /* row by row, plane sums on the matrix cores */
-#define SBVR_HIP_ROW_DEQ_ROWS 4          /* several rows, every weight decoded once */
+#define SBVR_HIP_ROW_DEQ_ROWS 4          /* several rows together: every weight decoded once, or (2 to 4) plane bits as they are */
 int sbvr_hip_row_deq_last_kernel(void);
 int sbvr_hip_row_deq_last_parts(void);
 

@@ -2852,7 +2852,7 @@ sbvr_row_deq_mfma_kernel(const uint16_t *__restrict__ x, const uint32_t *__restr
 // reading 16 columns meet different banks) and come back as the B operands of eight v_mfma_f32_32x32x16_f16 each, with the
 // batch rows, read from memory as they are, as A.  A workgroup owns 32 columns and 32 batch rows; its waves
 // take the tiles of K in turn and meet in LDS, and K is split across workgroups through the 64-bit accumulators.
-// Bound by the vector ALU: 731 operations a tile and wave with 4 planes (308 of them permutes), whatever the
+// Bound by the vector ALU: 640 operations a tile and wave with 4 planes, half of them permutes, whatever the
 // number of rows, where the kernels above take 384 per 64 k and row or an A image per row.  Four waves a workgroup and one
 // tile each, so that three workgroups share a CU (two tiles a wave and eight waves: 8 rows x 12032, K 4853 45 us, 34 so).
 constexpr int kDeqRowsWaves = 4, kDeqTile = 32 * 272;         // bytes of a tile
@@ -3105,6 +3105,247 @@ sbvr_row_deq_rows_kernel(const RowDeqArgs a)
     }
 }
 
+// Two to four rows (2 to 4 planes, groups of a multiple of 64 columns, hence an even number of column words): no weight is decoded at all.  The coefficient line of a
+// row k is the same for all columns of a group, so the coefficients go to the activations, z_j[m, k] = x[m, k] c_j, and the
+// product is plane bits times z.  A word of this layout is one row k of 32 columns, and the bits an MFMA wants along K lie
+// across rows: a first MFMA turns them.  v_mfma_f32_16x16x128_f8f6f4 takes the words of 64 rows as they lie (fp4 nibbles, five
+// operations a word) against an identity that picks 16 of the columns; its four blocks of 32 elements are four rows' words,
+// weighted 2^5, 2^6, 2^21 and 2^22 by their block scales and added to 2^23, so that a result's low mantissa bits are the four
+// rows' bits (exactly: tried for all of them), and one `and` leaves two of them as a pair of fp16 numbers, 2^-19 or 2^-18 each:
+// the B operand of v_mfma_f32_16x16x32_f16 for 32 rows k.  The A rows are z in three fp16 parts (22 bits, the product exactly), scaled
+// per tile by the row's largest activation and the tile's largest coefficient: rows 0 to 3 multiples of 2^-11 of the bound,
+// whose sums over a tile are exact, rows 4 to 7 multiples of 2^-22 of what is left, with exact sums too, rows 8 to 11 the rest.
+// (Rounded values and what is left of them, two parts, added up with the roundings of the MFMAs: sums were 1.7e-7 of the RMS
+// output off 64 bits where fp32 sums of exact products are 0.95e-7.)  A workgroup owns two column words and a part of K; its waves take two words x four tiles of 128 k at a time, and
+// the two waves of a tile make its A image together, a row each.  Bound by latency and the vector ALU: about 300 operations a
+// tile of 32 columns x 128 k and 60 a row, where decoding it takes 640 (us, that and this: 3 rows x 4096, K 4096 11.1 and
+// 9.1; 3 x 14336, K 4096 29.6 and 21.3; 4 x 8192, K 8192 29.3 and 25.6).
+constexpr int kFewWords = 2, kFewTiles = 4, kFewRows = 4;
+constexpr int kFewPlane = 4 * 4 * 272;      // bytes of a plane's A image: 4 MFMAs x 4 lane groups x (16 rows of 16 bytes, and 16: no bank conflicts)
+// wave_umax of two 16-bit numbers in one
+__device__ __forceinline__ uint32_t wave_umax_pair(uint32_t v)
+{
+    typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+    auto most = [](uint32_t p, uint32_t q) __attribute__((always_inline)) -> uint32_t {
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(v2us, p), __builtin_bit_cast(v2us, q)));
+    };
+    v = most(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xB1, 0xF, 0xF, true)));
+    v = most(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, true)));
+    v = most(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xF, 0xF, true)));
+    v = most(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x140, 0xF, 0xF, true)));
+    v = most(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), 16, 64)));
+    v = most(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), 32, 64)));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+
+template <int S>
+__global__ void __launch_bounds__(64 * kFewWords * kFewTiles)
+__attribute__((amdgpu_waves_per_eu(4, 8)))
+sbvr_row_deq_few_kernel(const RowDeqArgs a)
+{
+    extern __shared__ __align__(16) unsigned char dsm[];
+    constexpr int CW = (S + 1) / 2, kImage = S * kFewPlane;
+    const int lane = threadIdx.x & 63, col = lane & 15, blk = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), groups = static_cast<int>(blockDim.x) / (64 * kFewWords);
+    const int which = wave % kFewWords, group = wave / kFewWords;
+    const int M = a.M, N = a.N, K = a.K;
+    const int nw0 = kFewWords * blockIdx.x, nw = nw0 + which;
+    const int tiles = (K + 127) / 128;
+    const int t_begin = blockIdx.z * a.per_part, t_end = min(tiles, t_begin + a.per_part);
+    const uint32_t *const words = a.bvr + static_cast<size_t>(nw) * K * S;
+    const size_t ibase = static_cast<size_t>((nw0 * 32) / a.G) * K;
+    unsigned char *const image = dsm + group * kImage;
+    float *const scales = reinterpret_cast<float *>(dsm + groups * kImage) + group * kFewRows;
+
+    // rows k of the tile that this lane makes operands of, and where they go: MFMA 2 hf + p, lane group q, dword r
+    const int k_mine = 64 * (lane >> 5) + (lane & 31), p_mine = blk & 1;
+    unsigned char *const put = image + (2 * (lane >> 5) + p_mine) * (4 * 272) + ((lane >> 2) & 3) * 272 + (lane & 3) * 4;
+    const unsigned char *const get = image + blk * 272 + col * 16;
+
+    // the identity's columns 16 half + col (bit 4 q + t is nibble q of dword t, as 0.5, 1, 2 or 2), and the blocks' weights
+    v8i identity[2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+            identity[half][t] = t < 4 && (col & 3) == t ? (t == 0 ? 4 : (t == 1 ? 2 : 1)) << (4 * (4 * half + (col >> 2))) : 0;
+    const int weight = 127 + (blk == 0 ? 5 : (blk == 1 ? 6 : (blk == 2 ? 21 : 22)));
+    const float coarse = p_mine ? 1.5f * 67108864.f : 1.5f * 134217728.f, fine = p_mine ? 1.5f * 32768.f : 1.5f * 65536.f;      // 1.5 x 2^27 and 2^16
+    const v4f origin = {8388608.f, 8388608.f, 8388608.f, 8388608.f};
+
+    struct Stage {
+        Planes<S> w[2];
+        int lo[2], hi[2];
+        uint16_t x[kFewRows / 2][2];
+    };
+    auto load = [&](int t, Stage &s) __attribute__((always_inline)) {
+        const uint8_t *ib = static_cast<const uint8_t *>(a.idx);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            s.w[e] = load_planes<S>(words + static_cast<size_t>(min(128 * t + 64 * e + lane, K - 1)) * S);
+            const int k = min(128 * t + k_mine + 32 * e, K - 1);
+            const size_t at = (ibase + static_cast<size_t>(k)) << a.idx16;
+            s.lo[e] = ib[at];
+            s.hi[e] = ib[at + a.idx16];
+#pragma unroll
+            for (int i = 0; i < kFewRows / 2; ++i)
+                if (2 * i + which < M)                          // (wave-uniform)
+                    s.x[i][e] = a.x[static_cast<size_t>(2 * i + which) * K + k];
+        }
+    };
+    auto gather = [&](const Stage &s, uint32_t (&c)[2][CW]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int line = min(a.idx16 ? s.lo[e] | (s.hi[e] << 8) : s.lo[e], a.L - 1);
+            load_line_words<S>(a.cache + static_cast<size_t>(line) * S, c[e]);
+        }
+    };
+
+    v4f acc[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+    Stage now;
+    uint32_t c[2][CW];
+    if (t_begin + group < t_end) {                                   // wave-uniform
+        load(t_begin + group, now);
+        gather(now, c);
+    }
+    for (int t0 = t_begin; t0 < t_end; t0 += groups) {               // (the same for the whole workgroup)
+        const int t = t0 + group;
+        const bool mine = t < t_end;                                 // wave-uniform
+        if (mine) {
+            // -- this wave's planes of the tile's A image
+            float cf[2][S];
+            uint32_t most = 0;
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int j = 0; j < S; ++j) {
+                    const uint32_t bits = j & 1 ? c[e][j / 2] >> 16 : c[e][j / 2] & 0xffffu;
+                    most = max(most, bits & 0x7fffu);
+                    cf[e][j] = h2f(static_cast<uint16_t>(bits));
+                }
+            const int ec = static_cast<int>(wave_umax(most) >> 10);
+            // its rows of the tile's A image: which and which + 2
+            if (which < M) {
+                uint32_t xs[kFewRows / 2][2], peak = 0;
+#pragma unroll
+                for (int i = 0; i < kFewRows / 2; ++i) {
+                    // (past the end of K: zeros)
+                    xs[i][0] = 128 * t + k_mine < K ? now.x[i][0] : 0u;
+                    xs[i][1] = 128 * t + k_mine + 32 < K ? now.x[i][1] : 0u;
+                    peak |= max(xs[i][0] & 0x7fffu, xs[i][1] & 0x7fffu) << (16 * i);
+                }
+                peak = wave_umax_pair(peak);
+#pragma unroll
+                for (int i = 0; i < kFewRows / 2; ++i) {
+                    const int row = 2 * i + which;
+                    if (row >= M)                                    // (wave-uniform)
+                        break;
+                    // |x| < 2^(ex - 14), |c| < 2^(ec - 14): products below 2^15
+                    const int ex = static_cast<int>((peak >> (16 * i)) & 0xffffu) >> 10, up = 43 - ex - ec;
+                    const float by = __uint_as_float(static_cast<uint32_t>(127 + up - p_mine) << 23);
+                    const float f0 = h2f(static_cast<uint16_t>(xs[i][0])) * by, f1 = h2f(static_cast<uint16_t>(xs[i][1])) * by;
+                    if (lane == 0)
+                        scales[row] = __uint_as_float(static_cast<uint32_t>(127 + 19 - up) << 23);
+#pragma unroll
+                    for (int j = 0; j < S; ++j) {
+                        // multiples of 2^4 and of 2^-7 (a large number added and taken away), and what is left
+                        const float z[2] = {f0 * cf[0][j], f1 * cf[1][j]};
+                        v2h parts[3];
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) {
+                            const float first = z[e] + coarse - coarse, left = z[e] - first, second = left + fine - fine;
+                            parts[0][e] = static_cast<_Float16>(first);
+                            parts[1][e] = static_cast<_Float16>(second);
+                            parts[2][e] = static_cast<_Float16>(left - second);
+                        }
+#pragma unroll
+                        for (int part = 0; part < 3; ++part)
+                            *reinterpret_cast<uint32_t *>(put + j * kFewPlane + (4 * part + row) * 16) = __builtin_bit_cast(uint32_t, parts[part]);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        Stage next;
+        load(min(t + groups, tiles - 1), next);
+        __builtin_amdgcn_sched_barrier(0);
+        if (mine) {
+            v4f D[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int j = 0; j < S; ++j) {
+#pragma unroll
+                for (int hf = 0; hf < 2; ++hf) {
+                    const uint32_t w = now.w[hf].w[j];
+                    const v8i rows = {static_cast<int>(w & 0x11111111u), static_cast<int>(w & 0x22222222u), static_cast<int>(w & 0x44444444u),
+                                      static_cast<int>((w >> 1) & 0x44444444u), 0, 0, 0, 0};
+                    v4f turned[2];
+#pragma unroll
+                    for (int half = 0; half < 2; ++half)
+                        turned[half] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(rows, identity[half], origin, 4, 4, 0, 127, 0, weight);
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) {
+                        const v8h A = __builtin_bit_cast(v8h, *reinterpret_cast<const v4u *>(get + j * kFewPlane + (2 * hf + p) * (4 * 272)));
+#pragma unroll
+                        for (int half = 0; half < 2; ++half) {
+                            v4u B;
+#pragma unroll
+                            for (int r = 0; r < 4; ++r)
+                                B[r] = __float_as_uint(turned[half][r]) & (p ? 0x00400040u : 0x00200020u);
+                            D[half] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, __builtin_bit_cast(v8h, B), D[half], 0, 0, 0);
+                        }
+                    }
+                }
+                if (j == (S - 1) / 2)
+                    gather(next, c);
+            }
+            const v4f scale = *reinterpret_cast<const v4f *>(scales);
+#pragma unroll
+            for (int half = 0; half < 2; ++half)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[half][i] = fmaf(D[half][i], scale[i], acc[half][i]);
+            now = next;
+        }
+        __syncthreads();
+    }
+    // ---- partial results meet in LDS: row i's parts in lane groups 0, 1 and 2 (rows past M: not read)
+    float *const red = reinterpret_cast<float *>(dsm);
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            red[(wave * 8 + half * 4 + i) * 64 + lane] = acc[half][i];
+    __syncthreads();
+    for (int o = threadIdx.x; o < kFewWords * 32 * M; o += static_cast<int>(blockDim.x)) {
+        const int m = o / (kFewWords * 32), n = nw0 * 32 + o % (kFewWords * 32), word = (o / 32) % kFewWords, cc = o % 32;
+        const int from = (word * 8 + (cc >> 4) * 4 + m) * 64 + (cc & 15);
+        float total = 0.f;
+        for (int g = 0; g < groups; ++g)
+            total += red[from + g * kFewWords * 512] + (red[from + g * kFewWords * 512 + 16] + red[from + g * kFewWords * 512 + 32]);
+        // Not finite: activations or coefficients that are not.  Their products with the zeros of a plane would make NaN of outputs
+        // that do not select them: summed again, the selected coefficients alone.
+        if (!(fabsf(total) < INFINITY)) {
+            double again = 0.;
+            for (int k = 128 * t_begin; k < min(K, 128 * t_end); ++k)
+                again = row_deq_add<S>(a, n / 32, n % 32, k, m, again);
+            total = static_cast<float>(again);
+        }
+        const size_t at = static_cast<size_t>(m) * N + n;
+        if (a.ksplit > 1) {
+            bool marked = false;
+            if (!add_part(a.acc + at, a.ksplit, total, marked))
+                continue;
+            if (marked) {
+                double again = 0.;
+                for (int k = 0; k < K; ++k)
+                    again = row_deq_add<S>(a, n / 32, n % 32, k, m, again);
+                total = static_cast<float>(again);
+            }
+        }
+        a.out[at] = f2h(a.bias ? total + h2f(a.bias[n]) : total);
+    }
+}
+
 // Parts of K where the caller brings the accumulators.  Several rows: as many as give the CUs two workgroups each, of 4 tiles and
 // more.
 int row_deq_rows_parts(int M, int N, int K, int cus)
@@ -3163,6 +3404,39 @@ bool row_deq_rows(int M, int N, int K, int S, int G, int cus, bool room)
     const double their_us = 2.9 + (theirs > 1 ? 0.7 : 0.) + 0.3 * per_part * turns;
     const double our_us = 4.3 + 0.4 * load + (tiles + kDeqRowsWaves - 1) / kDeqRowsWaves * (2.05 + 1.25 * load) + (M > 16 ? 2.1 : (M > 8 ? 0.6 : 0.));
     return our_us < their_us;
+}
+
+// Whether two to four rows take sbvr_row_deq_few_kernel in place of that launch: where that one has more workgroups than the chip
+// has CUs, and so a second round of them.  (648 shapes, 2 to 8 rows, 512 to 14336 columns, K 640 to 14336, 2 to 4 planes.  Up to
+// 4 rows it is then 1.04 to 1.45 times as fast, 0.88 to 1.06 times otherwise; with 5 and 6 rows 0.92 to 1.26, with 8 0.87 to 1.17.)
+bool row_deq_few(int M, int N, int G, int parts, int cus)
+{
+    return M >= 2 && M <= kFewRows && G % 64 == 0 && static_cast<long>(N / 32) * parts > cus;
+}
+
+template <int S>
+hipError_t launch_row_deq_few(const RowDeqArgs &a, hipStream_t st)
+{
+    const int groups = std::min(kFewTiles, a.per_part);
+    // (the images and scales of a tile a group, afterwards the waves' results: 4 KiB a group)
+    const size_t lds = static_cast<size_t>(groups) * (S * kFewPlane + kFewRows * sizeof(float));
+    {
+        static bool raised_on[16] = {};
+        std::lock_guard<std::mutex> guard(g_dev_lock);
+        int dev_now = 0;
+        if (hipGetDevice(&dev_now) != hipSuccess || dev_now < 0 || dev_now >= 16)
+            dev_now = 0;
+        if (!raised_on[dev_now]) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(sbvr_row_deq_few_kernel<S>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     kFewTiles * (S * kFewPlane + kFewRows * static_cast<int>(sizeof(float))));
+            if (e != hipSuccess)
+                return e;
+            raised_on[dev_now] = true;
+        }
+    }
+    const dim3 grid(static_cast<unsigned>(a.N / (32 * kFewWords)), 1, static_cast<unsigned>(a.ksplit));
+    hipLaunchKernelGGL(sbvr_row_deq_few_kernel<S>, grid, dim3(64 * kFewWords * groups), lds, st, a);
+    return hipGetLastError();
 }
 
 template <int S>
@@ -4534,7 +4808,9 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
         a.ksplit = room ? row_deq_rows_parts(M, N, K, current_cus()) : 1;
         a.per_part = (tiles + a.ksplit - 1) / a.ksplit;
         const int waves = a.per_part < kDeqRowsWaves ? a.per_part : kDeqRowsWaves;
-        const hipError_t e = S == 4 ? launch_row_deq_rows<4>(a, waves, st) : (S == 3 ? launch_row_deq_rows<3>(a, waves, st) : launch_row_deq_rows<2>(a, waves, st));
+        const bool few = row_deq_few(M, N, G, a.ksplit, current_cus());
+        const hipError_t e = few ? (S == 4 ? launch_row_deq_few<4>(a, st) : (S == 3 ? launch_row_deq_few<3>(a, st) : launch_row_deq_few<2>(a, st))) :
+                             S == 4 ? launch_row_deq_rows<4>(a, waves, st) : (S == 3 ? launch_row_deq_rows<3>(a, waves, st) : launch_row_deq_rows<2>(a, waves, st));
         if (e != hipSuccess)
             return fail(SBVR_HIP_ELAUNCH, "row_deq launch: %s", hipGetErrorString(e));
         g_row_deq_kernel = SBVR_HIP_ROW_DEQ_ROWS;
