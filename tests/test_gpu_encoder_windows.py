@@ -1,0 +1,24 @@
+"""The encoder's policy on the device where groups meet the table in windows of 2048: the loop over blocks, bit for bit, with
+groups, misses and groups left to the host on both sides of a window's end."""
+import pytest
+import torch
+
+from test_gpu_encoder import _encode_both_ways
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("groups,S,odd", [
+    (2048, 2, ()),                              # one window exactly
+    (2049, 3, (2048,)),                         # a last window of one group, and that one left to the host
+    (4100, 2, (0, 2047, 2048, 2049, 4095, 4096)),
+    (6145, 2, (2046, 2047, 4095)),
+])
+def test_windows(groups, S, odd):
+    G = 32
+    w = torch.randn((groups, G), generator=torch.Generator().manual_seed(groups)) * 0.02
+    for g in odd:
+        w[g] += 2.0                             # (a mean that moves the offsets)
+    w[::97] *= 30.0                             # (groups that the table does not serve, also far behind)
+    stats = _encode_both_ways(w.to(torch.float16).to("cuda:0"), dict(num_sums=S, bvr_len=G, s_search_num=8, r_search_num=16, b_search_num=8))
+    assert stats["groups"] == groups
