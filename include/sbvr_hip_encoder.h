@@ -93,6 +93,15 @@ int sbvr_hip_online_encode_f16(const void *x, const void *points, uint32_t *bvr,
 int sbvr_hip_online_encode_lines_f16(const void *x, const void *lines, uint32_t *bvr, void *idx, int idx_bytes, int M, int K,
                                      int G, int S, void *stream);
 
+/* Both in one: x (M, K) fp16 encoded against lines (K/G, Sl) as above, times the encoded weight (N, K) of r_bvr, r_idx and
+ * r_cache (sbvr_hip_mm_T's right operand), plus bias (N) or NULL: out (M, N) fp16.  Where sbvr_hip_online_mm_T_scratch says 0 the
+ * two calls by themselves are the way; elsewhere `scratch` is memory of the call's own of that many bytes, 16-byte aligned, that
+ * nothing need clear. */
+size_t sbvr_hip_online_mm_T_scratch(const uint32_t *r_bvr, const void *r_cache, int M, int N, int K, int Sl, int Sr, int G);
+int sbvr_hip_online_mm_T(const void *x, const void *lines, const uint32_t *r_bvr, const void *r_idx, int r_idx_bytes, const void *r_cache,
+                         const void *bias, void *out, int M, int N, int K, int Sl, int Sr, int G, int Lr, void *scratch,
+                         size_t scratch_bytes, void *stream);
+
 /* The dense weight of an encoded one (sbvr/core.py:926-949, decode()): out (N, k_out), out[n, k] = the sum of the
  * coefficients cache[idx[k / G, n], j] whose plane j is set at (n, k), added up in fp32, rounded to fp16 once and
  * converted to out_type (0 fp16, 1 bf16, 2 fp32).  bvr (K/32, N, S) uint32, idx (K/G, N) uint8 or uint16 (idx_bytes),

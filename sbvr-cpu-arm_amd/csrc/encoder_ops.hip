@@ -11,6 +11,7 @@
 // two points per instruction), then an fp32 sum over the group in element order and one division.
 
 #include "../../include/sbvr_hip_encoder.h"
+#include "sbvr_internal.h"
 #include "sbvr_device.h"
 
 namespace {
@@ -846,17 +847,33 @@ long run_lines(const sbvr_hip_encoder_run &a, int wide, int S)
 // memory for itself took 20.5 us.)
 constexpr int kOnlineWaves = 4, kOnlineRows = 4;
 
-template <bool kLines>
+// kImage: also the encoded values as the A operands of sbvr_online_product_kernel (OnlineArgs), and a scale per group: the
+// power of two that puts the sum of the line's magnitudes below 2^15.
+template <bool kLines, bool kImage>
 __global__ void __launch_bounds__(64 * kOnlineWaves)
 sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ table, uint32_t *__restrict__ bvr,
-                          uint8_t *__restrict__ idx, int idx16, int M, int K, int G, int S)
+                          uint8_t *__restrict__ idx, int idx16, int M, int K, int G, int S, uint32_t *__restrict__ image,
+                          float *__restrict__ scales)
 {
     __shared__ __align__(16) uint16_t pts[2][256];
+    __shared__ float sums[kImage ? 2 : 1][kImage ? 256 : 1], ups[2];      // the points before their rounding, the powers of two
+    __shared__ float coeffs[2][8];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int P = 1 << S, padded = max(P, 8);
     const int k0 = blockIdx.x * 64;
     const int words = K / 32;
     const int groups = K / G, g0 = k0 / G, g1 = min((k0 + 32) / G, groups - 1);     // (G is a multiple of 32)
+    const int k = min(k0 + lane, K - 1);
+    static_assert(kOnlineRows == kOnlineWaves, "a row a wave");
+    const int m = blockIdx.y * kOnlineRows + wave;
+    // (everything asked for at once: the activation, and a coefficient a thread; fetched in the loop over the planes below, the
+    // coefficients alone took 2 us)
+    const _Float16 d = __builtin_bit_cast(_Float16, x[static_cast<size_t>(min(m, M - 1)) * K + k]);
+    if constexpr (kLines) {
+        if (threadIdx.x < 16 && (threadIdx.x & 7) < S)
+            coeffs[threadIdx.x >> 3][threadIdx.x & 7] = h2f(table[static_cast<size_t>(threadIdx.x >> 3 ? g1 : g0) * S + (threadIdx.x & 7)]);
+        __syncthreads();
+    }
     for (int i = threadIdx.x; i < 2 * padded; i += 64 * kOnlineWaves) {
         const int which = i >= padded, p = min(which ? i - padded : i, P - 1);       // (the last point again behind the end)
         const int g = which ? g1 : g0;
@@ -864,23 +881,33 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
         if constexpr (kLines) {
             float sum = 0.f;
             for (int j = 0; j < S; ++j) {
-                const float c = static_cast<float>(__builtin_bit_cast(_Float16, table[static_cast<size_t>(g) * S + j]));
+                const float c = coeffs[which][j];
                 sum += (p >> (S - 1 - j)) & 1 ? c : 0.f * c;       // (NaN where c is not finite, as a product would have it)
             }
-            v = __builtin_bit_cast(uint16_t, static_cast<_Float16>(sum));
+            v = f2h(sum);
+            if constexpr (kImage) {
+                if ((which ? i - padded : i) < P)
+                    sums[which][p] = sum;
+                if (p == 0) {
+                    float size = 0.f;
+                    for (int j = 0; j < S; ++j)
+                        size += fabsf(coeffs[which][j]);
+                    // (at least 2^-24 and below 2^19, or not finite: such outputs are added up plane by plane)
+                    const int exponent = static_cast<int>(__float_as_uint(size) >> 23);
+                    const int up = exponent == 255 || exponent == 0 ? 0 : 141 - exponent;
+                    ups[which] = __uint_as_float(static_cast<uint32_t>(127 + up) << 23);
+                    if (blockIdx.y == 0)
+                        scales[g] = __uint_as_float(static_cast<uint32_t>(127 + 24 - up) << 23);
+                }
+            }
         } else {
             v = table[static_cast<size_t>(g) * P + p];
         }
         pts[which][which ? i - padded : i] = v;
     }
     __syncthreads();
-    const int k = min(k0 + lane, K - 1);
     const uint4 *const mine = reinterpret_cast<const uint4 *>(pts[lane >> 5 & (g1 != g0)]);
-    for (int r = wave; r < kOnlineRows; r += kOnlineWaves) {
-        const int m = blockIdx.y * kOnlineRows + r;
-        if (m >= M)                                                                   // wave-uniform
-            break;
-        const _Float16 d = __builtin_bit_cast(_Float16, x[static_cast<size_t>(m) * K + k]);
+    if (m < M) {                                                                      // wave-uniform
         const v2h dd = {d, d};
         uint32_t best = 0xffffffffu;
 #pragma unroll 4
@@ -902,6 +929,18 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
         for (int j = 0; j < S; ++j) {                                                 // plane 0: the selector's top bit
             const unsigned long long bits = __builtin_amdgcn_ballot_w64(((sel >> (S - 1 - j)) & 1) != 0);
             out = (lane & 31) == j ? static_cast<uint32_t>(lane < 32 ? bits : bits >> 32) : out;
+        }
+        if constexpr (kImage) {                                                       // (K is a multiple of 128)
+            const int at = k0 + lane, i = at & 15, which = lane >> 5 & (g1 != g0);
+            const float v = sums[which][sel] * ups[which] * __uint_as_float(static_cast<uint32_t>(127 - (i & 7)) << 23);
+            const _Float16 head = static_cast<_Float16>(v), rest = static_cast<_Float16>(v - static_cast<float>(head));
+            const uint32_t both = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, head)) | static_cast<uint32_t>(__builtin_bit_cast(uint16_t, rest)) << 16;
+            const uint32_t other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(both), 16, 64));
+            // lanes 0 to 15 of 32 store the pair's heads, lanes 16 to 31 the rests
+            const int part = (lane >> 4) & 1;
+            const uint32_t pair = part ? __builtin_amdgcn_perm(both, other, 0x07060302u) : __builtin_amdgcn_perm(other, both, 0x05040100u);
+            const size_t tile = static_cast<size_t>(at >> 7) * ((M + 15) / 16) + (m >> 4);
+            image[(((tile * 4 + (i >> 2)) * 2 + part) * 64 + ((at >> 5) & 3) * 16 + (m & 15)) * 4 + (i & 3)] = pair;
         }
         const int kw = blockIdx.x * 2 + (lane >> 5);
         if ((lane & 31) < S && kw < words)
@@ -1082,6 +1121,12 @@ void launch_decode(int out_type, dim3 grid, hipStream_t st, const DecodeArgs &a)
         hipLaunchKernelGGL((sbvr_decode_weight_kernel<S, kOutF32>), grid, block, 0, st, a);
 }
 
+int device_cus()
+{
+    int device = 0, cus = 0;
+    return hipGetDevice(&device) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess ? cus : 256;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1192,8 +1237,8 @@ int sbvr_hip_online_encode_f16(const void *x, const void *points, uint32_t *bvr,
     if (S > 8 || G % 32 != 0 || K % G != 0 || M > 65535)
         return -2;
     const dim3 grid(static_cast<unsigned>((K + 63) / 64), static_cast<unsigned>((M + kOnlineRows - 1) / kOnlineRows)), block(64 * kOnlineWaves);
-    hipLaunchKernelGGL(sbvr_online_encode_kernel<false>, grid, block, 0, static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(x),
-                       static_cast<const uint16_t *>(points), bvr, nullptr, 0, M, K, G, S);
+    hipLaunchKernelGGL((sbvr_online_encode_kernel<false, false>), grid, block, 0, static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(x),
+                       static_cast<const uint16_t *>(points), bvr, nullptr, 0, M, K, G, S, nullptr, nullptr);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
@@ -1205,9 +1250,52 @@ int sbvr_hip_online_encode_lines_f16(const void *x, const void *lines, uint32_t 
     if (S > 8 || G % 32 != 0 || K % G != 0 || M > 65535 || (idx_bytes == 1 && K / G > 256) || K / G > 65536)
         return -2;
     const dim3 grid(static_cast<unsigned>((K + 63) / 64), static_cast<unsigned>((M + kOnlineRows - 1) / kOnlineRows)), block(64 * kOnlineWaves);
-    hipLaunchKernelGGL(sbvr_online_encode_kernel<true>, grid, block, 0, static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(x),
-                       static_cast<const uint16_t *>(lines), bvr, static_cast<uint8_t *>(idx), idx_bytes == 2 ? 1 : 0, M, K, G, S);
+    hipLaunchKernelGGL((sbvr_online_encode_kernel<true, false>), grid, block, 0, static_cast<hipStream_t>(stream), static_cast<const uint16_t *>(x),
+                       static_cast<const uint16_t *>(lines), bvr, static_cast<uint8_t *>(idx), idx_bytes == 2 ? 1 : 0, M, K, G, S, nullptr, nullptr);
     return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+size_t sbvr_hip_online_mm_T_scratch(const uint32_t *r_bvr, const void *r_cache, int M, int N, int K, int Sl, int Sr, int G)
+{
+    if (M <= 0 || N <= 0 || K <= 0 || Sl <= 0 || Sr <= 0 || G <= 0 || K % G != 0 || !online_product_ok(M, N, K, Sl, Sr, G, r_bvr, r_cache, device_cus()))
+        return 0;
+    const size_t image = static_cast<size_t>(K / 128) * ((M + 15) / 16) * 8192, planes = static_cast<size_t>(K / 32) * M * Sl * 4;
+    return image + planes + static_cast<size_t>(K / G) * sizeof(float);
+}
+
+int sbvr_hip_online_mm_T(const void *x, const void *lines, const uint32_t *r_bvr, const void *r_idx, int r_idx_bytes, const void *r_cache,
+                         const void *bias, void *out, int M, int N, int K, int Sl, int Sr, int G, int Lr, void *scratch,
+                         size_t scratch_bytes, void *stream)
+{
+    if (!x || !lines || !r_bvr || !r_idx || !r_cache || !out || !scratch || M <= 0 || N <= 0 || K <= 0 || Sl <= 0 || Sr <= 0 || G <= 0 || Lr <= 0 ||
+        (r_idx_bytes != 1 && r_idx_bytes != 2))
+        return -1;
+    const size_t need = sbvr_hip_online_mm_T_scratch(r_bvr, r_cache, M, N, K, Sl, Sr, G);
+    if (!need || scratch_bytes < need || reinterpret_cast<uintptr_t>(scratch) % 16 != 0 || K / G > 65536)
+        return -2;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    uint8_t *const at = static_cast<uint8_t *>(scratch);
+    const size_t image = static_cast<size_t>(K / 128) * ((M + 15) / 16) * 8192, planes = static_cast<size_t>(K / 32) * M * Sl * 4;
+    uint32_t *const bvr = reinterpret_cast<uint32_t *>(at + image);
+    float *const scales = reinterpret_cast<float *>(at + image + planes);
+    const dim3 grid(static_cast<unsigned>((K + 63) / 64), static_cast<unsigned>((M + kOnlineRows - 1) / kOnlineRows)), block(64 * kOnlineWaves);
+    hipLaunchKernelGGL((sbvr_online_encode_kernel<true, true>), grid, block, 0, st, static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(lines),
+                       bvr, nullptr, 0, M, K, G, Sl, reinterpret_cast<uint32_t *>(at), scales);
+    if (hipGetLastError() != hipSuccess)
+        return -3;
+    OnlineArgs a{};
+    a.l_bvr = bvr;
+    a.lines = static_cast<const uint16_t *>(lines);
+    a.r_bvr = r_bvr;
+    a.r_idx = r_idx;
+    a.r_cache = static_cast<const uint16_t *>(r_cache);
+    a.bias = static_cast<const uint16_t *>(bias);
+    a.out = static_cast<uint16_t *>(out);
+    a.image = reinterpret_cast<const v4u_image *>(at);
+    a.scales = scales;
+    a.M = M; a.N = N; a.K = K; a.Sl = Sl; a.Lr = Lr;
+    a.r_idx16 = r_idx_bytes == 2;
+    return launch_online_product(Sr, G, a, device_cus(), st) == hipSuccess ? 0 : -3;
 }
 
 int sbvr_hip_decode_weight(const uint32_t *bvr, const void *idx, int idx_bytes, const void *cache, void *out, int out_type, int N, int K,

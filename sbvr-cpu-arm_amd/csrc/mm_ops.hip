@@ -190,6 +190,167 @@ sbvr_mm_T_mfma_kernel(const MmArgs a)
     }
 }
 
+// Output (m, n) by one lane from the planes of both sides, in the order of sbvr_mm_T_mfma_kernel: per group and left plane the
+// popcounts times the column's coefficients, then the left coefficient.
+template <int SR>
+__device__ __forceinline__ float online_output(const OnlineArgs &a, int m, int n)
+{
+    float y = 0.f;
+    const int words = 4 * a.spg;
+#pragma unroll 1
+    for (int g = 0; g < a.K / 32 / words; ++g) {
+        const uint8_t *rb = static_cast<const uint8_t *>(a.r_idx);
+        const size_t at = (static_cast<size_t>(g) * a.N + n) << a.r_idx16;
+        const int line = min(a.r_idx16 ? rb[at] | (rb[at + 1] << 8) : rb[at], a.Lr - 1);
+#pragma unroll 1
+        for (int l = 0; l < a.Sl; ++l) {
+            float sum = 0.f;
+#pragma unroll 1
+            for (int j = 0; j < SR; ++j) {
+                int count = 0;
+                for (int w = g * words; w < (g + 1) * words; ++w)
+                    count += __popc(a.l_bvr[(static_cast<size_t>(w) * a.M + m) * a.Sl + l] & a.r_bvr[(static_cast<size_t>(w) * a.N + n) * SR + j]);
+                sum = fmaf(static_cast<float>(count), h2f(a.r_cache[static_cast<size_t>(line) * SR + j]), sum);
+            }
+            y = fmaf(h2f(a.lines[static_cast<size_t>(g) * a.Sl + l]), sum, y);
+        }
+    }
+    return y;
+}
+
+// ------------------------------------------------------- activations encoded on the fly, more than a few of them
+//
+// The left operand of that product is a dense matrix a_hat[m, k] = sum_l a_l(group) L_l[m, k]: its coefficient line belongs to
+// the group, not to the row, so the launch that encodes the activations leaves it as fp16 numbers too (two parts, 22
+// bits, in the order of the MFMA's A operand: OnlineImage), and the right planes' bits meet it as fp16 numbers: a word of
+// this layout holds 32 k of one column, and `word & 0x00010001 << i` is the pair (k = i, i + 16) as 2^(i - 24) each, a ready
+// dword of the B operand of v_mfma_f32_16x16x32_f16; the activations carry 2^-i.  So 16 left rows are one row tile of 8 MFMAs a
+// plane and 128 k, where their planes are 8 tiles above whose sums each want a multiplication: 17 operations a plane word
+// and 4 a plane's sums, against 7 + 20 for each of the 8 tiles.  A workgroup owns 16 columns and 16 RT rows; its W waves take
+// the sub-groups of 128 k in turn and meet in LDS.  Bound by latency, and by the image's way through the L1 (8 KiB a
+// sub-group and row tile, for every 16 columns).
+template <int SR, int RT, int W>
+__global__ void __launch_bounds__(64 * W)
+sbvr_online_product_kernel(const OnlineArgs a)
+{
+    constexpr int CW = (SR + 1) / 2;
+    __shared__ __align__(16) float red[W * RT * 256];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, blk = lane >> 4;
+    const int N = a.N, nsub = a.K / kMmSub;
+    const int n = blockIdx.x * 16 + col, n_ld = min(n, N - 1);
+    const int tiles = (a.M + 15) / 16, t0 = blockIdx.y * RT;         // row tiles of the image, and the first of this workgroup's
+
+    struct Stage {
+        Planes<SR> w;
+        int lo, hi;
+        uint32_t c[CW];
+        float scale;
+    };
+    auto load = [&](int sg, Stage &s) __attribute__((always_inline)) {
+        s.w = load_planes<SR>(a.r_bvr + (static_cast<size_t>(4 * sg + blk) * N + n_ld) * SR);
+        const uint8_t *rb = static_cast<const uint8_t *>(a.r_idx);
+        const size_t at = (static_cast<size_t>(sg / a.spg) * N + n_ld) << a.r_idx16;
+        s.lo = rb[at];
+        s.hi = rb[at + a.r_idx16];
+        s.scale = a.scales[sg / a.spg];
+    };
+    auto gather = [&](Stage &s) __attribute__((always_inline)) {
+        const int line = min(a.r_idx16 ? s.lo | (s.hi << 8) : s.lo, a.Lr - 1);
+        load_line_words<SR>(a.r_cache + static_cast<size_t>(line) * SR, s.c);
+    };
+    v4f y[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+        y[t] = v4f{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](int sg, const Stage &s) __attribute__((always_inline)) {
+        // (asked for a sub-group ahead, in 32 registers more, the image's operands cost 1 us of 6.5)
+        const v4u *const image = a.image + static_cast<size_t>(sg) * tiles * 512 + lane;
+        v4f D[SR][RT];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            v4u A[RT][2];
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int part = 0; part < 2; ++part)                 // (a tile past the last one repeats it)
+                    A[t][part] = image[(min(t0 + t, tiles - 1) * 4 + u) * 128 + part * 64];
+#pragma unroll
+            for (int part = 0; part < 2; ++part)
+#pragma unroll
+                for (int j = 0; j < SR; ++j) {
+                    const uint32_t w = u < 2 ? s.w.w[j] : s.w.w[j] >> 8;
+                    v4u B;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        B[e] = w & (0x00010001u << (4 * (u & 1) + e));
+#pragma unroll
+                    for (int t = 0; t < RT; ++t)
+                        D[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t][part]), __builtin_bit_cast(v8h, B),
+                                                                         u == 0 && part == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : D[j][t], 0, 0, 0);
+                }
+        }
+#pragma unroll
+        for (int j = 0; j < SR; ++j) {
+            const float c = h2f(static_cast<uint16_t>(j & 1 ? s.c[j / 2] >> 16 : s.c[j / 2] & 0xffffu)) * s.scale;
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    y[t][i] = fmaf(D[j][t][i], c, y[t][i]);
+        }
+    };
+    if (wave < nsub) {                                               // wave-uniform
+        Stage now, next;
+        load(wave, now);
+        gather(now);
+        for (int sg = wave; sg < nsub; sg += W) {
+            load(min(sg + W, nsub - 1), next);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(sg, now);
+            gather(next);
+            now = next;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            red[(wave * RT + t) * 256 + (4 * blk + i) * 16 + col] = y[t][i];
+    __syncthreads();
+    for (int o = threadIdx.x; o < RT * 256; o += 64 * W) {
+        const int m = t0 * 16 + (o >> 4), nn = blockIdx.x * 16 + (o & 15);
+        if (m >= a.M || nn >= N)
+            continue;
+        float total = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w)
+            total += red[w * RT * 256 + o];
+        if (!(fabsf(total) < INFINITY))                              // coefficients that are not finite: plane by plane, as above
+            total = online_output<SR>(a, m, nn);
+        uint16_t v = f2h(total);
+        if (a.bias)
+            v = hadd(v, a.bias[nn]);
+        a.out[static_cast<size_t>(m) * N + nn] = v;
+    }
+}
+
+template <int SR>
+hipError_t launch_online(int RT, int W, const OnlineArgs &a, hipStream_t st)
+{
+    const int tiles = (a.M + 15) / 16;
+    const dim3 grid(static_cast<unsigned>((a.N + 15) / 16), static_cast<unsigned>((tiles + RT - 1) / RT)), block(64 * W);
+    if (RT == 1 && W == 16)
+        hipLaunchKernelGGL((sbvr_online_product_kernel<SR, 1, 16>), grid, block, 0, st, a);
+    else if (RT == 1)
+        hipLaunchKernelGGL((sbvr_online_product_kernel<SR, 1, 8>), grid, block, 0, st, a);
+    else if (SR <= 4 && W == 16)
+        hipLaunchKernelGGL((sbvr_online_product_kernel<(SR <= 4 ? SR : 4), 2, 16>), grid, block, 0, st, a);
+    else                                 // (6 and 8 planes of two row tiles want more than a 16-wave workgroup's 128 registers)
+        hipLaunchKernelGGL((sbvr_online_product_kernel<SR, 2, 8>), grid, dim3(512), 0, st, a);
+    return hipGetLastError();
+}
+
 template <int SR>
 hipError_t launch_rt(int RT, int W, const MmArgs &a, hipStream_t st)
 {
@@ -242,5 +403,31 @@ hipError_t launch_mm_T_mfma(int Sr, int G, MmArgs a, int cus, hipStream_t st)
     case 4: return launch_rt<4>(RT, W, a, st);
     case 6: return launch_rt<6>(RT, W, a, st);
     default: return launch_rt<8>(RT, W, a, st);
+    }
+}
+
+// Where that way is the faster one: more than 64 (left row, plane) pairs, of more than 4 planes a row, and workgroups for three
+// quarters of the CUs.  us a call (both launches), planes and this, 8 left and 4 right planes: 9 rows x 4096, K 4096 14.1
+// and 12.3; 64 rows 35.9 and 26.1; 32 x 14336, K 4096 52.6 and 34.9; 48 x 1024, K 14336 43.6 and 38.2, but 16 x 1024, K
+// 14336 17.4 and 23.0; 64 x 512, K 4096 15.8 and 17.5; 4 left planes, 32 x 4096, K 4096 12.2 and 12.9.
+bool online_product_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r_bvr, const void *r_cache, int cus)
+{
+    return mm_T_mfma_ok(M, N, K, Sl, Sr, G, r_bvr, r_cache) && Sl > 4 && Sl <= 8 && M * Sl > 64 && M <= 4096 &&
+           static_cast<long>((N + 15) / 16) * ((M + 15) / 16) * 4 >= 3L * cus &&
+           static_cast<double>(M + 15) / 16 * (K / kMmSub) * 512 < 2147483648.0;
+}
+
+hipError_t launch_online_product(int Sr, int G, OnlineArgs a, int cus, hipStream_t st)
+{
+    a.spg = G / kMmSub;
+    const int tiles = (a.M + 15) / 16, cols = (a.N + 15) / 16;
+    const int RT = tiles > 1 && static_cast<long>(cols) * ((tiles + 1) / 2) * 4 >= 3L * cus ? 2 : 1;
+    const int W = static_cast<long>(cols) * ((tiles + RT - 1) / RT) >= 2L * cus ? 8 : 16;
+    switch (Sr) {
+    case 2: return launch_online<2>(RT, W, a, st);
+    case 3: return launch_online<3>(RT, W, a, st);
+    case 4: return launch_online<4>(RT, W, a, st);
+    case 6: return launch_online<6>(RT, W, a, st);
+    default: return launch_online<8>(RT, W, a, st);
     }
 }

@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+typedef uint32_t v4u_image __attribute__((ext_vector_type(4)));
+
 // The product of two encoded operands on the matrix cores (mm_ops.hip).
 struct MmArgs {
     const uint32_t *l_bvr;       // (K / 32, M, Sl)
@@ -23,6 +25,26 @@ struct MmArgs {
 // Whether that kernel covers the shape (pointers: r_bvr and r_cache 16-byte aligned).
 bool mm_T_mfma_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r_bvr, const void *r_cache);
 hipError_t launch_mm_T_mfma(int Sr, int G, MmArgs a, int cus, hipStream_t st);
+
+// The same product with a left operand encoded on the fly (mm_ops.hip, encoder_ops.hip).  image: per sub-group of 128 k and row
+// tile of 16 the A operands of eight v_mfma_f32_16x16x32_f16, [u = 0..3][part][lane] of 16 bytes, dword e of lane (row r,
+// block b) the pair k = 32 b + 4 u + e, + 16, each the sum of its selected coefficients times the group's power of two times
+// 2^-((4 u + e) % 8), part 0 rounded to fp16, part 1 what is left.  scales: per group 2^24 over that power of two.
+struct OnlineArgs {
+    const uint32_t *l_bvr;       // (K / 32, M, Sl)
+    const uint16_t *lines;       // (K / G, Sl)
+    const uint32_t *r_bvr;       // (K / 32, N, Sr)
+    const void *r_idx;
+    const uint16_t *r_cache;
+    const uint16_t *bias;
+    uint16_t *out;
+    const v4u_image *image;
+    const float *scales;
+    int M, N, K, Sl, Lr;
+    int spg, r_idx16;
+};
+bool online_product_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r_bvr, const void *r_cache, int cus);
+hipError_t launch_online_product(int Sr, int G, OnlineArgs a, int cus, hipStream_t st);
 
 // The prefill kernels (sbvr_hip.hip, prefill_ops.hip).
 struct GemmArgs {

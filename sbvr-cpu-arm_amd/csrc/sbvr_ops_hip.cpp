@@ -392,6 +392,27 @@ torch::Tensor sbvr_online_mm_T(torch::Tensor x, const torch::Tensor &lines, cons
     if (x.size(1) != K)
         x = at::constant_pad_nd(x, {0, K - x.size(1)});
     const torch::Tensor table = lines.contiguous();
+    if (x.size(0) > 0 && table.scalar_type() == torch::kFloat16 && table.device() == x.device() && r_bvr.dim() == 3 && r_bvr.scalar_type() == torch::kUInt32 &&
+        r_bvr.is_contiguous() && r_bvr.size(0) * 32 == K && r_coeff_cache.dim() == 2) {
+        const int64_t M = x.size(0), N = r_bvr.size(1), Sl = table.size(1), Sr = r_bvr.size(2), Lr = r_coeff_cache.size(0);
+        const size_t need = M < (1 << 20) && K < (1 << 30) ? sbvr_hip_online_mm_T_scratch(static_cast<const uint32_t *>(r_bvr.data_ptr()), r_coeff_cache.data_ptr(),
+                                                                                         M, N, K, Sl, Sr, bvr_len) : 0;
+        if (need) {
+            want(r_coeff_cache, "r_coeff_cache", torch::kFloat16, 2, &x);
+            const int rib = idx_bytes(r_coeff_idx, Lr, "r_coeff_idx", x);
+            SBVR_WANT(r_coeff_idx.size(1) == N && r_coeff_idx.size(0) * bvr_len == K && r_coeff_cache.size(1) == Sr,
+                      "index / table shapes do not match the bit planes");
+            const DeviceGuard guard(x.device());
+            const torch::Tensor xc = x.contiguous();
+            auto out = at::empty({M, N}, table.options());
+            auto scratch = at::empty({static_cast<int64_t>(need)}, table.options().dtype(torch::kUInt8));
+            const int rc = sbvr_hip_online_mm_T(xc.data_ptr(), table.data_ptr(), static_cast<const uint32_t *>(r_bvr.data_ptr()), r_coeff_idx.data_ptr(), rib,
+                                                r_coeff_cache.data_ptr(), bias_ptr(bias, N, x), out.data_ptr(), M, N, K, Sl, Sr, bvr_len, Lr,
+                                                scratch.data_ptr(), need, current_stream());
+            check_encoder(rc, "sbvr_hip_online_mm_T", " (M=", M, " N=", N, " K=", K, " bvr_len=", bvr_len, " S=", Sl, ",", Sr, ")");
+            return out;
+        }
+    }
     const auto [bvr, idx] = sbvr_online_encode_lines(x.contiguous(), table, bvr_len);
     return sbvr_mm_T(bvr, idx, table, r_bvr, r_coeff_idx, r_coeff_cache, bias, 0);
 }
