@@ -2066,22 +2066,41 @@ bool lut_path_ok(int M, int N, int K, int S, int G)
            static_cast<double>(K / 32) * N * S < 2147483648.0;
 }
 
-// Workgroups along K: until the 32-column blocks times the parts fill the CUs, a wave keeping 4 word pairs and more.
-int lut_ksplit(int N, int K, int cus)
+// Word pairs of a workgroup (an even number of them per workgroup and per wave: a loop iteration starts on an even pair,
+// which the shared coefficient line of the kShare instances relies on).
+int lut_pairs_per_wg(int pairs, int ksplit)
+{
+    return ((pairs + ksplit - 1) / ksplit + 1) / 2 * 2;
+}
+
+// Workgroups along K: the cheapest of up to 16 parts that keep a word pair for every wave and give a CU two workgroups at
+// most.  Costs in units of 1 / 16 us: a word pair of a wave in a workgroup that has its CU to itself 6 + S, two workgroups on
+// a CU each 1.75 + S / 20 times as long, the accumulators 20 and 2 more for each part.  (Fitted to 225 shapes, 600 to 7000
+// columns, K 2048 to 20480, 2, 4 and 8 planes, 12 and 24 rows, each with 1 to 16 parts: within 0.6 % of the best of them on
+// average, 3 % slower in one of them than doubling the parts until the CUs are full, which it replaces: that was 12 %
+// from the best, the worst where it kept K whole up to 4096 a part (600 columns, K 10240, 4 planes: 8.3 us against 5.9
+// now) or gave some of the CUs a second workgroup (5000 columns, K 4096: 9.5 against 7.9).)
+int lut_ksplit(int N, int K, int S, int cus)
 {
     const int blocks = (N + 31) / 32, pairs = K / 64;
-    int ks = 1;
-    while (blocks * ks < cus && pairs / (ks * 2) >= 4 * kLutWaves && ks < 16)
-        ks *= 2;
-    return ks;
+    int best = 1;
+    float best_cost = 0.f;
+    for (int ks = 1; ks <= 16 && (ks == 1 || (blocks * ks <= 2 * cus && pairs / ks >= kLutWaves)); ++ks) {
+        const int of_wave = (lut_pairs_per_wg(pairs, ks) + kLutWaves - 1) / kLutWaves;
+        const float share = blocks * ks <= cus ? 1.f : 1.75f + 0.05f * S;
+        const float cost = of_wave * (6 + S) * share + (ks > 1 ? 20.f + 2.f * ks : 2.f);
+        if (ks == 1 || cost < best_cost) {
+            best_cost = cost;
+            best = ks;
+        }
+    }
+    const int per_wg = lut_pairs_per_wg(pairs, best);       // (no workgroup without a pair)
+    return (pairs + per_wg - 1) / per_wg;
 }
 
 hipError_t launch_rows32_lut(int S, RowsArgs a, hipStream_t st)
 {
-    // (an even number of word pairs per workgroup and per wave: a loop iteration starts on an even pair, which the
-    // shared coefficient line of the kShare instances relies on)
-    const int pairs = a.K / 64;
-    a.pairs_per_wg = ((pairs + a.ksplit - 1) / a.ksplit + 1) / 2 * 2;
+    a.pairs_per_wg = lut_pairs_per_wg(a.K / 64, a.ksplit);
     const dim3 grid(static_cast<unsigned>((a.N + 31) / 32), static_cast<unsigned>(a.ksplit)), block(64 * kLutWaves);
     const bool half = a.M <= 16, share = a.words_per_group % 4 == 0;
 #define SBVR_LUT(SS)                                                                                          \
@@ -4468,7 +4487,7 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
         r.M = M; r.N = N; r.K = K; r.L = L;
         r.words_per_group = G / 32;
         r.idx16 = idx_bytes == 2;
-        r.ksplit = lut_ksplit(N, K, current_cus());
+        r.ksplit = lut_ksplit(N, K, S, current_cus());
         // (without the accumulators the launch is simply not split)
         if (r.ksplit > 1 && (!workspace || workspace_bytes < static_cast<size_t>(M) * N * sizeof(unsigned long long) ||
                              reinterpret_cast<uintptr_t>(workspace) % 8 != 0))
