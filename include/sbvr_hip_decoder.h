@@ -122,7 +122,7 @@ int sbvr_hip_dec_head_argmax_embed_f16(const void *x, const void *delta, const v
                                        const float *sin_table, int head_dim, float *rot_now, void *workspace,
                                        const void *embed, void *x_next, void *stream);
 
-/* A prompt's tokens, up to 4 at a time, through a layer, every row bit for bit what the one-row launches of a decode step
+/* A prompt's tokens, up to 8 at a time, through a layer, every row bit for bit what the one-row launches of a decode step
  * give it (the same parts of K in the same order, the same roundings), so that a prompt leaves the same caches whichever
  * way it came in.  out (rows, N) = the linear (default layout, as sbvr_hip_linear_f16) of
  *   ADD_RMSNORM  x_out = fp16(x + delta), RMSNorm of it: x, delta, x_out and h (rows, K), h left with the normed rows; the

@@ -142,6 +142,7 @@ sbvr_linear_portable_kernel(const uint16_t *__restrict__ x, const uint32_t *__re
 constexpr int kSub = 128;        // K elements per MFMA (one sub-group)
 constexpr int kMaxWaves = 16;    // waves of a workgroup; they split K among themselves
 constexpr int kMaxM = 16;        // batch rows of the decode kernel (row tiles of 4)
+constexpr int kRowTile = 4;
 constexpr int kUnitsAhead = 3;   // units of plane words a wave of the decode kernel keeps in flight
 constexpr int kUnitsFirst = 2;   // of those, requested before the wave makes its A operands (the rest right behind them)
 constexpr float kLastTermScale = 256.f;  // third fp8 term of an activation holds residual * 256
@@ -1203,6 +1204,14 @@ constexpr bool shape_ok_for(int MT, int CT, int SP)
     return CT * MT <= 16 && (MT == 1 || CT * SP * MT <= 16) && (MT != 2 || (SP <= 4 && CT * SP <= 8 && !(SP == 4 && CT > 1)));
 }
 
+// Two row tiles (5 to 8 tokens of a prompt) with a launch shape of one batch row: the shapes above, and up to 4 planes the
+// widest window, whose units fill 116 registers then.  (Its 7 tiles are what reads a 4096 -> 28672 weight in one round.)
+constexpr int kWideTilesMaxPlanes = 4;
+constexpr bool two_tiles_ok(int S, int CT, int SP)
+{
+    return shape_ok_for(2, CT, SP) || (CT == 7 && SP == 2 && S <= kWideTilesMaxPlanes);
+}
+
 bool has_instance(int CT, int SP)
 {
     for (int i = 0; i < kNumShapes; ++i)
@@ -1388,10 +1397,18 @@ hipError_t launch_gemv_mt(const GemvArgs &a, const GemvPlan &p, int xm, hipStrea
         return p.MT == 1 ? launch_gemv_shape<S, 1, kXFloor>(a, p, st) : hipErrorInvalidConfiguration;
     if (xm == kXPlanes)
         return p.MT == 1 ? launch_gemv_shape<S, 1, kXPlanes>(a, p, st) : hipErrorInvalidConfiguration;
+    if constexpr (S <= kWideTilesMaxPlanes)
+        if (p.MT == 2 && p.CT == 7 && p.SP == 2 && (xm == kXPlain || xm == kXSwiGLURows))
+            return xm == kXPlain ? launch_gemv_inst<S, 2, 7, 2, kXPlain>(a, p, st) : launch_gemv_inst<S, 2, 7, 2, kXSwiGLURows>(a, p, st);
     if (xm == kXSwiGLURows)
-        return p.MT == 1 ? launch_gemv_shape<S, 1, kXSwiGLURows>(a, p, st) : hipErrorInvalidConfiguration;
-    if (xm == kXPairs)
-        return p.MT == 1 && p.CT == 2 && p.SP == 1 && p.waves == kAoGroup ? launch_gemv_inst<S, 1, 2, 1, kXPairs>(a, p, st) : hipErrorInvalidConfiguration;
+        return p.MT == 1 ? launch_gemv_shape<S, 1, kXSwiGLURows>(a, p, st)
+                         : (p.MT == 2 ? launch_gemv_shape<S, 2, kXSwiGLURows>(a, p, st) : hipErrorInvalidConfiguration);
+    if (xm == kXPairs) {
+        if (p.CT != 2 || p.SP != 1 || p.waves != kAoGroup)
+            return hipErrorInvalidConfiguration;
+        return p.MT == 1 ? launch_gemv_inst<S, 1, 2, 1, kXPairs>(a, p, st)
+                         : (p.MT == 2 ? launch_gemv_inst<S, 2, 2, 1, kXPairs>(a, p, st) : hipErrorInvalidConfiguration);
+    }
     if (xm == kXHalves)
         return p.MT == 1 ? launch_gemv_shape<S, 1, kXHalves>(a, p, st)
                          : (p.MT == 2 ? launch_gemv_shape<S, 2, kXHalves>(a, p, st) : hipErrorInvalidConfiguration);
@@ -3850,6 +3867,7 @@ __global__ void sbvr_rows_advance_kernel(long long *pos, int rows, int max_seq, 
 constexpr int kAoWaves = 16, kAoThreads = 64 * kAoWaves;
 constexpr int kAoHead = 128;         // head size
 constexpr int kAoCols = 128;         // output columns of a workgroup: per head 4 waves x 2 column tiles
+constexpr int kAoRowsMax = 8;        // tokens of a prompt in a launch of the attention alone: keys and values of 2 KiB each
 constexpr int kAoMaxSeq = 4096;      // 24 bytes of LDS per cache position
 constexpr int kAoLdsFixed = 8192 + kAoWaves * 2048;
 
@@ -3886,7 +3904,7 @@ __device__ unsigned long long g_ao_trace[2 * 16 * 12];      // development build
 #define SBVR_AOSTAMP(i) do { } while (0)
 #endif
 
-// kRows: the attention alone of up to 4 tokens of a prompt, workgroup (g, e) for token e, which stands at position *pos_p + e.
+// kRows: the attention alone of up to 8 tokens of a prompt, workgroup (g, e) for token e, which stands at position *pos_p + e.
 // Its keys and values of the tokens before it in the same launch come from their rows of qkv (their cache rows are being
 // written meanwhile); the rest, and every sum, is as above.
 template <int S, bool kRows = false>
@@ -3897,7 +3915,7 @@ sbvr_attn_o_kernel(const AttnOArgs a)
     const int max_seq = a.max_seq;
     uint16_t *const qn = reinterpret_cast<uint16_t *>(smem);               // rotated queries of the group: 4 x 128
     uint16_t *const kn = kRows ? reinterpret_cast<uint16_t *>(smem + 6144) : qn + kAoGroup * kAoHead;      // rotated new key (kRows: keys)
-    uint16_t *const vn = kRows ? kn + 4 * kAoHead : kn + kAoHead;                                            // new value (kRows: values)
+    uint16_t *const vn = kRows ? kn + kAoRowsMax * kAoHead : kn + kAoHead;                                   // new value (kRows: values)
     float *const red_max = reinterpret_cast<float *>(smem + 1536);         // [wave][head]
     float *const red_sum = red_max + kAoWaves * kAoGroup;                  // [wave]
     float *const a_scale = red_sum + kAoWaves;                             // [head]: 2^-(e+1) of its A operand
@@ -3922,15 +3940,22 @@ sbvr_attn_o_kernel(const AttnOArgs a)
     SBVR_AOSTAMP(0);
     // the new token: waves 0..3 take query head `wave` of the group, wave 4 the key, wave 5 the value; lane d
     // holds elements d and d + 64 (a rotation pair)
-    uint16_t na = 0, nb = 0;
+    uint16_t na = 0, nb = 0, na2 = 0, nb2 = 0;
     float c_now = 0.f, s_now = 0.f;
-    const int fresh = wave & 3;              // (kRows: waves 4 to 7 the tokens' keys, 8 to 11 their values, up to token e)
+    const int fresh = wave & 3;              // (kRows: waves 4 to 7 the tokens' keys, 8 to 11 their values, up to token e:
+                                             // wave w of either four takes tokens w and w + 4)
     if constexpr (kRows) {
+        static_assert(kAoRowsMax == 8, "two tokens a wave");
+        const int row = wave < 4 ? kAoGroup * g + wave : (wave < 8 ? a.heads + g : a.heads + a.kv_heads + g);
+        const uint16_t *src = a.qkv + static_cast<size_t>(wave < 4 ? e : fresh) * a.qkv_stride + static_cast<size_t>(row) * kAoHead;
         if (wave < 4 || (wave < 12 && fresh <= e)) {
-            const int row = wave < 4 ? kAoGroup * g + wave : (wave < 8 ? a.heads + g : a.heads + a.kv_heads + g);
-            const uint16_t *src = a.qkv + static_cast<size_t>(wave < 4 ? e : fresh) * a.qkv_stride + static_cast<size_t>(row) * kAoHead;
             na = src[lane];
             nb = src[lane + kAoHead / 2];
+        }
+        if (wave >= 4 && wave < 12 && fresh + 4 <= e) {
+            src += static_cast<size_t>(4) * a.qkv_stride;
+            na2 = src[lane];
+            nb2 = src[lane + kAoHead / 2];
         }
     } else if (wave < 6) {                   // wave-uniform
         const int row = wave < 4 ? kAoGroup * g + wave : (wave == 4 ? a.heads + g : a.heads + a.kv_heads + g);
@@ -3971,31 +3996,42 @@ sbvr_attn_o_kernel(const AttnOArgs a)
     const int p = p64 < 0 ? 0 : (p64 >= max_seq ? max_seq - 1 : static_cast<int>(p64));
     SBVR_AOSTAMP(2);
     if constexpr (kRows) {
-        if (wave < 8 && (wave < 4 || fresh <= e)) {
-            const int at_row = wave < 4 ? p : max(p - e + fresh, 0);
-            c_now = a.cos_t[static_cast<size_t>(at_row) * (kAoHead / 2) + lane];
-            s_now = a.sin_t[static_cast<size_t>(at_row) * (kAoHead / 2) + lane];
-            // (the products and roundings that the one-token form compiles to)
-            const float xa = h2f(na), xb = h2f(nb), sb = __fmul_rn(s_now, xb), cb = __fmul_rn(c_now, xb);
-            const uint16_t r0 = __builtin_bit_cast(uint16_t, fma_half(c_now, xa, -sb)), r1 = __builtin_bit_cast(uint16_t, fma_half(s_now, xa, cb));
-            uint16_t *const dst = wave < 4 ? qn + wave * kAoHead : kn + fresh * kAoHead;
+        // (the products and roundings that the one-token form compiles to)
+        auto rotated_to = [&](uint16_t *dst, int at_row, uint16_t ha, uint16_t hb, bool append) __attribute__((always_inline)) {
+            const float c = a.cos_t[static_cast<size_t>(at_row) * (kAoHead / 2) + lane], s = a.sin_t[static_cast<size_t>(at_row) * (kAoHead / 2) + lane];
+            const float xa = h2f(ha), xb = h2f(hb), sb = __fmul_rn(s, xb), cb = __fmul_rn(c, xb);
+            const uint16_t r0 = __builtin_bit_cast(uint16_t, fma_half(c, xa, -sb)), r1 = __builtin_bit_cast(uint16_t, fma_half(s, xa, cb));
             dst[lane] = r0;
             dst[lane + kAoHead / 2] = r1;
-            if (wave >= 4 && fresh == e) {
+            if (append) {
                 uint16_t *const at = kc + static_cast<size_t>(p >> 4) * 2048 + (lane >> 5) * 512 + ((lane & 31) >> 3) * 128 +
                                      (p & 15) * 8 + (lane & 7);
                 at[0] = r0;
                 at[1024] = r1;
             }
-        } else if (wave >= 8 && wave < 12 && fresh <= e) {
-            vn[fresh * kAoHead + lane] = na;
-            vn[fresh * kAoHead + lane + kAoHead / 2] = nb;
-            if (fresh == e) {
+        };
+        auto value_to = [&](uint16_t *dst, uint16_t ha, uint16_t hb, bool append) __attribute__((always_inline)) {
+            dst[lane] = ha;
+            dst[lane + kAoHead / 2] = hb;
+            if (append) {
                 uint16_t *const at = vc + static_cast<size_t>(p >> 5) * 4096 + (lane >> 4) * 512 + ((p & 31) >> 3) * 128 +
                                      (lane & 15) * 8 + (p & 7);
-                at[0] = na;
-                at[2048] = nb;
+                at[0] = ha;
+                at[2048] = hb;
             }
+        };
+        if (wave < 4) {                      // wave-uniform, all of these
+            rotated_to(qn + wave * kAoHead, p, na, nb, false);
+        } else if (wave < 8) {
+            if (fresh <= e)
+                rotated_to(kn + fresh * kAoHead, max(p - e + fresh, 0), na, nb, fresh == e);
+            if (fresh + 4 <= e)
+                rotated_to(kn + (fresh + 4) * kAoHead, max(p - e + fresh + 4, 0), na2, nb2, fresh + 4 == e);
+        } else if (wave < 12) {
+            if (fresh <= e)
+                value_to(vn + fresh * kAoHead, na, nb, fresh == e);
+            if (fresh + 4 <= e)
+                value_to(vn + (fresh + 4) * kAoHead, na2, nb2, fresh + 4 == e);
         }
     } else if (wave < 5) {
         if (!a.rot_now) {
@@ -5161,7 +5197,7 @@ int sbvr_hip_dec_rows_linear_f16(int prologue, const void *x, const void *delta,
                            reinterpret_cast<uintptr_t>(coeff_cache);
     if (wide % 16 != 0)
         return fail(SBVR_HIP_EINVAL, "x, delta, norm_weight, x_out, h, bvr and coeff_cache must be 16-byte aligned");
-    if (rows > 4 || !mfma_path_ok(rows, N, K, S, G) || prologue < SBVR_HIP_DEC_ROWS_ADD_RMSNORM || prologue > SBVR_HIP_DEC_ROWS_HEADS)
+    if (rows > 2 * kRowTile || !mfma_path_ok(rows, N, K, S, G) || prologue < SBVR_HIP_DEC_ROWS_ADD_RMSNORM || prologue > SBVR_HIP_DEC_ROWS_HEADS)
         return fail(SBVR_HIP_EUNSUPPORTED, "rows of a prompt: prologue=%d rows=%d N=%d K=%d S=%d G=%d", prologue, rows, N, K, S, G);
     hipStream_t st = static_cast<hipStream_t>(stream);
     // the launch shapes of the one-row calls these rows stand for: the same parts of K in the same order
@@ -5182,6 +5218,12 @@ int sbvr_hip_dec_rows_linear_f16(int prologue, const void *x, const void *delta,
     }
     if (p.CT == 0)
         return fail(SBVR_HIP_EUNSUPPORTED, "no launch shape for N=%d K=%d S=%d", N, K, S);
+    // 5 to 8 rows: two row tiles over the same plane words, where that shape has them, or four rows and the rest in turn
+    const bool two_tiles = rows > kRowTile && two_tiles_ok(S, p.CT, p.SP);
+    if (two_tiles) {
+        p.MT = 2;
+        p.lds = static_cast<size_t>(p.waves) * (2048 + (p.CT * p.MT <= 8 ? 0 : p.CT * p.MT * 256));
+    }
     if (p.ksplit > 1 && (!workspace || workspace_bytes < static_cast<size_t>(rows) * N * sizeof(unsigned long long) || reinterpret_cast<uintptr_t>(workspace) % 8 != 0))
         return fail(SBVR_HIP_EWORKSPACE, "workspace of %zu bytes needed, %zu given", static_cast<size_t>(rows) * N * sizeof(unsigned long long), workspace_bytes);
     GemvArgs a{};
@@ -5207,7 +5249,17 @@ int sbvr_hip_dec_rows_linear_f16(int prologue, const void *x, const void *delta,
         else
             hipLaunchKernelGGL(sbvr_rows_add_norm_kernel<1>, grid, block, 0, st, xs, ds, ws, xo, hs, K, eps);
     }
-    hipError_t e = launch_gemv(S, a, p, xm, st);
+    hipError_t e = hipSuccess;
+    const int at_once = two_tiles ? rows : kRowTile;
+    for (int first = 0; first < rows && e == hipSuccess; first += at_once) {
+        GemvArgs part = a;
+        part.M = std::min(at_once, rows - first);
+        part.x += static_cast<size_t>(first) * a.xstride;
+        part.out += static_cast<size_t>(first) * N;
+        if (part.acc)
+            part.acc += static_cast<size_t>(first) * N;
+        e = launch_gemv(S, part, p, xm, st);
+    }
     if (e == hipSuccess)
         e = hipGetLastError();
     if (e != hipSuccess)
@@ -5223,7 +5275,7 @@ int sbvr_hip_dec_rows_attention_f16(const void *qkv, const float *cos_table, con
 {
     if (!qkv || !cos_table || !sin_table || !pos || !kcache || !vcache || !ctx)
         return fail(SBVR_HIP_EINVAL, "null pointer argument");
-    if (rows <= 0 || rows > 4 || !sbvr_hip_dec_attention_o_supported(heads, kv_heads, head_dim, max_seq, kAoCols, 4, kSub))
+    if (rows <= 0 || rows > kAoRowsMax || !sbvr_hip_dec_attention_o_supported(heads, kv_heads, head_dim, max_seq, kAoCols, 4, kSub))
         return fail(SBVR_HIP_EUNSUPPORTED, "attention of a prompt's tokens: rows=%d heads=%d kv_heads=%d head_dim=%d max_seq=%d", rows, heads, kv_heads,
                     head_dim, max_seq);
     if ((reinterpret_cast<uintptr_t>(kcache) | reinterpret_cast<uintptr_t>(vcache)) % 16 || reinterpret_cast<uintptr_t>(qkv) % 2 ||

@@ -123,15 +123,17 @@ class SbvrLlamaDecoder:
         self.generated = torch.zeros(max_seq, dtype=torch.int64, device=dev)
         self.logits = torch.empty((1, s.vocab), dtype=torch.float16, device=dev)
         self.head_ws = torch.zeros(2, dtype=torch.int64, device=dev)              # cross-workgroup argmax of the head kernel
-        # a prompt's tokens go through the layers a few at a time where attention + projection have their one launch
-        self.prompt_rows = hip.DEC_ROWS if self.attention_o else 0
+        # a prompt's tokens go through the layers `prompt_rows` at a time where attention + projection have their one launch,
+        # twice as many while that many are left
+        self.prompt_rows = hip.DEC_ROWS // 2 if self.attention_o else 0
         if self.prompt_rows:
-            rows = self.prompt_rows
+            rows = hip.DEC_ROWS
             self.rows_tok = torch.zeros(rows, dtype=torch.int64, device=dev)
             self.rows = {name: torch.zeros((rows, n), dtype=torch.float16, device=dev)
                          for name, n in (("x", s.hidden), ("x_alt", s.hidden), ("zero", s.hidden), ("h", s.hidden), ("ctx", q_out),
                                          ("qkv", q_out + 2 * kv_out), ("o", s.hidden), ("gate_up", 2 * s.ffn), ("down", s.hidden))}
-        self.graph = self.graph_rows = None
+        self.graph = None
+        self.graph_rows = {}                    # by the number of tokens
         self.graph_many, self.steps_per_replay = None, 1
         self.stream = torch.cuda.Stream(device=dev)
         # probe(layer, residual): called by an eager fused step with the residual stream as it enters each layer
@@ -214,13 +216,14 @@ class SbvrLlamaDecoder:
         hip.dec_argmax_advance(logits, self.tok, self.generated, self.pos, self.cos, self.sin, self.rot_now)
         return logits
 
-    def _rows_step(self):
-        """``prompt_rows`` tokens of a prompt (``rows_tok``) through all layers: the caches and the position as that many
+    def _rows_step(self, rows):
+        """The first ``rows`` tokens in ``rows_tok`` through all layers: the caches and the position as that many
         steps leave them, bit for bit; no head (a prompt's last token goes through a step of its own).  7 launches a
-        layer for 4 tokens where steps take 16: every launch of a step, and every byte of weight it reads, serves one token."""
-        s, r = self.shape, self.rows
+        layer for 4 or 8 tokens where steps take 16 or 32: every launch of a step, and every byte of weight it reads, serves
+        one token."""
+        s, r = self.shape, {name: t[:rows] for name, t in self.rows.items()}
         a, b, delta = r["x"], r["x_alt"], r["zero"]
-        torch.index_select(self.embed, 0, self.rows_tok, out=a)
+        torch.index_select(self.embed, 0, self.rows_tok[:rows], out=a)
         for layer in self.layers:
             qkv, o, gate_up, down = (layer[k] for k in ("qkv", "o", "gate_up", "down"))
             hip.dec_rows_add_rmsnorm(a, delta, layer["norm1"], s.rms_eps, b, r["h"], qkv.bvr, qkv.idx, qkv.cache, qkv.bvr_len, r["qkv"])
@@ -230,7 +233,7 @@ class SbvrLlamaDecoder:
             hip.dec_rows_add_rmsnorm(b, r["o"], layer["norm2"], s.rms_eps, a, r["h"], gate_up.bvr, gate_up.idx, gate_up.cache,
                                      gate_up.bvr_len, r["gate_up"])
             delta = hip.dec_rows_swiglu(r["gate_up"], down.bvr, down.idx, down.cache, down.bvr_len, r["down"])
-        hip.dec_rows_advance(self.pos, self.prompt_rows, self.cos, self.sin, self.rot_now)
+        hip.dec_rows_advance(self.pos, rows, self.cos, self.sin, self.rot_now)
 
     # -- driving ---------------------------------------------------------------
     def capture(self, steps_per_replay=16):
@@ -246,13 +249,13 @@ class SbvrLlamaDecoder:
             with torch.cuda.graph(self.graph, stream=self.stream):
                 self.step()
             torch.cuda.synchronize()
-            self.graph_rows = None
-            if self.prompt_rows and self.probe is None:
-                self._rows_step()
+            self.graph_rows = {}
+            for rows in (2 * self.prompt_rows, self.prompt_rows) if self.prompt_rows and self.probe is None else ():
+                self._rows_step(rows)
                 torch.cuda.synchronize()
-                self.graph_rows = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(self.graph_rows, stream=self.stream):
-                    self._rows_step()
+                self.graph_rows[rows] = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(self.graph_rows[rows], stream=self.stream):
+                    self._rows_step(rows)
                 torch.cuda.synchronize()
             self.graph_many, self.steps_per_replay = None, int(steps_per_replay)
             if self.steps_per_replay > 1:
@@ -280,7 +283,7 @@ class SbvrLlamaDecoder:
             self.step()
 
     def generate(self, prompt, new_tokens):
-        """Feeds `prompt` (1-D int64 tensor) `prompt_rows` tokens at a time, the rest and
+        """Feeds `prompt` (1-D int64 tensor) twice `prompt_rows` tokens at a time, then `prompt_rows`, the rest and
         the last one by themselves, then decodes `new_tokens` greedily.  Returns (tokens, seconds spent on the new tokens).
         `generated` holds what followed each position that a step took; those of the prompt that went through the layers
         with others, without the head, stay 0."""
@@ -291,13 +294,14 @@ class SbvrLlamaDecoder:
         with torch.cuda.stream(self.stream):
             fed = 0
             # (a probe looks at one step's residual stream at a time)
-            while self.prompt_rows and self.probe is None and len(prompt) - fed > self.prompt_rows:
-                self.rows_tok.copy_(prompt[fed:fed + self.prompt_rows])
-                if self.graph is not None and self.graph_rows is not None:
-                    self.graph_rows.replay()
-                else:
-                    self._rows_step()
-                fed += self.prompt_rows
+            for rows in (2 * self.prompt_rows, self.prompt_rows) if self.prompt_rows and self.probe is None else ():
+                while len(prompt) - fed > rows:
+                    self.rows_tok[:rows].copy_(prompt[fed:fed + rows])
+                    if self.graph is not None and rows in self.graph_rows:
+                        self.graph_rows[rows].replay()
+                    else:
+                        self._rows_step(rows)
+                    fed += rows
             for t in range(fed, len(prompt)):
                 self.tok.copy_(prompt[t:t + 1])
                 self._advance()

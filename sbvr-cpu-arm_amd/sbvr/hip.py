@@ -560,7 +560,7 @@ def dec_attention_o(qkv, cos, sin, pos, kcache, vcache, heads, kv_heads, head_di
     return out
 
 
-DEC_ROWS = 4                                  # tokens of a prompt that a launch takes at most
+DEC_ROWS = 8                                  # tokens of a prompt that a launch takes at most
 _ROWS_ADD_RMSNORM, _ROWS_SWIGLU, _ROWS_HEADS = 1, 2, 3
 
 
