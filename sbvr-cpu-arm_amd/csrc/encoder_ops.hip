@@ -965,10 +965,11 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
 // for 2, 3 and 4 planes (S), otherwise plane by plane in fp32 (S = 0: any number of planes).  Eight words of a row are 512
 // bytes of output; the 64-byte pieces of the lanes go through 4 KiB of LDS to lanes that follow each other along a
 // row, so that a store instruction writes two runs of 512 bytes.  Bound by memory: 2 bytes out per weight against S / 8
-// in.  An index beyond the table gives NaN (torch's indexing ends the process there).  4096 -> 14336, 4 planes: 27.8 us the
-// launch, 34.8 a call among others on weights that take turns = 4.2 TB/s, where a large copy reaches 5.2 (the torch
-// expression over unpacked 64-bit selectors took 4.4 ms); 2, 3, 6 and 8 planes 30.5, 32, 62 and 80 us the launch, the
-// last two bound by the vector ALU.
+// in.  An index beyond the table gives NaN (torch's indexing ends the process there).  4096 -> 14336, 4 planes: 29.6 us a call
+// among others on weights that take turns = 5.0 TB/s, where a large copy reaches 5.2 (the torch expression over unpacked
+// 64-bit selectors took 4.4 ms); 34.9 with the workgroups dealt out over the columns first, and 2 and 3 planes 22 and 23
+// where that took 28 and 30.  (Stores that pass the caches by: 27.0, but a copy of the result then took 47 where it takes
+// 33, so the caller would lose more than the call gains.)  6 and 8 planes: 66 and 80, bound by the vector ALU.
 struct DecodeArgs {
     const uint32_t *bvr;
     const uint8_t *idx;
@@ -999,7 +1000,13 @@ sbvr_decode_weight_kernel(const DecodeArgs a)
 {
     __shared__ v4u tiles[kDecWaves][256];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int w0 = (blockIdx.y * kDecWaves + wave) * 8, n0 = blockIdx.x * 8;
+    // Workgroups go to the 8 XCDs in turn: each takes a run of rows, along K first, so that what is written at one time is
+    // whole rows, and a cache line of plane words or indices that two windows of columns share is read by one L2.
+    unsigned lin = blockIdx.y * gridDim.x + blockIdx.x;
+    const unsigned run = gridDim.x * gridDim.y / 8;
+    if (lin < 8 * run)
+        lin = lin % 8 * run + lin / 8;
+    const int w0 = (lin % gridDim.y * kDecWaves + wave) * 8, n0 = lin / gridDim.y * 8;
     if (w0 >= a.words)                                        // wave-uniform; no barrier below
         return;
     v4u *const tile = tiles[wave];
