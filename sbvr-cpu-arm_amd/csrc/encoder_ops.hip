@@ -962,14 +962,17 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
 // rounded to fp16 once (reference sbvr/core.py:926-949), then converted to the tensor's own type (OUT: fp16, bf16
 // or fp32).  A wave takes 8 columns x 8 words of K: lane (n = lane % 8, word = lane / 8) loads its plane words (eight
 // neighbouring columns of a word are one or two cache lines) and decodes 32 weights in registers, by table look-up
-// for 2, 3 and 4 planes (S), otherwise plane by plane in fp32 (S = 0: any number of planes).  Eight words of a row are 512
+// for 2, 3 and 4 planes (S).  6 and 8 planes: two tables of fp32 sums a column in LDS, 8 or 16 entries each, where every such
+// sum is exact whatever its order (the table lines of all the wave's columns say so); otherwise, and for any other number
+// of planes (S = 0), plane by plane in fp32.  Eight words of a row are 512
 // bytes of output; the 64-byte pieces of the lanes go through 4 KiB of LDS to lanes that follow each other along a
 // row, so that a store instruction writes two runs of 512 bytes.  Bound by memory: 2 bytes out per weight against S / 8
 // in.  An index beyond the table gives NaN (torch's indexing ends the process there).  4096 -> 14336, 4 planes: 29.6 us a call
 // among others on weights that take turns = 5.0 TB/s, where a large copy reaches 5.2 (the torch expression over unpacked
 // 64-bit selectors took 4.4 ms); 34.9 with the workgroups dealt out over the columns first, and 2 and 3 planes 22 and 23
 // where that took 28 and 30.  (Stores that pass the caches by: 27.0, but a copy of the result then took 47 where it takes
-// 33, so the caller would lose more than the call gains.)  6 and 8 planes: 66 and 80, bound by the vector ALU.
+// 33, so the caller would lose more than the call gains.)  6 and 8 planes: 32 and 40, plane by plane 67 and 82, bound by the
+// vector ALU.
 struct DecodeArgs {
     const uint32_t *bvr;
     const uint8_t *idx;
@@ -998,7 +1001,9 @@ template <int S, int OUT>
 __global__ void __launch_bounds__(64 * kDecWaves)
 sbvr_decode_weight_kernel(const DecodeArgs a)
 {
-    __shared__ v4u tiles[kDecWaves][256];
+    constexpr bool kSums = S > 4;                 // two tables of fp32 sums
+    constexpr int H = kSums ? S / 2 : 4;          // planes of each
+    __shared__ v4u tiles[kDecWaves][S == 8 ? 512 : 256];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // Workgroups go to the 8 XCDs in turn: each takes a run of rows, along K first, so that what is written at one time is
     // whole rows, and a cache line of plane words or indices that two windows of columns share is read by one L2.
@@ -1016,7 +1021,83 @@ sbvr_decode_weight_kernel(const DecodeArgs a)
     const int lo = a.idx[at], hi = a.idx[at + a.idx16];
     const int line_read = a.idx16 ? lo | (hi << 8) : lo, line = min(line_read, a.L - 1);
     uint32_t D[16];                                           // elements 2i, 2i + 1 of the word
-    if constexpr (S != 0) {
+    // any planes, in their order
+    auto plane_by_plane = [&]() __attribute__((always_inline)) {
+        float w[32];
+#pragma unroll
+        for (int i = 0; i < 32; ++i)
+            w[i] = 0.f;
+        const uint32_t *src = a.bvr + (static_cast<size_t>(word) * a.N + n) * a.S;
+        const uint16_t *cs = a.cache + static_cast<size_t>(line) * a.S;
+#pragma unroll 1
+        for (int j = 0; j < a.S; ++j) {
+            const int bits = static_cast<int>(src[j]);
+            const uint32_t c = __float_as_uint(h2f(cs[j])), without = not_finite(cs[j]) ? 0x7fc00000u : 0u;   // (0 * c)
+#pragma unroll
+            for (int i = 0; i < 32; ++i) {
+                const uint32_t set = static_cast<uint32_t>(__builtin_amdgcn_sbfe(bits, i, 1));
+                w[i] += __uint_as_float((set & c) | (~set & without));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            D[i] = static_cast<uint32_t>(f2h(w[2 * i])) | (static_cast<uint32_t>(f2h(w[2 * i + 1])) << 16);
+    };
+    if constexpr (kSums) {
+        const Planes<S> pl = load_planes<S>(a.bvr + (static_cast<size_t>(word) * a.N + n) * S);
+        uint32_t c[(S + 1) / 2];
+        load_line_words<S>(a.cache + static_cast<size_t>(line) * S, c);
+        // Coefficients are multiples of 2^(least - 25) below 2^(most - 14), by their exponents.  Where these differ by 10 at
+        // most, a sum of eight is a number of 24 bits of that unit: exact, so in whatever order it is added up.
+        float f[S];
+        int most = 0, least = 31;
+#pragma unroll
+        for (int j = 0; j < S; ++j) {
+            const uint16_t h = static_cast<uint16_t>(j & 1 ? c[j / 2] >> 16 : c[j / 2]);
+            f[j] = h2f(h);
+            const int e = max((h >> 10) & 31, 1);
+            most = max(most, e);
+            least = (h & 0x7fff) != 0 ? min(least, e) : least;
+        }
+        if (__all(most < 31 && most - least <= 10)) {
+            // tables of the lane's own column: [low, high planes][sum][lane], no two lanes of a read in one bank
+            float *const sums = reinterpret_cast<float *>(tile) + lane;
+            uint32_t nibbles[2][4];           // nibble i of [.][p]: the planes' bits of element p + 4 i
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                float s[1 << H];
+                s[0] = 0.f;
+#pragma unroll
+                for (int b = 0; b < H; ++b)
+#pragma unroll
+                    for (int i = 0; i < 1 << b; ++i)
+                        s[(1 << b) + i] = s[i] + f[half * H + b];
+#pragma unroll
+                for (int i = 0; i < 1 << H; ++i)
+                    sums[((half << H) + i) * 64] = s[i];
+                const uint32_t *const w = pl.w + half * H;
+                const uint32_t w3 = H == 4 ? w[H - 1] : 0u;
+                const uint32_t even = bit_select(0x55555555u, w[0], w[1] << 1), odd = bit_select(0x55555555u, w[0] >> 1, w[1]);
+                const uint32_t even2 = bit_select(0x55555555u, w[2], w3 << 1), odd2 = bit_select(0x55555555u, w[2] >> 1, w3);
+                nibbles[half][0] = bit_select(0x33333333u, even, even2 << 2);
+                nibbles[half][1] = bit_select(0x33333333u, odd, odd2 << 2);
+                nibbles[half][2] = bit_select(0x33333333u, even >> 2, even2);
+                nibbles[half][3] = bit_select(0x33333333u, odd >> 2, odd2);
+            }
+            __builtin_amdgcn_wave_barrier();
+            auto weight = [&](int p, int i) __attribute__((always_inline)) -> float {
+                constexpr uint32_t kMask = (1u << H) - 1u;
+                return sums[((nibbles[0][p] >> (4 * i)) & kMask) * 64] + sums[((nibbles[1][p] >> (4 * i)) & kMask) * 64 + (64 << H)];
+            };
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                D[i] = static_cast<uint32_t>(f2h(weight(2 * (i & 1), i >> 1))) |
+                       (static_cast<uint32_t>(f2h(weight(2 * (i & 1) + 1, i >> 1))) << 16);
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            plane_by_plane();
+        }
+    } else if constexpr (S != 0) {
         const Planes<S> pl = load_planes<S>(a.bvr + (static_cast<size_t>(word) * a.N + n) * S);
         uint32_t c[(S + 1) / 2];
         load_line_words<S>(a.cache + static_cast<size_t>(line) * S, c);
@@ -1048,24 +1129,7 @@ sbvr_decode_weight_kernel(const DecodeArgs a)
             }
         }
     } else {
-        float w[32];
-#pragma unroll
-        for (int i = 0; i < 32; ++i)
-            w[i] = 0.f;
-        const uint32_t *src = a.bvr + (static_cast<size_t>(word) * a.N + n) * a.S;
-        const uint16_t *cs = a.cache + static_cast<size_t>(line) * a.S;
-        for (int j = 0; j < a.S; ++j) {
-            const int bits = static_cast<int>(src[j]);
-            const uint32_t c = __float_as_uint(h2f(cs[j])), without = not_finite(cs[j]) ? 0x7fc00000u : 0u;   // (0 * c)
-#pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                const uint32_t set = static_cast<uint32_t>(__builtin_amdgcn_sbfe(bits, i, 1));
-                w[i] += __uint_as_float((set & c) | (~set & without));
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            D[i] = static_cast<uint32_t>(f2h(w[2 * i])) | (static_cast<uint32_t>(f2h(w[2 * i + 1])) << 16);
+        plane_by_plane();
     }
     if (line_read >= a.L)
 #pragma unroll
@@ -1327,6 +1391,10 @@ int sbvr_hip_decode_weight(const uint32_t *bvr, const void *idx, int idx_bytes, 
         launch_decode<3>(out_type, grid, st, a);
     else if (aligned && S == 2)
         launch_decode<2>(out_type, grid, st, a);
+    else if (aligned && S == 6)
+        launch_decode<6>(out_type, grid, st, a);
+    else if (aligned && S == 8)
+        launch_decode<8>(out_type, grid, st, a);
     else
         launch_decode<0>(out_type, grid, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -3;
