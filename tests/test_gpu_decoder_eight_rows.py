@@ -15,17 +15,20 @@ pytestmark = pytest.mark.gpu
     # (hidden sizes with the one-launch head, which is what fills `logits`)
     (dict(hidden=2048, layers=2, heads=16, kv_heads=4, ffn=5632, vocab=1000), 3, 128, 90, True),
 ])
-def test_eight_prompt_rows_leave_what_single_steps_leave(shape, S, G, prompt, capture):
+def test_eight_prompt_rows_leave_what_single_steps_leave(shape, S, G, prompt, capture, monkeypatch):
     """The caches bit for bit, the tokens and the logits of the prompt fed token by token."""
+    from sbvr import hip
     from sbvr.decoder import LlamaShape, SbvrLlamaDecoder
-    made = []
+    made, passes = [], []
+    # (a wrapper around the module's function: one around the decoder's own method would make a reference cycle of it, whose
+    # recorded graphs the garbage collector might then end in the middle of the next decoder's recording, which aborts)
+    advance = hip.dec_rows_advance
+    monkeypatch.setattr(hip, "dec_rows_advance", lambda pos, rows, *rest: (passes.append(rows), advance(pos, rows, *rest)))
     tokens = torch.randint(0, shape["vocab"], (prompt,), generator=torch.Generator().manual_seed(prompt))
     for rows in (True, False):
         dec = SbvrLlamaDecoder(LlamaShape(**shape), "cuda:0", num_sums=S, bvr_len=G, max_seq=128, seed=5)
         assert dec.attention_o and dec.prompt_rows
-        passes = []
-        rows_step = dec._rows_step
-        dec._rows_step = lambda n: (passes.append(n), rows_step(n))
+        passes.clear()
         if not rows:
             dec.prompt_rows = 0
         if capture:
