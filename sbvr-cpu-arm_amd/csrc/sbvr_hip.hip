@@ -288,11 +288,11 @@ constexpr int kXPlanes = 5;
 //           (5 rows on: the 32-row kernels).  One thread per output, which took them before, 4096 -> 14336, 4 planes,
 //           one row: 1067 us; here 6.7.  (12800 -> 731, 6 planes, one row 4911 and 5.0; 8192 -> 28672, 2 rows 2219 and 25.7.)
 constexpr int kXHalves = 6;
-// A prompt's tokens, up to 4 rows, with the sums of the one-row launches they stand for, bit for bit:
+// A prompt's tokens, up to 8 rows, with the sums of the one-row launches they stand for, bit for bit:
 //   kXSwiGLURows  kXSwiGLU for every row;
 //   kXPairs       x itself, the four waves' results added pairwise as the one-launch attention + projection adds its heads'.
-// Four rows cost little more than one (the weight stream is read once): a layer of an 8B
-// shape takes four tokens in 47 us where four steps take 157.
+// Four rows cost little more than one (the weight stream is read once), eight 1.5 times as much (a second row tile's
+// operands and MFMAs): a layer of an 8B shape takes four tokens in 47 us and eight in 70 where four steps take 157.
 constexpr int kXSwiGLURows = 7, kXPairs = 8;
 constexpr int kHalvesMaxRows = 4;
 constexpr int kNormChunksMax = 2;             // 16-byte chunks of x a thread sums for the norm, at most
@@ -1874,8 +1874,8 @@ hipError_t launch_rows32(int S, RowsArgs a, hipStream_t st)
 // took 84 us where this takes 19 (24 rows x 1304, K 19200, 8 planes), 37 and 25 (32 x 14336, K 4096, 8 planes), 72 and 52
 // (26 x 9346, K 10496, 6 planes in groups of 64); 5 to 8 rows in groups of 64: 12.4 and 7.6 (6 x 4096, K 4096, 4 planes).
 constexpr int kLutWaves = 8;
-// Batch rows from which the linear takes this kernel.  Measured at 4096 -> 14336 / 14336 -> 4096, 4 planes: 15.3-16.1 us
-// for any row count up to 16 (17.3-17.5 at 32; 11.4-12.5 with 2 planes, 12.6-13.7 with 3), against 11.7-12.5 us at
+// Batch rows from which the linear takes this kernel.  Measured at 4096 -> 14336 / 14336 -> 4096, 4 planes: 12.6 and 13.7 us
+// for any row count up to 16 (9.2 and 10.9 with 2 planes, 10.2 and 11.9 with 3), against 10.2-11.3 us at
 // 5..8 rows and 17.9-20.9 us at 9..16 rows for the decode kernels (13.6-16.0 with 2 planes, 19.6-22.5 with 3).
 constexpr int kLutMinRows = 9;
 
@@ -2090,27 +2090,31 @@ int lut_pairs_per_wg(int pairs, int ksplit)
     return ((pairs + ksplit - 1) / ksplit + 1) / 2 * 2;
 }
 
-// Workgroups along K: the cheapest of up to 16 parts that keep a word pair for every wave and give a CU two workgroups at
-// most.  Costs in units of 1 / 16 us: a word pair of a wave in a workgroup that has its CU to itself 6 + S, two workgroups on
-// a CU each 1.75 + S / 20 times as long, the accumulators 20 and 2 more for each part.  (Fitted to 225 shapes, 600 to 7000
-// columns, K 2048 to 20480, 2, 4 and 8 planes, 12 and 24 rows, each with 1 to 16 parts: within 0.6 % of the best of them on
-// average, 3 % slower in one of them than doubling the parts until the CUs are full, which it replaces: that was 12 %
-// from the best, the worst where it kept K whole up to 4096 a part (600 columns, K 10240, 4 planes: 8.3 us against 5.9
-// now) or gave some of the CUs a second workgroup (5000 columns, K 4096: 9.5 against 7.9).)
+// Workgroups along K: parts doubled until the column blocks fill the CUs, a wave keeping 4 word pairs and more; or the cheapest
+// number of up to 16 that keeps a pair for every wave and gives a CU two workgroups at most, where that is estimated 4 %
+// cheaper.  Costs in units of 1 / 16 us: a word pair of a wave in a workgroup that has its CU to itself 7 + S (an odd one at the
+// end half as much again, the loop takes two), two workgroups on a CU each 1.75 + S / 20 times as long, the accumulators 25 and
+// 2 more for each part.  (Fitted to 785 launches, 600 to 8192 columns, K 2048 to 28672, 2 to 8 planes, 12 and 24 rows, each with
+// 1 to 16 parts: 1 % from the best of them on average where doubling alone is 9.7 %, and slower than that by more than 2 % in
+// two, by 3.2 % in one.  Doubling was at its worst
+// where it kept K whole up to 4096 a part (600 columns, K 10240, 4 planes: 8.3 us against 5.9) or gave some of the CUs a
+// second workgroup (5000 columns, K 4096: 9.5 against 7.9).  Without the 4 %: 4096 columns, K 14336, 3 planes, in 4 parts, 12.7 us
+// against 11.8 in 2.)
 int lut_ksplit(int N, int K, int S, int cus)
 {
     const int blocks = (N + 31) / 32, pairs = K / 64;
-    int best = 1;
-    float best_cost = 0.f;
-    for (int ks = 1; ks <= 16 && (ks == 1 || (blocks * ks <= 2 * cus && pairs / ks >= kLutWaves)); ++ks) {
+    auto cost = [&](int ks) {
         const int of_wave = (lut_pairs_per_wg(pairs, ks) + kLutWaves - 1) / kLutWaves;
-        const float share = blocks * ks <= cus ? 1.f : 1.75f + 0.05f * S;
-        const float cost = of_wave * (6 + S) * share + (ks > 1 ? 20.f + 2.f * ks : 2.f);
-        if (ks == 1 || cost < best_cost) {
-            best_cost = cost;
+        return (of_wave + 0.5 * (of_wave % 2)) * (7 + S) * (blocks * ks <= cus ? 1. : 1.75 + 0.05 * S) + (ks > 1 ? 25. : 0.) + 2. * ks;
+    };
+    int doubled = 1, best = 1;
+    while (blocks * doubled < cus && pairs / (doubled * 2) >= 4 * kLutWaves && doubled < 16)
+        doubled *= 2;
+    for (int ks = 2; ks <= 16 && blocks * ks <= 2 * cus && pairs / ks >= kLutWaves; ++ks)
+        if (cost(ks) < cost(best))
             best = ks;
-        }
-    }
+    if (cost(best) > 0.96 * cost(doubled))
+        best = doubled;
     const int per_wg = lut_pairs_per_wg(pairs, best);       // (no workgroup without a pair)
     return (pairs + per_wg - 1) / per_wg;
 }

@@ -12,13 +12,14 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,S,G,L,bias,parts", [
     (9, 32, 28672, 4, 128, 256, False, 14),         # one block of columns, the most parts
     (17, 600, 20480, 3, 256, 300, True, 10),        # uint16 indices, bias
-    (32, 601, 14272, 2, 64, 256, False, 10),        # 223 word pairs: an odd number, the last part shorter
+    (32, 601, 14272, 2, 64, 256, False, 7),         # 223 word pairs: an odd number, the last part shorter
     (24, 1300, 10240, 8, 128, 256, True, 5),
     (12, 2399, 6144, 4, 128, 256, False, 3),
+    (12, 4096, 14336, 3, 128, 256, False, 2),       # one workgroup a CU, though four parts come out nearly the same
     (16, 3000, 20480, 4, 64, 768, False, 5),        # two workgroups on most CUs
     (31, 5000, 4096, 3, 128, 256, True, 1),         # 157 blocks, whole
-    (6, 200, 2048, 6, 64, 256, False, 4),           # 8 pairs for the 8 waves of a part, taken by twos: four idle
-    (20, 513, 960, 8, 64, 16, False, 1),            # one pair short of that for two parts
+    (6, 200, 4096, 6, 64, 256, False, 4),           # two word pairs a wave
+    (20, 513, 576, 8, 64, 16, False, 1),            # 9 pairs, taken by twos: three waves without one
 ])
 def test_k_in_parts(M, N, K, S, G, L, bias, parts):
     """Against the products with decode()'s weights in 64 bits, as every call's; the accumulators left clean."""
