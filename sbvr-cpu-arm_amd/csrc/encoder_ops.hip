@@ -164,8 +164,9 @@ sbvr_encoder_candidates_kernel(const CandidateArgs a)
 // is left to the host the search says in the other slot, for the settling launch alone.
 // A workgroup's search is bound by the vector ALU (3 packed operations per two points and value); a wave stops when
 // all of its 64 lines are above the best error known.  1024 x 4096, groups of 128, 4 planes (241 misses): 269 to 327 ms
-// with about 50 launches and two waits a miss, 14.6 to 17.2 here: 23 us a search (2.6e5 to 4.6e5 lines; 38 to 59 without
-// the bound), 23 us (5 to 33) to settle it over up to 32768 groups.  512 x 2048, 3 planes 117 -> 5.2 ms; 64 x 512, 2 planes 36.6 -> 2.4.
+// with about 50 launches and two waits a miss, 9.6 to 10.9 here: 22 us a search (2.6e5 to 4.6e5 lines; 38 to 59 without
+// the bound), 8 to settle it (windows of 2048 groups meet the table as their turn comes near; 23 with all of up to 32768 groups
+// behind a miss meeting every line).
 struct EncoderState {
     int lines, misses, history, status, miss;
     int uncovered;                       // written by the search for the settling launch behind it: the group is the host's
