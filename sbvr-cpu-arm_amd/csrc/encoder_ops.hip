@@ -847,6 +847,7 @@ long run_lines(const sbvr_hip_encoder_run &a, int wide, int S)
 // three-way minimum, 2.5 operations a point.  (16 rows x 4096, 256 points: the lane that fetched every point from
 // memory for itself took 20.5 us.)
 constexpr int kOnlineWaves = 4, kOnlineRows = 4;
+constexpr float kOnlineCoarse = 1.5f * 134217728.f;       // 1.5 x 2^27, whose neighbours are 2^4 away
 
 // kImage: also the encoded values as the A operands of sbvr_online_product_kernel (OnlineArgs), and a scale per group: the
 // power of two that puts the sum of the line's magnitudes below 2^15.
@@ -898,7 +899,7 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
                     const int up = exponent == 255 || exponent == 0 ? 0 : 141 - exponent;
                     ups[which] = __uint_as_float(static_cast<uint32_t>(127 + up) << 23);
                     if (blockIdx.y == 0)
-                        scales[g] = __uint_as_float(static_cast<uint32_t>(127 + 24 - up) << 23);
+                        scales[g] = __uint_as_float(static_cast<uint32_t>(127 + 14 - up) << 23);
                 }
             }
         } else {
@@ -933,8 +934,9 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
         }
         if constexpr (kImage) {                                                       // (K is a multiple of 128)
             const int at = k0 + lane, i = at & 15, which = lane >> 5 & (g1 != g0);
-            const float v = sums[which][sel] * ups[which] * __uint_as_float(static_cast<uint32_t>(127 - (i & 7)) << 23);
-            const _Float16 head = static_cast<_Float16>(v), rest = static_cast<_Float16>(v - static_cast<float>(head));
+            const float v = sums[which][sel] * ups[which], by = __uint_as_float(static_cast<uint32_t>(128 - (1 << online_bit(i))) << 23);
+            const float tall = v + kOnlineCoarse - kOnlineCoarse;                     // (a multiple of 2^4)
+            const _Float16 head = static_cast<_Float16>(tall * by), rest = static_cast<_Float16>((v - tall) * by);
             const uint32_t both = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, head)) | static_cast<uint32_t>(__builtin_bit_cast(uint16_t, rest)) << 16;
             const uint32_t other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(both), 16, 64));
             // lanes 0 to 15 of 32 store the pair's heads, lanes 16 to 31 the rests

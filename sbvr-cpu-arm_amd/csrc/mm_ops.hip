@@ -221,14 +221,20 @@ __device__ __forceinline__ float online_output(const OnlineArgs &a, int m, int n
 // ------------------------------------------------------- activations encoded on the fly, more than a few of them
 //
 // The left operand of that product is a dense matrix a_hat[m, k] = sum_l a_l(group) L_l[m, k]: its coefficient line belongs to
-// the group, not to the row, so the launch that encodes the activations leaves it as fp16 numbers too (two parts, 22
-// bits, in the order of the MFMA's A operand: OnlineImage), and the right planes' bits meet it as fp16 numbers: a word of
-// this layout holds 32 k of one column, and `word & 0x00010001 << i` is the pair (k = i, i + 16) as 2^(i - 24) each, a ready
-// dword of the B operand of v_mfma_f32_16x16x32_f16; the activations carry 2^-i.  So 16 left rows are one row tile of 8 MFMAs a
-// plane and 128 k, where their planes are 8 tiles above whose sums each want a multiplication: 17 operations a plane word
-// and 4 a plane's sums, against 7 + 20 for each of the 8 tiles.  A workgroup owns 16 columns and 16 RT rows; its W waves take
-// the sub-groups of 128 k in turn and meet in LDS.  Bound by latency, and by the image's way through the L1 (8 KiB a
-// sub-group and row tile, for every 16 columns).
+// the group, not to the row, so the launch that encodes the activations leaves it as fp16 numbers too (two parts, in the
+// order of the MFMA's A operand: OnlineArgs), and the right planes' bits meet it as fp16 numbers: a word of this layout holds
+// 32 k of one column, shifted it has the pair (k = i, i + 16) at the same exponent bit of either half, and one `and` leaves a ready
+// dword of the B operand of v_mfma_f32_16x16x32_f16, a power of two each that the activations carry the inverse of.  So 16 left
+// rows are one row tile of 8 MFMAs a plane and 128 k, where their planes are 8 tiles above whose sums each want a
+// multiplication: 19 operations a plane word and 12 a plane's sums, against 7 + 20 for each of the 8 tiles.  A workgroup owns 16
+// columns and 16 RT rows; its W waves take the sub-groups of 128 k in turn and meet in LDS.  Bound by latency, and by the
+// image's way through the L1 (8 KiB a sub-group and row tile, for every 16 columns).
+// As exact as the planes' own product, in front of the output's rounding and over the RMS output: 0.45 to 0.9e-7 where that has
+// 0.8 to 2.0e-7, 0.4 to 0.76e-7 and 0.5 to 0.76e-7 with input coefficients of one sign (16 to 64 rows, 2 to 8 planes, K 128 to 14336).
+// Each of these matters: powers of two that are normal numbers (the bits where they lie are subnormal ones, which the matrix cores
+// line up by their least exponent: 25e-7); sums of the first parts, exact, and of the second ones apart, and differences of planes
+// (in one sum: 2e-7 with coefficients of one sign, and 64 rows x 4096, K 4096 in 25.7 us where this takes 29.2); the waves' sums
+// added up in 64 bits.
 template <int SR, int RT, int W>
 __global__ void __launch_bounds__(64 * W)
 sbvr_online_product_kernel(const OnlineArgs a)
@@ -259,6 +265,9 @@ sbvr_online_product_kernel(const OnlineArgs a)
         const int line = min(a.r_idx16 ? s.lo | (s.hi << 8) : s.lo, a.Lr - 1);
         load_line_words<SR>(a.r_cache + static_cast<size_t>(line) * SR, s.c);
     };
+    auto coefficient = [&](const Stage &s, int j) __attribute__((always_inline)) -> float {
+        return h2f(static_cast<uint16_t>(j & 1 ? s.c[j / 2] >> 16 : s.c[j / 2] & 0xffffu));
+    };
     v4f y[RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t)
@@ -266,7 +275,7 @@ sbvr_online_product_kernel(const OnlineArgs a)
     auto compute = [&](int sg, const Stage &s) __attribute__((always_inline)) {
         // (asked for a sub-group ahead, in 32 registers more, the image's operands cost 1 us of 6.5)
         const v4u *const image = a.image + static_cast<size_t>(sg) * tiles * 512 + lane;
-        v4f D[SR][RT];
+        v4f D[2][SR][RT];                                            // of the activations' first parts and of the second ones
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             v4u A[RT][2];
@@ -276,29 +285,41 @@ sbvr_online_product_kernel(const OnlineArgs a)
                 for (int part = 0; part < 2; ++part)                 // (a tile past the last one repeats it)
                     A[t][part] = image[(min(t0 + t, tiles - 1) * 4 + u) * 128 + part * 64];
 #pragma unroll
-            for (int part = 0; part < 2; ++part)
+            for (int j = 0; j < SR; ++j) {
+                const uint32_t w = s.w.w[j];
+                v4u B;
 #pragma unroll
-                for (int j = 0; j < SR; ++j) {
-                    const uint32_t w = u < 2 ? s.w.w[j] : s.w.w[j] >> 8;
-                    v4u B;
+                for (int e = 0; e < 4; ++e) {
+                    const int i = 4 * u + e;
+                    B[e] = (i < 5 ? w << 10 : (i < 10 ? w << 5 : (i < 15 ? w : w >> 1))) & (0x04000400u << online_bit(i));
+                }
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        B[e] = w & (0x00010001u << (4 * (u & 1) + e));
+                for (int part = 0; part < 2; ++part)
 #pragma unroll
                     for (int t = 0; t < RT; ++t)
-                        D[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t][part]), __builtin_bit_cast(v8h, B),
-                                                                         u == 0 && part == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : D[j][t], 0, 0, 0);
-                }
+                        D[part][j][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t][part]), __builtin_bit_cast(v8h, B),
+                                                                               u == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : D[part][j][t], 0, 0, 0);
+            }
         }
+        // A column's coefficients may almost cancel where its planes' sums are large and alike (activations of one sign).  The first
+        // parts' sums are exact, so what two planes' differ by is: that meets the coefficients, and the first plane's sum theirs.
+        float all = 0.f;
 #pragma unroll
-        for (int j = 0; j < SR; ++j) {
-            const float c = h2f(static_cast<uint16_t>(j & 1 ? s.c[j / 2] >> 16 : s.c[j / 2] & 0xffffu)) * s.scale;
+        for (int j = 0; j < SR; ++j)
+            all += coefficient(s, j);
 #pragma unroll
-            for (int t = 0; t < RT; ++t)
+        for (int t = 0; t < RT; ++t)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    y[t][i] = fmaf(D[j][t][i], c, y[t][i]);
-        }
+            for (int i = 0; i < 4; ++i) {
+                float sum = D[1][0][t][i] * coefficient(s, 0);
+#pragma unroll
+                for (int j = 1; j < SR; ++j)
+                    sum = fmaf(D[1][j][t][i], coefficient(s, j), sum);
+#pragma unroll
+                for (int j = 1; j < SR; ++j)
+                    sum = fmaf(D[0][j][t][i] - D[0][0][t][i], coefficient(s, j), sum);
+                y[t][i] = fmaf(fmaf(D[0][0][t][i], all, sum), s.scale, y[t][i]);
+            }
     };
     if (wave < nsub) {                                               // wave-uniform
         Stage now, next;
@@ -322,10 +343,11 @@ sbvr_online_product_kernel(const OnlineArgs a)
         const int m = t0 * 16 + (o >> 4), nn = blockIdx.x * 16 + (o & 15);
         if (m >= a.M || nn >= N)
             continue;
-        float total = 0.f;
+        double all_waves = 0.;
 #pragma unroll
         for (int w = 0; w < W; ++w)
-            total += red[w * RT * 256 + o];
+            all_waves += static_cast<double>(red[w * RT * 256 + o]);
+        float total = static_cast<float>(all_waves);
         if (!(fabsf(total) < INFINITY))                              // coefficients that are not finite: plane by plane, as above
             total = online_output<SR>(a, m, nn);
         uint16_t v = f2h(total);
@@ -335,20 +357,25 @@ sbvr_online_product_kernel(const OnlineArgs a)
     }
 }
 
+template <int SR, int RT, int W>
+hipError_t launch_online_inst(const OnlineArgs &a, hipStream_t st)
+{
+    const dim3 grid(static_cast<unsigned>((a.N + 15) / 16), static_cast<unsigned>((a.M + 16 * RT - 1) / (16 * RT)));
+    hipLaunchKernelGGL((sbvr_online_product_kernel<SR, RT, W>), grid, dim3(64 * W), 0, st, a);
+    return hipGetLastError();
+}
+
+// (two row tiles of more planes: 134 to 256 registers; more than 4 planes of a 16-wave workgroup: more than its 128)
 template <int SR>
 hipError_t launch_online(int RT, int W, const OnlineArgs &a, hipStream_t st)
 {
-    const int tiles = (a.M + 15) / 16;
-    const dim3 grid(static_cast<unsigned>((a.N + 15) / 16), static_cast<unsigned>((tiles + RT - 1) / RT)), block(64 * W);
-    if (RT == 1 && W == 16)
-        hipLaunchKernelGGL((sbvr_online_product_kernel<SR, 1, 16>), grid, block, 0, st, a);
-    else if (RT == 1)
-        hipLaunchKernelGGL((sbvr_online_product_kernel<SR, 1, 8>), grid, block, 0, st, a);
-    else if (SR <= 4 && W == 16)
-        hipLaunchKernelGGL((sbvr_online_product_kernel<(SR <= 4 ? SR : 4), 2, 16>), grid, block, 0, st, a);
-    else                                 // (6 and 8 planes of two row tiles want more than a 16-wave workgroup's 128 registers)
-        hipLaunchKernelGGL((sbvr_online_product_kernel<SR, 2, 8>), grid, dim3(512), 0, st, a);
-    return hipGetLastError();
+    if constexpr (SR == 2)
+        if (RT == 2)
+            return W == 16 ? launch_online_inst<SR, 2, 16>(a, st) : launch_online_inst<SR, 2, 8>(a, st);
+    if constexpr (SR <= 4)
+        if (W == 16)
+            return launch_online_inst<SR, 1, 16>(a, st);
+    return launch_online_inst<SR, 1, 8>(a, st);
 }
 
 template <int SR>
@@ -406,22 +433,27 @@ hipError_t launch_mm_T_mfma(int Sr, int G, MmArgs a, int cus, hipStream_t st)
     }
 }
 
-// Where that way is the faster one: more than 64 (left row, plane) pairs, of more than 4 planes a row, and workgroups for three
-// quarters of the CUs.  us a call (both launches), planes and this, 8 left and 4 right planes: 9 rows x 4096, K 4096 14.1
-// and 12.3; 64 rows 35.9 and 26.1; 32 x 14336, K 4096 52.6 and 34.9; 48 x 1024, K 14336 43.6 and 38.2, but 16 x 1024, K
-// 14336 17.4 and 23.0; 64 x 512, K 4096 15.8 and 17.5; 4 left planes, 32 x 4096, K 4096 12.2 and 12.9.
+// Where that way is the faster one: more than 4 left planes, workgroups for three quarters of the CUs, and row tiles for whose
+// rows the planes' launch takes a third more workgroups, of up to 64 (row, plane) pairs.  us a call (both launches), planes and
+// this, 8 left and 4 right planes: 9 rows x 4096, K 4096 13.5 and 12.3; 64 rows 35.9 and 29.2; 32 x 14336, K 4096 53.1 and
+// 39.4; 48 x 1024, K 14336 43.4 and 40.0; 2048 x 4096, K 4096 973 and 715; but (too few workgroups) 16 x 1024, K 14336 17.4 and
+// 23.0; 64 x 512, K 4096 15.8 and 17.5; (4 left planes) 32 x 4096, K 4096 12.2 and 12.9; (6 left planes: two workgroups, two tiles)
+// 20 rows 13.0 and 15.5.  At four workgroups to three tiles it is 0.8 to 1.35 times as fast, the mean of 140 shapes 1.
 bool online_product_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r_bvr, const void *r_cache, int cus)
 {
-    return mm_T_mfma_ok(M, N, K, Sl, Sr, G, r_bvr, r_cache) && Sl > 4 && Sl <= 8 && M * Sl > 64 && M <= 4096 &&
-           static_cast<long>((N + 15) / 16) * ((M + 15) / 16) * 4 >= 3L * cus &&
-           static_cast<double>(M + 15) / 16 * (K / kMmSub) * 512 < 2147483648.0;
+    const long tiles = (static_cast<long>(M) + 15) / 16;
+    return mm_T_mfma_ok(M, N, K, Sl, Sr, G, r_bvr, r_cache) && Sl > 4 && Sl <= 8 && M <= 4096 &&
+           3 * ((static_cast<long>(M) + 64 / Sl - 1) / (64 / Sl)) >= 4 * tiles && static_cast<long>((N + 15) / 16) * tiles * 4 >= 3L * cus &&
+           static_cast<double>(tiles) * (K / kMmSub) * 512 < 2147483648.0;
 }
 
+// Two row tiles share a plane word's operands where the registers hold both, with 2 planes.  (us a call, one and two, 64 rows x 4096, K
+// 4096: 4 planes 29.2 and 31.8, 3 planes, 33 rows 23.8 and 26.8.)
 hipError_t launch_online_product(int Sr, int G, OnlineArgs a, int cus, hipStream_t st)
 {
     a.spg = G / kMmSub;
     const int tiles = (a.M + 15) / 16, cols = (a.N + 15) / 16;
-    const int RT = tiles > 1 && static_cast<long>(cols) * ((tiles + 1) / 2) * 4 >= 3L * cus ? 2 : 1;
+    const int RT = Sr == 2 && tiles > 1 && static_cast<long>(cols) * ((tiles + 1) / 2) * 4 >= 3L * cus ? 2 : 1;
     const int W = static_cast<long>(cols) * ((tiles + RT - 1) / RT) >= 2L * cus ? 8 : 16;
     switch (Sr) {
     case 2: return launch_online<2>(RT, W, a, st);

@@ -26,10 +26,15 @@ struct MmArgs {
 bool mm_T_mfma_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r_bvr, const void *r_cache);
 hipError_t launch_mm_T_mfma(int Sr, int G, MmArgs a, int cus, hipStream_t st);
 
+// Activations encoded on the fly: which of the exponent's five bits (0 the lowest) of an fp16 number bit i of a plane word's half is
+// put on.  Alone there it is the normal number 2^(2^b - 15).
+__host__ __device__ constexpr int online_bit(int i) { return i == 15 ? 4 : i % 5; }
+
 // The same product with a left operand encoded on the fly (mm_ops.hip, encoder_ops.hip).  image: per sub-group of 128 k and row
 // tile of 16 the A operands of eight v_mfma_f32_16x16x32_f16, [u = 0..3][part][lane] of 16 bytes, dword e of lane (row r,
-// block b) the pair k = 32 b + 4 u + e, + 16, each the sum of its selected coefficients times the group's power of two times
-// 2^-((4 u + e) % 8), part 0 rounded to fp16, part 1 what is left.  scales: per group 2^24 over that power of two.
+// block b) the pair k = 32 b + 4 u + e, + 16, each the sum of its selected coefficients times the group's power of two (below
+// 2^15) in two parts, part 0 the nearest multiple of 2^4, part 1 what is left, both times 2^(1 - 2^online_bit(4 u + e)).  scales: per
+// group 2^14 over that power of two.
 struct OnlineArgs {
     const uint32_t *l_bvr;       // (K / 32, M, Sl)
     const uint16_t *lines;       // (K / G, Sl)
