@@ -894,12 +894,13 @@ sbvr_online_encode_kernel(const uint16_t *__restrict__ x, const uint16_t *__rest
                     float size = 0.f;
                     for (int j = 0; j < S; ++j)
                         size += fabsf(coeffs[which][j]);
-                    // (at least 2^-24 and below 2^19, or not finite: such outputs are added up plane by plane)
+                    // At least 2^-24 and below 2^19, or zero.  Or not finite: then the group's first point is NaN, every value
+                    // selects it, and no bit at all times that coefficient is NaN in every output.
                     const int exponent = static_cast<int>(__float_as_uint(size) >> 23);
                     const int up = exponent == 255 || exponent == 0 ? 0 : 141 - exponent;
                     ups[which] = __uint_as_float(static_cast<uint32_t>(127 + up) << 23);
                     if (blockIdx.y == 0)
-                        scales[g] = __uint_as_float(static_cast<uint32_t>(127 + 14 - up) << 23);
+                        scales[g] = exponent == 255 ? NAN : __uint_as_float(static_cast<uint32_t>(127 + 14 - up) << 23);
                 }
             }
         } else {

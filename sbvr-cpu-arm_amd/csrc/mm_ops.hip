@@ -190,34 +190,6 @@ sbvr_mm_T_mfma_kernel(const MmArgs a)
     }
 }
 
-// Output (m, n) by one lane from the planes of both sides, in the order of sbvr_mm_T_mfma_kernel: per group and left plane the
-// popcounts times the column's coefficients, then the left coefficient.
-template <int SR>
-__device__ __forceinline__ float online_output(const OnlineArgs &a, int m, int n)
-{
-    float y = 0.f;
-    const int words = 4 * a.spg;
-#pragma unroll 1
-    for (int g = 0; g < a.K / 32 / words; ++g) {
-        const uint8_t *rb = static_cast<const uint8_t *>(a.r_idx);
-        const size_t at = (static_cast<size_t>(g) * a.N + n) << a.r_idx16;
-        const int line = min(a.r_idx16 ? rb[at] | (rb[at + 1] << 8) : rb[at], a.Lr - 1);
-#pragma unroll 1
-        for (int l = 0; l < a.Sl; ++l) {
-            float sum = 0.f;
-#pragma unroll 1
-            for (int j = 0; j < SR; ++j) {
-                int count = 0;
-                for (int w = g * words; w < (g + 1) * words; ++w)
-                    count += __popc(a.l_bvr[(static_cast<size_t>(w) * a.M + m) * a.Sl + l] & a.r_bvr[(static_cast<size_t>(w) * a.N + n) * SR + j]);
-                sum = fmaf(static_cast<float>(count), h2f(a.r_cache[static_cast<size_t>(line) * SR + j]), sum);
-            }
-            y = fmaf(h2f(a.lines[static_cast<size_t>(g) * a.Sl + l]), sum, y);
-        }
-    }
-    return y;
-}
-
 // ------------------------------------------------------- activations encoded on the fly, more than a few of them
 //
 // The left operand of that product is a dense matrix a_hat[m, k] = sum_l a_l(group) L_l[m, k]: its coefficient line belongs to
@@ -272,6 +244,34 @@ sbvr_online_product_kernel(const OnlineArgs a)
 #pragma unroll
     for (int t = 0; t < RT; ++t)
         y[t] = v4f{0.f, 0.f, 0.f, 0.f};
+    // A sub-group by popcounts, as sbvr_mm_T_mfma_kernel has them, a left plane of all rows at a time: where a coefficient of one of
+    // the columns is not finite, a left plane that shares no bit with its plane makes NaN of the output (0 times infinity).
+    auto plane_by_plane = [&](int sg, const Stage &s) __attribute__((always_inline)) {
+#pragma unroll 1
+        for (int l = 0; l < a.Sl; ++l) {
+            const float c = h2f(a.lines[static_cast<size_t>(sg / a.spg) * a.Sl + l]);
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                const uint32_t left = a.l_bvr[(static_cast<size_t>(4 * sg + blk) * a.M + min((t0 + t) * 16 + col, a.M - 1)) * a.Sl + l];
+                const v8i A = {static_cast<int>((left << 2) & 0x44444444u), static_cast<int>(left & 0x22222222u),
+                               static_cast<int>((left >> 2) & 0x11111111u), static_cast<int>((left >> 3) & 0x11111111u), 0, 0, 0, 0};
+                v4f sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < SR; ++j) {
+                    const uint32_t w = s.w.w[j];
+                    const v8i B = {static_cast<int>(w & 0x11111111u), static_cast<int>(w & 0x22222222u), static_cast<int>(w & 0x44444444u),
+                                   static_cast<int>((w >> 1) & 0x44444444u), 0, 0, 0, 0};
+                    const v4f count = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(A, B, v4f{0.f, 0.f, 0.f, 0.f}, 4, 4, 0, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        sum[i] = fmaf(count[i], coefficient(s, j), sum[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    y[t][i] = fmaf(c, sum[i], y[t][i]);
+            }
+        }
+    };
     auto compute = [&](int sg, const Stage &s) __attribute__((always_inline)) {
         // (asked for a sub-group ahead, in 32 registers more, the image's operands cost 1 us of 6.5)
         const v4u *const image = a.image + static_cast<size_t>(sg) * tiles * 512 + lane;
@@ -304,9 +304,16 @@ sbvr_online_product_kernel(const OnlineArgs a)
         // A column's coefficients may almost cancel where its planes' sums are large and alike (activations of one sign).  The first
         // parts' sums are exact, so what two planes' differ by is: that meets the coefficients, and the first plane's sum theirs.
         float all = 0.f;
+        bool finite = true;
 #pragma unroll
-        for (int j = 0; j < SR; ++j)
+        for (int j = 0; j < SR; ++j) {
             all += coefficient(s, j);
+            finite = finite && fabsf(coefficient(s, j)) < INFINITY;
+        }
+        if (!__all(finite)) {
+            plane_by_plane(sg, s);
+            return;
+        }
 #pragma unroll
         for (int t = 0; t < RT; ++t)
 #pragma unroll
@@ -343,14 +350,11 @@ sbvr_online_product_kernel(const OnlineArgs a)
         const int m = t0 * 16 + (o >> 4), nn = blockIdx.x * 16 + (o & 15);
         if (m >= a.M || nn >= N)
             continue;
-        double all_waves = 0.;
+        double total = 0.;
 #pragma unroll
         for (int w = 0; w < W; ++w)
-            all_waves += static_cast<double>(red[w * RT * 256 + o]);
-        float total = static_cast<float>(all_waves);
-        if (!(fabsf(total) < INFINITY))                              // coefficients that are not finite: plane by plane, as above
-            total = online_output<SR>(a, m, nn);
-        uint16_t v = f2h(total);
+            total += static_cast<double>(red[w * RT * 256 + o]);
+        uint16_t v = f2h(static_cast<float>(total));
         if (a.bias)
             v = hadd(v, a.bias[nn]);
         a.out[static_cast<size_t>(m) * N + nn] = v;

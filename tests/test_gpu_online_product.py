@@ -79,8 +79,8 @@ def test_as_exact_as_plane_by_plane(N, K, S, Sl, G, sigma):
 
 
 def test_lines_that_are_not_finite():
-    """A group whose input coefficients hold an infinity and one with NaN: every output is finite, infinite or NaN as in the
-    planes' own product."""
+    """A group whose input coefficients hold an infinity: every output is finite, infinite or NaN as in the planes' own product
+    (NaN, all of them).  Without it, activations of which one is infinite and one NaN: finite outputs."""
     enc = _weight(3100, 768, 4, 128, 64, 8, 5)
     lines = enc.input_coeff.data.clone()
     lines[2, 3] = float("inf")
@@ -93,3 +93,27 @@ def test_lines_that_are_not_finite():
     lines[2, 3] = 1.0
     y, want = enc.online_mm_T(x), enc._online_mm_T_general(x, None)
     assert want.isfinite().all() and (y.float() - want.float()).abs().max() <= 2.0 ** -9 * max(1.0, want.float().abs().max().item())
+
+
+@pytest.mark.parametrize("M,N,K,S,G", [(16, 3100, 768, 4, 128), (33, 3100, 768, 2, 256), (20, 3100, 512, 8, 256)])
+def test_weights_that_are_not_finite(M, N, K, S, G):
+    """A line of the weight's table with an infinity, one with NaN and one with an infinity whose plane has no bits in the second half
+    of a group, which only some columns use: these outputs are infinite or NaN as in the planes' own product, which adds up 128
+    elements at a time; all others finite and as exact."""
+    enc = _weight(N, K, S, G, 64, 8, 5)
+    cache, idx, bvr = enc.coeff_cache.data.clone(), enc.coeff_idx.data.clone(), enc.bvr.data.clone()
+    cache[5, 1], cache[9, 0], cache[12, 1] = float("inf"), float("nan"), float("inf")
+    idx[idx == 5], idx[idx == 9], idx[idx == 12] = 1, 1, 1
+    idx[1, 100:2000:7], idx[0, 103:2000:70], idx[1, 3::9] = 5, 9, 12
+    if G > 128:
+        bvr.view(torch.int32)[(G + 128) // 32:2 * G // 32, 3::9, 1] = 0
+    enc.coeff_cache, enc.coeff_idx, enc.bvr = (torch.nn.Parameter(t, requires_grad=False) for t in (cache, idx, bvr))
+    enc.input_coeff = torch.nn.Parameter(enc.input_coeff.data.abs(), requires_grad=False)           # (of both signs: NaN, not infinite)
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(1)).abs().to(torch.float16).to("cuda:0")
+    assert _taken(enc, x, G)
+    y, want = enc.online_mm_T(x), enc._online_mm_T_general(x, None)
+    assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.isposinf(), want.isposinf()) and torch.equal(y.isneginf(), want.isneginf())
+    assert 0 < want.isinf().sum() < want.numel() / 2 and 0 < want.isnan().sum() < want.numel() / 2
+    finite = want.isfinite()
+    rms = want[finite].float().pow(2).mean().sqrt().item()
+    assert (y[finite].float() - want[finite].float()).abs().max() <= 2.0 ** -9 * max(rms, want[finite].float().abs().max().item())
