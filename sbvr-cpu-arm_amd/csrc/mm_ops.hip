@@ -442,13 +442,15 @@ hipError_t launch_mm_T_mfma(int Sr, int G, MmArgs a, int cus, hipStream_t st)
 // this, 8 left and 4 right planes: 9 rows x 4096, K 4096 13.5 and 12.3; 64 rows 35.9 and 29.2; 32 x 14336, K 4096 53.1 and
 // 39.4; 48 x 1024, K 14336 43.4 and 40.0; 2048 x 4096, K 4096 973 and 715; but (too few workgroups) 16 x 1024, K 14336 17.4 and
 // 23.0; 64 x 512, K 4096 15.8 and 17.5; (4 left planes) 32 x 4096, K 4096 12.2 and 12.9; (6 left planes: two workgroups, two tiles)
-// 20 rows 13.0 and 15.5.  At four workgroups to three tiles it is 0.8 to 1.35 times as fast, the mean of 140 shapes 1.
+// 20 rows 13.0 and 15.5.  At four workgroups to three tiles it is 0.8 to 1.35 times as fast, the mean of 140 shapes 1.  Images (4
+// bytes an activation, in memory of the call's own) up to the largest measured: 2048 x 1024, K 14336 1287 us and 1142.
+constexpr double kOnlineImageMost = 128 << 20;
 bool online_product_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r_bvr, const void *r_cache, int cus)
 {
     const long tiles = (static_cast<long>(M) + 15) / 16;
     return mm_T_mfma_ok(M, N, K, Sl, Sr, G, r_bvr, r_cache) && Sl > 4 && Sl <= 8 && M <= 4096 &&
            3 * ((static_cast<long>(M) + 64 / Sl - 1) / (64 / Sl)) >= 4 * tiles && static_cast<long>((N + 15) / 16) * tiles * 4 >= 3L * cus &&
-           static_cast<double>(tiles) * (K / kMmSub) * 512 < 2147483648.0;
+           static_cast<double>(tiles) * (K / kMmSub) * 8192 <= kOnlineImageMost;
 }
 
 // Two row tiles share a plane word's operands where the registers hold both, with 2 planes.  (us a call, one and two, 64 rows x 4096, K

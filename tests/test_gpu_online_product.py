@@ -117,3 +117,13 @@ def test_weights_that_are_not_finite(M, N, K, S, G):
     finite = want.isfinite()
     rms = want[finite].float().pow(2).mean().sqrt().item()
     assert (y[finite].float() - want[finite].float()).abs().max() <= 2.0 ** -9 * max(rms, want[finite].float().abs().max().item())
+
+
+@pytest.mark.parametrize("M,K,taken", [(2048, 16384, True), (2049, 16384, False), (4096, 8192, True), (4096, 8320, False)])
+def test_memory_of_the_call_is_bounded(M, K, taken):
+    """The activations as fp16 numbers take 128 MiB at most; beyond, the planes' own product needs their planes alone."""
+    from sbvr import hip
+    ask = hip._load().sbvr_hip_online_mm_T_scratch
+    ask.restype, ask.argtypes = ctypes.c_size_t, [ctypes.c_void_p] * 2 + [ctypes.c_int] * 6
+    need = ask(64, 64, M, 4096, K, 8, 4, 128)
+    assert (need > 0) == taken and need <= (128 << 20) + M * K + 4 * K
