@@ -39,11 +39,12 @@ int sbvr_hip_encoder_candidates_f16(const void *data, int G, const void *base, i
  * quantile and mean; table (table_lines, S) fp16; best (groups) fp32 and line (groups), the least error over the
  * table's lines and the first line that has it (infinity and -1 without lines); line_of (groups) and sel (groups, G), what
  * comes out; settled (groups), zeros; history, the errors of the searches so far, with room for one more per group; and
- * state, sbvr_hip_encoder_state_bytes() bytes: two slots of {int lines, misses, history, status, miss, 0; uint64
- * found}, then {int covered of slot 0, of slot 1}.  Slot 0 starts as {lines in the table, groups so far that were no table
- * hits, errors in `history`, 0, miss, 0, all ones}: best and line of the groups below `covered` are over all lines (miss 0, covered 0, or 1 with an empty table, is a start), and
- * miss is the first of them that misses, or covered.  A round that finds miss at covered lets the next groups meet the table.
- * A round reads slot (and leaves it but for `found`) and writes the other.  Afterwards the slot that the last round wrote
+ * state, sbvr_hip_encoder_state_bytes() bytes: two slots of {int lines, misses, history, status, miss, unmet; uint64
+ * found}.  Slot 0 starts as {lines in the table, groups so far that were no table hits, errors in `history`, 0, the first
+ * group that misses, 0, all ones}.  Or with the last `unmet` groups to meet the table still, a window of them at a time as their turn
+ * comes near: best and line are then over all lines for the groups in front of them (none of which need there be where the
+ * table has lines), and miss is the first of those that misses, or groups - unmet.  A round reads slot (and
+ * leaves it but for `found`) and writes the other.  Afterwards the slot that the last round wrote
  * holds the same; miss >= groups: nothing misses any more; status 1: group `miss` is left to the caller.
  * [0] and [1]: the plainer and the wider search: base (bases, S) and offsets fp16 as for
  * sbvr_hip_encoder_candidates_f16, axis_values values per axis of the grid.  scale_step, scale_narrow: 1 / number of scales,

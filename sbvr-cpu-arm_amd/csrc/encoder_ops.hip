@@ -161,7 +161,8 @@ sbvr_encoder_candidates_kernel(const CandidateArgs a)
 // those behind a group whose candidates these kernels do not form (status 1: the host takes that group through
 // the general path).  State: two slots, read one and written the other by turns, so that workgroups of a launch never
 // read what it changes, but for `found` of the slot read, which the search takes minima into (and reads as a bound).  That a group
-// is left to the host the search says in the other slot, for the settling launch alone.
+// is left to the host the search says in the other slot, for the settling launch: its group is this one already, where otherwise
+// it is one behind.
 // A workgroup's search is bound by the vector ALU (3 packed operations per two points and value); a wave stops when
 // all of its 64 lines are above the best error known.  1024 x 4096, groups of 128, 4 planes (241 misses): 269 to 327 ms
 // with about 50 launches and two waits a miss, 9.6 to 10.9 here: 22 us a search (2.6e5 to 4.6e5 lines; 38 to 59 without
@@ -169,12 +170,8 @@ sbvr_encoder_candidates_kernel(const CandidateArgs a)
 // behind a miss meeting every line).
 struct EncoderState {
     int lines, misses, history, status, miss;
-    int uncovered;                       // written by the search for the settling launch behind it: the group is the host's
+    int unmet;                           // groups at the end that have not met the table; those in front have met all of its lines
     unsigned long long found;            // error's bits << 32 | candidate: the least so far (all ones: none)
-};
-struct EncoderStates {
-    EncoderState slot[2];
-    int covered[2];                      // of either slot: groups below it have met every line of the table
 };
 
 constexpr int kEncMaxScales = 160, kEncMaxAxes = 4096;    // scales of a search, values of all its axes, at most
@@ -468,9 +465,9 @@ sbvr_encoder_search_kernel(const sbvr_hip_encoder_run a, int slot)
 {
     __shared__ __align__(16) SearchSpace sp;
     __shared__ unsigned long long least[kEncThreads / 64];
-    EncoderState *const states = static_cast<EncoderStates *>(a.state)->slot;
+    EncoderState *const states = static_cast<EncoderState *>(a.state);
     const EncoderState st = states[slot];
-    const int have_met = static_cast<EncoderStates *>(a.state)->covered[slot];
+    const int have_met = a.groups - st.unmet;
     const bool idle = st.status != 0 || st.miss >= have_met, extends = st.status == 0 && idle && have_met < a.groups;
     const int tid = threadIdx.x;
     const float known = idle || st.lines < a.warmup ? INFINITY : a.best[st.miss];
@@ -481,7 +478,6 @@ sbvr_encoder_search_kernel(const sbvr_hip_encoder_run a, int slot)
         const bool stays = idle ? !extends : !sp.covered;
         states[slot ^ 1].miss = stays ? st.miss : kEncNone;
         states[slot ^ 1].found = ~0ull;
-        states[slot ^ 1].uncovered = !idle && !sp.covered;
     }
     if (idle || !sp.covered)
         return;
@@ -573,7 +569,7 @@ __device__ __forceinline__ void winner(const sbvr_hip_encoder_run &a, const Enco
 // that has it.
 template <int S>
 __device__ __forceinline__ void meet_table(const sbvr_hip_encoder_run &a, const EncoderState &st, int have_met, EncoderState *other,
-                                           int *other_met, uint16_t *group, unsigned long long *least, double *part)
+                                           uint16_t *group, unsigned long long *least, double *part)
 {
     const int tid = threadIdx.x, end = min(a.groups, have_met + kEncWindow);
     const bool looks = st.lines >= a.warmup;
@@ -583,7 +579,7 @@ __device__ __forceinline__ void meet_table(const sbvr_hip_encoder_run &a, const 
         other->misses = st.misses;
         other->history = st.history;
         other->status = 0;
-        *other_met = end;
+        other->unmet = a.groups - end;
         atomicMin(&other->miss, looks ? end : have_met);
     }
     for (int g = have_met + static_cast<int>(blockIdx.x); g < end; g += static_cast<int>(gridDim.x)) {
@@ -642,27 +638,26 @@ sbvr_encoder_settle_kernel(const sbvr_hip_encoder_run a, int slot)
     __shared__ double part[kEncThreads];
     __shared__ unsigned long long least[kEncThreads / 64];
     __shared__ int twin, first_miss;
-    EncoderStates *const both = static_cast<EncoderStates *>(a.state);
-    EncoderState *const other = &both->slot[slot ^ 1];
-    const EncoderState st = both->slot[slot];
-    const int have_met = both->covered[slot];
+    EncoderState *const states = static_cast<EncoderState *>(a.state), *const other = &states[slot ^ 1];
+    const EncoderState st = states[slot];
+    const int have_met = a.groups - st.unmet;
     const int tid = threadIdx.x, m = st.miss;
     _Float16 *const table = static_cast<_Float16 *>(a.table);
     if (st.status == 0 && m >= have_met && have_met < a.groups) {
-        meet_table<S>(a, st, have_met, other, &both->covered[slot ^ 1], sh.group, least, part);
+        meet_table<S>(a, st, have_met, other, sh.group, least, part);
         return;
     }
     EncoderState next = st;                                            // (miss and found: written by the search and by minima)
     const bool found = st.found != ~0ull;
     // (nothing left, a group for the host, or one that neither the table nor any candidate has an error for: the state stays)
-    const bool uncovered = other->uncovered != 0;                      // (no workgroup of this launch writes it)
+    const bool uncovered = m < a.groups && other->miss == m;            // (what this launch takes minima of is behind m; or m, unserved)
     const bool stays = st.status != 0 || m >= a.groups || uncovered, unserved = !stays && !found && a.line[m] < 0;
     if (stays || unserved) {
         if (blockIdx.x == 0 && tid == 0) {
             other->lines = st.lines;
             other->misses = st.misses;
             other->history = st.history;
-            both->covered[slot ^ 1] = have_met;
+            other->unmet = st.unmet;
             other->status = unserved || uncovered ? 1 : st.status;
             if (unserved)
                 atomicMin(&other->miss, m);
@@ -724,7 +719,7 @@ sbvr_encoder_settle_kernel(const sbvr_hip_encoder_run a, int slot)
             other->lines = next.lines;
             other->misses = next.misses;
             other->history = next.history;
-            both->covered[slot ^ 1] = have_met;
+            other->unmet = st.unmet;
             other->status = 0;
             // (groups are searched one after the other until the table has its first lines)
             atomicMin(&other->miss, next.lines < a.warmup ? m + 1 : have_met);
@@ -1259,7 +1254,7 @@ int sbvr_hip_encoder_candidates_f16(const void *data, int G, const void *base, i
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-size_t sbvr_hip_encoder_state_bytes(void) { return sizeof(EncoderStates); }
+size_t sbvr_hip_encoder_state_bytes(void) { return 2 * sizeof(EncoderState); }
 
 int sbvr_hip_encoder_scales(int S, int G, int bases, int n_offsets, int axis_values)
 {

@@ -404,8 +404,7 @@ class GroupEncoder:
         # (groups below `covered` have met the whole table, and one that misses is looked for among them; the kernels take it on)
         def put(miss, covered):
             missed = c.group_idx - c.cache_hits
-            state.copy_(torch.tensor([c.num_coeff_cache_lines, missed, len(c.mse_history), 0, miss, 0, -1, -1] * 2 + [covered] * 2,
-                                     dtype=torch.int32))
+            state.copy_(torch.tensor([c.num_coeff_cache_lines, missed, len(c.mse_history), 0, miss, n - covered, -1, -1] * 2, dtype=torch.int32))
 
         def next_miss(first, covered):
             if c.num_coeff_cache_lines < c.cache_warmup_num:
@@ -419,9 +418,8 @@ class GroupEncoder:
         while miss < n:
             hip.encoder_rounds(run, S, max(lines), 0, rounds, dev)          # (an even number: the result is in slot 0 again)
             had = len(c.mse_history)
-            now = state.tolist()
-            c.num_coeff_cache_lines, missed, errors, status, miss = now[:5]
-            covered = now[-2]
+            c.num_coeff_cache_lines, missed, errors, status, miss, unmet = state[:6].tolist()
+            covered = n - unmet
             c.mse_history.extend(history[had:errors].tolist())
             c.group_idx, c.cache_hits = start + miss, start + miss - missed
             if progress is not None:

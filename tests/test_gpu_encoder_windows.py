@@ -22,3 +22,27 @@ def test_windows(groups, S, odd):
     w[::97] *= 30.0                             # (groups that the table does not serve, also far behind)
     stats = _encode_both_ways(w.to(torch.float16).to("cuda:0"), dict(num_sums=S, bvr_len=G, s_search_num=8, r_search_num=16, b_search_num=8))
     assert stats["groups"] == groups
+
+
+@pytest.mark.parametrize("groups", [300, 2500])
+def test_state_of_two_slots_all_groups_met(groups, monkeypatch):
+    """The state is two slots; one whose sixth word is 0 says that best and line are over all lines for all groups, as an empty
+    table's are, and is taken on from there without windows: the same arrays."""
+    import sys
+    from sbvr import hip
+    assert hip.encoder_state_words() == 16
+    real, started = hip.encoder_rounds, []
+
+    def rounds(run, S, lines, slot, many, device):
+        if not started:
+            state = sys._getframe(1).f_locals["state"]
+            assert state.tolist()[:5] == [0] * 5
+            state[5], state[13] = 0, 0
+            started.append(groups)
+        real(run, S, lines, slot, many, device)
+
+    monkeypatch.setattr(hip, "encoder_rounds", rounds)
+    w = torch.randn((groups, 32), generator=torch.Generator().manual_seed(groups)) * 0.02
+    w[5], w[::97] = w[5] + 2.0, w[::97] * 30.0
+    _encode_both_ways(w.to(torch.float16).to("cuda:0"), dict(num_sums=2, bvr_len=32, s_search_num=8, r_search_num=16, b_search_num=8))
+    assert started == [groups]
