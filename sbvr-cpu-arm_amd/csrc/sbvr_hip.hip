@@ -1207,8 +1207,13 @@ constexpr bool shape_ok_for(int MT, int CT, int SP)
 // Two row tiles (5 to 8 tokens of a prompt) with a launch shape of one batch row: the shapes above, and up to 4 planes the
 // widest window, whose units fill 116 registers then.  (Its 7 tiles are what reads a 4096 -> 28672 weight in one round.)
 constexpr int kWideTilesMaxPlanes = 4;
-constexpr bool two_tiles_ok(int S, int CT, int SP)
+constexpr bool two_tiles_ok(int S, int CT, int SP, int xm)
 {
+    // 8 planes, two sub-groups at a time: more than the registers hold (us for 8 rows, two tiles and four rows twice: SwiGLU
+    // 4 x 2, 14336 -> 4096 37.1 and 27.3, 28672 -> 8192 129 and 96; 2 x 2, 4096 -> 19840 56.8 and 54.1, but RMSNorm there 44.3
+    // and 52.7).  6 planes: 4 x 2 21.9 and 24.0, 76 and 82.
+    if (S == 8 && SP == 2 && (CT == 4 || (CT == 2 && xm == kXSwiGLURows)))
+        return false;
     return shape_ok_for(2, CT, SP) || (CT == 7 && SP == 2 && S <= kWideTilesMaxPlanes);
 }
 
@@ -5223,7 +5228,7 @@ int sbvr_hip_dec_rows_linear_f16(int prologue, const void *x, const void *delta,
     if (p.CT == 0)
         return fail(SBVR_HIP_EUNSUPPORTED, "no launch shape for N=%d K=%d S=%d", N, K, S);
     // 5 to 8 rows: two row tiles over the same plane words, where that shape has them, or four rows and the rest in turn
-    const bool two_tiles = rows > kRowTile && two_tiles_ok(S, p.CT, p.SP);
+    const bool two_tiles = rows > kRowTile && two_tiles_ok(S, p.CT, p.SP, xm);
     if (two_tiles) {
         p.MT = 2;
         p.lds = static_cast<size_t>(p.waves) * (2048 + (p.CT * p.MT <= 8 ? 0 : p.CT * p.MT * 256));
