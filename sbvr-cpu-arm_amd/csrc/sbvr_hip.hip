@@ -3930,7 +3930,9 @@ sbvr_attn_o_kernel(const AttnOArgs a)
     float *const a_scale = red_sum + kAoWaves;                             // [head]: 2^-(e+1) of its A operand
     float *const part = reinterpret_cast<float *>(smem + 2048);            // [position half][head][dimension]
     float *const ysum = reinterpret_cast<float *>(smem + 6144);            // [head][column of the window]
-    unsigned char *const abuf = smem + 8192;                               // the heads' A operand images, 2 KiB each
+    // the heads' A operand images, 2 KiB each (kRows: no projection, its values and the rest of its keys lie there)
+    unsigned char *const abuf = kRows ? nullptr : smem + 8192;
+    static_assert(6144 + 2 * kAoRowsMax * kAoHead * 2 <= kAoLdsFixed, "keys and values of a prompt's tokens");
     float *const scores = reinterpret_cast<float *>(smem + kAoLdsFixed);   // [head][position]
     uint16_t *const wts = reinterpret_cast<uint16_t *>(scores + kAoGroup * max_seq);   // [head][position], fp16
 
