@@ -47,6 +47,7 @@ const char *sbvr_hip_last_error(void);
 #define SBVR_HIP_KERNEL_PREFILL_SPLIT 5  /* the same with K split across workgroups (workspace given) */
 int sbvr_hip_last_kernel(void);
 int sbvr_hip_last_parts(void);           /* parts of K across workgroups of that launch (1: not split) */
+int sbvr_hip_last_row_blocks(void);      /* of the last prefill launch: row blocks of 32 of a workgroup (5 to 8: the kernel of prefill_ops.hip) */
 
 /* How that launch treated the weights (0 before the first):
  *   EXACT      coefficients applied to plane sums in fp32, no per-weight rounding (decode and portable kernels);
@@ -285,6 +286,7 @@ size_t sbvr_hip_row_deq_mm_T_workspace_for(int M, int N, int K, int S, int G);
 #define SBVR_HIP_ROW_DEQ_ROWS 4          /* several rows together: every weight decoded once, or (2 to 4) plane bits as they are */
 int sbvr_hip_row_deq_last_kernel(void);
 int sbvr_hip_row_deq_last_parts(void);
+int sbvr_hip_row_deq_last_turned(void);  /* SBVR_HIP_ROW_DEQ_ROWS: 1 where it took plane bits as they are */
 
 /*
  * Both operands SBVR-encoded (default uint32 layout on both sides):

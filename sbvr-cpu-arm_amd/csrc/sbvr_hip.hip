@@ -65,9 +65,11 @@ namespace {
 thread_local char g_err[256] = "";
 thread_local int g_last_kernel = 0;       // SBVR_HIP_KERNEL_* of the last linear launched from this thread
 thread_local int g_last_parts = 0;        // and its parts of K across workgroups
+thread_local int g_last_row_blocks = 0;   // row blocks of 32 of a workgroup of this thread's last prefill
 thread_local int g_last_rounding = 0;     // SBVR_HIP_ROUNDING_* of that launch
 thread_local int g_row_deq_kernel = 0;    // SBVR_HIP_ROW_DEQ_* of this thread's last transposed product
 thread_local int g_row_deq_parts = 0;     // and its parts of K across workgroups
+thread_local int g_row_deq_turned = 0;    // and whether it took plane bits as they are, turned by the matrix cores
 
 int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 int fail(int code, const char *fmt, ...)
@@ -4424,6 +4426,8 @@ int sbvr_hip_last_kernel(void) { return g_last_kernel; }
 
 int sbvr_hip_last_parts(void) { return g_last_parts; }
 
+int sbvr_hip_last_row_blocks(void) { return g_last_row_blocks; }
+
 int sbvr_hip_last_rounding(void) { return g_last_rounding; }
 
 int sbvr_hip_init(int device)
@@ -4734,6 +4738,7 @@ int linear_core(const void *x, const uint32_t *bvr, const void *coeff_idx,
             return fail(SBVR_HIP_ELAUNCH, "prefill (table look-up) launch: %s", hipGetErrorString(e));
         g_last_kernel = g.ksplit > 1 ? SBVR_HIP_KERNEL_PREFILL_SPLIT : SBVR_HIP_KERNEL_PREFILL;
         g_last_parts = g.ksplit;
+        g_last_row_blocks = plan.rb;
         // (6 and 8 planes: two entries added, closer than plane by plane.  Groups of 64: as decode() rounds, reported as the
         // looser of the two, which is what such a call has always said)
         g_last_rounding = S <= 4 && g.steps_per_group % 2 == 0 ? SBVR_HIP_ROUNDING_DECODE : SBVR_HIP_ROUNDING_PLANEWISE;
@@ -4881,6 +4886,7 @@ int sbvr_hip_row_deq_mm_T_ws(const void *x, const uint32_t *r_bvr, const void *r
             return fail(SBVR_HIP_ELAUNCH, "row_deq launch: %s", hipGetErrorString(e));
         g_row_deq_kernel = SBVR_HIP_ROW_DEQ_ROWS;
         g_row_deq_parts = a.ksplit;
+        g_row_deq_turned = few;
         return SBVR_HIP_OK;
     }
     if (row_deq_mfma_ok(M, K, S, G) && tables_aligned && reinterpret_cast<uintptr_t>(x) % 4 == 0 &&
@@ -4963,6 +4969,8 @@ int sbvr_hip_row_deq_mm_T(const void *x, const uint32_t *r_bvr, const void *r_co
 int sbvr_hip_row_deq_last_kernel(void) { return g_row_deq_kernel; }
 
 int sbvr_hip_row_deq_last_parts(void) { return g_row_deq_parts; }
+
+int sbvr_hip_row_deq_last_turned(void) { return g_row_deq_kernel == SBVR_HIP_ROW_DEQ_ROWS && g_row_deq_turned; }
 
 size_t sbvr_hip_row_deq_mm_T_workspace_for(int M, int N, int K, int S, int G)
 {

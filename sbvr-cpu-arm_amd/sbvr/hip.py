@@ -166,6 +166,12 @@ def last_parts():
     return _load().sbvr_hip_last_parts()
 
 
+def last_row_blocks():
+    """How many row blocks of 32 a workgroup of this thread's last prefill launch took (5 to 8: the kernel of
+    prefill_ops.hip)."""
+    return _load().sbvr_hip_last_row_blocks()
+
+
 ROUNDING_EXACT, ROUNDING_DECODE, ROUNDING_PLANEWISE = 1, 2, 3
 
 
@@ -183,6 +189,11 @@ def row_deq_last():
     """Which kernel the last transposed product of this thread launched (one of the ROW_DEQ_* codes), and in how many
     parts of K across workgroups."""
     return _load().sbvr_hip_row_deq_last_kernel(), _load().sbvr_hip_row_deq_last_parts()
+
+
+def row_deq_last_turned():
+    """Whether that was ROW_DEQ_ROWS with plane bits taken as they are (two to four rows)."""
+    return bool(_load().sbvr_hip_row_deq_last_turned())
 
 
 def _sbvr_hip_init(device=None):

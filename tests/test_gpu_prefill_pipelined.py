@@ -20,9 +20,16 @@ pytestmark = pytest.mark.gpu
     (700, 28417, 320, 6, 64, 256, False, 4),
     (512, 28433, 384, 8, 128, 256, True, 4),
     (512, 28672, 320, 8, 64, 256, False, 4),
-    (2048, 1001, 8192, 4, 128, 256, True, 5),          # K in parts, fp32 partial results at an odd width
+    (1458, 3075, 12800, 8, 256, 256, True, 5),         # K in parts, fp32 partial results at an odd width
+    (1983, 1644, 2816, 8, 64, 256, False, 5),          # seven row blocks
+    (1388, 2144, 4608, 4, 64, 256, False, 5),          # five
+    (403, 16386, 12544, 4, 256, 256, False, 5),        # parts that begin inside a group
+    (700, 5100, 11008, 3, 128, 256, False, 5),         # the last part shorter, three and two planes
+    (1400, 2050, 12288, 2, 64, 256, True, 5),
+    (400, 9000, 10240, 6, 128, 256, False, 5),
+    (2048, 1001, 8192, 4, 128, 256, True, 5),          # (parts of three and four row blocks, which sbvr_hip.hip's kernel takes)
     (1009, 2050, 6144, 3, 256, 256, False, 5),
-    (1300, 1025, 5376, 2, 64, 256, False, 5),          # parts of an even number of steps, the last one shorter
+    (1300, 1025, 5376, 2, 64, 256, False, 5),
 ])
 def test_where_steps_and_tiles_end(M, N, K, S, G, L, bias, kernel):
     """Against the products with decode()'s weights in 64 bits: what tests/parity.py allows fp16 results of fp32 sums."""
@@ -35,6 +42,7 @@ def test_where_steps_and_tiles_end(M, N, K, S, G, L, bias, kernel):
     b = (torch.randn(N, generator=gen) * 0.3).to(torch.float16).to(dev) if bias else None
     y = sbvr._sbvr_linear_f16(x, bvr, idx, cache, b, bvr_len=G)
     assert hip.last_kernel() == kernel
+    assert (hip.last_row_blocks() >= 5) == ((M, N) not in ((2048, 1001), (1009, 2050), (1300, 1025)))
     assert torch.equal(y, sbvr._sbvr_linear_f16(x, bvr, idx, cache, b, bvr_len=G))
     weight = sbvr.sbvr.from_parts(bvr, idx, cache, G).decode()
     want = x.double() @ weight.double().t()

@@ -26,6 +26,8 @@ def _call(x, bvr, idx, cache, G, bias=None):
     args = [torch.from_numpy(a).to(dev) for a in (x, bvr, idx, cache)] + [none.to(dev)]
     y = sbvr._sbvr_row_deq_mm_T(*args, 0, bvr_len=G)
     assert hip.row_deq_last()[0] == hip.ROW_DEQ_ROWS
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert hip.row_deq_last_turned()
     assert torch.equal(y.view(torch.int16), sbvr._sbvr_row_deq_mm_T(*args, 0, bvr_len=G).view(torch.int16))
     assert int(hip._workspace(8 * y.numel(), dev).count_nonzero()) == 0
     return y.float().cpu().numpy().astype(np.float64), hip.row_deq_last()[1]
@@ -79,6 +81,8 @@ def test_as_exact_as_fp32_sums(N, K, S, G):
     for M in (1, 3):
         y = sbvr._sbvr_row_deq_mm_T(x.to(dev).repeat(M, 1), *args, 0, bvr_len=G).float().cpu().numpy().astype(np.float64)
         assert hip.row_deq_last()[0] in ((hip.ROW_DEQ_LANES,) if M == 1 else (hip.ROW_DEQ_ROWS,))
+        if M > 1 and torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+            assert hip.row_deq_last_turned()
         error[M] = np.sqrt(np.mean((y - rest)[:, near] ** 2))
     assert error[3] <= error[1], (error[3] / rms, error[1] / rms)
 
