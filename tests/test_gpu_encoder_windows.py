@@ -46,3 +46,16 @@ def test_state_of_two_slots_all_groups_met(groups, monkeypatch):
     w[5], w[::97] = w[5] + 2.0, w[::97] * 30.0
     _encode_both_ways(w.to(torch.float16).to("cuda:0"), dict(num_sums=2, bvr_len=32, s_search_num=8, r_search_num=16, b_search_num=8))
     assert started == [groups]
+
+
+def test_searches_of_more_than_2_24_lines():
+    """The plainer search has less than 2^24 candidate lines, whose numbers are taken apart by products, the wider one more."""
+    from sbvr.encoder import EncoderConfig, GroupEncoder
+    dev = torch.device("cuda:0")
+    conf = dict(num_sums=3, bvr_len=32, r_search_num=280, b_search_num=200, s_search_num=110, cache_warmup_num=2, search_batch_size=1 << 27)
+    enc = GroupEncoder(EncoderConfig(**conf), torch.float16, dev)
+    w = (torch.randn((6, 64), generator=torch.Generator().manual_seed(3)) * 0.02).to(torch.float16).to(dev)
+    _, lines = enc._covered_on_device(w.reshape(-1))
+    assert lines[0] < 1 << 24 < lines[1]
+    stats = _encode_both_ways(w, conf)
+    assert stats["groups"] - stats["cache_hits"] > 2
