@@ -201,18 +201,18 @@ sbvr_mm_T_mfma_kernel(const MmArgs a)
 // multiplication: 19 operations a plane word and 12 a plane's sums, against 7 + 20 for each of the 8 tiles.  A workgroup owns 16
 // columns and 16 RT rows; its W waves take the sub-groups of 128 k in turn and meet in LDS.  Bound by latency, and by the
 // image's way through the L1 (8 KiB a sub-group and row tile, for every 16 columns).
-// As exact as the planes' own product, in front of the output's rounding and over the RMS output: 0.45 to 0.9e-7 where that has
-// 0.8 to 2.0e-7, 0.4 to 0.76e-7 and 0.5 to 0.76e-7 with input coefficients of one sign (16 to 64 rows, 2 to 8 planes, K 128 to 14336).
+// As exact as the planes' own product, in front of the output's rounding and over the RMS output: 0.37 to 0.51e-7 where that has
+// 0.8 to 2.0e-7, with input coefficients of one sign 0.39 to 0.48e-7 and 0.49 to 0.76e-7 (12 to 64 rows, 2 to 8 planes, K 128 to 14336).
 // Each of these matters: powers of two that are normal numbers (the bits where they lie are subnormal ones, which the matrix cores
 // line up by their least exponent: 25e-7); sums of the first parts, exact, and of the second ones apart, and differences of planes
-// (in one sum: 2e-7 with coefficients of one sign, and 64 rows x 4096, K 4096 in 25.7 us where this takes 29.2); the waves' sums
-// added up in 64 bits.
+// (in one sum 2e-7 with coefficients of one sign; 4 us of 30 less, 64 rows x 4096, K 4096); the sub-groups' sums added up in 64
+// bits (in 32: up to 0.9e-7, and as fast).
 template <int SR, int RT, int W>
 __global__ void __launch_bounds__(64 * W)
 sbvr_online_product_kernel(const OnlineArgs a)
 {
     constexpr int CW = (SR + 1) / 2;
-    __shared__ __align__(16) float red[W * RT * 256];
+    __shared__ __align__(16) double red[W * RT * 256];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, blk = lane >> 4;
     const int N = a.N, nsub = a.K / kMmSub;
@@ -240,13 +240,18 @@ sbvr_online_product_kernel(const OnlineArgs a)
     auto coefficient = [&](const Stage &s, int j) __attribute__((always_inline)) -> float {
         return h2f(static_cast<uint16_t>(j & 1 ? s.c[j / 2] >> 16 : s.c[j / 2] & 0xffffu));
     };
-    v4f y[RT];
+    double y[RT][4] = {};
+    // Whether a coefficient of this lane's column is not finite.
+    auto not_finite_line = [&](const Stage &s) __attribute__((always_inline)) -> bool {
+        bool bad = false;
 #pragma unroll
-    for (int t = 0; t < RT; ++t)
-        y[t] = v4f{0.f, 0.f, 0.f, 0.f};
-    // A sub-group by popcounts, as sbvr_mm_T_mfma_kernel has them, a left plane of all rows at a time: where a coefficient of one of
-    // the columns is not finite, a left plane that shares no bit with its plane makes NaN of the output (0 times infinity).
-    auto plane_by_plane = [&](int sg, const Stage &s) __attribute__((always_inline)) {
+        for (int j = 0; j < SR; ++j)
+            bad = bad || !(fabsf(coefficient(s, j)) < INFINITY);
+        return bad;
+    };
+    // Such a column's sub-group by popcounts, as sbvr_mm_T_mfma_kernel has them, a left plane of all rows at a time: a left plane
+    // that shares no bit with that coefficient's plane makes NaN of the output (0 times infinity).
+    auto plane_by_plane = [&](int sg, const Stage &s, bool mine) __attribute__((always_inline)) {
 #pragma unroll 1
         for (int l = 0; l < a.Sl; ++l) {
             const float c = h2f(a.lines[static_cast<size_t>(sg / a.spg) * a.Sl + l]);
@@ -268,10 +273,11 @@ sbvr_online_product_kernel(const OnlineArgs a)
                 }
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    y[t][i] = fmaf(c, sum[i], y[t][i]);
+                    y[t][i] += mine ? static_cast<double>(c * sum[i]) : 0.;
             }
         }
     };
+    bool any_bad = false;
     auto compute = [&](int sg, const Stage &s) __attribute__((always_inline)) {
         // (asked for a sub-group ahead, in 32 registers more, the image's operands cost 1 us of 6.5)
         const v4u *const image = a.image + static_cast<size_t>(sg) * tiles * 512 + lane;
@@ -303,29 +309,28 @@ sbvr_online_product_kernel(const OnlineArgs a)
         }
         // A column's coefficients may almost cancel where its planes' sums are large and alike (activations of one sign).  The first
         // parts' sums are exact, so what two planes' differ by is: that meets the coefficients, and the first plane's sum theirs.
-        float all = 0.f;
-        bool finite = true;
+        // (a line that is not finite counts as zeros here: its sub-groups follow at the end, without a branch in this loop, which
+        // took 0.5 us of 12)
+        const bool bad = not_finite_line(s);
+        any_bad = any_bad || bad;
+        float c[SR], all = 0.f;
 #pragma unroll
         for (int j = 0; j < SR; ++j) {
-            all += coefficient(s, j);
-            finite = finite && fabsf(coefficient(s, j)) < INFINITY;
-        }
-        if (!__all(finite)) {
-            plane_by_plane(sg, s);
-            return;
+            c[j] = bad ? 0.f : coefficient(s, j);
+            all += c[j];
         }
 #pragma unroll
         for (int t = 0; t < RT; ++t)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                float sum = D[1][0][t][i] * coefficient(s, 0);
+                float sum = D[1][0][t][i] * c[0];
 #pragma unroll
                 for (int j = 1; j < SR; ++j)
-                    sum = fmaf(D[1][j][t][i], coefficient(s, j), sum);
+                    sum = fmaf(D[1][j][t][i], c[j], sum);
 #pragma unroll
                 for (int j = 1; j < SR; ++j)
-                    sum = fmaf(D[0][j][t][i] - D[0][0][t][i], coefficient(s, j), sum);
-                y[t][i] = fmaf(fmaf(D[0][0][t][i], all, sum), s.scale, y[t][i]);
+                    sum = fmaf(D[0][j][t][i] - D[0][0][t][i], c[j], sum);
+                y[t][i] += static_cast<double>(fmaf(D[0][0][t][i], all, sum) * s.scale);
             }
     };
     if (wave < nsub) {                                               // wave-uniform
@@ -339,6 +344,15 @@ sbvr_online_product_kernel(const OnlineArgs a)
             gather(next);
             now = next;
         }
+        if (__any(any_bad))
+#pragma unroll 1
+            for (int sg = wave; sg < nsub; sg += W) {
+                load(sg, now);
+                gather(now);
+                const bool bad = not_finite_line(now);
+                if (__any(bad))
+                    plane_by_plane(sg, now, bad);
+            }
     }
 #pragma unroll
     for (int t = 0; t < RT; ++t)
@@ -353,7 +367,7 @@ sbvr_online_product_kernel(const OnlineArgs a)
         double total = 0.;
 #pragma unroll
         for (int w = 0; w < W; ++w)
-            total += static_cast<double>(red[w * RT * 256 + o]);
+            total += red[w * RT * 256 + o];
         uint16_t v = f2h(static_cast<float>(total));
         if (a.bias)
             v = hadd(v, a.bias[nn]);
@@ -369,14 +383,14 @@ hipError_t launch_online_inst(const OnlineArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
-// (two row tiles of more planes: 134 to 256 registers; more than 4 planes of a 16-wave workgroup: more than its 128)
+// (two row tiles of more planes: 130 to 248 registers; 8 planes of a 16-wave workgroup: more than its 128)
 template <int SR>
 hipError_t launch_online(int RT, int W, const OnlineArgs &a, hipStream_t st)
 {
     if constexpr (SR == 2)
         if (RT == 2)
             return W == 16 ? launch_online_inst<SR, 2, 16>(a, st) : launch_online_inst<SR, 2, 8>(a, st);
-    if constexpr (SR <= 4)
+    if constexpr (SR <= 6)
         if (W == 16)
             return launch_online_inst<SR, 1, 16>(a, st);
     return launch_online_inst<SR, 1, 8>(a, st);
@@ -439,11 +453,11 @@ hipError_t launch_mm_T_mfma(int Sr, int G, MmArgs a, int cus, hipStream_t st)
 
 // Where that way is the faster one: more than 4 left planes, workgroups for three quarters of the CUs, and row tiles for whose
 // rows the planes' launch takes a third more workgroups, of up to 64 (row, plane) pairs.  us a call (both launches), planes and
-// this, 8 left and 4 right planes: 9 rows x 4096, K 4096 13.5 and 12.3; 64 rows 35.9 and 29.2; 32 x 14336, K 4096 53.1 and
-// 39.4; 48 x 1024, K 14336 43.4 and 40.0; 2048 x 4096, K 4096 973 and 715; but (too few workgroups) 16 x 1024, K 14336 17.4 and
+// this, 8 left and 4 right planes: 9 rows x 4096, K 4096 13.7 and 11.9; 64 rows 36.2 and 29.9; 32 x 14336, K 4096 52.4 and
+// 39.6; 48 x 1024, K 14336 43.2 and 38.8; 2048 x 4096, K 4096 973 and 717; but (too few workgroups) 16 x 1024, K 14336 17.4 and
 // 23.0; 64 x 512, K 4096 15.8 and 17.5; (4 left planes) 32 x 4096, K 4096 12.2 and 12.9; (6 left planes: two workgroups, two tiles)
 // 20 rows 13.0 and 15.5.  At four workgroups to three tiles it is 0.8 to 1.35 times as fast, the mean of 140 shapes 1.  Images (4
-// bytes an activation, in memory of the call's own) up to the largest measured: 2048 x 1024, K 14336 1287 us and 1142.
+// bytes an activation, in memory of the call's own) up to the largest measured: 2048 x 1024, K 14336 1287 us and 1150.
 constexpr double kOnlineImageMost = 128 << 20;
 bool online_product_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r_bvr, const void *r_cache, int cus)
 {
@@ -454,7 +468,7 @@ bool online_product_ok(int M, int N, int K, int Sl, int Sr, int G, const void *r
 }
 
 // Two row tiles share a plane word's operands where the registers hold both, with 2 planes.  (us a call, one and two, 64 rows x 4096, K
-// 4096: 4 planes 29.2 and 31.8, 3 planes, 33 rows 23.8 and 26.8.)
+// 4096: 4 planes 29.5 and 30.7; 33 rows, 3 planes 21.1 and 24.8.)
 hipError_t launch_online_product(int Sr, int G, OnlineArgs a, int cus, hipStream_t st)
 {
     a.spg = G / kMmSub;
