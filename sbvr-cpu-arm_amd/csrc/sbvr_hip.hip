@@ -2101,7 +2101,8 @@ int lut_pairs_per_wg(int pairs, int ksplit)
 // number of up to 16 that keeps a pair for every wave and gives a CU two workgroups at most, where that is estimated 4 %
 // cheaper.  Costs in units of 1 / 16 us: a word pair of a wave in a workgroup that has its CU to itself 7 + S (an odd one at the
 // end half as much again, the loop takes two), two workgroups on a CU each 1.75 + S / 20 times as long, the accumulators 25 and
-// 2 more for each part.  (Fitted to 785 launches, 600 to 8192 columns, K 2048 to 28672, 2 to 8 planes, 12 and 24 rows, each with
+// 2 more for each part.  (Fitted to 785 launches, 600 to 8192 columns, K 2048 to 28672, 2 to 8 planes, 12 and 24 rows, one of either
+// half of the rows that this kernel takes (up to 16 rows half of the accumulators stay empty), each with
 // 1 to 16 parts: 1 % from the best of them on average where doubling alone is 9.7 %, and slower than that by more than 2 % in
 // two, by 3.2 % in one.  Doubling was at its worst
 // where it kept K whole up to 4096 a part (600 columns, K 10240, 4 planes: 8.3 us against 5.9) or gave some of the CUs a
@@ -2401,7 +2402,9 @@ bool gemm_lut_path_ok(int M, int N, int K, int S, int G)
 // 256 workgroups run at a time, up to 13 % faster where fewer do; beyond that a last turn that is not full counts 0.63.
 // (Fitted to launches whose parts lie in the workspace.  Parts in memory of the call's own need no clearing, which saves 4 to 5 us of
 // 39 to 42, see sbvr_gemm_reduce_kernel; the estimate does not tell the two apart, so that both run the same parts and give the
-// same bits, and the 1 % is the former's.)
+// same bits, and the 1 % is the former's.  Five to eight row blocks are since prefill_ops.hip's, whose steps are shorter: over 70
+// shapes, 100 to 2048 rows, every number of row blocks and most of parts measured, the plan picked is 1.6 % behind the fastest on
+// average and 9 % at most: 1249 x 5178, K 16640, 4 planes 261 us where 8 row blocks in 2 parts take 239.)
 // Against one tile height and parts by powers of two: 87 rows x 5378 columns, K 19456, 3 planes, 181 us unsplit (N no
 // multiple of 4 was never split) -> 37.5; 371 x 890, K 6144, 74.9 -> 23.2; 128 x 6144, K 4096, 30.6 -> 25.7.
 // The partial results take at most kGemmLutMaxParts bytes (384 tiles of 256 x 256): the bindings keep a workspace of the

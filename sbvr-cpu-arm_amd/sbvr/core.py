@@ -416,7 +416,9 @@ class sbvr(torch.nn.Module):
 
     def online_mm_T(self, rhs, bias=None):
         """``rhs`` (M, K) activations, encoded on the fly against the profiled input coefficients, times this
-        encoded weight transposed: (M, N) fp16 through the both-encoded operator."""
+        encoded weight transposed: (M, N) fp16.  A few rows go through the both-encoded operator; from 9 on (8 input planes)
+        the encoded values may meet the weight as numbers, an other order of the same sums: within a rounding of what
+        ``_online_tranfrom`` and ``mm_T`` give, not bit for bit, and a row's last bit may differ with the rows beside it."""
         p = self._parameters
         if "input_coeff" in p and type(self) is sbvr and isinstance(rhs, torch.Tensor):
             # (straight from the parameters: look-ups through Module.__getattr__ cost as much as the checks in the call)
